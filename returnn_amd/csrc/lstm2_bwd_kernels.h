@@ -24,7 +24,8 @@ struct Lstm2BwdParams {
   long long T;
   int B, n;
   int op_flags;  // OpFlags: kOpNoCarry, kOpH0IsCell select the gradient of LstmGenericBase (returnn/native_op.py:430-485)
-  int pad_;
+  int nc;        // persistent kernel: the caller's width (n of all arrays but W and the ring), a multiple of 16 bytes; the cells from
+                 // there to n are there for the matrix cores only: their inputs read as 0, so do their derivatives come out
   long long ldDY, ldDX;  // row pitch of DY and DX in elements (n and 4n when contiguous); H, C and the mask are contiguous
   const void* Wpk;  // per-frame launches: W in MFMA A-operand order, [n/16][4n/KM][64] fragments of 16 bytes (else null)
 };
@@ -384,10 +385,10 @@ __global__ __launch_bounds__(64 * WV) void k_lstm2_bwd_regw(const Lstm2BwdMulti 
   const int g = q.group_offset + bid / kblocks, k0 = (bid % kblocks) * 16 * MT;
   const int b_base = g * q.Bg;
   const int rows = min(q.Bg, p.B - b_base);
-  const long long bn = (long long)p.B * n;
-  const unsigned frame_bytes = (unsigned)((size_t)p.B * n4 * ES);
-  const unsigned dx_frame_bytes = (unsigned)((size_t)p.B * p.ldDX * ES);
-  const long long dy_frame = (long long)p.B * p.ldDY;  // elements from one frame of DY to the next
+  const int nc = p.nc;
+  const long long bn = (long long)p.B * nc;
+  const unsigned frame_bytes = (unsigned)((size_t)p.B * 4 * nc * ES);
+  const unsigned dx_frame_bytes = (unsigned)((size_t)p.B * p.ldDX * ES), dy_frame_bytes = (unsigned)((size_t)p.B * p.ldDY * ES);
   // the exchange ring of this group: kExRing frames of [4n/KM][4][Bp][16 bytes]
   const int Bp = q.Bp;
   const unsigned ex_frame = (unsigned)((size_t)n4 * Bp * ES), frag_stride = (unsigned)(64 * Bp);
@@ -434,17 +435,20 @@ __global__ __launch_bounds__(64 * WV) void k_lstm2_bwd_regw(const Lstm2BwdMulti 
   const int upper = SPLIT ? ((tid & 255) >> 7) : 0;                // SPLIT: which of a pair of tiles
   auto tile_of = [&](int j) { return SPLIT ? set + TS * (2 * j + upper) : set + TS * j; };
   const int b = b_base + ((bl < rows) ? bl : 0);
-  const long long dy_row = (long long)b * (p.ldDY - n);  // element idx = b*n + k of a contiguous array sits at dy_row + idx in DY
-  bool act[PT];  // the pair exists: the tile does, and the group has the row
+  bool act[PT];  // the pair exists: the tile does, the group has the row and the caller the cell
   long long idx[PT], io[PT];
+  unsigned off_h[PT], off_dy[PT], off_c[PT];  // byte offsets inside a frame of H, DY and C; out of range (0 comes back) for cells beyond nc
   float dyw[PT], dc[PT], dx0[PT][4];
 #pragma unroll
   for (int j = 0; j < PT; ++j) {
     const int mt = tile_of(j);
-    act[j] = (mt < MT) && (bl < rows);
     const int k = k0 + 16 * ((mt < MT) ? mt : 0) + kl;
-    idx[j] = (long long)b * n + k;
-    io[j] = (long long)b * n4 + k;
+    act[j] = (mt < MT) && (bl < rows) && k < nc;
+    idx[j] = (long long)b * nc + k;
+    io[j] = (long long)b * 4 * nc + k;
+    off_h[j] = k < nc ? (unsigned)(io[j] * ES) : kOobOffset;
+    off_dy[j] = k < nc ? (unsigned)(((long long)b * p.ldDY + k) * ES) : kOobOffset;
+    off_c[j] = k < nc ? (unsigned)(idx[j] * 4) : kOobOffset;
     dyw[j] = 0.f;
     dc[j] = act[j] ? q.Dd[idx[j]] : 0.f;
 #pragma unroll
@@ -462,7 +466,6 @@ __global__ __launch_bounds__(64 * WV) void k_lstm2_bwd_regw(const Lstm2BwdMulti 
   unsigned in_pc[PT], in_ph[PT];
   // the frame after, on its way: as the loads bring it (a conversion next to the loads would be scheduled among the
   // MFMAs and wait there for memory)
-  typedef typename std::conditional<ES == 2, unsigned short, unsigned>::type RawT;
   unsigned nx_gate[PT][4], nx_dy[PT], nx_pc[PT], nx_ph[PT];
   float nx_m;
   auto widen = [](unsigned raw) {
@@ -477,17 +480,21 @@ __global__ __launch_bounds__(64 * WV) void k_lstm2_bwd_regw(const Lstm2BwdMulti 
     __amdgpu_buffer_rsrc_t rs_c = __builtin_amdgcn_make_buffer_rsrc((void*)csrc, 0, from_h ? 0u : (unsigned)(bn * 4), kBufFlags);
     __amdgpu_buffer_rsrc_t rs_ph = __builtin_amdgcn_make_buffer_rsrc((unsigned char*)p.H + (size_t)(prev_t < 0 ? 0 : prev_t) * frame_bytes, 0,
                                                                      from_h ? frame_bytes : 0u, kBufFlags);
+    __amdgpu_buffer_rsrc_t rs_h = __builtin_amdgcn_make_buffer_rsrc((unsigned char*)p.H + (size_t)t * frame_bytes, 0, frame_bytes, kBufFlags);
+    __amdgpu_buffer_rsrc_t rs_dy = __builtin_amdgcn_make_buffer_rsrc((unsigned char*)p.DY + (size_t)t * dy_frame_bytes, 0, dy_frame_bytes, kBufFlags);
+    auto load = [](__amdgpu_buffer_rsrc_t rs, unsigned off, int soff) -> unsigned {
+      if constexpr (ES == 2)
+        return __builtin_amdgcn_raw_buffer_load_b16(rs, off, soff, 0);
+      else
+        return __builtin_amdgcn_raw_buffer_load_b32(rs, off, soff, 0);
+    };
 #pragma unroll
     for (int j = 0; j < PT; ++j) {
-      const long long fo = t * bn * 4 + io[j];
 #pragma unroll
-      for (int gq = 0; gq < 4; ++gq) nx_gate[j][gq] = ((const RawT*)p.H)[fo + (long long)gq * n];
-      nx_dy[j] = ((const RawT*)p.DY)[dy_frame * t + dy_row + idx[j]];
-      nx_pc[j] = __builtin_amdgcn_raw_buffer_load_b32(rs_c, (unsigned)(idx[j] * 4), 0, 0);
-      if constexpr (ES == 2)
-        nx_ph[j] = __builtin_amdgcn_raw_buffer_load_b16(rs_ph, (unsigned)(io[j] * ES), 0, 0);
-      else
-        nx_ph[j] = __builtin_amdgcn_raw_buffer_load_b32(rs_ph, (unsigned)(io[j] * ES), 0, 0);
+      for (int gq = 0; gq < 4; ++gq) nx_gate[j][gq] = load(rs_h, off_h[j], gq * nc * ES);
+      nx_dy[j] = load(rs_dy, off_dy[j], 0);
+      nx_pc[j] = __builtin_amdgcn_raw_buffer_load_b32(rs_c, off_c[j], 0, 0);
+      nx_ph[j] = load(rs_ph, off_h[j], 0);
     }
     nx_m = p.mask[t * p.B + b];
   };
@@ -730,7 +737,8 @@ __global__ __launch_bounds__(64 * WV) void k_lstm2_bwd_regw(const Lstm2BwdMulti 
         if (row < rows) {
           const u32x4 v = __builtin_bit_cast(u32x4, stage[c]);
           const unsigned eo = (unsigned)(((((gate * n + k0) / KE + piece) << bp_shift) + row) * 16);
-          const unsigned dxo = (unsigned)(((size_t)(b_base + row) * p.ldDX + (size_t)gate * n + k0 + piece * KE) * ES);
+          const int cell = k0 + piece * KE;
+          const unsigned dxo = cell < nc ? (unsigned)(((size_t)(b_base + row) * p.ldDX + (size_t)gate * nc + cell) * ES) : kOobOffset;
           if (local) {
             __builtin_amdgcn_raw_buffer_store_b128(v, rs_out, eo, 0, 0);
             __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, ones), rs_arm, eo, 0, 0);
@@ -767,7 +775,35 @@ __global__ __launch_bounds__(64 * WV) void k_lstm2_bwd_regw(const Lstm2BwdMulti 
       E::store(q.Dy0, idx[j], expired ? nan : dyw[j]);
       p.Dc0[idx[j]] = expired ? nan : dc[j];
 #pragma unroll
-      for (int gq = 0; gq < 4; ++gq) E::store(p.dx0, io[j] + (long long)gq * n, expired ? nan : dx0[j][gq]);
+      for (int gq = 0; gq < 4; ++gq) E::store(p.dx0, io[j] + (long long)gq * nc, expired ? nan : dx0[j][gq]);
+    }
+  }
+}
+
+// Everything the persistent gradient kernel needs in front of it, for all problems of a launch (blockIdx.y = problem):
+// status and XCD-check words cleared, the exchange ring armed with all-ones words, and where the kernel's width n is more
+// than the caller's nc, W zero-padded into wpad [n][4][n].  (These were three fills and copies per problem.)
+struct Lstm2BwdPrepare {
+  const void* w_from[kMaxBwdMulti];
+  void* w_pad[kMaxBwdMulti];  // null: nothing to pad
+  unsigned *words[kMaxBwdMulti], *ring[kMaxBwdMulti];
+  long long n_words, ring_words;
+};
+template <typename AT>
+__global__ void k_bwd_prepare(Lstm2BwdPrepare a, int n, int nc) {
+  const int k = blockIdx.y;
+  const long long gtid = blockIdx.x * (long long)blockDim.x + threadIdx.x, gsz = (long long)gridDim.x * blockDim.x;
+  for (long long i = gtid; i < a.n_words; i += gsz) a.words[k][i] = 0u;
+  for (long long i = gtid; i < a.ring_words / 4; i += gsz) ((i32x4*)a.ring[k])[i] = i32x4{-1, -1, -1, -1};
+  if (a.w_pad[k]) {
+    constexpr int PE = 16 / (int)sizeof(AT);  // nc is a multiple of PE here
+    const long long pieces = (long long)n * 4 * (n / PE);
+    for (long long i = gtid; i < pieces; i += gsz) {
+      const int cell = (int)(i % (n / PE)) * PE;
+      const long long rg = i / (n / PE), row = rg >> 2;  // (row, gate)
+      i32x4 v = i32x4{0, 0, 0, 0};
+      if (row < nc && cell < nc) v = *(const i32x4*)((const AT*)a.w_from[k] + (row * 4 + (rg & 3)) * nc + cell);
+      ((i32x4*)a.w_pad[k])[i] = v;
     }
   }
 }

@@ -12,12 +12,12 @@ namespace rtn {
 typedef void (*RegwKernel)(const Lstm2Multi);
 typedef void (*BwdRegwKernel)(const Lstm2BwdMulti);
 
-// Forward register kernel k_lstm2_regw<AT, MT, NT, KSMAX, HALF>; null if the decomposition has no build.
+// Forward register kernel k_lstm2_regw<AT, MT, NT, KSMAX, HALF, TAIL>; null if the decomposition has no build.
 // "lo": KSMAX of 2 or 4 macro steps per wavefront, "hi": 8 or 16.
-RegwKernel regw_table_bf16_lo(int MT, int NT, int KSMAX, bool half);
-RegwKernel regw_table_bf16_hi(int MT, int NT, int KSMAX, bool half);
-RegwKernel regw_table_f32_lo(int MT, int NT, int KSMAX, bool half);
-RegwKernel regw_table_f32_hi(int MT, int NT, int KSMAX, bool half);
+RegwKernel regw_table_bf16_lo(int MT, int NT, int KSMAX, bool half, bool tail);
+RegwKernel regw_table_bf16_hi(int MT, int NT, int KSMAX, bool half, bool tail);
+RegwKernel regw_table_f32_lo(int MT, int NT, int KSMAX, bool half, bool tail);
+RegwKernel regw_table_f32_hi(int MT, int NT, int KSMAX, bool half, bool tail);
 
 // Persistent gradient kernel k_lstm2_bwd_regw<AT, KSB, MT, WV, 0, HALF>; KSB: fragments of W per tile and wavefront,
 // MT: tiles of 16 values of k per workgroup, WV: wavefronts per workgroup.  "half": groups of at most 8 rows.
@@ -29,10 +29,10 @@ BwdRegwKernel bwd_regw_table_f32_full(int KSB, int MT, int WV);
 BwdRegwKernel bwd_regw_lds_table_bf16(int WV);
 BwdRegwKernel bwd_regw_lds_table_f32(int WV);
 
-inline RegwKernel regw_kernel(int dtype, int MT, int NT, int KSMAX, bool half) {
+inline RegwKernel regw_kernel(int dtype, int MT, int NT, int KSMAX, bool half, bool tail) {
   const bool lo = KSMAX <= 4;
-  if (dtype == 1 /* RTN_DTYPE_BF16 */) return lo ? regw_table_bf16_lo(MT, NT, KSMAX, half) : regw_table_bf16_hi(MT, NT, KSMAX, half);
-  return lo ? regw_table_f32_lo(MT, NT, KSMAX, half) : regw_table_f32_hi(MT, NT, KSMAX, half);
+  if (dtype == 1 /* RTN_DTYPE_BF16 */) return lo ? regw_table_bf16_lo(MT, NT, KSMAX, half, tail) : regw_table_bf16_hi(MT, NT, KSMAX, half, tail);
+  return lo ? regw_table_f32_lo(MT, NT, KSMAX, half, tail) : regw_table_f32_hi(MT, NT, KSMAX, half, tail);
 }
 
 }  // namespace rtn

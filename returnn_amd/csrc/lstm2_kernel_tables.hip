@@ -12,11 +12,11 @@ namespace rtn {
 namespace {
 
 // Forward.  HI: the builds with 8 or 16 macro steps of the contraction per wavefront, else those with 2 or 4.
-template <typename AT, bool HI>
+template <typename AT, bool HI, bool TAIL>
 RegwKernel regw_table(int MT, int NT, int KSMAX, bool half) {
   if (half) {
 #define RTN_CASE(mt, ks) \
-  if (MT == mt && NT == 1 && KSMAX == ks) return &k_lstm2_regw<AT, mt, 1, ks, true>;
+  if (MT == mt && NT == 1 && KSMAX == ks) return &k_lstm2_regw<AT, mt, 1, ks, true, TAIL>;
     if constexpr (HI) {
       RTN_CASE(2, 8) RTN_CASE(2, 16)
       RTN_CASE(4, 8)
@@ -29,7 +29,7 @@ RegwKernel regw_table(int MT, int NT, int KSMAX, bool half) {
     return nullptr;
   }
 #define RTN_CASE(mt, nt, ks) \
-  if (MT == mt && NT == nt && KSMAX == ks) return &k_lstm2_regw<AT, mt, nt, ks>;
+  if (MT == mt && NT == nt && KSMAX == ks) return &k_lstm2_regw<AT, mt, nt, ks, false, TAIL>;
   if constexpr (HI) {
     RTN_CASE(1, 1, 8) RTN_CASE(1, 2, 8) RTN_CASE(1, 4, 8)
     RTN_CASE(2, 1, 8) RTN_CASE(2, 2, 8) RTN_CASE(2, 4, 8)
@@ -77,13 +77,13 @@ BwdRegwKernel bwd_regw_lds_table(int WV) {
 }  // namespace
 
 #if RTN_TABLE_PART == 1
-RegwKernel regw_table_bf16_lo(int MT, int NT, int KSMAX, bool half) { return regw_table<__bf16, false>(MT, NT, KSMAX, half); }
+RegwKernel regw_table_bf16_lo(int MT, int NT, int KSMAX, bool half, bool tail) { return tail ? regw_table<__bf16, false, true>(MT, NT, KSMAX, half) : regw_table<__bf16, false, false>(MT, NT, KSMAX, half); }
 #elif RTN_TABLE_PART == 2
-RegwKernel regw_table_bf16_hi(int MT, int NT, int KSMAX, bool half) { return regw_table<__bf16, true>(MT, NT, KSMAX, half); }
+RegwKernel regw_table_bf16_hi(int MT, int NT, int KSMAX, bool half, bool tail) { return tail ? regw_table<__bf16, true, true>(MT, NT, KSMAX, half) : regw_table<__bf16, true, false>(MT, NT, KSMAX, half); }
 #elif RTN_TABLE_PART == 3
-RegwKernel regw_table_f32_lo(int MT, int NT, int KSMAX, bool half) { return regw_table<float, false>(MT, NT, KSMAX, half); }
+RegwKernel regw_table_f32_lo(int MT, int NT, int KSMAX, bool half, bool tail) { return tail ? regw_table<float, false, true>(MT, NT, KSMAX, half) : regw_table<float, false, false>(MT, NT, KSMAX, half); }
 #elif RTN_TABLE_PART == 4
-RegwKernel regw_table_f32_hi(int MT, int NT, int KSMAX, bool half) { return regw_table<float, true>(MT, NT, KSMAX, half); }
+RegwKernel regw_table_f32_hi(int MT, int NT, int KSMAX, bool half, bool tail) { return tail ? regw_table<float, true, true>(MT, NT, KSMAX, half) : regw_table<float, true, false>(MT, NT, KSMAX, half); }
 #elif RTN_TABLE_PART == 5
 BwdRegwKernel bwd_regw_table_bf16_half(int KSB, int MT, int WV) { return bwd_regw_table<__bf16, true>(KSB, MT, WV); }
 #elif RTN_TABLE_PART == 6

@@ -22,6 +22,7 @@ typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
 typedef __attribute__((__vector_size__(4 * sizeof(int)))) int i32x4;
 typedef __attribute__((__vector_size__(4 * sizeof(unsigned)))) unsigned u32x4;
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
+typedef u32x4 __attribute__((aligned(2))) u32x4_any;  // 16 bytes at any element's address (rows of odd widths)
 
 constexpr int kWgThreads = 256;  // 4 wavefronts of 64
 constexpr int kWaves = 4;
@@ -129,8 +130,8 @@ static __global__ void k_copy_f32(const float* __restrict__ src, float* __restri
 // H := X copy of the reference, returnn/native_op.py:1247).  Only launched when start > 0 or |step| > 1.
 template <typename AT>
 __global__ void k_fill_unvisited(Lstm2Params p) {
-  const long long bn = (long long)p.B * p.n;
-  const int n4 = 4 * p.n;
+  const long long bn = (long long)p.B * p.nc;
+  const int n4 = 4 * p.nc;
   const long long per_frame = bn * 4;
   const long long total = p.T * per_frame;
   for (long long idx = blockIdx.x * (long long)blockDim.x + threadIdx.x; idx < total;
@@ -147,7 +148,7 @@ __global__ void k_fill_unvisited(Lstm2Params p) {
     const long long row = t * p.B + rem / n4;  // (frame, sequence)
     ((AT*)p.H)[idx] = ((const AT*)p.X)[row * p.ldX + rem % n4];
     if (rem < bn) {
-      Elem<AT>::store(p.Y, (t * p.B + rem / p.n) * p.ldY + rem % p.n, 0.f);
+      Elem<AT>::store(p.Y, (t * p.B + rem / p.nc) * p.ldY + rem % p.nc, 0.f);
       p.C[t * bn + rem] = 0.f;
     }
   }
@@ -160,6 +161,8 @@ __global__ void k_fill_unvisited(Lstm2Params p) {
 // kg = lane/16, the KE elements W[KM*sm + KE*kg + e][gate*n + 4*m + cell] with
 // cell = i/4, gate = i%4 -- i.e. the 16 rows of an M-tile are the 4 gates of 4 adjacent cells,
 // so that after the MFMA one lane holds all four gate pre-activations of one (cell, sequence).
+// Rows and columns of W and cells of y0 beyond the caller's width become zeros: the cells that fill the width up to a
+// multiple of 32 then stay exactly 0 in every frame and add nothing to the others' sums.
 template <typename AT>
 __device__ __forceinline__ void prepare_mfma(const Lstm2Params& p, int n_flags) {
   constexpr int KE = Elem<AT>::KE;
@@ -175,7 +178,7 @@ __device__ __forceinline__ void prepare_mfma(const Lstm2Params& p, int n_flags) 
     const int b = (int)(idx / p.n), c = (int)(idx % p.n);
     const int g = b / p.Bg, bl = b % p.Bg;
     const long long dst = ((long long)g * p.hx_bufs) * hx_buf + ((long long)(c / KE) * p.Bp + bl) * KE + (c % KE);
-    ((AT*)p.hx)[dst] = ((const AT*)p.y0)[idx];
+    ((AT*)p.hx)[dst] = c < p.nc ? ((const AT*)p.y0)[(long long)b * p.nc + c] : (AT)0.f;
   }
   if (p.hx_sentinel) {
     // buffers 1.. of every group: all ones = "not yet written"
@@ -201,9 +204,18 @@ __device__ __forceinline__ void prepare_mfma(const Lstm2Params& p, int n_flags) 
     const int sm = t % S, m0 = (t / S) * MB;
     for (int c = (int)threadIdx.x; c < KM * 4 * CPS; c += (int)blockDim.x) {
       const int part = c % CPS, gate = (c / CPS) % 4, k = c / (4 * CPS);
-      const int cell = 4 * m0 + part * (16 / ES);
+      const int cell = 4 * m0 + part * (16 / ES), row = KM * sm + k;
       if (cell < p.n) {
-        const u32x4 v = *(const u32x4*)((const AT*)p.W + (long long)(KM * sm + k) * 4 * p.n + gate * p.n + cell);
+        u32x4 v = u32x4{0, 0, 0, 0};
+        const AT* src = (const AT*)p.W + (long long)row * 4 * p.nc + gate * p.nc + cell;
+        if (row < p.nc && cell + 16 / ES <= p.nc) {
+          v = *(const u32x4_any*)src;
+        } else if (row < p.nc && cell < p.nc) {
+          struct { AT v[16 / ES]; } piece;
+#pragma unroll
+          for (int e = 0; e < 16 / ES; ++e) piece.v[e] = cell + e < p.nc ? src[e] : (AT)0.f;
+          v = __builtin_bit_cast(u32x4, piece);
+        }
         unsigned* dst = tile + (k * ROWP + gate * SEGP + part * 16) / 4;
         dst[0] = v[0]; dst[1] = v[1]; dst[2] = v[2]; dst[3] = v[3];
       }
@@ -438,7 +450,8 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_mfma(const Lstm2Params p, 
   const int b_base = g * p.Bg;
   const int rows = min(p.Bg, p.B - b_base);
   const bool persist = (s_end - s_begin) > 1;
-  const long long bn = (long long)p.B * n;
+  const int nc = p.nc;
+  const long long bn = (long long)p.B * nc;
   const size_t hx_buf_bytes = (size_t)n * p.Bp * sizeof(AT);
   unsigned char* hx_g = (unsigned char*)p.hx + (size_t)g * p.hx_bufs * hx_buf_bytes;
   const unsigned* flags_g = p.flags + (size_t)g * p.wgs_per_group;
@@ -451,7 +464,7 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_mfma(const Lstm2Params p, 
   // State of the (sequence, cell) pairs this thread owns.
   float c_state[EPT], h_prev[EPT];
   int e_b[EPT], e_cell[EPT];
-  bool e_valid[EPT];
+  bool e_row[EPT], e_valid[EPT];  // the group has the row; ... and the caller the cell
 #pragma unroll
   for (int j = 0; j < EPT; ++j) {
     const int e = wave + kWaves * j;
@@ -459,11 +472,12 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_mfma(const Lstm2Params p, 
     const int bl = 16 * nt + (lane & 15);
     e_cell[j] = 4 * (r * MT + mt) + (lane >> 4);
     e_b[j] = bl;
-    e_valid[j] = (e < TILES) && (bl < rows);
+    e_row[j] = (e < TILES) && (bl < rows);
+    e_valid[j] = e_row[j] && e_cell[j] < nc;
     c_state[j] = 0.f;
     h_prev[j] = 0.f;
     if (e_valid[j]) {
-      const long long bc = (long long)(b_base + bl) * n + e_cell[j];
+      const long long bc = (long long)(b_base + bl) * nc + e_cell[j];
       if (s_begin == 0) {
         c_state[j] = p.c0[bc];
         h_prev[j] = E::load(p.y0, bc);
@@ -491,7 +505,7 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_mfma(const Lstm2Params p, 
       if (e_valid[j]) {
         const size_t xo = ((size_t)t * p.B + (b_base + e_b[j])) * (size_t)p.ldX + e_cell[j];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) xg[j][q] = E::load(p.X, xo + (size_t)q * n);
+        for (int q = 0; q < 4; ++q) xg[j][q] = E::load(p.X, xo + (size_t)q * nc);
         msk[j] = p.mask[t * p.B + b_base + e_b[j]];
       }
     }
@@ -577,7 +591,7 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_mfma(const Lstm2Params p, 
         a_out[j][1] = a1;
         a_out[j][2] = a2;
         a_out[j][3] = a3;
-        if (e_valid[j]) {
+        if (e_row[j]) {
           const unsigned ho =
               (unsigned)((((e_cell[j] / KE) * p.Bp + e_b[j]) * KE + (e_cell[j] % KE)) * (int)sizeof(AT));
           if (st_coherent)
@@ -602,10 +616,10 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_mfma(const Lstm2Params p, 
 #pragma unroll
     for (int j = 0; j < EPT; ++j) {
       if (e_valid[j]) {
-        const long long bc = (long long)(b_base + e_b[j]) * n + e_cell[j];
-        const size_t xo = ((size_t)t * p.B + (b_base + e_b[j])) * 4 * n + e_cell[j];
+        const long long bc = (long long)(b_base + e_b[j]) * nc + e_cell[j];
+        const size_t xo = ((size_t)t * p.B + (b_base + e_b[j])) * 4 * nc + e_cell[j];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) E::store(p.H, xo + (size_t)q * n, a_out[j][q]);
+        for (int q = 0; q < 4; ++q) E::store(p.H, xo + (size_t)q * nc, a_out[j][q]);
         p.C[t * bn + bc] = c_state[j];
         E::store(p.Y, ((size_t)t * p.B + (b_base + e_b[j])) * (size_t)p.ldY + e_cell[j], y_out[j]);
       }
@@ -619,7 +633,7 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_mfma(const Lstm2Params p, 
 #pragma unroll
     for (int j = 0; j < EPT; ++j) {
       if (e_valid[j]) {
-        const long long bc = (long long)(b_base + e_b[j]) * n + e_cell[j];
+        const long long bc = (long long)(b_base + e_b[j]) * nc + e_cell[j];
         p.d[bc] = expired ? __builtin_nanf("") : c_state[j];
         if (expired) E::store(p.Y, ((size_t)t_last * p.B + (b_base + e_b[j])) * (size_t)p.ldY + e_cell[j], __builtin_nanf(""));
       }
@@ -849,7 +863,9 @@ __device__ __forceinline__ bool group_on_one_xcd(unsigned* words, unsigned membe
 // only, and the pointwise part folds two tiles into one pass: lanes of rows 0..7 take tile 2u, lanes of rows 8..15 take
 // rows 0..7 of tile 2u + 1, so that a thread owns one (sequence, cell) pair where the plain mapping gives it two, one
 // of them of a row that does not exist.
-template <typename AT, int MT, int NT, int KSMAX, bool HALF = false>
+// TAIL: the caller's width cuts a chunk of 16 bytes (see the streams below).  A build of its own: the few instructions and
+// registers of the tail cost the other widths up to 6 % (op of 32 steps at n = 64: 54.4 us against 51.2).
+template <typename AT, int MT, int NT, int KSMAX, bool HALF = false, bool TAIL = false>
 __global__ __launch_bounds__(kWgThreads) void k_lstm2_regw(const Lstm2Multi multi) {
   static_assert(!HALF || (NT == 1 && MT % 2 == 0), "half-tile mapping: one batch tile, an even number of cell tiles");
   // Which of the launch's problems and which (group, rank) this workgroup works on (uniform over the workgroup).
@@ -893,11 +909,11 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_regw(const Lstm2Multi mult
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: keep it in a scalar register
-  const int n = p.n, S = n / KM;
+  const int n = p.n, S = n / KM, nc = p.nc;
   g += p.group_offset;
   const int b_base = g * p.Bg;
   const int rows = min(p.Bg, p.B - b_base);
-  const long long bn = (long long)p.B * n;
+  const long long bn = (long long)p.B * nc;
   const int nsteps = p.nsteps;
 
   // ---- the op's streams: X[t], mask[t] in; H[t], Y[t], C[t] out, as 16-byte (8-byte) chunks spread
@@ -905,6 +921,9 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_regw(const Lstm2Multi mult
   // before its own (a barrier lies between that copy and its readers); the outputs are staged in LDS by the threads that compute them and written
   // out after the barrier of the following step.  Chunks of rows the group does not have carry an
   // out-of-range buffer offset: their loads return 0 and their stores are dropped, without a branch.
+  // So do chunks that reach beyond the caller's width nc; the cells of a chunk that only partly does (the TAIL, at most
+  // KE - 1 cells, all in one workgroup of a group) go element by element between memory and the thread that owns the pair.
+  // (A width that is no multiple of 32 ran on zero-padded copies of all arrays before: bf16 n=1000 B=11 T=333 113 of 620 us.)
   float* Ml = (float*)(smem + L.ml);
   constexpr int SEG = CELLS * ES;               // contiguous bytes of one (row, gate) in X and H
   constexpr int CH = SEG < 16 ? 8 : 16;         // bytes moved per thread and chunk
@@ -925,8 +944,9 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_regw(const Lstm2Multi mult
   for (int i = 0; i < XCH; ++i) {
     const int c = tid + kWgThreads * i;
     const int row = c / (4 * CPS), gate = (c / CPS) % 4, part = c % CPS;
-    xoff[i] = row < rows ? (unsigned)(((long long)(b_base + row) * p.ldX + gate * n + cell0) * ES + part * CH) : kOobOffset;
-    hoff[i] = row < rows ? (unsigned)((((b_base + row) * 4 * n) + gate * n + cell0) * ES + part * CH) : kOobOffset;
+    const bool there = row < rows && cell0 + (part + 1) * (CH / ES) <= nc;
+    xoff[i] = there ? (unsigned)(((long long)(b_base + row) * p.ldX + gate * nc + cell0) * ES + part * CH) : kOobOffset;
+    hoff[i] = there ? (unsigned)(((long long)(b_base + row) * 4 * nc + gate * nc + cell0) * ES + part * CH) : kOobOffset;
     // threads beyond the tile write to / read from the spare slot at the end of the copy
     xlds[i] = row < ROWS ? (unsigned)(row * L.x_row + gate * SEG + part * CH) : (unsigned)(ROWS * L.x_row);
   }
@@ -934,18 +954,18 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_regw(const Lstm2Multi mult
   for (int i = 0; i < YCH; ++i) {
     const int c = tid + kWgThreads * i;
     const int row = c / (SEG / CHY), part = c % (SEG / CHY);
-    yoff[i] = row < rows ? (unsigned)(((long long)(b_base + row) * p.ldY + cell0) * ES + part * CHY) : kOobOffset;
+    yoff[i] = row < rows && cell0 + (part + 1) * (CHY / ES) <= nc ? (unsigned)(((long long)(b_base + row) * p.ldY + cell0) * ES + part * CHY) : kOobOffset;
     ylds[i] = (unsigned)(min(row, ROWS - 1) * L.y_row + part * CHY);
   }
 #pragma unroll
   for (int i = 0; i < CCH; ++i) {
     const int c = tid + kWgThreads * i;
     const int row = c / (SEGC / 16), part = c % (SEGC / 16);
-    coff[i] = row < rows ? (unsigned)(((b_base + row) * n + cell0) * 4 + part * 16) : kOobOffset;
+    coff[i] = row < rows && cell0 + (part + 1) * 4 <= nc ? (unsigned)(((b_base + row) * nc + cell0) * 4 + part * 16) : kOobOffset;
     clds[i] = (unsigned)(min(row, ROWS - 1) * L.c_row + part * 16);
   }
   const unsigned moff = tid < rows ? (unsigned)((b_base + tid) * 4) : kOobOffset;
-  const unsigned frame_x = (unsigned)((size_t)p.B * p.ldX * ES), frame_h = (unsigned)((size_t)p.B * 4 * n * ES),
+  const unsigned frame_x = (unsigned)((size_t)p.B * p.ldX * ES), frame_h = (unsigned)((size_t)p.B * 4 * nc * ES),
                  frame_y = (unsigned)((size_t)p.B * p.ldY * ES), frame_c = (unsigned)(bn * 4), frame_m = (unsigned)(p.B * 4);
   typename XC::T xv[2][XCH];
   float mv[2] = {0.f, 0.f};
@@ -1090,16 +1110,33 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_regw(const Lstm2Multi mult
     e_src[j] = (unsigned)src;
     e_row[j] = (unsigned)bl;
     e_cl[j] = (unsigned)(4 * mt + (lane >> 4));
-    e_valid[j] = (wave + kWaves * j < UNITS) && (bl < rows);
+    e_valid[j] = (wave + kWaves * j < UNITS) && (bl < rows) && cell < nc;
     e_hoff[j] = (unsigned)((((cell / KE) * p.Bp + bl) * KE + (cell % KE)) * ES);
     c_state[j] = 0.f;
     h_prev[j] = 0.f;
     if (e_valid[j]) {
-      const long long bc = (long long)(b_base + bl) * n + cell;
+      const long long bc = (long long)(b_base + bl) * nc + cell;
       c_state[j] = p.c0[bc];
       h_prev[j] = E::load(p.y0, bc);
     }
   }
+  // The tail: first cell (inside this workgroup's tile) of the chunk of X, H and Y, and of C, that the width cuts.
+  const int tail_x = nc - nc % (CH / ES) - cell0, tail_c = nc - nc % 4 - cell0;
+  const bool has_tail = TAIL && nc % (CH / ES) != 0 && tail_x >= 0 && tail_x < CELLS;  // uniform over the workgroup
+  AT x_tail[EPT][4];
+#pragma unroll
+  for (int j = 0; j < EPT; ++j)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) x_tail[j][q] = (AT)0.f;
+  auto fetch_tail = [&](int s) {  // the tail's gate inputs of step s, from memory
+#pragma unroll
+    for (int j = 0; j < EPT; ++j)
+      if (e_valid[j] && (int)e_cl[j] >= tail_x) {
+        const AT* xp = (const AT*)p.X + ((size_t)frame_of(p, s) * p.B + b_base + e_row[j]) * (size_t)p.ldX + cell0 + e_cl[j];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) x_tail[j][q] = xp[(size_t)q * nc];
+      }
+  };
 
   // An XCD-local plan rests on all workgroups of the group being on one XCD.  Check it: every workgroup adds its XCD
   // to the group's mask and then itself to the group's count (two words the prepare kernel cleared; device-scope
@@ -1335,6 +1372,14 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_regw(const Lstm2Multi mult
 #pragma unroll
           for (int nt = 0; nt < NT; ++nt) redbuf[wave][mt * NT + nt][lane] = acc[mt][nt];
       }
+      if (has_tail) {
+#pragma unroll
+        for (int j = 0; j < EPT; ++j)
+          if (e_valid[j] && (int)e_cl[j] >= tail_x) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) x_f[j][q] = (float)x_tail[j][q];
+          }
+      }
       RTN_TRACE_MARK(1)  // MFMA with the streams in their shadow, partial tiles to LDS
       __syncthreads();  // the one barrier of a step: partial tiles, X[t_{s+2}] and the outputs of step s-1 are in LDS
       RTN_TRACE_MARK(2)  // barrier
@@ -1397,6 +1442,19 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_regw(const Lstm2Multi mult
           *(float*)(smem + st_c + e_row[j] * L.c_row + e_cl[j] * 4) = c_state[j];
         }
       }
+      if (has_tail) {
+        const size_t frame_row = (size_t)frame_of(p, s) * p.B + b_base;
+#pragma unroll
+        for (int j = 0; j < EPT; ++j)
+          if (e_valid[j] && (int)e_cl[j] >= tail_x) {
+            const size_t row = frame_row + e_row[j], cell = (size_t)cell0 + e_cl[j];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) ((AT*)p.H)[row * 4 * nc + (size_t)q * nc + cell] = (AT)g_act[j][q];
+            ((AT*)p.Y)[row * (size_t)p.ldY + cell] = (AT)y_out[j];
+            if ((int)e_cl[j] >= tail_c) p.C[row * nc + cell] = c_state[j];
+          }
+        if (s + 1 < nsteps) fetch_tail(s + 1);
+      }
       if (s + 1 < nsteps) {
         for (int k = 0; k < delay; ++k) __builtin_amdgcn_s_sleep(1);
         issue(s + 1);
@@ -1412,6 +1470,7 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_regw(const Lstm2Multi mult
     if (nsteps > 2) fetch(2, IntTag<0>{});
     if (nsteps > 3) fetch(3, IntTag<1>{});
     __syncthreads();  // everybody has the gate inputs of step 0: its LDS copy may take X[t_2]
+    if (has_tail) fetch_tail(0);
     issue(0);
     int stage = 0;
     // frames of the outputs of step s-2 and of the inputs of step s+4, as the loop reaches step s
@@ -1432,9 +1491,9 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_regw(const Lstm2Multi mult
     RTN_TRACE_FLUSH(p, trace_id)
   };
   __syncthreads();  // s_local
-  if (p.exchange == kExNoWait) {
+  if (!TAIL && p.exchange == kExNoWait) {
     if (tid == 0) __hip_atomic_store(p.status, 2u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    run(IntTag<kExNoWait>{});
+    if constexpr (!TAIL) run(IntTag<kExNoWait>{});
   } else if (multi.local && s_local) {
     run(IntTag<kExLocal>{});
   } else {
@@ -1458,7 +1517,7 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_regw(const Lstm2Multi mult
 
 #pragma unroll
   for (int j = 0; j < EPT; ++j)
-    if (e_valid[j]) p.d[(long long)(b_base + e_row[j]) * n + 4 * MT * r + e_cl[j]] = expired ? __builtin_nanf("") : c_state[j];
+    if (e_valid[j]) p.d[(long long)(b_base + e_row[j]) * nc + 4 * MT * r + e_cl[j]] = expired ? __builtin_nanf("") : c_state[j];
 }
 
 

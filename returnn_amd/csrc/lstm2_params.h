@@ -49,7 +49,8 @@ struct Lstm2Params {
   long long ldX;  // elements between the rows of X of two consecutive (frame, sequence) pairs: 4n when X is contiguous; more when
                   // the caller's rows are wider (e.g. [T*B, 8n]: the pre-projected gates of two directions side by side)
   long long ldY;  // the same for the rows of Y: n when contiguous (2n: the two directions of a layer write into one [T,B,2n] array)
-  int B, n;
+  int B, n;    // n: width the kernels work at, a multiple of 32 on the matrix cores
+  int nc;      // the caller's width (nc <= n): the widths and pitches of the caller's arrays; cells nc ... n-1 do not exist
   int first;   // first visited frame
   int step;    // signed stride between visited frames
   int nsteps;  // number of visited frames

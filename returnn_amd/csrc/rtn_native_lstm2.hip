@@ -944,33 +944,13 @@ int check_dims(int64_t T, int32_t B, int32_t n, int32_t dtype) {
 // ---- widths the matrix-core kernels do not take ------------------------------------------------------------------
 // n that is not a multiple of 32 runs zero-padded to the next multiple: a padded cell has zero inputs, zero weights (rows
 // and columns) and a zero initial state, so its cell state and output are exactly 0 in every frame, it adds nothing to
-// the other cells' sums and all its gradients are 0 -- the results are those of the unpadded problem.  The copies cost
-// about the op's own memory traffic again, far less than the element-wise kernels that such widths would otherwise
-// run on (n=1000: 120 times slower).  Widths up to 32 stay on those kernels; RTN_LSTM2_NO_PAD=1 switches the padding off.
+// the other cells' sums and all its gradients are 0 -- the results are those of the unpadded problem.  The forward
+// kernels pad on the fly (Lstm2Params::nc: what they read beyond the caller's width is 0, what they would write there is
+// dropped), the gradient kernel does so where rows stay 16-byte aligned and runs on padded copies otherwise.  Widths up
+// to 32 stay on the element-wise kernels (n=1000 was 120 times slower on those); RTN_LSTM2_NO_PAD=1 switches the padding off.
 int padded_width(int n) {
   if (n % 32 == 0 || n <= 32 || env_long("RTN_LSTM2_NO_PAD", 0)) return n;
   return (n + 31) / 32 * 32;
-}
-
-// Padded copies of one forward call's tensors (byte offsets into its share of the workspace).
-struct FwdPadLayout {
-  size_t X = 0, W = 0, y0 = 0, c0 = 0, Y = 0, C = 0, H = 0, d = 0, total = 0;
-};
-FwdPadLayout fwd_pad_layout(int64_t T, int B, int np, int dtype) {
-  const size_t es = esize(dtype), tb = (size_t)T * B, bn = (size_t)B * np;
-  FwdPadLayout l;
-  size_t off = 0;
-  auto take = [&](size_t bytes) { const size_t at = off; off = align_up(off + bytes, 256); return at; };
-  l.X = take(tb * 4 * np * es);
-  l.W = take((size_t)np * 4 * np * es);
-  l.y0 = take(bn * es);
-  l.c0 = take(bn * 4);
-  l.Y = take(tb * np * es);
-  l.C = take(tb * np * 4);
-  l.H = take(tb * 4 * np * es);
-  l.d = take(bn * 4);
-  l.total = off;
-  return l;
 }
 
 // Padded copies of one gradient call's tensors.
@@ -1055,8 +1035,14 @@ int resolve_pitch(const char* name, long long given, long long contiguous, int B
   return RTN_OK;
 }
 
-// Workspace of one of `count` forward calls at a width the kernels take as it is.
-size_t workspace_each_exact(int count, int64_t T, int32_t B, int32_t n, int32_t dtype, int32_t mode) {
+// Workspace of one of `count` forward calls (call k's slice starts at k times this, with its status block first).
+size_t workspace_each(int count, int64_t T, int32_t B, int32_t n, int32_t dtype, int32_t mode) {
+  // For a padded width the size stays what it was when such widths ran on copies (X W y0 c0 Y C H d at the padded width):
+  // callers rely on the query, which is never smaller than for the width it is padded to plus those copies.
+  const int np = padded_width(n);
+  const size_t es = esize(dtype), tb = (size_t)T * B;
+  const size_t slack = np == n || T == 0 || B == 0 ? 0 : align_up(tb * np * (9 * es + 4) + (size_t)np * 4 * np * es + (size_t)B * np * (es + 8) + 8 * 256, 256);
+  n = np;
   size_t need = 0;
   Plan pl;
   std::string why;
@@ -1068,15 +1054,7 @@ size_t workspace_each_exact(int count, int64_t T, int32_t B, int32_t n, int32_t 
       if (make_plan(T, B, n, dtype, RTN_MODE_STEPWISE, true, &pl, &why)) need = std::max(need, pl.total);
     }
   }
-  return need;
-}
-
-// Workspace of one of `count` forward calls (call k's slice starts at k times this, with its status block first): for a
-// padded width, that of the padded problem followed by the padded copies.
-size_t workspace_each(int count, int64_t T, int32_t B, int32_t n, int32_t dtype, int32_t mode) {
-  const int np = padded_width(n);
-  if (np == n || T == 0 || B == 0) return workspace_each_exact(count, T, B, n, dtype, mode);
-  return workspace_each_exact(count, T, B, np, dtype, mode) + fwd_pad_layout(T, B, np, dtype).total;
+  return need + slack;
 }
 
 int static_scratch(void** out);
@@ -1120,63 +1098,12 @@ int probe_xcds(hipStream_t stream) {
   return RTN_OK;
 }
 
-int fwd_calls(const rtn_lstm2_call* calls, int count, int64_t T, int32_t B, int32_t n, int32_t dtype, int32_t mode,
-              void* workspace, size_t workspace_bytes, void* hip_stream, int op_flags = 0, size_t ws_stride = 0,
-              bool no_graph = false);
-
-// The problems zero-padded to a width the matrix-core kernels take (see padded_width), on copies in the workspace: slice
-// k = the workspace of the padded call k, then its padded copies.
-int fwd_padded(const rtn_lstm2_call* calls, int count, int64_t T, int32_t B, int32_t n, int np, int32_t dtype, int32_t mode,
-               void* workspace, size_t workspace_bytes, hipStream_t stream, int op_flags, bool no_graph) {
-  int rc = RTN_OK;
-  for (int k = 0; k < count; ++k) {
-    const rtn_lstm2_call& c = calls[k];
-    const void* ptrs[] = {c.X, c.W, c.y0, c.c0, c.i, c.Y, c.C, c.H, c.d};
-    const char* names[] = {"X", "W", "y0", "c0", "i", "Y", "C", "H", "d"};
-    for (int q = 0; q < 9; ++q)
-      if (!ptrs[q]) return fail(RTN_ERR_ARG, "NativeLstm2: %s must not be null", names[q]);
-  }
-  const size_t inner_each = workspace_each_exact(count, T, B, np, dtype, mode);
-  const FwdPadLayout L = fwd_pad_layout(T, B, np, dtype);
-  const size_t each = inner_each + L.total;
-  const size_t need = (size_t)count * each;
-  if (!workspace || workspace_bytes < need)
-    return fail(RTN_ERR_WORKSPACE, "NativeLstm2: workspace of %zu bytes needed, got %zu", need, workspace ? workspace_bytes : (size_t)0);
-  if (!aligned16(workspace)) return fail(RTN_ERR_ARG, "NativeLstm2: workspace must be 16-byte aligned");
-  const size_t es = esize(dtype);
-  const long long tb = (long long)T * B;
-  std::vector<rtn_lstm2_call> padded((size_t)count);
-  for (int k = 0; k < count; ++k) {
-    const rtn_lstm2_call& c = calls[k];
-    unsigned char* base = (unsigned char*)workspace + (size_t)k * each + inner_each;
-    long long ldX = 0, ldY = 0;
-    if ((rc = resolve_pitch("ldX", c.ldX, 4LL * n, B, es, &ldX)) != RTN_OK) return rc;
-    if ((rc = resolve_pitch("ldY", c.ldY, n, B, es, &ldY)) != RTN_OK) return rc;
-    if ((rc = launch_pad(c.X, base + L.X, tb, tb, 4, n, np, es, stream, ldX)) != RTN_OK) return rc;
-    if ((rc = launch_pad(c.W, base + L.W, n, np, 4, n, np, es, stream)) != RTN_OK) return rc;
-    if ((rc = launch_pad(c.y0, base + L.y0, B, B, 1, n, np, es, stream)) != RTN_OK) return rc;
-    if ((rc = launch_pad(c.c0, base + L.c0, B, B, 1, n, np, 4, stream)) != RTN_OK) return rc;
-    padded[(size_t)k] = {base + L.X, base + L.W, base + L.y0, (const float*)(base + L.c0), c.i, c.start, c.step,
-                         base + L.Y, (float*)(base + L.C), base + L.H, (float*)(base + L.d), 0, 0};
-  }
-  rc = fwd_calls(padded.data(), count, T, B, np, dtype, mode, workspace, need, (void*)stream, op_flags, each, no_graph);
-  if (rc != RTN_OK) return rc;
-  for (int k = 0; k < count; ++k) {
-    const rtn_lstm2_call& c = calls[k];
-    const rtn_lstm2_call& q = padded[(size_t)k];
-    if ((rc = launch_unpad(q.Y, c.Y, tb, 1, n, np, es, stream, c.ldY)) != RTN_OK) return rc;
-    if ((rc = launch_unpad(q.C, c.C, tb, 1, n, np, 4, stream)) != RTN_OK) return rc;
-    if ((rc = launch_unpad(q.H, c.H, tb, 4, n, np, es, stream)) != RTN_OK) return rc;
-    if ((rc = launch_unpad(q.d, c.d, B, 1, n, np, 4, stream)) != RTN_OK) return rc;
-  }
-  return RTN_OK;
-}
-
 // The plan of an entry, settled against the device: a persistent plan needs all its workgroups on the device together,
 // so it is checked against what the kernel really gets per CU, planned again for that if it was too optimistic, and
 // given up for per-step launches if that does not help.  *pk: the persistent kernel (null: launches per step);
 // *fused: problems per persistent launch.
-int settle_fwd_plan(int count, int64_t T, int B, int n, int dtype, int mode, bool capturing, Plan* plan, const void** pk, int* fused) {
+// nc: the caller's width, which the plan takes as n.
+int settle_fwd_plan(int count, int64_t T, int B, int nc, int n, int dtype, int mode, bool capturing, Plan* plan, const void** pk, int* fused) {
   Plan& pl = *plan;
   std::string why;
   int rc = RTN_OK;
@@ -1186,7 +1113,7 @@ int settle_fwd_plan(int count, int64_t T, int B, int n, int dtype, int mode, boo
   if (!make_plan(T, B, n, dtype, mode, capturing, &pl, &why, 2, plan_count))
     return fail(RTN_ERR_UNSUPPORTED, "NativeLstm2: persistent mode unavailable for T=%lld B=%d n=%d: %s", (long long)T, B, n, why.c_str());
   for (int attempt = 0; pl.kind == kPlanMfma && pl.mode == RTN_MODE_PERSISTENT; ++attempt) {
-    *pk = pl.regw ? (const void*)regw_kernel(dtype, pl.MT, pl.NT, pl.KSMAX, pl.half) : (const void*)mfma_kernel(dtype, pl.MT, pl.NT);
+    *pk = pl.regw ? (const void*)regw_kernel(dtype, pl.MT, pl.NT, pl.KSMAX, pl.half, nc % (int)(std::min<size_t>(16, 4 * pl.MT * esize(dtype)) / esize(dtype)) != 0) : (const void*)mfma_kernel(dtype, pl.MT, pl.NT);
     if (!*pk) return fail(RTN_ERR_UNSUPPORTED, "NativeLstm2: no kernel for mt=%d nt=%d ks=%d", pl.MT, pl.NT, pl.KSMAX);
     if ((rc = ensure_lds_limit(*pk, pl.lds_bytes)) != RTN_OK) return rc;
     const int wgs = pl.regw ? pl.grid : pl.groups * pl.wgs_per_group;
@@ -1213,8 +1140,8 @@ int settle_fwd_plan(int count, int64_t T, int B, int n, int dtype, int mode, boo
   return RTN_OK;
 }
 
-// The parameter block of call `c` on plan `pl` with its workspace slice at `ws`.
-int fill_fwd_params(const rtn_lstm2_call& c, const Plan& pl, bool persistent, unsigned char* ws, int64_t T, int B, int n, int dtype,
+// The parameter block of call `c` (width n, which the plan takes as np) on plan `pl` with its workspace slice at `ws`.
+int fill_fwd_params(const rtn_lstm2_call& c, const Plan& pl, bool persistent, unsigned char* ws, int64_t T, int B, int n, int np, int dtype,
                     int op_flags, Lstm2Params* out) {
   Lstm2Params& p = *out;
   int rc = RTN_OK;
@@ -1227,7 +1154,7 @@ int fill_fwd_params(const rtn_lstm2_call& c, const Plan& pl, bool persistent, un
   p.Wp = ws + pl.off_wp;
   p.ycarry = ws + pl.off_ycarry;
   p.trace = pl.off_trace ? (unsigned long long*)(ws + pl.off_trace) : nullptr;
-  p.T = T; p.B = B; p.n = n;
+  p.T = T; p.B = B; p.n = np; p.nc = n;
   if ((rc = resolve_pitch("ldX", c.ldX, 4LL * n, B, esize(dtype), &p.ldX)) != RTN_OK) return rc;
   if ((rc = resolve_pitch("ldY", c.ldY, n, B, esize(dtype), &p.ldY)) != RTN_OK) return rc;
   // returnn/native_op.py:1253-1259
@@ -1274,7 +1201,7 @@ int fill_fwd_params(const rtn_lstm2_call& c, const Plan& pl, bool persistent, un
 // When the persistent register kernel fits that many times on the device at once, all of them run
 // in one launch (every workgroup with a CU to itself); otherwise they are enqueued one after the other.
 int fwd_calls(const rtn_lstm2_call* calls, int count, int64_t T, int32_t B, int32_t n, int32_t dtype, int32_t mode,
-              void* workspace, size_t workspace_bytes, void* hip_stream, int op_flags, size_t ws_stride, bool no_graph) {
+              void* workspace, size_t workspace_bytes, void* hip_stream, int op_flags = 0, bool no_graph = false) {
   int rc = check_dims(T, B, n, dtype);
   if (rc != RTN_OK) return rc;
   if (mode < RTN_MODE_AUTO || mode > RTN_MODE_STEPWISE) return fail(RTN_ERR_ARG, "NativeLstm2: unknown mode %d", mode);
@@ -1292,8 +1219,7 @@ int fwd_calls(const rtn_lstm2_call* calls, int count, int64_t T, int32_t B, int3
     }
     return RTN_OK;
   }
-  const int np = padded_width(n);
-  if (np != n) return fwd_padded(calls, count, T, B, n, np, dtype, mode, workspace, workspace_bytes, stream, op_flags, no_graph);
+  const int np = padded_width(n);  // the width of the plan
   for (int k = 0; k < count; ++k) {
     const rtn_lstm2_call& c = calls[k];
     if (c.start < 0 || c.start >= T)
@@ -1303,9 +1229,9 @@ int fwd_calls(const rtn_lstm2_call* calls, int count, int64_t T, int32_t B, int3
     const char* names[] = {"X", "W", "y0", "c0", "i", "Y", "C", "H", "d"};
     for (int q = 0; q < 9; ++q) {
       if (!ptrs[q]) return fail(RTN_ERR_ARG, "NativeLstm2: %s must not be null", names[q]);
-      // W is read in 16-byte fragments by the MFMA kernels only (n a multiple of 32); the generic kernels read single
-      // elements, which lets LstmLowMem pass the recurrent rows of its stacked matrix at any element offset
-      if (q != 4 && !(q == 1 && n % 32 != 0) && !aligned16(ptrs[q]))
+      // 16-byte accesses are aligned ones where n is a multiple of 32 (at other widths rows lie anywhere, and LstmLowMem
+      // passes the recurrent rows of its stacked matrix at any element offset)
+      if (q != 4 && np == n && !(q == 1 && n % 32 != 0) && !aligned16(ptrs[q]))
         return fail(RTN_ERR_ARG, "NativeLstm2: %s must be 16-byte aligned", names[q]);
     }
   }
@@ -1317,9 +1243,8 @@ int fwd_calls(const rtn_lstm2_call* calls, int count, int64_t T, int32_t B, int3
   Plan pl;
   const void* pk = nullptr;  // the persistent kernel, if any
   int fused = 1;             // problems per persistent launch
-  if ((rc = settle_fwd_plan(count, T, B, n, dtype, mode, capturing, &pl, &pk, &fused)) != RTN_OK) return rc;
-  // distance between the calls' workspaces: given by a caller that keeps more than the workspace in a call's slice
-  const size_t each_ws = ws_stride ? ws_stride : (count > 1 ? workspace_each(count, T, B, n, dtype, mode) : pl.total);
+  if ((rc = settle_fwd_plan(count, T, B, n, np, dtype, mode, capturing, &pl, &pk, &fused)) != RTN_OK) return rc;
+  const size_t each_ws = count > 1 ? workspace_each(count, T, B, n, dtype, mode) : pl.total;  // distance between the calls' workspaces
   if (each_ws < pl.total) return fail(RTN_ERR_WORKSPACE, "NativeLstm2: internal: workspace slice %zu < layout %zu", each_ws, pl.total);
   if (!workspace || workspace_bytes < each_ws * (size_t)count)
     return fail(RTN_ERR_WORKSPACE, "NativeLstm2: workspace of %zu bytes needed, got %zu", each_ws * (size_t)count,
@@ -1334,7 +1259,7 @@ int fwd_calls(const rtn_lstm2_call* calls, int count, int64_t T, int32_t B, int3
   int pending = 0;  // problems prepared for the next persistent launch
   for (int k = 0; k < count; ++k) {
     Lstm2Params p;
-    if ((rc = fill_fwd_params(calls[k], pl, pk != nullptr, (unsigned char*)workspace + (size_t)k * each_ws, T, B, n, dtype, op_flags, &p)) != RTN_OK)
+    if ((rc = fill_fwd_params(calls[k], pl, pk != nullptr, (unsigned char*)workspace + (size_t)k * each_ws, T, B, n, np, dtype, op_flags, &p)) != RTN_OK)
       return rc;
 
     // Frames the loop never visits.
@@ -1355,7 +1280,7 @@ int fwd_calls(const rtn_lstm2_call* calls, int count, int64_t T, int32_t B, int3
         rc = ensure_lds_limit((const void*)mk, pl.lds_bytes);
         if (rc != RTN_OK) return rc;
       }
-      const long long work = std::max<long long>((long long)n * n, bn);
+      const long long work = std::max<long long>((long long)np * np, bn);
       const dim3 pgrid((unsigned)std::min<long long>((work + 255) / 256, 2048)), pblock(256);
       // (the problems of a fused launch are prepared by one launch, in front of it)
       const bool prepared_with_the_others = pk && pl.regw && pl.passes <= 1;
@@ -1450,13 +1375,13 @@ int blas_handle(rocblas_handle* out) {
   return RTN_OK;
 }
 
-// DW[n,4n] (row major, float32) += A[rows,n]^T * Bm[rows,4n] with A, Bm of element type `dtype`, row major.
-int dw_accumulate(rocblas_handle h, const void* A, const void* Bm, float* DW, long long rows, int n, int dtype, long long lda = 0,
-                  long long ldb = 0) {
+// DW[n,4n] (row major, float32) = A[rows,n]^T * Bm[rows,4n] + beta * DW with A, Bm of element type `dtype`, row major.
+int dw_product(rocblas_handle h, const void* A, const void* Bm, float beta, float* DW, long long rows, int n, int dtype, long long lda = 0,
+               long long ldb = 0) {
   if (rows <= 0) return RTN_OK;
   if (lda == 0) lda = n;
   if (ldb == 0) ldb = 4LL * n;
-  const float alpha = 1.f, beta = 1.f;
+  const float alpha = 1.f;
   const rocblas_datatype in = dtype == RTN_DTYPE_BF16 ? rocblas_datatype_bf16_r : rocblas_datatype_f32_r;
   // Row-major DW[n,4n] is column-major [4n,n]: DW^T = Bm^T * A, with row-major Bm[rows,4n] = column-major [4n,rows]
   // (no transpose) and row-major A[rows,n] = column-major [n,rows] (transpose).  lda, ldb: row pitch of A and Bm in
@@ -1698,7 +1623,7 @@ int rtn_native_lstm2_fwd_static(const void* X, const void* W, const void* y0, co
   rtn_lstm2_call call = {X, W, y0, c0, i, start, step, Y, C, H, d};
   // (nothing may be created at call time here: the persistent kernel keeps the cooperative launch, which needs no event)
   g_no_setup_objects = true;
-  rc = fwd_calls(&call, 1, T, B, n, dtype, mode, ws, (size_t)RTN_STATIC_SCRATCH_BYTES, hip_stream, 0, 0, /*no_graph=*/true);
+  rc = fwd_calls(&call, 1, T, B, n, dtype, mode, ws, (size_t)RTN_STATIC_SCRATCH_BYTES, hip_stream, 0, /*no_graph=*/true);
   g_no_setup_objects = false;
   return rc;
 }
@@ -1881,7 +1806,7 @@ struct BwdCtx {
   const rtn_lstm2_bwd_call* calls;
   int count;
   int64_t T;
-  int B, n, dtype, op_flags;
+  int B, n, np, dtype, op_flags;  // np: the width the kernels work at (>= n)
   hipStream_t stream;
   bool capturing;
   size_t es;     // bytes per activation element
@@ -1903,9 +1828,9 @@ struct BwdChoice {
 int bwd_calls(const rtn_lstm2_bwd_call* calls, int count, int64_t T, int32_t B, int32_t n, int32_t dtype, void* workspace,
               size_t workspace_bytes, void* hip_stream, int op_flags = 0, size_t ws_stride = 0);
 
-// Argument checks and the outputs that do not depend on the recurrence: DW := 0, Dc0 := Dd, and Dy0 := 0 where there is
-// no frame to run (returnn/native_op.py:1365-1370).
-int bwd_check_and_clear(const BwdCtx& x) {
+// Argument checks, and the outputs of a call without any frame: DW := 0, Dc0 := Dd, Dy0 := 0 (returnn/native_op.py:
+// 1365-1370).  With frames every output is written by the kernels and products themselves.
+int bwd_check(const BwdCtx& x) {
   const long long nn4 = (long long)x.n * x.n * 4;
   const dim3 fill_grid(256), fill_block(256);
   for (int k = 0; k < x.count; ++k) {
@@ -1913,22 +1838,21 @@ int bwd_check_and_clear(const BwdCtx& x) {
     if (nn4 > 0 && !c.DW) return fail(RTN_ERR_ARG, "NativeLstm2 backward: DW must not be null");
     if (x.bn > 0 && (!c.Dd || !c.Dy0 || !c.Dc0)) return fail(RTN_ERR_ARG, "NativeLstm2 backward: Dd, Dy0 and Dc0 must not be null");
   }
-  for (int k = 0; k < x.count; ++k) {
-    const rtn_lstm2_bwd_call& c = x.calls[k];
-    if (nn4 > 0) {
-      hipLaunchKernelGGL(k_fill_u32, fill_grid, fill_block, 0, x.stream, (unsigned*)c.DW, 0u, nn4);
-      RTN_HIP(hipGetLastError());
+  if (x.T == 0 || x.bn == 0 || x.count == 0) {
+    for (int k = 0; k < x.count; ++k) {
+      const rtn_lstm2_bwd_call& c = x.calls[k];
+      if (nn4 > 0) {
+        hipLaunchKernelGGL(k_fill_u32, fill_grid, fill_block, 0, x.stream, (unsigned*)c.DW, 0u, nn4);
+        RTN_HIP(hipGetLastError());
+      }
+      if (x.bn > 0) {
+        hipLaunchKernelGGL(k_copy_f32, fill_grid, fill_block, 0, x.stream, c.Dd, c.Dc0, x.bn);
+        hipLaunchKernelGGL(k_fill_u32, fill_grid, fill_block, 0, x.stream, (unsigned*)c.Dy0, 0u, (long long)(((size_t)x.bn * x.es + 3) / 4));
+        RTN_HIP(hipGetLastError());
+      }
     }
-    if (x.bn > 0) {
-      hipLaunchKernelGGL(k_copy_f32, fill_grid, fill_block, 0, x.stream, c.Dd, c.Dc0, x.bn);
-      RTN_HIP(hipGetLastError());
-    }
-    if ((x.T == 0 || x.bn == 0) && x.bn > 0) {
-      hipLaunchKernelGGL(k_fill_u32, fill_grid, fill_block, 0, x.stream, (unsigned*)c.Dy0, 0u, (long long)(((size_t)x.bn * x.es + 3) / 4));
-      RTN_HIP(hipGetLastError());
-    }
+    return RTN_OK;
   }
-  if (x.T == 0 || x.bn == 0 || x.count == 0) return RTN_OK;
   for (int k = 0; k < x.count; ++k) {
     const rtn_lstm2_bwd_call& c = x.calls[k];
     if (c.start < 0 || c.start >= x.T)
@@ -2001,7 +1925,7 @@ int bwd_padded(const BwdCtx& x, int np, void* workspace, size_t workspace_bytes)
 // per frame from the exchange ring), 1, 2 or 4 tiles of 16 values of k per workgroup (more tiles: fewer workgroups, more
 // MFMA time each) and 4 or 8 wavefronts per workgroup.  Leaves out->kernel null where no candidate fits.
 int choose_bwd_kernel(const BwdCtx& x, BwdChoice* out) {
-  const int n = x.n, B = x.B, dtype = x.dtype, count = x.count;
+  const int n = x.np, B = x.B, dtype = x.dtype, count = x.count;
   int rc = RTN_OK;
   BwdChoice best, turn;  // turn: the candidate that takes most rows per launch, for batches that need several launches
   long long turn_rows = 0;
@@ -2101,8 +2025,6 @@ int choose_bwd_kernel(const BwdCtx& x, BwdChoice* out) {
 int bwd_prepare_jobs(const BwdCtx& x, const BwdChoice& ch, const BwdLayout& lay, void* workspace, size_t stride, std::vector<BwdJob>* jobs) {
   const int n = x.n, B = x.B;
   const int64_t T = x.T;
-  const int bgroups = (B + ch.rows_per_group - 1) / ch.rows_per_group;
-  const dim3 fill_grid(256), fill_block(256);
   int rc = RTN_OK;
   jobs->assign((size_t)x.count, BwdJob());
   for (int k = 0; k < x.count; ++k) {
@@ -2115,13 +2037,11 @@ int bwd_prepare_jobs(const BwdCtx& x, const BwdChoice& ch, const BwdLayout& lay,
     j.ws = (unsigned char*)workspace + (size_t)k * stride;
     p.dyw = (float*)(j.ws + lay.off_dyw);
     p.dx0 = j.ws + lay.off_dx0;
-    p.T = T; p.B = B; p.n = n;
+    p.T = T; p.B = B; p.n = x.np; p.nc = n;
     p.op_flags = x.op_flags;
     if ((rc = resolve_pitch("ldY", c.ldY, n, B, x.es, &j.ldY)) != RTN_OK) return rc;
     if ((rc = resolve_pitch("ldDY", c.ldDY, n, B, x.es, &p.ldDY)) != RTN_OK) return rc;
     if ((rc = resolve_pitch("ldDX", c.ldDX, 4LL * n, B, x.es, &p.ldDX)) != RTN_OK) return rc;
-    hipLaunchKernelGGL(k_fill_u32, fill_grid, fill_block, 0, x.stream, (unsigned*)j.ws, 0u, (long long)(lay.off_wpk / 4));
-    RTN_HIP(hipGetLastError());
     j.abs_step = c.step > 0 ? c.step : -(long long)c.step;
     j.num_steps = (T - c.start + j.abs_step - 1) / j.abs_step;
     j.first = c.step > 0 ? c.start : T - c.start - 1;
@@ -2131,16 +2051,12 @@ int bwd_prepare_jobs(const BwdCtx& x, const BwdChoice& ch, const BwdLayout& lay,
       j.num_steps = (j.first - c.start) / j.abs_step + 1;
     }
     j.end = j.first + (j.num_steps - 1) * c.step;  // inclusive
-    if (ch.kernel) {
-      // the exchange ring starts armed: all-ones words (the visited frames of DX are written by the kernel, the others
-      // zeroed behind it)
-      const int bp = ch.rows_per_group > 8 ? 16 : 8;
-      const long long ring_words = (long long)((size_t)bgroups * kExRing * 4 * n * x.es * bp / 4);
-      if ((size_t)ring_words * 4 > lay.total - lay.off_ex)
-        return fail(RTN_ERR_WORKSPACE, "NativeLstm2 backward: internal: exchange ring of %lld bytes does not fit its section", ring_words * 4);
-      hipLaunchKernelGGL(k_fill_u32, dim3(256), fill_block, 0, x.stream, (unsigned*)(j.ws + lay.off_ex), 0xFFFFFFFFu, ring_words);
-      RTN_HIP(hipGetLastError());
-    } else if (j.num_steps != T) {
+    if (ch.kernel) continue;
+    // launches per frame: status, working copies of the errors and dx0 start at 0, the cell error at Dd
+    hipLaunchKernelGGL(k_fill_u32, dim3(256), dim3(256), 0, x.stream, (unsigned*)j.ws, 0u, (long long)(lay.off_wpk / 4));
+    hipLaunchKernelGGL(k_copy_f32, dim3(256), dim3(256), 0, x.stream, c.Dd, c.Dc0, x.bn);
+    RTN_HIP(hipGetLastError());
+    if (j.num_steps != T) {
       // frames the loop does not visit keep DX = 0 (:1385-1388): all rows cleared here, row by row
       if ((rc = launch_clear_rows(c.DX, (long long)T * B, 4LL * n, p.ldDX, x.es, x.stream)) != RTN_OK) return rc;
     }
@@ -2151,12 +2067,19 @@ int bwd_prepare_jobs(const BwdCtx& x, const BwdChoice& ch, const BwdLayout& lay,
 // The recurrence of all problems on the persistent kernel: one launch per share of the batch groups (a single one unless
 // the batch is too large for the device), then DX := 0 on the frames the forward pass did not visit.
 int bwd_launch_persistent(const BwdCtx& x, const BwdChoice& ch, const BwdLayout& lay, const std::vector<BwdJob>& jobs) {
-  const int n = x.n, B = x.B, count = x.count;
+  const int n = x.np, B = x.B, count = x.count;
   const int bgroups = (B + ch.rows_per_group - 1) / ch.rows_per_group;
   const dim3 fill_block(256);
   Lstm2BwdMulti multi;
   memset(&multi, 0, sizeof(multi));
   multi.count = count;
+  Lstm2BwdPrepare prep;
+  memset(&prep, 0, sizeof(prep));
+  // the exchange ring starts armed (the visited frames of DX are written by the kernel, the others zeroed behind it)
+  prep.ring_words = (long long)((size_t)bgroups * kExRing * 4 * n * x.es * (ch.rows_per_group > 8 ? 16 : 8) / 4);
+  prep.n_words = (long long)(lay.off_dyw / 4);  // status and the words of the XCD check
+  if ((size_t)prep.ring_words * 4 > lay.total - lay.off_ex)
+    return fail(RTN_ERR_WORKSPACE, "NativeLstm2 backward: internal: exchange ring of %lld bytes does not fit its section", prep.ring_words * 4);
   for (int k = 0; k < count; ++k) {
     Lstm2BwdPersistent& q = multi.q[k];
     const BwdJob& j = jobs[(size_t)k];
@@ -2187,6 +2110,22 @@ int bwd_launch_persistent(const BwdCtx& x, const BwdChoice& ch, const BwdLayout&
     q.ex = j.ws + lay.off_ex;
     q.Bp = ch.rows_per_group > 8 ? 16 : 8;
     q.bp_shift = ch.rows_per_group > 8 ? 4 : 3;
+    prep.words[k] = (unsigned*)j.ws;
+    prep.ring[k] = (unsigned*)(j.ws + lay.off_ex);
+    if (x.np != x.n) {
+      prep.w_from[k] = j.p.W;
+      prep.w_pad[k] = j.ws + lay.off_wpk;
+      q.p.W = prep.w_pad[k];
+    }
+  }
+  {
+    const long long work = std::max<long long>(prep.ring_words / 4, x.np != x.n ? (long long)n * n * 4 * (long long)x.es / 16 : 0);
+    const dim3 grid((unsigned)std::min<long long>((work + 255) / 256, 1024), (unsigned)count);
+    if (x.dtype == RTN_DTYPE_BF16)
+      hipLaunchKernelGGL(k_bwd_prepare<__bf16>, grid, fill_block, 0, x.stream, prep, n, x.n);
+    else
+      hipLaunchKernelGGL(k_bwd_prepare<float>, grid, fill_block, 0, x.stream, prep, n, x.n);
+    RTN_HIP(hipGetLastError());
   }
   multi.local = ch.local ? 1 : 0;
   multi.xcds = device_info().xcds;
@@ -2211,7 +2150,7 @@ int bwd_launch_persistent(const BwdCtx& x, const BwdChoice& ch, const BwdLayout&
   for (int k = 0; k < count; ++k) {
     const BwdJob& j = jobs[(size_t)k];
     if (j.num_steps == x.T) continue;
-    const long long row_words = (long long)((size_t)n * 4 * x.es / 4), pitch_words = (long long)((size_t)j.p.ldDX * x.es / 4);
+    const long long row_words = (long long)((size_t)x.n * 4 * x.es / 4), pitch_words = (long long)((size_t)j.p.ldDX * x.es / 4);
     if (x.dtype == RTN_DTYPE_BF16)
       hipLaunchKernelGGL(k_bwd_zero_unvisited<__bf16>, dim3(1024), fill_block, 0, x.stream, x.calls[k].DX, (long long)x.T, (long long)B, row_words,
                          pitch_words, j.first, (long long)x.calls[k].step, j.num_steps);
@@ -2308,18 +2247,18 @@ int bwd_weight_gradients(const BwdCtx& x, rocblas_handle blas, const std::vector
     if (j.num_steps > 1) {
       if (j.abs_step == 1) {
         const long long lo = std::min(j.first, j.end);
-        rc = dw_accumulate(blas, Yb + (size_t)(lo + std::max(0, -step)) * B * j.ldY * x.es,
-                           DXb + (size_t)(lo + std::max(0, step)) * B * j.p.ldDX * x.es, c.DW, (j.num_steps - 1) * B, n, x.dtype, j.ldY, j.p.ldDX);
+        rc = dw_product(blas, Yb + (size_t)(lo + std::max(0, -step)) * B * j.ldY * x.es,
+                           DXb + (size_t)(lo + std::max(0, step)) * B * j.p.ldDX * x.es, 0.f, c.DW, (j.num_steps - 1) * B, n, x.dtype, j.ldY, j.p.ldDX);
         if (rc != RTN_OK) return rc;
       } else {
         for (long long t = j.end - step; step > 0 ? t >= j.first : t <= j.first; t -= step) {
-          rc = dw_accumulate(blas, Yb + (size_t)t * B * j.ldY * x.es, DXb + (size_t)(t + step) * B * j.p.ldDX * x.es, c.DW, B, n, x.dtype, j.ldY,
+          rc = dw_product(blas, Yb + (size_t)t * B * j.ldY * x.es, DXb + (size_t)(t + step) * B * j.p.ldDX * x.es, t == j.end - step ? 0.f : 1.f, c.DW, B, n, x.dtype, j.ldY,
                              j.p.ldDX);
           if (rc != RTN_OK) return rc;
         }
       }
     }
-    rc = dw_accumulate(blas, c.y0, j.p.dx0, c.DW, B, n, x.dtype);
+    rc = dw_product(blas, c.y0, j.p.dx0, j.num_steps > 1 ? 1.f : 0.f, c.DW, B, n, x.dtype);
     if (rc != RTN_OK) return rc;
     if (!persistent) {
       if (x.dtype == RTN_DTYPE_BF16)
@@ -2341,7 +2280,7 @@ int bwd_calls(const rtn_lstm2_bwd_call* calls, int count, int64_t T, int32_t B, 
   if (rc != RTN_OK) return rc;
   if (count < 0 || (count > 0 && !calls)) return fail(RTN_ERR_ARG, "NativeLstm2 backward: bad call list");
   BwdCtx x;
-  x.calls = calls; x.count = count; x.T = T; x.B = B; x.n = n; x.dtype = dtype; x.op_flags = op_flags;
+  x.calls = calls; x.count = count; x.T = T; x.B = B; x.n = n; x.np = padded_width(n); x.dtype = dtype; x.op_flags = op_flags;
   x.stream = (hipStream_t)hip_stream;
   x.es = esize(dtype);
   x.bn = (long long)B * n;
@@ -2353,13 +2292,16 @@ int bwd_calls(const rtn_lstm2_bwd_call* calls, int count, int64_t T, int32_t B, 
   // first use).
   x.capturing = cap_status != hipStreamCaptureStatusNone;
   if (!x.capturing && T > 0 && x.bn > 0 && (rc = probe_xcds(x.stream)) != RTN_OK) return rc;
-  if ((rc = bwd_check_and_clear(x)) != RTN_OK) return rc;
+  if ((rc = bwd_check(x)) != RTN_OK) return rc;
   if (T == 0 || x.bn == 0 || count == 0) return RTN_OK;
-  const int np = padded_width(n);
-  if (np != n) return bwd_padded(x, np, workspace, workspace_bytes);
+  // A width that the kernels take padded: the persistent kernel pads on the fly as long as rows stay 16-byte aligned
+  // (below); everything else runs on padded copies.
+  const int np = x.np;
+  if (np != n && n % (int)(16 / x.es) != 0) return bwd_padded(x, np, workspace, workspace_bytes);
 
-  const BwdLayout lay = bwd_layout(B, n, dtype);
-  const size_t stride = ws_stride ? ws_stride : lay.total;  // distance between the calls' workspaces
+  const BwdLayout lay = bwd_layout(B, np, dtype);
+  // distance between the calls' workspaces
+  const size_t stride = ws_stride ? ws_stride : rtn_native_lstm2_bwd_workspace_bytes(T, B, n, dtype);
   if (stride < lay.total) return fail(RTN_ERR_WORKSPACE, "NativeLstm2 backward: internal: workspace slice %zu < layout %zu", stride, lay.total);
   if (!workspace || workspace_bytes < stride * (size_t)(count - 1) + lay.total)
     return fail(RTN_ERR_WORKSPACE, "NativeLstm2 backward: workspace of %zu bytes needed, got %zu", stride * (size_t)(count - 1) + lay.total,
@@ -2369,13 +2311,14 @@ int bwd_calls(const rtn_lstm2_bwd_call* calls, int count, int64_t T, int32_t B, 
   rc = blas_handle(&blas);
   if (rc != RTN_OK) return rc;
   if (rocblas_set_stream(blas, x.stream) != rocblas_status_success) return fail(RTN_ERR_HIP, "NativeLstm2 backward: rocblas_set_stream failed");
-  const bool mfma = (n % 16) == 0 && !env_long("RTN_LSTM2_FORCE_GENERIC", 0);
+  const bool mfma = (np % 16) == 0 && !env_long("RTN_LSTM2_FORCE_GENERIC", 0);
 
   BwdChoice ch;
   const long bwd_kernel = env_long("RTN_LSTM2_BWD_KERNEL", 0);  // 0 auto, 1 per-frame launches, 2 persistent
   const int KM = dtype == RTN_DTYPE_BF16 ? 32 : 16;
-  if (mfma && (4 * n) % KM == 0 && bwd_kernel != 1 && (!x.capturing || capture_keeps_persistent()) && device_info().cooperative && count <= kMaxBwdMulti)
+  if (mfma && (4 * np) % KM == 0 && bwd_kernel != 1 && (!x.capturing || capture_keeps_persistent()) && device_info().cooperative && count <= kMaxBwdMulti)
     if ((rc = choose_bwd_kernel(x, &ch)) != RTN_OK) return rc;
+  if (!ch.kernel && np != n) return bwd_padded(x, np, workspace, workspace_bytes);
   if (!ch.kernel && count > 1) {
     // no joint launch: one call after the other, each with its own slice of the workspace
     for (int k = 0; k < count; ++k) {
@@ -2391,7 +2334,7 @@ int bwd_calls(const rtn_lstm2_bwd_call* calls, int count, int64_t T, int32_t B, 
     char buf[256];
     if (ch.kernel)
       snprintf(buf, sizeof(buf), "kernel=%s problems=%d rows_per_group=%d groups=%d tiles=%d waves=%d wgs_per_group=%d launches=%d",
-               ch.local ? "bwd_regw_xcd" : "bwd_regw", count, ch.rows_per_group, bgroups, ch.tiles, ch.waves, n / (16 * ch.tiles),
+               ch.local ? "bwd_regw_xcd" : "bwd_regw", count, ch.rows_per_group, bgroups, ch.tiles, ch.waves, np / (16 * ch.tiles),
                (bgroups + ch.groups_per_launch - 1) / std::max(ch.groups_per_launch, 1));
     else
       snprintf(buf, sizeof(buf), "kernel=%s problems=%d launches_per_frame=%d", mfma ? "bwd_step" : "bwd_generic", count, mfma ? 1 : 2);

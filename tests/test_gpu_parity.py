@@ -716,3 +716,51 @@ def test_forward_recorded_into_a_callers_graph(T, B, n, dtype):
             assert torch.equal(a, b), (k, name)
         want = oracle.native_lstm2_fwd(*problems[k], 0, 1)
         (check_f32 if dtype == "f32" else check_bf16)([t.float().cpu().numpy() for t in got], want[:4], "captured replay %i" % k)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("n", [33, 41, 63, 65, 116, 127, 524])
+def test_widths_that_cut_a_chunk(n, dtype):
+    """Widths whose last 16-byte piece of a row is cut (by 1 ... 7 cells) or whole: every element of the outputs is written,
+    nothing beyond them is, X and Y with a row pitch included, forwards and backwards in time, with and without frames that
+    are not visited."""
+    from returnn_amd import lib
+    from _gpu_util import to_dev
+
+    announce("cut chunk", n, dtype)
+    get_op()
+    cabi = lib.load()
+    T, B = 6, 5
+    act = torch.bfloat16 if dtype == "bf16" else torch.float32
+    dt = lib.DTYPE_BF16 if dtype == "bf16" else lib.DTYPE_F32
+    X, W, y0, c0, i = random_problem(400 + n, T, B, n)
+    Xd, Wd, y0d = (to_dev(a, dtype) for a in (X, W, y0))
+    c0d, id_ = (to_dev(a, "f32") for a in (c0, i))
+    stream = torch.cuda.current_stream().cuda_stream
+    for start, step, pad in [(0, 1, 0), (0, -1, 8), (1, 2, 0)]:
+        f = lambda t: t.float().cpu().numpy()  # noqa: E731
+        want = oracle.native_lstm2_fwd(f(Xd), f(Wd), f(y0d), c0, i, start, step)
+        Xp = torch.full((T, B, 4 * n + pad), 7.0, dtype=act, device="cuda:0")
+        Xp[:, :, : 4 * n] = Xd
+        guard = lambda shape, t: torch.full((int(numpy.prod(shape)) + 64,), float("nan"), dtype=t, device="cuda:0")  # noqa: E731
+        shapes = {"Y": ((T, B, n + pad), act), "C": ((T, B, n), torch.float32), "H": ((T, B, 4 * n), act), "d": ((B, n), torch.float32)}
+        bufs = {k: guard(sh, t) for k, (sh, t) in shapes.items()}
+        ws = torch.empty((lib.workspace_bytes(T, B, n, dt, lib.MODE_AUTO),), dtype=torch.uint8, device="cuda:0")
+        arr = (lib.Lstm2Call * 1)(lib.Lstm2Call(
+            Xp.data_ptr(), Wd.data_ptr(), y0d.data_ptr(), c0d.data_ptr(), id_.data_ptr(), start, step, bufs["Y"].data_ptr(), bufs["C"].data_ptr(),
+            bufs["H"].data_ptr(), bufs["d"].data_ptr(), 4 * n + pad, n + pad))  # fmt: skip
+        rc = cabi.rtn_native_lstm2_fwd_multi(arr, 1, T, B, n, dt, lib.MODE_AUTO, ws.data_ptr(), ws.numel(), stream)
+        if (4 * n + pad) % (16 // Xd.element_size()) and pad and rc == lib.RTN_ERR_ARG:
+            continue  # (a pitch that the entry refuses)
+        lib.check(rc)
+        torch.cuda.synchronize()
+        got = []
+        for k, (sh, _) in shapes.items():
+            m = int(numpy.prod(sh))
+            assert torch.isnan(bufs[k][m:]).all(), "%s: written beyond its end" % k
+            a = bufs[k][:m].view(sh)
+            if k == "Y" and pad:
+                assert torch.isnan(a[:, :, n:]).all(), "Y: written between its rows"
+                a = a[:, :, :n]
+            got.append(f(a))
+        (check_f32 if dtype == "f32" else check_bf16)(got, want[:4], "cut chunk %s" % ((n, start, step, pad),))
