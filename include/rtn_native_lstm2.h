@@ -160,6 +160,9 @@ typedef struct rtn_lstm2_call {
    * outputs into one [T, B, 2n] array (Y = base + 0 and base + n, ldY = 2n).  Rows must stay 16-byte aligned. */
   int64_t ldX;
   int64_t ldY;
+  /* Optional (null: not wanted): [B,n] takes each sequence's final output, what rtn_native_lstm2_last_output gives for a
+   * mask of zeros and ones -- the output carried over masked frames, y0 for a sequence without a valid frame. */
+  void* hN;
 } rtn_lstm2_call;
 
 int rtn_native_lstm2_fwd_multi(const rtn_lstm2_call* calls, int32_t count, int64_t T, int32_t B, int32_t n,
@@ -357,6 +360,28 @@ size_t rtn_lstm_low_mem_bwd_workspace_bytes(int64_t T, int32_t B, int32_t n_in, 
 int rtn_native_lstm2_last_output(const void* Y, const void* y0, const float* i, int32_t start, int32_t step,
                                  void* out, int64_t T, int32_t B, int32_t n, int32_t dtype, int64_t ldY, void* hip_stream);
 
+/* lengths [B] -> mask [T,B]: 1 for the frames t < lengths[b], else 0 (returnn/torch/util/array_.py:196-208). */
+int rtn_sequence_mask(const int64_t* lengths, float* mask, int64_t T, int32_t B, void* hip_stream);
+
+/*
+ * One step of an LSTM layer with its input projection (a recurrent decoder's call, once per output label; what
+ * returnn/frontend/rec.py:16-77 computes with single_step_dim): gates = bias + ff . x + rec^T . h,
+ * c_out = sigmoid(f) c + sigmoid(i) tanh(g), y = h_out = tanh(c_out) sigmoid(o).
+ * x [B,in], h [B,n], ff [4n,in], rec [n,4n], bias [4n] (or null), y and h_out [B,n] in element type `dtype`; c, c_out
+ * [B,n] float32; gate blocks in the op's order cell-in, input, forget, output.  Any widths and element alignment; one
+ * launch, no workspace.  y and h_out may be the same array; no output may overlap an input.
+ */
+int rtn_lstm_step(const void* x, const void* h, const float* c, const void* ff, const void* rec, const void* bias, void* y, void* h_out,
+                  float* c_out, int32_t B, int32_t in_dim, int32_t n, int32_t dtype, void* hip_stream);
+
+/*
+ * Where the calling thread's calls report an expired bounded wait, besides the status word of their workspace: a kernel
+ * whose wait expires stores `id` into *word (a 32-bit word the device can write, e.g. of pinned host memory; null, the
+ * initial setting: nowhere).  Holds for all later calls of this thread.  The word has to stay valid until their kernels
+ * have ended.  (What lets a caller notice without a copy or an event per call; no counterpart in the reference.)
+ */
+void rtn_set_abort_word(void* word, uint32_t id);
+
 /* Text of the calling thread's last error ("" if none).  Stands in for the message of the
  * exception TORCH_CHECK raises (returnn/native_op.cpp:660). */
 const char* rtn_last_error(void);
@@ -404,7 +429,7 @@ const char* rtn_native_lstm2_bwd_plan_text(void);
  */
 void rtn_native_lstm2_reload_env(void);
 
-/* ABI version of this header: 13. */
+/* ABI version of this header: 14. */
 int rtn_native_lstm2_abi_version(void);
 
 #ifdef __cplusplus

@@ -22,8 +22,11 @@ HOST_SOURCE = "rtn_native_lstm2.hip"
 TABLES_SOURCE = "lstm2_kernel_tables.hip"  # compiled once per part: the instantiations of the persistent kernels
 TABLE_PARTS = 8
 SOURCES = [HOST_SOURCE, TABLES_SOURCE]
-HEADERS = ["lstm2_kernels.h", "lstm2_bwd_kernels.h", "lstm2_params.h", "lstm2_kernel_tables.h",
+HEADERS = ["lstm2_kernels.h", "lstm2_step_kernel.h", "lstm2_bwd_kernels.h", "lstm2_params.h", "lstm2_kernel_tables.h",
            os.path.join("..", "..", "include", "rtn_native_lstm2.h")]  # fmt: skip
+# the torch side of the calls (host code only)
+BINDING_SOURCE = "rtn_torch_binding.cpp"
+BINDING_PATH = os.path.join(_dir, "_rtn_torch.so")
 OBJ_DIR = os.path.join(CSRC_DIR, "_obj")
 OFFLOAD_ARCH = "gfx950"
 ROCM_LIB_DIR = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "lib")  # rocBLAS (weight-gradient GEMM of the backward op)
@@ -75,11 +78,27 @@ def link_command(output: Optional[str] = None, obj_dir: Optional[str] = None) ->
     ]  # fmt: skip
 
 
+def binding_command(output: Optional[str] = None) -> List[str]:
+    """The g++ line of the torch binding: against the torch and HIP headers, no device code.  The HIP runtime is the one
+    torch has loaded by then."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    cmd = [os.environ.get("CXX") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-Wno-unknown-pragmas", "-Wno-attributes"]
+    cmd += ["-D_GLIBCXX_USE_CXX11_ABI=%i" % int(torch._C._GLIBCXX_USE_CXX11_ABI), "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-DTORCH_EXTENSION_NAME=_rtn_torch"]
+    cmd += ["-isystem" + d for d in cpp_extension.include_paths("cuda") + [sysconfig.get_paths()["include"]] if os.path.isdir(d)]
+    cmd += [os.path.join(CSRC_DIR, BINDING_SOURCE), "-o", output or BINDING_PATH, "-L" + torch_lib, "-L" + ROCM_LIB_DIR]
+    return cmd + ["-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch", "-ltorch_python", "-lamdhip64"]
+
+
 def needs_build() -> bool:
-    if not os.path.exists(LIB_PATH):
+    if not os.path.exists(LIB_PATH) or not os.path.exists(BINDING_PATH):
         return True
-    t = os.path.getmtime(LIB_PATH)
-    deps = [os.path.join(CSRC_DIR, f) for f in SOURCES + HEADERS] + [os.path.abspath(__file__)]
+    t = min(os.path.getmtime(LIB_PATH), os.path.getmtime(BINDING_PATH))
+    deps = [os.path.join(CSRC_DIR, f) for f in SOURCES + HEADERS + [BINDING_SOURCE]] + [os.path.abspath(__file__)]
     return any(os.path.getmtime(d) > t for d in deps if os.path.exists(d))
 
 
@@ -106,6 +125,7 @@ def build_library(force: bool = True, verbose: bool = False) -> str:
     obj_dir = OBJ_DIR + ".tmp.%i" % os.getpid()
     os.makedirs(obj_dir, exist_ok=True)
     tmp = LIB_PATH + ".tmp.%i" % os.getpid()
+    tmp_binding = BINDING_PATH + ".tmp.%i" % os.getpid()
 
     def run(cmd):
         if verbose:
@@ -115,18 +135,20 @@ def build_library(force: bool = True, verbose: bool = False) -> str:
 
     try:
         with ThreadPoolExecutor(max_workers=_jobs()) as pool:
-            results = list(pool.map(run, compile_commands(obj_dir)))
+            results = list(pool.map(run, [binding_command(tmp_binding)] + compile_commands(obj_dir)))
         results.append(run(link_command(tmp, obj_dir)) if all(rc == 0 for _, rc, _ in results) else (["(link skipped)"], 0, ""))
         for cmd, rc, out in results:
             if rc != 0:
-                raise RuntimeError("hipcc failed (%i):\n$ %s\n%s" % (rc, " ".join(cmd), out))
+                raise RuntimeError("the compiler failed (%i):\n$ %s\n%s" % (rc, " ".join(cmd), out))
             if verbose and out.strip():
                 print(out, file=sys.stderr)
         os.replace(tmp, LIB_PATH)
+        os.replace(tmp_binding, BINDING_PATH)
     finally:
         shutil.rmtree(obj_dir, ignore_errors=True)
-        if os.path.exists(tmp):
-            os.remove(tmp)
+        for left in (tmp, tmp_binding):
+            if os.path.exists(left):
+                os.remove(left)
     return LIB_PATH
 
 

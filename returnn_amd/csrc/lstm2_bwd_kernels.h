@@ -768,6 +768,7 @@ __global__ __launch_bounds__(64 * WV) void k_lstm2_bwd_regw(const Lstm2BwdMulti 
   // After a wait that ran into its bound the gradients are wrong without looking it: the workgroups that see the mark
   // hand out NaN, so that a caller who never asks for the status still finds a non-finite gradient.
   const bool expired = wait_expired(q.status);
+  if (expired && tid == 0) report_expired(q.status);
   const float nan = __builtin_nanf("");
 #pragma unroll
   for (int j = 0; j < PT; ++j) {
@@ -788,12 +789,14 @@ struct Lstm2BwdPrepare {
   void* w_pad[kMaxBwdMulti];  // null: nothing to pad
   unsigned *words[kMaxBwdMulti], *ring[kMaxBwdMulti];
   long long n_words, ring_words;
+  unsigned long long abort_word;  // see StatusWords
+  unsigned abort_id;
 };
 template <typename AT>
 __global__ void k_bwd_prepare(Lstm2BwdPrepare a, int n, int nc) {
   const int k = blockIdx.y;
   const long long gtid = blockIdx.x * (long long)blockDim.x + threadIdx.x, gsz = (long long)gridDim.x * blockDim.x;
-  for (long long i = gtid; i < a.n_words; i += gsz) a.words[k][i] = 0u;
+  for (long long i = gtid; i < a.n_words; i += gsz) a.words[k][i] = status_word((int)min(i, 63LL), a.abort_word, a.abort_id);
   for (long long i = gtid; i < a.ring_words / 4; i += gsz) ((i32x4*)a.ring[k])[i] = i32x4{-1, -1, -1, -1};
   if (a.w_pad[k]) {
     constexpr int PE = 16 / (int)sizeof(AT);  // nc is a multiple of PE here

@@ -104,6 +104,17 @@ struct Act<__bf16> {
 __device__ __forceinline__ bool wait_expired(const unsigned* status) {
   return __hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 1u;
 }
+// By a kernel that ends with an expired wait behind it (one thread of a workgroup): the call's number into the word its
+// caller looks at (see StatusWords).  At the end and not in the waits: those sit in the steps' critical path, where the few
+// instructions more cost a single sequence 3 %.
+__device__ __forceinline__ void report_expired(const unsigned* status) {
+  const unsigned long long word = ((unsigned long long)status[kStatusAbortWord + 1] << 32) | status[kStatusAbortWord];
+  if (word) __hip_atomic_store((unsigned*)word, status[kStatusAbortId], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+// What word i of a call's status block holds when the call starts.
+__device__ __forceinline__ unsigned status_word(int i, unsigned long long abort_word, unsigned abort_id) {
+  return i == kStatusAbortWord ? (unsigned)abort_word : i == kStatusAbortWord + 1 ? (unsigned)(abort_word >> 32) : i == kStatusAbortId ? abort_id : 0u;
+}
 // A 32-bit word full of quiet NaNs of the activation type.
 template <typename AT>
 inline constexpr unsigned kNanWords = 0x7FC00000u;
@@ -169,7 +180,7 @@ __device__ __forceinline__ void prepare_mfma(const Lstm2Params& p, int n_flags) 
   constexpr int KM = Elem<AT>::KM;
   const long long gtid = blockIdx.x * (long long)blockDim.x + threadIdx.x;
   const long long gsz = (long long)gridDim.x * blockDim.x;
-  for (long long i = gtid; i < 64; i += gsz) p.status[i] = 0;
+  for (long long i = gtid; i < 64; i += gsz) p.status[i] = status_word((int)i, p.abort_word, p.abort_id);
   for (long long i = gtid; i < n_flags; i += gsz) p.flags[i] = 0;
   // y0 -> hx[g][0][kb][b_local][e]
   const long long bn = (long long)p.B * p.n;
@@ -295,6 +306,12 @@ __global__ void k_add_bias(void* data, const void* bias, long long count, int wi
     Elem<AT>::store(data, i, Elem<AT>::load(data, i) + Elem<AT>::load(bias, i % width));
 }
 
+// [B] lengths -> [T,B] mask of ones and zeros
+static __global__ void k_sequence_mask(const long long* lengths, float* mask, long long total, int B) {
+  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < total; i += (long long)gridDim.x * blockDim.x)
+    mask[i] = i / B < lengths[i % B] ? 1.f : 0.f;
+}
+
 static __global__ void k_clear_status(unsigned* status) {
   if (threadIdx.x < 64) status[threadIdx.x] = 0;
 }
@@ -363,8 +380,12 @@ __global__ void k_step_generic(Lstm2Params p, int s) {
   p.C[t * bn + idx] = c;
   const float y = Elem<AT>::round(Act<AT>::tanh(c) * a3 * m);
   Elem<AT>::store(p.Y, ((size_t)t * p.B + b) * (size_t)p.ldY + j, y);
-  Elem<AT>::store(y_out, idx, (p.op_flags & kOpNoCarry) ? y : y + Elem<AT>::load(y_in, idx) * (1.f - m));
-  if (s == p.nsteps - 1) p.d[idx] = c;
+  const float carried = (p.op_flags & kOpNoCarry) ? y : y + Elem<AT>::load(y_in, idx) * (1.f - m);
+  Elem<AT>::store(y_out, idx, carried);
+  if (s == p.nsteps - 1) {
+    p.d[idx] = c;
+    if (p.hN) Elem<AT>::store(p.hN, idx, carried);
+  }
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -629,12 +650,14 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_mfma(const Lstm2Params p, 
   if (s_end == p.nsteps) {
     // after a wait that ran into its bound: NaN as the final cell state and in the last visited frame of Y
     const bool expired = wait_expired(p.status);
+    if (expired && tid == 0) report_expired(p.status);
     const long long t_last = frame_of(p, p.nsteps - 1);
 #pragma unroll
     for (int j = 0; j < EPT; ++j) {
       if (e_valid[j]) {
         const long long bc = (long long)(b_base + e_b[j]) * nc + e_cell[j];
         p.d[bc] = expired ? __builtin_nanf("") : c_state[j];
+        if (p.hN) E::store(p.hN, bc, expired ? __builtin_nanf("") : h_prev[j]);
         if (expired) E::store(p.Y, ((size_t)t_last * p.B + (b_base + e_b[j])) * (size_t)p.ldY + e_cell[j], __builtin_nanf(""));
       }
     }
@@ -1510,6 +1533,7 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_regw(const Lstm2Multi mult
   // NaN as the final cell state and as the last visited frame of Y.
   const bool expired = wait_expired(p.status);
   if (expired) {
+    if (tid == 0) report_expired(p.status);
 #pragma unroll
     for (int i = 0; i < YCH; ++i) fy[i] = YC::fill(kNanWords<AT>);
   }
@@ -1517,7 +1541,11 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_regw(const Lstm2Multi mult
 
 #pragma unroll
   for (int j = 0; j < EPT; ++j)
-    if (e_valid[j]) p.d[(long long)(b_base + e_row[j]) * nc + 4 * MT * r + e_cl[j]] = expired ? __builtin_nanf("") : c_state[j];
+    if (e_valid[j]) {
+      const long long bc = (long long)(b_base + e_row[j]) * nc + 4 * MT * r + e_cl[j];
+      p.d[bc] = expired ? __builtin_nanf("") : c_state[j];
+      if (p.hN) E::store(p.hN, bc, expired ? __builtin_nanf("") : h_prev[j]);
+    }
 }
 
 

@@ -26,6 +26,14 @@ enum OpFlags : int {
                      // not down to frame 0 (LstmLowMem's loop bounds, returnn/native_op.py:827-833)
 };
 
+// The words of a call's status block that mean something.
+enum StatusWords {
+  kStatusExpired = 0,   // 1: a bounded wait expired (2: a measurement run)
+  kStatusXcds = 1,      // the XCDs of a group that was planned for one and found on several
+  kStatusAbortWord = 8, // 8, 9: address of a word that takes the call's number when a wait expires (pinned host memory; 0: none)
+  kStatusAbortId = 10,  // that number
+};
+
 struct Lstm2Params {
   // inputs (device)
   const void* X;      // [T,B,4n] AT
@@ -38,8 +46,9 @@ struct Lstm2Params {
   float* C;  // [T,B,n]
   void* H;   // [T,B,4n] AT
   float* d;  // [B,n]
+  void* hN;  // [B,n] AT, or null: the output carried behind the last step
   // workspace sections (device)
-  unsigned* status;  // [64]   status[0] != 0: a bounded wait expired
+  unsigned* status;  // [64]   see StatusWords
   unsigned* flags;   // [groups_total*wgs_per_group] last published step (+1) of each workgroup
   void* hx;          // [groups_total][hx_bufs][n/KE][Bp][KE] AT: hidden state in MFMA B-operand order, ring of buffers
   void* Wp;          // [n/4][S][64][16 bytes]: W in MFMA A-operand order
@@ -74,6 +83,8 @@ struct Lstm2Params {
   int zero;           // always 0; an operand the compiler cannot fold (idempotent atomics used as L2 reads)
   int sync_policy;    // SyncBits
   unsigned long long timeout_ticks;  // bound of one flag wait, in 100 MHz wall-clock ticks
+  unsigned long long abort_word;     // for the status block
+  unsigned abort_id;
 };
 
 // Several independent problems of one shape in one launch of the persistent register kernel: workgroups

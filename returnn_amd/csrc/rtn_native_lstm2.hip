@@ -28,6 +28,7 @@
 #include "lstm2_bwd_kernels.h"
 #include "lstm2_kernel_tables.h"
 #include "lstm2_kernels.h"
+#include "lstm2_step_kernel.h"
 
 // Scratch memory of rtn_native_lstm2_fwd_static, the entry point for callers that cannot allocate: a fixed array in the
 // code object, one copy per GPU the library runs on, held until the process ends.  Host code never uses this name as an
@@ -41,6 +42,8 @@ namespace {
 
 thread_local std::string g_last_error;
 thread_local std::string g_plan_text;
+thread_local void* t_abort_word = nullptr;  // where this thread's calls report an expired wait, and as which number
+thread_local unsigned t_abort_id = 0;
 
 int fail(int code, const char* fmt, ...) {
   char buf[512];
@@ -790,8 +793,11 @@ int launch_steps(const Lstm2Params& p, const Plan& pl, int dtype, hipStream_t st
   return launch_steps(p, pl, dtype, sink);
 }
 
-int launch_steps_graph(const Lstm2Params& p, const Plan& pl, int dtype, hipStream_t stream) {
+int launch_steps_graph(const Lstm2Params& call, const Plan& pl, int dtype, hipStream_t stream) {
   std::string key("fwd");
+  Lstm2Params p = call;
+  p.abort_word = 0;  // (the steps wait for nothing; a number of its own for every call would have every node rewritten)
+  p.abort_id = 0;
   int dev = 0;
   RTN_HIP(hipGetDevice(&dev));
   Lstm2Params shape = p;  // the caller zeroed p before filling it in: padding compares equal
@@ -799,6 +805,7 @@ int launch_steps_graph(const Lstm2Params& p, const Plan& pl, int dtype, hipStrea
   shape.c0 = shape.mask = nullptr;
   shape.Y = shape.H = nullptr;
   shape.C = shape.d = nullptr;
+  shape.hN = nullptr;
   shape.status = shape.flags = nullptr;
   shape.hx = shape.Wp = shape.ycarry = nullptr;
   shape.trace = nullptr;
@@ -1147,7 +1154,7 @@ int fill_fwd_params(const rtn_lstm2_call& c, const Plan& pl, bool persistent, un
   int rc = RTN_OK;
   memset(&p, 0, sizeof(p));
   p.X = c.X; p.W = c.W; p.y0 = c.y0; p.c0 = c.c0; p.mask = c.i;
-  p.Y = c.Y; p.C = c.C; p.H = c.H; p.d = c.d;
+  p.Y = c.Y; p.C = c.C; p.H = c.H; p.d = c.d; p.hN = c.hN;
   p.status = (unsigned*)(ws + pl.off_status);
   p.flags = (unsigned*)(ws + pl.off_flags);
   p.hx = ws + pl.off_hx;
@@ -1193,6 +1200,8 @@ int fill_fwd_params(const rtn_lstm2_call& c, const Plan& pl, bool persistent, un
   if (!((p.sync_policy & (kStoreCoherent | kReleaseFence)) && (p.sync_policy & (kLoadCoherent | kAcquireFence))))
     return fail(RTN_ERR_ARG, "NativeLstm2: RTN_LSTM2_SYNC=%d is not a valid publication policy", p.sync_policy);
   p.timeout_ticks = (unsigned long long)env_long("RTN_LSTM2_TIMEOUT_TICKS", 200000000L);  // 2 s at 100 MHz
+  p.abort_word = (unsigned long long)(uintptr_t)t_abort_word;
+  p.abort_id = t_abort_id;
   return RTN_OK;
 }
 
@@ -1216,6 +1225,7 @@ int fwd_calls(const rtn_lstm2_call* calls, int count, int64_t T, int32_t B, int3
       hipLaunchKernelGGL(k_copy_f32, dim3((unsigned)std::min<long long>((bn + 255) / 256, 1024)), dim3(256), 0, stream,
                          calls[k].c0, calls[k].d, bn);
       RTN_HIP(hipGetLastError());
+      if (calls[k].hN && calls[k].y0 && (rc = launch_pad(calls[k].y0, calls[k].hN, B, B, 1, n, n, esize(dtype), stream)) != RTN_OK) return rc;
     }
     return RTN_OK;
   }
@@ -1528,7 +1538,7 @@ using namespace rtn;
 
 extern "C" {
 
-int rtn_native_lstm2_abi_version(void) { return 13; }
+int rtn_native_lstm2_abi_version(void) { return 14; }
 
 const char* rtn_native_lstm2_bwd_plan_text(void) { return g_bwd_plan_text.c_str(); }
 
@@ -1634,6 +1644,50 @@ int rtn_native_lstm2_fwd_multi(const rtn_lstm2_call* calls, int32_t count, int64
   if (count < 0 || (count > 0 && !calls)) return fail(RTN_ERR_ARG, "NativeLstm2: bad call list (count=%d)", count);
   if (count == 0) return RTN_OK;
   return fwd_calls(calls, count, T, B, n, dtype, mode, workspace, workspace_bytes, hip_stream);
+}
+
+void rtn_set_abort_word(void* word, uint32_t id) {
+  t_abort_word = word;
+  t_abort_id = id;
+}
+
+int rtn_sequence_mask(const int64_t* lengths, float* mask, int64_t T, int32_t B, void* hip_stream) {
+  g_last_error.clear();
+  if (T < 0 || B < 0) return fail(RTN_ERR_SHAPE, "sequence mask: T=%lld, B=%d", (long long)T, B);
+  const long long total = (long long)T * B;
+  if (total == 0) return RTN_OK;
+  if (!lengths || !mask) return fail(RTN_ERR_ARG, "sequence mask: null pointer");
+  hipLaunchKernelGGL(k_sequence_mask, dim3((unsigned)std::min<long long>((total + 255) / 256, 2048)), dim3(256), 0, (hipStream_t)hip_stream,
+                     (const long long*)lengths, mask, total, B);
+  RTN_HIP(hipGetLastError());
+  return RTN_OK;
+}
+
+int rtn_lstm_step(const void* x, const void* h, const float* c, const void* ff, const void* rec, const void* bias, void* y, void* h_out,
+                  float* c_out, int32_t B, int32_t in_dim, int32_t n, int32_t dtype, void* hip_stream) {
+  g_last_error.clear();
+  const int rc = check_dims(1, B, n, dtype);
+  if (rc != RTN_OK) return rc;
+  if (in_dim < 0 || (long long)in_dim * n > 0x7fffffffLL / 16) return fail(RTN_ERR_SHAPE, "LSTM step: bad input dimension %d (n=%d)", in_dim, n);
+  if ((long long)B * n == 0) return RTN_OK;
+  if (!h || !c || !rec || !y || !h_out || !c_out || (in_dim > 0 && (!x || !ff))) return fail(RTN_ERR_ARG, "LSTM step: null pointer");
+  LstmStepParams p = {x, h, c, ff, rec, bias, y, h_out, c_out, B, in_dim, n};
+  // 16, 32 or 64 rows per workgroup, several shares of the batch beyond that (the weights then come from the L2 again)
+  const int NT = B <= 16 ? 1 : (B <= 32 ? 2 : 4);
+  const int blocks = (n + kStepCells - 1) / kStepCells;
+  const dim3 grid((unsigned)((blocks + 7) / 8 * 8), (unsigned)((B + 16 * NT - 1) / (16 * NT))), block(kStepThreads);
+  const hipStream_t stream = (hipStream_t)hip_stream;
+#define RTN_STEP(nt)                                                              \
+  if (NT == nt) {                                                                 \
+    if (dtype == RTN_DTYPE_BF16)                                                  \
+      hipLaunchKernelGGL((k_lstm_step<__bf16, nt>), grid, block, 0, stream, p);   \
+    else                                                                          \
+      hipLaunchKernelGGL((k_lstm_step<float, nt>), grid, block, 0, stream, p);    \
+  }
+  RTN_STEP(1) RTN_STEP(2) RTN_STEP(4)
+#undef RTN_STEP
+  RTN_HIP(hipGetLastError());
+  return RTN_OK;
 }
 
 int rtn_handover_latency_probe(void* workspace, size_t workspace_bytes, int32_t rounds, void* hip_stream) {
@@ -2078,6 +2132,8 @@ int bwd_launch_persistent(const BwdCtx& x, const BwdChoice& ch, const BwdLayout&
   // the exchange ring starts armed (the visited frames of DX are written by the kernel, the others zeroed behind it)
   prep.ring_words = (long long)((size_t)bgroups * kExRing * 4 * n * x.es * (ch.rows_per_group > 8 ? 16 : 8) / 4);
   prep.n_words = (long long)(lay.off_dyw / 4);  // status and the words of the XCD check
+  prep.abort_word = (unsigned long long)(uintptr_t)t_abort_word;
+  prep.abort_id = t_abort_id;
   if ((size_t)prep.ring_words * 4 > lay.total - lay.off_ex)
     return fail(RTN_ERR_WORKSPACE, "NativeLstm2 backward: internal: exchange ring of %lld bytes does not fit its section", prep.ring_words * 4);
   for (int k = 0; k < count; ++k) {

@@ -31,7 +31,7 @@ MODE_PERSISTENT = 1
 MODE_GRAPH = 2
 MODE_STEPWISE = 3
 # The ABI version the structs and argument lists below were written for (rtn_native_lstm2_abi_version()).
-EXPECTED_ABI = 13
+EXPECTED_ABI = 14
 
 MODES = {"auto": MODE_AUTO, "persistent": MODE_PERSISTENT, "graph": MODE_GRAPH, "stepwise": MODE_STEPWISE}
 
@@ -60,6 +60,9 @@ SYMBOLS = (
     "rtn_lstm_low_mem_bwd",
     "rtn_lstm_low_mem_bwd_workspace_bytes",
     "rtn_native_lstm2_last_output",
+    "rtn_lstm_step",
+    "rtn_sequence_mask",
+    "rtn_set_abort_word",
     "rtn_last_error",
     "rtn_native_lstm2_describe_plan",
     "rtn_native_lstm2_describe_multi_plan",
@@ -89,6 +92,7 @@ class Lstm2Call(ctypes.Structure):
         ("d", ctypes.c_void_p),
         ("ldX", ctypes.c_int64),  # row pitch of X in elements, 0 = contiguous (4n)
         ("ldY", ctypes.c_int64),  # row pitch of Y in elements, 0 = contiguous (n)
+        ("hN", ctypes.c_void_p),  # final outputs, or null
     ]
 
 
@@ -204,6 +208,12 @@ def load() -> ctypes.CDLL:
         lib.rtn_handover_latency_probe.argtypes = [vp, sz, i32, vp]
         lib.rtn_native_lstm2_last_output.restype = ctypes.c_int
         lib.rtn_native_lstm2_last_output.argtypes = [vp, vp, vp, i32, i32, vp, i64, i32, i32, i32, i64, vp]
+        lib.rtn_lstm_step.restype = ctypes.c_int
+        lib.rtn_lstm_step.argtypes = [vp] * 9 + [i32, i32, i32, i32, vp]
+        lib.rtn_sequence_mask.restype = ctypes.c_int
+        lib.rtn_sequence_mask.argtypes = [vp, vp, i64, i32, vp]
+        lib.rtn_set_abort_word.restype = None
+        lib.rtn_set_abort_word.argtypes = [vp, ctypes.c_uint32]
         lib.rtn_last_error.restype = ctypes.c_char_p
         lib.rtn_last_error.argtypes = []
         lib.rtn_native_lstm2_describe_plan.restype = ctypes.c_char_p

@@ -35,7 +35,7 @@ from typing import NamedTuple, Optional, Sequence, Tuple, Union
 import torch
 
 from . import native_op
-from .torch_native_op import NativeLstm2BidirFunction, NativeLstm2Function, lstm_last_output, make_op, native_lstm2_multi
+from .torch_native_op import make_op, native
 
 __all__ = [
     "lstm", "blstm", "prepare_weights", "prepare_blstm_weights", "join_weights", "LstmWeights", "BlstmWeights", "LSTM", "BLSTM",
@@ -204,55 +204,33 @@ def lstm(
         raise ValueError("lstm: source has %i features, ff_weight expects %i" % (in_dim, weights.ff.shape[0]))
     if tuple(state_h.shape) != (B, n) or tuple(state_c.shape) != (B, n):
         raise ValueError("lstm: state_h %s / state_c %s, expected %s" % (tuple(state_h.shape), tuple(state_c.shape), (B, n)))
-    device = source.device
-    X = _project(source, weights, act)
-    if seq_lens is None:
-        mask = torch.ones((T, B), dtype=torch.float32, device=device)
-    else:
-        if tuple(seq_lens.shape) != (B,):
-            raise ValueError("lstm: seq_lens must be [B]=[%i], got %s" % (B, tuple(seq_lens.shape)))
-        mask = sequence_mask_time_major(seq_lens.to(device), maxlen=T)
-    if _wants_grad(X, weights.rec, state_h, state_c):
-        _native_lstm2()
-        Y, _C, _H, d = NativeLstm2Function.apply(X, weights.rec, state_h, state_c, mask, 0, direction)
-        h = _last_output_autograd(Y, state_h, seq_lens, direction)
-    else:
-        Y, _C, _H, d = _native_lstm2()(X, weights.rec, state_h, state_c, mask, 0, direction)
-        h = lstm_last_output(Y, state_h, mask, 0, direction) if T > 0 else state_h.to(act)
+    _native_lstm2()  # registers the op and fails loudly without the library
+    if single_step and seq_lens is None and not _wants_grad(source, *weights, state_h, state_c):
+        # one launch: projection, recurrent product and gates
+        y, h, c = native().lstm_step(source[0], state_h, state_c, weights.ff.t(), weights.rec, weights.bias)
+        return y, (h, c)
+    Y, last, cells = native().lstm_layer(
+        source.to(act), weights.ff.to(act), None if weights.bias is None else weights.bias.to(act), _mask(seq_lens, source),
+        [(weights.rec.to(act), state_h, state_c)], direction, T > 0,
+    )  # fmt: skip
+    h = last[0] if T > 0 else state_h.to(act)
     if single_step:
         Y = Y[0]
-    return Y, (h, d)
+    return Y, (h, cells[0])
+
+
+def _mask(seq_lens: Optional[torch.Tensor], source: torch.Tensor) -> torch.Tensor:
+    """[T,B] mask of a time-major ``source``."""
+    T, B = source.shape[:2]
+    if seq_lens is None:
+        return torch.ones((T, B), dtype=torch.float32, device=source.device)
+    if tuple(seq_lens.shape) != (B,):
+        raise ValueError("lstm: seq_lens must be [B]=[%i], got %s" % (B, tuple(seq_lens.shape)))
+    return native().sequence_mask(seq_lens.to(source.device), T)
 
 
 def _wants_grad(*tensors) -> bool:
     return torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors)
-
-
-def _last_output_autograd(Y: torch.Tensor, y0: torch.Tensor, seq_lens: Optional[torch.Tensor], direction: int) -> torch.Tensor:
-    """
-    The final output per sequence with torch indexing, so that gradients flow (the library routine behind
-    :func:`lstm_last_output` has no gradient).  Valid for the right-padded masks this module builds from lengths: the
-    last processed valid frame is ``len-1`` going forward and frame 0 going backward; empty sequences keep ``y0``.
-    """
-    T, B, n = Y.shape
-    if T == 0:
-        return y0.to(Y.dtype)
-    lens = torch.full((B,), T, dtype=torch.int64, device=Y.device) if seq_lens is None else seq_lens.to(Y.device).to(torch.int64).clamp(max=T)
-    if direction > 0:
-        idx = (lens - 1).clamp(min=0)
-        last = Y[idx, torch.arange(B, device=Y.device)]
-    else:
-        last = Y[0]
-    return torch.where((lens > 0)[:, None], last, y0.to(Y.dtype))
-
-
-def _project(source: torch.Tensor, weights: LstmWeights, act: torch.dtype) -> torch.Tensor:
-    """``X = source . ff + bias`` in the op's layout [T,B,4*out]."""
-    T, B, in_dim = source.shape
-    src2 = source.to(act).reshape(T * B, in_dim)
-    ff = weights.ff.to(act)
-    X = torch.addmm(weights.bias.to(act), src2, ff) if weights.bias is not None else torch.mm(src2, ff)
-    return X.view(T, B, ff.shape[1])
 
 
 def blstm(
@@ -264,7 +242,9 @@ def blstm(
     state_fwd: LstmState,
     state_bwd: LstmState,
     seq_lens: Optional[torch.Tensor] = None,
-) -> Tuple[torch.Tensor, LstmState, LstmState]:
+    mask: Optional[torch.Tensor] = None,
+    want_states: bool = True,
+) -> Tuple[torch.Tensor, Optional[LstmState], Optional[LstmState]]:
     """
     Forward-in-time and backward-in-time layer on the same input: ONE projection ``[T*B, 8*out]`` for both directions,
     then both recurrences through the library's multi-call entry (one launch when the device holds both), each reading
@@ -274,6 +254,8 @@ def blstm(
     :param source: [T,B,in]
     :param weights: joint weights (:func:`prepare_blstm_weights`), or ``fwd`` and ``bwd`` prepared one by one (joined here,
         which copies the projection matrices)
+    :param mask: [T,B] float32 mask of ``seq_lens``, if the caller has it already
+    :param want_states: False: the new states are not computed (None in their places)
     :return: [T,B,2*out] (forward | backward), new forward state, new backward state
     """
     if source.dim() != 3:
@@ -292,35 +274,19 @@ def blstm(
     for st in (state_fwd, state_bwd):
         if tuple(st.h.shape) != (B, n) or tuple(st.c.shape) != (B, n):
             raise ValueError("blstm: state %s / %s, expected %s" % (tuple(st.h.shape), tuple(st.c.shape), (B, n)))
-    if seq_lens is None:
-        mask = torch.ones((T, B), dtype=torch.float32, device=source.device)
-    else:
-        if tuple(seq_lens.shape) != (B,):
-            raise ValueError("blstm: seq_lens must be [B]=[%i], got %s" % (B, tuple(seq_lens.shape)))
-        mask = sequence_mask_time_major(seq_lens.to(source.device), maxlen=T)
+    if mask is None:
+        mask = _mask(seq_lens, source)
     _native_lstm2()  # registers the op and fails loudly without the library
-    P = _project(source, LstmWeights(ff=weights.ff, rec=weights.rec_fwd, bias=weights.bias), act)  # [T,B,8n]
-    if _wants_grad(P, weights.rec_fwd, weights.rec_bwd, state_fwd.h, state_fwd.c, state_bwd.h, state_bwd.c):
-        # training: both directions in one differentiable call (forward and gradient each one library entry)
-        Y, df, db = NativeLstm2BidirFunction.apply(
-            P, weights.rec_fwd, state_fwd.h, state_fwd.c, weights.rec_bwd, state_bwd.h, state_bwd.c, mask
-        )
-        hf = _last_output_autograd(Y[:, :, :n], state_fwd.h, seq_lens, 1)
-        hb = _last_output_autograd(Y[:, :, n:], state_bwd.h, seq_lens, -1)
-        return Y, LstmState(h=hf, c=df), LstmState(h=hb, c=db)
-    ((Yf, _, _, df), (Yb, _, _, db)), Y = native_lstm2_multi(
-        [
-            (P[:, :, : 4 * n], weights.rec_fwd, state_fwd.h, state_fwd.c, mask, 0, 1),
-            (P[:, :, 4 * n :], weights.rec_bwd, state_bwd.h, state_bwd.c, mask, 0, -1),
-        ],
-        joint_output=True,
-    )
-    if T > 0:
-        hf = lstm_last_output(Yf, state_fwd.h, mask, 0, 1)
-        hb = lstm_last_output(Yb, state_bwd.h, mask, 0, -1)
-    else:
-        hf, hb = state_fwd.h.to(act), state_bwd.h.to(act)
-    return Y, LstmState(h=hf, c=df), LstmState(h=hb, c=db)
+    # both directions read their columns of one projection and write theirs of one output; forward and gradient each go
+    # through one entry of the library
+    Y, last, cells = native().lstm_layer(
+        source.to(act), weights.ff.to(act), None if weights.bias is None else weights.bias.to(act), mask,
+        [(weights.rec_fwd.to(act), state_fwd.h, state_fwd.c), (weights.rec_bwd.to(act), state_bwd.h, state_bwd.c)], 1, want_states and T > 0,
+    )  # fmt: skip
+    if not want_states:
+        return Y, None, None
+    hf, hb = last if T > 0 else (state_fwd.h.to(act), state_bwd.h.to(act))
+    return Y, LstmState(h=hf, c=cells[0]), LstmState(h=hb, c=cells[1])
 
 
 class LSTM(torch.nn.Module):
@@ -551,11 +517,12 @@ class BLSTM(torch.nn.Module):
 
     def forward(
         self, source: torch.Tensor, *, state_fwd: Optional[LstmState] = None, state_bwd: Optional[LstmState] = None,
-        seq_lens: Optional[torch.Tensor] = None,
-    ) -> Tuple[torch.Tensor, LstmState, LstmState]:  # fmt: skip
+        seq_lens: Optional[torch.Tensor] = None, mask: Optional[torch.Tensor] = None, want_states: bool = True,
+    ) -> Tuple[torch.Tensor, Optional[LstmState], Optional[LstmState]]:  # fmt: skip
         """
         :param source: [T,B,in]
         :param state_fwd, state_bwd: initial states, default zeros
+        :param mask, want_states: as for :func:`blstm`
         :return: [T,B,2*out_dim] (forward | backward), new forward state, new backward state
         """
         if source.dim() != 3 or source.shape[-1] != self.in_dim:
@@ -564,7 +531,8 @@ class BLSTM(torch.nn.Module):
         zero = None
         if state_fwd is None or state_bwd is None:
             zero = self.default_initial_state(batch_dims=(source.shape[1],), device=source.device, dtype=act)
-        return blstm(source, weights=self.weights(act), state_fwd=state_fwd or zero, state_bwd=state_bwd or zero, seq_lens=seq_lens)
+        return blstm(source, weights=self.weights(act), state_fwd=state_fwd or zero, state_bwd=state_bwd or zero, seq_lens=seq_lens,
+                     mask=mask, want_states=want_states)  # fmt: skip
 
     def extra_repr(self) -> str:
         return "in_dim=%i, out_dim=%i, with_bias=%s" % (self.in_dim, self.out_dim, self.bias is not None)
@@ -614,7 +582,13 @@ class BlstmEncoder(torch.nn.Module):
         """
         x = source
         states = []
+        kw = {}
+        if self.num_layers > 1 and source.dim() == 3 and source.is_cuda:
+            # what all layers share: the mask and the initial state
+            act = torch.bfloat16 if source.dtype == torch.bfloat16 else torch.float32
+            zero = self.layers[0].default_initial_state(batch_dims=(source.shape[1],), device=source.device, dtype=act)
+            kw = dict(mask=_mask(seq_lens, source), state_fwd=zero, state_bwd=zero)
         for layer in self.layers:
-            x, sf, sb = layer(x, seq_lens=seq_lens)
+            x, sf, sb = layer(x, seq_lens=seq_lens, want_states=collect_states, **kw)
             states.append((sf, sb))
         return (x, states) if collect_states else x

@@ -9,8 +9,9 @@ the schema the reference's generator would register (:242-277)::
         -> (Tensor, Tensor, Tensor, Tensor)
 
 Where the reference generates and compiles a C++ translation unit per op, this module registers the schema
-with ``torch.library`` from Python and the device implementation calls the prebuilt gfx950 library through
-its C ABI with raw device pointers and the current stream.  PyTorch only supplies memory and streams.
+with ``torch.library`` from Python; the device implementation (native code, ``csrc/rtn_torch_binding.cpp``; Python for
+the sibling ops) calls the prebuilt gfx950 library through its C ABI with raw device pointers and the current stream.
+PyTorch only supplies memory and streams.
 
 Argument handling follows the generated wrapper (:144-193): dtype normalisation, ndim checks,
 ``.contiguous()`` for ``need_contiguous`` inputs, device guard on the first tensor, outputs allocated on
@@ -21,8 +22,8 @@ every element; CPU tensors are rejected (no CPU implementation is shipped).
 
 from __future__ import annotations
 
-import collections
-import os
+import contextlib
+import ctypes
 import sys
 from threading import RLock
 from typing import Any, Dict, Optional
@@ -32,6 +33,30 @@ import torch
 from . import lib as _lib
 from . import native_op
 from .native_op import OpDescription
+
+_native_lock = RLock()
+_native_module = None
+
+
+def native():
+    """The native part of the torch path (``_rtn_torch.so``), given the entry points of the library: loaded once, never built
+    here, no fallback."""
+    global _native_module
+    if _native_module is not None:
+        return _native_module
+    with _native_lock:
+        if _native_module is None:
+            lib = _lib.load()
+            try:
+                from . import _rtn_torch
+            except ImportError as exc:
+                raise _lib.NativeLibraryMissing(
+                    "the torch binding could not be loaded (%s).  Build it with `python -m returnn_amd.build`." % exc
+                ) from exc
+            _rtn_torch.init({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in _lib.SYMBOLS}, NativeOpAborted)
+            _native_module = _rtn_torch
+    return _native_module
+
 
 _DTYPE_MAP = {"float32": torch.float32, "int32": torch.int32}
 
@@ -95,9 +120,10 @@ class OpMaker:
         return "%s(%s) -> (%s)" % (self.op_name, args, rets)
 
     def _impl_for(self):
-        _lib.load()  # fail now, loudly, if the HIP library is not there
+        native()  # fail now, loudly, if the HIP library is not there
+        if self.description.c_abi_fw == "rtn_native_lstm2_fwd":
+            return None  # (native code, registered for every mode when the binding is loaded)
         impl = {
-            "rtn_native_lstm2_fwd": _native_lstm2_device_impl,
             "rtn_lstm_generic_base_fwd": _lstm_generic_base_device_impl,
             "rtn_lstm_low_mem_fwd": _lstm_low_mem_device_impl,
         }.get(self.description.c_abi_fw)
@@ -117,7 +143,8 @@ class OpMaker:
             impl = self._impl_for()
             tlib = torch.library.Library(self.op_name, "DEF")
             tlib.define(self.schema())
-            tlib.impl(self.op_name, impl, "CUDA")  # the dispatch key PyTorch-ROCm uses for HIP tensors
+            if impl is not None:
+                tlib.impl(self.op_name, impl, "CUDA")  # the dispatch key PyTorch-ROCm uses for HIP tensors
             tlib.impl(self.op_name, _cpu_not_supported(self.op_name), "CPU")
             self._register_fake_impl()
             op = getattr(getattr(torch.ops, self.op_name), self.op_name)
@@ -260,78 +287,57 @@ class NativeOpAborted(RuntimeError):
 
 class StatusWatch:
     """
-    Looks after the status words of the library's workspaces without stalling the stream.
+    Looks after bounded waits of the library's kernels without touching the stream.
 
     The persistent kernels bound every wait for another workgroup (2 s of wall clock by default).  A wait that runs
-    into its bound sets the first word of the call's workspace slice to 1 and the workgroups that see it put NaN into
-    results every caller consumes (final cell state, last visited frame of Y; Dy0 and Dc0 of the gradient).  On top of
-    that, every op call here queues a copy of its status words to pinned host memory behind its kernels and records an
-    event; the next op call (or :meth:`poll`) looks at the copies whose event has completed and raises
-    :class:`NativeOpAborted` for a word that is 1.  Nothing waits for the device.
+    into its bound sets the first word of the call's workspace slice to 1, the workgroups that see it put NaN into
+    results every caller consumes (final cell state, last visited frame of Y; Dy0 and Dc0 of the gradient), and the
+    kernel writes the number of its call into a word of pinned host memory, where the next op call (or :meth:`poll`) finds
+    it and raises :class:`NativeOpAborted`.  Nothing is copied, recorded or waited for on the way.
 
     ``RTN_LSTM2_CHECK_STATUS=1`` in the environment (or ``status_watch.synchronous = True``) makes every op call wait
     for its own kernels and check at once: the error then names the call that failed, at the price of one stream
-    synchronisation per call.  ``RTN_LSTM2_CHECK_STATUS=0`` switches the watch off.  Under stream capture nothing is
-    queued (a captured copy would be replayed without anybody looking at it); captured calls rely on the NaN marks.
+    synchronisation per call.  ``RTN_LSTM2_CHECK_STATUS=0`` switches the watch off.  Calls under stream capture are not
+    watched (they would be replayed without anybody looking); they rely on the NaN marks.
     """
 
-    SLOTS = 64  # status words per pinned block; a block is reused once its event has completed
-
     def __init__(self):
-        self.lock = RLock()
-        self.pending = collections.deque()  # (event, host block, number of words, what)
-        self.free_blocks = []
-        self.synchronous: Optional[bool] = None  # None: from the environment, read at each call
-        self.checked = 0  # completed calls looked at so far (for tests)
+        self._synchronous: Optional[bool] = None
 
-    def _setting(self) -> str:
-        if self.synchronous is not None:
-            return "1" if self.synchronous else "lazy"
-        return os.environ.get("RTN_LSTM2_CHECK_STATUS", "lazy")
+    @property
+    def synchronous(self) -> Optional[bool]:
+        """None: from the environment, read at each call"""
+        return self._synchronous
 
-    def after_call(self, what: str, ws: torch.Tensor, count: int, device) -> None:
-        """Queue the look at the status word of each of the ``count`` equal slices of ``ws`` (current device = ``device``)."""
-        setting = self._setting()
-        if setting == "0" or count > self.SLOTS or torch.cuda.is_current_stream_capturing():
-            return
-        each = ws.numel() // count
-        words = ws.view(torch.int32)[: (count - 1) * (each // 4) + 1 : max(each // 4, 1)]
-        with self.lock:
-            block = self.free_blocks.pop() if self.free_blocks else torch.zeros((self.SLOTS,), dtype=torch.int32, pin_memory=True)
-        block[:count].copy_(words, non_blocking=True)
-        event = torch.cuda.Event()
-        event.record(torch.cuda.current_stream(device))
-        with self.lock:
-            self.pending.append((event, block, count, what))
-        if setting == "1":
-            event.synchronize()
-            self.poll()
+    @synchronous.setter
+    def synchronous(self, value: Optional[bool]) -> None:
+        self._synchronous = value
+        native().watch_synchronous(-1 if value is None else int(bool(value)))
+
+    @property
+    def checked(self) -> int:
+        """calls waited for and looked at so far (for tests)"""
+        return int(native().watch_checked())
+
+    @contextlib.contextmanager
+    def call(self, what: str, count: int = 1):
+        """Around one call of the library (current device and stream)."""
+        watched = native().watch_before(what, count)
+        failed = True
+        try:
+            yield
+            failed = False
+        finally:
+            if watched:
+                native().watch_after(failed)
 
     def poll(self) -> None:
-        """Raise for the oldest completed call whose status word says that a wait expired; never blocks."""
-        if torch.cuda.is_current_stream_capturing():
-            return  # (no queries while a capture is under way)
-        failed = None
-        with self.lock:
-            while self.pending and self.pending[0][0].query():
-                _, block, count, what = self.pending.popleft()
-                self.checked += 1
-                if failed is None and any(int(w) == 1 for w in block[:count].tolist()):
-                    failed = what
-                self.free_blocks.append(block)
-        if failed is not None:
-            raise NativeOpAborted(
-                "%s: a bounded wait in the persistent kernel expired (device shared, preempted or paused?); the results of "
-                "that call are invalid.  RTN_LSTM2_TIMEOUT_TICKS sets the bound in 10 ns ticks." % failed
-            )
+        """Raise for a call whose wait expired; never blocks."""
+        native().watch_poll()
 
     def drain(self) -> None:
-        """Wait for every queued look and check it (end of a step, end of the program, tests)."""
-        with self.lock:
-            events = [e for e, _, _, _ in self.pending]
-        for e in events:
-            e.synchronize()
-        self.poll()
+        """Wait for every call so far and check (end of a step, end of the program, tests)."""
+        native().watch_drain()
 
 
 status_watch = StatusWatch()
@@ -350,86 +356,6 @@ def _cpu_not_supported(name):
 def _check_ndim(t: torch.Tensor, info: Dict[str, Any]):
     if t.dim() != info["ndim"]:
         raise RuntimeError("%s shape ndim is not %i, got shape %s" % (info["name"], info["ndim"], tuple(t.shape)))
-
-
-def _row_pitch(t: torch.Tensor, *, itemsize: int) -> int:
-    """
-    Row pitch in elements if ``t`` ([T,B,width]) can be handed to the library as it is: unit stride along the last axis,
-    rows of consecutive (frame, sequence) pairs a constant number of elements apart, 16-byte aligned rows.  0 if not
-    (the caller then makes a contiguous copy).  A contiguous tensor gives ``width``.
-    """
-    if t.dim() != 3:
-        return 0
-    T, B, width = t.shape
-    if T * B * width == 0:
-        return width if t.is_contiguous() else 0
-    ld = t.stride(1) if B > 1 else (t.stride(0) if T > 1 else width)
-    ok = (width == 1 or t.stride(2) == 1) and ld >= width and (B == 1 or t.stride(1) == ld) and (T == 1 or t.stride(0) == B * ld)
-    ok = ok and (ld * itemsize) % 16 == 0 and t.data_ptr() % 16 == 0
-    return int(ld) if ok else 0
-
-
-def _normalise_lstm2_args(X, W, y0, c0, i, *, pitched_x: bool = False):
-    """Argument handling of the generated wrapper (returnn/torch/util/native_op.py:144-193) plus the op's shape
-    asserts (returnn/native_op.py:1215-1223) as hard errors.  Returns the tensors to hand to the library and (T, B, n, bf16)."""
-    infos = native_op.NativeLstm2.in_info
-    for t, info in zip((X, W, y0, c0, i), infos):
-        _check_ndim(t, info)
-    device = X.device
-    for t, info in zip((W, y0, c0, i), infos[1:]):
-        if t.device != device:
-            raise RuntimeError("%s is on %s but X is on %s" % (info["name"], t.device, device))
-    bf16 = X.dtype == torch.bfloat16
-    act = torch.bfloat16 if bf16 else torch.float32
-    X, W, y0 = (t if t.dtype == act else t.to(act) for t in (X, W, y0))
-    c0, i = (t if t.dtype == torch.float32 else t.to(torch.float32) for t in (c0, i))
-    if not (pitched_x and _row_pitch(X, itemsize=X.element_size())):  # (a view with a row pitch goes to the library as it is)
-        X = X if X.is_contiguous() else X.contiguous()
-    W, y0, c0, i = (t if t.is_contiguous() else t.contiguous() for t in (W, y0, c0, i))
-    T, B = i.shape
-    n = y0.shape[1]
-    expect = {"X": (T, B, 4 * n), "W": (n, 4 * n), "y0": (B, n), "c0": (B, n)}
-    for name, t in (("X", X), ("W", W), ("y0", y0), ("c0", c0)):
-        if tuple(t.shape) != expect[name]:
-            raise RuntimeError(
-                "NativeLstm2: %s has shape %s, expected %s (T=%i, B=%i from i; n=%i from y0)"
-                % (name, tuple(t.shape), expect[name], T, B, n)
-            )
-    return (X, W, y0, c0, i), (T, B, n, bf16)
-
-
-def _alloc_lstm2_outputs(T, B, n, bf16, device):
-    act = torch.bfloat16 if bf16 else torch.float32
-    Y = torch.empty((T, B, n), dtype=act, device=device)
-    C = torch.empty((T, B, n), dtype=torch.float32, device=device)
-    H = torch.empty((T, B, 4 * n), dtype=act, device=device)
-    d = torch.empty((B, n), dtype=torch.float32, device=device)
-    return Y, C, H, d
-
-
-def _native_lstm2_device_impl(X, W, y0, c0, i, start, step, *, mode=_lib.MODE_AUTO):
-    """``NativeLstm2`` on HIP tensors: normalise the arguments, allocate outputs and scratch, enqueue the library call."""
-    (X, W, y0, c0, i), (T, B, n, bf16) = _normalise_lstm2_args(X, W, y0, c0, i)
-    device = X.device
-    lib = _lib.load()
-    dtype = _lib.DTYPE_BF16 if bf16 else _lib.DTYPE_F32
-    with torch.cuda.device(device):
-        status_watch.poll()
-        Y, C, H, d = _alloc_lstm2_outputs(T, B, n, bf16, device)
-        ws_bytes = int(lib.rtn_native_lstm2_fwd_workspace_bytes(T, B, n, dtype, mode))
-        ws = torch.empty((max(ws_bytes, 256),), dtype=torch.uint8, device=device)
-        stream = torch.cuda.current_stream(device).cuda_stream
-        rc = lib.rtn_native_lstm2_fwd(
-            X.data_ptr(), W.data_ptr(), y0.data_ptr(), c0.data_ptr(), i.data_ptr(), int(start), int(step),
-            Y.data_ptr(), C.data_ptr(), H.data_ptr(), d.data_ptr(), T, B, n, dtype, mode,
-            ws.data_ptr(), ws.numel(), stream,
-        )  # fmt: skip
-        _lib.check(rc)
-        if T * B * n > 0:  # (an empty problem does not touch its workspace)
-            status_watch.after_call("NativeLstm2", ws, 1, device)
-    # The workspace goes back to the caching allocator here; the allocator keeps it out of other
-    # streams' hands until the work queued on this stream has passed it (stream-ordered reuse).
-    return Y, C, H, d
 
 
 def _act_and_dtype(first: torch.Tensor):
@@ -456,18 +382,16 @@ def _lstm_generic_base_device_impl(Z, V_h, c, i, *, mode=_lib.MODE_AUTO):
             raise RuntimeError("LstmGenericBase: %s is on %s but Z is on %s" % (name, t.device, device))
     lib = _lib.load()
     with torch.cuda.device(device):
-        status_watch.poll()
         Y = torch.empty((T, B, n), dtype=act, device=device)
         H = torch.empty((T, B, 4 * n), dtype=act, device=device)
         d = torch.empty((B, n), dtype=torch.float32, device=device)
         ws = torch.empty((max(int(lib.rtn_lstm_generic_base_fwd_workspace_bytes(T, B, n, dtype, mode)), 256),), dtype=torch.uint8, device=device)
-        rc = lib.rtn_lstm_generic_base_fwd(
-            Z.data_ptr(), V_h.data_ptr(), c.data_ptr(), i.data_ptr(), Y.data_ptr(), H.data_ptr(), d.data_ptr(), T, B, n, dtype, mode,
-            ws.data_ptr(), ws.numel(), torch.cuda.current_stream(device).cuda_stream,
-        )  # fmt: skip
-        _lib.check(rc)
-        if T * B * n > 0:  # (an empty problem does not touch its workspace)
-            status_watch.after_call("LstmGenericBase", ws, 1, device)
+        with status_watch.call("LstmGenericBase"):
+            rc = lib.rtn_lstm_generic_base_fwd(
+                Z.data_ptr(), V_h.data_ptr(), c.data_ptr(), i.data_ptr(), Y.data_ptr(), H.data_ptr(), d.data_ptr(), T, B, n, dtype, mode,
+                ws.data_ptr(), ws.numel(), torch.cuda.current_stream(device).cuda_stream,
+            )  # fmt: skip
+            _lib.check(rc)
     return Y, H, d
 
 
@@ -489,19 +413,17 @@ def _lstm_low_mem_device_impl(X, W, b, y0, c0, i, start, step, *, mode=_lib.MODE
             raise RuntimeError("LstmLowMem: %s is on %s but X is on %s" % (name, t.device, device))
     lib = _lib.load()
     with torch.cuda.device(device):
-        status_watch.poll()
         Y = torch.empty((T, B, n), dtype=act, device=device)
         C = torch.empty((T, B, n), dtype=torch.float32, device=device)
         d = torch.empty((B, n), dtype=torch.float32, device=device)
         ws = torch.empty((max(int(lib.rtn_lstm_low_mem_fwd_workspace_bytes(T, B, n_in, n, dtype, mode)), 256),), dtype=torch.uint8, device=device)
-        rc = lib.rtn_lstm_low_mem_fwd(
-            X.data_ptr(), W.data_ptr(), b.data_ptr(), y0.data_ptr(), c0.data_ptr(), i.data_ptr(), int(start), int(step),
-            Y.data_ptr(), C.data_ptr(), d.data_ptr(), T, B, n_in, n, dtype, mode, ws.data_ptr(), ws.numel(),
-            torch.cuda.current_stream(device).cuda_stream,
-        )  # fmt: skip
-        _lib.check(rc)
-        if T * B * n > 0:  # (an empty problem does not touch its workspace)
-            status_watch.after_call("LstmLowMem", ws, 1, device)
+        with status_watch.call("LstmLowMem"):
+            rc = lib.rtn_lstm_low_mem_fwd(
+                X.data_ptr(), W.data_ptr(), b.data_ptr(), y0.data_ptr(), c0.data_ptr(), i.data_ptr(), int(start), int(step),
+                Y.data_ptr(), C.data_ptr(), d.data_ptr(), T, B, n_in, n, dtype, mode, ws.data_ptr(), ws.numel(),
+                torch.cuda.current_stream(device).cuda_stream,
+            )  # fmt: skip
+            _lib.check(rc)
     return Y, C, d
 
 
@@ -523,81 +445,7 @@ def native_lstm2_multi(calls, *, mode: Optional[str] = None, joint_output: bool 
     calls = list(calls)
     if not calls:
         return []
-    lib = _lib.load()
-    norm = [_normalise_lstm2_args(*c[:5], pitched_x=True) for c in calls]
-    shape = norm[0][1]
-    device = norm[0][0][0].device
-    for tensors, sh in norm:
-        if sh != shape:
-            raise RuntimeError("native_lstm2_multi: all calls need the same T, B, n and element type; got %r and %r" % (shape, sh))
-        if tensors[0].device != device:
-            raise RuntimeError("native_lstm2_multi: all calls must be on one device")
-    if not norm[0][0][0].is_cuda:
-        raise RuntimeError("NativeLstm2: this build implements the op for HIP (MI355X) tensors only; got CPU tensors.")
-    T, B, n, bf16 = shape
-    dtype = _lib.DTYPE_BF16 if bf16 else _lib.DTYPE_F32
-    mode_code = _lib.MODES[mode or "auto"]
-    count = len(calls)
-    arr = (_lib.Lstm2Call * count)()
-    outs = []
-    with torch.cuda.device(device):
-        status_watch.poll()
-        act = torch.bfloat16 if bf16 else torch.float32
-        joint = torch.empty((T, B, count * n), dtype=act, device=device) if joint_output else None
-        if joint is not None and ((n * joint.element_size()) % 16 != 0):
-            joint = None  # (columns of the calls would not be 16-byte aligned: separate arrays, joined below)
-        for k, ((X, W, y0, c0, i), c) in enumerate(zip((t for t, _ in norm), calls)):
-            Y, C, H, d = _alloc_lstm2_outputs(T, B, n, bf16, device)
-            if joint is not None:
-                Y = joint[:, :, k * n : (k + 1) * n]
-            outs.append((Y, C, H, d))
-            arr[k] = _lib.Lstm2Call(
-                X.data_ptr(), W.data_ptr(), y0.data_ptr(), c0.data_ptr(), i.data_ptr(), int(c[5]), int(c[6]),
-                Y.data_ptr(), C.data_ptr(), H.data_ptr(), d.data_ptr(),
-                0 if X.is_contiguous() else _row_pitch(X, itemsize=X.element_size()), 0 if joint is None else count * n,
-            )  # fmt: skip
-        ws_bytes = int(lib.rtn_native_lstm2_fwd_multi_workspace_bytes(count, T, B, n, dtype, mode_code))
-        ws = torch.empty((max(ws_bytes, 256),), dtype=torch.uint8, device=device)
-        stream = torch.cuda.current_stream(device).cuda_stream
-        rc = lib.rtn_native_lstm2_fwd_multi(arr, count, T, B, n, dtype, mode_code, ws.data_ptr(), ws.numel(), stream)
-        _lib.check(rc)
-        if T * B * n > 0:  # (an empty problem does not touch its workspace)
-            status_watch.after_call("NativeLstm2 (%i calls)" % count, ws, count, device)
-    del norm  # the normalised inputs stay alive until here; the stream-ordered allocator covers the rest
-    if joint_output:
-        return outs, (joint if joint is not None else torch.cat([o[0] for o in outs], dim=-1))
-    return outs
-
-
-def _normalise_grad_args(W, y0, c0, i, Y, C, H, DY, Dd):
-    if not Y.is_cuda:
-        raise RuntimeError("NativeLstm2 gradient: this build implements the op for HIP (MI355X) tensors only; got CPU tensors.")
-    bf16 = Y.dtype == torch.bfloat16
-    act = torch.bfloat16 if bf16 else torch.float32
-    device = Y.device
-    W, y0, H = (t.to(act).contiguous() for t in (W, y0, H))
-    # (Y and DY may be views with a row pitch, e.g. one direction's half of a [T,B,2n] array: handed over as they are)
-    Y, DY = (t if _row_pitch(t, itemsize=t.element_size()) else t.contiguous() for t in (Y.to(act), DY.to(act)))
-    c0, i, C, Dd = (t.to(torch.float32).contiguous() for t in (c0, i, C, Dd))
-    T, B = i.shape
-    n = y0.shape[1]
-    expect = {"W": (n, 4 * n), "y0": (B, n), "c0": (B, n), "Y": (T, B, n), "C": (T, B, n), "H": (T, B, 4 * n),
-              "DY": (T, B, n), "Dd": (B, n)}  # fmt: skip
-    for name, t in (("W", W), ("y0", y0), ("c0", c0), ("Y", Y), ("C", C), ("H", H), ("DY", DY), ("Dd", Dd)):
-        if tuple(t.shape) != expect[name]:
-            raise RuntimeError("NativeLstm2 gradient: %s has shape %s, expected %s" % (name, tuple(t.shape), expect[name]))
-        if t.device != device:
-            raise RuntimeError("NativeLstm2 gradient: %s is on %s but Y is on %s" % (name, t.device, device))
-    return (W, y0, c0, i, Y, C, H, DY, Dd), (T, B, n, bf16)
-
-
-def _alloc_grad_outputs(T, B, n, bf16, device):
-    act = torch.bfloat16 if bf16 else torch.float32
-    DX = torch.empty((T, B, 4 * n), dtype=act, device=device)
-    DW = torch.empty((n, 4 * n), dtype=torch.float32, device=device)
-    Dy0 = torch.empty((B, n), dtype=act, device=device)
-    Dc0 = torch.empty((B, n), dtype=torch.float32, device=device)
-    return DX, DW, Dy0, Dc0
+    return native().lstm2_multi(calls, _lib.MODES[mode or "auto"], joint_output)
 
 
 def native_lstm2_grad(W, y0, c0, i, start, step, Y, C, H, DY, Dd):
@@ -627,46 +475,7 @@ def native_lstm2_grad_multi(calls, *, joint_dx: bool = False):
     calls = list(calls)
     if not calls:
         return ([], None) if joint_dx else []
-    norm = []
-    shape = None
-    for W, y0, c0, i, start, step, Y, C, H, DY, Dd in calls:
-        tensors, this = _normalise_grad_args(W, y0, c0, i, Y, C, H, DY, Dd)
-        if shape is None:
-            shape, device = this, tensors[4].device
-        elif this != shape or tensors[4].device != device:
-            raise RuntimeError("native_lstm2_grad_multi: all calls must have one shape, dtype and device; got %r and %r" % (shape, this))
-        norm.append((tensors, int(start), int(step)))
-    T, B, n, bf16 = shape
-    lib = _lib.load()
-    dtype = _lib.DTYPE_BF16 if bf16 else _lib.DTYPE_F32
-    count = len(norm)
-    with torch.cuda.device(device):
-        status_watch.poll()
-        outs = [_alloc_grad_outputs(T, B, n, bf16, device) for _ in range(count)]
-        joint = None
-        if joint_dx and (4 * n * outs[0][0].element_size()) % 16 == 0:  # (else: separate arrays, joined below)
-            joint = torch.empty((T, B, count * 4 * n), dtype=outs[0][0].dtype, device=device)
-            outs = [(joint[:, :, k * 4 * n : (k + 1) * 4 * n],) + o[1:] for k, o in enumerate(outs)]
-        ws_bytes = int(lib.rtn_native_lstm2_bwd_multi_workspace_bytes(count, T, B, n, dtype))
-        ws = torch.empty((max(ws_bytes, 256),), dtype=torch.uint8, device=device)
-        arr = (_lib.Lstm2BwdCall * count)()
-        for k, ((W, y0, c0, i, Y, C, H, DY, Dd), start, step) in enumerate(norm):
-            DX, DW, Dy0, Dc0 = outs[k]
-            arr[k] = _lib.Lstm2BwdCall(
-                W.data_ptr(), y0.data_ptr(), c0.data_ptr(), i.data_ptr(), start, step, Y.data_ptr(), C.data_ptr(), H.data_ptr(),
-                DY.data_ptr(), Dd.data_ptr(), DX.data_ptr(), DW.data_ptr(), Dy0.data_ptr(), Dc0.data_ptr(),
-                0 if Y.is_contiguous() else _row_pitch(Y, itemsize=Y.element_size()),
-                0 if DY.is_contiguous() else _row_pitch(DY, itemsize=DY.element_size()),
-                0 if joint is None else count * 4 * n,
-            )  # fmt: skip
-        rc = lib.rtn_native_lstm2_bwd_multi(arr, count, T, B, n, dtype, ws.data_ptr(), ws.numel(), torch.cuda.current_stream(device).cuda_stream)
-        _lib.check(rc)
-        if T * B * n > 0:  # (an empty problem does not touch its workspace)
-            status_watch.after_call("NativeLstm2 gradient (%i calls)" % count, ws, count, device)
-    del norm  # (the normalised inputs stay alive until here; the stream-ordered allocator covers the rest)
-    if joint_dx:
-        return outs, (joint if joint is not None else torch.cat([o[0] for o in outs], dim=-1))
-    return outs
+    return native().lstm2_grad_multi(calls, joint_dx)
 
 
 class NativeLstm2Function(torch.autograd.Function):
@@ -724,18 +533,16 @@ def lstm_generic_base_grad(V_h, c, i, Y, H, DY, Dd):
     lib = _lib.load()
     dtype = _lib.DTYPE_BF16 if bf16 else _lib.DTYPE_F32
     with torch.cuda.device(device):
-        status_watch.poll()
         DZ = torch.empty((T, B, 4 * n), dtype=act, device=device)
         DV_h = torch.empty((n, 4 * n), dtype=torch.float32, device=device)
         Dc = torch.empty((B, n), dtype=torch.float32, device=device)
         ws = torch.empty((max(int(lib.rtn_lstm_generic_base_bwd_workspace_bytes(T, B, n, dtype)), 256),), dtype=torch.uint8, device=device)
-        rc = lib.rtn_lstm_generic_base_bwd(
-            V_h.data_ptr(), c.data_ptr(), i.data_ptr(), Y.data_ptr(), H.data_ptr(), DY.data_ptr(), Dd.data_ptr(), DZ.data_ptr(),
-            DV_h.data_ptr(), Dc.data_ptr(), T, B, n, dtype, ws.data_ptr(), ws.numel(), torch.cuda.current_stream(device).cuda_stream,
-        )  # fmt: skip
-        _lib.check(rc)
-        if T * B * n > 0:  # (an empty problem does not touch its workspace)
-            status_watch.after_call("LstmGenericBase gradient", ws, 1, device)
+        with status_watch.call("LstmGenericBase gradient"):
+            rc = lib.rtn_lstm_generic_base_bwd(
+                V_h.data_ptr(), c.data_ptr(), i.data_ptr(), Y.data_ptr(), H.data_ptr(), DY.data_ptr(), Dd.data_ptr(), DZ.data_ptr(),
+                DV_h.data_ptr(), Dc.data_ptr(), T, B, n, dtype, ws.data_ptr(), ws.numel(), torch.cuda.current_stream(device).cuda_stream,
+            )  # fmt: skip
+            _lib.check(rc)
     return DZ, DV_h, Dc
 
 
@@ -789,21 +596,19 @@ def lstm_low_mem_grad(X, W, b, y0, c0, i, start, step, Y, C, DY, Dd):
     lib = _lib.load()
     dtype = _lib.DTYPE_BF16 if bf16 else _lib.DTYPE_F32
     with torch.cuda.device(device):
-        status_watch.poll()
         DX = torch.empty((T, B, n_in), dtype=act, device=device)
         DW = torch.empty((n_in + n, 4 * n), dtype=torch.float32, device=device)
         Db = torch.empty((4 * n,), dtype=torch.float32, device=device)
         Dh = torch.empty((B, n), dtype=act, device=device)
         Dc = torch.empty((B, n), dtype=torch.float32, device=device)
         ws = torch.empty((max(int(lib.rtn_lstm_low_mem_bwd_workspace_bytes(T, B, n_in, n, dtype)), 256),), dtype=torch.uint8, device=device)
-        rc = lib.rtn_lstm_low_mem_bwd(
-            X.data_ptr(), W.data_ptr(), b.data_ptr(), y0.data_ptr(), c0.data_ptr(), i.data_ptr(), int(start), int(step), Y.data_ptr(),
-            C.data_ptr(), DY.data_ptr(), Dd.data_ptr(), DX.data_ptr(), DW.data_ptr(), Db.data_ptr(), Dh.data_ptr(), Dc.data_ptr(),
-            T, B, n_in, n, dtype, ws.data_ptr(), ws.numel(), torch.cuda.current_stream(device).cuda_stream,
-        )  # fmt: skip
-        _lib.check(rc)
-        if T * B * n > 0:  # (an empty problem does not touch its workspace)
-            status_watch.after_call("LstmLowMem gradient", ws, 1, device)
+        with status_watch.call("LstmLowMem gradient"):
+            rc = lib.rtn_lstm_low_mem_bwd(
+                X.data_ptr(), W.data_ptr(), b.data_ptr(), y0.data_ptr(), c0.data_ptr(), i.data_ptr(), int(start), int(step), Y.data_ptr(),
+                C.data_ptr(), DY.data_ptr(), Dd.data_ptr(), DX.data_ptr(), DW.data_ptr(), Db.data_ptr(), Dh.data_ptr(), Dc.data_ptr(),
+                T, B, n_in, n, dtype, ws.data_ptr(), ws.numel(), torch.cuda.current_stream(device).cuda_stream,
+            )  # fmt: skip
+            _lib.check(rc)
     return DX, DW, Db, Dh, Dc
 
 
@@ -914,25 +719,4 @@ def lstm_last_output(Y: torch.Tensor, y0: torch.Tensor, i: torch.Tensor, start: 
     :param i: [T,B] mask
     :return: [B,n]
     """
-    if not Y.is_cuda:
-        raise RuntimeError("lstm_last_output: this build implements the op for HIP (MI355X) tensors only")
-    bf16 = Y.dtype == torch.bfloat16
-    act = torch.bfloat16 if bf16 else torch.float32
-    Y = Y.to(act)
-    ldY = _row_pitch(Y, itemsize=Y.element_size())
-    if not ldY:
-        Y, ldY = Y.contiguous(), Y.shape[2]
-    y0 = y0.to(act).contiguous()
-    i = i.to(torch.float32).contiguous()
-    T, B, n = Y.shape
-    if tuple(y0.shape) != (B, n) or tuple(i.shape) != (T, B):
-        raise RuntimeError("lstm_last_output: y0 %s / i %s do not match Y %s" % (tuple(y0.shape), tuple(i.shape), tuple(Y.shape)))
-    lib = _lib.load()
-    with torch.cuda.device(Y.device):
-        out = torch.empty((B, n), dtype=act, device=Y.device)
-        rc = lib.rtn_native_lstm2_last_output(
-            Y.data_ptr(), y0.data_ptr(), i.data_ptr(), int(start), int(step), out.data_ptr(), T, B, n,
-            _lib.DTYPE_BF16 if bf16 else _lib.DTYPE_F32, int(ldY), torch.cuda.current_stream(Y.device).cuda_stream,
-        )  # fmt: skip
-    _lib.check(rc)
-    return out
+    return native().last_output(Y, y0, i, int(start), int(step))

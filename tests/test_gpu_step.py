@@ -1,0 +1,45 @@
+"""One step of a layer, projection included (``rtn_lstm_step``), against the same step in float64 on the CPU."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from _gpu_util import announce
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize(
+    "B,n_in,n,bias",
+    [(1, 1, 1, True), (1, 40, 32, False), (3, 33, 7, True), (16, 512, 64, True), (17, 31, 100, True), (33, 80, 1000, False), (64, 65, 72, True),
+     (65, 16, 33, True), (130, 200, 136, True), (12, 512, 1024, True)],
+)  # fmt: skip
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_step_against_float64(B, n_in, n, bias, dtype):
+    announce("lstm_step", B, n_in, n, bias, dtype)
+    from returnn_amd.lstm import LSTM, LstmState
+
+    act = torch.bfloat16 if dtype == "bf16" else torch.float32
+    gen = torch.Generator().manual_seed(B + 7 * n_in + 31 * n)
+    m = LSTM(n_in, n, with_bias=bias)
+    m.reset_parameters(gen)
+    if bias:
+        with torch.no_grad():
+            m.bias.uniform_(-0.5, 0.5, generator=gen)
+    m = m.to(act).requires_grad_(False)
+    x, h = (torch.randn((B, k), generator=gen).mul(0.5).to(act) for k in (n_in, n))
+    c = torch.randn((B, n), generator=gen)
+    gates = x.double() @ m.ff.double().t() + h.double() @ m.rec.double()
+    if bias:
+        gates = gates + m.bias.double()
+    g, i, f, o = gates.chunk(4, dim=1)
+    want_c = torch.sigmoid(f) * c.double() + torch.sigmoid(i) * torch.tanh(g)
+    want_y = torch.sigmoid(o) * torch.tanh(want_c)
+    y, st = m.to("cuda:0")(x.cuda(), state=LstmState(h=h.cuda(), c=c.cuda()))
+    torch.cuda.synchronize()
+    assert y.dtype == act and st.h.dtype == act and st.c.dtype == torch.float32
+    assert torch.equal(y, st.h) and y.data_ptr() != st.h.data_ptr()
+    tol = 1e-2 if dtype == "bf16" else 2e-6
+    for got, want in ((y, want_y), (st.c, want_c)):
+        assert float((got.cpu().double() - want).abs().max()) <= tol
