@@ -6,6 +6,7 @@
 
 #include "lstm2_bwd_kernels.h"
 #include "lstm2_kernels.h"
+#include "lstm2_wide_kernel.h"
 
 namespace rtn {
 
@@ -18,6 +19,16 @@ RegwKernel regw_table_bf16_lo(int MT, int NT, int KSMAX, bool half, bool tail);
 RegwKernel regw_table_bf16_hi(int MT, int NT, int KSMAX, bool half, bool tail);
 RegwKernel regw_table_f32_lo(int MT, int NT, int KSMAX, bool half, bool tail);
 RegwKernel regw_table_f32_hi(int MT, int NT, int KSMAX, bool half, bool tail);
+
+// Forward kernel for wide layers k_lstm2_wide<AT, MT, NT, KS, LF>.
+typedef void (*WideKernel)(const Lstm2Params);
+struct WideBuild {
+  WideKernel kernel;
+  int dtype, MT, NT, KS, LF;
+};
+// The build for a layer of width n on `cus` CUs and `rows` rows per launch; the last one in the list if rows are more than
+// any build for that width takes; kernel null: none.
+WideBuild wide_kernel(int dtype, int n, int cus, int rows);
 
 // Persistent gradient kernel k_lstm2_bwd_regw<AT, KSB, MT, WV, 0, HALF>; KSB: fragments of W per tile and wavefront,
 // MT: tiles of 16 values of k per workgroup, WV: wavefronts per workgroup.  "half": groups of at most 8 rows.

@@ -5,7 +5,7 @@
 #include "lstm2_kernel_tables.h"
 
 #ifndef RTN_TABLE_PART
-#error "compile with -DRTN_TABLE_PART=<1..8>"
+#error "compile with -DRTN_TABLE_PART=<1..9>"
 #endif
 
 namespace rtn {
@@ -94,8 +94,29 @@ BwdRegwKernel bwd_regw_table_f32_half(int KSB, int MT, int WV) { return bwd_regw
 #elif RTN_TABLE_PART == 8
 BwdRegwKernel bwd_regw_table_f32_full(int KSB, int MT, int WV) { return bwd_regw_table<float, false>(KSB, MT, WV); }
 BwdRegwKernel bwd_regw_lds_table_f32(int WV) { return bwd_regw_lds_table<float>(WV); }
+#elif RTN_TABLE_PART == 9
+// Ascending by the width that MT tiles on 256 CUs and KS macro steps per wavefront take, then by rows.  What bounds NT: W,
+// 4 MT NT accumulator registers and two chunks of h per wavefront in 512 registers.
+WideBuild wide_kernel(int dtype, int n, int cus, int rows) {
+#define RTN_WIDE(at, dt, mt, nt, ks, lf) {&k_lstm2_wide<at, mt, nt, ks, lf>, dt, mt, nt, ks, lf}
+  static const WideBuild builds[] = {
+      RTN_WIDE(float, 0, 2, 1, 32, 0), RTN_WIDE(float, 0, 2, 2, 32, 0), RTN_WIDE(float, 0, 3, 1, 44, 36),
+      RTN_WIDE(__bf16, 1, 3, 1, 24, 0), RTN_WIDE(__bf16, 1, 3, 2, 24, 0), RTN_WIDE(__bf16, 1, 4, 1, 32, 32),
+  };
+#undef RTN_WIDE
+  WideBuild best = {nullptr, 0, 0, 0, 0, 0};
+  for (const WideBuild& b : builds) {
+    if (b.dtype != dtype) continue;
+    const int KM = dtype == 1 ? 32 : 16;
+    if ((n / 4 + b.MT - 1) / b.MT > cus || (n / KM + kWaves - 1) / kWaves > b.KS) continue;
+    if (best.kernel && (b.MT != best.MT || b.KS != best.KS)) break;  // (the narrowest builds that take the width)
+    best = b;
+    if (rows <= 16 * b.NT) break;
+  }
+  return best;
+}
 #else
-#error "RTN_TABLE_PART must be 1..8"
+#error "RTN_TABLE_PART must be 1..9"
 #endif
 
 }  // namespace rtn

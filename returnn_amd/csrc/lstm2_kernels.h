@@ -197,6 +197,8 @@ __device__ __forceinline__ void prepare_mfma(const Lstm2Params& p, int n_flags) 
     const long long total = (long long)p.groups_total * p.hx_bufs * words_per_buf;
     for (long long w = gtid; w < total; w += gsz)
       if ((w / words_per_buf) % p.hx_bufs != 0) ((unsigned*)p.hx)[w] = 0xFFFFFFFFu;
+    if (p.hxl)
+      for (long long w = gtid; w < (long long)p.xcds * p.hx_bufs * words_per_buf; w += gsz) ((unsigned*)p.hxl)[w] = 0xFFFFFFFFu;
   }
   // W -> Wp
   const int S = p.n / KM;

@@ -50,6 +50,7 @@ struct Lstm2Params {
   // workspace sections (device)
   unsigned* status;  // [64]   see StatusWords
   unsigned* flags;   // [groups_total*wgs_per_group] last published step (+1) of each workgroup
+  void* hxl;         // k_lstm2_wide: [xcds][hx_bufs][n/KE][Bp][KE] AT, the copies of h for one launch
   void* hx;          // [groups_total][hx_bufs][n/KE][Bp][KE] AT: hidden state in MFMA B-operand order, ring of buffers
   void* Wp;          // [n/4][S][64][16 bytes]: W in MFMA A-operand order
   void* ycarry;      // [2][B][n] AT: hidden-state carry of the generic per-step kernels

@@ -170,6 +170,8 @@ struct Plan {
   int mode = RTN_MODE_STEPWISE;  // resolved: PERSISTENT, GRAPH or STEPWISE
   bool regw = false;             // persistent kernel with W in registers and self-validating exchange
   bool local = false;            // regw: every batch group on one XCD, hidden state exchanged through that XCD's L2
+  bool wide = false;             // persistent kernel for layers whose W takes registers and LDS of the whole device
+  WideBuild wide_build = {nullptr, 0, 0, 0, 0, 0};
   bool half = false;             // regw: groups of at most 8 rows, two tiles folded into one pass of the pointwise part
   int grid = 0;                  // workgroups launched by the persistent kernel
   int KSMAX = 0;                 // its macro steps per wavefront (template bound)
@@ -180,7 +182,7 @@ struct Plan {
   size_t lds_bytes = 0;
   bool w_direct = false;         // per-step launches read W from memory without an LDS copy
   // workspace layout (byte offsets)
-  size_t off_status = 0, off_flags = 0, off_hx = 0, off_wp = 0, off_ycarry = 0, off_trace = 0, total = 0;
+  size_t off_status = 0, off_flags = 0, off_hx = 0, off_wp = 0, off_ycarry = 0, off_hxl = 0, off_trace = 0, total = 0;
   int n_flags = 0;
 };
 
@@ -416,6 +418,31 @@ bool make_plan_uncached(int64_t T, int B, int n, int dtype, int want_mode, bool 
         pl.lds_bytes = chosen.lds;
         persistent_ok = true;
       }
+      // Layers beyond the register kernel's widths (n > 2048 in bf16, > 1024 in float32): the wide kernel, which takes the
+      // whole device for every 16 or 32 rows.  Only against a device that is there, since it uses its registers and LDS
+      // to the last.
+      if (KSMAX == 0 && di.valid && di.xcds >= 1 && (env_kernel == 0 || env_kernel == 3)) {
+        const WideBuild wb = wide_kernel(dtype, n, di.cus, B);
+        const int rows = 16 * wb.NT, turns = wb.kernel ? (B + rows - 1) / rows : 0;
+        const int G = wb.kernel ? (n / 4 + wb.MT - 1) / wb.MT : 0;
+        const long env_passes = env_long("RTN_LSTM2_MAX_PASSES", -1);
+        const size_t lds = wb.kernel ? wide_lds_bytes(wb.MT, wb.NT, wb.LF) + 64 : 0;
+        if (wb.kernel && turns <= (env_passes >= 0 ? env_passes : kMaxPassesOverSteps) && lds <= di.lds_per_wg && G >= 2 * di.xcds &&
+            (n / (dtype == RTN_DTYPE_BF16 ? 8 : 4) * rows + G / di.xcds - 1) / (G / di.xcds) <= kWideForward * kWgThreads) {
+          pl = Plan();
+          pl.kind = kPlanMfma;
+          pl.wide = true;
+          pl.wide_build = wb;
+          pl.MT = wb.MT;
+          pl.NT = wb.NT;
+          pl.Bg = (B + turns - 1) / turns;
+          pl.wgs_per_group = pl.grid = G;
+          pl.groups = 1;
+          pl.groups_total = pl.passes = turns;
+          pl.lds_bytes = lds - 64;
+          persistent_ok = true;
+        }
+      }
       if (!persistent_ok && why) *why = "no decomposition keeps W on chip with all workgroups co-resident";
     }
     if (persistent_ok && capturing && !capture_keeps_persistent()) {
@@ -429,7 +456,7 @@ bool make_plan_uncached(int64_t T, int B, int n, int dtype, int want_mode, bool 
     if (!persistent_ok) {
       // Per-step launches have no co-residency limit: 4 cells per workgroup, groups of <= 64 rows.
       int MT = 1;
-      pl.regw = false;
+      pl.regw = pl.wide = false;
       pl.local = pl.half = false;
       pl.KSMAX = 0;
       // A step's launch takes W from memory straight into the matrix cores (every fragment is used once per launch).
@@ -471,6 +498,10 @@ bool make_plan_uncached(int64_t T, int B, int n, int dtype, int want_mode, bool 
   if (pl.kind == kPlanMfma) {
     pl.off_hx = off;
     off = align_up(off + (size_t)pl.groups_total * kHxRing * n * pl.Bp * es, 256);
+    if (pl.wide) {
+      pl.off_hxl = off;  // one set of copies, which the launches use in turn
+      off = align_up(off + (size_t)di.xcds * kHxRing * n * pl.Bp * es, 256);
+    }
     pl.off_wp = off;
     off = align_up(off + (size_t)4 * n * n * es, 256);
   } else {
@@ -807,7 +838,7 @@ int launch_steps_graph(const Lstm2Params& call, const Plan& pl, int dtype, hipSt
   shape.C = shape.d = nullptr;
   shape.hN = nullptr;
   shape.status = shape.flags = nullptr;
-  shape.hx = shape.Wp = shape.ycarry = nullptr;
+  shape.hx = shape.hxl = shape.Wp = shape.ycarry = nullptr;
   shape.trace = nullptr;
   key.append(reinterpret_cast<const char*>(&shape), sizeof(shape));
   key_append(&key, dtype); key_append(&key, pl.MT); key_append(&key, pl.NT); key_append(&key, (int)pl.kind);
@@ -1120,10 +1151,10 @@ int settle_fwd_plan(int count, int64_t T, int B, int nc, int n, int dtype, int m
   if (!make_plan(T, B, n, dtype, mode, capturing, &pl, &why, 2, plan_count))
     return fail(RTN_ERR_UNSUPPORTED, "NativeLstm2: persistent mode unavailable for T=%lld B=%d n=%d: %s", (long long)T, B, n, why.c_str());
   for (int attempt = 0; pl.kind == kPlanMfma && pl.mode == RTN_MODE_PERSISTENT; ++attempt) {
-    *pk = pl.regw ? (const void*)regw_kernel(dtype, pl.MT, pl.NT, pl.KSMAX, pl.half, nc % (int)(std::min<size_t>(16, 4 * pl.MT * esize(dtype)) / esize(dtype)) != 0) : (const void*)mfma_kernel(dtype, pl.MT, pl.NT);
+    *pk = pl.wide ? (const void*)pl.wide_build.kernel : pl.regw ? (const void*)regw_kernel(dtype, pl.MT, pl.NT, pl.KSMAX, pl.half, nc % (int)(std::min<size_t>(16, 4 * pl.MT * esize(dtype)) / esize(dtype)) != 0) : (const void*)mfma_kernel(dtype, pl.MT, pl.NT);
     if (!*pk) return fail(RTN_ERR_UNSUPPORTED, "NativeLstm2: no kernel for mt=%d nt=%d ks=%d", pl.MT, pl.NT, pl.KSMAX);
     if ((rc = ensure_lds_limit(*pk, pl.lds_bytes)) != RTN_OK) return rc;
-    const int wgs = pl.regw ? pl.grid : pl.groups * pl.wgs_per_group;
+    const int wgs = pl.regw || pl.wide ? pl.grid : pl.groups * pl.wgs_per_group;
     int per_cu = 0;
     if ((rc = occupancy_per_cu(*pk, kWgThreads, pl.lds_bytes, &per_cu)) != RTN_OK) return rc;
     const long long capacity = (long long)per_cu * device_info().cus;
@@ -1158,6 +1189,7 @@ int fill_fwd_params(const rtn_lstm2_call& c, const Plan& pl, bool persistent, un
   p.status = (unsigned*)(ws + pl.off_status);
   p.flags = (unsigned*)(ws + pl.off_flags);
   p.hx = ws + pl.off_hx;
+  p.hxl = pl.off_hxl ? ws + pl.off_hxl : nullptr;
   p.Wp = ws + pl.off_wp;
   p.ycarry = ws + pl.off_ycarry;
   p.trace = pl.off_trace ? (unsigned long long*)(ws + pl.off_trace) : nullptr;
@@ -1180,7 +1212,7 @@ int fill_fwd_params(const rtn_lstm2_call& c, const Plan& pl, bool persistent, un
   p.op_flags = op_flags;
   p.w_direct = (!persistent && pl.kind == kPlanMfma && pl.w_direct) ? 1 : 0;
   p.hx_bufs = kHxRing;
-  p.hx_sentinel = pl.regw ? 1 : 0;
+  p.hx_sentinel = pl.regw || pl.wide ? 1 : 0;
   p.exchange = (int)env_long("RTN_LSTM2_EXCHANGE", 0);
   if (p.exchange != kExNoWait) p.exchange = kExDevice;  // no-wait: a timing aid, results invalid (status 2)
   // Device-scope stores take about a microsecond to become visible: a first read issued at once would
@@ -1284,8 +1316,8 @@ int fwd_calls(const rtn_lstm2_call* calls, int count, int64_t T, int32_t B, int3
     }
 
     if (pl.kind == kPlanMfma) {
-      MfmaKernel mk = mfma_kernel(dtype, pl.MT, pl.NT);
       if (!pk) {
+        MfmaKernel mk = mfma_kernel(dtype, pl.MT, pl.NT);
         if (!mk) return fail(RTN_ERR_UNSUPPORTED, "NativeLstm2: no kernel for mt=%d nt=%d", pl.MT, pl.NT);
         rc = ensure_lds_limit((const void*)mk, pl.lds_bytes);
         if (rc != RTN_OK) return rc;
@@ -1300,6 +1332,21 @@ int fwd_calls(const rtn_lstm2_call* calls, int count, int64_t T, int32_t B, int3
         else
           hipLaunchKernelGGL(k_prepare_mfma<float>, pgrid, pblock, 0, stream, p, pl.n_flags);
         RTN_HIP(hipGetLastError());
+      }
+      if (pk && pl.wide) {
+        // the batch in turns, each on the whole device
+        for (int g0 = 0; g0 < pl.groups_total; ++g0) {
+          p.group_offset = g0;
+          p.groups = 1;
+          if (g0 > 0) {  // (the first turn's copies were armed by the preparation)
+            hipLaunchKernelGGL(k_fill_u32, dim3(512), dim3(256), 0, stream, (unsigned*)p.hxl, ~0u, (long long)((size_t)p.xcds * kHxRing * np * pl.Bp * esize(dtype) / 4));
+            RTN_HIP(hipGetLastError());
+          }
+          void* args[] = {(void*)&p};
+          rc = launch_coresident(pk, dim3(pl.grid), dim3(kWgThreads), args, (unsigned)pl.lds_bytes, stream, capturing);
+          if (rc != RTN_OK) return rc;
+        }
+        continue;
       }
       if (pk && pl.regw && pl.passes > 1) {
         // the batch groups in turns: one persistent launch per share of them
@@ -1590,8 +1637,8 @@ const char* rtn_native_lstm2_describe_multi_plan(int32_t count, int64_t T, int32
   } else {
     snprintf(buf, sizeof(buf), "mode=%s kernel=%s mt=%d nt=%d groups=%d wgs_per_group=%d wgs=%d rows_per_group=%d launches=%d lds=%zu workspace=%zu",
              mode_name(pl.mode),
-             pl.kind == kPlanMfma ? (pl.regw ? (pl.local ? (pl.half ? "mfma_regw_xcd_half" : "mfma_regw_xcd") : "mfma_regw") : "mfma_lds") : (pl.kind == kPlanGeneric ? "generic" : "empty"), pl.MT,
-             pl.NT, pl.groups, pl.wgs_per_group, (pl.mode == RTN_MODE_PERSISTENT && pl.regw) ? pl.grid : pl.groups * pl.wgs_per_group,
+             pl.kind == kPlanMfma ? (pl.wide ? "mfma_wide" : pl.regw ? (pl.local ? (pl.half ? "mfma_regw_xcd_half" : "mfma_regw_xcd") : "mfma_regw") : "mfma_lds") : (pl.kind == kPlanGeneric ? "generic" : "empty"), pl.MT,
+             pl.NT, pl.groups, pl.wgs_per_group, (pl.mode == RTN_MODE_PERSISTENT && (pl.regw || pl.wide)) ? pl.grid : pl.groups * pl.wgs_per_group,
              pl.Bg, pl.passes, pl.lds_bytes,
              (count > 1 || n != n_asked) ? workspace_each(count, T, B, n_asked, dtype, mode) : pl.total);
     if (n != n_asked) snprintf(buf + strlen(buf), sizeof(buf) - strlen(buf), " padded_width=%d", n);

@@ -1,0 +1,63 @@
+"""The kernel for layers whose recurrent weights take the registers and the LDS of the whole device, against per-step
+launches, bit for bit."""
+
+from __future__ import annotations
+
+import numpy
+import pytest
+
+from returnn_amd import lib
+
+from _gpu_util import announce, env, random_problem, run_raw
+
+pytestmark = pytest.mark.gpu
+
+# the narrowest and the widest layer of every build, few rows, full and partly filled turns, an odd width
+CASES = [
+    (7, 16, 4096, "bf16", 0, 1), (6, 1, 4096, "bf16", 0, -1), (5, 37, 3104, "bf16", 1, 1), (6, 32, 3072, "bf16", 0, 1), (5, 17, 2080, "bf16", 0, -2),
+    (6, 50, 2399, "bf16", 0, 1), (6, 3, 1056, "f32", 0, 1), (5, 33, 2048, "f32", 0, -1), (5, 16, 2816, "f32", 0, 1), (4, 19, 2080, "f32", 1, 1),
+]  # fmt: skip
+
+
+@pytest.mark.parametrize("T,B,n,dtype,start,step", CASES)
+def test_wide_layers_equal_per_step_launches(T, B, n, dtype, start, step):
+    announce("wide kernel", T, B, n, dtype, start, step)
+    p = random_problem(7000 + n + B, T, B, n)
+    i = (numpy.random.default_rng(n).uniform(size=(T, B)) < 0.8).astype(numpy.float32)
+    p = (*p[:4], i)
+    rc, status, want = run_raw(*p, start, step, dtype=dtype, mode="stepwise")
+    assert rc == 0 and status == 0
+    rc, status, got = run_raw(*p, start, step, dtype=dtype)
+    plan = lib.describe_plan(T, B, n, lib.DTYPE_BF16 if dtype == "bf16" else lib.DTYPE_F32, lib.MODE_AUTO)
+    assert "kernel=mfma_wide" in plan, plan
+    assert rc == 0 and status == 0
+    for name, a, b in zip("YCHd", got, want):
+        assert numpy.isfinite(a).all(), name
+        assert numpy.array_equal(a, b), "%s differs from per-step launches (%s)" % (name, plan)
+
+
+def test_wrong_xcd_count_exchanges_at_device_scope():
+    announce("wide kernel with a wrong XCD count")
+    p = random_problem(71, 6, 5, 2304)
+    rc, status, want = run_raw(*p, 0, 1, dtype="bf16", mode="stepwise")
+    assert rc == 0 and status == 0
+    with env(RTN_LSTM2_XCDS=4):
+        rc, status, got = run_raw(*p, 0, 1, dtype="bf16")
+    assert rc == 0 and status == 0
+    for name, a, b in zip("YCHd", got, want):
+        assert numpy.array_equal(a, b), name
+
+
+def test_bounded_wait_expires_cleanly():
+    announce("wide kernel, bounded wait")
+    p = random_problem(72, 9, 4, 2304)
+    with env(RTN_LSTM2_TIMEOUT_TICKS=0):
+        rc, status, got = run_raw(*p, 0, 1, dtype="bf16")
+    assert rc == 0 and status in (lib.RTN_OK, lib.RTN_ERR_ABORTED)
+    if status == lib.RTN_ERR_ABORTED:
+        assert numpy.isnan(got[3]).any() and numpy.isnan(got[0][-1]).any()
+    rc, status, got = run_raw(*p, 0, 1, dtype="bf16")
+    rc2, status2, want = run_raw(*p, 0, 1, dtype="bf16", mode="stepwise")
+    assert (rc, status, rc2, status2) == (0, 0, 0, 0)
+    for name, a, b in zip("YCHd", got, want):
+        assert numpy.array_equal(a, b), name
