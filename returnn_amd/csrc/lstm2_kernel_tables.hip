@@ -101,7 +101,7 @@ WideBuild wide_kernel(int dtype, int n, int cus, int rows) {
 #define RTN_WIDE(at, dt, mt, nt, ks, lf) {&k_lstm2_wide<at, mt, nt, ks, lf>, dt, mt, nt, ks, lf}
   static const WideBuild builds[] = {
       RTN_WIDE(float, 0, 2, 1, 32, 0), RTN_WIDE(float, 0, 2, 2, 32, 0), RTN_WIDE(float, 0, 3, 1, 44, 36),
-      RTN_WIDE(__bf16, 1, 3, 1, 24, 0), RTN_WIDE(__bf16, 1, 3, 2, 24, 0), RTN_WIDE(__bf16, 1, 4, 1, 32, 32),
+      RTN_WIDE(__bf16, 1, 3, 1, 24, 0), RTN_WIDE(__bf16, 1, 3, 2, 24, 0), RTN_WIDE(__bf16, 1, 4, 1, 32, 35),
   };
 #undef RTN_WIDE
   WideBuild best = {nullptr, 0, 0, 0, 0, 0};

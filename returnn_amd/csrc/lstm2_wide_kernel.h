@@ -26,10 +26,21 @@ namespace rtn {
 //    all of h_s, so every workgroup has finished step s-1, so every XCD had brought h_{s-1} over.
 //  * ring of the XCD: a workgroup that brings its part of h_s over re-arms its part of h_{s-2}: it has seen all of h_{s-1}
 //    there, of which every workgroup of the XCD brought its part when it had finished reading h_{s-2}.
-// A re-arm is acknowledged (vmcnt(0) in front of the next publication) before anything that lets a reader ask for that slot.
+// A re-arm is acknowledged before anything that lets a reader ask for that slot: between it and the wavefront's next stores
+// into the same ring lies the wait for the loads that bring the next h over, and a wavefront's memory operations are
+// waited for in their order.
 // That the workgroups id % xcds share an XCD is checked at the start; if not, the copies are stored at device scope.
 // Waits are bounded as everywhere.
 // ---------------------------------------------------------------------------------------------
+// Fragments in LDS of a wavefront in the order the product takes them: how many come before tile mt of macro step ks.
+constexpr int wide_lds_slot(int MT, int KS, int RF, int ks, int mt) {
+  int count = 0;
+  for (int k = 0; k <= ks; ++k)
+    for (int m = 0; m < MT; ++m)
+      if ((k < ks || m < mt) && m * KS + k >= RF) ++count;
+  return count;
+}
+
 constexpr unsigned wide_lds_bytes(int MT, int NT, int LF) {
   return (unsigned)(kWaves * LF * kTileBytes + kWaves * MT * NT * kTileBytes);
 }
@@ -44,7 +55,7 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_wide(const Lstm2Params p) 
   using LM = LaneMax<AT>;
   constexpr int KE = E::KE, KM = E::KM, ES = (int)sizeof(AT);
   constexpr int TILES = MT * NT, EPT = (TILES + kWaves - 1) / kWaves, RF = MT * KS - LF;
-  constexpr int CH = NT == 1 ? 4 : 2, NC = KS / CH;  // macro steps of h per chunk, chunks
+      constexpr int CH = NT == 1 ? 4 : 2, NB = 3, NC = KS / CH;  // macro steps of h per chunk, chunks in flight, chunks
   static_assert(KS % CH == 0 && LF >= 0 && RF > 0, "fragment counts");
 
   extern __shared__ __align__(16) unsigned char smem[];
@@ -78,7 +89,7 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_wide(const Lstm2Params p) 
     if (f < RF)
       wreg[f] = v;
     else
-      Wl[(wave * LF + f - RF) * 64 + lane] = v;
+      Wl[(wave * LF + wide_lds_slot(MT, KS, RF, ks, mt)) * 64 + lane] = v;
   }
 
   // The (row, cell) pairs whose state this thread keeps.
@@ -108,9 +119,11 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_wide(const Lstm2Params p) 
     const int q = tid + kWgThreads * i, f = member * part + q;
     f_off[i] = q < part && f < frags && f % p.Bp < rows ? (unsigned)(f * kFragBytes) : kOobOffset;
   }
-  unsigned b_off[NT];  // this lane's fragment of macro step `wave`
+  // This lane's fragment of macro step `wave`.  Lanes of rows that do not exist load beyond the buffer (zeros): a branch around
+  // the loads would have the compiler wait for all of them at every use, since any of them could be the last one issued.
+  unsigned b_off[NT];
 #pragma unroll
-  for (int nt = 0; nt < NT; ++nt) b_off[nt] = (unsigned)(((4 * wave + kg) * p.Bp + 16 * nt + jl) * kFragBytes);
+  for (int nt = 0; nt < NT; ++nt) b_off[nt] = 16 * nt + jl < rows ? (unsigned)(((4 * wave + kg) * p.Bp + 16 * nt + jl) * kFragBytes) : kOobOffset;
   const unsigned ks_stride = (unsigned)(4 * kWaves * p.Bp * kFragBytes);  // from one macro step of the share to the next
 
   __shared__ int s_one_xcd;
@@ -118,21 +131,70 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_wide(const Lstm2Params p) 
   __syncthreads();
   const bool one_xcd = s_one_xcd != 0;
 
-  AT xin[EPT][4];
-  float msk[EPT];
+  // The op's streams, a pair per thread: gate inputs and mask come in one step ahead, behind the loads of the product; a step's
+  // outputs leave behind the next step's.  Without a branch: pairs and frames that do not exist have offsets beyond any
+  // frame.  (With branches the compiler has to wait for these loads and stores, and the
+  // trip to memory they take, wherever it waits for a chunk of h.)
+  unsigned x_at[EPT], h_at[EPT], y_at[EPT], c_at[EPT], m_at[EPT];  // byte offsets inside a frame
+#pragma unroll
+  for (int j = 0; j < EPT; ++j) {
+    const long long row = b_base + e_b[j];
+    x_at[j] = e_valid[j] ? (unsigned)((row * p.ldX + e_cell[j]) * ES) : kOobOffset;
+    h_at[j] = e_valid[j] ? (unsigned)((row * 4 * nc + e_cell[j]) * ES) : kOobOffset;
+    y_at[j] = e_valid[j] ? (unsigned)((row * p.ldY + e_cell[j]) * ES) : kOobOffset;
+    c_at[j] = e_valid[j] ? (unsigned)((row * nc + e_cell[j]) * 4) : kOobOffset;
+    m_at[j] = e_valid[j] ? (unsigned)(row * 4) : kOobOffset;
+  }
+  const unsigned frame_x = (unsigned)((size_t)p.B * p.ldX * ES), frame_h = (unsigned)((size_t)p.B * 4 * nc * ES), frame_y = (unsigned)((size_t)p.B * p.ldY * ES),
+                 frame_c = (unsigned)(bn * 4), frame_m = (unsigned)(p.B * 4), gate = (unsigned)(nc * ES);  // (gate: from one of a row's four blocks to the next)
+  AT xin[EPT][4], xnext[EPT][4];
+  float msk[EPT], mnext[EPT];
+  // (frames that do not exist: all offsets beyond; not a buffer of no bytes, whose range check a scalar offset would wrap)
+  auto frame = [&](const void* base, int s, unsigned bytes, bool there) {
+    return __builtin_amdgcn_make_buffer_rsrc((unsigned char*)base + (there ? frame_of(p, s) : 0) * (long long)bytes, 0, bytes, kBufFlags);
+  };
   auto fetch = [&](int s) {
-    const size_t t = (size_t)frame_of(p, s);
+    const bool there = s < nsteps;
+    __amdgpu_buffer_rsrc_t xr = frame(p.X, s, frame_x, there), mr = frame(p.mask, s, frame_m, there);
 #pragma unroll
     for (int j = 0; j < EPT; ++j) {
-      msk[j] = 0.f;
+      const unsigned at = there ? x_at[j] : kOobOffset;
 #pragma unroll
-      for (int q = 0; q < 4; ++q) xin[j][q] = (AT)0.f;
-      if (e_valid[j]) {
-        const AT* xp = (const AT*)p.X + (t * p.B + b_base + e_b[j]) * (size_t)p.ldX + e_cell[j];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) xin[j][q] = xp[(size_t)q * nc];
-        msk[j] = p.mask[t * p.B + b_base + e_b[j]];
+      for (int q = 0; q < 4; ++q) {
+        if constexpr (ES == 2)
+          xnext[j][q] = __builtin_bit_cast(AT, __builtin_amdgcn_raw_buffer_load_b16(xr, at, q * gate, 0));
+        else
+          xnext[j][q] = __builtin_bit_cast(AT, __builtin_amdgcn_raw_buffer_load_b32(xr, at, q * gate, 0));
       }
+      mnext[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(mr, there ? m_at[j] : kOobOffset, 0, 0));
+    }
+  };
+  auto take = [&]() {
+#pragma unroll
+    for (int j = 0; j < EPT; ++j) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) xin[j][q] = xnext[j][q];
+      msk[j] = mnext[j];
+    }
+  };
+  AT a_out[EPT][4], y_out[EPT];
+#pragma unroll
+  for (int j = 0; j < EPT; ++j) a_out[j][0] = a_out[j][1] = a_out[j][2] = a_out[j][3] = y_out[j] = (AT)0.f;
+  auto put = [&](int s) {
+    const bool there = s >= 0;
+    __amdgpu_buffer_rsrc_t hr = frame(p.H, s, frame_h, there), yr = frame(p.Y, s, frame_y, there), cr = frame(p.C, s, frame_c, there);
+    auto store = [&](AT v, __amdgpu_buffer_rsrc_t rs, unsigned off, unsigned block) {
+      if constexpr (ES == 2)
+        __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(unsigned short, v), rs, off, block, 0);
+      else
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), rs, off, block, 0);
+    };
+#pragma unroll
+    for (int j = 0; j < EPT; ++j) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) store(a_out[j][q], hr, there ? h_at[j] : kOobOffset, q * gate);
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, c_state[j]), cr, there ? c_at[j] : kOobOffset, 0, 0);
+      store(y_out[j], yr, there ? y_at[j] : kOobOffset, 0);
     }
   };
   // Bookkeeping of one repeated read: false when the wait is over for good.
@@ -150,22 +212,18 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_wide(const Lstm2Params p) 
     }
     return true;
   };
-  auto incomplete = [&](const i32x4* v, int count) {
-    unsigned m[4] = {0, 0, 0, 0};
+  // Running maxima over the elements of fragments, and whether one of them was not written yet.
+  auto fold = [&](unsigned (&m)[4], const i32x4& v) {
 #pragma unroll
-    for (int i = 0; i < count; ++i)
-#pragma unroll
-      for (int w = 0; w < 4; ++w) m[w] = LM::fold(m[w], (unsigned)v[i][w]);
-    return __any(LM::has_sentinel(LM::fold(LM::fold(m[0], m[1]), LM::fold(m[2], m[3])))) != 0;
+    for (int w = 0; w < 4; ++w) m[w] = LM::fold(m[w], (unsigned)v[w]);
   };
+  auto seen_mark = [&](const unsigned (&m)[4]) { return __any(LM::has_sentinel(LM::fold(LM::fold(m[0], m[1]), LM::fold(m[2], m[3])))) != 0; };
 
-  i32x4 bf[2][CH * NT];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int u = 0; u < CH * NT; ++u) bf[i][u] = i32x4{0, 0, 0, 0};
+  i32x4 bf[NB][CH * NT];
   fetch(0);
+  take();
   int delay = p.poll_delay;
+  RTN_TRACE_DECL
   for (int s = 0; s < nsteps; ++s) {
     const unsigned slot = (unsigned)(s & (kHxRing - 1)) * slot_bytes, old = (unsigned)((s + 2) & (kHxRing - 1)) * slot_bytes;
     // ---- bring this workgroup's part of h_s over
@@ -174,12 +232,19 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_wide(const Lstm2Params p) 
       unsigned spins = 0;
       if (s > 0)
         for (int k = 0; k < delay; ++k) __builtin_amdgcn_s_sleep(1);
+      bool again;
       do {
         asm volatile("" ::: "memory");
+        unsigned m[4] = {0, 0, 0, 0};
 #pragma unroll
         for (int i = 0; i < kWideForward; ++i)
           fv[i] = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(ring, f_off[i], slot, kAuxDevice));
-      } while (incomplete(fv, kWideForward) && keep_waiting(spins));
+#pragma unroll
+        for (int i = 0; i < kWideForward; ++i) fold(m, fv[i]);
+        again = seen_mark(m) && keep_waiting(spins);
+      } while (again);
+      RTN_TRACE_MARK(0)  // h_s arrives across the XCDs
+      RTN_TRACE_ADD(6, spins)
       // (a repeated read costs a trip to memory: the delay in front of the first adapts, as in k_lstm2_regw)
       if (spins)
         delay = min(delay + p.delay_inc, 64);
@@ -197,19 +262,18 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_wide(const Lstm2Params p) 
         }
       }
     }
-    // ---- the product, chunk by chunk
+    // ---- the product, chunk by chunk; a chunk is checked behind the MFMAs of the one before (checked in front of its own, with
+    // the matrix core idle meanwhile, each of them cost 0.1 us)
     auto load_chunk = [&](int c) {
       asm volatile("" ::: "memory");
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt)
-        if (16 * nt + jl < rows) {
 #pragma unroll
-          for (int u = 0; u < CH; ++u) {
-            const int ks = c * CH + u;
-            // (past the share: any complete fragment, against zeros of W)
-            bf[c & 1][u * NT + nt] =
-                __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(local, b_off[nt], slot + (ks < ks_count ? (unsigned)ks : 0u) * ks_stride, kAuxDevice));
-          }
+        for (int u = 0; u < CH; ++u) {
+          const int ks = c * CH + u;
+          // (past the share: any complete fragment, against zeros of W)
+          bf[c % NB][u * NT + nt] =
+              __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(local, b_off[nt], slot + (ks < ks_count ? (unsigned)ks : 0u) * ks_stride, kAuxDevice));
         }
     };
     f32x4 acc[MT][NT];
@@ -217,43 +281,83 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_wide(const Lstm2Params p) 
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    load_chunk(0);
     unsigned spins = 0;
+    auto complete = [&](int c, bool mark) {  // read chunk c again until it is complete
+      while (mark && keep_waiting(spins)) {
+        load_chunk(c);
+        unsigned m[4] = {0, 0, 0, 0};
+#pragma unroll
+        for (int u = 0; u < CH * NT; ++u) fold(m, bf[c % NB][u]);
+        mark = seen_mark(m);
+      }
+    };
+    load_chunk(0);
+    // the fragments in LDS are read WP ahead of their MFMA (read where they are needed, each of them cost 80 clocks)
+    constexpr int WP = LF ? 2 : 1;
+    i32x4 wl[WP];
+    if constexpr (LF > 0) {
+#pragma unroll
+      for (int i = 0; i < WP; ++i) wl[i] = Wl[(wave * LF + i) * 64 + lane];
+    }
+    {
+      unsigned m[4] = {0, 0, 0, 0};
+#pragma unroll
+      for (int u = 0; u < CH * NT; ++u) fold(m, bf[0][u]);
+      complete(0, seen_mark(m));
+    }
+    // (the others behind it: asked for together with the first one, they are in the way of its repeats)
+#pragma unroll
+    for (int c = 1; c < NB - 1; ++c) load_chunk(c);
+    RTN_TRACE_MARK(1)  // brought over, first chunk back
+    RTN_TRACE_ADD(7, spins)
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
-      if (c + 1 < NC) load_chunk(c + 1);
-      while (incomplete(bf[c & 1], CH * NT) && keep_waiting(spins)) load_chunk(c);
+      if (c + NB - 1 < NC) load_chunk(c + NB - 1);
+      if (c + NB - 1 == NC - 1 || (NC < NB && c == 0)) {
+        put(s - 1);
+        fetch(s + 1);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      unsigned m[4] = {0, 0, 0, 0};
 #pragma unroll
-      for (int u = 0; u < CH; ++u)
+      for (int u = 0; u < CH; ++u) {
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
-          const int f = mt * KS + c * CH + u;
-          const i32x4 a = f < RF ? wreg[f < RF ? f : 0] : Wl[(wave * LF + f - RF) * 64 + lane];
+          const int f = mt * KS + c * CH + u, q = wide_lds_slot(MT, KS, RF, c * CH + u, mt);
+          const i32x4 a = f < RF ? wreg[f < RF ? f : 0] : wl[q % WP];
 #pragma unroll
-          for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = E::mma(a, bf[c & 1][u * NT + nt], acc[mt][nt]);
+          for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = E::mma(a, bf[c % NB][u * NT + nt], acc[mt][nt]);
+          if (f >= RF && q + WP < LF) wl[q % WP] = Wl[(wave * LF + q + WP) * 64 + lane];
         }
+        if (c + 1 < NC)
+#pragma unroll
+          for (int nt = 0; nt < NT; ++nt) fold(m, bf[(c + 1) % NB][u * NT + nt]);
+      }
+      const bool mark = c + 1 < NC && seen_mark(m);
       __builtin_amdgcn_sched_barrier(0);
+      if (c + 1 < NC) complete(c + 1, mark);
     }
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) red[(wave * TILES + mt * NT + nt) * 64 + lane] = acc[mt][nt];
-    // everything this wavefront stored before (re-arms included) is acknowledged before its new values go out
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-    asm volatile("" ::: "memory");
+    RTN_TRACE_MARK(2)  // product
     __syncthreads();
+    RTN_TRACE_MARK(3)  // barrier
 
     // ---- gates and cell update, new hidden values out
-    float a_out[EPT][4], y_out[EPT];
     const unsigned nxt = (unsigned)((s + 1) & (kHxRing - 1)) * slot_bytes, arm = (unsigned)((s + 3) & (kHxRing - 1)) * slot_bytes;
 #pragma unroll
     for (int j = 0; j < EPT; ++j) {
       const int e = wave + kWaves * j;
-      y_out[j] = a_out[j][0] = a_out[j][1] = a_out[j][2] = a_out[j][3] = 0.f;
       if (e < TILES) {
-        f32x4 gsum = red[e * 64 + lane];
+        f32x4 part[kWaves];
 #pragma unroll
-        for (int w = 1; w < kWaves; ++w) gsum += red[(w * TILES + e) * 64 + lane];
+        for (int w = 0; w < kWaves; ++w) part[w] = red[(w * TILES + e) * 64 + lane];
+        __builtin_amdgcn_sched_barrier(0);
+        f32x4 gsum = part[0];
+#pragma unroll
+        for (int w = 1; w < kWaves; ++w) gsum += part[w];
         const float m = msk[j];
         const float a0 = Act<AT>::tanh(gsum[0] + (float)xin[j][0]);
         const float a1 = Act<AT>::sigmoid(gsum[1] + (float)xin[j][1]);
@@ -265,9 +369,9 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_wide(const Lstm2Params p) 
         const float hn = (p.op_flags & kOpNoCarry) ? y : E::round(y + h_prev[j] * (1.f - m));
         c_state[j] = c;
         h_prev[j] = hn;
-        y_out[j] = y;
-        a_out[j][0] = (p.op_flags & kOpH0IsCell) ? c : a0;
-        a_out[j][1] = a1; a_out[j][2] = a2; a_out[j][3] = a3;
+        y_out[j] = (AT)y;
+        a_out[j][0] = (AT)((p.op_flags & kOpH0IsCell) ? c : a0);
+        a_out[j][1] = (AT)a1; a_out[j][2] = (AT)a2; a_out[j][3] = (AT)a3;
         if (e_own[j]) {
           const unsigned ho = (unsigned)((((e_cell[j] / KE) * p.Bp + e_b[j]) * KE + (e_cell[j] % KE)) * ES);
           SN::template store<kAuxDevice>(ring, ho + nxt, SN::bits(hn));
@@ -275,20 +379,14 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_wide(const Lstm2Params p) 
         }
       }
     }
-    // ---- while they travel: the op's outputs, and the next step's inputs
-    const size_t t = (size_t)frame_of(p, s);
-#pragma unroll
-    for (int j = 0; j < EPT; ++j)
-      if (e_valid[j]) {
-        const size_t row = t * p.B + b_base + e_b[j];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) E::store(p.H, row * 4 * nc + (size_t)q * nc + e_cell[j], a_out[j][q]);
-        p.C[row * nc + e_cell[j]] = c_state[j];
-        E::store(p.Y, row * (size_t)p.ldY + e_cell[j], y_out[j]);
-      }
-    if (s + 1 < nsteps) fetch(s + 1);
+    RTN_TRACE_MARK(4)  // gates, new values out
+    take();
     __syncthreads();  // `red` may take the next step's partial tiles
+    RTN_TRACE_MARK(5)  // next inputs, barrier
   }
+  RTN_TRACE_FLUSH(p, blockIdx.x)
+
+  put(nsteps - 1);
 
   // after a wait that ran into its bound: NaN as the final cell state and in the last visited frame of Y
   const bool expired = wait_expired(p.status);

@@ -29,7 +29,7 @@ def test_wide_layers_equal_per_step_launches(T, B, n, dtype, start, step):
     assert rc == 0 and status == 0
     rc, status, got = run_raw(*p, start, step, dtype=dtype)
     plan = lib.describe_plan(T, B, n, lib.DTYPE_BF16 if dtype == "bf16" else lib.DTYPE_F32, lib.MODE_AUTO)
-    assert "kernel=mfma_wide" in plan, plan
+    assert "kernel=mfma_regw_wide" in plan, plan
     assert rc == 0 and status == 0
     for name, a, b in zip("YCHd", got, want):
         assert numpy.isfinite(a).all(), name
