@@ -6,6 +6,7 @@
 
 #include "lstm2_bwd_kernels.h"
 #include "lstm2_kernels.h"
+#include "lstm2_solo_kernel.h"
 #include "lstm2_wide_kernel.h"
 
 namespace rtn {
@@ -19,6 +20,13 @@ RegwKernel regw_table_bf16_lo(int MT, int NT, int KSMAX, bool half, bool tail);
 RegwKernel regw_table_bf16_hi(int MT, int NT, int KSMAX, bool half, bool tail);
 RegwKernel regw_table_f32_lo(int MT, int NT, int KSMAX, bool half, bool tail);
 RegwKernel regw_table_f32_hi(int MT, int NT, int KSMAX, bool half, bool tail);
+
+// Forward kernel for small layers k_lstm2_solo<AT, S>: the build for width n; kernel null: none.
+struct SoloBuild {
+  RegwKernel kernel;
+  int threads;
+};
+SoloBuild solo_kernel(int dtype, int n);
 
 // Forward kernel for wide layers k_lstm2_wide<AT, MT, NT, KS, LF>.
 typedef void (*WideKernel)(const Lstm2Params);

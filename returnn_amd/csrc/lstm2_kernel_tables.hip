@@ -115,6 +115,17 @@ WideBuild wide_kernel(int dtype, int n, int cus, int rows) {
   }
   return best;
 }
+// float32 up to n = 128, bf16 up to 160: what the wavefronts' registers hold without spilling.
+SoloBuild solo_kernel(int dtype, int n) {
+#define RTN_SOLO(at, s) if (n <= s * Elem<at>::KM) return {&k_lstm2_solo<at, s>, 64 * solo_waves<at>(s)};
+  if (dtype == 1) {
+    RTN_SOLO(__bf16, 1) RTN_SOLO(__bf16, 2) RTN_SOLO(__bf16, 3) RTN_SOLO(__bf16, 4) RTN_SOLO(__bf16, 5)
+  } else {
+    RTN_SOLO(float, 2) RTN_SOLO(float, 4) RTN_SOLO(float, 6) RTN_SOLO(float, 8)
+  }
+#undef RTN_SOLO
+  return {nullptr, 0};
+}
 #else
 #error "RTN_TABLE_PART must be 1..9"
 #endif

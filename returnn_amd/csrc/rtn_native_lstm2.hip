@@ -163,7 +163,7 @@ DeviceInfo device_info() {
   return di;
 }
 
-enum PlanKind { kPlanEmpty, kPlanGeneric, kPlanMfma };
+enum PlanKind { kPlanEmpty, kPlanGeneric, kPlanMfma, kPlanSolo };
 
 struct Plan {
   PlanKind kind = kPlanGeneric;
@@ -172,6 +172,8 @@ struct Plan {
   bool local = false;            // regw: every batch group on one XCD, hidden state exchanged through that XCD's L2
   bool wide = false;             // persistent kernel for layers whose W takes registers and LDS of the whole device
   WideBuild wide_build = {nullptr, 0, 0, 0, 0, 0};
+  bool solo = false;             // small layer: every workgroup takes 4 rows through all steps by itself
+  SoloBuild solo_build = {nullptr, 0};
   bool half = false;             // regw: groups of at most 8 rows, two tiles folded into one pass of the pointwise part
   int grid = 0;                  // workgroups launched by the persistent kernel
   int KSMAX = 0;                 // its macro steps per wavefront (template bound)
@@ -226,7 +228,18 @@ bool make_plan_uncached(int64_t T, int B, int n, int dtype, int want_mode, bool 
   const bool mfma_shape = (n % 32) == 0;
   const long force_generic = env_long("RTN_LSTM2_FORCE_GENERIC", 0);
   bool persistent_ok = false;
-  if (mfma_shape && !force_generic) {
+  // A small layer whose rows find a CU per four: no workgroup needs another one.  (A batch beyond that keeps several rows per
+  // tile busy on the kernels below; a decomposition or kernel asked for by the environment is one of theirs.)
+  if (want_mode == RTN_MODE_AUTO && di.valid && !force_generic && B <= kSoloRows * di.cus / std::max(1, std::min(count, kMaxMulti)) && !env_long("RTN_LSTM2_NO_PAD", 0) &&
+      !env_long("RTN_LSTM2_MT", 0) && !env_long("RTN_LSTM2_GROUPS", 0) && !env_long("RTN_LSTM2_KERNEL", 0) && env_long("RTN_LSTM2_LOCAL", -1) < 0 && !env_long("RTN_LSTM2_NO_SOLO", 0))
+    pl.solo_build = solo_kernel(dtype, n);
+  if (pl.solo_build.kernel) {
+    pl.kind = kPlanSolo;
+    pl.solo = true;
+    pl.grid = pl.groups = pl.groups_total = (B + kSoloRows - 1) / kSoloRows;
+    pl.Bg = kSoloRows;
+    persistent_ok = true;
+  } else if (mfma_shape && !force_generic) {
     pl.kind = kPlanMfma;
     // Persistent candidates: every (MT, groups) whose grid fits the device with W on chip.  The register
     // kernel is preferred; among its candidates the estimated step time decides: MFMA cycles of one
@@ -427,7 +440,7 @@ bool make_plan_uncached(int64_t T, int B, int n, int dtype, int want_mode, bool 
         const int G = wb.kernel ? (n / 4 + wb.MT - 1) / wb.MT : 0;
         const long env_passes = env_long("RTN_LSTM2_MAX_PASSES", -1);
         const size_t lds = wb.kernel ? wide_lds_bytes(wb.MT, wb.NT, wb.LF) + 64 : 0;
-        if (wb.kernel && turns <= (env_passes >= 0 ? env_passes : kMaxPassesOverSteps) && lds <= di.lds_per_wg && G >= 2 * di.xcds &&
+        if (wb.kernel && turns <= (env_passes >= 0 ? env_passes : kMaxPassesOverSteps * 4) && lds <= di.lds_per_wg && G >= 2 * di.xcds &&
             (n / (dtype == RTN_DTYPE_BF16 ? 8 : 4) * rows + G / di.xcds - 1) / (G / di.xcds) <= kWideForward * kWgThreads) {
           pl = Plan();
           pl.kind = kPlanMfma;
@@ -504,7 +517,7 @@ bool make_plan_uncached(int64_t T, int B, int n, int dtype, int want_mode, bool 
     }
     pl.off_wp = off;
     off = align_up(off + (size_t)4 * n * n * es, 256);
-  } else {
+  } else if (pl.kind != kPlanSolo) {
     pl.off_ycarry = off;
     off = align_up(off + (size_t)2 * B * n * es, 256);
   }
@@ -1304,6 +1317,9 @@ int fwd_calls(const rtn_lstm2_call* calls, int count, int64_t T, int32_t B, int3
     if ((rc = fill_fwd_params(calls[k], pl, pk != nullptr, (unsigned char*)workspace + (size_t)k * each_ws, T, B, n, np, dtype, op_flags, &p)) != RTN_OK)
       return rc;
 
+    if (pl.solo) {
+      multi.p[pending++] = p;
+    }
     // Frames the loop never visits.
     if (p.nsteps != T) {
       const long long total = T * bn * 4;
@@ -1315,6 +1331,15 @@ int fwd_calls(const rtn_lstm2_call* calls, int count, int64_t T, int32_t B, int3
       RTN_HIP(hipGetLastError());
     }
 
+    if (pl.solo) {
+      if (pending == kMaxMulti || k + 1 == count) {
+        multi.count = pending;
+        hipLaunchKernelGGL(pl.solo_build.kernel, dim3((unsigned)pl.grid, (unsigned)pending), dim3((unsigned)pl.solo_build.threads), 0, stream, multi);
+        RTN_HIP(hipGetLastError());
+        pending = 0;
+      }
+      continue;
+    }
     if (pl.kind == kPlanMfma) {
       if (!pk) {
         MfmaKernel mk = mfma_kernel(dtype, pl.MT, pl.NT);
@@ -1637,8 +1662,8 @@ const char* rtn_native_lstm2_describe_multi_plan(int32_t count, int64_t T, int32
   } else {
     snprintf(buf, sizeof(buf), "mode=%s kernel=%s mt=%d nt=%d groups=%d wgs_per_group=%d wgs=%d rows_per_group=%d launches=%d lds=%zu workspace=%zu",
              mode_name(pl.mode),
-             pl.kind == kPlanMfma ? (pl.wide ? "mfma_regw_wide" : pl.regw ? (pl.local ? (pl.half ? "mfma_regw_xcd_half" : "mfma_regw_xcd") : "mfma_regw") : "mfma_lds") : (pl.kind == kPlanGeneric ? "generic" : "empty"), pl.MT,
-             pl.NT, pl.groups, pl.wgs_per_group, (pl.mode == RTN_MODE_PERSISTENT && (pl.regw || pl.wide)) ? pl.grid : pl.groups * pl.wgs_per_group,
+             pl.solo ? "mfma_regw_solo" : pl.kind == kPlanMfma ? (pl.wide ? "mfma_regw_wide" : pl.regw ? (pl.local ? (pl.half ? "mfma_regw_xcd_half" : "mfma_regw_xcd") : "mfma_regw") : "mfma_lds") : (pl.kind == kPlanGeneric ? "generic" : "empty"), pl.MT,
+             pl.NT, pl.groups, pl.wgs_per_group, (pl.mode == RTN_MODE_PERSISTENT && (pl.regw || pl.wide || pl.solo)) ? pl.grid : pl.groups * pl.wgs_per_group,
              pl.Bg, pl.passes, pl.lds_bytes,
              (count > 1 || n != n_asked) ? workspace_each(count, T, B, n_asked, dtype, mode) : pl.total);
     if (n != n_asked) snprintf(buf + strlen(buf), sizeof(buf) - strlen(buf), " padded_width=%d", n);
