@@ -115,13 +115,15 @@ WideBuild wide_kernel(int dtype, int n, int cus, int rows) {
   }
   return best;
 }
-// float32 up to n = 128, bf16 up to 160: what the wavefronts' registers hold without spilling.
+// float32 up to n = 64, bf16 up to 128.  Measured at T = 500, B = 4 ... 256, us per step, against k_lstm2_regw: float32 n = 32 / 64
+// 0.63 / 0.73 against 1.03; n = 96 / 128 (8 wavefronts' MFMAs on one CU) would take 1.36 / 1.64 against 1.03; bf16 n = 32 / 64 / 96
+// / 128 0.41 / 0.55 / 0.71 / 0.87 against 0.83 (and 5 us less for not packing W); n = 160 would take 1.7 against 0.85.
 SoloBuild solo_kernel(int dtype, int n) {
 #define RTN_SOLO(at, s) if (n <= s * Elem<at>::KM) return {&k_lstm2_solo<at, s>, 64 * solo_waves<at>(s)};
   if (dtype == 1) {
-    RTN_SOLO(__bf16, 1) RTN_SOLO(__bf16, 2) RTN_SOLO(__bf16, 3) RTN_SOLO(__bf16, 4) RTN_SOLO(__bf16, 5)
+    RTN_SOLO(__bf16, 1) RTN_SOLO(__bf16, 2) RTN_SOLO(__bf16, 3) RTN_SOLO(__bf16, 4)
   } else {
-    RTN_SOLO(float, 2) RTN_SOLO(float, 4) RTN_SOLO(float, 6) RTN_SOLO(float, 8)
+    RTN_SOLO(float, 2) RTN_SOLO(float, 4)
   }
 #undef RTN_SOLO
   return {nullptr, 0};

@@ -3,8 +3,6 @@
 
 #include <hip/hip_runtime.h>
 
-#include <utility>
-
 #include "lstm2_kernels.h"
 
 namespace rtn {
@@ -25,19 +23,15 @@ namespace rtn {
 //    in columns 4 t ... 4 t + 3 and zeros elsewhere.
 // The order of additions per element is that of the other kernels (their four wavefronts' shares of k are four
 // accumulators here), so the results are theirs bit for bit.
-// Measured (float32, T = 32, B = 4, n = 64): 5.3 + 36.5 us for packing and k_lstm2_regw before.
+// Measured (float32, T = 32, B = 4, n = 64): one call 27 us; 45 us with packing (5.3) and k_lstm2_regw (36.5).
 // ---------------------------------------------------------------------------------------------
 constexpr int kSoloRows = 4;
 constexpr int kSoloCells = 16;  // cells per wavefront
-constexpr int kSoloAhead = 4;   // steps that the gate inputs are fetched ahead
+constexpr int kSoloAhead = 4;   // sets of gate inputs: the loads of a step's are issued three steps before it
 
 // S: macro steps of the contraction, which with it gives the width: wavefronts = S (float32) or 2 S (bf16).
 template <typename AT>
 constexpr int solo_waves(int S) { return S * Elem<AT>::KM / kSoloCells; }
-
-// Compile-time index for the broadcast operand of the 4x4x1 MFMA.
-template <int K>
-__device__ __forceinline__ f32x4 mfma_4x4x1_from(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, c, 4, K, 0); }
 
 // k = 0 ... 15 of macro steps 4 j ... 4 j + 3, in the order in which a 16x16x4 MFMA of fragments of 4 takes them (0, 4, 8, 12,
 // 1, 5, ...); the four macro steps go to four accumulators, which hides the MFMA's latency.
@@ -47,7 +41,7 @@ __device__ __forceinline__ void solo_mfma_f32(const float (&h)[S], const float (
      constexpr int k = (I >> 2) + 4 * (I & 3);
 #pragma unroll
      for (int v = 0; v < 4; ++v)
-       if (4 * J + v < S) acc[v] = mfma_4x4x1_from<k>(h[4 * J + v < S ? 4 * J + v : 0], w[16 * (4 * J + v < S ? 4 * J + v : 0) + k], acc[v]);
+       if (4 * J + v < S) acc[v] = mfma_4x4x1<k>(h[4 * J + v < S ? 4 * J + v : 0], w[16 * (4 * J + v < S ? 4 * J + v : 0) + k], acc[v]);
    }()),
    ...);
 }
@@ -56,23 +50,10 @@ __device__ __forceinline__ void solo_mfma_f32_all(const float (&h)[S], const flo
   (solo_mfma_f32<S, J>(h, w, acc, std::make_integer_sequence<int, 16>{}), ...);
 }
 
-template <int PERM>
-__device__ __forceinline__ float quad_perm(float v) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), PERM, 0xF, 0xF, true));
-}
-// In every quad of lanes: lane g holds rows 0 ... 3 of column g; it gets columns 0 ... 3 of row g.
-__device__ __forceinline__ f32x4 quad_transpose(f32x4 a, int lane) {
-  const bool p = lane & 1, b = lane & 2;
-  const float r0 = quad_perm<0xB1>(p ? a[0] : a[1]), k0 = p ? a[1] : a[0];  // with the neighbour: rows p and p + 2 of two columns
-  const float r1 = quad_perm<0xB1>(p ? a[2] : a[3]), k1 = p ? a[3] : a[2];
-  const float n0 = p ? r0 : k0, n1 = p ? k0 : r0, n2 = p ? r1 : k1, n3 = p ? k1 : r1;
-  const float s0 = quad_perm<0x4E>(b ? n0 : n2), s1 = quad_perm<0x4E>(b ? n1 : n3);
-  const float q0 = b ? n2 : n0, q1 = b ? n3 : n1;
-  return b ? f32x4{s0, s1, q0, q1} : f32x4{q0, q1, s0, s1};
-}
-
+// (Two wavefronts per SIMD allowed for, which none of the builds needs more registers than: the compiler then keeps the
+// accumulators in the vector registers the pointwise part reads them from.)
 template <typename AT, int S>
-__global__ __launch_bounds__(64 * solo_waves<AT>(S)) void k_lstm2_solo(const Lstm2Multi multi) {
+__global__ __launch_bounds__(64 * solo_waves<AT>(S)) __attribute__((amdgpu_waves_per_eu(2))) void k_lstm2_solo(const Lstm2Multi multi) {
   using E = Elem<AT>;
   constexpr int KM = E::KM, ES = (int)sizeof(AT);
   constexpr bool F32 = ES == 4;
@@ -85,43 +66,6 @@ __global__ __launch_bounds__(64 * solo_waves<AT>(S)) void k_lstm2_solo(const Lst
   const int b_base = (int)blockIdx.x * kSoloRows, rows = min(kSoloRows, p.B - b_base);
   const long long bn = (long long)p.B * nc;
   if (blockIdx.x == 0 && tid < 64) p.status[tid] = status_word(tid, p.abort_word, p.abort_id);
-
-  // W of this wavefront's cells.  float32: a lane's column is gate lane % 4 of cell lane / 4, one register per k.  bf16: row
-  // i = lane % 16 of tile t is gate i % 4 of cell 4 (i / 4) + t: a lane loads four neighbouring cells at once.
-  float wf[F32 ? 16 * S : 1];
-  i32x4 wb[F32 ? 1 : 4][F32 ? 1 : S];
-  if constexpr (F32) {
-    const int cell = kSoloCells * wave + (lane >> 2);
-#pragma unroll
-    for (int k = 0; k < 16 * S; ++k) wf[k] = k < nc && cell < nc ? ((const float*)p.W)[(size_t)k * 4 * nc + (size_t)(lane & 3) * nc + cell] : 0.f;
-  } else {
-    const int i = lane & 15, kg = lane >> 4, cell = kSoloCells * wave + 4 * (i >> 2);
-    typedef unsigned long long u64_any __attribute__((aligned(2)));
-#pragma unroll
-    for (int s = 0; s < S; ++s) {
-      unsigned long long v[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int k = KM * s + 8 * kg + e;
-        v[e] = 0;
-        if (k < nc && cell < nc) {
-          const unsigned short* src = (const unsigned short*)p.W + (size_t)k * 4 * nc + (size_t)(i & 3) * nc + cell;
-          if (cell + 4 <= nc) {
-            v[e] = *(const u64_any*)src;
-          } else {
-#pragma unroll
-            for (int c = 0; c < 3; ++c)
-              if (cell + c < nc) v[e] |= (unsigned long long)src[c] << (16 * c);
-          }
-        }
-      }
-#pragma unroll
-      for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int w = 0; w < 4; ++w)
-          wb[t][s][w] = (int)(((unsigned)(v[2 * w] >> (16 * t)) & 0xFFFFu) | ((unsigned)(v[2 * w + 1] >> (16 * t)) << 16));
-    }
-  }
 
   // The pair of this lane.
   const int row = lane & 3, cell = kSoloCells * wave + (F32 ? lane >> 2 : 4 * (lane >> 4) + ((lane >> 2) & 3));
@@ -181,6 +125,54 @@ __global__ __launch_bounds__(64 * solo_waves<AT>(S)) void k_lstm2_solo(const Lst
     __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, c_state), cr, there ? c_at : kOobOffset, 0, 0);
   };
 
+  fetch(0, IntTag<0>{});
+  fetch(1, IntTag<1>{});
+  fetch(2, IntTag<2>{});
+  // W of this wavefront's cells.  float32: a lane's column is gate lane % 4 of cell lane / 4, one register per k.  bf16: row
+  // i = lane % 16 of tile t is gate i % 4 of cell 4 (i / 4) + t: a lane loads four neighbouring cells at once.  (What lies
+  // beyond the width is loaded from inside and replaced by zeros: no branches between the loads.)
+  float wf[F32 ? 16 * S : 1];
+  i32x4 wb[F32 ? 1 : 4][F32 ? 1 : S];
+  if constexpr (F32) {
+    const int wcell = kSoloCells * wave + (lane >> 2);
+    const float* src = (const float*)p.W + (size_t)(lane & 3) * nc + min(wcell, nc - 1);
+#pragma unroll
+    for (int k = 0; k < 16 * S; ++k) wf[k] = src[(size_t)min(k, nc - 1) * 4 * nc];
+#pragma unroll
+    for (int k = 0; k < 16 * S; ++k) wf[k] = k < nc && wcell < nc ? wf[k] : 0.f;
+  } else {
+    const int i = lane & 15, kg = lane >> 4, wcell = kSoloCells * wave + 4 * (i >> 2);
+    typedef unsigned long long u64_any __attribute__((aligned(2)));
+    const unsigned short* src = (const unsigned short*)p.W + (size_t)(i & 3) * nc;
+    const bool whole = nc % 4 == 0;  // (no lane's four cells are cut)
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      unsigned long long v[8];
+      if (whole) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = *(const u64_any*)(src + (size_t)min(KM * s + 8 * kg + e, nc - 1) * 4 * nc + min(wcell, nc - 4));
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = KM * s + 8 * kg + e < nc && wcell < nc ? v[e] : 0;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int k = KM * s + 8 * kg + e;
+          v[e] = 0;
+#pragma unroll
+          for (int c = 0; c < 4; ++c) {
+            const unsigned long long x = src[(size_t)min(k, nc - 1) * 4 * nc + min(wcell + c, nc - 1)];
+            v[e] |= (k < nc && wcell + c < nc ? x : 0) << (16 * c);
+          }
+        }
+      }
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int w = 0; w < 4; ++w)
+          wb[t][s][w] = (int)(((unsigned)(v[2 * w] >> (16 * t)) & 0xFFFFu) | ((unsigned)(v[2 * w + 1] >> (16 * t)) << 16));
+    }
+  }
+
   auto step = [&](int s, auto slot_tag) {
     constexpr int K = decltype(slot_tag)::value;
     const unsigned char* hb = hbuf[K & 1];
@@ -191,13 +183,15 @@ __global__ __launch_bounds__(64 * solo_waves<AT>(S)) void k_lstm2_solo(const Lst
       float h[S];
 #pragma unroll
       for (int i = 0; i < S; ++i) h[i] = *(const float*)(hb + i * 256 + lane * 4);
-      put(s - 1);  // (in the shadow of the LDS reads)
+      put(s - 1);  // (these two in the shadow of the LDS reads and of the MFMAs)
+      fetch(s + kSoloAhead - 1, IntTag<(K + kSoloAhead - 1) % kSoloAhead>{});
       solo_mfma_f32_all<S>(h, wf, acc, std::make_integer_sequence<int, (S + 3) / 4>{});
     } else {
       i32x4 h[S];
 #pragma unroll
       for (int i = 0; i < S; ++i) h[i] = *(const i32x4*)(hb + (((4 * i + (lane >> 4)) * kSoloRows) + (lane & 3)) * 16);
       put(s - 1);
+      fetch(s + kSoloAhead - 1, IntTag<(K + kSoloAhead - 1) % kSoloAhead>{});
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
         const int keep = ((lane >> 2) & 3) == t ? -1 : 0;
@@ -207,6 +201,11 @@ __global__ __launch_bounds__(64 * solo_waves<AT>(S)) void k_lstm2_solo(const Lst
           acc[i & 3] = E::mma(wb[t][i], b, acc[i & 3]);
         }
       }
+    }
+#pragma unroll
+    for (int i = 0; i < (F32 ? 16 * S : 4 * S); ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                // an MFMA ...
+      __builtin_amdgcn_sched_group_barrier(0x076, F32 ? 1 : 3, 0);  // ... and what fits behind it of everything else but LDS
     }
     f32x4 g = acc[0];
 #pragma unroll
@@ -227,13 +226,8 @@ __global__ __launch_bounds__(64 * solo_waves<AT>(S)) void k_lstm2_solo(const Lst
     y_out = (AT)y;
     a_out[0] = (AT)((p.op_flags & kOpH0IsCell) ? c : a0);
     a_out[1] = (AT)a1; a_out[2] = (AT)a2; a_out[3] = (AT)a3;
-    fetch(s + kSoloAhead, slot_tag);
     __syncthreads();
   };
-  fetch(0, IntTag<0>{});
-  fetch(1, IntTag<1>{});
-  fetch(2, IntTag<2>{});
-  fetch(3, IntTag<3>{});
   __syncthreads();
   for (int s = 0; s < nsteps; s += kSoloAhead) {
     step(s, IntTag<0>{});
