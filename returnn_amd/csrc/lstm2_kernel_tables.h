@@ -48,7 +48,12 @@ BwdRegwKernel bwd_regw_table_f32_full(int KSB, int MT, int WV);
 BwdRegwKernel bwd_regw_lds_table_bf16(int WV);
 BwdRegwKernel bwd_regw_lds_table_f32(int WV);
 
-inline RegwKernel regw_kernel(int dtype, int MT, int NT, int KSMAX, bool half, bool tail) {
+// k_lstm2_regw<float, MT, 1, KSMAX, false, TAIL, RQ>: the product in quads of rows.
+RegwKernel regw_table_f32_quad(int MT, int KSMAX, bool tail, int RQ);
+
+// rq > 0: the product in quads of rows (float32)
+inline RegwKernel regw_kernel(int dtype, int MT, int NT, int KSMAX, bool half, bool tail, int rq) {
+  if (rq > 0) return dtype == 0 && NT == 1 ? regw_table_f32_quad(MT, KSMAX, tail, rq) : nullptr;
   const bool lo = KSMAX <= 4;
   if (dtype == 1 /* RTN_DTYPE_BF16 */) return lo ? regw_table_bf16_lo(MT, NT, KSMAX, half, tail) : regw_table_bf16_hi(MT, NT, KSMAX, half, tail);
   return lo ? regw_table_f32_lo(MT, NT, KSMAX, half, tail) : regw_table_f32_hi(MT, NT, KSMAX, half, tail);

@@ -5,7 +5,7 @@
 #include "lstm2_kernel_tables.h"
 
 #ifndef RTN_TABLE_PART
-#error "compile with -DRTN_TABLE_PART=<1..9>"
+#error "compile with -DRTN_TABLE_PART=<1..11>"
 #endif
 
 namespace rtn {
@@ -46,6 +46,19 @@ RegwKernel regw_table(int MT, int NT, int KSMAX, bool half) {
     RTN_CASE(4, 1, 4) RTN_CASE(4, 2, 4)
   }
 #undef RTN_CASE
+  return nullptr;
+}
+
+// Forward, float32 in quads of rows.
+template <bool TAIL>
+RegwKernel regw_table_quad(int MT, int KSMAX, int RQ) {
+#define RTN_CASE(mt, ks) \
+  if (MT == mt && KSMAX == ks) \
+    return RQ == 1 ? &k_lstm2_regw<float, mt, 1, ks, false, TAIL, 1> : RQ == 2 ? &k_lstm2_regw<float, mt, 1, ks, false, TAIL, 2> : RQ == 3 ? &k_lstm2_regw<float, mt, 1, ks, false, TAIL, 3> : nullptr;
+  RTN_CASE(4, 4) RTN_CASE(4, 8)
+  RTN_CASE(8, 8)
+#undef RTN_CASE
+  if (MT == 4 && KSMAX == 2 && RQ == 1) return &k_lstm2_regw<float, 4, 1, 2, false, TAIL, 1>;
   return nullptr;
 }
 
@@ -128,8 +141,13 @@ SoloBuild solo_kernel(int dtype, int n) {
 #undef RTN_SOLO
   return {nullptr, 0};
 }
+#elif RTN_TABLE_PART == 10
+RegwKernel regw_table_f32_quad_tail(int MT, int KSMAX, int RQ) { return regw_table_quad<true>(MT, KSMAX, RQ); }
+#elif RTN_TABLE_PART == 11
+RegwKernel regw_table_f32_quad_tail(int MT, int KSMAX, int RQ);
+RegwKernel regw_table_f32_quad(int MT, int KSMAX, bool tail, int RQ) { return tail ? regw_table_f32_quad_tail(MT, KSMAX, RQ) : regw_table_quad<false>(MT, KSMAX, RQ); }
 #else
-#error "RTN_TABLE_PART must be 1..9"
+#error "RTN_TABLE_PART must be 1..11"
 #endif
 
 }  // namespace rtn

@@ -14,6 +14,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <utility>
+
 #include "lstm2_params.h"
 
 namespace rtn {
@@ -884,14 +886,59 @@ __device__ __forceinline__ bool group_on_one_xcd(unsigned* words, unsigned membe
   return ok;
 }
 
+// Float32 products in quads of rows (see k_lstm2_regw).
+template <int PERM>
+__device__ __forceinline__ float quad_perm(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), PERM, 0xF, 0xF, true));
+}
+// In every quad of lanes: lane g holds rows 0 ... 3 of column g; it gets columns 0 ... 3 of row g.
+__device__ __forceinline__ f32x4 quad_transpose(f32x4 a, int lane) {
+  const bool p = lane & 1, b = lane & 2;
+  const float r0 = quad_perm<0xB1>(p ? a[0] : a[1]), k0 = p ? a[1] : a[0];  // with the neighbour: rows p and p + 2 of two columns
+  const float r1 = quad_perm<0xB1>(p ? a[2] : a[3]), k1 = p ? a[3] : a[2];
+  const float n0 = p ? r0 : k0, n1 = p ? k0 : r0, n2 = p ? r1 : k1, n3 = p ? k1 : r1;
+  const float s0 = quad_perm<0x4E>(b ? n0 : n2), s1 = quad_perm<0x4E>(b ? n1 : n3);
+  const float q0 = b ? n2 : n0, q1 = b ? n3 : n1;
+  return b ? f32x4{s0, s1, q0, q1} : f32x4{q0, q1, s0, s1};
+}
+
+template <int ABID>
+__device__ __forceinline__ f32x4 mfma_4x4x1(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, c, 4, ABID, 0); }
+// One macro step: I counts (e, kg, row quad); UP: the rows sit in the upper half of every group of 16 lanes.
+template <int MT, int RQ, int UP, int... I>
+__device__ __forceinline__ void quad_macro_step(const i32x4 (&wbits)[MT], const i32x4& hbits, f32x4 (&acc)[MT / 4 * RQ], std::integer_sequence<int, I...>) {
+  const f32x4 h = __builtin_bit_cast(f32x4, hbits);
+  f32x4 w[MT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) w[i] = __builtin_bit_cast(f32x4, wbits[i]);
+  (([&] {
+     constexpr int e = I / (4 * RQ), kg = I / RQ % 4, rq = I % RQ;
+#pragma unroll
+     for (int cb = 0; cb < MT / 4; ++cb)
+       acc[cb * RQ + rq] = mfma_4x4x1<4 * kg + rq + 2 * UP>(h[e], w[4 * cb + kg][e], acc[cb * RQ + rq]);
+   }()),
+   ...);
+}
+
 // HALF: the groups have at most 8 rows (NT == 1, MT even).  A tile then holds valid results in the lanes of rows 0..7
 // only, and the pointwise part folds two tiles into one pass: lanes of rows 0..7 take tile 2u, lanes of rows 8..15 take
 // rows 0..7 of tile 2u + 1, so that a thread owns one (sequence, cell) pair where the plain mapping gives it two, one
 // of them of a row that does not exist.
 // TAIL: the caller's width cuts a chunk of 16 bytes (see the streams below).  A build of its own: the few instructions and
 // registers of the tail cost the other widths up to 6 % (op of 32 steps at n = 64: 54.4 us against 51.2).
-template <typename AT, int MT, int NT, int KSMAX, bool HALF = false, bool TAIL = false>
+// RQ > 0 (float32, groups of at most 4 RQ rows, MT a multiple of 4): the product in v_mfma_f32_4x4x1 instead of 16x16x4.  16
+// blocks of 4 rows x 4 columns and one k, with the block of h that holds the wanted k and rows broadcast to all of them, are
+// 4 rows x 64 gate columns in 8 clocks: 32 multiply-adds a clock like the 16x16x4, but in units of 4 rows -- a group of 8
+// rows takes half the time of a 16-row tile, which is padded to twice its rows.  Fragments of h are used as they are loaded:
+// register e of lane (kg, row) is k = 4 kg + e of that row, so block 4 kg + row / 4 holds what a quad of rows needs of that k.
+// The order of additions per element is the 16x16x4's (both are chains of fused multiply-adds, k = 0, 4, 8, 12, 1, ...), the
+// results are the same bits.  What comes out is gate by gate in the lanes of a quad, and is transposed there.
+// (n = 512, groups of 8 rows on one XCD: 2048 clocks of MFMAs per step instead of 4096, which is what makes the XCD-local
+// plan the better one in float32.)
+template <typename AT, int MT, int NT, int KSMAX, bool HALF = false, bool TAIL = false, int RQ = 0>
 __global__ __launch_bounds__(kWgThreads) void k_lstm2_regw(const Lstm2Multi multi) {
+  constexpr bool QUAD = RQ > 0;
+  static_assert(!QUAD || (sizeof(AT) == 4 && NT == 1 && MT % 4 == 0 && RQ <= 4), "quads of rows: float32, one batch tile, whole blocks of 64 columns");
   static_assert(!HALF || (NT == 1 && MT % 2 == 0), "half-tile mapping: one batch tile, an even number of cell tiles");
   // Which of the launch's problems and which (group, rank) this workgroup works on (uniform over the workgroup).
   int which, g, r;
@@ -921,8 +968,8 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_regw(const Lstm2Multi mult
   constexpr int KE = E::KE;
   constexpr int KM = E::KM;
   constexpr int ES = (int)sizeof(AT);
-  constexpr int TILES = MT * NT;
-  constexpr int UNITS = HALF ? TILES / 2 : TILES;  // passes of the pointwise part over all wavefronts
+  constexpr int TILES = QUAD ? MT / 4 * RQ : MT * NT;  // partial tiles (QUAD: 64 columns x 4 rows)
+  constexpr int UNITS = HALF && !QUAD ? TILES / 2 : TILES;  // passes of the pointwise part over all wavefronts
   constexpr int EPT = (UNITS + kWaves - 1) / kWaves;
   constexpr int ROWS = 16 * NT;   // rows of the MFMA tiles (>= valid rows of the group)
   constexpr int CELLS = 4 * MT;   // cells owned by this workgroup
@@ -1080,7 +1127,7 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_regw(const Lstm2Multi mult
   // CU's load path takes a wavefront's load instruction at about 16 clocks whatever its width, and the four wavefronts'
   // loads are what the wait for h consists of).  The odd macro step's rows reach the lanes of rows 0-7 through a
   // shift by 8 inside each group of 16 lanes.
-  constexpr bool PAIRED = HALF && NT == 1 && KSMAX % 2 == 0;
+  constexpr bool PAIRED = (QUAD ? RQ <= 2 : HALF && NT == 1) && KSMAX % 2 == 0;
   constexpr int NLD = PAIRED ? KSMAX / 2 : KSMAX;  // loads of B fragments per step
   i32x4 wreg[MT][KSMAX];
   unsigned foff[KSMAX][NT];  // where this lane's B-operand fragments are inside a ring buffer
@@ -1091,7 +1138,9 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_regw(const Lstm2Multi mult
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
       wreg[mt][ks] = i32x4{0, 0, 0, 0};
-      if (mine) wreg[mt][ks] = ((const i32x4*)p.Wp)[((size_t)(r * MT + mt) * S + sm) * 64 + lane];
+      // (QUAD: register 4 cb + kg is k = 4 kg ... 4 kg + 3 of the lane's column of block cb, which is row lane % 16 of tile lane / 16)
+      const int m = QUAD ? r * MT + (mt & ~3) + kg : r * MT + mt;
+      if (mine) wreg[mt][ks] = ((const i32x4*)p.Wp)[((size_t)m * S + sm) * 64 + (QUAD ? 16 * (mt & 3) + jl : lane)];
     }
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
@@ -1120,7 +1169,11 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_regw(const Lstm2Multi mult
   for (int j = 0; j < EPT; ++j) {
     const int u = min(wave + kWaves * j, UNITS - 1);
     int e, bl, src;
-    if (HALF) {
+    if (QUAD) {
+      e = u;
+      bl = 4 * (u % RQ) + (lane & 3);
+      src = lane;
+    } else if (HALF) {
       e = 2 * u + ((lane >> 3) & 1);
       bl = lane & 7;
       src = (lane & 0x30) | bl;
@@ -1129,12 +1182,12 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_regw(const Lstm2Multi mult
       bl = 16 * (e % NT) + (lane & 15);
       src = lane;
     }
-    const int mt = e / NT;
-    const int cell = 4 * (r * MT + mt) + (lane >> 4);
+    const int cl = QUAD ? 16 * (u / RQ) + (lane >> 2) : 4 * (e / NT) + (lane >> 4);  // cell inside the workgroup's
+    const int cell = 4 * r * MT + cl;
     e_tile[j] = (unsigned)e;
     e_src[j] = (unsigned)src;
     e_row[j] = (unsigned)bl;
-    e_cl[j] = (unsigned)(4 * mt + (lane >> 4));
+    e_cl[j] = (unsigned)cl;
     e_valid[j] = (wave + kWaves * j < UNITS) && (bl < rows) && cell < nc;
     e_hoff[j] = (unsigned)((((cell / KE) * p.Bp + bl) * KE + (cell % KE)) * ES);
     c_state[j] = 0.f;
@@ -1305,7 +1358,7 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_regw(const Lstm2Multi mult
       // accumulator: columns 0-7 collect tile 2u, columns 8-15 tile 2u+1 (the other tile contributes exact zeros, so
       // every sum is bit for bit what a tile of its own would hold).  Half the accumulators, half the partial tiles
       // through LDS -- written by all 64 lanes, in the very lane order the pointwise part reads them in.
-      constexpr int NACC = PAIRED ? MT / 2 : MT;
+      constexpr int NACC = QUAD ? TILES : PAIRED ? MT / 2 : MT;
       f32x4 acc[NACC][NT];
 #pragma unroll
       for (int mt = 0; mt < NACC; ++mt)
@@ -1322,7 +1375,30 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_regw(const Lstm2Multi mult
       // every group of 16 lanes.  Four B operands are made of it: each step's rows in columns 0-7 (for the even tiles)
       // and in columns 8-15 (for the odd tiles), zeros in the other half -- a mask where the rows stay, a row shift by 8
       // lanes (data parallel primitive; lanes without a source take 0) where they move.
-      if constexpr (PAIRED) {
+      if constexpr (QUAD) {
+        flush_read_at(rd_h, rd_y, rd_c);
+        load_gate_inputs(IntTag<1 - PAR>{});
+        put(par_tag);
+        flush_write_at(h_out, y_out_p, c_out, s >= 2);
+        fetch_at(x_next, m_next, s + 4 < nsteps, par_tag);
+        widen_gate_inputs(par_tag);
+        f32x4(&qacc)[TILES] = reinterpret_cast<f32x4(&)[TILES]>(acc);
+#pragma unroll
+        for (int ks = 0; ks < KSMAX; ++ks) {
+          i32x4 w[MT];
+#pragma unroll
+          for (int mt = 0; mt < MT; ++mt) w[mt] = wreg[mt][ks];
+          if (PAIRED && (ks & 1))
+            quad_macro_step<MT, RQ, PAIRED ? 1 : 0>(w, bf[ks >> 1][0], qacc, std::make_integer_sequence<int, 16 * RQ>{});
+          else
+            quad_macro_step<MT, RQ, 0>(w, bf[PAIRED ? ks >> 1 : ks][0], qacc, std::make_integer_sequence<int, 16 * RQ>{});
+        }
+#pragma unroll
+        for (int i = 0; i < KSMAX * 16 * TILES; ++i) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // an MFMA of 8 clocks takes two issue turns of 4 ...
+          __builtin_amdgcn_sched_group_barrier(0x096, 1, 0);  // ... one of which anything else may have
+        }
+      } else if constexpr (PAIRED) {
         // The MFMAs go in chunks of NACC -- one per accumulator: (macro step, even tiles), (macro step, odd tiles), ... --
         // so that two MFMAs into the same accumulator are NACC apart.  The compiler's scheduler would otherwise line up
         // the MFMAs of one accumulator, each waiting for the one before; nothing moves from one chunk to another
@@ -1388,7 +1464,7 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_regw(const Lstm2Multi mult
             }
       }
       h_out += step_h; y_out_p += step_y; c_out += step_c; x_next += step_x; m_next += step_m;
-      if constexpr (PAIRED) {
+      if constexpr (PAIRED || QUAD) {
 #pragma unroll
         for (int u = 0; u < NACC; ++u) redbuf[wave][u][lane] = acc[u][0];
       } else if (!HALF || (lane & 8) == 0) {  // (with at most 8 rows only the lanes of rows 0..7 hold columns anybody reads)
@@ -1420,11 +1496,12 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_regw(const Lstm2Multi mult
           // after the other through one set of registers and pays the LDS latency three times)
           f32x4 part[kWaves];
 #pragma unroll
-          for (int w = 0; w < kWaves; ++w) part[w] = PAIRED ? redbuf[w][wave + kWaves * j][lane] : redbuf[w][e_tile[j]][e_src[j]];
+          for (int w = 0; w < kWaves; ++w) part[w] = PAIRED || QUAD ? redbuf[w][wave + kWaves * j][lane] : redbuf[w][e_tile[j]][e_src[j]];
           __builtin_amdgcn_sched_barrier(0);
           f32x4 gsum = part[0];
 #pragma unroll
           for (int w = 1; w < kWaves; ++w) gsum += part[w];
+          if constexpr (QUAD) gsum = quad_transpose(gsum, lane);
           const float m = m_f[j];
           const float a0 = Act<AT>::tanh(gsum[0] + x_f[j][0]);
           const float a1 = Act<AT>::sigmoid(gsum[1] + x_f[j][1]);
@@ -1559,10 +1636,10 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_regw(const Lstm2Multi mult
 // registers, the partial tiles through LDS with the step's one barrier, and their sum in wave order (kept as a running
 // value so that nothing can be dropped).  No exchange, no streams, no pointwise arithmetic.  The time of a launch over
 // the op's algorithmic flops is the MFMA roofline a kernel of this decomposition could reach at most.
-template <typename AT, int MT, int NT, int KSMAX, bool HALF>
+template <typename AT, int MT, int NT, int KSMAX, bool HALF, int RQ = 0>
 __global__ __launch_bounds__(kWgThreads) void k_mfma_sequence(float* out, int steps) {
   using E = Elem<AT>;
-  constexpr int TILES = MT * NT;
+  constexpr int TILES = RQ ? MT / 4 * RQ : MT * NT;  // (RQ: float32 in quads of rows, as in k_lstm2_regw)
   constexpr int UNITS = HALF ? TILES / 2 : TILES;
   constexpr int EPT = (UNITS + kWaves - 1) / kWaves;
   extern __shared__ __align__(16) unsigned char smem[];
@@ -1596,7 +1673,7 @@ __global__ __launch_bounds__(kWgThreads) void k_mfma_sequence(float* out, int st
   f32x4 total = f32x4{0.f, 0.f, 0.f, 0.f};
   constexpr bool PAIRED = HALF && NT == 1 && KSMAX % 2 == 0;  // as in k_lstm2_regw: two tiles share an accumulator
   constexpr int NLD = PAIRED ? KSMAX / 2 : KSMAX;
-  constexpr int NACC = PAIRED ? MT / 2 : MT;
+  constexpr int NACC = RQ ? TILES : PAIRED ? MT / 2 : MT;
   auto step = [&](auto par_tag) {
     constexpr int PAR = decltype(par_tag)::value;
     RedBuf& redbuf = red[PAR];
@@ -1631,6 +1708,19 @@ __global__ __launch_bounds__(kWgThreads) void k_mfma_sequence(float* out, int st
           for (int u = 0; u < NACC; ++u) acc[u][0] = E::mma(wreg[2 * u + odd][ks], odd ? b_hi[ks] : b_lo[ks], acc[u][0]);
 #pragma unroll
       for (int u = 0; u < NACC; ++u) redbuf[wave][u][lane] = acc[u][0];
+    } else if constexpr (RQ > 0) {
+      f32x4 quad[TILES];
+#pragma unroll
+      for (int u = 0; u < TILES; ++u) quad[u] = acc[u][0];
+#pragma unroll
+      for (int ks = 0; ks < KSMAX; ++ks) {
+        i32x4 w[MT];
+#pragma unroll
+        for (int i = 0; i < MT; ++i) w[i] = wreg[i][ks];
+        quad_macro_step<MT, RQ, 0>(w, bf[ks][0], quad, std::make_integer_sequence<int, 16 * RQ>());
+      }
+#pragma unroll
+      for (int u = 0; u < TILES; ++u) redbuf[wave][u][lane] = quad[u];
     } else {
 #pragma unroll
       for (int ks = 0; ks < KSMAX; ++ks)
@@ -1681,7 +1771,7 @@ __global__ __launch_bounds__(kWgThreads) void k_mfma_sequence(float* out, int st
 // recurrent GEMM that no arrangement of the rest of the step can exceed.
 // OTHERS > 0: that many vector instructions (register moves) behind every MFMA -- what a wavefront can issue in an
 // MFMA's shadow before the matrix core has to wait for it.
-template <typename AT, int MT, int NT, int KSMAX, int THREADS = kWgThreads, int OTHERS = 0>
+template <typename AT, int MT, int NT, int KSMAX, int THREADS = kWgThreads, int OTHERS = 0, int RQ = 0>
 __global__ __launch_bounds__(THREADS) void k_mfma_issue(float* out, int steps) {
   using E = Elem<AT>;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -1721,6 +1811,20 @@ __global__ __launch_bounds__(THREADS) void k_mfma_issue(float* out, int steps) {
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if constexpr (RQ > 0) {  // float32 in quads of rows: MT / 4 * RQ accumulators
+      f32x4 quad[MT / 4 * RQ];
+#pragma unroll
+      for (int u = 0; u < MT / 4 * RQ; ++u) quad[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ks = 0; ks < KSMAX; ++ks) {
+        i32x4 w[MT];
+#pragma unroll
+        for (int i = 0; i < MT; ++i) w[i] = wreg[i][ks];
+        quad_macro_step<MT, RQ, 0>(w, bf[ks][0], quad, std::make_integer_sequence<int, 16 * RQ>());
+      }
+#pragma unroll
+      for (int u = 0; u < MT / 4 * RQ; ++u) acc[u][0] = quad[u];
+    } else
 #pragma unroll
     for (int ks = 0; ks < KSMAX; ++ks)
 #pragma unroll

@@ -170,6 +170,7 @@ struct Plan {
   int mode = RTN_MODE_STEPWISE;  // resolved: PERSISTENT, GRAPH or STEPWISE
   bool regw = false;             // persistent kernel with W in registers and self-validating exchange
   bool local = false;            // regw: every batch group on one XCD, hidden state exchanged through that XCD's L2
+  int rq = 0;                    // regw, float32: quads of rows per group where the product goes in them, else 0
   bool wide = false;             // persistent kernel for layers whose W takes registers and LDS of the whole device
   WideBuild wide_build = {nullptr, 0, 0, 0, 0, 0};
   bool solo = false;             // small layer: every workgroup takes 4 rows through all steps by itself
@@ -255,9 +256,25 @@ bool make_plan_uncached(int64_t T, int B, int n, int dtype, int want_mode, bool 
     if (want_mode == RTN_MODE_AUTO || want_mode == RTN_MODE_PERSISTENT) {
       struct Cand {
         bool ok = false, regw = false, local = false, half = false;
+        int rq = 0;  // quads of rows
+        double mfma_us = 0;
         int KSMAX = 0, MT = 1, NT = 1, groups = 1, G = 1, Bg = 1, grid = 0;
         size_t lds = 0;
         double est = 1e30;
+      };
+      // Float32 products in quads of rows (k_lstm2_regw with RQ): blocks of 64 columns, up to 3 quads (a fourth would take as
+      // long as a 16-row tile).  A wavefront's MFMA issue time then goes with the quads.  Two or three quads of a layer of up
+      // to 128 cells are left to the half tiles (1.06 us per step against 1.08 with two: the product is a tenth of the step
+      // there), and above 512 cells a group of 64 columns a workgroup has no XCD to itself and no shorter product.
+      auto quads = [&](int MT, int NT, int Bg) {
+        if (dtype != RTN_DTYPE_F32 || !di.valid || NT != 1 || Bg > 12 || env_long("RTN_LSTM2_NO_QUAD", 0)) return 0;
+        if (!(MT == 4 && KSMAX <= 8) && !(MT == 8 && KSMAX == 8)) return 0;
+        const int rq = (Bg + 3) / 4;
+        return KSMAX == 2 && rq > 1 ? 0 : rq;
+      };
+      auto issue_us = [&](int MT, int NT, int rq) {
+        const double clocks = rq ? (double)(MT / 4) * KSMAX * 16 * rq * (MT / 4 * rq == 1 ? 13 : 8.3) : (double)MT * NT * ks * (dtype == RTN_DTYPE_BF16 ? 16 : 128);
+        return clocks / 2400.0;
       };
       // XCD-local decompositions: a group's workgroups (one per CU) all on one XCD, so that the hidden state is handed
       // over through that XCD's L2 (a hand-over between XCDs goes through memory and takes about twice as long).  A group
@@ -291,15 +308,16 @@ bool make_plan_uncached(int64_t T, int B, int n, int dtype, int want_mode, bool 
           const bool half = Bg <= 8 && NT == 1 && MT % 2 == 0 && !env_long("RTN_LSTM2_NO_HALF", 0);
           const size_t lds = (size_t)regw_lds((int)es, MT, NT).total;
           if (lds > di.lds_per_wg) continue;
-          const double mfma_us = (double)MT * NT * ks * (dtype == RTN_DTYPE_BF16 ? 16 : 128) / 2400.0;
-          const int units = half ? MT / 2 : MT * NT;
+          const int rq = quads(MT, NT, Bg);
+          const double mfma_us = issue_us(MT, NT, rq);
+          const int units = rq ? MT / 4 * rq : half ? MT / 2 : MT * NT;
           const int ept = (units + kWaves - 1) / kWaves;
           // Step time in microseconds, fitted to MI355X measurements (n = 1024 bf16 with 1, 4 and 8 rows per group,
           // n = 512 float32 with 8): a constant, the MFMA issue time of a wavefront and the KB of hidden state every
           // CU fetches per step; a second pass of the pointwise part costs about a quarter of a microsecond.
           const double est = 1.16 + 0.873 * mfma_us + 0.020 * (double)Bg * n * es / 1024.0 + 0.25 * (ept - 1);
           if (est < best.est) {
-            best.ok = true; best.regw = true; best.local = true; best.half = half;
+            best.ok = true; best.regw = true; best.local = true; best.half = half && !rq; best.rq = rq; best.mfma_us = mfma_us;
             best.est = est; best.KSMAX = KSMAX; best.MT = MT; best.NT = NT; best.groups = groups; best.G = G; best.Bg = Bg;
             best.lds = lds;
             const int total_groups = groups * std::max(problems, 1);
@@ -340,8 +358,9 @@ bool make_plan_uncached(int64_t T, int B, int n, int dtype, int want_mode, bool 
               // wavefront, a second round of gate arithmetic when a thread owns two pairs, the number of
               // workgroups that exchange with each other, the fragments a wavefront reads per step and
               // the fragments it holds.
-              const double mfma_us = (double)MT * NT * ks * (dtype == RTN_DTYPE_BF16 ? 16 : 128) / 2400.0;
-              const int ept = (MT * NT + kWaves - 1) / kWaves;
+              const int rq = use_regw ? quads(MT, NT, Bg) : 0;
+              const double mfma_us = issue_us(MT, NT, rq);
+              const int ept = ((rq ? MT / 4 * rq : MT * NT) + kWaves - 1) / kWaves;
               double est = 2.0 * mfma_us + 0.4 * (ept - 1) + 0.004 * G + 0.03 * ks * NT + 0.01 * MT * ks;
               // Several problems in one launch: as long as every workgroup has a CU to itself they do not slow
               // each other down; sharing CUs costs about a third, running in turns costs the whole time again.
@@ -359,6 +378,8 @@ bool make_plan_uncached(int64_t T, int B, int n, int dtype, int want_mode, bool 
                 best.ok = true;
                 best.est = est;
                 best.regw = use_regw != 0;
+                best.rq = rq;
+                best.mfma_us = mfma_us;
                 best.KSMAX = use_regw ? KSMAX : 0;
                 best.MT = MT;
                 best.NT = NT;
@@ -385,16 +406,17 @@ bool make_plan_uncached(int64_t T, int B, int n, int dtype, int want_mode, bool 
         // spread launch always go local.
         bool take_local = loc.ok && !(chosen.ok && chosen.regw);
         if (loc.ok && chosen.ok && chosen.regw) {
-          auto mfma_us = [&](const Cand& c) { return (double)c.MT * c.NT * ks * (dtype == RTN_DTYPE_BF16 ? 16 : 128) / 2400.0; };
-          auto passes = [&](const Cand& c) { return ((c.half ? c.MT / 2 : c.MT * c.NT) + kWaves - 1) / kWaves; };
+          auto passes = [&](const Cand& c) { return ((c.rq ? c.MT / 4 * c.rq : c.half ? c.MT / 2 : c.MT * c.NT) + kWaves - 1) / kWaves; };
           const long long each = (long long)align_up((size_t)(chosen.groups * chosen.G), (size_t)di.xcds);
           const bool shares = count > 1 && di.cus / each < count;
-          const double cost = 0.873 * (mfma_us(loc) - mfma_us(chosen)) + 0.25 * (passes(loc) - passes(chosen));
+          const double cost = 0.873 * (loc.mfma_us - chosen.mfma_us) + 0.25 * (passes(loc) - passes(chosen));
           const double more_kb = std::max(0, chosen.Bg - loc.Bg) * (double)n * es / 1024.0;  // hidden state per CU and step
           // (bf16: 0.40 since two tiles of a group of up to 8 rows share an accumulator -- measured again at n = 256 ... 1024
           // with 1 ... 64 rows: the XCD-local plan is ahead or level everywhere, a single sequence of n = 1024 included)
           const double gain = (dtype == RTN_DTYPE_BF16 ? 0.40 : 0.20) + (each * std::max(count, 1) > di.cus / 2 ? 0.25 : 0.0) + 0.005 * more_kb;
-          take_local = shares || cost < gain;
+          // (float32 in one quad of rows: ahead of the spread plan wherever both exist, measured at n = 128 ... 512: 1.64 us
+          // against 1.89 at n = 512 with one row)
+          take_local = shares || loc.rq == 1 || cost < gain;
         }
         if (loc.ok && (env_long("RTN_LSTM2_LOCAL", -1) == 1 || take_local)) chosen = loc;
       }
@@ -419,6 +441,7 @@ bool make_plan_uncached(int64_t T, int B, int n, int dtype, int want_mode, bool 
         pl.regw = chosen.regw;
         pl.local = chosen.local;
         pl.half = chosen.half;
+        pl.rq = chosen.rq;
         pl.KSMAX = chosen.KSMAX;
         pl.MT = chosen.MT;
         pl.NT = chosen.NT;
@@ -471,7 +494,7 @@ bool make_plan_uncached(int64_t T, int B, int n, int dtype, int want_mode, bool 
       int MT = 1;
       pl.regw = pl.wide = false;
       pl.local = pl.half = false;
-      pl.KSMAX = 0;
+      pl.KSMAX = pl.rq = 0;
       // A step's launch takes W from memory straight into the matrix cores (every fragment is used once per launch).
       pl.w_direct = env_long("RTN_LSTM2_W_DIRECT", 1) != 0;
       if (!pl.w_direct && mfma_lds_bytes(n, dtype, 1, 4) > di.lds_per_wg) {
@@ -1164,7 +1187,7 @@ int settle_fwd_plan(int count, int64_t T, int B, int nc, int n, int dtype, int m
   if (!make_plan(T, B, n, dtype, mode, capturing, &pl, &why, 2, plan_count))
     return fail(RTN_ERR_UNSUPPORTED, "NativeLstm2: persistent mode unavailable for T=%lld B=%d n=%d: %s", (long long)T, B, n, why.c_str());
   for (int attempt = 0; pl.kind == kPlanMfma && pl.mode == RTN_MODE_PERSISTENT; ++attempt) {
-    *pk = pl.wide ? (const void*)pl.wide_build.kernel : pl.regw ? (const void*)regw_kernel(dtype, pl.MT, pl.NT, pl.KSMAX, pl.half, nc % (int)(std::min<size_t>(16, 4 * pl.MT * esize(dtype)) / esize(dtype)) != 0) : (const void*)mfma_kernel(dtype, pl.MT, pl.NT);
+    *pk = pl.wide ? (const void*)pl.wide_build.kernel : pl.regw ? (const void*)regw_kernel(dtype, pl.MT, pl.NT, pl.KSMAX, pl.half, nc % (int)(std::min<size_t>(16, 4 * pl.MT * esize(dtype)) / esize(dtype)) != 0, pl.rq) : (const void*)mfma_kernel(dtype, pl.MT, pl.NT);
     if (!*pk) return fail(RTN_ERR_UNSUPPORTED, "NativeLstm2: no kernel for mt=%d nt=%d ks=%d", pl.MT, pl.NT, pl.KSMAX);
     if ((rc = ensure_lds_limit(*pk, pl.lds_bytes)) != RTN_OK) return rc;
     const int wgs = pl.regw || pl.wide ? pl.grid : pl.groups * pl.wgs_per_group;
@@ -1513,6 +1536,13 @@ BwdLayout bwd_layout(int B, int n, int dtype) {
 }
 
 typedef void (*SeqKernel)(float*, int);
+// (float32 in quads of rows, rq of them: the sequence or the MFMAs alone)
+template <int MT, int KSMAX>
+SeqKernel quad_probe_for(int rq, bool issue_only) {
+  if (rq == 1) return issue_only ? &k_mfma_issue<float, MT, 1, KSMAX, kWgThreads, 0, 1> : &k_mfma_sequence<float, MT, 1, KSMAX, false, 1>;
+  if (rq == 2) return issue_only ? &k_mfma_issue<float, MT, 1, KSMAX, kWgThreads, 0, 2> : &k_mfma_sequence<float, MT, 1, KSMAX, false, 2>;
+  return issue_only ? &k_mfma_issue<float, MT, 1, KSMAX, kWgThreads, 0, 3> : &k_mfma_sequence<float, MT, 1, KSMAX, false, 3>;
+}
 template <typename AT>
 SeqKernel seq_kernel_for(int MT, int NT, int KSMAX, bool half) {
   // the decompositions of the benchmark configurations and their neighbours
@@ -1565,7 +1595,9 @@ int mfma_probe(bool issue_only, int32_t count, int64_t T, int32_t B, int32_t n, 
     // wavefront can issue in the MFMAs' shadow
     const long others = env_long("RTN_LSTM2_PROBE_OTHERS", 0);
     k = others == 1 ? &k_mfma_issue<__bf16, 8, 1, 8, kWgThreads, 1> : others == 2 ? &k_mfma_issue<__bf16, 8, 1, 8, kWgThreads, 2> : &k_mfma_issue<__bf16, 8, 1, 8, kWgThreads, 3>;
-  } else if (issue_only)
+  } else if (pl.rq)
+    k = pl.MT == 8 && pl.KSMAX == 8 ? quad_probe_for<8, 8>(pl.rq, issue_only) : pl.MT == 4 && pl.KSMAX == 8 ? quad_probe_for<4, 8>(pl.rq, issue_only) : nullptr;
+  else if (issue_only)
     k = dtype == RTN_DTYPE_BF16 ? issue_kernel_for<__bf16>(pl.MT, pl.NT, pl.KSMAX) : issue_kernel_for<float>(pl.MT, pl.NT, pl.KSMAX);
   else
     k = dtype == RTN_DTYPE_BF16 ? seq_kernel_for<__bf16>(pl.MT, pl.NT, pl.KSMAX, pl.half) : seq_kernel_for<float>(pl.MT, pl.NT, pl.KSMAX, pl.half);
@@ -1666,6 +1698,7 @@ const char* rtn_native_lstm2_describe_multi_plan(int32_t count, int64_t T, int32
              pl.NT, pl.groups, pl.wgs_per_group, (pl.mode == RTN_MODE_PERSISTENT && (pl.regw || pl.wide || pl.solo)) ? pl.grid : pl.groups * pl.wgs_per_group,
              pl.Bg, pl.passes, pl.lds_bytes,
              (count > 1 || n != n_asked) ? workspace_each(count, T, B, n_asked, dtype, mode) : pl.total);
+    if (pl.rq) snprintf(buf + strlen(buf), sizeof(buf) - strlen(buf), " row_quads=%d", pl.rq);
     if (n != n_asked) snprintf(buf + strlen(buf), sizeof(buf) - strlen(buf), " padded_width=%d", n);
     if (pl.off_trace) snprintf(buf + strlen(buf), sizeof(buf) - strlen(buf), " trace_offset=%zu", pl.off_trace);
     g_plan_text = buf;
