@@ -5,7 +5,7 @@
 #include "lstm2_kernel_tables.h"
 
 #ifndef RTN_TABLE_PART
-#error "compile with -DRTN_TABLE_PART=<1..11>"
+#error "compile with -DRTN_TABLE_PART=<1..13>"
 #endif
 
 namespace rtn {
@@ -81,6 +81,18 @@ BwdRegwKernel bwd_regw_table(int KSB, int MT, int WV) {
   return nullptr;
 }
 
+// (float32 in quads of rows)
+template <int RQ>
+BwdRegwKernel bwd_regw_table_quad(int KSB, int MT, int WV) {
+#define RTN_CASE(ks, mt, wv) \
+  if (KSB == ks && MT == mt && WV == wv) return &k_lstm2_bwd_regw<float, ks, mt, wv, 0, true, RQ>;
+  RTN_CASE(2, 1, 4) RTN_CASE(4, 1, 4) RTN_CASE(8, 1, 4) RTN_CASE(16, 1, 4) RTN_CASE(32, 1, 4)
+  RTN_CASE(2, 2, 4) RTN_CASE(4, 2, 4) RTN_CASE(8, 2, 4) RTN_CASE(16, 2, 4) RTN_CASE(32, 2, 4)
+  RTN_CASE(2, 4, 4) RTN_CASE(4, 4, 4) RTN_CASE(8, 4, 4) RTN_CASE(16, 4, 4)
+#undef RTN_CASE
+  return nullptr;
+}
+
 template <typename AT>
 BwdRegwKernel bwd_regw_lds_table(int WV) {
   if (WV == 8) return &k_lstm2_bwd_regw<AT, 16, 1, 8, 16>;
@@ -146,8 +158,13 @@ RegwKernel regw_table_f32_quad_tail(int MT, int KSMAX, int RQ) { return regw_tab
 #elif RTN_TABLE_PART == 11
 RegwKernel regw_table_f32_quad_tail(int MT, int KSMAX, int RQ);
 RegwKernel regw_table_f32_quad(int MT, int KSMAX, bool tail, int RQ) { return tail ? regw_table_f32_quad_tail(MT, KSMAX, RQ) : regw_table_quad<false>(MT, KSMAX, RQ); }
+#elif RTN_TABLE_PART == 12
+BwdRegwKernel bwd_regw_table_f32_quads2(int KSB, int MT, int WV);
+BwdRegwKernel bwd_regw_table_f32_quads(int KSB, int MT, int WV, int RQ) { return RQ == 1 ? bwd_regw_table_quad<1>(KSB, MT, WV) : RQ == 2 ? bwd_regw_table_f32_quads2(KSB, MT, WV) : nullptr; }
+#elif RTN_TABLE_PART == 13
+BwdRegwKernel bwd_regw_table_f32_quads2(int KSB, int MT, int WV) { return bwd_regw_table_quad<2>(KSB, MT, WV); }
 #else
-#error "RTN_TABLE_PART must be 1..11"
+#error "RTN_TABLE_PART must be 1..13"
 #endif
 
 }  // namespace rtn

@@ -1982,6 +1982,7 @@ struct BwdChoice {
   int groups_per_launch = 0;   // batch groups of every problem that one launch takes
   bool local = false;          // every group on one XCD
   size_t lds = 0;              // dynamic shared memory of the kernel
+  int rq = 0;                  // float32: quads of rows per group where the product goes in them, else 0
 };
 
 int bwd_calls(const rtn_lstm2_bwd_call* calls, int count, int64_t T, int32_t B, int32_t n, int32_t dtype, void* workspace,
@@ -2106,6 +2107,40 @@ int choose_bwd_kernel(const BwdCtx& x, BwdChoice* out) {
   const int candidates[][4] = {{4, 2, 4, 1}, {8, 1, 4, 0}, {8, 1, 8, 0}, {8, 2, 4, 0}, {16, 1, 4, 0}, {16, 1, 8, 0}, {16, 2, 4, 0}, {8, 4, 4, 0}, {16, 4, 4, 0}};
   const DeviceInfo di = device_info();
   const long want_local = env_long("RTN_LSTM2_BWD_LOCAL", 1);
+  // Groups of up to 8 rows in float32: the product in quads of rows (a group's rows: the batch dealt evenly to the groups).
+  auto quads = [&](int rows) {
+    const int groups = (B + rows - 1) / rows, bg = (B + groups - 1) / groups;
+    return dtype == RTN_DTYPE_F32 && bg <= 8 && !env_long("RTN_LSTM2_NO_QUAD", 0) ? (bg + 3) / 4 : 0;
+  };
+  // Where float32 groups of up to 8 rows fit an XCD each: tiles per workgroup and rows per group with the fewest MFMAs per
+  // frame (tiles * quads); among these the fewest tiles (two directions, n = 256, B = 40: 1 tile and 5 rows against 2 tiles and
+  // 4 rows, 1.09 ms against 1.18 for a training step of 200 frames), unless more tiles spare every CU 32 KB of derivatives
+  // per frame (n = 512, B = 64: 2 tiles and 4 rows against 1 tile and 8 rows, 1.52 ms against 1.58).
+  if (dtype == RTN_DTYPE_F32 && want_local && di.xcds > 1 && !env_mt && !env_rows && !env_waves && quads(1)) {
+    for (int mt = 1; mt <= 4; mt *= 2) {
+      const int ksb = (S + kWaves - 1) / kWaves;
+      int room = 2;
+      while (room < ksb) room *= 2;
+      if (mt * room > 64 || (n / 16) % mt) continue;
+      const long long G = n / (16 * mt), cap = (long long)di.xcds * (di.cus / di.xcds / G) / count;
+      if (cap < 1) continue;
+      const int rows = std::max<int>(4, (int)((B + cap - 1) / cap));
+      if (rows > 8) continue;
+      const int rq = quads(rows);
+      const bool fewer_bytes = best.kernel && (best.rows_per_group - rows) * 16LL * n >= 32 * 1024;
+      if (best.kernel && (mt * rq > best.tiles * best.rq || (mt * rq == best.tiles * best.rq && !fewer_bytes))) continue;
+      BwdChoice c;
+      c.kernel = (const void*)bwd_regw_table_f32_quads(room, mt, kWaves, rq);
+      if (!c.kernel) continue;
+      c.ksb = ksb; c.tiles = mt; c.rows_per_group = rows; c.rq = rq; c.local = true;
+      c.groups_per_launch = (B + rows - 1) / rows;
+      best = c;
+    }
+    if (best.kernel) {
+      *out = best;
+      return RTN_OK;
+    }
+  }
   for (const auto& cand : candidates) {
     const int rows = cand[0], mt = cand[1];
     const int wv = env_waves ? (int)env_waves : cand[2];
@@ -2124,8 +2159,12 @@ int choose_bwd_kernel(const BwdCtx& x, BwdChoice* out) {
     // spills part of W, in float32 most of it): half of it lives in LDS.
     const bool lds_share = ksb_room * wv == 256;
     if (lds_share && (mt != 1 || (wv != 4 && wv != 8))) continue;
-    BwdRegwKernel kfn;
-    if (lds_share)
+    BwdRegwKernel kfn = nullptr;
+    int rq = 0;
+    if (!lds_share && use_rows <= 8 && (rq = quads(use_rows)) && !(kfn = bwd_regw_table_f32_quads(ksb_room, mt, wv, rq))) rq = 0;
+    if (kfn)
+      ;
+    else if (lds_share)
       kfn = dtype == RTN_DTYPE_BF16 ? bwd_regw_lds_table_bf16(wv) : bwd_regw_lds_table_f32(wv);
     else
       // ring frames of 8 rows: the variant whose loads take two macro steps at once
@@ -2138,6 +2177,7 @@ int choose_bwd_kernel(const BwdCtx& x, BwdChoice* out) {
     c.tiles = mt;
     c.waves = wv;
     c.rows_per_group = use_rows;
+    c.rq = rq;
     c.lds = lds_share ? kBwdLdsShareBytes : 0;
     if (c.lds && (rc = ensure_lds_limit(c.kernel, c.lds)) != RTN_OK) return rc;
     int per_cu = 0;
@@ -2255,10 +2295,11 @@ int bwd_launch_persistent(const BwdCtx& x, const BwdChoice& ch, const BwdLayout&
     q.ksb = ch.ksb;
     // The kernels that keep one (row, k) pair per thread ask for a frame's inputs in front of the MFMAs, so only the
     // delay stands between a frame's stores and the read of its ring slot: inside an XCD it is a fixed one there, as in
-    // the forward kernel (measured: 2.77 ms at 10 units against 2.82 adaptive and 2.87 / 2.86 at 4 / 16 for the layer).
+    // the forward kernel (measured: 2.77 ms at 10 units against 2.82 adaptive and 2.87 / 2.86 at 4 / 16 for the layer; float32
+    // in quads of rows 1.085 ms at 5 units, 1.117 adaptive, 1.087 / 1.087 / 1.125 at 0 / 10 / 20).
     const bool one_pair = ch.rows_per_group <= 8 && ((ch.tiles + ch.waves / 4 - 1) / (ch.waves / 4)) % 2 == 0;
-    const bool fixed_delay = ch.local && one_pair;
-    q.poll_delay = (int)std::max<long>(0, std::min<long>(64, env_long("RTN_LSTM2_BWD_POLL_DELAY", fixed_delay ? 10 : 20)));
+    const bool fixed_delay = ch.local && (one_pair || ch.rq > 0);
+    q.poll_delay = (int)std::max<long>(0, std::min<long>(64, env_long("RTN_LSTM2_BWD_POLL_DELAY", fixed_delay ? (ch.rq > 0 ? 5 : 10) : 20)));
     q.delay_inc = (int)std::max<long>(0, std::min<long>(16, env_long("RTN_LSTM2_BWD_DELAY_INC", fixed_delay ? 0 : 2)));
     {
       long dec = env_long("RTN_LSTM2_BWD_DELAY_DEC", 16);  // steps per unit of downward adaptation: a power of two
@@ -2494,9 +2535,9 @@ int bwd_calls(const rtn_lstm2_bwd_call* calls, int count, int64_t T, int32_t B, 
     const int bgroups = (B + ch.rows_per_group - 1) / ch.rows_per_group;
     char buf[256];
     if (ch.kernel)
-      snprintf(buf, sizeof(buf), "kernel=%s problems=%d rows_per_group=%d groups=%d tiles=%d waves=%d wgs_per_group=%d launches=%d",
+      snprintf(buf, sizeof(buf), "kernel=%s problems=%d rows_per_group=%d groups=%d tiles=%d waves=%d wgs_per_group=%d launches=%d row_quads=%d",
                ch.local ? "bwd_regw_xcd" : "bwd_regw", count, ch.rows_per_group, bgroups, ch.tiles, ch.waves, np / (16 * ch.tiles),
-               (bgroups + ch.groups_per_launch - 1) / std::max(ch.groups_per_launch, 1));
+               (bgroups + ch.groups_per_launch - 1) / std::max(ch.groups_per_launch, 1), ch.rq);
     else
       snprintf(buf, sizeof(buf), "kernel=%s problems=%d launches_per_frame=%d", mfma ? "bwd_step" : "bwd_generic", count, mfma ? 1 : 2);
     g_bwd_plan_text = buf;

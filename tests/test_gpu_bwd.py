@@ -85,6 +85,21 @@ def test_bwd_forced_decompositions(rows, tiles, waves, dtype):
         assert _rel_to_max(a, b) <= bar, (name, _rel_to_max(a, b), plan)
 
 
+# float32 groups of up to 8 rows on one XCD each: one and two quads of rows with 1, 2 and 4 tiles, cut quads and groups, every
+# number of macro steps per wavefront, odd widths
+@pytest.mark.parametrize("B,n,tiles,quads", [(1, 512, 1, 1), (30, 500, 1, 1), (61, 512, 2, 1), (37, 512, 1, 2), (128, 512, 2, 2), (97, 301, 2, 2), (60, 256, 1, 1), (205, 224, 2, 2),
+                                             (300, 256, 4, 2), (17, 128, 1, 1), (9, 64, 1, 1), (6, 33, 1, 1)])
+def test_bwd_quads_of_rows(B, n, tiles, quads):
+    announce("bwd quads of rows", B, n, tiles, quads)
+    for start, step in [(0, 1), (1, -2)]:
+        got, want, _ = _run(6, B, n, "f32", start, step, seed=B + n)
+        plan = lib.bwd_plan_text()
+        assert "bwd_regw_xcd" in plan and "tiles=%i " % tiles in plan and "row_quads=%i" % quads in plan, plan
+        for name, a, b in zip(("DX", "DW", "Dy0", "Dc0"), got, want):
+            assert numpy.isfinite(a).all(), name
+            assert _rel_to_max(a, b) <= 2e-5, (name, _rel_to_max(a, b), plan)
+
+
 def test_bwd_read_delay_only_moves_time():
     """The delay between a frame's stores and the read of its ring slot (and whether it adapts) decides how often a read is
     repeated, never what is read: every setting gives the same bits, on a plan with one pair per thread and on one without."""
