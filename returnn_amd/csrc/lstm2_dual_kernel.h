@@ -1,0 +1,380 @@
+// gfx950 kernel of the NativeLstm2 forward op for batches that take the register kernel several launches: two launches' rows
+// in one, taken in turn step by step.
+#pragma once
+
+#include "lstm2_kernels.h"
+
+namespace rtn {
+
+// LDS: the partial tiles of either set, then per set one copy of X and the mask and of the staged H, Y and C.
+struct DualLds {
+  unsigned red, xl, hs, ys, cs, ml, set, total;  // xl ... ml: inside a set's part, which starts at red + index * set behind the tiles
+  unsigned x_row, y_row, c_row;
+};
+__host__ __device__ constexpr DualLds dual_lds(int es, int MT) {
+  DualLds l{};
+  const unsigned cells = 4u * MT;
+  l.x_row = 4u * cells * es + kRowPad;
+  l.y_row = cells * es + kRowPad;
+  l.c_row = cells * 4u + kRowPad;
+  l.red = 2u * kWaves * MT * kTileBytes;
+  unsigned off = 0;
+  l.xl = off; off += 16u * l.x_row + 16u;
+  l.hs = off; off += 16u * l.x_row + 16u;
+  l.ys = off; off += (16u * l.y_row + 15u) / 16u * 16u;
+  l.cs = off; off += 16u * l.c_row;
+  l.ml = off; off += 16u * 4u + 16u;
+  l.set = off;
+  l.total = l.red + 2u * l.set;
+  return l;
+}
+
+// A workgroup holds its slice of W in registers as k_lstm2_regw does and works on TWO groups of up to 16 rows with it: group
+// g of multi.p[0] and group g of multi.p[1] (the same problem at another group_offset).  A step of one group is a chain --
+// hidden state in, MFMAs, partial tiles through LDS, gates, hidden state out and to every other CU of the XCD -- of which the
+// matrix cores take a fifth and the hand-over about half; here the one group's hand-over runs while the other's products and
+// gates are worked on.  Each half step asks for the other group's hidden state behind its MFMAs (it left its writers half a
+// step ago), so that what remains exposed are the two groups' own MFMAs, barriers and gates.
+// With two barriers per step one LDS copy of every stream is enough: X and the mask of one group move from registers to LDS
+// in the other group's half, staged outputs leave in the own group's next half.
+// What bounds it now is how fast one wavefront per SIMD issues: of 8000 clocks per step of both groups (bf16 n = 1024, B = 256:
+// 3.3 us, 4.3 in turns) 3600 are the MFMAs (2048 alone) with the loads, stores and LDS traffic between them, 2100 the gates,
+// 700 staging, 1100 looking over h, 400 the barriers.  (The gates of one group woven into the other's MFMAs took 5200 clocks
+// instead of 3600 + 2100, and left the hand-over exposed: 842 us against 690.)
+// The order of additions is that of k_lstm2_regw: the same bits.
+template <typename AT, int MT, int KS>
+__global__ __launch_bounds__(kWgThreads) void k_lstm2_dual(const Lstm2Multi multi) {
+  using E = Elem<AT>;
+  using SN = Sentinel<AT>;
+  using LM = LaneMax<AT>;
+  constexpr int KE = E::KE, KM = E::KM, ES = (int)sizeof(AT);
+  constexpr int EPT = MT / kWaves, CELLS = 4 * MT, ROWS = 16;
+  static_assert(MT % kWaves == 0, "whole tiles per wavefront in the pointwise part");
+  constexpr DualLds L = dual_lds(ES, MT);
+  const Lstm2Params p = multi.p[0];
+  const int X = multi.xcds, G = p.wgs_per_group;
+  const int xcd = (int)blockIdx.x % X, slot = (int)blockIdx.x / X;
+  const int g = (slot / G) * X + xcd, r = slot % G;
+  if (g >= p.groups) return;
+
+  extern __shared__ __align__(16) unsigned char smem[];
+  typedef f32x4 RedBuf[kWaves][MT][64];
+  RedBuf* red = (RedBuf*)smem;  // [2]
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = p.n, S = n / KM, nc = p.nc, nsteps = p.nsteps;
+  const long long bn = (long long)p.B * nc;
+  const int group[2] = {g + p.group_offset, g + multi.p[1].group_offset};
+  const int kg = lane >> 4, jl = lane & 15;
+
+  // Streams, as in k_lstm2_regw; offsets are relative to a group's first row, rows beyond the batch end lie behind the frame.
+  constexpr int SEG = CELLS * ES, CPS = SEG / 16, XCH = (ROWS * 4 * CPS + kWgThreads - 1) / kWgThreads;
+  constexpr int YCH = (ROWS * CPS + kWgThreads - 1) / kWgThreads;
+  constexpr int SEGC = CELLS * 4, CCH = (ROWS * (SEGC / 16) + kWgThreads - 1) / kWgThreads;
+  typedef Chunk<16> CK;
+  const int cell0 = CELLS * r;
+  unsigned xoff[XCH], hoff[XCH], yoff[YCH], coff[CCH], xlds[XCH], ylds[YCH], clds[CCH];
+#pragma unroll
+  for (int i = 0; i < XCH; ++i) {
+    const int c = tid + kWgThreads * i;
+    const int row = c / (4 * CPS), gate = (c / CPS) % 4, part = c % CPS;
+    const bool there = row < p.Bg && cell0 + (part + 1) * KE <= nc;
+    xoff[i] = there ? (unsigned)(((long long)row * p.ldX + gate * nc + cell0) * ES + part * 16) : kOobOffset;
+    hoff[i] = there ? (unsigned)(((long long)row * 4 * nc + gate * nc + cell0) * ES + part * 16) : kOobOffset;
+    xlds[i] = row < ROWS ? (unsigned)(row * L.x_row + gate * SEG + part * 16) : (unsigned)(ROWS * L.x_row);
+  }
+#pragma unroll
+  for (int i = 0; i < YCH; ++i) {
+    const int c = tid + kWgThreads * i, row = c / CPS, part = c % CPS;
+    yoff[i] = row < p.Bg && cell0 + (part + 1) * KE <= nc ? (unsigned)(((long long)row * p.ldY + cell0) * ES + part * 16) : kOobOffset;
+    ylds[i] = (unsigned)(min(row, ROWS - 1) * L.y_row + part * 16);
+  }
+#pragma unroll
+  for (int i = 0; i < CCH; ++i) {
+    const int c = tid + kWgThreads * i, row = c / (SEGC / 16), part = c % (SEGC / 16);
+    coff[i] = row < p.Bg && cell0 + (part + 1) * 4 <= nc ? (unsigned)((row * nc + cell0) * 4 + part * 16) : kOobOffset;
+    clds[i] = (unsigned)(min(row, ROWS - 1) * L.c_row + part * 16);
+  }
+  const unsigned moff = tid < p.Bg ? (unsigned)(tid * 4) : kOobOffset;
+  const long long frame_x = (long long)p.B * p.ldX * ES, frame_h = (long long)p.B * 4 * nc * ES, frame_y = (long long)p.B * p.ldY * ES,
+                  frame_c = bn * 4, frame_m = (long long)p.B * 4;
+
+  // ---- per group
+  const unsigned hx_buf_bytes = (unsigned)((size_t)n * p.Bp * ES);
+  __amdgpu_buffer_rsrc_t ring[2];
+  const unsigned char *x_at[2], *m_at[2];  // the frame that is fetched next, at the group's first row
+  unsigned char *h_at[2], *y_at[2], *c_at[2];  // the frame whose staged outputs leave next
+  unsigned left_x[2], left_h[2], left_y[2], left_c[2], left_m[2];  // bytes of a frame from the group's first row on (0: no such row)
+  unsigned frag[2];  // this lane's fragment of macro step `wave` in a ring buffer; out of range: a row the group does not have
+  int rows[2];
+#pragma unroll
+  for (int d = 0; d < 2; ++d) {
+    const long long b0 = (long long)group[d] * p.Bg, t0 = frame_of(p, 0);
+    rows[d] = (int)max(0LL, min((long long)p.Bg, p.B - b0));
+    ring[d] = __builtin_amdgcn_make_buffer_rsrc((unsigned char*)p.hx + (size_t)group[d] * kHxRing * hx_buf_bytes, 0, kHxRing * hx_buf_bytes, kBufFlags);
+    const long long bs = min(b0, (long long)p.B);
+    x_at[d] = (const unsigned char*)p.X + t0 * frame_x + bs * p.ldX * ES;
+    m_at[d] = (const unsigned char*)p.mask + t0 * frame_m + bs * 4;
+    h_at[d] = (unsigned char*)p.H + t0 * frame_h + bs * 4 * nc * ES;
+    y_at[d] = (unsigned char*)p.Y + t0 * frame_y + bs * p.ldY * ES;
+    c_at[d] = (unsigned char*)p.C + t0 * frame_c + bs * nc * 4;
+    left_x[d] = (unsigned)(frame_x - bs * p.ldX * ES);
+    left_h[d] = (unsigned)(frame_h - bs * 4 * nc * ES);
+    left_y[d] = (unsigned)(frame_y - bs * p.ldY * ES);
+    left_c[d] = (unsigned)(frame_c - bs * nc * 4);
+    left_m[d] = (unsigned)(frame_m - bs * 4);
+    frag[d] = jl < rows[d] ? (unsigned)(((4 * wave + kg) * p.Bp + jl) * kFragBytes) : kOobOffset;
+  }
+  const long long step_x = (long long)p.step * frame_x, step_h = (long long)p.step * frame_h, step_y = (long long)p.step * frame_y,
+                  step_c = (long long)p.step * frame_c, step_m = (long long)p.step * frame_m;
+  CK::T xv[2][XCH];
+  float mv[2] = {0.f, 0.f};
+  auto fetch = [&](auto set_tag, bool enabled) {  // the next frame of X and the mask into registers
+    constexpr int D = decltype(set_tag)::value;
+    __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void*)x_at[D], 0, enabled ? left_x[D] : 0u, kBufFlags);
+    __amdgpu_buffer_rsrc_t mr = __builtin_amdgcn_make_buffer_rsrc((void*)m_at[D], 0, enabled ? left_m[D] : 0u, kBufFlags);
+#pragma unroll
+    for (int i = 0; i < XCH; ++i) xv[D][i] = CK::load(xr, xoff[i]);
+    mv[D] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(mr, moff, 0, 0));
+    x_at[D] += step_x;
+    m_at[D] += step_m;
+  };
+  auto put = [&](auto set_tag) {  // registers -> LDS
+    constexpr int D = decltype(set_tag)::value;
+    unsigned char* base = smem + L.red + D * L.set;
+#pragma unroll
+    for (int i = 0; i < XCH; ++i) *(CK::T*)(base + L.xl + xlds[i]) = xv[D][i];
+    ((float*)(base + L.ml))[tid < ROWS ? tid : ROWS] = mv[D];
+  };
+  CK::T fh[XCH], fy[YCH], fc[CCH];
+  auto flush_read = [&](auto set_tag) {  // staged outputs -> registers
+    constexpr int D = decltype(set_tag)::value;
+    const unsigned char* base = smem + L.red + D * L.set;
+#pragma unroll
+    for (int i = 0; i < XCH; ++i) fh[i] = *(const CK::T*)(base + L.hs + xlds[i]);
+#pragma unroll
+    for (int i = 0; i < YCH; ++i) fy[i] = *(const CK::T*)(base + L.ys + ylds[i]);
+#pragma unroll
+    for (int i = 0; i < CCH; ++i) fc[i] = *(const CK::T*)(base + L.cs + clds[i]);
+  };
+  auto flush_write = [&](auto set_tag, bool enabled) {  // ... -> H, Y, C (a frame that does not exist: a buffer of no bytes)
+    constexpr int D = decltype(set_tag)::value;
+    __amdgpu_buffer_rsrc_t hr = __builtin_amdgcn_make_buffer_rsrc((void*)h_at[D], 0, enabled ? left_h[D] : 0u, kBufFlags);
+    __amdgpu_buffer_rsrc_t yr = __builtin_amdgcn_make_buffer_rsrc((void*)y_at[D], 0, enabled ? left_y[D] : 0u, kBufFlags);
+    __amdgpu_buffer_rsrc_t cr = __builtin_amdgcn_make_buffer_rsrc((void*)c_at[D], 0, enabled ? left_c[D] : 0u, kBufFlags);
+#pragma unroll
+    for (int i = 0; i < XCH; ++i) CK::store(fh[i], hr, hoff[i]);
+#pragma unroll
+    for (int i = 0; i < YCH; ++i) CK::store(fy[i], yr, yoff[i]);
+#pragma unroll
+    for (int i = 0; i < CCH; ++i) CK::store(fc[i], cr, coff[i]);
+    h_at[D] += enabled ? step_h : 0;
+    y_at[D] += enabled ? step_y : 0;
+    c_at[D] += enabled ? step_c : 0;
+  };
+
+  // W: this wavefront's macro steps of the workgroup's tiles; slots past its share hold zeros and meet the fragment of slot 0.
+  const int ks_count = S > wave ? (S - wave + kWaves - 1) / kWaves : 0;
+  i32x4 wreg[MT][KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      wreg[mt][ks] = i32x4{0, 0, 0, 0};
+      if (ks < ks_count) wreg[mt][ks] = ((const i32x4*)p.Wp)[((size_t)(r * MT + mt) * S + wave + kWaves * ks) * 64 + lane];
+    }
+
+  // The (sequence, cell) pairs of this thread, the same in both groups.
+  float c_state[2][EPT], h_prev[2][EPT];
+  unsigned e_hoff[EPT], e_cl[EPT];
+  const unsigned e_row = (unsigned)jl;
+#pragma unroll
+  for (int j = 0; j < EPT; ++j) {
+    const int cl = 4 * (wave + kWaves * j) + kg, cell = cell0 + cl;
+    e_cl[j] = (unsigned)cl;
+    e_hoff[j] = (unsigned)((((cell / KE) * p.Bp + jl) * KE + (cell % KE)) * ES);
+#pragma unroll
+    for (int d = 0; d < 2; ++d) {
+      c_state[d][j] = h_prev[d][j] = 0.f;
+      if (jl < rows[d] && cell < nc) {
+        const long long bc = ((long long)group[d] * p.Bg + jl) * nc + cell;
+        c_state[d][j] = p.c0[bc];
+        h_prev[d][j] = E::load(p.y0, bc);
+      }
+    }
+  }
+
+  // That all workgroups of a group share an XCD is checked (both groups of a workgroup have the same workgroups).
+  __shared__ int s_local;
+  if (tid == 0) s_local = group_on_one_xcd(p.flags + (size_t)group[0] * G, (unsigned)G, p.status, p.timeout_ticks) ? 1 : 0;
+
+  auto run = [&](auto ex_tag) {
+    constexpr int AUXS = decltype(ex_tag)::value == kExDevice ? kAuxDevice : 0, AUXL = kAuxDevice;
+    RTN_TRACE_DECL
+    i32x4 bf[2][KS];
+    auto load = [&](auto set_tag, int s, int ks) {
+      constexpr int D = decltype(set_tag)::value;
+      const unsigned soff = (unsigned)(s & (kHxRing - 1)) * hx_buf_bytes + (ks < ks_count ? ks : 0) * (unsigned)(4 * kWaves * kFragBytes) * p.Bp;
+      bf[D][ks] = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(ring[D], frag[D], soff, AUXL));
+    };
+    auto issue = [&](auto set_tag, int s) {  // read the hidden state that enters step s
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) load(set_tag, s, ks);
+      asm volatile("" ::: "memory");
+    };
+    auto half = [&](int s, auto set_tag) {
+      constexpr int D = decltype(set_tag)::value, O = 1 - D;
+      unsigned char* const base = smem + L.red + D * L.set;
+      auto complete = [&]() {
+        unsigned m[4] = {0, 0, 0, 0};
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+          for (int w = 0; w < 4; ++w) m[w] = LM::fold(m[w], (unsigned)bf[D][ks][w]);
+        return !__any(LM::has_sentinel(LM::fold(LM::fold(m[0], m[1]), LM::fold(m[2], m[3]))));
+      };
+      // (The first look stands outside the loop: behind these loads stand the other group's stores, for which a wait that
+      // also has to serve the loop's own reads would wait too.)
+      if (!complete()) {
+        unsigned long long t0 = 0;
+        unsigned spins = 0;
+        do {
+          if ((spins++ & 15u) == 0) {
+            if (__hip_atomic_load(p.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) break;
+            const unsigned long long now = wall_clock64();
+            if (spins == 1) {
+              t0 = now;
+            } else if (now - t0 > p.timeout_ticks) {
+              __hip_atomic_store(p.status, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+              break;
+            }
+          }
+          issue(set_tag, s);
+        } while (!complete());
+      }
+      RTN_TRACE_MARK(0)  // wait for h_{s-1}
+      // (Vector memory operations of a wavefront end in the order they were issued: with h_{s-1}, asked for behind the stores
+      // of this group's step s-1, the re-arming stores of that step have ended too, before anything of step s goes out.)
+      f32x4 acc[MT];
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) acc[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+      AT x_in[EPT][4];
+      const unsigned char* xin = base + L.xl + e_row * L.x_row;
+#pragma unroll
+      for (int j = 0; j < EPT; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) x_in[j][q] = *(const AT*)(xin + e_cl[j] * ES + q * SEG);
+      const float m = ((const float*)(base + L.ml))[e_row];
+      flush_read(set_tag);
+      put(IntTag<O>{});
+      flush_write(set_tag, s > 0);
+      // The other group's hidden state is asked for between the MFMAs of the second half, a load every MT / 2 of them (a CU
+      // takes 16 clocks for each of the four wavefronts' loads): it was handed over a quarter of a step before, about the time
+      // it takes to be visible on the other CUs.  (n = 1024, B = 256: 669 us for 200 steps; all loads behind the last MFMA 690,
+      // behind the barrier 735, behind the gates 797, at the end 852; all in the middle 710, in front of the MFMAs 807.)
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int i = 0; i < KS * MT; ++i) {
+        const int ks = i / MT, mt = i % MT;
+        if (i >= KS * MT / 2 && i % (MT / 2) == 0) {
+          __builtin_amdgcn_sched_barrier(0);
+          load(IntTag<O>{}, D ? s + 1 : s, i / (MT / 2) - KS);
+        }
+        acc[mt] = E::mma(wreg[mt][ks], bf[D][ks], acc[mt]);
+        __builtin_amdgcn_sched_group_barrier(0x008, sizeof(AT) == 2 ? 1 : 4, 0);
+        __builtin_amdgcn_sched_group_barrier(0x096, 3, 0);
+      }
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+      // The other group's X for the half step after next: behind the loads of h, which would wait for it otherwise.
+      fetch(IntTag<O>{}, D ? s + 2 < nsteps : s + 1 < nsteps);
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) red[D][wave][mt][lane] = acc[mt];
+      RTN_TRACE_MARK(1)  // MFMAs, streams, partial tiles to LDS
+      __syncthreads();
+      RTN_TRACE_MARK(2)  // barrier
+      unsigned h_bits[EPT];
+      float g_act[EPT][4], y_out[EPT];
+#pragma unroll
+      for (int j = 0; j < EPT; ++j) {
+        f32x4 part[kWaves];
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) part[w] = red[D][w][wave + kWaves * j][lane];
+        __builtin_amdgcn_sched_barrier(0);
+        f32x4 gsum = part[0];
+#pragma unroll
+        for (int w = 1; w < kWaves; ++w) gsum += part[w];
+        const float a0 = Act<AT>::tanh(gsum[0] + (float)x_in[j][0]);
+        const float a1 = Act<AT>::sigmoid(gsum[1] + (float)x_in[j][1]);
+        const float a2 = Act<AT>::sigmoid(gsum[2] + (float)x_in[j][2]);
+        const float a3 = Act<AT>::sigmoid(gsum[3] + (float)x_in[j][3]);
+        const float om = 1.f - m, pc = c_state[D][j];
+        const float c = (pc * a2 + a0 * a1) * m + pc * om;
+        const float y = E::round(Act<AT>::tanh(c) * a3 * m);
+        const float hn = (p.op_flags & kOpNoCarry) ? y : E::round(y + h_prev[D][j] * om);
+        c_state[D][j] = c;
+        h_prev[D][j] = hn;
+        h_bits[j] = SN::bits(hn);
+        g_act[j][0] = (p.op_flags & kOpH0IsCell) ? c : a0;
+        g_act[j][1] = a1; g_act[j][2] = a2; g_act[j][3] = a3;
+        y_out[j] = y;
+      }
+      const unsigned nxt = (unsigned)((s + 1) & (kHxRing - 1)) * hx_buf_bytes, arm = (unsigned)((s + 3) & (kHxRing - 1)) * hx_buf_bytes;
+#pragma unroll
+      for (int j = 0; j < EPT; ++j) SN::template store<AUXS>(ring[D], e_hoff[j] + nxt, h_bits[j]);
+#pragma unroll
+      for (int j = 0; j < EPT; ++j) SN::template store<AUXS>(ring[D], e_hoff[j] + arm, SN::kSentinel);
+      RTN_TRACE_MARK(3)  // gates, exchange stores
+#pragma unroll
+      for (int j = 0; j < EPT; ++j) {
+        unsigned char* hq = base + L.hs + e_row * L.x_row + e_cl[j] * ES;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) *(AT*)(hq + q * SEG) = (AT)g_act[j][q];
+        *(AT*)(base + L.ys + e_row * L.y_row + e_cl[j] * ES) = (AT)y_out[j];
+        *(float*)(base + L.cs + e_row * L.c_row + e_cl[j] * 4) = c_state[D][j];
+      }
+      RTN_TRACE_MARK(4)  // staging
+    };
+    fetch(IntTag<0>{}, true);
+    fetch(IntTag<1>{}, true);
+    put(IntTag<0>{});
+    fetch(IntTag<0>{}, nsteps > 1);
+    issue(IntTag<0>{}, 0);
+    __syncthreads();
+    for (int s = 0; s < nsteps; ++s) {
+      half(s, IntTag<0>{});
+      half(s, IntTag<1>{});
+    }
+    RTN_TRACE_FLUSH(p, g * G + r)
+  };
+  __syncthreads();  // s_local
+  if (s_local)
+    run(IntTag<kExLocal>{});
+  else
+    run(IntTag<kExDevice>{});
+  __syncthreads();  // the last step's outputs are staged
+  // (As in k_lstm2_regw: an expired wait must show in what a consumer reads.)
+  const bool expired = wait_expired(p.status);
+  if (expired && tid == 0) report_expired(p.status);
+  auto finish = [&](auto set_tag) {
+    constexpr int D = decltype(set_tag)::value;
+    flush_read(set_tag);
+    if (expired) {
+#pragma unroll
+      for (int i = 0; i < YCH; ++i) fy[i] = CK::fill(kNanWords<AT>);
+    }
+    flush_write(set_tag, true);
+#pragma unroll
+    for (int j = 0; j < EPT; ++j)
+      if (jl < rows[D] && cell0 + (int)e_cl[j] < nc) {
+        const long long bc = ((long long)group[D] * p.Bg + jl) * nc + cell0 + e_cl[j];
+        p.d[bc] = expired ? __builtin_nanf("") : c_state[D][j];
+        if (p.hN) E::store(p.hN, bc, expired ? __builtin_nanf("") : h_prev[D][j]);
+      }
+  };
+  finish(IntTag<0>{});
+  finish(IntTag<1>{});
+}
+
+}  // namespace rtn

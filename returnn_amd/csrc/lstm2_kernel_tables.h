@@ -6,6 +6,7 @@
 
 #include "lstm2_bwd_kernels.h"
 #include "lstm2_kernels.h"
+#include "lstm2_dual_kernel.h"
 #include "lstm2_solo_kernel.h"
 #include "lstm2_wide_kernel.h"
 
@@ -27,6 +28,9 @@ struct SoloBuild {
   int threads;
 };
 SoloBuild solo_kernel(int dtype, int n);
+
+// k_lstm2_dual<__bf16, 8, 8>: two turns of a large batch in one launch.
+RegwKernel dual_kernel();
 
 // Forward kernel for wide layers k_lstm2_wide<AT, MT, NT, KS, LF>.
 typedef void (*WideKernel)(const Lstm2Params);

@@ -5,7 +5,7 @@
 #include "lstm2_kernel_tables.h"
 
 #ifndef RTN_TABLE_PART
-#error "compile with -DRTN_TABLE_PART=<1..13>"
+#error "compile with -DRTN_TABLE_PART=<1..14>"
 #endif
 
 namespace rtn {
@@ -163,8 +163,10 @@ BwdRegwKernel bwd_regw_table_f32_quads2(int KSB, int MT, int WV);
 BwdRegwKernel bwd_regw_table_f32_quads(int KSB, int MT, int WV, int RQ) { return RQ == 1 ? bwd_regw_table_quad<1>(KSB, MT, WV) : RQ == 2 ? bwd_regw_table_f32_quads2(KSB, MT, WV) : nullptr; }
 #elif RTN_TABLE_PART == 13
 BwdRegwKernel bwd_regw_table_f32_quads2(int KSB, int MT, int WV) { return bwd_regw_table_quad<2>(KSB, MT, WV); }
+#elif RTN_TABLE_PART == 14
+RegwKernel dual_kernel() { return &k_lstm2_dual<__bf16, 8, 8>; }
 #else
-#error "RTN_TABLE_PART must be 1..13"
+#error "RTN_TABLE_PART must be 1..14"
 #endif
 
 }  // namespace rtn

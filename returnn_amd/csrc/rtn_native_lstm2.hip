@@ -171,6 +171,7 @@ struct Plan {
   bool regw = false;             // persistent kernel with W in registers and self-validating exchange
   bool local = false;            // regw: every batch group on one XCD, hidden state exchanged through that XCD's L2
   int rq = 0;                    // regw, float32: quads of rows per group where the product goes in them, else 0
+  bool dual = false;             // regw in turns: two turns' groups in one launch, taken in turn step by step
   bool wide = false;             // persistent kernel for layers whose W takes registers and LDS of the whole device
   WideBuild wide_build = {nullptr, 0, 0, 0, 0, 0};
   bool solo = false;             // small layer: every workgroup takes 4 rows through all steps by itself
@@ -180,6 +181,7 @@ struct Plan {
   int KSMAX = 0;                 // its macro steps per wavefront (template bound)
   int MT = 1, NT = 1;
   int groups = 1, wgs_per_group = 1, Bg = 1, Bp = 16;  // groups: per persistent launch
+  int groups_alloc = 1;          // groups the workspace has room for
   int groups_total = 1;          // groups of the whole batch
   int passes = 1;                // persistent launches in turn, each on `groups` of the groups (the last on the rest)
   size_t lds_bytes = 0;
@@ -452,6 +454,10 @@ bool make_plan_uncached(int64_t T, int B, int n, int dtype, int want_mode, bool 
         pl.passes = (pl.groups_total + pl.groups - 1) / pl.groups;
         pl.grid = chosen.local ? chosen.grid : pl.groups * chosen.G;
         pl.lds_bytes = chosen.lds;
+        // Two turns in one launch (k_lstm2_dual): on XCD-local groups with tiles and shares of W for which there is a build.
+        // (bf16 n = 1024, B = 256, T = 200: 869 us as two launches, 669 as one.)
+        pl.dual = di.valid && chosen.local && pl.passes > 1 && dtype == RTN_DTYPE_BF16 && chosen.MT == 8 && chosen.NT == 1 && chosen.KSMAX == 8 &&
+                  dual_lds((int)es, chosen.MT).total + 64 <= di.lds_per_wg && !env_long("RTN_LSTM2_NO_DUAL", 0);
         persistent_ok = true;
       }
       // Layers beyond the register kernel's widths (n > 2048 in bf16, > 1024 in float32): the wide kernel, which takes the
@@ -529,11 +535,13 @@ bool make_plan_uncached(int64_t T, int B, int n, int dtype, int want_mode, bool 
   pl.off_status = off;
   off += 256;
   pl.off_flags = off;
-  pl.n_flags = (pl.kind == kPlanMfma) ? pl.groups_total * pl.wgs_per_group : 0;
+  // (interleaved turns: the last one may have groups without rows, whose ring is there all the same)
+  pl.groups_alloc = pl.dual ? pl.passes * pl.groups : pl.groups_total;
+  pl.n_flags = (pl.kind == kPlanMfma) ? pl.groups_alloc * pl.wgs_per_group : 0;
   off = align_up(off + (size_t)pl.n_flags * 4, 256);
   if (pl.kind == kPlanMfma) {
     pl.off_hx = off;
-    off = align_up(off + (size_t)pl.groups_total * kHxRing * n * pl.Bp * es, 256);
+    off = align_up(off + (size_t)pl.groups_alloc * kHxRing * n * pl.Bp * es, 256);
     if (pl.wide) {
       pl.off_hxl = off;  // one set of copies, which the launches use in turn
       off = align_up(off + (size_t)di.xcds * kHxRing * n * pl.Bp * es, 256);
@@ -1243,7 +1251,7 @@ int fill_fwd_params(const rtn_lstm2_call& c, const Plan& pl, bool persistent, un
     p.nsteps = (int)((p.first - last) / (-(long long)c.step) + 1);
   }
   p.step = c.step;
-  p.groups = p.groups_total = pl.groups_total; p.wgs_per_group = pl.wgs_per_group; p.Bg = pl.Bg; p.Bp = pl.Bp;
+  p.groups = pl.groups_total; p.groups_total = pl.groups_alloc; p.wgs_per_group = pl.wgs_per_group; p.Bg = pl.Bg; p.Bp = pl.Bp;
   p.group_offset = 0;
   p.op_flags = op_flags;
   p.w_direct = (!persistent && pl.kind == kPlanMfma && pl.w_direct) ? 1 : 0;
@@ -1411,6 +1419,15 @@ int fwd_calls(const rtn_lstm2_call* calls, int count, int64_t T, int32_t B, int3
           one.grid = pl.local ? one.xcds * pl.wgs_per_group * ((one.p[0].groups + one.xcds - 1) / one.xcds) : one.p[0].groups * pl.wgs_per_group;
           one.wgs_each = (int)align_up((size_t)one.grid, (size_t)device_info().xcds);
           void* args[] = {(void*)&one};
+          // (k_lstm2_dual moves whole chunks of 16 bytes only)
+          if (pl.dual && g0 + pl.groups < pl.groups_total && p.nc % 8 == 0 && p.exchange == 0) {
+            const void* dk = (const void*)dual_kernel();
+            const size_t lds = dual_lds((int)esize(dtype), pl.MT).total;
+            one.p[1] = one.p[0];
+            one.p[1].group_offset = g0 += pl.groups;
+            if ((rc = ensure_lds_limit(dk, lds)) != RTN_OK || (rc = launch_coresident(dk, dim3(one.grid), dim3(kWgThreads), args, (unsigned)lds, stream, capturing)) != RTN_OK) return rc;
+            continue;
+          }
           rc = launch_coresident(pk, dim3(one.grid), dim3(kWgThreads), args, (unsigned)pl.lds_bytes, stream, capturing);
           if (rc != RTN_OK) return rc;
         }
@@ -1698,6 +1715,7 @@ const char* rtn_native_lstm2_describe_multi_plan(int32_t count, int64_t T, int32
              pl.NT, pl.groups, pl.wgs_per_group, (pl.mode == RTN_MODE_PERSISTENT && (pl.regw || pl.wide || pl.solo)) ? pl.grid : pl.groups * pl.wgs_per_group,
              pl.Bg, pl.passes, pl.lds_bytes,
              (count > 1 || n != n_asked) ? workspace_each(count, T, B, n_asked, dtype, mode) : pl.total);
+    if (pl.dual) snprintf(buf + strlen(buf), sizeof(buf) - strlen(buf), " interleaved=2");
     if (pl.rq) snprintf(buf + strlen(buf), sizeof(buf) - strlen(buf), " row_quads=%d", pl.rq);
     if (n != n_asked) snprintf(buf + strlen(buf), sizeof(buf) - strlen(buf), " padded_width=%d", n);
     if (pl.off_trace) snprintf(buf + strlen(buf), sizeof(buf) - strlen(buf), " trace_offset=%zu", pl.off_trace);
