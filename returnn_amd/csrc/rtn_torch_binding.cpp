@@ -6,7 +6,9 @@
 #include <torch/extension.h>
 
 #include <ATen/ATen.h>
+#include <ATen/autocast_mode.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPStream.h>
 
 #include <atomic>
@@ -173,6 +175,20 @@ struct Watched {
   void done(const at::Device& device, hipStream_t stream) {
     if (on) watch().after(device, stream);
   }
+};
+
+// ---- autocast -----------------------------------------------------------------------------------------------------
+// In an autocast region the layers' projection is a matrix product like torch's own: its operands take the region's type, by
+// casts that autograd sees (the errors come back in the operands' types, and no copy without a way back to its parameter
+// lands in the region's cache), and the recurrence runs in the type that the result has for the op (bfloat16, else float32).
+// Behind these casts autocast is off: the products below autograd, forward and gradient, choose their types themselves.
+std::optional<at::ScalarType> autocast_type() {
+  if (!at::autocast::is_autocast_enabled(at::kCUDA)) return std::nullopt;
+  return at::autocast::get_autocast_dtype(at::kCUDA);
+}
+
+struct NoAutocast {
+  c10::impl::ExcludeDispatchKeyGuard guard{c10::autocast_dispatch_keyset};
 };
 
 // ---- arguments ----------------------------------------------------------------------------------------------------
@@ -353,31 +369,6 @@ Tensor last_output(const Tensor& Y_in, const Tensor& y0_in, const Tensor& i_in, 
   return out;
 }
 
-// One step of a layer, projection included: (y, h, c) of x [B,in] and the state before (rtn_lstm_step).
-std::tuple<Tensor, Tensor, Tensor> lstm_step(const Tensor& x_in, const Tensor& h_in, const Tensor& c_in, const Tensor& ff_in, const Tensor& rec_in,
-                                             const std::optional<Tensor>& bias_in) {
-  TORCH_CHECK(ready, "NativeLstm2: the library is not loaded");
-  TORCH_CHECK(x_in.is_cuda(), "lstm: this build implements the LSTM for HIP (MI355X) tensors only; got a CPU tensor");
-  const bool bf16 = x_in.scalar_type() == at::kBFloat16;
-  const at::ScalarType act = bf16 ? at::kBFloat16 : at::kFloat;
-  const Tensor x = packed(as_type(x_in, act)), h = packed(as_type(h_in, act)), c = packed(as_type(c_in, at::kFloat)), ff = packed(as_type(ff_in, act)),
-               rec = packed(as_type(rec_in, act));
-  Tensor bias;
-  if (bias_in.has_value()) bias = packed(as_type(*bias_in, act));
-  const int64_t B = x.size(0), in = x.size(1), n = rec.size(0);
-  TORCH_CHECK(x.dim() == 2 && rec.dim() == 2 && rec.size(1) == 4 * n && ff.sizes() == at::IntArrayRef({4 * n, in}) && (!bias.defined() || bias.sizes() == at::IntArrayRef({4 * n})),
-              "lstm: parameters ", ff.sizes(), " / ", rec.sizes(), " do not match each other or the input ", x.sizes());
-  TORCH_CHECK(h.sizes() == at::IntArrayRef({B, n}) && c.sizes() == at::IntArrayRef({B, n}), "lstm: state_h ", h.sizes(), " / state_c ", c.sizes(), ", expected ",
-              at::IntArrayRef({B, n}));
-  for (const Tensor* t : {&h, &c, &ff, &rec}) TORCH_CHECK(t->device() == x.device(), "lstm: a tensor is on ", t->device(), " but the input is on ", x.device());
-  TORCH_CHECK(!bias.defined() || bias.device() == x.device(), "lstm: the bias is on another device than the input");
-  c10::DeviceGuard guard(x.device());
-  Tensor y = at::empty({B, n}, x.options()), h_out = at::empty({B, n}, x.options()), c_out = at::empty({B, n}, c.options());
-  check_rc(rtn_abi.lstm_step(x.data_ptr(), h.data_ptr(), c.data_ptr<float>(), ff.data_ptr(), rec.data_ptr(), bias.defined() ? bias.data_ptr() : nullptr, y.data_ptr(),
-                         h_out.data_ptr(), c_out.data_ptr<float>(), (int)B, (int)in, (int)n, bf16 ? RTN_DTYPE_BF16 : RTN_DTYPE_F32, current_stream(x.device())));
-  return {y, h_out, c_out};
-}
-
 // ---- the gradient op ----------------------------------------------------------------------------------------------
 struct BwdArgs {
   Tensor W, y0, c0, i, Y, C, H, DY, Dd;
@@ -494,7 +485,8 @@ struct Direction {
   int64_t step;
 };
 
-// P = source . ff + bias, rows of D * 4n gates; then the recurrences on it, their outputs side by side.
+// P = source . ff + bias, rows of D * 4n gates; then the recurrences on it, their outputs side by side.  (source, ff and bias
+// of one type, which need not be one of the op's: the recurrences take P as the op takes its input.)
 struct LayerRun {
   std::vector<Out4> outs;  // (Y view, C, H, d) per direction
   Tensor Y;                // [T,B,D*n]
@@ -519,6 +511,44 @@ LayerRun layer_forward(const Tensor& source, const Tensor& ff, const Tensor& bia
   return run;
 }
 
+// One step of a layer as a sequence of one frame, projected in `type`.
+std::tuple<Tensor, Tensor, Tensor> one_frame(const Tensor& x, const Tensor& h, const Tensor& c, const Tensor& ff, const Tensor& rec, const std::optional<Tensor>& bias,
+                                             at::ScalarType type) {
+  TORCH_CHECK(x.dim() == 2 && ff.dim() == 2 && ff.size(1) == x.size(1), "lstm: parameters ", ff.sizes(), " do not match the input ", x.sizes());
+  c10::DeviceGuard guard(x.device());
+  const Tensor mask = at::ones({1, x.size(0)}, x.options().dtype(at::kFloat));
+  const LayerRun run = layer_forward(as_type(x, type).unsqueeze(0), as_type(ff, type).t(), bias.has_value() ? as_type(*bias, type) : Tensor(), {{rec, h, c, 1}}, mask, true);
+  return {run.Y.select(0, 0), run.last[0], std::get<3>(run.outs[0])};
+}
+
+// One step of a layer, projection included: (y, h, c) of x [B,in] and the state before (rtn_lstm_step).
+std::tuple<Tensor, Tensor, Tensor> lstm_step(const Tensor& x_in, const Tensor& h_in, const Tensor& c_in, const Tensor& ff_in, const Tensor& rec_in,
+                                             const std::optional<Tensor>& bias_in) {
+  TORCH_CHECK(ready, "NativeLstm2: the library is not loaded");
+  TORCH_CHECK(x_in.is_cuda(), "lstm: this build implements the LSTM for HIP (MI355X) tensors only; got a CPU tensor");
+  const std::optional<at::ScalarType> region = autocast_type();
+  const NoAutocast no_autocast;
+  const bool bf16 = (region.has_value() ? *region : x_in.scalar_type()) == at::kBFloat16;
+  const at::ScalarType act = bf16 ? at::kBFloat16 : at::kFloat;
+  if (region.has_value() && *region != act) return one_frame(x_in, h_in, c_in, ff_in, rec_in, bias_in, *region);
+  const Tensor x = packed(as_type(x_in, act)), h = packed(as_type(h_in, act)), c = packed(as_type(c_in, at::kFloat)), ff = packed(as_type(ff_in, act)),
+               rec = packed(as_type(rec_in, act));
+  Tensor bias;
+  if (bias_in.has_value()) bias = packed(as_type(*bias_in, act));
+  const int64_t B = x.size(0), in = x.size(1), n = rec.size(0);
+  TORCH_CHECK(x.dim() == 2 && rec.dim() == 2 && rec.size(1) == 4 * n && ff.sizes() == at::IntArrayRef({4 * n, in}) && (!bias.defined() || bias.sizes() == at::IntArrayRef({4 * n})),
+              "lstm: parameters ", ff.sizes(), " / ", rec.sizes(), " do not match each other or the input ", x.sizes());
+  TORCH_CHECK(h.sizes() == at::IntArrayRef({B, n}) && c.sizes() == at::IntArrayRef({B, n}), "lstm: state_h ", h.sizes(), " / state_c ", c.sizes(), ", expected ",
+              at::IntArrayRef({B, n}));
+  for (const Tensor* t : {&h, &c, &ff, &rec}) TORCH_CHECK(t->device() == x.device(), "lstm: a tensor is on ", t->device(), " but the input is on ", x.device());
+  TORCH_CHECK(!bias.defined() || bias.device() == x.device(), "lstm: the bias is on another device than the input");
+  c10::DeviceGuard guard(x.device());
+  Tensor y = at::empty({B, n}, x.options()), h_out = at::empty({B, n}, x.options()), c_out = at::empty({B, n}, c.options());
+  check_rc(rtn_abi.lstm_step(x.data_ptr(), h.data_ptr(), c.data_ptr<float>(), ff.data_ptr(), rec.data_ptr(), bias.defined() ? bias.data_ptr() : nullptr, y.data_ptr(),
+                         h_out.data_ptr(), c_out.data_ptr<float>(), (int)B, (int)in, (int)n, bf16 ? RTN_DTYPE_BF16 : RTN_DTYPE_F32, current_stream(x.device())));
+  return {y, h_out, c_out};
+}
+
 using torch::autograd::AutogradContext;
 using torch::autograd::variable_list;
 
@@ -529,6 +559,7 @@ struct LayerFunction : torch::autograd::Function<LayerFunction> {
                                const Tensor& y00, const Tensor& c00, const std::optional<Tensor>& W1, const std::optional<Tensor>& y01, const std::optional<Tensor>& c01,
                                int64_t step0) {
     at::AutoDispatchBelowADInplaceOrView below;
+    const NoAutocast no_autocast;
     std::vector<Direction> dirs{{W0, y00, c00, step0}};
     if (W1.has_value()) dirs.push_back({*W1, *y01, *c01, -step0});
     const LayerRun run = layer_forward(source, ff, bias.has_value() ? *bias : Tensor(), dirs, mask, false);
@@ -545,6 +576,7 @@ struct LayerFunction : torch::autograd::Function<LayerFunction> {
   }
 
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const NoAutocast no_autocast;
     const auto saved = ctx->get_saved_variables();
     const Tensor &source = saved[0], &ff = saved[1], &mask = saved[2], &Y = saved[3];
     const int64_t step0 = ctx->saved_data["step"].toInt();
@@ -560,7 +592,7 @@ struct LayerFunction : torch::autograd::Function<LayerFunction> {
     }
     auto res = lstm2_grad_multi(args, true);
     const int64_t rows = source.size(0) * source.size(1);
-    const Tensor DP = res.second.view({rows, ff.size(1)});
+    const Tensor DP = as_type(res.second.view({rows, ff.size(1)}), ff.scalar_type());  // (the error of a projection of another type than the op's)
     variable_list out(11);
     if (ctx->needs_input_grad(0)) out[0] = at::mm(DP, ff.t()).view(source.sizes());
     // (the gradient of ff comes out in the layout of a [4n,in] parameter, whose transposed view ff usually is)
@@ -601,11 +633,17 @@ struct LastOutputFunction : torch::autograd::Function<LastOutputFunction> {
 
 // source [T,B,in], ff [in,D*4n], bias or None, mask [T,B]; W, y0, c0 per direction (the second runs against the first).
 // Returns Y [T,B,D*n], the final outputs (want_last) and the final cell states.
-py::tuple lstm_layer(const Tensor& source, const Tensor& ff, const std::optional<Tensor>& bias, const Tensor& mask, const std::vector<std::tuple<Tensor, Tensor, Tensor>>& directions,
+py::tuple lstm_layer(Tensor source, Tensor ff, std::optional<Tensor> bias, const Tensor& mask, const std::vector<std::tuple<Tensor, Tensor, Tensor>>& directions,
                      int64_t step, bool want_last) {
   std::vector<Direction> dirs;
   for (const auto& d : directions) dirs.push_back({std::get<0>(d), std::get<1>(d), std::get<2>(d), dirs.empty() ? step : -step});
   TORCH_CHECK(source.dim() == 3 && ff.dim() == 2 && (dirs.size() == 1 || dirs.size() == 2), "lstm_layer: bad arguments");
+  if (const auto region = autocast_type()) {
+    source = as_type(source, *region);
+    ff = as_type(ff, *region);
+    if (bias.has_value()) bias = as_type(*bias, *region);
+  }
+  const NoAutocast no_autocast;
   bool grad = false;
   if (at::GradMode::is_enabled()) {
     grad = source.requires_grad() || ff.requires_grad() || (bias.has_value() && bias->requires_grad());

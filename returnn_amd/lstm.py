@@ -182,7 +182,8 @@ def lstm(
     :param seq_lens: [B] integer lengths (any device), None = all sequences have T frames
     :param direction: +1, or -1 for the backward-in-time layer of a bidirectional pair
     :return: output [T,B,out] (or [B,out]), (h [B,out], c [B,out]) after each sequence's last processed frame;
-        output and h in the type of ``source``, c in float32
+        output and h in the type of ``source`` (bfloat16 or float32; under ``torch.autocast`` the projection runs in the
+        region's type, and output and h are bfloat16 where that is), c in float32
     """
     if direction not in (1, -1):
         raise ValueError("lstm: direction must be +1 or -1")
