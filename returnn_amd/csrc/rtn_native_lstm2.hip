@@ -196,6 +196,10 @@ struct Plan {
 constexpr int kMaxPassesOverLds = 3;
 constexpr int kMaxPassesOverSteps = 12;
 
+// Most turns of the wide kernel, and the frames from which on its plan does not depend on T any more.
+constexpr int kMaxWideTurns = 48;
+constexpr int64_t kWidePlanFrames = 256;
+
 size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 size_t esize(int dtype) { return dtype == RTN_DTYPE_BF16 ? 2 : 4; }
 int round_nt(int nt) { return nt <= 1 ? 1 : (nt <= 2 ? 2 : 4); }
@@ -203,6 +207,29 @@ int round_nt(int nt) { return nt <= 1 ? 1 : (nt <= 2 ? 2 : 4); }
 size_t mfma_lds_bytes(int n, int dtype, int MT, int NT) {
   const int KM = dtype == RTN_DTYPE_BF16 ? 32 : 16;
   return (size_t)MT * (n / KM) * kTileBytes + (size_t)kWaves * MT * NT * kTileBytes;
+}
+
+// Microseconds of `frames` steps of B rows on the wide kernel, in turns of up to 16 NT rows: every turn loads all of W (at 3.6
+// TB/s, and 8 us for a launch that follows another), and a step of it is the exchange and the MFMAs of one wavefront.
+double wide_turns_us(const WideBuild& wb, int64_t frames, int B, int n, int dtype) {
+  const int KM = dtype == RTN_DTYPE_BF16 ? 32 : 16, ks = (n / KM + kWaves - 1) / kWaves;
+  const double mb = 4e-6 * n * n * (double)esize(dtype), mfma_us = (double)wb.MT * wb.NT * ks * (dtype == RTN_DTYPE_BF16 ? 16 : 128) / 2400.0;
+  const int turns = (B + 16 * wb.NT - 1) / (16 * wb.NT);
+  return turns * (8 + mb / 3.6 + (1.3 + 2 * wb.NT + mfma_us) * (double)frames);
+}
+
+// ... and as one launch per step, which reads W once for up to 64 rows.
+double step_launches_us(int64_t frames, int B, int n, int dtype) {
+  const double mb = 4e-6 * n * n * (double)esize(dtype);
+  const int groups = (B + 63) / 64, rows = (B + groups - 1) / groups;
+  double step;
+  if (rows <= 16)
+    step = 2 + mb / 6.4;
+  else if (dtype == RTN_DTYPE_BF16)
+    step = rows <= 32 ? 9 + mb / 7 : groups == 1 ? 15 + mb / 6.2 : 6 + mb / 4.6;
+  else
+    step = rows <= 32 ? 2 + mb / 2.75 : groups == 1 ? mb / 1.9 : 2 + mb / 2.5;
+  return 18 + groups * step * (double)frames;
 }
 
 // Whether calls made under stream capture keep the persistent kernels (default) or record per-step launches.
@@ -469,7 +496,14 @@ bool make_plan_uncached(int64_t T, int B, int n, int dtype, int want_mode, bool 
         const int G = wb.kernel ? (n / 4 + wb.MT - 1) / wb.MT : 0;
         const long env_passes = env_long("RTN_LSTM2_MAX_PASSES", -1);
         const size_t lds = wb.kernel ? wide_lds_bytes(wb.MT, wb.NT, wb.LF) + 64 : 0;
-        if (wb.kernel && turns <= (env_passes >= 0 ? env_passes : kMaxPassesOverSteps * 4) && lds <= di.lds_per_wg && G >= 2 * di.xcds &&
+        // Few frames in many turns: launches per step, which read W once per step for up to 64 rows, are ahead of turns that
+        // load all of it for 16 or 32.  The two estimates are fitted to MI355X (us per call, wide / per step: bf16 n = 4096 with
+        // B = 256, T = 1, 8, 16: 806 / 206, 1359 / 1176, 1958 / 2287; n = 2080, B = 768, T = 1, 8: 625 / 184, 1720 / 1263; float32
+        // n = 2816, B = 64, T = 2, 8: 294 / 208, 564 / 663; float32 n = 1280, B = 100 at any T: 123 / 60 ... 1517 / 1274); of 554 calls with 1
+        // to 768 rows and 1 to 32 frames they take the slower side by more than 2 % in 22, the worst by 13 %.
+        // kMaxWideTurns is how far turns were measured (B = 768 at n = 4096 and 2816).
+        const bool worth = want_mode != RTN_MODE_AUTO || env_kernel == 3 || chosen.ok || (wb.kernel && wide_turns_us(wb, T, B, n, dtype) <= step_launches_us(T, B, n, dtype));
+        if (wb.kernel && worth && turns <= (env_passes >= 0 ? env_passes : kMaxWideTurns) && lds <= di.lds_per_wg && G >= 2 * di.xcds &&
             (n / (dtype == RTN_DTYPE_BF16 ? 8 : 4) * rows + G / di.xcds - 1) / (G / di.xcds) <= kWideForward * kWgThreads) {
           pl = Plan();
           pl.kind = kPlanMfma;
@@ -564,14 +598,14 @@ bool make_plan_uncached(int64_t T, int B, int n, int dtype, int want_mode, bool 
 
 // Plans are kept per (shape class, element type, mode, capture state, workgroups per CU, problems per launch, device,
 // environment snapshot): the search above runs once per key, and two threads that plan the same call get the same plan.
-// (T only matters as "no frames at all".)
+// (T only matters as "no frames at all", and up to kWidePlanFrames for layers that the wide kernel may take.)
 struct PlanCacheEntry {
   bool ok;
   Plan plan;
   std::string why;
 };
 std::mutex g_plan_mu;
-std::map<std::tuple<bool, int, int, int, int, bool, int, int, int, unsigned long long>, PlanCacheEntry> g_plans;
+std::map<std::tuple<int64_t, int, int, int, int, bool, int, int, int, unsigned long long>, PlanCacheEntry> g_plans;
 constexpr size_t kMaxCachedPlans = 4096;
 
 bool make_plan(int64_t T, int B, int n, int dtype, int want_mode, bool capturing, Plan* out, std::string* why,
@@ -581,7 +615,8 @@ bool make_plan(int64_t T, int B, int n, int dtype, int want_mode, bool capturing
     (void)hipGetLastError();
     dev = -1;
   }
-  const auto key = std::make_tuple(T == 0, B, n, dtype, want_mode, capturing, max_wgs_per_cu, count, dev, env_snapshot()->generation);
+  T = std::min<int64_t>(T, n > (dtype == RTN_DTYPE_BF16 ? 2048 : 1024) ? kWidePlanFrames : 1);
+  const auto key = std::make_tuple(T, B, n, dtype, want_mode, capturing, max_wgs_per_cu, count, dev, env_snapshot()->generation);
   {
     std::lock_guard<std::mutex> lock(g_plan_mu);
     auto it = g_plans.find(key);

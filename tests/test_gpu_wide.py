@@ -61,3 +61,24 @@ def test_bounded_wait_expires_cleanly():
     assert (rc, status, rc2, status2) == (0, 0, 0, 0)
     for name, a, b in zip("YCHd", got, want):
         assert numpy.array_equal(a, b), name
+
+
+@pytest.mark.parametrize("T,B,n,dtype", [(1, 65, 4096, "bf16"), (2, 80, 2080, "bf16"), (3, 300, 1280, "f32"), (2, 49, 2816, "f32")])
+def test_few_frames_of_many_rows_run_as_one_launch_per_step(T, B, n, dtype):
+    """Turns that load all of W for 16 or 32 rows are only taken where there are frames enough to make up for it; asked for,
+    they give the same bits.  A workspace that is enough for a longer call is enough for a shorter one on another plan."""
+    announce("wide layers, few frames", T, B, n, dtype)
+    p = random_problem(7100 + n, T, B, n)
+    dt = lib.DTYPE_BF16 if dtype == "bf16" else lib.DTYPE_F32
+    plan = lib.describe_plan(T, B, n, dt, lib.MODE_AUTO)
+    assert "mode=graph" in plan and "kernel=mfma_lds" in plan, plan
+    assert "kernel=mfma_regw_wide" in lib.describe_plan(200, 16, n, dt, lib.MODE_AUTO)
+    assert lib.workspace_bytes(T, B, n, dt, lib.MODE_AUTO) <= lib.workspace_bytes(200, B, n, dt, lib.MODE_AUTO)
+    rc, status, got = run_raw(*p, 0, 1, dtype=dtype)
+    assert rc == 0 and status == 0
+    with env(RTN_LSTM2_KERNEL=3):
+        plan = lib.describe_plan(T, B, n, dt, lib.MODE_AUTO)
+        rc, status, want = run_raw(*p, 0, 1, dtype=dtype)
+    assert "kernel=mfma_regw_wide" in plan and rc == 0 and status == 0
+    for name, a, b in zip("YCHd", got, want):
+        assert numpy.array_equal(a, b), name
