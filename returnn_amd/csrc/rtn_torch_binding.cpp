@@ -511,38 +511,44 @@ LayerRun layer_forward(const Tensor& source, const Tensor& ff, const Tensor& bia
   return run;
 }
 
-// One step of a layer as a sequence of one frame, projected in `type`.
-std::tuple<Tensor, Tensor, Tensor> one_frame(const Tensor& x, const Tensor& h, const Tensor& c, const Tensor& ff, const Tensor& rec, const std::optional<Tensor>& bias,
-                                             at::ScalarType type) {
-  TORCH_CHECK(x.dim() == 2 && ff.dim() == 2 && ff.size(1) == x.size(1), "lstm: parameters ", ff.sizes(), " do not match the input ", x.sizes());
-  c10::DeviceGuard guard(x.device());
-  const Tensor mask = at::ones({1, x.size(0)}, x.options().dtype(at::kFloat));
-  const LayerRun run = layer_forward(as_type(x, type).unsqueeze(0), as_type(ff, type).t(), bias.has_value() ? as_type(*bias, type) : Tensor(), {{rec, h, c, 1}}, mask, true);
-  return {run.Y.select(0, 0), run.last[0], std::get<3>(run.outs[0])};
-}
+// The one-step kernel reads all weights again for every 64 rows; a GEMM and the recurrent kernels take over where that is more
+// traffic than they make up for with their launches.  Measured on MI355X (us per call, one-step kernel / GEMM and recurrent
+// kernel): bf16 n = 1024 of 512 inputs, 12 to 2048 rows: 9 / 50 ... 148 / 156, 4096 rows (805 MB): 289 / 282; n = 2048 of 2048, 384
+// rows (403 MB): 167 / 205, 512 (537 MB): 214 / 142; float32 n = 1024 of 512, 512 rows (201 MB): 118 / 171, 1024 (403 MB): 232 / 191;
+// n = 2048 of 2048, 64 rows: 75 / 87, 128 (268 MB): 155 / 130.  Up to 64 rows it is ahead at every width measured (128 to 4096).
+constexpr double kStepTrafficBf16 = 410e6, kStepTrafficF32 = 260e6;
 
-// One step of a layer, projection included: (y, h, c) of x [B,in] and the state before (rtn_lstm_step).
+// One step of a layer, projection included: (y, h, c) of x [B,in] and the state before (rtn_lstm_step, or a sequence of one frame).
 std::tuple<Tensor, Tensor, Tensor> lstm_step(const Tensor& x_in, const Tensor& h_in, const Tensor& c_in, const Tensor& ff_in, const Tensor& rec_in,
                                              const std::optional<Tensor>& bias_in) {
   TORCH_CHECK(ready, "NativeLstm2: the library is not loaded");
   TORCH_CHECK(x_in.is_cuda(), "lstm: this build implements the LSTM for HIP (MI355X) tensors only; got a CPU tensor");
-  const std::optional<at::ScalarType> region = autocast_type();
-  const NoAutocast no_autocast;
-  const bool bf16 = (region.has_value() ? *region : x_in.scalar_type()) == at::kBFloat16;
-  const at::ScalarType act = bf16 ? at::kBFloat16 : at::kFloat;
-  if (region.has_value() && *region != act) return one_frame(x_in, h_in, c_in, ff_in, rec_in, bias_in, *region);
-  const Tensor x = packed(as_type(x_in, act)), h = packed(as_type(h_in, act)), c = packed(as_type(c_in, at::kFloat)), ff = packed(as_type(ff_in, act)),
-               rec = packed(as_type(rec_in, act));
-  Tensor bias;
-  if (bias_in.has_value()) bias = packed(as_type(*bias_in, act));
-  const int64_t B = x.size(0), in = x.size(1), n = rec.size(0);
-  TORCH_CHECK(x.dim() == 2 && rec.dim() == 2 && rec.size(1) == 4 * n && ff.sizes() == at::IntArrayRef({4 * n, in}) && (!bias.defined() || bias.sizes() == at::IntArrayRef({4 * n})),
-              "lstm: parameters ", ff.sizes(), " / ", rec.sizes(), " do not match each other or the input ", x.sizes());
-  TORCH_CHECK(h.sizes() == at::IntArrayRef({B, n}) && c.sizes() == at::IntArrayRef({B, n}), "lstm: state_h ", h.sizes(), " / state_c ", c.sizes(), ", expected ",
+  TORCH_CHECK(x_in.dim() == 2 && rec_in.dim() == 2, "lstm: input ", x_in.sizes(), " / rec ", rec_in.sizes());
+  const int64_t B = x_in.size(0), in = x_in.size(1), n = rec_in.size(0);
+  TORCH_CHECK(rec_in.size(1) == 4 * n && ff_in.sizes() == at::IntArrayRef({4 * n, in}) && (!bias_in.has_value() || bias_in->sizes() == at::IntArrayRef({4 * n})),
+              "lstm: parameters ", ff_in.sizes(), " / ", rec_in.sizes(), " do not match each other or the input ", x_in.sizes());
+  TORCH_CHECK(h_in.sizes() == at::IntArrayRef({B, n}) && c_in.sizes() == at::IntArrayRef({B, n}), "lstm: state_h ", h_in.sizes(), " / state_c ", c_in.sizes(), ", expected ",
               at::IntArrayRef({B, n}));
-  for (const Tensor* t : {&h, &c, &ff, &rec}) TORCH_CHECK(t->device() == x.device(), "lstm: a tensor is on ", t->device(), " but the input is on ", x.device());
-  TORCH_CHECK(!bias.defined() || bias.device() == x.device(), "lstm: the bias is on another device than the input");
-  c10::DeviceGuard guard(x.device());
+  for (const Tensor* t : {&h_in, &c_in, &ff_in, &rec_in}) TORCH_CHECK(t->device() == x_in.device(), "lstm: a tensor is on ", t->device(), " but the input is on ", x_in.device());
+  TORCH_CHECK(!bias_in.has_value() || bias_in->device() == x_in.device(), "lstm: the bias is on another device than the input");
+  c10::DeviceGuard guard(x_in.device());
+  // the type of the projection: the region's, else the op's
+  const at::ScalarType type = autocast_type().value_or(x_in.scalar_type() == at::kBFloat16 ? at::kBFloat16 : at::kFloat);
+  const NoAutocast no_autocast;
+  const bool bf16 = type == at::kBFloat16;
+  Tensor x = as_type(x_in, type), ff = as_type(ff_in, type), bias;
+  if (bias_in.has_value()) bias = as_type(*bias_in, type);
+  const int64_t shares = (B + 63) / 64;
+  const double traffic = (double)shares * 4 * n * (in + n) * (bf16 ? 2 : 4);
+  if ((!bf16 && type != at::kFloat) || (shares > 1 && traffic > (bf16 ? kStepTrafficBf16 : kStepTrafficF32))) {
+    const Tensor mask = at::ones({1, B}, x.options().dtype(at::kFloat));
+    const LayerRun run = layer_forward(x.unsqueeze(0), ff.t(), bias, {{rec_in, h_in, c_in, 1}}, mask, true);
+    return {run.Y.select(0, 0), run.last[0], std::get<3>(run.outs[0])};
+  }
+  x = packed(x);
+  ff = packed(ff);
+  if (bias.defined()) bias = packed(bias);
+  const Tensor h = packed(as_type(h_in, type)), c = packed(as_type(c_in, at::kFloat)), rec = packed(as_type(rec_in, type));
   Tensor y = at::empty({B, n}, x.options()), h_out = at::empty({B, n}, x.options()), c_out = at::empty({B, n}, c.options());
   check_rc(rtn_abi.lstm_step(x.data_ptr(), h.data_ptr(), c.data_ptr<float>(), ff.data_ptr(), rec.data_ptr(), bias.defined() ? bias.data_ptr() : nullptr, y.data_ptr(),
                          h_out.data_ptr(), c_out.data_ptr<float>(), (int)B, (int)in, (int)n, bf16 ? RTN_DTYPE_BF16 : RTN_DTYPE_F32, current_stream(x.device())));

@@ -43,3 +43,27 @@ def test_step_against_float64(B, n_in, n, bias, dtype):
     tol = 1e-2 if dtype == "bf16" else 2e-6
     for got, want in ((y, want_y), (st.c, want_c)):
         assert float((got.cpu().double() - want).abs().max()) <= tol
+
+
+@pytest.mark.parametrize("B,n_in,n,dtype", [(385, 2048, 2048, "bf16"), (65, 2048, 4096, "f32"), (641, 512, 1024, "f32"), (4096, 1024, 1000, "bf16")])
+def test_many_rows_run_as_a_sequence_of_one_frame(B, n_in, n, dtype):
+    """Where the one-step kernel would read the weights too often, the projection is a GEMM and the recurrent kernels follow:
+    the bits of a sequence of one frame.  (The one-step kernel adds in another order: one share of the batch has other bits.)"""
+    announce("lstm_step, many rows", B, n_in, n, dtype)
+    from returnn_amd.lstm import LSTM, LstmState
+
+    act = torch.bfloat16 if dtype == "bf16" else torch.float32
+    gen = torch.Generator(device="cuda").manual_seed(B)
+    m = LSTM(n_in, n, device="cuda", dtype=act).requires_grad_(False)
+    m.reset_parameters(gen)
+    x, h = (torch.randn((B, k), device="cuda", generator=gen).to(act) for k in (n_in, n))
+    st = LstmState(h=h, c=torch.randn((B, n), device="cuda", generator=gen))
+    y, new = m(x, state=st)
+    want, want_new = m(x[None], state=st)
+    assert torch.equal(y, want[0]) and torch.equal(new.h, want_new.h) and torch.equal(new.c, want_new.c)
+    assert new.h.data_ptr() != y.data_ptr()
+    few, _ = m(x[:64], state=LstmState(h=h[:64], c=st.c[:64]))
+    # (bfloat16: the sequence rounds the projection, values below 4 by up to 2^-7, which the four gates pass on with slopes of
+    # at most 1 + 1/4 + |c| / 4 + 1/4 < 2.75, and each output is rounded by 2^-9; float32: two orders of sums of up to 6144
+    # products, whose rounding errors of 2^-25 of sums below 4 add up like a random walk: 80 * 2^-23 < 1e-5)
+    assert not torch.equal(few, y[:64]) and float((few.float() - y[:64].float()).abs().max()) <= (2**-5 if dtype == "bf16" else 1e-5)
