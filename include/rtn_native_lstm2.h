@@ -44,8 +44,9 @@ extern "C" {
 #define RTN_DTYPE_BF16 1
 
 /* Widths: the matrix-core kernels take n that is a multiple of 32.  Any other n above 32 runs zero-padded to the next
- * multiple of 32 on copies inside the workspace (the size queries include them); the results are those of the
- * unpadded problem, since a padded cell has zero inputs, weights and state.  n up to 32 runs on element-wise kernels. */
+ * multiple of 32: the forward kernels pad on the fly, the gradient too where rows stay 16-byte aligned, else on copies
+ * inside the workspace (its size query includes them).  The results are those of the unpadded problem, since a padded
+ * cell has zero inputs, weights and state.  n below 32 runs on the small-layer kernel or on element-wise kernels. */
 
 /* Execution mode.
  * AUTO:       PERSISTENT when the shape and device allow it, else GRAPH.
@@ -109,8 +110,7 @@ size_t rtn_native_lstm2_fwd_workspace_bytes(int64_t T, int32_t B, int32_t n, int
  * It has no counterpart in the reference.  The scratch lives in a fixed array inside the library's code object
  * (20 MiB per GPU the library runs on, held until the process ends), so the problem's workspace
  * (rtn_native_lstm2_fwd_workspace_bytes) must fit 20 MiB -- that covers widths up to 1024 in both element types with
- * batches up to 128 rows (widths that are not a multiple of 32 need padded copies of all tensors and fit only when
- * small) -- else RTN_ERR_WORKSPACE.  The call allocates nothing on the device and calls
+ * batches up to 128 rows -- else RTN_ERR_WORKSPACE.  The call allocates nothing on the device and calls
  * no allocating runtime routine: AUTO resolves to PERSISTENT or to plain per-step launches, GRAPH is refused
  * (RTN_ERR_UNSUPPORTED).  Arguments, results and error codes are otherwise those of rtn_native_lstm2_fwd, bit for bit.
  * All calls on one GPU share that GPU's array: calls that overlap in time on one GPU race (keep them on one stream,

@@ -1154,12 +1154,7 @@ int resolve_pitch(const char* name, long long given, long long contiguous, int B
 
 // Workspace of one of `count` forward calls (call k's slice starts at k times this, with its status block first).
 size_t workspace_each(int count, int64_t T, int32_t B, int32_t n, int32_t dtype, int32_t mode) {
-  // For a padded width the size stays what it was when such widths ran on copies (X W y0 c0 Y C H d at the padded width):
-  // callers rely on the query, which is never smaller than for the width it is padded to plus those copies.
-  const int np = padded_width(n);
-  const size_t es = esize(dtype), tb = (size_t)T * B;
-  const size_t slack = np == n || T == 0 || B == 0 ? 0 : align_up(tb * np * (9 * es + 4) + (size_t)np * 4 * np * es + (size_t)B * np * (es + 8) + 8 * 256, 256);
-  n = np;
+  n = padded_width(n);  // (the kernels pad on the fly: the layout is that of the padded width)
   size_t need = 0;
   Plan pl;
   std::string why;
@@ -1171,7 +1166,7 @@ size_t workspace_each(int count, int64_t T, int32_t B, int32_t n, int32_t dtype,
       if (make_plan(T, B, n, dtype, RTN_MODE_STEPWISE, true, &pl, &why)) need = std::max(need, pl.total);
     }
   }
-  return need + slack;
+  return need;
 }
 
 int static_scratch(void** out);

@@ -63,8 +63,9 @@ def _run_static(X, W, y0, c0, i, start, step, dtype, mode):
         ("f32", "auto", (20, 16, 512), (7, 3, 64)),
         ("f32", "stepwise", (6, 4, 96), (3, 2, 32)),          # plain per-step launches
         ("f32", "auto", (5, 3, 24), (4, 2, 7)),               # element-wise kernels (widths below 32)
-        ("f32", "auto", (6, 4, 100), (3, 2, 40)),             # widths run zero-padded: the padded copies live in the array too
+        ("f32", "auto", (6, 4, 100), (3, 2, 40)),             # widths run zero-padded, on the fly
         ("bf16", "auto", (5, 8, 200), (4, 3, 72)),
+        ("bf16", "auto", (400, 32, 1000), (60, 7, 905)),      # ... so the array holds them however many frames there are
     ],
 )
 def test_static_entry_equals_the_workspace_entry_twice(dtype, mode, first, second):
@@ -100,3 +101,28 @@ def test_static_entry_limits():
                                           lib.DTYPE_F32, lib.MODE_AUTO, stream)
     assert rc == lib.RTN_ERR_RANGE
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("T,B,n,dtype,mode", [(90, 5, 100, "bf16", "auto"), (40, 9, 1000, "bf16", "auto"), (30, 140, 1000, "bf16", "auto"), (40, 11, 500, "f32", "auto"),
+                                              (20, 3, 2401, "bf16", "auto"), (25, 6, 333, "f32", "stepwise"), (25, 6, 333, "bf16", "graph"), (30, 7, 20, "f32", "stepwise")])  # fmt: skip
+def test_workspace_of_cut_widths_is_enough(T, B, n, dtype, mode):
+    """The kernels that pad on the fly stay within the bytes asked for, which are those of the padded width."""
+    announce("workspace of cut widths", T, B, n, dtype, mode)
+    cabi = lib.load()
+    X, W, y0, c0, i = random_problem(60 + n, T, B, n)
+    _, _, want = run_raw(X, W, y0, c0, i, 0, 1, dtype=dtype, mode="stepwise")
+    act = torch.bfloat16 if dtype == "bf16" else torch.float32
+    dt, md = (lib.DTYPE_BF16 if dtype == "bf16" else lib.DTYPE_F32), lib.MODES[mode]
+    Xd, Wd, y0d = (to_dev(a, dtype) for a in (X, W, y0))
+    c0d, id_ = (to_dev(a, "f32") for a in (c0, i))
+    out = [torch.empty(shape, dtype=ty, device="cuda:0") for shape, ty in (((T, B, n), act), ((T, B, n), torch.float32), ((T, B, 4 * n), act), ((B, n), torch.float32))]
+    size = lib.workspace_bytes(T, B, n, dt, md)
+    assert size == lib.workspace_bytes(T + 1, B, n, dt, md) and (n <= 32 or size == lib.workspace_bytes(T, B, (n + 31) // 32 * 32, dt, md))
+    ws = torch.full((size + 4096,), 0x5A, dtype=torch.uint8, device="cuda:0")
+    rc = cabi.rtn_native_lstm2_fwd(*(t.data_ptr() for t in (Xd, Wd, y0d, c0d, id_)), 0, 1, *(t.data_ptr() for t in out), T, B, n, dt, md, ws.data_ptr(), size,
+                                   torch.cuda.current_stream().cuda_stream)  # fmt: skip
+    assert rc == lib.RTN_OK, lib.last_error()
+    torch.cuda.synchronize()
+    assert bool((ws[size:] == 0x5A).all())
+    for name, a, b in zip("YCHd", out, want):
+        assert numpy.array_equal(a.float().cpu().numpy(), b), name
