@@ -1233,6 +1233,16 @@ int settle_fwd_plan(int count, int64_t T, int B, int nc, int n, int dtype, int m
     if ((rc = occupancy_per_cu(*pk, kWgThreads, pl.lds_bytes, &per_cu)) != RTN_OK) return rc;
     const long long capacity = (long long)per_cu * device_info().cus;
     if (capacity >= wgs) {
+      if (pl.dual) {
+        // Two turns in one launch take another kernel, with more LDS and registers: where that does not fit, the turns go one
+        // after the other.  (RTN_LSTM2_DUAL_PER_CU pretends an answer of the runtime.)
+        const void* dk = (const void*)dual_kernel();
+        const size_t lds = dual_lds((int)esize(dtype), pl.MT).total;
+        int dual_per_cu = 0;
+        if ((rc = ensure_lds_limit(dk, lds)) != RTN_OK || (rc = occupancy_per_cu(dk, kWgThreads, lds, &dual_per_cu)) != RTN_OK) return rc;
+        dual_per_cu = (int)env_long("RTN_LSTM2_DUAL_PER_CU", dual_per_cu);
+        pl.dual = (long long)dual_per_cu * device_info().cus >= wgs;
+      }
       if (pl.local) {
         *fused = plan_count;  // the plan's grid holds the groups of that many problems
       } else if (pl.regw && count > 1 && pl.passes == 1 && !env_long("RTN_LSTM2_NO_FUSE", 0)) {
@@ -1455,7 +1465,7 @@ int fwd_calls(const rtn_lstm2_call* calls, int count, int64_t T, int32_t B, int3
             const size_t lds = dual_lds((int)esize(dtype), pl.MT).total;
             one.p[1] = one.p[0];
             one.p[1].group_offset = g0 += pl.groups;
-            if ((rc = ensure_lds_limit(dk, lds)) != RTN_OK || (rc = launch_coresident(dk, dim3(one.grid), dim3(kWgThreads), args, (unsigned)lds, stream, capturing)) != RTN_OK) return rc;
+            if ((rc = launch_coresident(dk, dim3(one.grid), dim3(kWgThreads), args, (unsigned)lds, stream, capturing)) != RTN_OK) return rc;
             continue;
           }
           rc = launch_coresident(pk, dim3(one.grid), dim3(kWgThreads), args, (unsigned)pl.lds_bytes, stream, capturing);

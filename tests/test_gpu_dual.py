@@ -3,12 +3,15 @@ launches, bit for bit."""
 
 from __future__ import annotations
 
+import re
+
 import numpy
 import pytest
+import torch
 
 from returnn_amd import lib
 
-from _gpu_util import announce, env, random_problem, run_raw
+from _gpu_util import announce, env, get_op, random_problem, run_raw, to_dev
 
 pytestmark = pytest.mark.gpu
 
@@ -32,3 +35,29 @@ def test_interleaved_turns_equal_per_step_launches(T, B, n, start, step):
         for name, a, b in zip("YCHd", got, want):
             assert numpy.isfinite(a).all(), name
             assert numpy.array_equal(a, b), "%s differs from per-step launches (%s)" % (name, plan)
+
+
+def test_turns_one_by_one_where_two_do_not_fit():
+    """The plan's two turns in one launch need another kernel than the turns: where the device does not hold that one, the call
+    runs as two launches, with the same results (counted as recorded under stream capture)."""
+    announce("dual kernel that does not fit")
+    X, W, y0, c0, i = random_problem(8100, 5, 200, 1024)
+    args = [to_dev(a, "bf16") for a in (X, W, y0)] + [to_dev(a, "f32") for a in (c0, i)]
+    op = get_op()
+    launches = []
+    for per_cu in (None, 0):
+        with env(RTN_LSTM2_DUAL_PER_CU=per_cu):
+            want = op(*args, 0, 1)
+            torch.cuda.synchronize()
+            before = sum(int(v) for v in re.findall(r"\d+(?= as)", lib.capture_report()))
+            graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+            side.wait_stream(torch.cuda.current_stream())
+            with torch.cuda.graph(graph, stream=side):
+                got = op(*args, 0, 1)
+            launches.append(sum(int(v) for v in re.findall(r"\d+(?= as)", lib.capture_report())) - before)
+        for _ in range(3):
+            graph.replay()
+            torch.cuda.synchronize()
+            for name, a, b in zip("YCHd", got, want):
+                assert torch.equal(a, b), name
+    assert launches == [1, 2], launches
