@@ -398,3 +398,46 @@ def test_gradient_from_two_host_threads_on_their_own_streams():
                 assert _rel_to_max(a.double().cpu().numpy(), b.double().cpu().numpy()) <= 1e-5, (k, r, name)
             else:
                 assert torch.equal(a, b), "thread %i, round %i: %s differs from the single-threaded result" % (k, r, name)
+
+
+@pytest.mark.parametrize("dtype,bar", [("f32", 2e-5), ("bf16", 2e-2)])
+@pytest.mark.parametrize("B,n", [(5, 72), (3, 30)])
+def test_autograd_functions_of_two_directions(B, n, dtype, bar):
+    """The differentiable calls of both directions, on separate gates and on one projection, against two of one direction."""
+    T = 6
+    announce("autograd of two directions", B, n, dtype)
+    get_op()
+    single, pair, bidir = torch_native_op.NativeLstm2Function, torch_native_op.NativeLstm2PairFunction, torch_native_op.NativeLstm2BidirFunction
+    leaves, weights = [], []
+    for k in range(2):
+        X, W, y0, c0, i = random_problem(6100 + k, T, B, n)
+        leaves.append([to_dev(a, dtype) for a in (X, W, y0)] + [to_dev(c0, "f32")])
+        mask = to_dev(i, "f32")
+        rng = numpy.random.default_rng(6200 + k)
+        weights.append((to_dev(rng.normal(0, 1, (T, B, n)), dtype), to_dev(rng.normal(0, 1, (B, n)), "f32")))
+
+    def gradients(run):
+        args = [[t.clone().requires_grad_() for t in direction] for direction in leaves]
+        Y, d = run(*args)
+        torch.autograd.backward(list(Y) + list(d), [w for w, _ in weights] + [w for _, w in weights])
+        return [t.detach() for t in (*Y, *d)] + [t.grad for direction in args for t in direction]
+
+    def run_single(f, b):
+        outs = [single.apply(*f, mask, 0, 1), single.apply(*b, mask, 0, -1)]
+        return [o[0] for o in outs], [o[3] for o in outs]
+
+    def run_pair(f, b):
+        Yf, _, _, df, Yb, _, _, db = pair.apply(*f, *b, mask)
+        return [Yf, Yb], [df, db]
+
+    def run_bidir(f, b):
+        Y, df, db = bidir.apply(torch.cat((f[0], b[0]), -1), *f[1:], *b[1:], mask)
+        return [Y[..., :n], Y[..., n:]], [df, db]
+
+    want = gradients(run_single)
+    for run in (run_pair, run_bidir):
+        for k, (a, b) in enumerate(zip(gradients(run), want)):
+            assert a.shape == b.shape and a.dtype == b.dtype
+            if k < 4:
+                assert torch.equal(a, b), (run.__name__, k)
+            assert _rel_to_max(a.float().cpu().numpy(), b.float().cpu().numpy()) <= bar, (run.__name__, k)
