@@ -63,6 +63,15 @@ def measured_traffic(workload: str, launches: int, plan: str):
     return None, None
 
 
+def forward_kernel(plan: str):
+    """-> (the kernel a forward plan runs on, whether that is the register kernel whose steps the library's probes repeat)"""
+    name = plan.split("kernel=")[1].split()[0]
+    kernel = {"mfma_regw_solo": "k_lstm2_solo", "mfma_regw_wide": "k_lstm2_wide", "mfma_lds": "k_lstm2_mfma"}.get(name, "k_step_generic")
+    if name in ("mfma_regw", "mfma_regw_xcd", "mfma_regw_xcd_half"):
+        kernel = "k_lstm2_dual" if "interleaved=2" in plan else "k_lstm2_regw"
+    return kernel, kernel == "k_lstm2_regw"
+
+
 def algorithmic_bytes_per_unit(n: int, dtype: str) -> int:
     """HBM bytes per timestep x sequence: read X (4n), write H (4n), Y (n) in the activation type,
     write C (n, fp32), read the mask (4 bytes)."""
@@ -874,6 +883,8 @@ def main():
     assert measuring_only or all(bool(torch.isfinite(o["d"]).all()) for o in outs)
 
     call_ms = sum(a.elapsed_time(b) for a, b in events) / len(events)
+    plan = lib.describe_multi_plan(2 if fused else 1, T, B, n, dt_code, mode)
+    kernel, has_probes = forward_kernel(plan)
 
     # The latency of one hand-over of values between CUs (device-scope store -> load), measured live with the library's
     # probe: a lower bound of a time step of any kernel that keeps W spread over CUs.
@@ -881,7 +892,7 @@ def main():
     probe_rounds = 4000
     probe_ws = torch.empty((32768,), dtype=torch.uint8, device=dev)
     pe = []
-    for _ in range(1 + 3):
+    for _ in range(1 + 3 if kernel != "k_lstm2_solo" else 0):  # (which hands nothing over)
         e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
         e0.record(stream)
         rc = cabi.rtn_handover_latency_probe(probe_ws.data_ptr(), probe_ws.numel(), probe_rounds, stream.cuda_stream)
@@ -911,8 +922,8 @@ def main():
         torch.cuda.synchronize()
         return min(a.elapsed_time(b) for a, b in se[1:])
 
-    seq_ms = time_probe(cabi.rtn_mfma_sequence_probe)
-    issue_ms = time_probe(cabi.rtn_mfma_issue_probe)
+    seq_ms = time_probe(cabi.rtn_mfma_sequence_probe) if has_probes else None
+    issue_ms = time_probe(cabi.rtn_mfma_issue_probe) if has_probes else None
     issue_clock_mhz = None
     if issue_ms is not None:
         # threads 1 and 2 of every workgroup of the issue probe leave the loop's duration in shader clocks and in ticks
@@ -949,7 +960,7 @@ def main():
     # results are invalid and the status word says so): what a step costs when the hidden state is there for free.
     # The difference to the measured launch is what the step spends on getting it.
     nowait_ms = None
-    if "mfma_regw" in lib.describe_multi_plan(2 if fused else 1, T, B, n, dt_code, mode) and not measuring_only and not args.no_step_budget:
+    if has_probes and not measuring_only and not args.no_step_budget:
         os.environ["RTN_LSTM2_EXCHANGE"] = "3"
         lib.reload_env()
         try:
@@ -978,7 +989,6 @@ def main():
     achieved = flops_per_launch / (call_ms * 1e-3)
     peak = PEAK_MFMA[dtype]
     bytes_per_launch = algorithmic_bytes_per_unit(n, dtype) * units_per_launch
-    plan = lib.describe_multi_plan(2 if fused else 1, T, B, n, dt_code, mode)
     traffic, traffic_source = measured_traffic(args.workload, launches, plan)
 
     result = {
@@ -1018,8 +1028,7 @@ def main():
             "traffic_unit": "bytes per launch (rocprofv3 FETCH_SIZE + WRITE_SIZE, transcribed from the profile summary named in "
             "traffic_source, not measured by this run); algorithmic: %i" % bytes_per_launch,
             "kernel": "%s (one launch = %i op call(s) = %i units of T*B, 8*n^2 flops each)"
-            % ("k_lstm2_regw" if "mfma_regw" in plan else ("k_lstm2_mfma" if "mfma_lds" in plan else "k_step_generic"),
-               len(directions) // launches, units_per_launch),
+            % (kernel, len(directions) // launches, units_per_launch),
             "launch_ms": call_ms,
             **ceiling_fields(probe_us, seq_ms, issue_ms, units_per_launch // T, n, dtype, T, call_ms),
             "mfma_issue_clock_mhz": issue_clock_mhz,

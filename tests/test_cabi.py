@@ -279,3 +279,15 @@ def test_fake_impl_shapes(cabi):
     with FakeTensorMode():
         outs = op(torch.zeros(T, B, 4 * n), torch.zeros(n, 4 * n), torch.zeros(B, n), torch.zeros(B, n), torch.ones(T, B), 0, 1)
     assert [tuple(o.shape) for o in outs] == [(T, B, n), (T, B, n), (T, B, 4 * n), (B, n)]
+
+
+def test_bench_names_the_kernel_of_the_plan():
+    """bench.py's report names the kernel that ran, and applies the probes of the register kernel's steps to that one only."""
+    import bench
+
+    plan = "mode=persistent kernel=%s mt=8 nt=1 groups=4 wgs_per_group=32 wgs=256 rows_per_group=8 launches=1 lds=1 workspace=1"
+    for name, want in (("mfma_regw", "k_lstm2_regw"), ("mfma_regw_xcd", "k_lstm2_regw"), ("mfma_regw_xcd_half", "k_lstm2_regw"), ("mfma_regw_solo", "k_lstm2_solo"),
+                       ("mfma_regw_wide", "k_lstm2_wide"), ("mfma_lds", "k_lstm2_mfma"), ("generic", "k_step_generic")):  # fmt: skip
+        assert bench.forward_kernel(plan % name) == (want, want == "k_lstm2_regw")
+    assert bench.forward_kernel(plan % "mfma_regw_xcd" + " interleaved=2") == ("k_lstm2_dual", False)
+    assert bench.forward_kernel(lib.describe_plan(1000, 32, 1024, lib.DTYPE_BF16, lib.MODE_AUTO)) == ("k_lstm2_regw", True)
