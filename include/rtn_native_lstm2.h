@@ -375,6 +375,15 @@ int rtn_lstm_step(const void* x, const void* h, const float* c, const void* ff, 
                   float* c_out, int32_t B, int32_t in_dim, int32_t n, int32_t dtype, void* hip_stream);
 
 /*
+ * out [width] = sums over the rows of data [rows,width] (contiguous, 16-byte aligned, width a multiple of 4), accumulated
+ * in float32 and stored in element type `out_dtype`: the gradient of a bias that was added to all frames.  Kernel launches
+ * only, nothing is cleared first, so that a caller's graph can record it.  `workspace`: rtn_column_sums_workspace_bytes().
+ */
+int rtn_column_sums(const void* data, int64_t rows, int32_t width, int32_t dtype, void* out, int32_t out_dtype, void* workspace,
+                    size_t workspace_bytes, void* hip_stream);
+size_t rtn_column_sums_workspace_bytes(int64_t rows, int32_t width);
+
+/*
  * Where the calling thread's calls report an expired bounded wait, besides the status word of their workspace: a kernel
  * whose wait expires stores `id` into *word (a 32-bit word the device can write, e.g. of pinned host memory; null, the
  * initial setting: nowhere).  Holds for all later calls of this thread.  The word has to stay valid until their kernels
@@ -429,7 +438,7 @@ const char* rtn_native_lstm2_bwd_plan_text(void);
  */
 void rtn_native_lstm2_reload_env(void);
 
-/* ABI version of this header: 14. */
+/* ABI version of this header: 15. */
 int rtn_native_lstm2_abi_version(void);
 
 #ifdef __cplusplus

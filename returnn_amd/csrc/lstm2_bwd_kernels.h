@@ -921,22 +921,53 @@ __global__ void k_low_mem_gates(void* data, const void* bias, long long rows, in
   }
 }
 
-// Column sums of data[rows, width] in two deterministic stages: partial[r, c] = sum of rows r, r + R, ... (R = gridDim.y),
-// then out[c] = sum over r in ascending order.
-template <typename AT>
-__global__ void k_column_partial_sums(const void* data, float* partial, long long rows, int width) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= width) return;
-  float acc = 0.f;
-  for (long long r = blockIdx.y; r < rows; r += gridDim.y) acc += Elem<AT>::load(data, r * width + c);
-  partial[(long long)blockIdx.y * width + c] = acc;
-}
-static __global__ void k_column_final_sums(const float* partial, float* out, int parts, int width) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= width) return;
-  float acc = 0.f;
-  for (int r = 0; r < parts; ++r) acc += partial[(long long)r * width + c];
-  out[c] = acc;
+// Sums over the rows of data[rows, width] (width a multiple of V, V elements = 8 or 16 aligned bytes): block (x, y) sums rows
+// y * R ... y * R + R - 1 of 64 V columns into out[y, width].  Bound by reading data once: a wavefront's load is 1 KB of a row, four of
+// which are in flight.  Wavefront w takes rows w, w + 4, ... into four sums per column, which are added pairwise, as are the
+// wavefronts': short chains of additions, and the same order in every call.
+template <typename AT, typename OT, int V>
+__global__ __launch_bounds__(256) void k_column_sums(const void* data, void* out, long long rows, int width, int R) {
+  struct __attribute__((aligned(sizeof(AT) * V))) Piece { AT v[V]; };
+  __shared__ float red[3][V][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = ((int)blockIdx.x * 64 + lane) * V;
+  const long long first = (long long)blockIdx.y * R, end = first + R < rows ? first + R : rows;
+  float acc[4][V];
+#pragma unroll
+  for (int u = 0; u < 4; ++u)
+#pragma unroll
+    for (int v = 0; v < V; ++v) acc[u][v] = 0.f;
+  if (c < width) {
+    const AT* at = (const AT*)data + c;
+    long long r = first + wave;
+    for (; r + 12 < end; r += 16) {
+      Piece p[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) p[u] = *(const Piece*)(at + (r + 4 * u) * width);
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int v = 0; v < V; ++v) acc[u][v] += (float)p[u].v[v];
+    }
+#pragma unroll
+    for (int u = 0; u < 3; ++u, r += 4)
+      if (r < end) {
+        const Piece p = *(const Piece*)(at + r * width);
+#pragma unroll
+        for (int v = 0; v < V; ++v) acc[u][v] += (float)p.v[v];
+      }
+  }
+  float sum[V];
+#pragma unroll
+  for (int v = 0; v < V; ++v) {
+    sum[v] = (acc[0][v] + acc[1][v]) + (acc[2][v] + acc[3][v]);
+    if (wave) red[wave - 1][v][lane] = sum[v];
+  }
+  __syncthreads();
+  if (wave == 0 && c < width) {
+#pragma unroll
+    for (int v = 0; v < V; ++v)
+      Elem<OT>::store(out, (long long)blockIdx.y * width + c + v, (sum[v] + red[0][v][lane]) + (red[1][v][lane] + red[2][v][lane]));
+  }
 }
 
 }  // namespace rtn

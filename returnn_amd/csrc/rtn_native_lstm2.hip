@@ -1674,6 +1674,49 @@ int mfma_probe(bool issue_only, int32_t count, int64_t T, int32_t B, int32_t n, 
   return RTN_OK;
 }
 
+// Rows per part of a sum over the rows of a matrix: at most 128 parts, whose sums a second launch adds.
+int column_sum_rows(int64_t rows) { return (int)align_up((size_t)std::max<int64_t>(64, (rows + 127) / 128), 16); }
+
+size_t column_sums_bytes(int64_t rows, int width) {
+  const int64_t R = column_sum_rows(rows), parts = (rows + R - 1) / R;
+  return parts > 1 ? align_up((size_t)parts * width * 4, 256) : 0;
+}
+
+// out[width] (element type out_dtype) = sums over the rows of data[rows, width], in float32.  Two launches and no clearing of
+// memory, so that it can be recorded into a graph (torch's sum over many rows records a memset, after which replays have
+// given other values).
+template <typename AT, typename OT>
+int column_sums_of(const void* data, int64_t rows, int width, void* out, void* workspace, hipStream_t stream) {
+  constexpr int V = 16 / (int)sizeof(AT);
+  const int R = column_sum_rows(rows), parts = (int)std::max<int64_t>(1, (rows + R - 1) / R);
+  const dim3 block(256);
+  const auto launch = [&](auto piece, auto type) {
+    constexpr int P = decltype(piece)::value;
+    hipLaunchKernelGGL((k_column_sums<AT, decltype(type), P>), dim3((unsigned)((width + 64 * P - 1) / (64 * P)), (unsigned)parts), block, 0, stream, data, parts > 1 ? workspace : out,
+                       (long long)rows, width, R);
+  };
+  const auto by_width = [&](auto type) {
+    if (width % V == 0)
+      launch(std::integral_constant<int, V>{}, type);
+    else
+      launch(std::integral_constant<int, 4>{}, type);
+  };
+  if (parts == 1)
+    by_width(OT{});
+  else {
+    by_width(float{});
+    hipLaunchKernelGGL((k_column_sums<float, OT, 4>), dim3((unsigned)((width + 255) / 256)), block, 0, stream, workspace, out, (long long)parts, width, parts);
+  }
+  RTN_HIP(hipGetLastError());
+  return RTN_OK;
+}
+
+int column_sums(const void* data, int64_t rows, int width, int dtype, void* out, int out_dtype, void* workspace, hipStream_t stream) {
+  if (dtype == RTN_DTYPE_BF16)
+    return out_dtype == RTN_DTYPE_BF16 ? column_sums_of<__bf16, __bf16>(data, rows, width, out, workspace, stream) : column_sums_of<__bf16, float>(data, rows, width, out, workspace, stream);
+  return out_dtype == RTN_DTYPE_BF16 ? column_sums_of<float, __bf16>(data, rows, width, out, workspace, stream) : column_sums_of<float, float>(data, rows, width, out, workspace, stream);
+}
+
 // Device address of this GPU's copy of `scratch`: asked of the runtime once per device, with that device current.
 int static_scratch(void** out) {
   static std::mutex mu;
@@ -1699,7 +1742,7 @@ using namespace rtn;
 
 extern "C" {
 
-int rtn_native_lstm2_abi_version(void) { return 14; }
+int rtn_native_lstm2_abi_version(void) { return 15; }
 
 const char* rtn_native_lstm2_bwd_plan_text(void) { return g_bwd_plan_text.c_str(); }
 
@@ -2652,7 +2695,6 @@ int rtn_lstm_generic_base_bwd(const void* V_h, const float* c, const float* i, c
 }
 
 namespace {
-constexpr int kColumnSumParts = 64;
 struct LowMemBwdLayout {
   size_t bwd = 0, H = 0, DI = 0, partial = 0, total = 0;
 };
@@ -2666,7 +2708,7 @@ void low_mem_bwd_layout(int64_t T, int B, int n, int dtype, LowMemBwdLayout* out
   l.DI = off;
   off += frames;
   l.partial = off;
-  off += align_up((size_t)kColumnSumParts * 4 * n * 4, 256);
+  off += column_sums_bytes(T * B, 4 * n);
   l.total = off;
   *out = l;
 }
@@ -2730,7 +2772,7 @@ int rtn_lstm_low_mem_bwd(const void* X, const void* W, const void* b, const void
   unsigned char* ws = (unsigned char*)workspace;
   void* H = ws + L.H;
   void* DI = ws + L.DI;
-  float* partial = (float*)(ws + L.partial);
+  void* partial = ws + L.partial;
   const unsigned char* W_rec = (const unsigned char*)W + (size_t)n_in * 4 * n * es;  // rows n_in.. of W: the recurrent part
   float* DW_rec = DW + (size_t)n_in * 4 * n;
   rocblas_handle blas = nullptr;
@@ -2793,16 +2835,24 @@ int rtn_lstm_low_mem_bwd(const void* X, const void* W, const void* b, const void
     rc = gemm_row_major(blas, true, false, n_in, n4, rows, X, n_in, DI, n4, ty, 0.f, DW, n4, rocblas_datatype_f32_r);
     if (rc != RTN_OK) return rc;
   }
-  {
-    const dim3 block(256), grid1((unsigned)((n4 + 255) / 256), kColumnSumParts), grid2((unsigned)((n4 + 255) / 256));
-    if (dtype == RTN_DTYPE_BF16)
-      hipLaunchKernelGGL(k_column_partial_sums<__bf16>, grid1, block, 0, stream, DI, partial, rows, n4);
-    else
-      hipLaunchKernelGGL(k_column_partial_sums<float>, grid1, block, 0, stream, DI, partial, rows, n4);
-    hipLaunchKernelGGL(k_column_final_sums, grid2, block, 0, stream, partial, Db, kColumnSumParts, n4);
-    RTN_HIP(hipGetLastError());
-  }
-  return RTN_OK;
+  return column_sums(DI, rows, n4, dtype, Db, RTN_DTYPE_F32, partial, stream);
+}
+
+size_t rtn_column_sums_workspace_bytes(int64_t rows, int32_t width) { return rows < 0 || width < 0 ? 0 : column_sums_bytes(rows, width); }
+
+int rtn_column_sums(const void* data, int64_t rows, int32_t width, int32_t dtype, void* out, int32_t out_dtype, void* workspace, size_t workspace_bytes,
+                    void* hip_stream) {
+  g_last_error.clear();
+  if (rows < 0 || width < 0 || width % 4 != 0) return fail(RTN_ERR_SHAPE, "column sums: %lld rows of %d, a multiple of 4 needed", (long long)rows, width);
+  for (int t : {dtype, out_dtype})
+    if (t != RTN_DTYPE_F32 && t != RTN_DTYPE_BF16) return fail(RTN_ERR_ARG, "column sums: unknown dtype %d", t);
+  if (width == 0) return RTN_OK;
+  if ((rows > 0 && !data) || !out) return fail(RTN_ERR_ARG, "column sums: null pointer");
+  if (!aligned16(data)) return fail(RTN_ERR_ARG, "column sums: data must be 16-byte aligned");
+  const size_t need = column_sums_bytes(rows, width);
+  if (need && (!workspace || workspace_bytes < need)) return fail(RTN_ERR_WORKSPACE, "column sums: workspace of %zu bytes needed", need);
+  if (!aligned16(workspace)) return fail(RTN_ERR_ARG, "column sums: workspace must be 16-byte aligned");
+  return column_sums(data, rows, width, dtype, out, out_dtype, workspace, (hipStream_t)hip_stream);
 }
 
 size_t rtn_native_lstm2_bwd_multi_workspace_bytes(int32_t count, int64_t T, int32_t B, int32_t n, int32_t dtype) {

@@ -37,6 +37,8 @@ struct Abi {
   decltype(&rtn_native_lstm2_bwd_multi_workspace_bytes) bwd_multi_workspace_bytes;
   decltype(&rtn_lstm_step) lstm_step;
   decltype(&rtn_sequence_mask) sequence_mask;
+  decltype(&rtn_column_sums) column_sums;
+  decltype(&rtn_column_sums_workspace_bytes) column_sums_workspace_bytes;
 } rtn_abi;
 bool ready = false;
 
@@ -479,6 +481,18 @@ Tensor sequence_mask(const Tensor& lengths, int64_t T) {
   return mask;
 }
 
+// Sums over the rows of a contiguous [rows,width] matrix of one of the op's types, as `type` (one of them, too).  (Not torch's
+// sum: over many rows that records a memset into a captured graph, whose replays then add to values of other replays.)
+Tensor column_sums(const Tensor& m, at::ScalarType type) {
+  const int64_t rows = m.size(0), width = m.size(1);
+  Tensor out = at::empty({width}, m.options().dtype(type));
+  if (m.numel() == 0) return out.zero_();
+  auto code = [](at::ScalarType t) { return t == at::kBFloat16 ? RTN_DTYPE_BF16 : RTN_DTYPE_F32; };
+  const Tensor ws = workspace(rtn_abi.column_sums_workspace_bytes(rows, (int)width), m);
+  check_rc(rtn_abi.column_sums(m.data_ptr(), rows, (int)width, code(m.scalar_type()), out.data_ptr(), code(type), ws.data_ptr(), (size_t)ws.numel(), current_stream(m.device())));
+  return out;
+}
+
 // One direction: (W [n,4n], y0 [B,n], c0 [B,n], step).
 struct Direction {
   Tensor W, y0, c0;
@@ -598,12 +612,15 @@ struct LayerFunction : torch::autograd::Function<LayerFunction> {
     }
     auto res = lstm2_grad_multi(args, true);
     const int64_t rows = source.size(0) * source.size(1);
-    const Tensor DP = as_type(res.second.view({rows, ff.size(1)}), ff.scalar_type());  // (the error of a projection of another type than the op's)
+    const Tensor DPo = res.second.view({rows, ff.size(1)}), DP = as_type(DPo, ff.scalar_type());  // (the error of a projection of another type than the op's)
     variable_list out(11);
     if (ctx->needs_input_grad(0)) out[0] = at::mm(DP, ff.t()).view(source.sizes());
     // (the gradient of ff comes out in the layout of a [4n,in] parameter, whose transposed view ff usually is)
     if (ctx->needs_input_grad(1)) out[1] = at::mm(DP.t(), source.reshape({rows, source.size(2)})).t();
-    if (ctx->saved_data["bias"].toBool() && ctx->needs_input_grad(2)) out[2] = DP.sum(0);
+    if (ctx->saved_data["bias"].toBool() && ctx->needs_input_grad(2)) {
+      c10::DeviceGuard guard(DPo.device());
+      out[2] = as_type(column_sums(DPo, ff.scalar_type() == DPo.scalar_type() ? DPo.scalar_type() : at::kFloat), ff.scalar_type());
+    }
     for (int k = 0; k < count; ++k) {
       const Tensor* s = &saved[4 + 5 * k];
       const Out4& o = res.first[k];
@@ -621,7 +638,6 @@ struct LastOutputFunction : torch::autograd::Function<LastOutputFunction> {
     at::AutoDispatchBelowADInplaceOrView below;
     ctx->save_for_backward({mask});
     ctx->saved_data["step"] = step;
-    ctx->saved_data["shape"] = Y.sizes().vec();
     ctx->saved_data["y0_type"] = (int64_t)y0.scalar_type();
     return last_output(Y, y0, mask, 0, step);
   }
@@ -629,11 +645,14 @@ struct LastOutputFunction : torch::autograd::Function<LastOutputFunction> {
     const Tensor mask = ctx->get_saved_variables()[0], &g = grads[0];
     const int64_t step = ctx->saved_data["step"].toInt();
     if (!g.defined()) return {Tensor(), Tensor(), Tensor(), Tensor()};
-    const Tensor len = mask.sum(0).to(at::kLong), some = (len > 0).unsqueeze(1);
-    const Tensor at_frame = step > 0 ? (len - 1).clamp_min(0) : at::zeros_like(len);
-    const Tensor dY = at::zeros(ctx->saved_data["shape"].toIntVector(), g.options());
-    dY.scatter_(0, at_frame.view({1, -1, 1}).expand({1, dY.size(1), dY.size(2)}), at::where(some, g, at::zeros_like(g)).unsqueeze(0));
-    return {dY, at::where(some, at::zeros_like(g), g).to((at::ScalarType)ctx->saved_data["y0_type"].toInt()), Tensor(), Tensor()};
+    // the frame that g belongs to, per sequence: the last one of the mask, or the first where there is one (no sum over the
+    // frames: see column_sums)
+    const Tensor valid = mask > 0, some = valid.select(0, 0).unsqueeze(1), none = at::zeros_like(valid.narrow(0, 0, 1));
+    const int64_t T = valid.size(0);
+    const Tensor at_frame = step > 0 ? valid.logical_and(at::cat({valid.narrow(0, 1, T - 1), none}).logical_not())
+                                     : at::cat({valid.narrow(0, 0, 1), none.expand({T - 1, valid.size(1)})});
+    const Tensor zero = at::zeros({}, g.options()), dY = at::where(at_frame.unsqueeze(2), g.unsqueeze(0), zero);
+    return {dY, at::where(some, zero, g).to((at::ScalarType)ctx->saved_data["y0_type"].toInt()), Tensor(), Tensor()};
   }
 };
 
@@ -695,6 +714,8 @@ void init(const py::dict& symbols, const py::object& aborted) {
   take(rtn_abi.bwd_multi_workspace_bytes, symbols, "rtn_native_lstm2_bwd_multi_workspace_bytes");
   take(rtn_abi.lstm_step, symbols, "rtn_lstm_step");
   take(rtn_abi.sequence_mask, symbols, "rtn_sequence_mask");
+  take(rtn_abi.column_sums, symbols, "rtn_column_sums");
+  take(rtn_abi.column_sums_workspace_bytes, symbols, "rtn_column_sums_workspace_bytes");
   watch().exception = aborted;
   ready = true;
 }

@@ -441,3 +441,31 @@ def test_autograd_functions_of_two_directions(B, n, dtype, bar):
             if k < 4:
                 assert torch.equal(a, b), (run.__name__, k)
             assert _rel_to_max(a.float().cpu().numpy(), b.float().cpu().numpy()) <= bar, (run.__name__, k)
+
+
+# one part and many, full and partly filled, rows that leave wavefronts without any; widths of one lane, of cut blocks, of pieces
+# of 8 and of 16 bytes
+@pytest.mark.parametrize("rows,width", [(1, 4), (3, 12), (63, 260), (64, 8), (65, 516), (129, 1000), (1000, 4000), (8200, 300), (20000, 2048)])
+@pytest.mark.parametrize("dtype,out_dtype", [("f32", "f32"), ("bf16", "bf16"), ("bf16", "f32"), ("f32", "bf16")])
+def test_column_sums(rows, width, dtype, out_dtype):
+    announce("column sums", rows, width, dtype, out_dtype)
+    get_op()
+    cabi = lib.load()
+    code = {"f32": lib.DTYPE_F32, "bf16": lib.DTYPE_BF16}
+    x = torch.randn((rows, width), generator=torch.Generator().manual_seed(rows + width)).to(torch.bfloat16 if dtype == "bf16" else torch.float32)
+    xd = x.to("cuda:0")
+    out = torch.full((width + 64,), 7.0, dtype=torch.bfloat16 if out_dtype == "bf16" else torch.float32, device="cuda:0")
+    size = int(cabi.rtn_column_sums_workspace_bytes(rows, width))
+    ws = torch.full((size + 256,), 0x5A, dtype=torch.uint8, device="cuda:0")
+    lib.check(cabi.rtn_column_sums(xd.data_ptr(), rows, width, code[dtype], out.data_ptr(), code[out_dtype], ws.data_ptr(), size, torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    assert bool((ws[size:] == 0x5A).all()) and bool((out[width:] == 7.0).all())
+    want = x.double().sum(0)
+    # (at most 128 parts of max(64, rows / 128) rows, rounded up to 16: chains of a sixteenth of either, and 4 more additions in each launch)
+    part = -(-max(64, -(-rows // 128)) // 16) * 16
+    chain = part // 16 + 1 + -(-rows // part) // 16 + 1 + 8
+    bound = chain * 2.0**-24 * x.double().abs().sum(0) + (2.0**-8 * want.abs() if out_dtype == "bf16" else 0)
+    assert bool(((out[:width].double().cpu() - want).abs() <= bound).all())
+    if size:
+        assert cabi.rtn_column_sums(xd.data_ptr(), rows, width, 0, out.data_ptr(), 0, ws.data_ptr(), size - 1, None) == lib.RTN_ERR_WORKSPACE
+    assert cabi.rtn_column_sums(xd.data_ptr(), rows, width + 1, 0, out.data_ptr(), 0, ws.data_ptr(), size, None) == lib.RTN_ERR_SHAPE

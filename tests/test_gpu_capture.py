@@ -133,3 +133,84 @@ def test_training_step_at_benchmark_shape():
     t_replay = _timed(graph.replay, reps=3)
     print("[capture] training step: eager %.3f ms, replay %.3f ms" % (t_eager, t_replay), flush=True)
     assert t_replay <= 1.3 * t_eager, (t_replay, t_eager)
+
+
+@pytest.mark.parametrize("T,B,n_in,n,dtype", [(64, 64, 48, 128, "f32"), (50, 80, 64, 256, "bf16"), (9, 300, 32, 96, "bf16")])
+def test_training_step_of_a_layer_with_many_rows(T, B, n_in, n, dtype):
+    """The bias gradient of thousands of rows is a sum over many workgroups: every replay of a recorded training step, with the
+    program's own work in between, gives the gradients of an eager step on the same inputs."""
+    announce("captured layer with many rows", T, B, n_in, n, dtype)
+    from returnn_amd.lstm import BLSTM
+
+    act = torch.bfloat16 if dtype == "bf16" else torch.float32
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    m = BLSTM(n_in, n, device="cuda", dtype=act)
+    m.reset_parameters(gen)
+    x = torch.randn((T, B, n_in), device="cuda", generator=gen).to(act).requires_grad_()
+    dy = torch.randn((T, B, 2 * n), device="cuda", generator=gen).to(act)
+    lens = torch.randint(1, T + 1, (B,), device="cuda", generator=gen)
+    leaves = [x, *m.parameters()]
+
+    def step():
+        return torch.autograd.grad(m(x, seq_lens=lens, want_states=False)[0], leaves, dy)
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        step()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        recorded = step()
+    bar = 2e-2 if dtype == "bf16" else 2e-5
+    for k in range(5):
+        with torch.no_grad():
+            x.copy_(torch.randn((T, B, n_in), device="cuda", generator=gen))
+            dy.copy_(torch.randn((T, B, 2 * n), device="cuda", generator=gen))
+        graph.replay()
+        torch.cuda.synchronize()
+        for idx, (a, e) in enumerate(zip(recorded, step())):
+            assert float((a.float() - e.float()).abs().max()) <= bar * float(e.float().abs().max()), (k, idx)
+        _ = float((dy.float() ** 2).sum() + x.detach().float().sum())  # eager sums over many workgroups between replays
+
+
+@pytest.mark.parametrize("direction", [1, -1])
+def test_gradient_through_the_final_state_of_long_sequences(direction):
+    """The error of the final output goes to the last frame of the mask (the first one, backwards in time), also in replays with
+    other lengths."""
+    announce("captured final state", direction)
+    from returnn_amd.lstm import LSTM
+
+    T, B, n = 1500, 3, 64
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    m = LSTM(16, n, device="cuda")
+    m.reset_parameters(gen)
+    x = torch.randn((T, B, 16), device="cuda", generator=gen).requires_grad_()
+    dh = torch.randn((B, n), device="cuda", generator=gen)
+    lens = torch.tensor([T, 3, 700], device="cuda")
+    state = m.default_initial_state(batch_dims=(B,))
+
+    def step():
+        return torch.autograd.grad(m(x, state=state, seq_lens=lens, direction=direction)[1].h, [x, *m.parameters()], dh)
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        step()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        recorded = step()
+    for k, other in enumerate(([T, 3, 700], [5, 0, T], [T - 1, T, 1], [2, 1000, 64])):
+        lens.copy_(torch.tensor(other))
+        dh.copy_(torch.randn((B, n), device="cuda", generator=gen))
+        graph.replay()
+        torch.cuda.synchronize()
+        eager = step()
+        # (what autograd makes of indexing the output)
+        y = m(x, state=state, seq_lens=lens, direction=direction)[0]
+        h = y[(lens - 1).clamp(min=0) if direction > 0 else torch.zeros_like(lens), torch.arange(B, device="cuda")]
+        want = torch.autograd.grad(torch.where((lens > 0)[:, None], h, state.h), [x, *m.parameters()], dh)
+        for idx, (a, e, w) in enumerate(zip(recorded, eager, want)):
+            bar = 2e-5 * max(float(w.abs().max()), 1e-30)
+            assert float((a - e).abs().max()) <= bar and float((e - w).abs().max()) <= bar, (k, idx)
