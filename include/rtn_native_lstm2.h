@@ -57,8 +57,10 @@ extern "C" {
  *             in registers and the workgroups hand the hidden state over through a ring
  *             of buffers in the workspace that validates itself (a word that still holds
  *             the "not yet written" pattern is read again): no barrier and no flags.
- *             Wider layers fall back to a kernel that keeps W in LDS and separates
- *             the steps with a flag wait.  Every wait is bounded: when one expires the
+ *             Small layers need no other workgroup: each takes four rows through all steps
+ *             by itself.  Wider layers keep W in the registers and the LDS of the whole device
+ *             (calls with frames enough to pay for loading it) or, where it fits, in LDS alone
+ *             with a flag wait between the steps.  Every wait is bounded: when one expires the
  *             status word of the workspace is set, the kernel still ends, and NaN is
  *             written into d and the last visited frame of Y (Dy0 and Dc0 in the gradient),
  *             so that a caller who never asks for the status sees non-finite results.
@@ -398,7 +400,10 @@ const char* rtn_last_error(void);
 /* The plan the library would use for this problem, as text
  * ("mode=persistent kernel=mfma_regw mt=2 nt=1 groups=2 wgs_per_group=128 wgs=256 rows_per_group=16
  * launches=1 lds=22176 workspace=...": groups, workgroups and rows per group of one persistent launch, and how many
- * launches in turn take the whole batch); for logs and tests.
+ * launches in turn take the whole batch; "interleaved=2": two of these turns share a launch; "row_quads=q": the float32
+ * product goes in q quads of rows; "padded_width=n": of a width that is no multiple of 32); for logs and tests.
+ * kernel: mfma_regw (W in registers), _xcd (every batch group on one XCD), _xcd_half (of at most 8 rows), mfma_regw_solo (small
+ * layers), mfma_regw_wide (W in registers and LDS of the whole device), mfma_lds, generic.
  * Counterpart of the reference's compile log next to the .so (returnn/util/native_code_compiler.py:348-352). */
 const char* rtn_native_lstm2_describe_plan(int64_t T, int32_t B, int32_t n, int32_t dtype, int32_t mode);
 

@@ -37,10 +37,10 @@ __host__ __device__ constexpr DualLds dual_lds(int es, int MT) {
 // step ago), so that what remains exposed are the two groups' own MFMAs, barriers and gates.
 // With two barriers per step one LDS copy of every stream is enough: X and the mask of one group move from registers to LDS
 // in the other group's half, staged outputs leave in the own group's next half.
-// What bounds it now is how fast one wavefront per SIMD issues: of 8000 clocks per step of both groups (bf16 n = 1024, B = 256:
-// 3.3 us, 4.3 in turns) 3600 are the MFMAs (2048 alone) with the loads, stores and LDS traffic between them, 2100 the gates,
-// 700 staging, 1100 looking over h, 400 the barriers.  (The gates of one group woven into the other's MFMAs took 5200 clocks
-// instead of 3600 + 2100, and left the hand-over exposed: 842 us against 690.)
+// What bounds it now is how fast one wavefront per SIMD issues: of 7500 clocks per wavefront and step of both groups (bf16
+// n = 1024, B = 256: 3.3 us, 4.3 in turns) the matrix cores are busy for 2050, vector instructions issue in 2300, 2200 go by with an
+// instruction waiting for its turn and 1600 with none to issue; 23 % of the clocks the LDS is busy are bank conflicts.  (The gates
+// of one group woven into the other's MFMAs left the hand-over exposed: 842 us against 690.)
 // The order of additions is that of k_lstm2_regw: the same bits.
 template <typename AT, int MT, int KS>
 __global__ __launch_bounds__(kWgThreads) void k_lstm2_dual(const Lstm2Multi multi) {

@@ -140,9 +140,11 @@ WideBuild wide_kernel(int dtype, int n, int cus, int rows) {
   }
   return best;
 }
-// float32 up to n = 64, bf16 up to 128.  Measured at T = 500, B = 4 ... 256, us per step, against k_lstm2_regw: float32 n = 32 / 64
-// 0.63 / 0.73 against 1.03; n = 96 / 128 (8 wavefronts' MFMAs on one CU) would take 1.36 / 1.64 against 1.03; bf16 n = 32 / 64 / 96
-// / 128 0.41 / 0.55 / 0.71 / 0.87 against 0.83 (and 5 us less for not packing W); n = 160 would take 1.7 against 0.85.
+// float32 up to n = 64, bf16 up to 128.  Measured at T = 4, 32 and 300 with B = 4 ... 1024, us per call, against k_lstm2_regw: T = 300, B = 4 /
+// 1024: float32 n = 32 184 / 204 against 312 / 396, n = 64 211 / 250 against 310 / 473; bf16 n = 32 121 / 143 against 249 / 296, n = 64 186 / 209
+// against 248 / 349, n = 96 213 / 281 against 253 / 505, n = 128 263 / 338 against 255 / 547 (the one case behind, by 3 %:
+// 4 rows of 300 frames; 64 rows 264 against 266, T = 32 37 / 41 against 39 / 66, since no W is packed).  Beyond, 8 wavefronts' MFMAs on one CU take longer than a
+// hand-over: float32 n = 96 / 128 1.36 / 1.64 us per step against 1.03, bf16 n = 160 1.7 against 0.85.
 SoloBuild solo_kernel(int dtype, int n) {
 #define RTN_SOLO(at, s) if (n <= s * Elem<at>::KM) return {&k_lstm2_solo<at, s>, 64 * solo_waves<at>(s)};
   if (dtype == 1) {

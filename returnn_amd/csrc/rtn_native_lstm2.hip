@@ -258,8 +258,9 @@ bool make_plan_uncached(int64_t T, int B, int n, int dtype, int want_mode, bool 
   const bool mfma_shape = (n % 32) == 0;
   const long force_generic = env_long("RTN_LSTM2_FORCE_GENERIC", 0);
   bool persistent_ok = false;
-  // A small layer whose rows find a CU per four: no workgroup needs another one.  (A batch beyond that keeps several rows per
-  // tile busy on the kernels below; a decomposition or kernel asked for by the environment is one of theirs.)
+  // A small layer whose rows find a CU per four: no workgroup needs another one.  (Ahead up to that many rows at every width it
+  // takes, see solo_kernel; a batch beyond keeps several rows per tile busy on the kernels below.  A decomposition or kernel
+  // asked for by the environment is one of theirs.)
   if (want_mode == RTN_MODE_AUTO && di.valid && !force_generic && B <= kSoloRows * di.cus / std::max(1, std::min(count, kMaxMulti)) && !env_long("RTN_LSTM2_NO_PAD", 0) &&
       !env_long("RTN_LSTM2_MT", 0) && !env_long("RTN_LSTM2_GROUPS", 0) && !env_long("RTN_LSTM2_KERNEL", 0) && env_long("RTN_LSTM2_LOCAL", -1) < 0 && !env_long("RTN_LSTM2_NO_SOLO", 0))
     pl.solo_build = solo_kernel(dtype, n);
@@ -1055,9 +1056,6 @@ int check_dims(int64_t T, int32_t B, int32_t n, int32_t dtype) {
   return RTN_OK;
 }
 
-
-// Workspace of one problem of an entry with `count` problems: the largest layout any resolution of `mode`
-// can need (AUTO may fall back to per-step launches, and the plan depends on how many problems share a launch).
 // ---- widths the matrix-core kernels do not take ------------------------------------------------------------------
 // n that is not a multiple of 32 runs zero-padded to the next multiple: a padded cell has zero inputs, zero weights (rows
 // and columns) and a zero initial state, so its cell state and output are exactly 0 in every frame, it adds nothing to
@@ -1143,7 +1141,7 @@ int resolve_pitch(const char* name, long long given, long long contiguous, int B
   const long long ld = given ? given : contiguous;
   if (ld < contiguous) return fail(RTN_ERR_ARG, "NativeLstm2: row pitch %s=%lld is below the row length %lld", name, ld, contiguous);
   if (ld != contiguous && ((size_t)ld * es) % 4 != 0) return fail(RTN_ERR_ARG, "NativeLstm2: row pitch %s=%lld must keep rows 4-byte aligned", name, ld);
-  // (widths whose contiguous rows are not 16-byte aligned run on element-wise kernels or on padded copies)
+  // (widths whose contiguous rows are not 16-byte aligned run on kernels that move smaller pieces)
   if (((size_t)contiguous * es) % 16 == 0 && ((size_t)ld * es) % 16 != 0)
     return fail(RTN_ERR_ARG, "NativeLstm2: row pitch %s=%lld must keep rows 16-byte aligned", name, ld);
   if ((unsigned long long)B * (unsigned long long)ld * es >= 0xFFFFFF00ull)
@@ -1152,7 +1150,9 @@ int resolve_pitch(const char* name, long long given, long long contiguous, int B
   return RTN_OK;
 }
 
-// Workspace of one of `count` forward calls (call k's slice starts at k times this, with its status block first).
+// Workspace of one of `count` forward calls (call k's slice starts at k times this, with its status block first): the largest
+// layout any resolution of `mode` can need (AUTO may fall back to per-step launches, and the plan depends on how many
+// problems share a launch).
 size_t workspace_each(int count, int64_t T, int32_t B, int32_t n, int32_t dtype, int32_t mode) {
   n = padded_width(n);  // (the kernels pad on the fly: the layout is that of the padded width)
   size_t need = 0;

@@ -16,8 +16,9 @@ then one ``NativeLstm2`` call with the right-padded 0/1 mask; output frames beyo
 ``direction=-1`` runs the recurrence from each sequence's last frame to its first without reversing anything
 in memory (the caller protocol of returnn/tf/layers/rec.py:1229-1270).
 
-With gradients enabled and an input that requires them, the same functions go through
-``NativeLstm2Function`` (the op with its gradient op) and torch's autograd, so the layer trains like ``rf.LSTM``.
+With gradients enabled and an input that requires them, the same functions go through one autograd node in native code
+(projection and op; its gradient: the gradient op, the projection's products, the bias gradient), so the layer trains
+like ``rf.LSTM``.  One step ``[B,in]`` without gradients is a kernel of its own.
 
 :class:`LSTM` and :class:`LstmState` mirror the module and its state (parameters in the frontend's names and layout).
 :class:`BLSTM` is one bidirectional layer (:func:`blstm`: ONE projection for both directions, which then go through the

@@ -134,7 +134,8 @@ def test_plan_of_large_batches_padded_widths_and_wide_layers(cabi):
     assert "workspace=%i " % padded in lib.describe_plan(100, 32, 1000, lib.DTYPE_BF16, lib.MODE_AUTO)
     assert cabi.rtn_native_lstm2_bwd_workspace_bytes(100, 32, 1000, lib.DTYPE_BF16) > cabi.rtn_native_lstm2_bwd_workspace_bytes(100, 32, 1024, lib.DTYPE_BF16)
     assert "padded_width" not in lib.describe_plan(100, 32, 20, lib.DTYPE_F32, lib.MODE_AUTO)  # tiny layers stay as they are
-    # W does not fit on chip: one launch per step, a few KB of LDS (W goes from memory straight to the matrix cores)
+    # W does not fit the registers of the device: one launch per step, a few KB of LDS (W goes from memory straight to the matrix
+    # cores).  (The kernel that takes registers and LDS of the whole device is only planned for a device that is there.)
     text = lib.describe_plan(100, 16, 4096, lib.DTYPE_BF16, lib.MODE_AUTO)
     assert "mode=graph" in text and "kernel=mfma_lds" in text and "lds=4096 " in text, text
 
@@ -148,7 +149,8 @@ def test_xcd_local_plans(cabi):
     # a single bf16 sequence goes to one XCD too (its hidden state then never leaves that XCD's L2)
     single = lib.describe_plan(4000, 1, 1024, lib.DTYPE_BF16, lib.MODE_AUTO)
     assert "kernel=mfma_regw_xcd_half mt=8 nt=1 groups=1 wgs_per_group=32 " in single, single
-    # float32 at n = 512 keeps W spread over more CUs (fewer MFMAs per wavefront and step)
+    # float32 at n = 512 keeps W spread over more CUs (fewer MFMAs per wavefront and step) where the product goes in tiles of 16
+    # rows, as it is planned without a device; with one it goes in quads of rows, on one XCD per group
     assert "kernel=mfma_regw " in lib.describe_plan(500, 64, 512, lib.DTYPE_F32, lib.MODE_AUTO)
     # the environment switch: read once, and again when the library is told to
     os.environ["RTN_LSTM2_LOCAL"] = "0"

@@ -592,8 +592,8 @@ def test_expired_wait_reaches_the_torch_caller():
     [(12, 8, 2048, "bf16"), (8, 300, 256, "bf16"), (6, 256, 1024, "bf16"), (5, 300, 512, "f32"), (4, 70, 1536, "bf16"), (8, 513, 128, "f32"), (6, 130, 1024, "bf16"), (5, 4, 3072, "bf16"), (7, 9, 736, "f32"), (9, 1, 4096, "bf16")],
 )
 def test_wide_and_large_shapes(T, B, n, dtype):
-    """Shapes beyond the benchmark configurations cfg1-cfg5: very wide layers (W no longer fits the registers of the device: the plan
-    falls back to the LDS kernel per step), many sequences (several batch groups, partly filled last group), a width that
+    """Shapes beyond the benchmark configurations cfg1-cfg5: very wide layers (W no longer fits the registers of the device: the wide
+    kernel, which takes its LDS as well), many sequences (several batch groups, partly filled last group), a width that
     is a multiple of 32 but not of 64.  Forward against the oracle, then the gradient op on the GPU's own results."""
     announce("wide_and_large", T, B, n, dtype)
     p = random_problem(900 + T + B + n, T, B, n)
