@@ -5,10 +5,11 @@ from __future__ import annotations
 
 import numpy
 import pytest
+import torch
 
 from returnn_amd import lib
 
-from _gpu_util import announce, env, random_problem, run_raw
+from _gpu_util import announce, env, get_op, random_problem, run_raw, to_dev
 
 pytestmark = pytest.mark.gpu
 
@@ -82,3 +83,17 @@ def test_few_frames_of_many_rows_run_as_one_launch_per_step(T, B, n, dtype):
     assert "kernel=mfma_regw_wide" in plan and rc == 0 and status == 0
     for name, a, b in zip("YCHd", got, want):
         assert numpy.array_equal(a, b), name
+    # ... and recorded into a graph, as launches per step
+    op = get_op()
+    args = [to_dev(a, dtype) for a in p[:3]] + [to_dev(a, "f32") for a in p[3:]]
+    before = lib.capture_report()
+    graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.graph(graph, stream=side):
+        recorded = op(*args, 0, 1)
+    assert lib.capture_report() == before
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        for name, a, b in zip("YCHd", recorded, want):
+            assert numpy.array_equal(a.float().cpu().numpy(), b), name
