@@ -2,7 +2,7 @@
 GPU parity of the NativeLstm2 gradient op (C ABI ``rtn_native_lstm2_bwd``) against the CPU oracle of the reference's
 gradient code, on the forward results of the HIP path itself.
 
-Tolerances.  The north star fixes tolerances for the forward outputs only; gradients are sums over up to T*B terms
+Tolerances.  The tolerances asked of the op are those of the forward outputs only; gradients are sums over up to T*B terms
 whose summation order differs between MFMA tiles and a sequential loop, so they are judged relative to the largest
 magnitude of each array: float32 within 2e-5 of it (the float32 oracle itself is that far from the float64 oracle),
 bfloat16 (bf16 activations, gates and DX; float32 accumulation) within 2e-2 of it.
