@@ -52,24 +52,44 @@ __global__ void k_bwd_pack_w(const void* __restrict__ W, void* __restrict__ Wpk,
 //   h0: first block of H -- tanh(cell-in), or with kOpH0IsCell the cell state, from which tanh(cell-in) is recovered as
 //   the reference's gradient kernel does: (state - forget * old_state) / max(input, 1e-16)  (:462-463)
 //   err_y, err_c: error of the output and of the cell state, already multiplied by the mask
+// In two parts: what the errors do not enter (BwdCell::of, which the persistent kernel works out ahead of them), and the rest.
+template <typename AT>
+struct BwdCell {
+  float p[4], dtanh, a_out, a_fg;  // derivative factors of the gates, 1 - tanh(c)^2, two of the gates
+
+  static __device__ __forceinline__ BwdCell of(int op_flags, float h0, float a_in, float a_fg, float a_out, float c_before) {
+    float a_cell, tanh_c;  // tanh(cell-in) and tanh of the frame's cell state
+    if (op_flags & kOpH0IsCell) {
+      tanh_c = Act<AT>::tanh(h0);
+      a_cell = (h0 - a_fg * c_before) / fmaxf(a_in, 1e-16f);
+    } else {
+      a_cell = h0;
+      tanh_c = Act<AT>::tanh(c_before * a_fg + a_cell * a_in);
+    }
+    BwdCell r;
+    r.p[0] = (1.f - a_cell * a_cell) * a_in;
+    r.p[1] = (1.f - a_in) * a_in * a_cell;
+    r.p[2] = (1.f - a_fg) * a_fg * c_before;
+    r.p[3] = (1.f - a_out) * a_out * tanh_c;
+    r.dtanh = 1.f - tanh_c * tanh_c;
+    r.a_out = a_out;
+    r.a_fg = a_fg;
+    return r;
+  }
+  // dx: the gates' derivatives; returns the total error on the frame's cell state
+  __device__ __forceinline__ float apply(float err_y, float err_c, float (&dx)[4]) const {
+    using E = Elem<AT>;
+    const float err_cell = err_c + a_out * err_y * dtanh;
+#pragma unroll
+    for (int g = 0; g < 3; ++g) dx[g] = E::round(p[g] * err_cell);
+    dx[3] = E::round(p[3] * err_y);
+    return err_cell;
+  }
+};
 template <typename AT>
 __device__ __forceinline__ float bwd_cell(int op_flags, float h0, float a_in, float a_fg, float a_out, float c_before, float err_y,
                                           float err_c, float (&dx)[4]) {
-  using E = Elem<AT>;
-  float a_cell, tanh_c;  // tanh(cell-in) and tanh of the frame's cell state
-  if (op_flags & kOpH0IsCell) {
-    tanh_c = Act<AT>::tanh(h0);
-    a_cell = (h0 - a_fg * c_before) / fmaxf(a_in, 1e-16f);
-  } else {
-    a_cell = h0;
-    tanh_c = Act<AT>::tanh(c_before * a_fg + a_cell * a_in);
-  }
-  const float err_cell = err_c + a_out * err_y * (1.f - tanh_c * tanh_c);  // total error on the frame's cell state
-  dx[0] = E::round((1.f - a_cell * a_cell) * a_in * err_cell);
-  dx[1] = E::round((1.f - a_in) * a_in * a_cell * err_cell);
-  dx[2] = E::round((1.f - a_fg) * a_fg * c_before * err_cell);
-  dx[3] = E::round((1.f - a_out) * a_out * tanh_c * err_y);
-  return err_cell;
+  return BwdCell<AT>::of(op_flags, h0, a_in, a_fg, a_out, c_before).apply(err_y, err_c, dx);
 }
 
 // Cell state of the frame before: the forward pass's C, or with kOpH0IsCell the first block of H of that frame.
@@ -344,49 +364,9 @@ struct Lstm2BwdMulti {
 // accumulators, the first valid in columns 0-7, the second in columns 8-15, which are added when the partial tiles of
 // the wavefronts are.  Same number of MFMAs, half the load instructions, no data movement.
 //
-// RQ > 0 (float32, HALF, at most 4 RQ rows): the product in v_mfma_f32_4x4x1, whose 16 blocks of 4 rows x 4 values of k are
-// 4 rows x 64 products in 8 clocks, the rate of the 16x16x4 without its padding of 8 rows to 16.  With MT tiles of 16 values
-// of k, 4 MT blocks take one element of the contraction range and 4 / MT of them go at once: lane group kg of a fragment
-// holds elements 4 kg ... 4 kg + 3, and of every 4 MT blocks the one that holds the wanted rows of register i's element is
-// broadcast to the others.  The 4 / MT partial sums are added across the lanes before they go through LDS.
-template <int MT, int ABID>
-__device__ __forceinline__ f32x4 bwd_quad_mma(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, c, MT == 4 ? 4 : MT == 2 ? 3 : 2, ABID, 0); }
-// Two macro steps whose fragments share a register (rows 0-7 and 8-15 of every lane group); I counts (e, i, macro step, quad).
-template <int MT, int RQ, int... I>
-__device__ __forceinline__ void bwd_quad_steps(const i32x4 (&w0)[MT], const i32x4 (&w1)[MT], const i32x4& xbits, f32x4 (&acc)[RQ][2], std::integer_sequence<int, I...>) {
-  const f32x4 x = __builtin_bit_cast(f32x4, xbits);
-  f32x4 w[2][MT];
-#pragma unroll
-  for (int i = 0; i < MT; ++i) {
-    w[0][i] = __builtin_bit_cast(f32x4, w0[i]);
-    w[1][i] = __builtin_bit_cast(f32x4, w1[i]);
-  }
-  (([&] {
-     constexpr int rq = I % RQ, up = I / RQ % 2, i = I / (2 * RQ) % MT, e = I / (2 * RQ * MT);
-     acc[rq][up] = bwd_quad_mma<MT, 4 * i + rq + 2 * up>(x[e], w[up][i][e], acc[rq][up]);
-   }()),
-   ...);
-}
-// a + b of the lanes 32 (SHIFT = 32) or 16 apart: lanes without the bit get a's sum, lanes with it b's.
-template <int SHIFT>
-__device__ __forceinline__ f32x4 lane_pair_sum(f32x4 a, f32x4 b) {
-  f32x4 r;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const unsigned x = __builtin_bit_cast(unsigned, (float)a[j]), y = __builtin_bit_cast(unsigned, (float)b[j]);
-    const u32x2 t = SHIFT == 32 ? __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(x, y, false, false))
-                                : __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(x, y, false, false));
-    const unsigned lo = t[0], hi = t[1];
-    r[j] = __builtin_bit_cast(float, lo) + __builtin_bit_cast(float, hi);
-  }
-  return r;
-}
-
-template <typename AT, int KSB, int MT, int WV, int KSL = 0, bool HALF = false, int RQ = 0>
+template <typename AT, int KSB, int MT, int WV, int KSL = 0, bool HALF = false>
 __global__ __launch_bounds__(64 * WV) void k_lstm2_bwd_regw(const Lstm2BwdMulti multi) {
   static_assert(!HALF || KSL == 0, "the paired loads are not written for the chunked variants");
-  constexpr bool QUAD = RQ > 0;
-  static_assert(!QUAD || (sizeof(AT) == 4 && HALF && RQ <= 2 && KSB % 2 == 0), "quads of rows: float32, paired loads");
   constexpr int KST = KSB + KSL;           // fragment slots of a wavefront
   constexpr int TS = WV / 4;               // thread sets of 256
   // tiles whose pairs a thread keeps.  A set of 256 threads covers 16 rows x 16 values of k; with at most 8 rows the
@@ -417,10 +397,8 @@ __global__ __launch_bounds__(64 * WV) void k_lstm2_bwd_regw(const Lstm2BwdMulti 
   constexpr int kRedGroup = 20;
   // (two copies where they are small, frames alternate: no barrier then between the sums of one frame and the partial
   // tiles of the next)
-  // (QUAD: [quad][k] of 4 rows each, two quads of up to 32 values of k in one 64 lanes wide slot)
-  constexpr int kRedSlots = QUAD ? (MT == 4 ? RQ : 1) : MT, kRedLanes = QUAD ? 64 : 4 * kRedGroup;
-  constexpr int kRedCopies = (WV * kRedSlots * kRedLanes * 16 <= 24 * 1024) ? 2 : 1;
-  __shared__ f32x4 red2[kRedCopies][WV][kRedSlots][kRedLanes];
+  constexpr int kRedCopies = (WV * MT * 4 * kRedGroup * 16 <= 24 * 1024) ? 2 : 1;
+  __shared__ f32x4 red2[kRedCopies][WV][MT][4 * kRedGroup];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // 0..WV-1
   const int n = p.n, n4 = 4 * n;
@@ -457,9 +435,7 @@ __global__ __launch_bounds__(64 * WV) void k_lstm2_bwd_regw(const Lstm2BwdMulti 
   i32x4* wl = (i32x4*)bwd_smem + (size_t)wave * (KSL > 0 ? KSL : 1) * 64 + lane;  // [WV][KSL][64]: slot s of this lane at wl[s * 64]
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
-    // (QUAD: register i of a lane is k = lane % (16 MT), elements 4 (i + MT * (lane / (16 MT))) ... + 3 of the macro step)
-    const AT* Wr = (const AT*)p.W + (size_t)(k0 + (QUAD ? lane & (16 * MT - 1) : 16 * mt + (lane & 15))) * n4 + (size_t)KM * ksb * wave +
-                   KE * (QUAD ? mt + MT * (lane / (16 * MT)) : lane >> 4);
+    const AT* Wr = (const AT*)p.W + (size_t)(k0 + 16 * mt + (lane & 15)) * n4 + (size_t)KM * ksb * wave + KE * (lane >> 4);
 #pragma unroll
     for (int ks = 0; ks < KSB; ++ks) wreg[mt][ks] = (ks < ks_here) ? *(const i32x4*)(Wr + (size_t)KM * ks) : i32x4{0, 0, 0, 0};
     if constexpr (KSL > 0) {
@@ -500,8 +476,8 @@ __global__ __launch_bounds__(64 * WV) void k_lstm2_bwd_regw(const Lstm2BwdMulti 
     for (int gq = 0; gq < 4; ++gq) dx0[j][gq] = 0.f;
   }
   // where a pair's element of the summed tile is: tile element D[kl][bl] sits in lane (kl/4)*16 + bl, component kl%4
-  const int red_lane = QUAD ? (RQ == 2 ? (bl >> 2) & 1 : 0) * (MT == 4 ? 64 : 32) + kl : (kl >> 2) * kRedGroup + (HALF ? (bl & 7) : bl);
-  const int red_comp = QUAD ? bl & 3 : kl & 3;
+  const int red_lane = (kl >> 2) * kRedGroup + (HALF ? (bl & 7) : bl);
+  const int red_comp = kl & 3;
 
   // Inputs of a frame, fetched one frame ahead.  No branches around the loads and no arithmetic on what they bring: a
   // register that receives its value on two paths, or feeds an instruction, makes the compiler wait for every load in
@@ -565,8 +541,7 @@ __global__ __launch_bounds__(64 * WV) void k_lstm2_bwd_regw(const Lstm2BwdMulti 
   };
   const int F = q.nframes;
   // EARLY: a frame's inputs are asked for two frames ahead, in front of the MFMAs (see gemm); otherwise one frame ahead,
-  // at the end of a frame.  (Measured: the kernels that keep one pair per thread gain 4 % from EARLY, the others lose;
-  // so do quads of rows with one tile, by 11 %.)
+  // at the end of a frame.  (Measured: the kernels that keep one pair per thread gain 4 % from EARLY, the others lose.)
   constexpr bool EARLY = SPLIT;
   auto frame = [&](int f) { return q.t_end - (long long)f * q.step; };
 
@@ -619,7 +594,6 @@ __global__ __launch_bounds__(64 * WV) void k_lstm2_bwd_regw(const Lstm2BwdMulti 
     // independent partial sums keep the MFMA pipeline full (one chain would wait for every result)
     constexpr int NACC = HALF ? 2 : ((MT >= 4 || KSB < 2) ? 1 : (MT == 2 || KSB < 4 ? 2 : 4));
     f32x4 part[MT][NACC];
-    f32x4 quad[QUAD ? RQ : 1][2];
 #pragma unroll
     for (int c = 0; c < NCH; ++c) {
       const int slot = c & 1;
@@ -680,21 +654,8 @@ __global__ __launch_bounds__(64 * WV) void k_lstm2_bwd_regw(const Lstm2BwdMulti 
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
           for (int a = 0; a < NACC; ++a) part[mt][a] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int q = 0; q < (QUAD ? RQ : 1); ++q) quad[q][0] = quad[q][1] = f32x4{0.f, 0.f, 0.f, 0.f};
       }
-      if constexpr (QUAD) {
-#pragma unroll
-        for (int a = 0; a < NB; ++a) {
-          i32x4 w0[MT], w1[MT];
-#pragma unroll
-          for (int mt = 0; mt < MT; ++mt) {
-            w0[mt] = wreg[mt][2 * a];
-            w1[mt] = wreg[mt][2 * a + 1];
-          }
-          bwd_quad_steps<MT, RQ>(w0, w1, bf[slot][a], quad, std::make_integer_sequence<int, 8 * MT * RQ>());
-        }
-      } else if constexpr (HALF) {
+      if constexpr (HALF) {
 #pragma unroll
         for (int a = 0; a < NB; ++a)
 #pragma unroll
@@ -713,19 +674,6 @@ __global__ __launch_bounds__(64 * WV) void k_lstm2_bwd_regw(const Lstm2BwdMulti 
           }
       }
     }
-    if constexpr (QUAD) {
-      f32x4 sum[RQ];
-#pragma unroll
-      for (int q = 0; q < RQ; ++q) sum[q] = quad[q][0] + quad[q][1];
-      if constexpr (MT == 4) {
-#pragma unroll
-        for (int q = 0; q < RQ; ++q) red[wave][q][lane] = sum[q];
-      } else {
-        f32x4 acc = lane_pair_sum<32>(sum[0], sum[RQ - 1]);
-        if constexpr (MT == 1) acc = lane_pair_sum<16>(acc, acc);
-        red[wave][0][lane] = acc;
-      }
-    } else
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
       f32x4 acc = part[mt][0];
@@ -750,10 +698,6 @@ __global__ __launch_bounds__(64 * WV) void k_lstm2_bwd_regw(const Lstm2BwdMulti 
       float sum = 0.f;
 #pragma unroll
       for (int w = 0; w < WV; ++w) {
-        if constexpr (QUAD) {
-          sum += ((const float*)(&red[w][0][0] + red_lane + 16 * mt))[red_comp];
-          continue;
-        }
         sum += ((const float*)&red[w][mt][red_lane])[red_comp];
         if constexpr (HALF) sum += ((const float*)&red[w][mt][red_lane + 8])[red_comp];
       }

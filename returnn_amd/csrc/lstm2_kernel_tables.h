@@ -5,6 +5,7 @@
 #pragma once
 
 #include "lstm2_bwd_kernels.h"
+#include "lstm2_bwd_local_kernel.h"
 #include "lstm2_kernels.h"
 #include "lstm2_dual_kernel.h"
 #include "lstm2_solo_kernel.h"
@@ -48,8 +49,9 @@ BwdRegwKernel bwd_regw_table_bf16_half(int KSB, int MT, int WV);
 BwdRegwKernel bwd_regw_table_bf16_full(int KSB, int MT, int WV);
 BwdRegwKernel bwd_regw_table_f32_half(int KSB, int MT, int WV);
 BwdRegwKernel bwd_regw_table_f32_full(int KSB, int MT, int WV);
-// k_lstm2_bwd_regw<float, KSB, MT, WV, 0, true, RQ>: groups of at most 4 RQ rows, the product in quads of rows.
-BwdRegwKernel bwd_regw_table_f32_quads(int KSB, int MT, int WV, int RQ);
+// k_lstm2_bwd_local<AT, KSB, MT, RQ>: groups of at most 8 rows on one XCD each; float32: of at most 4 RQ rows, the product in quads.
+BwdRegwKernel bwd_local_table_bf16(int KSB, int MT);
+BwdRegwKernel bwd_local_table_f32(int KSB, int MT, int RQ);
 // The variants with half of a wavefront's share of W in registers and half in LDS (one tile per workgroup).
 BwdRegwKernel bwd_regw_lds_table_bf16(int WV);
 BwdRegwKernel bwd_regw_lds_table_f32(int WV);

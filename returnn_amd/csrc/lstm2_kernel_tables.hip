@@ -5,7 +5,7 @@
 #include "lstm2_kernel_tables.h"
 
 #ifndef RTN_TABLE_PART
-#error "compile with -DRTN_TABLE_PART=<1..14>"
+#error "compile with -DRTN_TABLE_PART=<1..15>"
 #endif
 
 namespace rtn {
@@ -81,14 +81,14 @@ BwdRegwKernel bwd_regw_table(int KSB, int MT, int WV) {
   return nullptr;
 }
 
-// (float32 in quads of rows)
-template <int RQ>
-BwdRegwKernel bwd_regw_table_quad(int KSB, int MT, int WV) {
-#define RTN_CASE(ks, mt, wv) \
-  if (KSB == ks && MT == mt && WV == wv) return &k_lstm2_bwd_regw<float, ks, mt, wv, 0, true, RQ>;
-  RTN_CASE(2, 1, 4) RTN_CASE(4, 1, 4) RTN_CASE(8, 1, 4) RTN_CASE(16, 1, 4) RTN_CASE(32, 1, 4)
-  RTN_CASE(2, 2, 4) RTN_CASE(4, 2, 4) RTN_CASE(8, 2, 4) RTN_CASE(16, 2, 4) RTN_CASE(32, 2, 4)
-  RTN_CASE(2, 4, 4) RTN_CASE(4, 4, 4) RTN_CASE(8, 4, 4) RTN_CASE(16, 4, 4)
+// (groups of up to 8 rows on one XCD each; RQ: float32 in quads of rows)
+template <typename AT, int RQ>
+BwdRegwKernel bwd_local_table(int KSB, int MT) {
+#define RTN_CASE(ks, mt) \
+  if (KSB == ks && MT == mt) return &k_lstm2_bwd_local<AT, ks, mt, RQ>;
+  RTN_CASE(2, 1) RTN_CASE(4, 1) RTN_CASE(8, 1) RTN_CASE(16, 1) RTN_CASE(32, 1)
+  RTN_CASE(2, 2) RTN_CASE(4, 2) RTN_CASE(8, 2) RTN_CASE(16, 2) RTN_CASE(32, 2)
+  RTN_CASE(2, 4) RTN_CASE(4, 4) RTN_CASE(8, 4) RTN_CASE(16, 4)
 #undef RTN_CASE
   return nullptr;
 }
@@ -161,14 +161,16 @@ RegwKernel regw_table_f32_quad_tail(int MT, int KSMAX, int RQ) { return regw_tab
 RegwKernel regw_table_f32_quad_tail(int MT, int KSMAX, int RQ);
 RegwKernel regw_table_f32_quad(int MT, int KSMAX, bool tail, int RQ) { return tail ? regw_table_f32_quad_tail(MT, KSMAX, RQ) : regw_table_quad<false>(MT, KSMAX, RQ); }
 #elif RTN_TABLE_PART == 12
-BwdRegwKernel bwd_regw_table_f32_quads2(int KSB, int MT, int WV);
-BwdRegwKernel bwd_regw_table_f32_quads(int KSB, int MT, int WV, int RQ) { return RQ == 1 ? bwd_regw_table_quad<1>(KSB, MT, WV) : RQ == 2 ? bwd_regw_table_f32_quads2(KSB, MT, WV) : nullptr; }
+BwdRegwKernel bwd_local_table_f32_two(int KSB, int MT);
+BwdRegwKernel bwd_local_table_f32(int KSB, int MT, int RQ) { return RQ == 1 ? bwd_local_table<float, 1>(KSB, MT) : RQ == 2 ? bwd_local_table_f32_two(KSB, MT) : nullptr; }
 #elif RTN_TABLE_PART == 13
-BwdRegwKernel bwd_regw_table_f32_quads2(int KSB, int MT, int WV) { return bwd_regw_table_quad<2>(KSB, MT, WV); }
+BwdRegwKernel bwd_local_table_f32_two(int KSB, int MT) { return bwd_local_table<float, 2>(KSB, MT); }
 #elif RTN_TABLE_PART == 14
 RegwKernel dual_kernel() { return &k_lstm2_dual<__bf16, 8, 8>; }
+#elif RTN_TABLE_PART == 15
+BwdRegwKernel bwd_local_table_bf16(int KSB, int MT) { return bwd_local_table<__bf16, 0>(KSB, MT); }
 #else
-#error "RTN_TABLE_PART must be 1..14"
+#error "RTN_TABLE_PART must be 1..15"
 #endif
 
 }  // namespace rtn

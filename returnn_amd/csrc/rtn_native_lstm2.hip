@@ -2083,6 +2083,7 @@ struct BwdChoice {
   int groups_per_launch = 0;   // batch groups of every problem that one launch takes
   bool local = false;          // every group on one XCD
   size_t lds = 0;              // dynamic shared memory of the kernel
+  bool one_xcd_kernel = false; // k_lstm2_bwd_local: local, rows_per_group <= 8
   int rq = 0;                  // float32: quads of rows per group where the product goes in them, else 0
 };
 
@@ -2231,9 +2232,9 @@ int choose_bwd_kernel(const BwdCtx& x, BwdChoice* out) {
       const bool fewer_bytes = best.kernel && (best.rows_per_group - rows) * 16LL * n >= 32 * 1024;
       if (best.kernel && (mt * rq > best.tiles * best.rq || (mt * rq == best.tiles * best.rq && !fewer_bytes))) continue;
       BwdChoice c;
-      c.kernel = (const void*)bwd_regw_table_f32_quads(room, mt, kWaves, rq);
+      c.kernel = (const void*)bwd_local_table_f32(room, mt, rq);
       if (!c.kernel) continue;
-      c.ksb = ksb; c.tiles = mt; c.rows_per_group = rows; c.rq = rq; c.local = true;
+      c.ksb = ksb; c.tiles = mt; c.rows_per_group = rows; c.rq = rq; c.local = c.one_xcd_kernel = true;
       c.groups_per_launch = (B + rows - 1) / rows;
       best = c;
     }
@@ -2261,11 +2262,7 @@ int choose_bwd_kernel(const BwdCtx& x, BwdChoice* out) {
     const bool lds_share = ksb_room * wv == 256;
     if (lds_share && (mt != 1 || (wv != 4 && wv != 8))) continue;
     BwdRegwKernel kfn = nullptr;
-    int rq = 0;
-    if (!lds_share && use_rows <= 8 && (rq = quads(use_rows)) && !(kfn = bwd_regw_table_f32_quads(ksb_room, mt, wv, rq))) rq = 0;
-    if (kfn)
-      ;
-    else if (lds_share)
+    if (lds_share)
       kfn = dtype == RTN_DTYPE_BF16 ? bwd_regw_lds_table_bf16(wv) : bwd_regw_lds_table_f32(wv);
     else
       // ring frames of 8 rows: the variant whose loads take two macro steps at once
@@ -2278,7 +2275,6 @@ int choose_bwd_kernel(const BwdCtx& x, BwdChoice* out) {
     c.tiles = mt;
     c.waves = wv;
     c.rows_per_group = use_rows;
-    c.rq = rq;
     c.lds = lds_share ? kBwdLdsShareBytes : 0;
     if (c.lds && (rc = ensure_lds_limit(c.kernel, c.lds)) != RTN_OK) return rc;
     int per_cu = 0;
@@ -2287,10 +2283,28 @@ int choose_bwd_kernel(const BwdCtx& x, BwdChoice* out) {
     const long long G_wgs = n / (16 * mt), cu_x = di.xcds > 0 ? di.cus / di.xcds : 0;
     if (local_only && n / 16 <= cu_x * per_cu) continue;  // (groups of one tile per workgroup fit an XCD themselves)
     if (local_only && 2 * (long long)count * groups_needed * G_wgs < di.cus) continue;  // (few rows: the wider spread wins, cfg5 7.98 against 8.41 ms)
-    const bool fits_xcd = want_local && di.xcds > 1 && per_cu >= 1 && G_wgs <= cu_x * per_cu;
-    if (fits_xcd && (long long)di.xcds * ((cu_x * per_cu) / G_wgs) >= (long long)count * groups_needed) {
+    // Groups on one XCD each: how many a launch holds with `fit` workgroups to a CU.
+    auto on_xcds = [&](int fit) { return want_local && di.xcds > 1 && fit >= 1 && G_wgs <= cu_x * fit ? (long long)di.xcds * ((cu_x * fit) / G_wgs) : 0LL; };
+    // Groups of up to 8 rows have a kernel of their own there (float32: in quads of rows).  It takes more registers: where fewer of
+    // the launch's groups fit with it, the general one stays.
+    const int rq = quads(use_rows);
+    BwdRegwKernel lfn = nullptr;
+    if (use_rows <= 8 && wv == kWaves && !lds_share) lfn = dtype == RTN_DTYPE_BF16 ? bwd_local_table_bf16(ksb_room, mt) : rq > 0 ? bwd_local_table_f32(ksb_room, mt, rq) : nullptr;
+    int own_per_cu = 0;
+    if (lfn && (rc = occupancy_per_cu((const void*)lfn, 64 * wv, 0, &own_per_cu)) != RTN_OK) return rc;
+    auto take_local = [&](BwdChoice* p, bool own) {
+      p->local = true;
+      if (own) {
+        p->kernel = (const void*)lfn;
+        p->one_xcd_kernel = true;
+        p->rq = rq;
+      }
+    };
+    const long long wanted = (long long)count * groups_needed;
+    const bool own_fits = lfn && on_xcds(own_per_cu) >= wanted;
+    if (own_fits || on_xcds(per_cu) >= wanted) {
       c.groups_per_launch = (int)groups_needed;
-      c.local = true;
+      take_local(&c, own_fits);
       best = c;
       break;
     }
@@ -2305,14 +2319,14 @@ int choose_bwd_kernel(const BwdCtx& x, BwdChoice* out) {
     // Too many rows for one launch: remember the candidate that takes most rows per launch; the batch groups
     // then run in turns (the rows of a batch are independent of each other).  A turn whose groups fit an XCD each
     // is an XCD-local launch, unless that costs more than an eighth of the groups a launch can hold.
-    const long long fit_local = fits_xcd ? (long long)di.xcds * ((cu_x * per_cu) / G_wgs) / count : 0;
+    const long long fit_local = on_xcds(per_cu) / count;
     const bool local_turns = fit_local >= 1 && fit_local * 8 >= fit * 7;
     const long long turn_fit = local_turns ? fit_local : fit;
     if (turn_fit >= 1 && turn_fit * use_rows > turn_rows &&
         (groups_needed + turn_fit - 1) / turn_fit <= env_long("RTN_LSTM2_MAX_PASSES", kMaxPassesOverSteps)) {
       turn_rows = turn_fit * use_rows;
       c.groups_per_launch = (int)turn_fit;
-      c.local = local_turns;
+      if (local_turns) take_local(&c, lfn && on_xcds(own_per_cu) / count >= fit_local);
       turn = c;
     }
   }
@@ -2394,13 +2408,15 @@ int bwd_launch_persistent(const BwdCtx& x, const BwdChoice& ch, const BwdLayout&
     q.nframes = (int)j.num_steps;
     q.Bg = (B + bgroups - 1) / bgroups;
     q.ksb = ch.ksb;
-    // The kernels that keep one (row, k) pair per thread ask for a frame's inputs in front of the MFMAs, so only the
-    // delay stands between a frame's stores and the read of its ring slot: inside an XCD it is a fixed one there, as in
-    // the forward kernel (measured: 2.77 ms at 10 units against 2.82 adaptive and 2.87 / 2.86 at 4 / 16 for the layer; float32
-    // in quads of rows 1.085 ms at 5 units, 1.117 adaptive, 1.087 / 1.087 / 1.125 at 0 / 10 / 20).
+    // A fixed delay between a frame's stores and the read of its ring slot for groups of up to 8 rows inside an XCD, as in the forward
+    // kernel; the others adapt.  In the kernel for such groups what passes of it with the next frame's factors is not counted.  (us per frame
+    // of the gradient op at 0 / 2 / 4 / 8 / 12 units: bf16 n = 1024, two of 32 rows, 2.52 / 2.52 / 2.50 / 2.58 / 2.67; n = 512, two of 16 rows,
+    // 1.76 / 1.76 / 1.74 / 1.71 / 1.74; float32 n = 500, two of 40 rows, 4.90 / 4.90 / 4.94 / 5.03 / 5.14.  The general kernel: 2.77 ms for a
+    // layer at 10 units, 2.82 adaptive, 2.87 / 2.86 at 4 / 16.)
     const bool one_pair = ch.rows_per_group <= 8 && ((ch.tiles + ch.waves / 4 - 1) / (ch.waves / 4)) % 2 == 0;
-    const bool fixed_delay = ch.local && (one_pair || ch.rq > 0);
-    q.poll_delay = (int)std::max<long>(0, std::min<long>(64, env_long("RTN_LSTM2_BWD_POLL_DELAY", fixed_delay ? (ch.rq > 0 ? 5 : 10) : 20)));
+    const bool fixed_delay = ch.one_xcd_kernel || (ch.local && one_pair);
+    const long first_delay = !fixed_delay ? 20 : !ch.one_xcd_kernel ? 10 : x.dtype == RTN_DTYPE_BF16 && n > 256 ? (ch.tiles == 1 ? 8 : 4) : 2;
+    q.poll_delay = (int)std::max<long>(0, std::min<long>(64, env_long("RTN_LSTM2_BWD_POLL_DELAY", first_delay)));
     q.delay_inc = (int)std::max<long>(0, std::min<long>(16, env_long("RTN_LSTM2_BWD_DELAY_INC", fixed_delay ? 0 : 2)));
     {
       long dec = env_long("RTN_LSTM2_BWD_DELAY_DEC", 16);  // steps per unit of downward adaptation: a power of two

@@ -100,6 +100,45 @@ def test_bwd_quads_of_rows(B, n, tiles, quads):
             assert _rel_to_max(a, b) <= 2e-5, (name, _rel_to_max(a, b), plan)
 
 
+# The kernel for groups of up to 8 rows on one XCD each: one, two and four tiles, shares of one, of an odd and of a full number of
+# macro steps per wavefront, cut groups, and runs of one and two frames (the first is in front of the kernel's loop).
+@pytest.mark.parametrize("dtype,B,n", [("bf16", 3, 16), ("bf16", 9, 80), ("bf16", 21, 208), ("bf16", 17, 512), ("bf16", 30, 1024), ("bf16", 130, 256), ("bf16", 250, 256),
+                                       ("f32", 2, 16), ("f32", 5, 144), ("f32", 13, 512), ("f32", 61, 512), ("f32", 250, 256)])
+def test_bwd_groups_of_one_xcd(dtype, B, n):
+    """Against the oracle and against the plan that spreads a group over the XCDs (another kernel: equal to rounding, 1e-5 of the
+    largest magnitude in float32, one bfloat16 step of it in bfloat16).  Rows are independent: errors that are not finite stay in
+    their row, and every other row keeps its bits."""
+    from _gpu_util import env
+
+    announce("bwd groups of one xcd", dtype, B, n)
+    bar, step_bar = (2e-2, 2.0**-7) if dtype == "bf16" else (2e-5, 1e-5)
+    for T, start, step in [(1, 0, 1), (2, 0, -1), (7, 1, 2)]:
+        got, want, _ = _run(T, B, n, dtype, start, step, seed=T + B + n)
+        plan = lib.bwd_plan_text()
+        assert "bwd_regw_xcd" in plan, plan
+        with env(RTN_LSTM2_BWD_LOCAL=0):
+            spread, _, _ = _run(T, B, n, dtype, start, step, seed=T + B + n)
+            assert "bwd_regw_xcd" not in lib.bwd_plan_text(), lib.bwd_plan_text()
+        for name, a, b, c in zip(("DX", "DW", "Dy0", "Dc0"), got, want, spread):
+            assert _rel_to_max(a, b) <= bar, (T, name, _rel_to_max(a, b), plan)
+            assert _rel_to_max(a, c) <= step_bar, (T, name, _rel_to_max(a, c), plan)
+    X, W, y0, c0, i = random_problem(n, 5, B, n)
+    i[:] = 1.0
+    Xd, Wd, y0d = (to_dev(a, dtype) for a in (X, W, y0))
+    c0d, id_ = to_dev(c0, "f32"), to_dev(i, "f32")
+    Y, C, H, _ = get_op()(Xd, Wd, y0d, c0d, id_, 0, 1)
+    DY, Dd = torch.ones_like(Y), torch.ones_like(c0d)
+    clean = torch_native_op.native_lstm2_grad(Wd, y0d, c0d, id_, 0, 1, Y, C, H, DY, Dd)
+    row = B // 2
+    for value in (float("inf"), float("nan")):
+        DY[3, row, n // 2] = value
+        hit = torch_native_op.native_lstm2_grad(Wd, y0d, c0d, id_, 0, 1, Y, C, H, DY, Dd)
+        others = [b for b in range(B) if b != row]
+        assert torch.equal(hit[0][:, others], clean[0][:, others]) and torch.equal(hit[2][others], clean[2][others]) and torch.equal(hit[3][others], clean[3][others])
+        assert not torch.isfinite(hit[0][:4, row].float()).all(-1).any()
+        assert torch.equal(hit[0][4, row], clean[0][4, row])
+
+
 def test_bwd_read_delay_only_moves_time():
     """The delay between a frame's stores and the read of its ring slot (and whether it adapts) decides how often a read is
     repeated, never what is read: every setting gives the same bits, on a plan with one pair per thread and on one without."""
