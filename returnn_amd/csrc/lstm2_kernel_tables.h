@@ -23,12 +23,13 @@ RegwKernel regw_table_bf16_hi(int MT, int NT, int KSMAX, bool half, bool tail);
 RegwKernel regw_table_f32_lo(int MT, int NT, int KSMAX, bool half, bool tail);
 RegwKernel regw_table_f32_hi(int MT, int NT, int KSMAX, bool half, bool tail);
 
-// Forward kernel for small layers k_lstm2_solo<AT, S>: the build for width n; kernel null: none.
+// Forward kernel for small layers k_lstm2_solo<AT, S, R>: the build for width n (one_row: the one with a row per workgroup, if
+// the width has it); kernel null: none.
 struct SoloBuild {
   RegwKernel kernel;
-  int threads;
+  int threads, rows;
 };
-SoloBuild solo_kernel(int dtype, int n);
+SoloBuild solo_kernel(int dtype, int n, bool one_row);
 
 // k_lstm2_dual<__bf16, 8, 8>: two turns of a large batch in one launch.
 RegwKernel dual_kernel();

@@ -140,20 +140,27 @@ WideBuild wide_kernel(int dtype, int n, int cus, int rows) {
   }
   return best;
 }
-// float32 up to n = 64, bf16 up to 128.  Measured at T = 4, 32 and 300 with B = 4 ... 1024, us per call, against k_lstm2_regw: T = 300, B = 4 /
+// Four rows per workgroup: float32 up to n = 64, bf16 up to 128.  Measured at T = 4, 32 and 300 with B = 4 ... 1024, us per call, against k_lstm2_regw: T = 300, B = 4 /
 // 1024: float32 n = 32 184 / 204 against 312 / 396, n = 64 211 / 250 against 310 / 473; bf16 n = 32 121 / 143 against 249 / 296, n = 64 186 / 209
-// against 248 / 349, n = 96 213 / 281 against 253 / 505, n = 128 263 / 338 against 255 / 547 (the one case behind, by 3 %:
-// 4 rows of 300 frames; 64 rows 264 against 266, T = 32 37 / 41 against 39 / 66, since no W is packed).  Beyond, 8 wavefronts' MFMAs on one CU take longer than a
+// against 248 / 349, n = 96 213 / 281 against 253 / 505, n = 128 263 / 338 against 255 / 547.  Beyond, 8 wavefronts' MFMAs on one CU take longer than a
 // hand-over: float32 n = 96 / 128 1.36 / 1.64 us per step against 1.03, bf16 n = 160 1.7 against 0.85.
-SoloBuild solo_kernel(int dtype, int n) {
-#define RTN_SOLO(at, s) if (n <= s * Elem<at>::KM) return {&k_lstm2_solo<at, s>, 64 * solo_waves<at>(s)};
-  if (dtype == 1) {
+// One row per workgroup: float32 up to n = 128 (there 1.01 us per step against 1.06 of k_lstm2_regw with few rows, 1.07 against 1.39 with 256), where W takes
+// half of the CU's registers; bf16 up to 128 (12 wavefronts for n = 160 have too few registers each).
+SoloBuild solo_kernel(int dtype, int n, bool one_row) {
+#define RTN_SOLO(at, s) if (n <= s * Elem<at>::KM) return {&k_lstm2_solo<at, s>, 64 * solo_waves<at>(s), kSoloRows};
+#define RTN_SOLO_ROW(at, s) if (n <= s * Elem<at>::KM) return {&k_lstm2_solo_row<at, s>, 64 * solo_waves<at>(s), 1};
+  if (one_row && dtype == 1) {
+    RTN_SOLO_ROW(__bf16, 1) RTN_SOLO_ROW(__bf16, 2) RTN_SOLO_ROW(__bf16, 3) RTN_SOLO_ROW(__bf16, 4)
+  } else if (one_row) {
+    RTN_SOLO_ROW(float, 2) RTN_SOLO_ROW(float, 4) RTN_SOLO_ROW(float, 6) RTN_SOLO_ROW(float, 8)
+  } else if (dtype == 1) {
     RTN_SOLO(__bf16, 1) RTN_SOLO(__bf16, 2) RTN_SOLO(__bf16, 3) RTN_SOLO(__bf16, 4)
   } else {
     RTN_SOLO(float, 2) RTN_SOLO(float, 4)
   }
 #undef RTN_SOLO
-  return {nullptr, 0};
+#undef RTN_SOLO_ROW
+  return {nullptr, 0, 0};
 }
 #elif RTN_TABLE_PART == 10
 RegwKernel regw_table_f32_quad_tail(int MT, int KSMAX, int RQ) { return regw_table_quad<true>(MT, KSMAX, RQ); }

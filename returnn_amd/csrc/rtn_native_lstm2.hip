@@ -175,7 +175,7 @@ struct Plan {
   bool wide = false;             // persistent kernel for layers whose W takes registers and LDS of the whole device
   WideBuild wide_build = {nullptr, 0, 0, 0, 0, 0};
   bool solo = false;             // small layer: every workgroup takes 4 rows through all steps by itself
-  SoloBuild solo_build = {nullptr, 0};
+  SoloBuild solo_build = {nullptr, 0, 0};
   bool half = false;             // regw: groups of at most 8 rows, two tiles folded into one pass of the pointwise part
   int grid = 0;                  // workgroups launched by the persistent kernel
   int KSMAX = 0;                 // its macro steps per wavefront (template bound)
@@ -260,15 +260,22 @@ bool make_plan_uncached(int64_t T, int B, int n, int dtype, int want_mode, bool 
   bool persistent_ok = false;
   // A small layer whose rows find a CU per four: no workgroup needs another one.  (Ahead up to that many rows at every width it
   // takes, see solo_kernel; a batch beyond keeps several rows per tile busy on the kernels below.  A decomposition or kernel
-  // asked for by the environment is one of theirs.)
-  if (want_mode == RTN_MODE_AUTO && di.valid && !force_generic && B <= kSoloRows * di.cus / std::max(1, std::min(count, kMaxMulti)) && !env_long("RTN_LSTM2_NO_PAD", 0) &&
-      !env_long("RTN_LSTM2_MT", 0) && !env_long("RTN_LSTM2_GROUPS", 0) && !env_long("RTN_LSTM2_KERNEL", 0) && env_long("RTN_LSTM2_LOCAL", -1) < 0 && !env_long("RTN_LSTM2_NO_SOLO", 0))
-    pl.solo_build = solo_kernel(dtype, n);
+  // asked for by the environment is one of theirs.)  With a workgroup per row as long as that gives no SIMD more than two wavefronts, or no CU
+  // more than one workgroup: us per step with one / four rows per workgroup, T = 300, 400 rows (beyond a CU per row): float32 n = 32
+  // 0.57 / 0.66, n = 64 0.74 / 0.78, bf16 n = 32 0.41 / 0.45, n = 64 0.54 / 0.61, n = 96 0.98 / 0.74; 800 rows: n = 32 0.64 / 0.69 and 0.43 / 0.45, n = 64
+  // 1.21 / 0.82 and 0.88 / 0.69.  float32 above 64 has no kernel with four rows: 400 rows of n = 96 take 1.88 against 1.59 of the kernels below; above 96
+  // those keep calls of few rows (n = 128, 4 / 100 / 256 rows: 1.01 / 1.06 / 1.07 against 1.06 / 1.11 / 1.39).
+  const long long all_rows = (long long)B * std::max(1, std::min(count, kMaxMulti));
+  if (want_mode == RTN_MODE_AUTO && di.valid && !force_generic && all_rows <= (long long)kSoloRows * di.cus && !env_long("RTN_LSTM2_NO_PAD", 0) &&
+      !env_long("RTN_LSTM2_MT", 0) && !env_long("RTN_LSTM2_GROUPS", 0) && !env_long("RTN_LSTM2_KERNEL", 0) && env_long("RTN_LSTM2_LOCAL", -1) < 0 && !env_long("RTN_LSTM2_NO_SOLO", 0)) {
+    if (dtype != RTN_DTYPE_F32 || n <= 96 || all_rows > 128) pl.solo_build = solo_kernel(dtype, n, true);
+    if (pl.solo_build.kernel && all_rows > (long long)std::max(1, 8 * 64 / pl.solo_build.threads) * di.cus) pl.solo_build = solo_kernel(dtype, n, false);
+  }
   if (pl.solo_build.kernel) {
     pl.kind = kPlanSolo;
     pl.solo = true;
-    pl.grid = pl.groups = pl.groups_total = (B + kSoloRows - 1) / kSoloRows;
-    pl.Bg = kSoloRows;
+    pl.grid = pl.groups = pl.groups_total = (B + pl.solo_build.rows - 1) / pl.solo_build.rows;
+    pl.Bg = pl.solo_build.rows;
     persistent_ok = true;
   } else if (mfma_shape && !force_generic) {
     pl.kind = kPlanMfma;

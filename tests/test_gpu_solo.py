@@ -65,3 +65,51 @@ def test_several_calls_and_final_outputs():
         single = torch_native_op.native_lstm2_multi([c], mode="stepwise")[0]
         for a, b in zip(o, single):
             assert torch.equal(a, b)
+
+
+# one row per workgroup: every build, widths with copied cells (whole quads of them, a wavefront of them, cut quads); and the number of
+# rows up to which a workgroup has one, which depends on the build's wavefronts, from both sides
+@pytest.mark.parametrize("T,B,n,dtype,groups", [
+    (5, 3, 32, "f32", 3), (4, 2, 65, "f32", 2), (6, 5, 96, "f32", 5), (3, 130, 97, "f32", 130), (9, 129, 128, "f32", 129), (5, 2, 34, "bf16", 2), (5, 3, 68, "bf16", 3), (3, 2, 1, "f32", 2),
+    (2, 1024, 32, "f32", 1024), (2, 512, 64, "f32", 512), (2, 513, 64, "f32", 129), (2, 256, 128, "f32", 256), (2, 512, 40, "bf16", 512), (2, 520, 40, "bf16", 130),
+    (2, 256, 96, "bf16", 256), (2, 257, 96, "bf16", 65),
+])  # fmt: skip
+def test_a_row_per_workgroup(T, B, n, dtype, groups):
+    announce("solo kernel, rows", T, B, n, dtype)
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the limits are those of 256 CUs")
+    plan = lib.describe_plan(T, B, n, lib.DTYPE_BF16 if dtype == "bf16" else lib.DTYPE_F32, lib.MODE_AUTO)
+    assert "kernel=mfma_regw_solo" in plan and " groups=%i " % groups in plan, plan
+    p = random_problem(7800 + n + B, T, B, n)
+    p = (*p[:4], (numpy.random.default_rng(n).uniform(size=(T, B)) < 0.8).astype(numpy.float32))
+    for step in (1, -1):
+        rc, status, got = run_raw(*p, 0, step, dtype=dtype)
+        assert rc == 0 and status == 0
+        if n < 32:
+            want, bars = oracle.native_lstm2_fwd(*p, 0, step), 2e-6
+        else:
+            rc, status, want = run_raw(*p, 0, step, dtype=dtype, mode="stepwise")
+            assert rc == 0 and status == 0
+            bars = 0.0
+        for name, a, b in zip("YCHd", got, want):
+            assert numpy.isfinite(a).all(), name
+            assert numpy.abs(a - b).max() <= bars, (name, plan)
+
+
+@pytest.mark.parametrize("n,dtype", [(70, "f32"), (34, "bf16"), (128, "bf16")])
+def test_values_that_are_not_finite_stay_in_their_row(n, dtype):
+    announce("solo kernel, not finite", n, dtype)
+    T, B = 6, 3
+    X, W, y0, c0, i = random_problem(7900 + n, T, B, n)
+    i[:] = 1.0
+    rc, status, clean = run_raw(X, W, y0, c0, i, 0, 1, dtype=dtype)
+    assert rc == 0 and status == 0
+    for value in (numpy.inf, numpy.nan):
+        X[2, 1, n - 1] = value
+        rc, status, got = run_raw(X, W, y0, c0, i, 0, 1, dtype=dtype)
+        assert rc == 0 and status == 0
+        for name, a, b in zip("YCH", got, clean):
+            assert numpy.array_equal(a[:, [0, 2]], b[:, [0, 2]]) and numpy.array_equal(a[:2], b[:2]), name
+        rc, status, want = run_raw(X, W, y0, c0, i, 0, 1, dtype=dtype, mode="stepwise")
+        for name, a, b in zip("YCHd", got, want):
+            assert numpy.array_equal(a, b, equal_nan=True), name
