@@ -6,6 +6,7 @@ import pytest
 import torch
 
 from _gpu_util import announce
+import returnn_amd.lstm as lstm_mod
 
 pytestmark = pytest.mark.gpu
 
@@ -67,3 +68,39 @@ def test_many_rows_run_as_a_sequence_of_one_frame(B, n_in, n, dtype):
     # at most 1 + 1/4 + |c| / 4 + 1/4 < 2.75, and each output is rounded by 2^-9; float32: two orders of sums of up to 6144
     # products, whose rounding errors of 2^-25 of sums below 4 add up like a random walk: 80 * 2^-23 < 1e-5)
     assert not torch.equal(few, y[:64]) and float((few.float() - y[:64].float()).abs().max()) <= (2**-5 if dtype == "bf16" else 1e-5)
+
+
+@pytest.mark.parametrize("source,params", [("f32", "f32"), ("bf16", "bf16"), ("bf16", "f32"), ("f32", "bf16")])
+def test_module_step_takes_the_same_way_as_the_function(source, params):
+    """The module's step without views of its parameters against :func:`lstm` with prepared ones, in every combination of types, plain and
+    under autocast; what it must hand on -- a gradient wanted, shapes that do not fit, CPU tensors -- does what it did."""
+    dtypes = {"f32": torch.float32, "bf16": torch.bfloat16}
+    B, k, n = 5, 24, 40
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    module = lstm_mod.LSTM(k, n, device="cuda", dtype=dtypes[params])
+    module.reset_parameters(gen)
+    x = torch.randn((B, k), device="cuda", generator=gen).to(dtypes[source])
+    h = torch.randn((B, n), device="cuda", generator=gen).to(dtypes[source])
+    c = torch.randn((B, n), device="cuda", generator=gen)
+    state = lstm_mod.LstmState(h=h, c=c)
+    for region in (False, True):
+        with torch.autocast("cuda", dtype=torch.bfloat16, enabled=region):
+            with torch.no_grad():
+                y, new = module(x, state=state)
+                want, (want_h, want_c) = lstm_mod.lstm(x, state_h=h, state_c=c, weights=module.weights(dtypes[source]))
+                back, _ = module(x, state=state, direction=-1)
+            assert torch.equal(y, want) and torch.equal(new.h, want_h) and torch.equal(new.c, want_c) and torch.equal(back, y)
+            assert y.dtype == want.dtype and new.h.dtype == want_h.dtype and new.c.dtype == torch.float32
+    y, _ = module(x, state=state)
+    assert y.requires_grad
+    y.float().sum().backward()
+    assert module.ff.grad is not None and bool(torch.isfinite(module.rec.grad.float()).all())
+    with torch.no_grad():
+        with pytest.raises(ValueError, match="state_h"):
+            module(x, state=lstm_mod.LstmState(h=h[:, :-1], c=c))
+        with pytest.raises(ValueError, match="in_dim"):
+            module(x[:, :-1], state=state)
+        with pytest.raises(ValueError, match="direction"):
+            module(x, state=state, direction=2)
+        with pytest.raises(RuntimeError, match="HIP"):
+            module(x.cpu(), state=state)
