@@ -41,8 +41,11 @@ __host__ __device__ constexpr DualLds dual_lds(int es, int MT) {
 // n = 1024, B = 256: 3.3 us, 4.3 in turns) the matrix cores are busy for 2050, vector instructions issue in 2300, 2200 go by with an
 // instruction waiting for its turn and 1600 with none to issue; 23 % of the clocks the LDS is busy are bank conflicts.  (The gates
 // of one group woven into the other's MFMAs left the hand-over exposed: 842 us against 690.)
+// SPREAD: groups over all XCDs, for layers of 1024 < n <= 2048, which no XCD holds.  There a step alone is mostly hand-over (of 7400 clocks
+// of 32 rows of n = 2048 the matrix cores had 1400): n = 2048, B = 64, T = 64 4.3 us per step of both, 5.7 in turns; n = 1280, B = 90 3.8, 9.5 in the
+// three turns that two tiles of rows per workgroup made.
 // The order of additions is that of k_lstm2_regw: the same bits.
-template <typename AT, int MT, int KS>
+template <typename AT, int MT, int KS, bool SPREAD>
 __global__ __launch_bounds__(kWgThreads) void k_lstm2_dual(const Lstm2Multi multi) {
   using E = Elem<AT>;
   using SN = Sentinel<AT>;
@@ -53,8 +56,14 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_dual(const Lstm2Multi mult
   constexpr DualLds L = dual_lds(ES, MT);
   const Lstm2Params p = multi.p[0];
   const int X = multi.xcds, G = p.wgs_per_group;
-  const int xcd = (int)blockIdx.x % X, slot = (int)blockIdx.x / X;
-  const int g = (slot / G) * X + xcd, r = slot % G;
+  int g, r;
+  if constexpr (SPREAD) {
+    map_block(p, (int)blockIdx.x, g, r);
+  } else {
+    const int xcd = (int)blockIdx.x % X, slot = (int)blockIdx.x / X;
+    g = (slot / G) * X + xcd;
+    r = slot % G;
+  }
   if (g >= p.groups) return;
 
   extern __shared__ __align__(16) unsigned char smem[];
@@ -206,16 +215,17 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_dual(const Lstm2Multi mult
 
   // That all workgroups of a group share an XCD is checked (both groups of a workgroup have the same workgroups).
   __shared__ int s_local;
-  if (tid == 0) s_local = group_on_one_xcd(p.flags + (size_t)group[0] * G, (unsigned)G, p.status, p.timeout_ticks) ? 1 : 0;
+  if (!SPREAD && tid == 0) s_local = group_on_one_xcd(p.flags + (size_t)group[0] * G, (unsigned)G, p.status, p.timeout_ticks) ? 1 : 0;
 
   auto run = [&](auto ex_tag) {
     constexpr int AUXS = decltype(ex_tag)::value == kExDevice ? kAuxDevice : 0, AUXL = kAuxDevice;
     RTN_TRACE_DECL
-    i32x4 bf[2][KS];
+    constexpr int SETS = SPREAD ? 1 : 2;  // (SPREAD: a group's registers are free when the other group's are asked for)
+    i32x4 bf[SETS][KS];
     auto load = [&](auto set_tag, int s, int ks) {
       constexpr int D = decltype(set_tag)::value;
       const unsigned soff = (unsigned)(s & (kHxRing - 1)) * hx_buf_bytes + (ks < ks_count ? ks : 0) * (unsigned)(4 * kWaves * kFragBytes) * p.Bp;
-      bf[D][ks] = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(ring[D], frag[D], soff, AUXL));
+      bf[D % SETS][ks] = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(ring[D], frag[D], soff, AUXL));
     };
     auto issue = [&](auto set_tag, int s) {  // read the hidden state that enters step s
       asm volatile("" ::: "memory");
@@ -231,7 +241,7 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_dual(const Lstm2Multi mult
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
-          for (int w = 0; w < 4; ++w) m[w] = LM::fold(m[w], (unsigned)bf[D][ks][w]);
+          for (int w = 0; w < 4; ++w) m[w] = LM::fold(m[w], (unsigned)bf[D % SETS][ks][w]);
         return !__any(LM::has_sentinel(LM::fold(LM::fold(m[0], m[1]), LM::fold(m[2], m[3]))));
       };
       // (The first look stands outside the loop: behind these loads stand the other group's stores, for which a wait that
@@ -277,16 +287,20 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_dual(const Lstm2Multi mult
 #pragma unroll
       for (int i = 0; i < KS * MT; ++i) {
         const int ks = i / MT, mt = i % MT;
-        if (i >= KS * MT / 2 && i % (MT / 2) == 0) {
+        if (!SPREAD && i >= KS * MT / 2 && i % (MT / 2) == 0) {
           __builtin_amdgcn_sched_barrier(0);
           load(IntTag<O>{}, D ? s + 1 : s, i / (MT / 2) - KS);
         }
-        acc[mt] = E::mma(wreg[mt][ks], bf[D][ks], acc[mt]);
+        acc[mt] = E::mma(wreg[mt][ks], bf[D % SETS][ks], acc[mt]);
         __builtin_amdgcn_sched_group_barrier(0x008, sizeof(AT) == 2 ? 1 : 4, 0);
         __builtin_amdgcn_sched_group_barrier(0x096, 3, 0);
       }
       asm volatile("" ::: "memory");
       __builtin_amdgcn_sched_barrier(0);
+      // SPREAD: the hand-over takes longer than the half step between, and a read that comes too early is made again, 64 KB per CU
+      // through the memory fabric (n = 2048, B = 64, T = 64, us per step of both: in the second half of the MFMAs 5.4, here 4.3, behind the
+      // barrier 4.3, behind the gates 5.0, at the end 5.1; here with a delay of 2 / 4 / 8 units of 64 clocks in front 4.5 / 4.7 / 4.8).
+      if (SPREAD) issue(IntTag<O>{}, D ? s + 1 : s);
       // The other group's X for the half step after next: behind the loads of h, which would wait for it otherwise.
       fetch(IntTag<O>{}, D ? s + 2 < nsteps : s + 1 < nsteps);
 #pragma unroll
@@ -349,10 +363,13 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_dual(const Lstm2Multi mult
     RTN_TRACE_FLUSH(p, g * G + r)
   };
   __syncthreads();  // s_local
-  if (s_local)
-    run(IntTag<kExLocal>{});
-  else
+  if constexpr (SPREAD) {
     run(IntTag<kExDevice>{});
+  } else if (s_local) {
+    run(IntTag<kExLocal>{});
+  } else {
+    run(IntTag<kExDevice>{});
+  }
   __syncthreads();  // the last step's outputs are staged
   // (As in k_lstm2_regw: an expired wait must show in what a consumer reads.)
   const bool expired = wait_expired(p.status);

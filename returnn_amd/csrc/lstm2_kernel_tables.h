@@ -31,8 +31,8 @@ struct SoloBuild {
 };
 SoloBuild solo_kernel(int dtype, int n, bool one_row);
 
-// k_lstm2_dual<__bf16, 8, 8>: two turns of a large batch in one launch.
-RegwKernel dual_kernel();
+// k_lstm2_dual<__bf16, MT, KSMAX, !local>: two turns of a large batch in one launch; null if the decomposition has no build.
+RegwKernel dual_kernel(int MT, int KSMAX, bool local);
 
 // Forward kernel for wide layers k_lstm2_wide<AT, MT, NT, KS, LF>.
 typedef void (*WideKernel)(const Lstm2Params);

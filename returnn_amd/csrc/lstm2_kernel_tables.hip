@@ -37,6 +37,7 @@ RegwKernel regw_table(int MT, int NT, int KSMAX, bool half) {
     RTN_CASE(8, 1, 8)
     RTN_CASE(1, 1, 16) RTN_CASE(1, 2, 16)
     RTN_CASE(2, 1, 16) RTN_CASE(2, 2, 16)
+    if constexpr (sizeof(AT) == 2) { RTN_CASE(4, 1, 16) }
   } else {
     RTN_CASE(1, 1, 2) RTN_CASE(1, 2, 2) RTN_CASE(1, 4, 2)
     RTN_CASE(2, 1, 2) RTN_CASE(2, 2, 2) RTN_CASE(2, 4, 2)
@@ -173,7 +174,10 @@ BwdRegwKernel bwd_local_table_f32(int KSB, int MT, int RQ) { return RQ == 1 ? bw
 #elif RTN_TABLE_PART == 13
 BwdRegwKernel bwd_local_table_f32_two(int KSB, int MT) { return bwd_local_table<float, 2>(KSB, MT); }
 #elif RTN_TABLE_PART == 14
-RegwKernel dual_kernel() { return &k_lstm2_dual<__bf16, 8, 8>; }
+RegwKernel dual_kernel(int MT, int KSMAX, bool local) {
+  if (local) return MT == 8 && KSMAX == 8 ? &k_lstm2_dual<__bf16, 8, 8, false> : nullptr;
+  return MT == 4 && KSMAX == 16 ? &k_lstm2_dual<__bf16, 4, 16, true> : nullptr;
+}
 #elif RTN_TABLE_PART == 15
 BwdRegwKernel bwd_local_table_bf16(int KSB, int MT) { return bwd_local_table<__bf16, 0>(KSB, MT); }
 #else

@@ -377,7 +377,12 @@ bool make_plan_uncached(int64_t T, int B, int n, int dtype, int want_mode, bool 
             // Workgroups that can share a CU: the register kernel with few fragments per wavefront fits twice.
             const int per_cu = (use_regw && MT * KSMAX <= 32 && KSMAX <= 8) ? max_wgs_per_cu : 1;
             if (G > di.cus * per_cu) continue;
-            if (use_regw && (MT * KSMAX > (KSMAX == 16 ? 32 : 64) || (MT == 8 && KSMAX != 8))) continue;
+            // (bf16 with 16 macro steps per wavefront: four tiles of cells with one of rows.  A layer of 1024 < n <= 2048 hands its hidden state
+            // over through the memory fabric, 4 KB per row and CU at n = 2048: half the rows per group are half of that, us per step for 32 rows of
+            // n = 2048 2.94 against 3.85 of two tiles of each, 17 of n = 1536 2.53 / 3.33, 48 of n = 1280 2.60 / 6.36 in two turns.  float32: 8 times
+            // the MFMA time, and as many registers.)
+            const bool four_tiles = dtype == RTN_DTYPE_BF16 && KSMAX == 16;
+            if (use_regw && (MT * KSMAX > (KSMAX == 16 && !four_tiles ? 32 : 64) || (MT == 8 && KSMAX != 8))) continue;
             const int max_groups = di.cus * per_cu / G;
             for (int groups = 1; groups <= std::min(max_groups, Bq); ++groups) {
               if (env_groups && groups != std::min<long>(env_groups, std::min(max_groups, Bq))) continue;
@@ -386,6 +391,7 @@ bool make_plan_uncached(int64_t T, int B, int n, int dtype, int want_mode, bool 
               if ((Bg + 15) / 16 > 4) continue;
               const int NT = round_nt((Bg + 15) / 16);
               if (use_regw && (NT * KSMAX > 32 || MT * NT > 8)) continue;  // register budget of one wavefront
+              if (use_regw && four_tiles && MT == 4 && NT != 1) continue;
               const size_t lds = use_regw ? (size_t)regw_lds((int)es, MT, NT).total : mfma_lds_bytes(n, dtype, MT, NT);
               if (lds > di.lds_per_wg) continue;
               int pc = per_cu;  // workgroups per CU that LDS allows as well
@@ -489,9 +495,9 @@ bool make_plan_uncached(int64_t T, int B, int n, int dtype, int want_mode, bool 
         pl.passes = (pl.groups_total + pl.groups - 1) / pl.groups;
         pl.grid = chosen.local ? chosen.grid : pl.groups * chosen.G;
         pl.lds_bytes = chosen.lds;
-        // Two turns in one launch (k_lstm2_dual): on XCD-local groups with tiles and shares of W for which there is a build.
-        // (bf16 n = 1024, B = 256, T = 200: 869 us as two launches, 669 as one.)
-        pl.dual = di.valid && chosen.local && pl.passes > 1 && dtype == RTN_DTYPE_BF16 && chosen.MT == 8 && chosen.NT == 1 && chosen.KSMAX == 8 &&
+        // Two turns in one launch (k_lstm2_dual): with tiles and shares of W for which there is a build.  (bf16 n = 1024, B = 256, T = 200: 869 us as
+        // two launches, 669 as one; n = 2048, B = 64, T = 64 362 and 276, n = 1536, B = 40 314 and 246.)
+        pl.dual = di.valid && pl.passes > 1 && dtype == RTN_DTYPE_BF16 && chosen.regw && chosen.NT == 1 && dual_kernel(chosen.MT, chosen.KSMAX, chosen.local) &&
                   dual_lds((int)es, chosen.MT).total + 64 <= di.lds_per_wg && !env_long("RTN_LSTM2_NO_DUAL", 0);
         persistent_ok = true;
       }
@@ -1243,7 +1249,7 @@ int settle_fwd_plan(int count, int64_t T, int B, int nc, int n, int dtype, int m
       if (pl.dual) {
         // Two turns in one launch take another kernel, with more LDS and registers: where that does not fit, the turns go one
         // after the other.  (RTN_LSTM2_DUAL_PER_CU pretends an answer of the runtime.)
-        const void* dk = (const void*)dual_kernel();
+        const void* dk = (const void*)dual_kernel(pl.MT, pl.KSMAX, pl.local);
         const size_t lds = dual_lds((int)esize(dtype), pl.MT).total;
         int dual_per_cu = 0;
         if ((rc = ensure_lds_limit(dk, lds)) != RTN_OK || (rc = occupancy_per_cu(dk, kWgThreads, lds, &dual_per_cu)) != RTN_OK) return rc;
@@ -1468,7 +1474,7 @@ int fwd_calls(const rtn_lstm2_call* calls, int count, int64_t T, int32_t B, int3
           void* args[] = {(void*)&one};
           // (k_lstm2_dual moves whole chunks of 16 bytes only)
           if (pl.dual && g0 + pl.groups < pl.groups_total && p.nc % 8 == 0 && p.exchange == 0) {
-            const void* dk = (const void*)dual_kernel();
+            const void* dk = (const void*)dual_kernel(pl.MT, pl.KSMAX, pl.local);
             const size_t lds = dual_lds((int)esize(dtype), pl.MT).total;
             one.p[1] = one.p[0];
             one.p[1].group_offset = g0 += pl.groups;
