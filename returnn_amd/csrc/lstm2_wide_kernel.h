@@ -10,10 +10,11 @@ namespace rtn {
 
 // ---------------------------------------------------------------------------------------------
 // W of n = 4096 in bf16 is 128 MB: 512 KB for each of the 256 CUs, which have 512 KB of registers and 160 KB of LDS.
-// Launches per step read W from memory every step (22.6 us at 6 TB/s); here a turn reads it once, and a step takes 4.7 us: T = 200,
-// B = 16 4.58 ms as launches per step, 1.00 now, 0.05 of it for the packing.  What bounds a step: the matrix cores are busy for
-// 2048 of its 11 200 clocks, vector instructions issue in 1700, and half of the clocks a wavefront waits for memory -- the
-// two hops of h.  (Fewer frames than pay for a turn's load of W run as launches per step: wide_turns_us in the host code.)
+// Launches per step read W from memory every step (22.6 us at 6 TB/s); here a turn reads it once, and a step takes 4.6 us: T = 200,
+// B = 16 4.58 ms as launches per step, 0.97 now, 0.05 of it for the packing.  What bounds a step: the matrix cores are busy for
+// 2048 of its 10 800 clocks, vector instructions issue in 1700, and half of the clocks a wavefront waits for memory -- the
+// two hops of h.  (More of h in flight, 14 loads per wavefront instead of 8, in smaller chunks: 5 % slower.  What a chunk
+// waits for is the last workgroup that brings its part over.)  (Fewer frames than pay for a turn's load of W run as launches per step: wide_turns_us in the host code.)
 //
 // One batch group of up to 16 * NT rows per launch, on all workgroups: workgroup r owns MT tiles of 4 cells, wavefront w
 // of it the macro steps w, w + 4, ... of k: KS fragments per tile, all but the last LF of the MT * KS in registers, those in
@@ -225,16 +226,16 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_wide(const Lstm2Params p) 
   i32x4 bf[NB][CH * NT];
   fetch(0);
   take();
-  int delay = p.poll_delay;
   RTN_TRACE_DECL
   for (int s = 0; s < nsteps; ++s) {
     const unsigned slot = (unsigned)(s & (kHxRing - 1)) * slot_bytes, old = (unsigned)((s + 2) & (kHxRing - 1)) * slot_bytes;
     // ---- bring this workgroup's part of h_s over
     {
+      // (No delay in front of the first read, as the kernels whose CUs read all of h across the XCDs have it: a repeat is 4 KB per CU and
+      // costs the others nothing.  us per step without / with one that adapts: n = 4096, 16 rows 4.85 / 5.05, one row 5.18 / 5.63; n = 2560, 16 rows 4.01 / 4.45,
+      // 32 rows 6.05 / 6.43.)
       i32x4 fv[kWideForward];
       unsigned spins = 0;
-      if (s > 0)
-        for (int k = 0; k < delay; ++k) __builtin_amdgcn_s_sleep(1);
       bool again;
       do {
         asm volatile("" ::: "memory");
@@ -248,11 +249,6 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_wide(const Lstm2Params p) 
       } while (again);
       RTN_TRACE_MARK(0)  // h_s arrives across the XCDs
       RTN_TRACE_ADD(6, spins)
-      // (a repeated read costs a trip to memory: the delay in front of the first adapts, as in k_lstm2_regw)
-      if (spins)
-        delay = min(delay + p.delay_inc, 64);
-      else if (p.delay_inc && (s & p.delay_dec_mask) == p.delay_dec_mask && delay > 0)
-        --delay;
       const u32x4 ones = u32x4{~0u, ~0u, ~0u, ~0u};
 #pragma unroll
       for (int i = 0; i < kWideForward; ++i) {
