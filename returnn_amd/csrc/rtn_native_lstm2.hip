@@ -1106,34 +1106,46 @@ BwdPadLayout bwd_pad_layout(int64_t T, int B, int np, int dtype) {
   return l;
 }
 
-// dst[rows_dst][blocks][np] := src[rows_src][blocks][n], zeros elsewhere; elements of `es` bytes.
-int launch_pad(const void* src, void* dst, long long rows_src, long long rows_dst, int blocks, int n, int np, size_t es, hipStream_t stream,
-               long long src_pitch = 0) {
-  const long long total = rows_dst * blocks * np;
-  if (total <= 0) return RTN_OK;
-  if (src_pitch == 0) src_pitch = (long long)blocks * n;
-  const dim3 grid((unsigned)std::min<long long>((total + 255) / 256, 8192)), block(256);
-  if (es == 2)
-    hipLaunchKernelGGL(k_pad_cells<unsigned short>, grid, block, 0, stream, (const unsigned short*)src, (unsigned short*)dst, rows_src, rows_dst, blocks, n, np, src_pitch);
-  else
-    hipLaunchKernelGGL(k_pad_cells<unsigned>, grid, block, 0, stream, (const unsigned*)src, (unsigned*)dst, rows_src, rows_dst, blocks, n, np, src_pitch);
-  RTN_HIP(hipGetLastError());
-  return RTN_OK;
-}
+// Copies of rows between a width and its padded one, gathered and launched together (k_pad_rows).
+class PadList {
+ public:
+  explicit PadList(hipStream_t stream) : stream_(stream) {}
+  // dst[rows][blocks][dst_n] := src[rows_src][blocks][src_n] of elements of `es` bytes, cut or zeros elsewhere; a pitch (elements from one row to
+  // the next) of 0: contiguous.  blocks: 1 or 4.
+  int add(const void* src, long long src_pitch, int src_n, long long rows_src, void* dst, long long dst_pitch, int dst_n, long long rows, int blocks, size_t es) {
+    if (rows <= 0 || blocks <= 0 || dst_n <= 0) return RTN_OK;
+    PadJob q;
+    q.src = (const unsigned char*)src;
+    q.dst = (unsigned char*)dst;
+    q.src_pitch = (src_pitch ? src_pitch : (long long)blocks * src_n) * (long long)es;
+    q.dst_pitch = (dst_pitch ? dst_pitch : (long long)blocks * dst_n) * (long long)es;
+    q.rows_src = rows_src;
+    q.rows = rows;
+    q.src_bytes = (int)(src_n * es);
+    q.dst_bytes = (int)(dst_n * es);
+    q.block_shift = blocks == 4 ? 2 : 0;
+    const unsigned long long all = (unsigned long long)(uintptr_t)src | (unsigned long long)(uintptr_t)dst | (unsigned long long)q.src_pitch | (unsigned long long)q.dst_pitch |
+                                   (unsigned long long)q.src_bytes | (unsigned long long)q.dst_bytes;
+    q.unit = all % 16 == 0 ? 16 : all % 8 == 0 ? 8 : all % 4 == 0 ? 4 : 2;
+    jobs_.job[count_++] = q;
+    blocks_ = std::max(blocks_, (rows * blocks + 15) / 16);  // (four wavefronts of four rows)
+    return count_ == kMaxPadJobs ? launch() : RTN_OK;
+  }
+  int launch() {
+    if (!count_) return RTN_OK;
+    hipLaunchKernelGGL(k_pad_rows, dim3((unsigned)std::min<long long>(blocks_, 2048), (unsigned)count_), dim3(kWgThreads), 0, stream_, jobs_);
+    RTN_HIP(hipGetLastError());
+    count_ = 0;
+    blocks_ = 0;
+    return RTN_OK;
+  }
 
-// dst[rows][blocks][n] := src[rows][blocks][np]; dst_pitch: elements from one row of dst to the next (0: blocks * n).
-int launch_unpad(const void* src, void* dst, long long rows, int blocks, int n, int np, size_t es, hipStream_t stream, long long dst_pitch = 0) {
-  const long long total = rows * blocks * n;
-  if (total <= 0) return RTN_OK;
-  if (dst_pitch == 0) dst_pitch = (long long)blocks * n;
-  const dim3 grid((unsigned)std::min<long long>((total + 255) / 256, 8192)), block(256);
-  if (es == 2)
-    hipLaunchKernelGGL(k_unpad_cells<unsigned short>, grid, block, 0, stream, (const unsigned short*)src, (unsigned short*)dst, rows, blocks, n, np, dst_pitch);
-  else
-    hipLaunchKernelGGL(k_unpad_cells<unsigned>, grid, block, 0, stream, (const unsigned*)src, (unsigned*)dst, rows, blocks, n, np, dst_pitch);
-  RTN_HIP(hipGetLastError());
-  return RTN_OK;
-}
+ private:
+  hipStream_t stream_;
+  PadJobs jobs_;
+  int count_ = 0;
+  long long blocks_ = 0;
+};
 
 // rows x row_elems elements := 0, rows pitch elements apart (row_elems * es a multiple of 4)
 int launch_clear_rows(void* dst, long long rows, long long row_elems, long long pitch, size_t es, hipStream_t stream) {
@@ -1354,7 +1366,8 @@ int fwd_calls(const rtn_lstm2_call* calls, int count, int64_t T, int32_t B, int3
       hipLaunchKernelGGL(k_copy_f32, dim3((unsigned)std::min<long long>((bn + 255) / 256, 1024)), dim3(256), 0, stream,
                          calls[k].c0, calls[k].d, bn);
       RTN_HIP(hipGetLastError());
-      if (calls[k].hN && calls[k].y0 && (rc = launch_pad(calls[k].y0, calls[k].hN, B, B, 1, n, n, esize(dtype), stream)) != RTN_OK) return rc;
+      PadList copy(stream);
+      if (calls[k].hN && calls[k].y0 && ((rc = copy.add(calls[k].y0, 0, n, B, calls[k].hN, 0, n, B, 1, esize(dtype))) != RTN_OK || (rc = copy.launch()) != RTN_OK)) return rc;
     }
     return RTN_OK;
   }
@@ -2160,38 +2173,38 @@ int bwd_padded(const BwdCtx& x, int np, void* workspace, size_t workspace_bytes)
   const long long tb = (long long)x.T * B;
   int rc = RTN_OK;
   std::vector<rtn_lstm2_bwd_call> padded((size_t)x.count);
+  PadList pads(x.stream);
   for (int k = 0; k < x.count; ++k) {
     const rtn_lstm2_bwd_call& c = x.calls[k];
     unsigned char* base = (unsigned char*)workspace + (size_t)k * each + lay_p.total;
-    if ((rc = launch_pad(c.W, base + L.W, n, np, 4, n, np, es, x.stream)) != RTN_OK) return rc;
-    if ((rc = launch_pad(c.y0, base + L.y0, B, B, 1, n, np, es, x.stream)) != RTN_OK) return rc;
-    if ((rc = launch_pad(c.c0, base + L.c0, B, B, 1, n, np, 4, x.stream)) != RTN_OK) return rc;
     long long ldY = 0, ldDY = 0, ldDX = 0;
     if ((rc = resolve_pitch("ldY", c.ldY, n, B, es, &ldY)) != RTN_OK) return rc;
     if ((rc = resolve_pitch("ldDY", c.ldDY, n, B, es, &ldDY)) != RTN_OK) return rc;
     if ((rc = resolve_pitch("ldDX", c.ldDX, 4LL * n, B, es, &ldDX)) != RTN_OK) return rc;
-    if ((rc = launch_pad(c.Y, base + L.Y, tb, tb, 1, n, np, es, x.stream, ldY)) != RTN_OK) return rc;
+    auto in = [&](const void* src, size_t at, long long rows, int blocks, size_t size, long long pitch = 0) { return pads.add(src, pitch, n, rows, base + at, 0, np, rows, blocks, size); };
+    if ((rc = in(c.H, L.H, tb, 4, es)) != RTN_OK || (rc = in(c.Y, L.Y, tb, 1, es, ldY)) != RTN_OK || (rc = in(c.DY, L.DY, tb, 1, es, ldDY)) != RTN_OK) return rc;
     // the sibling op that keeps its cell states in H hands H in for C as well; it is not read then
-    if (!(x.op_flags & kOpH0IsCell) && (rc = launch_pad(c.C, base + L.C, tb, tb, 1, n, np, 4, x.stream)) != RTN_OK) return rc;
-    if ((rc = launch_pad(c.H, base + L.H, tb, tb, 4, n, np, es, x.stream)) != RTN_OK) return rc;
-    if ((rc = launch_pad(c.DY, base + L.DY, tb, tb, 1, n, np, es, x.stream, ldDY)) != RTN_OK) return rc;
-    if ((rc = launch_pad(c.Dd, base + L.Dd, B, B, 1, n, np, 4, x.stream)) != RTN_OK) return rc;
+    if (!(x.op_flags & kOpH0IsCell) && (rc = in(c.C, L.C, tb, 1, 4)) != RTN_OK) return rc;
+    if ((rc = pads.add(c.W, 0, n, n, base + L.W, 0, np, np, 4, es)) != RTN_OK || (rc = in(c.y0, L.y0, B, 1, es)) != RTN_OK || (rc = in(c.c0, L.c0, B, 1, 4)) != RTN_OK ||
+        (rc = in(c.Dd, L.Dd, B, 1, 4)) != RTN_OK)
+      return rc;
     padded[(size_t)k] = {base + L.W, base + L.y0, (const float*)(base + L.c0), c.i, c.start, c.step, base + L.Y,
                          (const float*)(base + ((x.op_flags & kOpH0IsCell) ? L.H : L.C)), base + L.H, base + L.DY,
                          (const float*)(base + L.Dd), base + L.DX, (float*)(base + L.DW), base + L.Dy0, (float*)(base + L.Dc0),
                          0, 0, 0};
   }
+  if ((rc = pads.launch()) != RTN_OK) return rc;
   rc = bwd_calls(padded.data(), x.count, x.T, B, np, x.dtype, workspace, need, (void*)x.stream, x.op_flags, each);
   if (rc != RTN_OK) return rc;
   for (int k = 0; k < x.count; ++k) {
     const rtn_lstm2_bwd_call& c = x.calls[k];
     const rtn_lstm2_bwd_call& q = padded[(size_t)k];
-    if ((rc = launch_unpad(q.DX, c.DX, tb, 4, n, np, es, x.stream, c.ldDX)) != RTN_OK) return rc;
-    if ((rc = launch_unpad(q.DW, c.DW, n, 4, n, np, 4, x.stream)) != RTN_OK) return rc;
-    if ((rc = launch_unpad(q.Dy0, c.Dy0, B, 1, n, np, es, x.stream)) != RTN_OK) return rc;
-    if ((rc = launch_unpad(q.Dc0, c.Dc0, B, 1, n, np, 4, x.stream)) != RTN_OK) return rc;
+    auto out = [&](const void* src, void* dst, long long rows, int blocks, size_t size, long long pitch = 0) { return pads.add(src, 0, np, rows, dst, pitch, n, rows, blocks, size); };
+    if ((rc = out(q.DX, c.DX, tb, 4, es, c.ldDX)) != RTN_OK || (rc = out(q.DW, c.DW, n, 4, 4)) != RTN_OK || (rc = out(q.Dy0, c.Dy0, B, 1, es)) != RTN_OK ||
+        (rc = out(q.Dc0, c.Dc0, B, 1, 4)) != RTN_OK)
+      return rc;
   }
-  return RTN_OK;
+  return pads.launch();
 }
 
 // Persistent kernel: W in registers for the whole call, if a wavefront's share of the 16 x 4n slice fits (2..32

@@ -508,3 +508,24 @@ def test_column_sums(rows, width, dtype, out_dtype):
     if size:
         assert cabi.rtn_column_sums(xd.data_ptr(), rows, width, 0, out.data_ptr(), 0, ws.data_ptr(), size - 1, None) == lib.RTN_ERR_WORKSPACE
     assert cabi.rtn_column_sums(xd.data_ptr(), rows, width + 1, 0, out.data_ptr(), 0, ws.data_ptr(), size, None) == lib.RTN_ERR_SHAPE
+
+
+# widths whose rows are not aligned to 16 bytes run on padded copies: pieces of 2, 4 and 8 bytes, rows beyond a multiple of four, one and two
+# calls (more arrays than one launch of the copies takes), a pitch that decides the piece
+@pytest.mark.parametrize("dtype,B,n", [("bf16", 5, 33), ("bf16", 3, 34), ("bf16", 7, 60), ("bf16", 2, 101), ("f32", 5, 33), ("f32", 3, 34), ("f32", 1, 65)])
+def test_bwd_padded_copies(dtype, B, n):
+    announce("bwd padded copies", dtype, B, n)
+    bar = 2e-2 if dtype == "bf16" else 2e-5
+    for T, step in [(1, 1), (6, -1)]:
+        got, want, (X, W, y0, c0, i, DY, Dd) = _run(T, B, n, dtype, 0, step, seed=T + n)
+        for name, a, b in zip(("DX", "DW", "Dy0", "Dc0"), got, want):
+            assert a.shape == b.shape and _rel_to_max(a, b) <= bar, (T, name, _rel_to_max(a, b))
+        Xd, Wd, y0d, DYd = (to_dev(a, dtype) for a in (X, W, y0, DY))
+        c0d, id_, Ddd = (to_dev(a, "f32") for a in (c0, i, Dd))
+        Y, C, H, _ = get_op()(Xd, Wd, y0d, c0d, id_, 0, step)
+        wide = torch.full((T, B, n + 19), float("nan"), dtype=DYd.dtype, device="cuda:0")  # (rows further apart, and not aligned like the width)
+        wide[..., 16 : 16 + n] = DYd
+        calls = [(Wd, y0d, c0d, id_, 0, step, Y, C, H, dy, Ddd) for dy in (DYd, wide[..., 16 : 16 + n])]
+        for grads in torch_native_op.native_lstm2_grad_multi(calls):
+            for name, a, b in zip(("DX", "DW", "Dy0", "Dc0"), grads, got):
+                assert _rel_to_max(a.float().cpu().numpy(), b) <= (1e-5 if dtype == "f32" else 2.0**-7), (T, name)
