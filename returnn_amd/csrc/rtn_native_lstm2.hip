@@ -2229,10 +2229,10 @@ int choose_bwd_kernel(const BwdCtx& x, BwdChoice* out) {
   // 2.55 / 2.79, 8 x 2 x 4: 3.4); the first whose workgroups are all on the device together.  A candidate whose groups
   // fit an XCD each (n / (16 * tiles) workgroups, all groups of all problems in one launch) runs XCD-local: the ring
   // then goes from writer to readers through that XCD's L2 instead of through memory.
-  // In front of them, for bf16 only and only where its groups fit an XCD each: 4 rows x 2 tiles, the kernel with one
+  // In front of them, for bf16 only and only where its groups fit an XCD each: 4 rows x 2 tiles or, for more rows, 8 x 2, the kernel with one
   // (row, k) pair per thread (one problem of cfg3: 4.82 ms against 5.03 for 8 x 1 x 4, whose groups of 64 workgroups
   // span two XCDs; in float32 two tiles double an MFMA time that is long already: cfg2 3.1 ms against 2.3).
-  const int candidates[][4] = {{4, 2, 4, 1}, {8, 1, 4, 0}, {8, 1, 8, 0}, {8, 2, 4, 0}, {16, 1, 4, 0}, {16, 1, 8, 0}, {16, 2, 4, 0}, {8, 4, 4, 0}, {16, 4, 4, 0}};
+  const int candidates[][4] = {{4, 2, 4, 1}, {8, 2, 4, 1}, {8, 1, 4, 0}, {8, 1, 8, 0}, {8, 2, 4, 0}, {16, 1, 4, 0}, {16, 1, 8, 0}, {16, 2, 4, 0}, {8, 4, 4, 0}, {16, 4, 4, 0}};
   const DeviceInfo di = device_info();
   const long want_local = env_long("RTN_LSTM2_BWD_LOCAL", 1);
   // Groups of up to 8 rows in float32: the product in quads of rows (a group's rows: the batch dealt evenly to the groups).
@@ -2308,7 +2308,6 @@ int choose_bwd_kernel(const BwdCtx& x, BwdChoice* out) {
     const long long groups_needed = (B + use_rows - 1) / use_rows;
     const long long G_wgs = n / (16 * mt), cu_x = di.xcds > 0 ? di.cus / di.xcds : 0;
     if (local_only && n / 16 <= cu_x * per_cu) continue;  // (groups of one tile per workgroup fit an XCD themselves)
-    if (local_only && 2 * (long long)count * groups_needed * G_wgs < di.cus) continue;  // (few rows: the wider spread wins, cfg5 7.98 against 8.41 ms)
     // Groups on one XCD each: how many a launch holds with `fit` workgroups to a CU.
     auto on_xcds = [&](int fit) { return want_local && di.xcds > 1 && fit >= 1 && G_wgs <= cu_x * fit ? (long long)di.xcds * ((cu_x * fit) / G_wgs) : 0LL; };
     // Groups of up to 8 rows have a kernel of their own there (float32: in quads of rows).  It takes more registers: where fewer of
@@ -2328,6 +2327,9 @@ int choose_bwd_kernel(const BwdCtx& x, BwdChoice* out) {
     };
     const long long wanted = (long long)count * groups_needed;
     const bool own_fits = lfn && on_xcds(own_per_cu) >= wanted;
+    // (The general kernel with few rows: the wider spread wins, bf16 n = 1024 with one row 7.98 against 8.41 ms for 4000 frames.  The other one is ahead of it:
+    // us per frame n = 1024, one row 2.02 against 2.27, 8 rows 2.15 / 2.34; n = 640, two of 20 rows 2.33 / 2.62; n = 768, 4 rows 2.06 / 2.26.)
+    if (local_only && !own_fits && 2 * (long long)count * groups_needed * G_wgs < di.cus) continue;
     if (own_fits || on_xcds(per_cu) >= wanted) {
       c.groups_per_launch = (int)groups_needed;
       take_local(&c, own_fits);
