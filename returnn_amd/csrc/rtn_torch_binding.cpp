@@ -328,7 +328,7 @@ std::pair<std::vector<Out4>, Tensor> lstm2_multi(const std::vector<FwdArgs>& arg
   if (joint && !Yj.defined()) {
     std::vector<Tensor> ys;
     for (const Out4& o : outs) ys.push_back(std::get<0>(o));
-    Yj = at::cat(ys, -1);
+    Yj = count == 1 ? ys[0] : at::cat(ys, -1);  // (one array joined with nothing is a copy of all of it: n = 604, T B = 69 696, bf16 29 us)
   }
   return {outs, Yj};
 }
@@ -451,7 +451,7 @@ std::pair<std::vector<Out4>, Tensor> lstm2_grad_multi(const std::vector<BwdArgs>
   if (joint && !DXj.defined()) {
     std::vector<Tensor> dx;
     for (const Out4& o : outs) dx.push_back(std::get<0>(o));
-    DXj = at::cat(dx, -1);
+    DXj = count == 1 ? dx[0] : at::cat(dx, -1);
   }
   return {outs, DXj};
 }
