@@ -22,7 +22,7 @@ HOST_SOURCE = "rtn_native_lstm2.hip"
 TABLES_SOURCE = "lstm2_kernel_tables.hip"  # compiled once per part: the instantiations of the persistent kernels
 TABLE_PARTS = 15
 SOURCES = [HOST_SOURCE, TABLES_SOURCE]
-HEADERS = ["lstm2_kernels.h", "lstm2_step_kernel.h", "lstm2_wide_kernel.h", "lstm2_solo_kernel.h", "lstm2_dual_kernel.h", "lstm2_bwd_kernels.h", "lstm2_bwd_local_kernel.h", "lstm2_params.h", "lstm2_kernel_tables.h",
+HEADERS = ["lstm2_kernels.h", "lstm2_step_kernel.h", "lstm2_wide_kernel.h", "lstm2_solo_kernel.h", "lstm2_dual_kernel.h", "lstm2_bwd_kernels.h", "lstm2_bwd_local_kernel.h", "weight_grad_kernel.h", "lstm2_params.h", "lstm2_kernel_tables.h",
            os.path.join("..", "..", "include", "rtn_native_lstm2.h")]  # fmt: skip
 # the torch side of the calls (host code only)
 BINDING_SOURCE = "rtn_torch_binding.cpp"

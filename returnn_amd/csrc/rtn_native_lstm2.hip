@@ -29,6 +29,7 @@
 #include "lstm2_kernel_tables.h"
 #include "lstm2_kernels.h"
 #include "lstm2_step_kernel.h"
+#include "weight_grad_kernel.h"
 
 // Scratch memory of rtn_native_lstm2_fwd_static, the entry point for callers that cannot allocate: a fixed array in the
 // code object, one copy per GPU the library runs on, held until the process ends.  Host code never uses this name as an
@@ -1596,8 +1597,19 @@ int gemm_row_major(rocblas_handle h, bool trans_a, bool trans_b, long long M, lo
   return RTN_OK;
 }
 
+// Slices of the rows that the weight gradient of a layer of width n is summed in at most (see weight_grad_kernel.h): two workgroups per CU
+// in all; 0: the product goes to the library, which with more tiles of output fills the chip itself (gradient op, us, library / this, for T B = 80, 2000, 30 000:
+// float32 n = 256 55 / 53, 189 / 187, 937 / 662, n = 384 72 / 73, 275 / 266, 1398 / 1292, n = 512 73 / 79, 289 / 291, 1415 / 1474; bf16, whose products the library takes at 8
+// times the rate, n = 192 60 / 43, 162 / 152, 538 / 514, n = 256 62 / 44, 165 / 162, 555 / 535, n = 320 63 / 50, 175 / 180, 675 / 758).
+int weight_grad_slices(int n, int dtype) {
+  if (n % 4 != 0 || n < 4 || n > (dtype == RTN_DTYPE_BF16 ? 256 : 384)) return 0;
+  const int tiles = ((n + kWeightTile - 1) / kWeightTile) * ((4 * n + kWeightTile - 1) / kWeightTile);
+  const int slices = std::max(1, 512 / tiles);
+  return slices >= 8 ? slices / 8 * 8 : slices;
+}
+
 struct BwdLayout {
-  size_t off_sync = 0, off_dyw = 0, off_dx0 = 0, off_wpk = 0, off_ex = 0, total = 0;  // [0, off_wpk) is cleared at the start of a call
+  size_t off_sync = 0, off_dyw = 0, off_dx0 = 0, off_wpk = 0, off_ex = 0, off_part = 0, total = 0;  // [0, off_wpk) is cleared at the start of a call
 };
 BwdLayout bwd_layout(int B, int n, int dtype) {
   BwdLayout l;
@@ -1614,6 +1626,8 @@ BwdLayout bwd_layout(int B, int n, int dtype) {
   // rows in frames of 8, or of more than 8 rows in frames of 16: never more than 2B + 16 rows in all
   l.off_ex = off;
   if (n % 16 == 0) off = align_up(off + (size_t)kExRing * 4 * n * esize(dtype) * (2 * (size_t)B + 16), 256);
+  l.off_part = off;  // the weight gradient's slices and y0^T dx0
+  if (const int slices = weight_grad_slices(n, dtype)) off = align_up(off + (size_t)(slices + 1) * 4 * n * n * 4, 256);
   l.total = off;
   return l;
 }
@@ -2579,19 +2593,81 @@ int bwd_launch_per_frame(const BwdCtx& x, bool mfma, const BwdLayout& lay, BwdJo
   return replay_graph(key, &p, sizeof(p), stream, record);
 }
 
+// The weight gradients of x's calls by k_weight_grad, as many calls per launch as it takes; *done: whether it does (layers for which the
+// library's products leave most of the chip idle; consecutive frames; rows a multiple of four elements apart).
+int bwd_own_weight_gradients(const BwdCtx& x, const BwdLayout& lay, const std::vector<BwdJob>& jobs, bool* done) {
+  const int n = x.n, max_slices = weight_grad_slices(n, x.dtype);
+  *done = false;
+  if (!max_slices) return RTN_OK;
+  long long longest = 0, widest = 4LL * n;
+  for (int k = 0; k < x.count; ++k) {
+    const BwdJob& j = jobs[(size_t)k];
+    if (j.num_steps > 1 && j.abs_step != 1) return RTN_OK;
+    if (j.ldY % 4 != 0 || j.p.ldDX % 4 != 0) return RTN_OK;
+    longest = std::max(longest, (j.num_steps - 1) * x.B);
+    widest = std::max({widest, (long long)j.ldY, (long long)j.p.ldDX});
+  }
+  constexpr int kRound = 2 * 4 * kWaves * kWeightAhead;  // rows of one round of the kernel's loop
+  WeightGradArgs args;
+  memset(&args, 0, sizeof(args));
+  args.m = n;
+  args.n = 4 * n;
+  args.slices = (int)std::max<long long>(1, std::min<long long>(max_slices, (longest + kRound - 1) / kRound));
+  args.slice_rows = (std::max<long long>(longest, 1) + args.slices - 1) / args.slices;
+  args.parts = args.slices + 1;
+  // (float32 n = 320, 2000 rows: 251 us in the library, 257 here; 30 000 rows 1384 and 1154)
+  if (n > 256 && longest < 8192) return RTN_OK;
+  // (offsets inside a slice, with the rows asked for behind it, are 32 bits wide)
+  if ((std::max<long long>(args.slice_rows, x.B) + 2 * kRound) * widest * (long long)x.es >= (1LL << 30)) return RTN_OK;
+  const int tiles = ((args.m + kWeightTile - 1) / kWeightTile) * ((args.n + kWeightTile - 1) / kWeightTile);
+  for (int k = 0; k < x.count; k += kMaxWeightCalls) {
+    const int now = std::min(kMaxWeightCalls, x.count - k);
+    for (int i = 0; i < now; ++i) {
+      const rtn_lstm2_bwd_call& c = x.calls[k + i];
+      const BwdJob& j = jobs[(size_t)(k + i)];
+      const long long lo = std::min(j.first, j.end);
+      WeightGradCall& q = args.call[i];
+      q.a[0] = (const unsigned char*)c.Y + (size_t)(lo + std::max(0, -c.step)) * x.B * j.ldY * x.es;
+      q.b[0] = (const unsigned char*)c.DX + (size_t)(lo + std::max(0, c.step)) * x.B * j.p.ldDX * x.es;
+      q.rows[0] = (j.num_steps - 1) * x.B;
+      q.lda[0] = j.ldY;
+      q.ldb[0] = j.p.ldDX;
+      q.a[1] = c.y0;
+      q.b[1] = j.p.dx0;
+      q.rows[1] = x.B;
+      q.lda[1] = n;
+      q.ldb[1] = 4 * n;
+      q.part = (float*)(j.ws + lay.off_part);
+      q.out = c.DW;
+    }
+    const dim3 grid((unsigned)(tiles * args.parts), (unsigned)now), block(kWgThreads);
+    if (x.dtype == RTN_DTYPE_BF16)
+      hipLaunchKernelGGL(k_weight_grad<__bf16>, grid, block, 0, x.stream, args);
+    else
+      hipLaunchKernelGGL(k_weight_grad<float>, grid, block, 0, x.stream, args);
+    RTN_HIP(hipGetLastError());
+    hipLaunchKernelGGL(k_weight_grad_sum, dim3((unsigned)(((long long)args.m * args.n / 4 + 63) / 64), (unsigned)now), block, 0, x.stream, args);
+    RTN_HIP(hipGetLastError());
+  }
+  *done = true;
+  return RTN_OK;
+}
+
 // DW = sum over consecutive visited frames Y[t - step]^T * DX[t]  (returnn/native_op.py:1433-1452), then += y0^T * dx0
-// (:1456-1460), in rocBLAS; where the recurrence ran per frame, Dy0 from its float32 working copy.
-int bwd_weight_gradients(const BwdCtx& x, rocblas_handle blas, const std::vector<BwdJob>& jobs, bool persistent) {
+// (:1456-1460), by the kernel for small layers or in rocBLAS; where the recurrence ran per frame, Dy0 from its float32 working copy.
+int bwd_weight_gradients(const BwdCtx& x, rocblas_handle blas, const BwdLayout& lay, const std::vector<BwdJob>& jobs, bool persistent) {
   const int n = x.n, B = x.B;
   const dim3 fill_grid(256), fill_block(256);
-  int rc = RTN_OK;
+  bool own = false;
+  int rc = bwd_own_weight_gradients(x, lay, jobs, &own);
+  if (rc != RTN_OK) return rc;
   for (int k = 0; k < x.count; ++k) {
     const rtn_lstm2_bwd_call& c = x.calls[k];
     const BwdJob& j = jobs[(size_t)k];
     const int step = c.step;
     const unsigned char* Yb = (const unsigned char*)c.Y;
     const unsigned char* DXb = (const unsigned char*)c.DX;
-    if (j.num_steps > 1) {
+    if (j.num_steps > 1 && !own) {
       if (j.abs_step == 1) {
         const long long lo = std::min(j.first, j.end);
         rc = dw_product(blas, Yb + (size_t)(lo + std::max(0, -step)) * B * j.ldY * x.es,
@@ -2605,8 +2681,7 @@ int bwd_weight_gradients(const BwdCtx& x, rocblas_handle blas, const std::vector
         }
       }
     }
-    rc = dw_product(blas, c.y0, j.p.dx0, j.num_steps > 1 ? 1.f : 0.f, c.DW, B, n, x.dtype);
-    if (rc != RTN_OK) return rc;
+    if (!own && (rc = dw_product(blas, c.y0, j.p.dx0, j.num_steps > 1 ? 1.f : 0.f, c.DW, B, n, x.dtype)) != RTN_OK) return rc;
     if (!persistent) {
       if (x.dtype == RTN_DTYPE_BF16)
         hipLaunchKernelGGL(k_convert_from_f32<__bf16>, fill_grid, fill_block, 0, x.stream, j.p.dyw, c.Dy0, x.bn);
@@ -2692,7 +2767,7 @@ int bwd_calls(const rtn_lstm2_bwd_call* calls, int count, int64_t T, int32_t B, 
   if ((rc = bwd_prepare_jobs(x, ch, lay, workspace, stride, &jobs)) != RTN_OK) return rc;
   rc = ch.kernel ? bwd_launch_persistent(x, ch, lay, jobs) : bwd_launch_per_frame(x, mfma, lay, jobs[0]);  // (per frame: count == 1)
   if (rc != RTN_OK) return rc;
-  return bwd_weight_gradients(x, blas, jobs, ch.kernel != nullptr);
+  return bwd_weight_gradients(x, blas, lay, jobs, ch.kernel != nullptr);
 }
 
 }  // namespace

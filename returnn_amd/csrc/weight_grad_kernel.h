@@ -1,0 +1,135 @@
+// gfx950 kernels of the recurrent weight gradient: C = A^T B with few columns and very many rows.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include "lstm2_kernels.h"
+
+namespace rtn {
+
+// ---------------------------------------------------------------------------------------------------------------
+// DW[n,4n] = sum over frames and sequences of Y[row]^T DX[row], plus y0^T dx0: the matrices are [T B, n] and [T B, 4n].  For small
+// layers the product has a few tiles of output and ten thousands of rows, and a library product that gives a workgroup a tile leaves
+// most of the chip idle.  Here the rows are dealt to slices, a workgroup takes 64 x 64 of the output of one slice, and a second
+// kernel adds the slices' results; y0^T dx0 is one slice more.
+//
+// A and B are used as they lie: v_mfma_f32_16x16x4 takes ONE k per lane group, so lane (kg, i) needs row k + kg at column i, and with
+// four neighbouring columns per lane one load of 16 bytes (8 in bf16, widened: the products are exact) is the operand of four tiles, whose columns are then
+// 4 apart: tile t has columns 4 i + t.  Four rows are 2 loads for 16 MFMAs of 32 clocks, no LDS, no transposition.  The four wavefronts take
+// every fourth four rows and add their tiles through LDS.  A slice's workgroups are on one XCD (slice = id % slices), whose L2 they share.
+// Bound by the float32 matrix rate from n = 256 on (26 GFLOP at n = 256, T B = 49 750: 172 us at 152 TFLOP/s), below by the two launches.
+// Measured (gradient op with the recurrence, us, library / this): float32 n = 128, T = 300, B = 100 804 / 437, n = 256 937 / 662; bf16 n = 64 422 / 333,
+// n = 128 474 / 399, T = 20, B = 4 61 / 40.  Largest error against float64, of the largest element: float32 1.9e-7 ... 4.9e-7 / 0.9e-7 ... 1.5e-7,
+// bf16 inputs 0.9e-7 ... 6.9e-7 / 0.7e-7 ... 1.3e-7.
+// ---------------------------------------------------------------------------------------------------------------
+constexpr int kWeightTile = 64;       // columns of A and of B per workgroup
+constexpr int kWeightAhead = 4;       // steps of 16 rows whose loads are in flight together
+constexpr int kMaxWeightCalls = 2;
+struct WeightGradCall {
+  const void *a[2], *b[2];            // [rows][m], [rows][n]: the long product's and the other's
+  long long rows[2], lda[2], ldb[2];  // elements from one row to the next
+  float* part;                        // [slices + 1][m][n], or the result itself where there is one slice only
+  float* out;                         // [m][n]
+};
+struct WeightGradArgs {
+  int m, n;                           // multiples of 4
+  int slices;                         // of the long product
+  int parts;                          // slices, and one more for the other product
+  long long slice_rows;
+  WeightGradCall call[kMaxWeightCalls];
+};
+
+template <typename AT>
+__global__ __launch_bounds__(kWgThreads) void k_weight_grad(const WeightGradArgs args) {
+  constexpr int ES = (int)sizeof(AT);
+  typedef std::conditional_t<ES == 4, u32x4, u32x2> Quad4;  // four neighbouring elements
+  __shared__ f32x4 red[kWaves][16][64];
+  const WeightGradCall& q = args.call[blockIdx.y];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), kg = lane >> 4, i = lane & 15;
+  const int tiles_m = (args.m + kWeightTile - 1) / kWeightTile, tiles = tiles_m * ((args.n + kWeightTile - 1) / kWeightTile);
+  const bool other = (int)blockIdx.x >= tiles * args.slices;
+  const int which = other ? 1 : 0, slice = other ? 0 : (int)blockIdx.x % args.slices, tile = other ? (int)blockIdx.x - tiles * args.slices : (int)blockIdx.x / args.slices;
+  const int m0 = kWeightTile * (tile % tiles_m), n0 = kWeightTile * (tile / tiles_m);
+  const long long first = other ? 0 : slice * args.slice_rows;
+  const int rows = (int)max(0LL, min(other ? q.rows[1] : args.slice_rows, q.rows[which] - first));
+  const unsigned pitch_a = (unsigned)(q.lda[which] * ES), pitch_b = (unsigned)(q.ldb[which] * ES);
+  // (rows behind the slice lie behind the buffer, and so do lanes whose columns do not exist: zeros come back)
+  __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((unsigned char*)q.a[which] + first * q.lda[which] * ES, 0, rows > 0 ? (rows - 1) * pitch_a + args.m * ES : 0u, kBufFlags);
+  __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((unsigned char*)q.b[which] + first * q.ldb[which] * ES, 0, rows > 0 ? (rows - 1) * pitch_b + args.n * ES : 0u, kBufFlags);
+  unsigned at_a = m0 + 4 * i < args.m ? (4 * wave + kg) * pitch_a + (m0 + 4 * i) * ES : kOobOffset, at_b = n0 + 4 * i < args.n ? (4 * wave + kg) * pitch_b + (n0 + 4 * i) * ES : kOobOffset;
+  const unsigned step_a = 4 * kWaves * pitch_a, step_b = 4 * kWaves * pitch_b;
+  auto load = [](__amdgpu_buffer_rsrc_t rs, unsigned at) {
+    if constexpr (ES == 4)
+      return __builtin_bit_cast(Quad4, __builtin_amdgcn_raw_buffer_load_b128(rs, at, 0, 0));
+    else
+      return __builtin_bit_cast(Quad4, __builtin_amdgcn_raw_buffer_load_b64(rs, at, 0, 0));
+  };
+  auto element = [](Quad4 v, int k) {
+    if constexpr (ES == 4)
+      return __builtin_bit_cast(float, (unsigned)v[k]);
+    else
+      return __builtin_bit_cast(float, k & 1 ? v[k >> 1] & 0xFFFF0000u : v[k >> 1] << 16);
+  };
+  f32x4 acc[4][4];
+#pragma unroll
+  for (int a = 0; a < 4; ++a)
+#pragma unroll
+    for (int b = 0; b < 4; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+  Quad4 va[2][kWeightAhead], vb[2][kWeightAhead];
+  auto fetch = [&](auto set_tag) {
+    constexpr int S = decltype(set_tag)::value;
+#pragma unroll
+    for (int u = 0; u < kWeightAhead; ++u) {
+      va[S][u] = load(ra, at_a);
+      vb[S][u] = load(rb, at_b);
+      at_a += step_a;
+      at_b += step_b;
+    }
+  };
+  auto multiply = [&](auto set_tag) {
+    constexpr int S = decltype(set_tag)::value;
+#pragma unroll
+    for (int u = 0; u < kWeightAhead; ++u)
+#pragma unroll
+      for (int a = 0; a < 4; ++a)
+#pragma unroll
+        for (int b = 0; b < 4; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(element(va[S][u], a), element(vb[S][u], b), acc[a][b], 0, 0, 0);
+  };
+  constexpr int kRows = 4 * kWaves * kWeightAhead;
+  fetch(IntTag<0>{});
+  for (int r = 0; r < rows; r += 2 * kRows) {
+    fetch(IntTag<1>{});
+    multiply(IntTag<0>{});
+    fetch(IntTag<0>{});
+    multiply(IntTag<1>{});
+  }
+#pragma unroll
+  for (int a = 0; a < 4; ++a)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) red[wave][4 * a + r][lane] = f32x4{acc[a][0][r], acc[a][1][r], acc[a][2][r], acc[a][3][r]};
+  __syncthreads();
+  float* out = q.part + (size_t)(other ? args.slices : slice) * args.m * args.n;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {  // entry 4 a + r of a lane: row 4 (4 kg + r) + a of the tile, columns 4 i ... 4 i + 3
+    const int entry = 4 * wave + e, row = m0 + 4 * (4 * kg + (entry & 3)) + (entry >> 2), col = n0 + 4 * i;
+    const f32x4 sum = ((red[0][entry][lane] + red[1][entry][lane]) + red[2][entry][lane]) + red[3][entry][lane];
+    if (row < args.m && col < args.n) *(f32x4*)(out + (size_t)row * args.n + col) = sum;
+  }
+}
+
+// out := the sum of the parts, four elements per lane; the wavefronts take every fourth part.
+static __global__ __launch_bounds__(kWgThreads) void k_weight_grad_sum(const WeightGradArgs args) {
+  __shared__ f32x4 red[kWaves][64];
+  const WeightGradCall& q = args.call[blockIdx.y];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const long long quads = (long long)args.m * args.n / 4, at = blockIdx.x * 64LL + lane;
+  f32x4 sum = f32x4{0.f, 0.f, 0.f, 0.f};
+  if (at < quads)
+#pragma unroll 8
+    for (int s = wave; s < args.parts; s += kWaves) sum += ((const f32x4*)q.part)[s * quads + at];
+  red[wave][lane] = sum;
+  __syncthreads();
+  if (wave == 0 && at < quads) ((f32x4*)q.out)[at] = ((red[0][lane] + red[1][lane]) + red[2][lane]) + red[3][lane];
+}
+
+}  // namespace rtn

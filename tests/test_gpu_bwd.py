@@ -529,3 +529,33 @@ def test_bwd_padded_copies(dtype, B, n):
         for grads in torch_native_op.native_lstm2_grad_multi(calls):
             for name, a, b in zip(("DX", "DW", "Dy0", "Dc0"), grads, got):
                 assert _rel_to_max(a.float().cpu().numpy(), b) <= (1e-5 if dtype == "f32" else 2.0**-7), (T, name)
+
+
+# the weight gradient of small layers in slices of the rows: one slice and many, rows that leave a slice cut or empty, widths that cut a tile,
+# rows further apart than they are wide (two calls side by side), no frame but the first
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("T,B,n,count", [(1, 3, 32, 1), (2, 1, 64, 2), (9, 15, 4, 1), (40, 33, 100, 2), (130, 9, 68, 1), (65, 64, 256, 1), (30, 7, 192, 2), (300, 40, 36, 1), (64, 130, 384, 1)])
+def test_bwd_weight_gradient_of_small_layers(T, B, n, count, dtype):
+    """Against float64 products of what the op itself returned (dx0 is DX of the first visited frame where no frame is masked): the order of
+    additions is all that differs, so within a few float32 roundings of the sum of magnitudes (64 of them, for up to 12 000 terms in slices)."""
+    announce("bwd weight gradient", T, B, n, count, dtype)
+    X, W, y0, c0, i = random_problem(n + T, T, B, n)
+    i[:] = 1.0  # (no padding: dx0 is DX of the first frame)
+    rng = numpy.random.default_rng(T)
+    Xd, Wd, y0d = (to_dev(a, dtype) for a in (X, W, y0))
+    c0d, id_ = to_dev(c0, "f32"), to_dev(i, "f32")
+    op = get_op()
+    wide = to_dev(rng.normal(0, 1, (T, B, 2 * n)), dtype)
+    calls = []
+    for k in range(count):
+        Y, C, H, _ = op(Xd, Wd, y0d, c0d, id_, 0, 1 - 2 * k)
+        calls.append((Wd, y0d, c0d, id_, 0, 1 - 2 * k, Y, C, H, wide[..., k * n : (k + 1) * n], to_dev(rng.normal(0, 1, (B, n)), "f32")))
+    f = lambda t: t.float().cpu().numpy().astype(numpy.float64)  # noqa: E731
+    for call, (DX, DW, _, _) in zip(calls, torch_native_op.native_lstm2_grad_multi(calls)):
+        Y, DX = f(call[6]), f(DX)
+        if call[5] < 0:
+            Y, DX = Y[::-1], DX[::-1]
+        before = numpy.concatenate([f(y0d)[None], Y[:-1]]).reshape(T * B, n)
+        DX = DX.reshape(T * B, 4 * n)
+        bound = 64 * 2.0**-24 * (numpy.abs(before).T @ numpy.abs(DX)) + 1e-30
+        assert (numpy.abs(f(DW) - before.T @ DX) <= bound).all()
