@@ -386,6 +386,16 @@ int rtn_column_sums(const void* data, int64_t rows, int32_t width, int32_t dtype
 size_t rtn_column_sums_workspace_bytes(int64_t rows, int32_t width);
 
 /*
+ * out [m,n] (element type `out_dtype`, contiguous, 16-byte aligned) = A^T B of A [rows,m] (rows lda elements apart, m and lda multiples of 4,
+ * 16-byte aligned) and B [rows,n] (rows ldb elements apart), accumulated in float32: the gradient of a layer's input weights, few columns and
+ * many rows.  rtn_transposed_product_workspace_bytes() is 0 for products that are not taken, because a library's are faster there;
+ * the call then fails with RTN_ERR_SHAPE.  Two kernel launches.
+ */
+int rtn_transposed_product(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t rows, int32_t m, int32_t n, int32_t dtype, void* out,
+                           int32_t out_dtype, void* workspace, size_t workspace_bytes, void* hip_stream);
+size_t rtn_transposed_product_workspace_bytes(int64_t rows, int32_t m, int32_t n, int32_t dtype);
+
+/*
  * Where the calling thread's calls report an expired bounded wait, besides the status word of their workspace: a kernel
  * whose wait expires stores `id` into *word (a 32-bit word the device can write, e.g. of pinned host memory; null, the
  * initial setting: nowhere).  Holds for all later calls of this thread.  The word has to stay valid until their kernels

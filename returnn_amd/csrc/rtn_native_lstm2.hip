@@ -1597,15 +1597,35 @@ int gemm_row_major(rocblas_handle h, bool trans_a, bool trans_b, long long M, lo
   return RTN_OK;
 }
 
+int weight_tiles(int m, int n) { return (int)std::min<long long>((long long)((m + kWeightTile - 1LL) / kWeightTile) * ((n + kWeightTile - 1LL) / kWeightTile), 1 << 30); }
+// (two workgroups per CU in all; a multiple of the XCDs, which then have a slice's workgroups to themselves)
+int slices_of_tiles(int tiles) {
+  const int slices = std::max(1, 512 / std::max(tiles, 1));
+  return slices >= 8 ? slices / 8 * 8 : slices;
+}
+constexpr int kWeightRound = 2 * 4 * kWaves * kWeightAhead;  // rows of one round of k_weight_grad's loop
+
+// Slices for the product A^T B of [rows,m] and [rows,n]; 0: the library's product is the better one, or a slice is too long for 32-bit offsets.
+// A library's product gives few workgroups a long serial sum (us for 80, 2000, 30 000 rows, library / this, timed as calls: float32 1024 x 128
+// 20 / 8, 21 / 15, 193 / 72; 1024 x 256, 64 tiles, 21 / 8, 22 / 19, 376 / 130; 2048 x 256, 128 tiles, 21 / 9, 25 / 27, 387 / 245; 2048 x 400, 224
+// tiles, 21 / 10, 41 / 41, 420 / 484; bf16, which the library takes at 8 times the rate, 256 x 128 21 / 8, 23 / 10, 107 / 29; 1024 x 128, 32 tiles,
+// 21 / 8, 25 / 15, 109 / 76; 2048 x 128, 64 tiles, 21 / 9, 25 / 19, 108 / 137).
+int product_slices(long long rows, int m, int n, int dtype) {
+  if (rows <= 0 || m <= 0 || n <= 0 || m % 4 != 0) return 0;
+  const int tiles = weight_tiles(m, n);
+  if (tiles > (dtype == RTN_DTYPE_BF16 ? 32 : rows >= 8192 ? 128 : 64)) return 0;
+  const long long slices = std::min<long long>(slices_of_tiles(tiles), (rows + kWeightRound - 1) / kWeightRound);
+  if (((rows + slices - 1) / slices + 2 * kWeightRound) * std::max(m, n) * (long long)esize(dtype) >= (1LL << 30)) return 0;
+  return (int)slices;
+}
+
 // Slices of the rows that the weight gradient of a layer of width n is summed in at most (see weight_grad_kernel.h): two workgroups per CU
 // in all; 0: the product goes to the library, which with more tiles of output fills the chip itself (gradient op, us, library / this, for T B = 80, 2000, 30 000:
 // float32 n = 256 55 / 53, 189 / 187, 937 / 662, n = 384 72 / 73, 275 / 266, 1398 / 1292, n = 512 73 / 79, 289 / 291, 1415 / 1474; bf16, whose products the library takes at 8
 // times the rate, n = 192 60 / 43, 162 / 152, 538 / 514, n = 256 62 / 44, 165 / 162, 555 / 535, n = 320 63 / 50, 175 / 180, 675 / 758).
 int weight_grad_slices(int n, int dtype) {
   if (n % 4 != 0 || n < 4 || n > (dtype == RTN_DTYPE_BF16 ? 256 : 384)) return 0;
-  const int tiles = ((n + kWeightTile - 1) / kWeightTile) * ((4 * n + kWeightTile - 1) / kWeightTile);
-  const int slices = std::max(1, 512 / tiles);
-  return slices >= 8 ? slices / 8 * 8 : slices;
+  return slices_of_tiles(weight_tiles(n, 4 * n));
 }
 
 struct BwdLayout {
@@ -1782,7 +1802,7 @@ using namespace rtn;
 
 extern "C" {
 
-int rtn_native_lstm2_abi_version(void) { return 15; }
+int rtn_native_lstm2_abi_version(void) { return 16; }
 
 const char* rtn_native_lstm2_bwd_plan_text(void) { return g_bwd_plan_text.c_str(); }
 
@@ -2607,19 +2627,18 @@ int bwd_own_weight_gradients(const BwdCtx& x, const BwdLayout& lay, const std::v
     longest = std::max(longest, (j.num_steps - 1) * x.B);
     widest = std::max({widest, (long long)j.ldY, (long long)j.p.ldDX});
   }
-  constexpr int kRound = 2 * 4 * kWaves * kWeightAhead;  // rows of one round of the kernel's loop
   WeightGradArgs args;
   memset(&args, 0, sizeof(args));
   args.m = n;
   args.n = 4 * n;
-  args.slices = (int)std::max<long long>(1, std::min<long long>(max_slices, (longest + kRound - 1) / kRound));
+  args.slices = (int)std::max<long long>(1, std::min<long long>(max_slices, (longest + kWeightRound - 1) / kWeightRound));
   args.slice_rows = (std::max<long long>(longest, 1) + args.slices - 1) / args.slices;
   args.parts = args.slices + 1;
   // (float32 n = 320, 2000 rows: 251 us in the library, 257 here; 30 000 rows 1384 and 1154)
   if (n > 256 && longest < 8192) return RTN_OK;
   // (offsets inside a slice, with the rows asked for behind it, are 32 bits wide)
-  if ((std::max<long long>(args.slice_rows, x.B) + 2 * kRound) * widest * (long long)x.es >= (1LL << 30)) return RTN_OK;
-  const int tiles = ((args.m + kWeightTile - 1) / kWeightTile) * ((args.n + kWeightTile - 1) / kWeightTile);
+  if ((std::max<long long>(args.slice_rows, x.B) + 2 * kWeightRound) * widest * (long long)x.es >= (1LL << 30)) return RTN_OK;
+  const int tiles = weight_tiles(args.m, args.n);
   for (int k = 0; k < x.count; k += kMaxWeightCalls) {
     const int now = std::min(kMaxWeightCalls, x.count - k);
     for (int i = 0; i < now; ++i) {
@@ -2642,11 +2661,11 @@ int bwd_own_weight_gradients(const BwdCtx& x, const BwdLayout& lay, const std::v
     }
     const dim3 grid((unsigned)(tiles * args.parts), (unsigned)now), block(kWgThreads);
     if (x.dtype == RTN_DTYPE_BF16)
-      hipLaunchKernelGGL(k_weight_grad<__bf16>, grid, block, 0, x.stream, args);
+      hipLaunchKernelGGL((k_weight_grad<__bf16, false>), grid, block, 0, x.stream, args);
     else
-      hipLaunchKernelGGL(k_weight_grad<float>, grid, block, 0, x.stream, args);
+      hipLaunchKernelGGL((k_weight_grad<float, false>), grid, block, 0, x.stream, args);
     RTN_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_weight_grad_sum, dim3((unsigned)(((long long)args.m * args.n / 4 + 63) / 64), (unsigned)now), block, 0, x.stream, args);
+    hipLaunchKernelGGL(k_weight_grad_sum<float>, dim3((unsigned)(((long long)args.m * args.n / 4 + 63) / 64), (unsigned)now), block, 0, x.stream, args);
     RTN_HIP(hipGetLastError());
   }
   *done = true;
@@ -2972,6 +2991,60 @@ int rtn_column_sums(const void* data, int64_t rows, int32_t width, int32_t dtype
   if (need && (!workspace || workspace_bytes < need)) return fail(RTN_ERR_WORKSPACE, "column sums: workspace of %zu bytes needed", need);
   if (!aligned16(workspace)) return fail(RTN_ERR_ARG, "column sums: workspace must be 16-byte aligned");
   return column_sums(data, rows, width, dtype, out, out_dtype, workspace, (hipStream_t)hip_stream);
+}
+
+size_t rtn_transposed_product_workspace_bytes(int64_t rows, int32_t m, int32_t n, int32_t dtype) {
+  return (size_t)product_slices(rows, m, n, dtype) * (size_t)std::max(m, 0) * (size_t)std::max(n, 0) * 4;
+}
+
+int rtn_transposed_product(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t rows, int32_t m, int32_t n, int32_t dtype, void* out, int32_t out_dtype,
+                           void* workspace, size_t workspace_bytes, void* hip_stream) {
+  g_last_error.clear();
+  for (int t : {dtype, out_dtype})
+    if (t != RTN_DTYPE_F32 && t != RTN_DTYPE_BF16) return fail(RTN_ERR_ARG, "transposed product: unknown dtype %d", t);
+  const int slices = product_slices(rows, m, n, dtype);
+  if (!slices || lda < m || ldb < n || lda % 4 != 0) return fail(RTN_ERR_SHAPE, "transposed product: not taken: %lld rows, m=%d, n=%d, rows %lld and %lld apart", (long long)rows, m, n, (long long)lda, (long long)ldb);
+  if (!a || !b || !out) return fail(RTN_ERR_ARG, "transposed product: null pointer");
+  if (!aligned16(a) || !aligned16(out)) return fail(RTN_ERR_ARG, "transposed product: a and out must be 16-byte aligned");
+  const size_t need = rtn_transposed_product_workspace_bytes(rows, m, n, dtype);
+  if (!workspace || workspace_bytes < need) return fail(RTN_ERR_WORKSPACE, "transposed product: workspace of %zu bytes needed", need);
+  if (!aligned16(workspace)) return fail(RTN_ERR_ARG, "transposed product: workspace must be 16-byte aligned");
+  WeightGradArgs args;
+  memset(&args, 0, sizeof(args));
+  args.m = m;
+  args.n = n;
+  args.slices = args.parts = slices;
+  args.slice_rows = (rows + slices - 1) / slices;
+  if ((args.slice_rows + 2 * kWeightRound) * std::max(lda, ldb) * (long long)esize(dtype) >= (1LL << 30))
+    return fail(RTN_ERR_SHAPE, "transposed product: not taken: a slice of %lld rows, %lld and %lld apart", args.slice_rows, (long long)lda, (long long)ldb);
+  args.call[0].a[0] = a;
+  args.call[0].b[0] = b;
+  args.call[0].rows[0] = rows;
+  args.call[0].lda[0] = lda;
+  args.call[0].ldb[0] = ldb;
+  args.call[0].part = (float*)workspace;
+  args.call[0].out = out;
+  const bool any = n % 4 != 0 || ldb % 4 != 0 || !aligned16(b);
+  const hipStream_t stream = (hipStream_t)hip_stream;
+  const dim3 grid((unsigned)(weight_tiles(m, n) * slices)), block(kWgThreads), sums((unsigned)(((long long)m * n / 4 + 63) / 64));
+  if (dtype == RTN_DTYPE_BF16) {
+    if (any)
+      hipLaunchKernelGGL((k_weight_grad<__bf16, true>), grid, block, 0, stream, args);
+    else
+      hipLaunchKernelGGL((k_weight_grad<__bf16, false>), grid, block, 0, stream, args);
+  } else {
+    if (any)
+      hipLaunchKernelGGL((k_weight_grad<float, true>), grid, block, 0, stream, args);
+    else
+      hipLaunchKernelGGL((k_weight_grad<float, false>), grid, block, 0, stream, args);
+  }
+  RTN_HIP(hipGetLastError());
+  if (out_dtype == RTN_DTYPE_BF16)
+    hipLaunchKernelGGL(k_weight_grad_sum<__bf16>, sums, block, 0, stream, args);
+  else
+    hipLaunchKernelGGL(k_weight_grad_sum<float>, sums, block, 0, stream, args);
+  RTN_HIP(hipGetLastError());
+  return RTN_OK;
 }
 
 size_t rtn_native_lstm2_bwd_multi_workspace_bytes(int32_t count, int64_t T, int32_t B, int32_t n, int32_t dtype) {

@@ -39,6 +39,8 @@ struct Abi {
   decltype(&rtn_sequence_mask) sequence_mask;
   decltype(&rtn_column_sums) column_sums;
   decltype(&rtn_column_sums_workspace_bytes) column_sums_workspace_bytes;
+  decltype(&rtn_transposed_product) transposed_product;
+  decltype(&rtn_transposed_product_workspace_bytes) transposed_product_workspace_bytes;
 } rtn_abi;
 bool ready = false;
 
@@ -493,6 +495,21 @@ Tensor column_sums(const Tensor& m, at::ScalarType type) {
   return out;
 }
 
+// a^T b of [rows,m] and [rows,n].  (With gradients of gradients on, the product that autograd knows.)
+Tensor transposed_product(const Tensor& a, const Tensor& b) {
+  const int64_t rows = a.size(0), m = a.size(1), n = b.size(1);
+  const bool known = !at::GradMode::is_enabled() && (a.scalar_type() == at::kBFloat16 || a.scalar_type() == at::kFloat) && a.scalar_type() == b.scalar_type() && a.is_contiguous() && b.is_contiguous() &&
+                     rows > 0 && m < (1 << 20) && n < (1 << 20) && (uintptr_t)a.data_ptr() % 16 == 0;
+  const int dtype = a.scalar_type() == at::kBFloat16 ? RTN_DTYPE_BF16 : RTN_DTYPE_F32;
+  const size_t bytes = known ? rtn_abi.transposed_product_workspace_bytes(rows, (int)m, (int)n, dtype) : 0;
+  if (!bytes) return at::mm(a.t(), b);
+  c10::DeviceGuard guard(a.device());
+  const Tensor out = at::empty({m, n}, a.options()), ws = workspace(bytes, a);
+  check_rc(rtn_abi.transposed_product(a.data_ptr(), m, b.data_ptr(), n, rows, (int)m, (int)n, dtype, out.data_ptr(), dtype, ws.data_ptr(), (size_t)ws.numel(),
+                                      current_stream(a.device())));
+  return out;
+}
+
 // One direction: (W [n,4n], y0 [B,n], c0 [B,n], step).
 struct Direction {
   Tensor W, y0, c0;
@@ -616,7 +633,7 @@ struct LayerFunction : torch::autograd::Function<LayerFunction> {
     variable_list out(11);
     if (ctx->needs_input_grad(0)) out[0] = at::mm(DP, ff.t()).view(source.sizes());
     // (the gradient of ff comes out in the layout of a [4n,in] parameter, whose transposed view ff usually is)
-    if (ctx->needs_input_grad(1)) out[1] = at::mm(DP.t(), source.reshape({rows, source.size(2)})).t();
+    if (ctx->needs_input_grad(1)) out[1] = transposed_product(DP, source.reshape({rows, source.size(2)})).t();
     if (ctx->saved_data["bias"].toBool() && ctx->needs_input_grad(2)) {
       c10::DeviceGuard guard(DPo.device());
       out[2] = as_type(column_sums(DPo, ff.scalar_type() == DPo.scalar_type() ? DPo.scalar_type() : at::kFloat), ff.scalar_type());
@@ -716,6 +733,8 @@ void init(const py::dict& symbols, const py::object& aborted) {
   take(rtn_abi.sequence_mask, symbols, "rtn_sequence_mask");
   take(rtn_abi.column_sums, symbols, "rtn_column_sums");
   take(rtn_abi.column_sums_workspace_bytes, symbols, "rtn_column_sums_workspace_bytes");
+  take(rtn_abi.transposed_product, symbols, "rtn_transposed_product");
+  take(rtn_abi.transposed_product_workspace_bytes, symbols, "rtn_transposed_product_workspace_bytes");
   watch().exception = aborted;
   ready = true;
 }

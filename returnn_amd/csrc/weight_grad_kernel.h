@@ -1,4 +1,4 @@
-// gfx950 kernels of the recurrent weight gradient: C = A^T B with few columns and very many rows.
+// gfx950 kernels of the weight gradients: C = A^T B with few columns and very many rows.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -11,7 +11,7 @@ namespace rtn {
 // DW[n,4n] = sum over frames and sequences of Y[row]^T DX[row], plus y0^T dx0: the matrices are [T B, n] and [T B, 4n].  For small
 // layers the product has a few tiles of output and ten thousands of rows, and a library product that gives a workgroup a tile leaves
 // most of the chip idle.  Here the rows are dealt to slices, a workgroup takes 64 x 64 of the output of one slice, and a second
-// kernel adds the slices' results; y0^T dx0 is one slice more.
+// kernel adds the slices' results; y0^T dx0 is one slice more.  (The gradient of the input's weights, DX^T source, is such a product too.)
 //
 // A and B are used as they lie: v_mfma_f32_16x16x4 takes ONE k per lane group, so lane (kg, i) needs row k + kg at column i, and with
 // four neighbouring columns per lane one load of 16 bytes (8 in bf16, widened: the products are exact) is the operand of four tiles, whose columns are then
@@ -28,18 +28,19 @@ constexpr int kMaxWeightCalls = 2;
 struct WeightGradCall {
   const void *a[2], *b[2];            // [rows][m], [rows][n]: the long product's and the other's
   long long rows[2], lda[2], ldb[2];  // elements from one row to the next
-  float* part;                        // [slices + 1][m][n], or the result itself where there is one slice only
-  float* out;                         // [m][n]
+  float* part;                        // [parts][m][n]
+  void* out;                          // [m][n]
 };
 struct WeightGradArgs {
-  int m, n;                           // multiples of 4
+  int m, n;                           // m: a multiple of 4
   int slices;                         // of the long product
   int parts;                          // slices, and one more for the other product
   long long slice_rows;
   WeightGradCall call[kMaxWeightCalls];
 };
 
-template <typename AT>
+// ANY: n, and the distance between the rows of B, need not be multiples of 4: B comes in and the result goes out by element.
+template <typename AT, bool ANY>
 __global__ __launch_bounds__(kWgThreads) void k_weight_grad(const WeightGradArgs args) {
   constexpr int ES = (int)sizeof(AT);
   typedef std::conditional_t<ES == 4, u32x4, u32x2> Quad4;  // four neighbouring elements
@@ -56,6 +57,11 @@ __global__ __launch_bounds__(kWgThreads) void k_weight_grad(const WeightGradArgs
   // (rows behind the slice lie behind the buffer, and so do lanes whose columns do not exist: zeros come back)
   __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((unsigned char*)q.a[which] + first * q.lda[which] * ES, 0, rows > 0 ? (rows - 1) * pitch_a + args.m * ES : 0u, kBufFlags);
   __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((unsigned char*)q.b[which] + first * q.ldb[which] * ES, 0, rows > 0 ? (rows - 1) * pitch_b + args.n * ES : 0u, kBufFlags);
+  unsigned at_each[ANY ? 4 : 1];
+  if constexpr (ANY) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) at_each[k] = n0 + 4 * i + k < args.n ? (4 * wave + kg) * pitch_b + (n0 + 4 * i + k) * ES : kOobOffset;
+  }
   unsigned at_a = m0 + 4 * i < args.m ? (4 * wave + kg) * pitch_a + (m0 + 4 * i) * ES : kOobOffset, at_b = n0 + 4 * i < args.n ? (4 * wave + kg) * pitch_b + (n0 + 4 * i) * ES : kOobOffset;
   const unsigned step_a = 4 * kWaves * pitch_a, step_b = 4 * kWaves * pitch_b;
   auto load = [](__amdgpu_buffer_rsrc_t rs, unsigned at) {
@@ -75,15 +81,29 @@ __global__ __launch_bounds__(kWgThreads) void k_weight_grad(const WeightGradArgs
   for (int a = 0; a < 4; ++a)
 #pragma unroll
     for (int b = 0; b < 4; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-  Quad4 va[2][kWeightAhead], vb[2][kWeightAhead];
+  Quad4 va[2][kWeightAhead], vb[2][ANY ? 1 : kWeightAhead];
+  u32x4 each[2][ANY ? kWeightAhead : 1];  // (as the loads bring them)
   auto fetch = [&](auto set_tag) {
     constexpr int S = decltype(set_tag)::value;
 #pragma unroll
     for (int u = 0; u < kWeightAhead; ++u) {
       va[S][u] = load(ra, at_a);
-      vb[S][u] = load(rb, at_b);
+      if constexpr (ANY) {
+        unsigned v[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          if constexpr (ES == 4)
+            v[k] = __builtin_amdgcn_raw_buffer_load_b32(rb, at_each[k], 0, 0);
+          else
+            v[k] = __builtin_amdgcn_raw_buffer_load_b16(rb, at_each[k], 0, 0);
+          at_each[k] += step_b;
+        }
+        each[S][u] = u32x4{v[0], v[1], v[2], v[3]};
+      } else {
+        vb[S][u] = load(rb, at_b);
+        at_b += step_b;
+      }
       at_a += step_a;
-      at_b += step_b;
     }
   };
   auto multiply = [&](auto set_tag) {
@@ -93,7 +113,14 @@ __global__ __launch_bounds__(kWgThreads) void k_weight_grad(const WeightGradArgs
 #pragma unroll
       for (int a = 0; a < 4; ++a)
 #pragma unroll
-        for (int b = 0; b < 4; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(element(va[S][u], a), element(vb[S][u], b), acc[a][b], 0, 0, 0);
+        for (int b = 0; b < 4; ++b) {
+          float right;
+          if constexpr (ANY)
+            right = __builtin_bit_cast(float, ES == 4 ? (unsigned)each[S][u][b] : (unsigned)each[S][u][b] << 16);
+          else
+            right = element(vb[S][u], b);
+          acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(element(va[S][u], a), right, acc[a][b], 0, 0, 0);
+        }
   };
   constexpr int kRows = 4 * kWaves * kWeightAhead;
   fetch(IntTag<0>{});
@@ -113,12 +140,19 @@ __global__ __launch_bounds__(kWgThreads) void k_weight_grad(const WeightGradArgs
   for (int e = 0; e < 4; ++e) {  // entry 4 a + r of a lane: row 4 (4 kg + r) + a of the tile, columns 4 i ... 4 i + 3
     const int entry = 4 * wave + e, row = m0 + 4 * (4 * kg + (entry & 3)) + (entry >> 2), col = n0 + 4 * i;
     const f32x4 sum = ((red[0][entry][lane] + red[1][entry][lane]) + red[2][entry][lane]) + red[3][entry][lane];
-    if (row < args.m && col < args.n) *(f32x4*)(out + (size_t)row * args.n + col) = sum;
+    if constexpr (ANY) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if (row < args.m && col + k < args.n) out[(size_t)row * args.n + col + k] = sum[k];
+    } else {
+      if (row < args.m && col < args.n) *(f32x4*)(out + (size_t)row * args.n + col) = sum;
+    }
   }
 }
 
 // out := the sum of the parts, four elements per lane; the wavefronts take every fourth part.
-static __global__ __launch_bounds__(kWgThreads) void k_weight_grad_sum(const WeightGradArgs args) {
+template <typename OT>
+__global__ __launch_bounds__(kWgThreads) void k_weight_grad_sum(const WeightGradArgs args) {
   __shared__ f32x4 red[kWaves][64];
   const WeightGradCall& q = args.call[blockIdx.y];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
@@ -129,7 +163,15 @@ static __global__ __launch_bounds__(kWgThreads) void k_weight_grad_sum(const Wei
     for (int s = wave; s < args.parts; s += kWaves) sum += ((const f32x4*)q.part)[s * quads + at];
   red[wave][lane] = sum;
   __syncthreads();
-  if (wave == 0 && at < quads) ((f32x4*)q.out)[at] = ((red[0][lane] + red[1][lane]) + red[2][lane]) + red[3][lane];
+  if (wave == 0 && at < quads) {
+    const f32x4 all = ((red[0][lane] + red[1][lane]) + red[2][lane]) + red[3][lane];
+    if constexpr (sizeof(OT) == 4) {
+      ((f32x4*)q.out)[at] = all;
+    } else {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) Elem<OT>::store(q.out, 4 * at + k, all[k]);
+    }
+  }
 }
 
 }  // namespace rtn

@@ -31,7 +31,7 @@ MODE_PERSISTENT = 1
 MODE_GRAPH = 2
 MODE_STEPWISE = 3
 # The ABI version the structs and argument lists below were written for (rtn_native_lstm2_abi_version()).
-EXPECTED_ABI = 15
+EXPECTED_ABI = 16
 
 MODES = {"auto": MODE_AUTO, "persistent": MODE_PERSISTENT, "graph": MODE_GRAPH, "stepwise": MODE_STEPWISE}
 
@@ -64,6 +64,8 @@ SYMBOLS = (
     "rtn_sequence_mask",
     "rtn_column_sums",
     "rtn_column_sums_workspace_bytes",
+    "rtn_transposed_product",
+    "rtn_transposed_product_workspace_bytes",
     "rtn_set_abort_word",
     "rtn_last_error",
     "rtn_native_lstm2_describe_plan",
@@ -217,6 +219,10 @@ def load() -> ctypes.CDLL:
         lib.rtn_column_sums.argtypes = [vp, i64, i32, i32, vp, i32, vp, sz, vp]
         lib.rtn_column_sums_workspace_bytes.restype = sz
         lib.rtn_column_sums_workspace_bytes.argtypes = [i64, i32]
+        lib.rtn_transposed_product.restype = ctypes.c_int
+        lib.rtn_transposed_product.argtypes = [vp, i64, vp, i64, i64, i32, i32, i32, vp, i32, vp, sz, vp]
+        lib.rtn_transposed_product_workspace_bytes.restype = sz
+        lib.rtn_transposed_product_workspace_bytes.argtypes = [i64, i32, i32, i32]
         lib.rtn_set_abort_word.restype = None
         lib.rtn_set_abort_word.argtypes = [vp, ctypes.c_uint32]
         lib.rtn_last_error.restype = ctypes.c_char_p

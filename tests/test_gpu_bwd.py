@@ -559,3 +559,34 @@ def test_bwd_weight_gradient_of_small_layers(T, B, n, count, dtype):
         DX = DX.reshape(T * B, 4 * n)
         bound = 64 * 2.0**-24 * (numpy.abs(before).T @ numpy.abs(DX)) + 1e-30
         assert (numpy.abs(f(DW) - before.T @ DX) <= bound).all()
+
+
+# a^T b in slices of the rows: widths that cut a tile, odd ones and rows that are farther apart (by element), one row, a slice's edge, and
+# more rows than a round of every slice takes
+@pytest.mark.parametrize("rows,m,n", [(1, 4, 1), (127, 64, 64), (129, 68, 77), (700, 180, 45), (9001, 256, 40), (20000, 128, 3)])
+@pytest.mark.parametrize("dtype,out_dtype", [("f32", "f32"), ("bf16", "bf16"), ("bf16", "f32")])
+@pytest.mark.parametrize("pad", [0, 3])
+def test_transposed_product(rows, m, n, dtype, out_dtype, pad):
+    announce("transposed product", rows, m, n, dtype, out_dtype, pad)
+    code = {"f32": 0, "bf16": 1}
+    rng = numpy.random.default_rng(6)
+    a = to_dev(rng.normal(0, 1, (rows, m + 4 * pad)), dtype)
+    b = to_dev(rng.normal(0, 1, (rows, n + pad)), dtype)
+    out = torch.full((m, n), float("nan"), device="cuda", dtype=torch.float32 if out_dtype == "f32" else torch.bfloat16)
+    cabi = lib.load()
+    size = int(cabi.rtn_transposed_product_workspace_bytes(rows, m, n, code[dtype]))
+    assert size > 0
+    ws = torch.empty(size, dtype=torch.uint8, device="cuda")
+
+    def call(size=size, lda=m + 4 * pad):
+        return cabi.rtn_transposed_product(a.data_ptr(), lda, b.data_ptr(), n + pad, rows, m, n, code[dtype], out.data_ptr(), code[out_dtype], ws.data_ptr(), size, torch.cuda.current_stream().cuda_stream)
+
+    assert call(size - 1) == lib.RTN_ERR_WORKSPACE and call(lda=m + 2) == lib.RTN_ERR_SHAPE
+    lib.check(call())
+    wide = a[:, :m].cpu().double(), b[:, :n].cpu().double()
+    want, size_of_terms = wide[0].t() @ wide[1], wide[0].abs().t() @ wide[1].abs()
+    # float32 sums of `rows` terms in any order, then the rounding of the result
+    bound = size_of_terms * (rows + 8) * 2.0**-24 + want.abs() * (2.0**-8 if out_dtype == "bf16" else 2.0**-23) + 1e-30
+    assert bool(((out.cpu().double() - want).abs() <= bound).all())
+    assert int(cabi.rtn_transposed_product_workspace_bytes(rows, m + 2, n, code[dtype])) == 0  # (not whole quads)
+    assert int(cabi.rtn_transposed_product_workspace_bytes(rows, 4096, 4096, code[dtype])) == 0  # (the library's)
