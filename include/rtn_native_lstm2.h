@@ -281,6 +281,9 @@ typedef struct rtn_lstm2_bwd_call {
   int64_t ldY;
   int64_t ldDY;
   int64_t ldDX;
+  /* DW in the element type `dtype` (16-byte aligned), or null.  If given, this is the result and DW, which is needed all the same, holds sums on
+   * their way. */
+  void* DW_act;
 } rtn_lstm2_bwd_call;
 
 int rtn_native_lstm2_bwd_multi(const rtn_lstm2_bwd_call* calls, int32_t count, int64_t T, int32_t B, int32_t n,

@@ -1802,7 +1802,7 @@ using namespace rtn;
 
 extern "C" {
 
-int rtn_native_lstm2_abi_version(void) { return 16; }
+int rtn_native_lstm2_abi_version(void) { return 17; }
 
 const char* rtn_native_lstm2_bwd_plan_text(void) { return g_bwd_plan_text.c_str(); }
 
@@ -2165,6 +2165,7 @@ int bwd_check(const BwdCtx& x) {
       const rtn_lstm2_bwd_call& c = x.calls[k];
       if (nn4 > 0) {
         hipLaunchKernelGGL(k_fill_u32, fill_grid, fill_block, 0, x.stream, (unsigned*)c.DW, 0u, nn4);
+        if (c.DW_act) hipLaunchKernelGGL(k_fill_u32, fill_grid, fill_block, 0, x.stream, (unsigned*)c.DW_act, 0u, nn4 * (long long)x.es / 4);
         RTN_HIP(hipGetLastError());
       }
       if (x.bn > 0) {
@@ -2188,7 +2189,19 @@ int bwd_check(const BwdCtx& x) {
       // a multiple of 4n elements, which is aligned then)
       if (q != 3 && !(q == 0 && x.n % 16 != 0) && !aligned16(ptrs[q])) return fail(RTN_ERR_ARG, "NativeLstm2 backward: %s must be 16-byte aligned", names[q]);
     }
+    if (c.DW_act && !aligned16(c.DW_act)) return fail(RTN_ERR_ARG, "NativeLstm2 backward: DW_act must be 16-byte aligned");
   }
+  return RTN_OK;
+}
+
+// DW_act := DW in the op's element type.
+int bwd_convert_weights(const BwdCtx& x, const rtn_lstm2_bwd_call& c) {
+  const long long nn4 = (long long)x.n * x.n * 4;
+  if (x.dtype == RTN_DTYPE_BF16)
+    hipLaunchKernelGGL(k_convert_from_f32<__bf16>, dim3(512), dim3(256), 0, x.stream, (const float*)c.DW, c.DW_act, nn4);
+  else
+    hipLaunchKernelGGL(k_convert_from_f32<float>, dim3(512), dim3(256), 0, x.stream, (const float*)c.DW, c.DW_act, nn4);
+  RTN_HIP(hipGetLastError());
   return RTN_OK;
 }
 
@@ -2225,7 +2238,7 @@ int bwd_padded(const BwdCtx& x, int np, void* workspace, size_t workspace_bytes)
     padded[(size_t)k] = {base + L.W, base + L.y0, (const float*)(base + L.c0), c.i, c.start, c.step, base + L.Y,
                          (const float*)(base + ((x.op_flags & kOpH0IsCell) ? L.H : L.C)), base + L.H, base + L.DY,
                          (const float*)(base + L.Dd), base + L.DX, (float*)(base + L.DW), base + L.Dy0, (float*)(base + L.Dc0),
-                         0, 0, 0};
+                         0, 0, 0, nullptr};
   }
   if ((rc = pads.launch()) != RTN_OK) return rc;
   rc = bwd_calls(padded.data(), x.count, x.T, B, np, x.dtype, workspace, need, (void*)x.stream, x.op_flags, each);
@@ -2238,7 +2251,10 @@ int bwd_padded(const BwdCtx& x, int np, void* workspace, size_t workspace_bytes)
         (rc = out(q.Dc0, c.Dc0, B, 1, 4)) != RTN_OK)
       return rc;
   }
-  return pads.launch();
+  if ((rc = pads.launch()) != RTN_OK) return rc;
+  for (int k = 0; k < x.count; ++k)
+    if (x.calls[k].DW_act && (rc = bwd_convert_weights(x, x.calls[k])) != RTN_OK) return rc;
+  return RTN_OK;
 }
 
 // Persistent kernel: W in registers for the whole call, if a wavefront's share of the 16 x 4n slice fits (2..32
@@ -2613,6 +2629,13 @@ int bwd_launch_per_frame(const BwdCtx& x, bool mfma, const BwdLayout& lay, BwdJo
   return replay_graph(key, &p, sizeof(p), stream, record);
 }
 
+// Whether all calls want their weight gradient in one type.
+bool same_weight_type(const BwdCtx& x) {
+  for (int k = 1; k < x.count; ++k)
+    if (!x.calls[k].DW_act != !x.calls[0].DW_act) return false;
+  return true;
+}
+
 // The weight gradients of x's calls by k_weight_grad, as many calls per launch as it takes; *done: whether it does (layers for which the
 // library's products leave most of the chip idle; consecutive frames; rows a multiple of four elements apart).
 int bwd_own_weight_gradients(const BwdCtx& x, const BwdLayout& lay, const std::vector<BwdJob>& jobs, bool* done) {
@@ -2639,8 +2662,10 @@ int bwd_own_weight_gradients(const BwdCtx& x, const BwdLayout& lay, const std::v
   // (offsets inside a slice, with the rows asked for behind it, are 32 bits wide)
   if ((std::max<long long>(args.slice_rows, x.B) + 2 * kWeightRound) * widest * (long long)x.es >= (1LL << 30)) return RTN_OK;
   const int tiles = weight_tiles(args.m, args.n);
-  for (int k = 0; k < x.count; k += kMaxWeightCalls) {
-    const int now = std::min(kMaxWeightCalls, x.count - k);
+  const bool same = same_weight_type(x);
+  for (int k = 0; k < x.count; k += same ? kMaxWeightCalls : 1) {
+    const int now = same ? std::min(kMaxWeightCalls, x.count - k) : 1;
+    int acts = 0;
     for (int i = 0; i < now; ++i) {
       const rtn_lstm2_bwd_call& c = x.calls[k + i];
       const BwdJob& j = jobs[(size_t)(k + i)];
@@ -2657,7 +2682,8 @@ int bwd_own_weight_gradients(const BwdCtx& x, const BwdLayout& lay, const std::v
       q.lda[1] = n;
       q.ldb[1] = 4 * n;
       q.part = (float*)(j.ws + lay.off_part);
-      q.out = c.DW;
+      q.out = c.DW_act ? c.DW_act : (void*)c.DW;
+      acts += c.DW_act != nullptr;
     }
     const dim3 grid((unsigned)(tiles * args.parts), (unsigned)now), block(kWgThreads);
     if (x.dtype == RTN_DTYPE_BF16)
@@ -2665,7 +2691,56 @@ int bwd_own_weight_gradients(const BwdCtx& x, const BwdLayout& lay, const std::v
     else
       hipLaunchKernelGGL((k_weight_grad<float, false>), grid, block, 0, x.stream, args);
     RTN_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_weight_grad_sum<float>, dim3((unsigned)(((long long)args.m * args.n / 4 + 63) / 64), (unsigned)now), block, 0, x.stream, args);
+    const dim3 sums((unsigned)(((long long)args.m * args.n / 4 + 63) / 64), (unsigned)now);
+    if (acts && x.dtype == RTN_DTYPE_BF16)
+      hipLaunchKernelGGL(k_weight_grad_sum<__bf16>, sums, block, 0, x.stream, args);
+    else
+      hipLaunchKernelGGL(k_weight_grad_sum<float>, sums, block, 0, x.stream, args);
+    RTN_HIP(hipGetLastError());
+  }
+  *done = true;
+  return RTN_OK;
+}
+
+// The share y0^T dx0 of the weight gradients, added to DW (where there is anything yet), and DW in the wanted type, for as many calls per launch as the
+// kernel takes; *done: whether it does.  (Few rows: the float32 product then hides behind the pass over DW.  Training steps, us, library product and
+// conversion / this: bf16 one layer n = 2048, B = 64 1288 / 1266, B = 16 670 / 642, n = 1024, B = 128 732 / 726, B = 250 689 / 688, three bidirectional
+// layers n = 512, B = 32 870 / 829, n = 1024 2290 / 2237; float32 three of n = 500, B = 40 2195 / 2179, one n = 512, B = 128 649 / 651.)
+int bwd_last_weight_gradients(const BwdCtx& x, const std::vector<BwdJob>& jobs, bool* done) {
+  const int n = x.n;
+  *done = false;
+  if (n % 4 != 0 || x.B > (x.dtype == RTN_DTYPE_BF16 ? 128 : 64)) return RTN_OK;
+  WeightGradArgs args;
+  memset(&args, 0, sizeof(args));
+  args.m = n;
+  args.n = 4 * n;
+  args.slices = args.parts = 1;
+  args.slice_rows = x.B;
+  const bool same = same_weight_type(x);
+  for (int k = 0; k < x.count; k += same ? kMaxWeightCalls : 1) {
+    const int now = same ? std::min(kMaxWeightCalls, x.count - k) : 1;
+    int acts = 0;
+    for (int i = 0; i < now; ++i) {
+      const rtn_lstm2_bwd_call& c = x.calls[k + i];
+      const BwdJob& j = jobs[(size_t)(k + i)];
+      WeightGradCall& q = args.call[i];
+      q.a[0] = c.y0;
+      q.b[0] = j.p.dx0;
+      q.rows[0] = x.B;
+      q.lda[0] = n;
+      q.ldb[0] = 4 * n;
+      q.part = c.DW;
+      q.out = c.DW_act ? c.DW_act : (void*)c.DW;
+      q.add = j.num_steps > 1;
+      acts += c.DW_act != nullptr;
+    }
+    const dim3 grid((unsigned)weight_tiles(args.m, args.n), (unsigned)now), block(kWgThreads);
+    if (x.dtype != RTN_DTYPE_BF16)
+      hipLaunchKernelGGL((k_weight_grad<float, false, float>), grid, block, 0, x.stream, args);
+    else if (acts)
+      hipLaunchKernelGGL((k_weight_grad<__bf16, false, __bf16>), grid, block, 0, x.stream, args);
+    else
+      hipLaunchKernelGGL((k_weight_grad<__bf16, false, float>), grid, block, 0, x.stream, args);
     RTN_HIP(hipGetLastError());
   }
   *done = true;
@@ -2700,7 +2775,6 @@ int bwd_weight_gradients(const BwdCtx& x, rocblas_handle blas, const BwdLayout& 
         }
       }
     }
-    if (!own && (rc = dw_product(blas, c.y0, j.p.dx0, j.num_steps > 1 ? 1.f : 0.f, c.DW, B, n, x.dtype)) != RTN_OK) return rc;
     if (!persistent) {
       if (x.dtype == RTN_DTYPE_BF16)
         hipLaunchKernelGGL(k_convert_from_f32<__bf16>, fill_grid, fill_block, 0, x.stream, j.p.dyw, c.Dy0, x.bn);
@@ -2708,6 +2782,14 @@ int bwd_weight_gradients(const BwdCtx& x, rocblas_handle blas, const BwdLayout& 
         hipLaunchKernelGGL(k_convert_from_f32<float>, fill_grid, fill_block, 0, x.stream, j.p.dyw, c.Dy0, x.bn);
       RTN_HIP(hipGetLastError());
     }
+  }
+  bool last = own;
+  if (!own && (rc = bwd_last_weight_gradients(x, jobs, &last)) != RTN_OK) return rc;
+  for (int k = 0; k < x.count && !last; ++k) {
+    const rtn_lstm2_bwd_call& c = x.calls[k];
+    const BwdJob& j = jobs[(size_t)k];
+    if ((rc = dw_product(blas, c.y0, j.p.dx0, j.num_steps > 1 ? 1.f : 0.f, c.DW, B, n, x.dtype)) != RTN_OK) return rc;
+    if (c.DW_act && (rc = bwd_convert_weights(x, c)) != RTN_OK) return rc;
   }
   return RTN_OK;
 }

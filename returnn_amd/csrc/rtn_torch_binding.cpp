@@ -421,8 +421,8 @@ BwdArgs bwd_args(const Tensor& W, const Tensor& y0, const Tensor& c0, const Tens
   return a;
 }
 
-// (DX, DW, Dy0, Dc0) per call; `joint`: their DX side by side in one [T,B,count*4n] array.
-std::pair<std::vector<Out4>, Tensor> lstm2_grad_multi(const std::vector<BwdArgs>& args, bool joint) {
+// (DX, DW, Dy0, Dc0) per call; `joint`: their DX side by side in one [T,B,count*4n] array; `own_type`: DW in the op's type.
+std::pair<std::vector<Out4>, Tensor> lstm2_grad_multi(const std::vector<BwdArgs>& args, bool joint, bool own_type = false) {
   TORCH_CHECK(ready, "NativeLstm2: the library is not loaded");
   const BwdArgs& f = args[0];
   for (const BwdArgs& a : args)
@@ -437,15 +437,23 @@ std::pair<std::vector<Out4>, Tensor> lstm2_grad_multi(const std::vector<BwdArgs>
   Tensor DXj;
   if (joint && (4 * f.n * f.Y.element_size()) % 16 == 0) DXj = at::empty({f.T, f.B, count * 4 * f.n}, act);  // (else: separate arrays, joined below)
   std::vector<Out4> outs;
+  std::vector<Tensor> sums;  // (DW on its way)
   std::vector<rtn_lstm2_bwd_call> calls(count);
   for (int k = 0; k < count; ++k) {
     const BwdArgs& a = args[k];
     Tensor DX = DXj.defined() ? DXj.slice(2, k * 4 * f.n, (k + 1) * 4 * f.n) : at::empty({f.T, f.B, 4 * f.n}, act);
     outs.emplace_back(DX, at::empty({f.n, 4 * f.n}, f32), at::empty({f.B, f.n}, act), at::empty({f.B, f.n}, f32));
-    const Out4& o = outs.back();
+    Out4& o = outs.back();
+    void* DW_act = nullptr;
+    const Tensor DW = std::get<1>(o);
+    if (own_type && f.bf16) {
+      sums.push_back(DW);
+      std::get<1>(o) = at::empty({f.n, 4 * f.n}, act);
+      DW_act = std::get<1>(o).data_ptr();
+    }
     calls[k] = {a.W.data_ptr(), a.y0.data_ptr(), a.c0.data_ptr<float>(), a.i.data_ptr<float>(), (int)a.start, (int)a.step, a.Y.data_ptr(), a.C.data_ptr<float>(),
-                a.H.data_ptr(), a.DY.data_ptr(), a.Dd.data_ptr<float>(), DX.data_ptr(), std::get<1>(o).data_ptr<float>(), std::get<2>(o).data_ptr(),
-                std::get<3>(o).data_ptr<float>(), a.ldY, a.ldDY, DXj.defined() ? count * 4 * f.n : 0};
+                a.H.data_ptr(), a.DY.data_ptr(), a.Dd.data_ptr<float>(), DX.data_ptr(), DW.data_ptr<float>(), std::get<2>(o).data_ptr(),
+                std::get<3>(o).data_ptr<float>(), a.ldY, a.ldDY, DXj.defined() ? count * 4 * f.n : 0, DW_act};
   }
   const Tensor ws = workspace(rtn_abi.bwd_multi_workspace_bytes(count, f.T, (int)f.B, (int)f.n, dtype), f.Y);
   check_rc(rtn_abi.bwd_multi(calls.data(), count, f.T, (int)f.B, (int)f.n, dtype, ws.data_ptr(), (size_t)ws.numel(), stream));
@@ -627,7 +635,9 @@ struct LayerFunction : torch::autograd::Function<LayerFunction> {
       args.push_back(bwd_args(s[0], s[1], s[2], mask, 0, k ? -step0 : step0, half(Y), s[3], s[4], half(DY),
                               grads[1 + k].defined() ? grads[1 + k] : at::zeros_like(s[2], s[2].options().dtype(at::kFloat))));
     }
-    auto res = lstm2_grad_multi(args, true);
+    bool own_type = true;  // (the weights have the op's type)
+    for (int k = 0; k < count; ++k) own_type = own_type && saved[4 + 5 * k].scalar_type() == Y.scalar_type();
+    auto res = lstm2_grad_multi(args, true, own_type);
     const int64_t rows = source.size(0) * source.size(1);
     const Tensor DPo = res.second.view({rows, ff.size(1)}), DP = as_type(DPo, ff.scalar_type());  // (the error of a projection of another type than the op's)
     variable_list out(11);

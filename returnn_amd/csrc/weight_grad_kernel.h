@@ -30,6 +30,7 @@ struct WeightGradCall {
   long long rows[2], lda[2], ldb[2];  // elements from one row to the next
   float* part;                        // [parts][m][n]
   void* out;                          // [m][n]
+  int add;                            // OT: out = part + A^T B
 };
 struct WeightGradArgs {
   int m, n;                           // m: a multiple of 4
@@ -40,7 +41,10 @@ struct WeightGradArgs {
 };
 
 // ANY: n, and the distance between the rows of B, need not be multiples of 4: B comes in and the result goes out by element.
-template <typename AT, bool ANY>
+// OT (one short product, slices = parts = 1): out = A^T B in that type, plus what is in part if the call says so: the last frame's share y0^T dx0
+// of a wide layer's gradient, whose long product is the library's, and the conversion to the parameter's type in one pass over DW for all
+// directions.  Bound by that pass.
+template <typename AT, bool ANY, typename OT = void>
 __global__ __launch_bounds__(kWgThreads) void k_weight_grad(const WeightGradArgs args) {
   constexpr int ES = (int)sizeof(AT);
   typedef std::conditional_t<ES == 4, u32x4, u32x2> Quad4;  // four neighbouring elements
@@ -123,12 +127,29 @@ __global__ __launch_bounds__(kWgThreads) void k_weight_grad(const WeightGradArgs
         }
   };
   constexpr int kRows = 4 * kWaves * kWeightAhead;
+  constexpr bool LAST = !std::is_void_v<OT>;
+  // entry 4 a + r of a lane: row 4 (4 kg + r) + a of the tile, columns 4 i ... 4 i + 3
+  auto row_of = [&](int entry) { return m0 + 4 * (4 * kg + (entry & 3)) + (entry >> 2); };
+  const int col = n0 + 4 * i;
+  f32x4 before[4];
   fetch(IntTag<0>{});
-  for (int r = 0; r < rows; r += 2 * kRows) {
-    fetch(IntTag<1>{});
-    multiply(IntTag<0>{});
-    fetch(IntTag<0>{});
-    multiply(IntTag<1>{});
+  if constexpr (LAST) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {  // (on their way during the product)
+      const int row = row_of(4 * wave + e);
+      before[e] = q.add && row < args.m && col < args.n ? *(const f32x4*)(q.part + (size_t)row * args.n + col) : f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    for (int r = 0; r < rows; r += kRows) {
+      multiply(IntTag<0>{});
+      if (r + kRows < rows) fetch(IntTag<0>{});
+    }
+  } else {
+    for (int r = 0; r < rows; r += 2 * kRows) {
+      fetch(IntTag<1>{});
+      multiply(IntTag<0>{});
+      fetch(IntTag<0>{});
+      multiply(IntTag<1>{});
+    }
   }
 #pragma unroll
   for (int a = 0; a < 4; ++a)
@@ -137,10 +158,22 @@ __global__ __launch_bounds__(kWgThreads) void k_weight_grad(const WeightGradArgs
   __syncthreads();
   float* out = q.part + (size_t)(other ? args.slices : slice) * args.m * args.n;
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {  // entry 4 a + r of a lane: row 4 (4 kg + r) + a of the tile, columns 4 i ... 4 i + 3
-    const int entry = 4 * wave + e, row = m0 + 4 * (4 * kg + (entry & 3)) + (entry >> 2), col = n0 + 4 * i;
+  for (int e = 0; e < 4; ++e) {
+    const int entry = 4 * wave + e, row = row_of(entry);
     const f32x4 sum = ((red[0][entry][lane] + red[1][entry][lane]) + red[2][entry][lane]) + red[3][entry][lane];
-    if constexpr (ANY) {
+    if constexpr (LAST) {
+      static_assert(!ANY);
+      if (row < args.m && col < args.n) {
+        const f32x4 all = before[e] + sum;
+        const size_t at = (size_t)row * args.n + col;
+        if constexpr (std::is_same_v<OT, float>) {
+          *(f32x4*)((float*)q.out + at) = all;
+        } else {
+          typedef OT Out4v __attribute__((ext_vector_type(4)));
+          *(Out4v*)((OT*)q.out + at) = __builtin_convertvector(all, Out4v);
+        }
+      }
+    } else if constexpr (ANY) {
 #pragma unroll
       for (int k = 0; k < 4; ++k)
         if (row < args.m && col + k < args.n) out[(size_t)row * args.n + col + k] = sum[k];

@@ -31,7 +31,7 @@ MODE_PERSISTENT = 1
 MODE_GRAPH = 2
 MODE_STEPWISE = 3
 # The ABI version the structs and argument lists below were written for (rtn_native_lstm2_abi_version()).
-EXPECTED_ABI = 16
+EXPECTED_ABI = 17
 
 MODES = {"auto": MODE_AUTO, "persistent": MODE_PERSISTENT, "graph": MODE_GRAPH, "stepwise": MODE_STEPWISE}
 
@@ -121,6 +121,7 @@ class Lstm2BwdCall(ctypes.Structure):
         ("ldY", ctypes.c_int64),  # row pitch of Y in elements, 0 = contiguous (n)
         ("ldDY", ctypes.c_int64),  # row pitch of DY in elements, 0 = contiguous (n)
         ("ldDX", ctypes.c_int64),  # row pitch of DX in elements, 0 = contiguous (4n)
+        ("DW_act", ctypes.c_void_p),  # DW in the op's element type, or null
     ]
 
 

@@ -590,3 +590,44 @@ def test_transposed_product(rows, m, n, dtype, out_dtype, pad):
     assert bool(((out.cpu().double() - want).abs() <= bound).all())
     assert int(cabi.rtn_transposed_product_workspace_bytes(rows, m + 2, n, code[dtype])) == 0  # (not whole quads)
     assert int(cabi.rtn_transposed_product_workspace_bytes(rows, 4096, 4096, code[dtype])) == 0  # (the library's)
+
+
+# The weight gradient in the op's type: own kernel (n = 64), last share in a pass of its own (few rows; tiles of the output cut, no long product
+# with one frame), library and conversion (many rows, also every second frame), padded copies (n = 45); one of the two calls only: a launch each.
+@pytest.mark.parametrize("T,B,n,step", [(7, 5, 64, 1), (6, 5, 420, 1), (1, 3, 512, 1), (9, 64, 1024, -1), (5, 130, 512, 1), (7, 4, 512, 2), (5, 3, 45, 1)])
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("wanted", [(True, True), (False, True)])
+def test_bwd_weight_gradient_in_the_ops_type(T, B, n, step, dtype, wanted):
+    announce("bwd weight gradient type", T, B, n, step, dtype, wanted)
+    cabi = lib.load()
+    act, code = (torch.bfloat16, lib.DTYPE_BF16) if dtype == "bf16" else (torch.float32, lib.DTYPE_F32)
+    op = get_op()
+    arr, keep = (lib.Lstm2BwdCall * 2)(), []
+    for k in range(2):
+        X, W, y0, c0, i = random_problem(700 + k, T, B, n)
+        args = [to_dev(X, dtype), to_dev(W, dtype), to_dev(y0, dtype), to_dev(c0, "f32"), to_dev(i, "f32")]
+        s = step if k == 0 else -step
+        Y, C, H, _ = op(*args, 0, s)
+        rng = numpy.random.default_rng(60 + k)
+        DY, Dd = to_dev(rng.normal(0, 1, (T, B, n)), dtype), to_dev(rng.normal(0, 1, (B, n)), "f32")
+        DX = torch.empty((T, B, 4 * n), dtype=act, device="cuda")
+        DW = torch.full((n, 4 * n), float("nan"), device="cuda")
+        DW_act = torch.full((n, 4 * n), float("nan"), device="cuda", dtype=act) if wanted[k] else None
+        Dy0, Dc0 = torch.empty((B, n), dtype=act, device="cuda"), torch.empty((B, n), device="cuda")
+        arr[k] = lib.Lstm2BwdCall(*[a.data_ptr() for a in args[1:]], 0, s, Y.data_ptr(), C.data_ptr(), H.data_ptr(), DY.data_ptr(), Dd.data_ptr(), DX.data_ptr(),
+                                  DW.data_ptr(), Dy0.data_ptr(), Dc0.data_ptr(), 0, 0, 0, DW_act.data_ptr() if wanted[k] else None)  # fmt: skip
+        g = lambda t: t.float().cpu().numpy().astype(numpy.float64)  # noqa: E731
+        want = oracle.native_lstm2_bwd(g(args[0]), g(args[1]), g(args[2]), c0, i, 0, s, g(Y), g(C), g(H), g(DY), g(Dd), dtype=numpy.float64)[1]
+        keep.append((args, Y, C, H, DY, Dd, DX, DW, DW_act, Dy0, Dc0, want))
+    ws = torch.empty(int(cabi.rtn_native_lstm2_bwd_multi_workspace_bytes(2, T, B, n, code)), dtype=torch.uint8, device="cuda")
+    lib.check(cabi.rtn_native_lstm2_bwd_multi(arr, 2, T, B, n, code, ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream))
+    for k in range(2):
+        got, want = keep[k][8] if wanted[k] else keep[k][7], keep[k][11]
+        scale = float(numpy.abs(want).max())
+        # (the bounds of the gradient tests above; the result itself rounds to 2^-9 of its size)
+        assert float(numpy.abs(got.float().cpu().numpy() - want).max()) <= scale * (2e-2 if dtype == "bf16" else 2e-5)
+        if wanted[k] and dtype == "f32":
+            assert got.dtype == torch.float32
+    if wanted[0]:
+        arr[0].DW_act += 4
+        assert cabi.rtn_native_lstm2_bwd_multi(arr, 2, T, B, n, code, ws.data_ptr(), ws.numel(), None) == lib.RTN_ERR_ARG
