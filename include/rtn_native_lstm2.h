@@ -284,6 +284,8 @@ typedef struct rtn_lstm2_bwd_call {
   /* DW in the element type `dtype` (16-byte aligned), or null.  If given, this is the result and DW, which is needed all the same, holds sums on
    * their way. */
   void* DW_act;
+  /* Not 0: there is no error on the final cell state; Dd is not read and may be null. */
+  int32_t Dd_is_zero;
 } rtn_lstm2_bwd_call;
 
 int rtn_native_lstm2_bwd_multi(const rtn_lstm2_bwd_call* calls, int32_t count, int64_t T, int32_t B, int32_t n,

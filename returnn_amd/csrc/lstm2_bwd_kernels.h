@@ -271,11 +271,13 @@ __global__ void k_bwd_gemm_dy_generic(Lstm2BwdParams p, long long t) {
   p.dyw[idx] = acc;
 }
 
-// float32 -> AT copy (the final Dy0).
+// float32 -> AT copy (the final Dy0, a weight gradient), four elements per lane; both 16-byte aligned.
 template <typename AT>
 __global__ void k_convert_from_f32(const float* src, void* dst, long long count) {
-  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < count; i += (long long)gridDim.x * blockDim.x)
-    Elem<AT>::store(dst, i, src[i]);
+  typedef AT Four __attribute__((ext_vector_type(4)));
+  const long long first = blockIdx.x * (long long)blockDim.x + threadIdx.x, step = (long long)gridDim.x * blockDim.x;
+  for (long long i = first; i < count / 4; i += step) ((Four*)dst)[i] = __builtin_convertvector(((const f32x4*)src)[i], Four);
+  for (long long i = count / 4 * 4 + first; i < count; i += step) Elem<AT>::store(dst, i, src[i]);
 }
 
 
@@ -304,7 +306,7 @@ __global__ void k_convert_from_f32(const float* src, void* dst, long long count)
 //  * all waits are bounded as in the forward kernel (status[0] = 1, everybody leaves).
 struct Lstm2BwdPersistent {
   Lstm2BwdParams p;
-  const float* Dd;    // [B,n]
+  const float* Dd;    // [B,n], null: zero
   void* Dy0;          // [B,n] AT, out
   unsigned* status;   // [0] != 0: a bounded wait expired
   long long t_end;    // first frame processed (the last one the forward pass visited)
@@ -471,7 +473,7 @@ __global__ __launch_bounds__(64 * WV) void k_lstm2_bwd_regw(const Lstm2BwdMulti 
     off_dy[j] = k < nc ? (unsigned)(((long long)b * p.ldDY + k) * ES) : kOobOffset;
     off_c[j] = k < nc ? (unsigned)(idx[j] * 4) : kOobOffset;
     dyw[j] = 0.f;
-    dc[j] = act[j] ? q.Dd[idx[j]] : 0.f;
+    dc[j] = act[j] && q.Dd ? q.Dd[idx[j]] : 0.f;
 #pragma unroll
     for (int gq = 0; gq < 4; ++gq) dx0[j][gq] = 0.f;
   }

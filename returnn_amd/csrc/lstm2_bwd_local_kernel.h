@@ -207,7 +207,7 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_bwd_local(const Lstm2BwdMu
     ring_at[j] = bl < rows ? (unsigned)((((gate * n + first) / KE * 8 + bl) * KE + first % KE) * ES) : kOobOffset;
     dx_at[j] = bl < rows && first < nc ? (unsigned)(((long long)b * p.ldDX + (long long)gate * nc + first) * ES) : kOobOffset;
     dyw[j] = 0.f;
-    dc[j] = act[j] ? q.Dd[idx[j]] : 0.f;
+    dc[j] = act[j] && q.Dd ? q.Dd[idx[j]] : 0.f;
 #pragma unroll
     for (int gq = 0; gq < 4; ++gq) dx0[j][gq] = 0.f;
   }

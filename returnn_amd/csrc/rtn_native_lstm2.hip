@@ -1802,7 +1802,7 @@ using namespace rtn;
 
 extern "C" {
 
-int rtn_native_lstm2_abi_version(void) { return 17; }
+int rtn_native_lstm2_abi_version(void) { return 18; }
 
 const char* rtn_native_lstm2_bwd_plan_text(void) { return g_bwd_plan_text.c_str(); }
 
@@ -2150,6 +2150,14 @@ struct BwdChoice {
 int bwd_calls(const rtn_lstm2_bwd_call* calls, int count, int64_t T, int32_t B, int32_t n, int32_t dtype, void* workspace,
               size_t workspace_bytes, void* hip_stream, int op_flags = 0, size_t ws_stride = 0);
 
+// Dc0 := Dd
+void start_cell_error(const BwdCtx& x, const rtn_lstm2_bwd_call& c) {
+  if (c.Dd_is_zero)
+    hipLaunchKernelGGL(k_fill_u32, dim3(256), dim3(256), 0, x.stream, (unsigned*)c.Dc0, 0u, x.bn);
+  else
+    hipLaunchKernelGGL(k_copy_f32, dim3(256), dim3(256), 0, x.stream, c.Dd, c.Dc0, x.bn);
+}
+
 // Argument checks, and the outputs of a call without any frame: DW := 0, Dc0 := Dd, Dy0 := 0 (returnn/native_op.py:
 // 1365-1370).  With frames every output is written by the kernels and products themselves.
 int bwd_check(const BwdCtx& x) {
@@ -2158,7 +2166,7 @@ int bwd_check(const BwdCtx& x) {
   for (int k = 0; k < x.count; ++k) {
     const rtn_lstm2_bwd_call& c = x.calls[k];
     if (nn4 > 0 && !c.DW) return fail(RTN_ERR_ARG, "NativeLstm2 backward: DW must not be null");
-    if (x.bn > 0 && (!c.Dd || !c.Dy0 || !c.Dc0)) return fail(RTN_ERR_ARG, "NativeLstm2 backward: Dd, Dy0 and Dc0 must not be null");
+    if (x.bn > 0 && ((!c.Dd && !c.Dd_is_zero) || !c.Dy0 || !c.Dc0)) return fail(RTN_ERR_ARG, "NativeLstm2 backward: Dd, Dy0 and Dc0 must not be null");
   }
   if (x.T == 0 || x.bn == 0 || x.count == 0) {
     for (int k = 0; k < x.count; ++k) {
@@ -2169,7 +2177,7 @@ int bwd_check(const BwdCtx& x) {
         RTN_HIP(hipGetLastError());
       }
       if (x.bn > 0) {
-        hipLaunchKernelGGL(k_copy_f32, fill_grid, fill_block, 0, x.stream, c.Dd, c.Dc0, x.bn);
+        start_cell_error(x, c);
         hipLaunchKernelGGL(k_fill_u32, fill_grid, fill_block, 0, x.stream, (unsigned*)c.Dy0, 0u, (long long)(((size_t)x.bn * x.es + 3) / 4));
         RTN_HIP(hipGetLastError());
       }
@@ -2184,6 +2192,7 @@ int bwd_check(const BwdCtx& x) {
     const void* ptrs[] = {c.W, c.y0, c.c0, c.i, c.Y, c.C, c.H, c.DY, c.Dd, c.DX, c.DW, c.Dy0, c.Dc0};
     const char* names[] = {"W", "y0", "c0", "i", "Y", "C", "H", "DY", "Dd", "DX", "DW", "Dy0", "Dc0"};
     for (int q = 0; q < 13; ++q) {
+      if (q == 8 && c.Dd_is_zero) continue;
       if (!ptrs[q]) return fail(RTN_ERR_ARG, "NativeLstm2 backward: %s must not be null", names[q]);
       // (W is read in 16-byte fragments only where n is a multiple of 16; the recurrent rows of a stacked matrix start at
       // a multiple of 4n elements, which is aligned then)
@@ -2233,12 +2242,12 @@ int bwd_padded(const BwdCtx& x, int np, void* workspace, size_t workspace_bytes)
     // the sibling op that keeps its cell states in H hands H in for C as well; it is not read then
     if (!(x.op_flags & kOpH0IsCell) && (rc = in(c.C, L.C, tb, 1, 4)) != RTN_OK) return rc;
     if ((rc = pads.add(c.W, 0, n, n, base + L.W, 0, np, np, 4, es)) != RTN_OK || (rc = in(c.y0, L.y0, B, 1, es)) != RTN_OK || (rc = in(c.c0, L.c0, B, 1, 4)) != RTN_OK ||
-        (rc = in(c.Dd, L.Dd, B, 1, 4)) != RTN_OK)
+        (!c.Dd_is_zero && (rc = in(c.Dd, L.Dd, B, 1, 4)) != RTN_OK))
       return rc;
     padded[(size_t)k] = {base + L.W, base + L.y0, (const float*)(base + L.c0), c.i, c.start, c.step, base + L.Y,
                          (const float*)(base + ((x.op_flags & kOpH0IsCell) ? L.H : L.C)), base + L.H, base + L.DY,
                          (const float*)(base + L.Dd), base + L.DX, (float*)(base + L.DW), base + L.Dy0, (float*)(base + L.Dc0),
-                         0, 0, 0, nullptr};
+                         0, 0, 0, nullptr, c.Dd_is_zero};
   }
   if ((rc = pads.launch()) != RTN_OK) return rc;
   rc = bwd_calls(padded.data(), x.count, x.T, B, np, x.dtype, workspace, need, (void*)x.stream, x.op_flags, each);
@@ -2446,7 +2455,7 @@ int bwd_prepare_jobs(const BwdCtx& x, const BwdChoice& ch, const BwdLayout& lay,
     if (ch.kernel) continue;
     // launches per frame: status, working copies of the errors and dx0 start at 0, the cell error at Dd
     hipLaunchKernelGGL(k_fill_u32, dim3(256), dim3(256), 0, x.stream, (unsigned*)j.ws, 0u, (long long)(lay.off_wpk / 4));
-    hipLaunchKernelGGL(k_copy_f32, dim3(256), dim3(256), 0, x.stream, c.Dd, c.Dc0, x.bn);
+    start_cell_error(x, c);
     RTN_HIP(hipGetLastError());
     if (j.num_steps != T) {
       // frames the loop does not visit keep DX = 0 (:1385-1388): all rows cleared here, row by row
@@ -2478,7 +2487,7 @@ int bwd_launch_persistent(const BwdCtx& x, const BwdChoice& ch, const BwdLayout&
     Lstm2BwdPersistent& q = multi.q[k];
     const BwdJob& j = jobs[(size_t)k];
     q.p = j.p;
-    q.Dd = x.calls[k].Dd;
+    q.Dd = x.calls[k].Dd_is_zero ? nullptr : x.calls[k].Dd;
     q.Dy0 = x.calls[k].Dy0;
     q.status = (unsigned*)j.ws;
     q.t_end = j.end;
@@ -2704,7 +2713,7 @@ int bwd_own_weight_gradients(const BwdCtx& x, const BwdLayout& lay, const std::v
 
 // The share y0^T dx0 of the weight gradients, added to DW (where there is anything yet), and DW in the wanted type, for as many calls per launch as the
 // kernel takes; *done: whether it does.  (Few rows: the float32 product then hides behind the pass over DW.  Training steps, us, library product and
-// conversion / this: bf16 one layer n = 2048, B = 64 1288 / 1266, B = 16 670 / 642, n = 1024, B = 128 732 / 726, B = 250 689 / 688, three bidirectional
+// conversion / this: bf16 one layer n = 2048, B = 64 1288 / 1266, B = 16 670 / 642, n = 1024, T = 32, B = 128 396 / 395, B = 250 733 / 739, three bidirectional
 // layers n = 512, B = 32 870 / 829, n = 1024 2290 / 2237; float32 three of n = 500, B = 40 2195 / 2179, one n = 512, B = 128 649 / 651.)
 int bwd_last_weight_gradients(const BwdCtx& x, const std::vector<BwdJob>& jobs, bool* done) {
   const int n = x.n;

@@ -375,7 +375,7 @@ Tensor last_output(const Tensor& Y_in, const Tensor& y0_in, const Tensor& i_in, 
 
 // ---- the gradient op ----------------------------------------------------------------------------------------------
 struct BwdArgs {
-  Tensor W, y0, c0, i, Y, C, H, DY, Dd;
+  Tensor W, y0, c0, i, Y, C, H, DY, Dd;     // (Dd undefined: zero)
   int64_t start, step, T, B, n, ldY, ldDY;  // (pitches: 0 = contiguous)
   bool bf16;
 };
@@ -399,7 +399,7 @@ BwdArgs bwd_args(const Tensor& W, const Tensor& y0, const Tensor& c0, const Tens
   a.c0 = packed(as_type(c0, at::kFloat));
   a.i = packed(as_type(i, at::kFloat));
   a.C = packed(as_type(C, at::kFloat));
-  a.Dd = packed(as_type(Dd, at::kFloat));
+  if (Dd.defined()) a.Dd = packed(as_type(Dd, at::kFloat));
   a.start = start;
   a.step = step;
   TORCH_CHECK(a.i.dim() == 2 && a.y0.dim() == 2, "NativeLstm2 gradient: i ", a.i.sizes(), " / y0 ", a.y0.sizes());
@@ -417,7 +417,7 @@ BwdArgs bwd_args(const Tensor& W, const Tensor& y0, const Tensor& c0, const Tens
   expect("C", a.C, {a.T, a.B, a.n});
   expect("H", a.H, {a.T, a.B, 4 * a.n});
   expect("DY", a.DY, {a.T, a.B, a.n});
-  expect("Dd", a.Dd, {a.B, a.n});
+  if (a.Dd.defined()) expect("Dd", a.Dd, {a.B, a.n});
   return a;
 }
 
@@ -452,8 +452,8 @@ std::pair<std::vector<Out4>, Tensor> lstm2_grad_multi(const std::vector<BwdArgs>
       DW_act = std::get<1>(o).data_ptr();
     }
     calls[k] = {a.W.data_ptr(), a.y0.data_ptr(), a.c0.data_ptr<float>(), a.i.data_ptr<float>(), (int)a.start, (int)a.step, a.Y.data_ptr(), a.C.data_ptr<float>(),
-                a.H.data_ptr(), a.DY.data_ptr(), a.Dd.data_ptr<float>(), DX.data_ptr(), DW.data_ptr<float>(), std::get<2>(o).data_ptr(),
-                std::get<3>(o).data_ptr<float>(), a.ldY, a.ldDY, DXj.defined() ? count * 4 * f.n : 0, DW_act};
+                a.H.data_ptr(), a.DY.data_ptr(), a.Dd.defined() ? a.Dd.data_ptr<float>() : nullptr, DX.data_ptr(), DW.data_ptr<float>(), std::get<2>(o).data_ptr(),
+                std::get<3>(o).data_ptr<float>(), a.ldY, a.ldDY, DXj.defined() ? count * 4 * f.n : 0, DW_act, a.Dd.defined() ? 0 : 1};
   }
   const Tensor ws = workspace(rtn_abi.bwd_multi_workspace_bytes(count, f.T, (int)f.B, (int)f.n, dtype), f.Y);
   check_rc(rtn_abi.bwd_multi(calls.data(), count, f.T, (int)f.B, (int)f.n, dtype, ws.data_ptr(), (size_t)ws.numel(), stream));
@@ -632,8 +632,7 @@ struct LayerFunction : torch::autograd::Function<LayerFunction> {
       const Tensor* s = &saved[4 + 5 * k];  // W, y0, c0, C, H
       const int64_t n = s[1].size(1);
       auto half = [&](const Tensor& t) { return count == 1 ? t : t.slice(2, k * n, (k + 1) * n); };
-      args.push_back(bwd_args(s[0], s[1], s[2], mask, 0, k ? -step0 : step0, half(Y), s[3], s[4], half(DY),
-                              grads[1 + k].defined() ? grads[1 + k] : at::zeros_like(s[2], s[2].options().dtype(at::kFloat))));
+      args.push_back(bwd_args(s[0], s[1], s[2], mask, 0, k ? -step0 : step0, half(Y), s[3], s[4], half(DY), grads[1 + k]));
     }
     bool own_type = true;  // (the weights have the op's type)
     for (int k = 0; k < count; ++k) own_type = own_type && saved[4 + 5 * k].scalar_type() == Y.scalar_type();

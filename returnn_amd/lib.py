@@ -31,7 +31,7 @@ MODE_PERSISTENT = 1
 MODE_GRAPH = 2
 MODE_STEPWISE = 3
 # The ABI version the structs and argument lists below were written for (rtn_native_lstm2_abi_version()).
-EXPECTED_ABI = 17
+EXPECTED_ABI = 18
 
 MODES = {"auto": MODE_AUTO, "persistent": MODE_PERSISTENT, "graph": MODE_GRAPH, "stepwise": MODE_STEPWISE}
 
@@ -122,6 +122,7 @@ class Lstm2BwdCall(ctypes.Structure):
         ("ldDY", ctypes.c_int64),  # row pitch of DY in elements, 0 = contiguous (n)
         ("ldDX", ctypes.c_int64),  # row pitch of DX in elements, 0 = contiguous (4n)
         ("DW_act", ctypes.c_void_p),  # DW in the op's element type, or null
+        ("Dd_is_zero", ctypes.c_int32),  # no error on the final cell state: Dd is not read
     ]
 
 

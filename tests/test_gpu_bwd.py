@@ -594,7 +594,7 @@ def test_transposed_product(rows, m, n, dtype, out_dtype, pad):
 
 # The weight gradient in the op's type: own kernel (n = 64), last share in a pass of its own (few rows; tiles of the output cut, no long product
 # with one frame), library and conversion (many rows, also every second frame), padded copies (n = 45); one of the two calls only: a launch each.
-@pytest.mark.parametrize("T,B,n,step", [(7, 5, 64, 1), (6, 5, 420, 1), (1, 3, 512, 1), (9, 64, 1024, -1), (5, 130, 512, 1), (7, 4, 512, 2), (5, 3, 45, 1)])
+@pytest.mark.parametrize("T,B,n,step", [(7, 5, 64, 1), (6, 5, 420, 1), (1, 3, 512, 1), (9, 64, 1024, -1), (5, 260, 512, 1), (7, 4, 512, 2), (5, 3, 45, 1)])
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
 @pytest.mark.parametrize("wanted", [(True, True), (False, True)])
 def test_bwd_weight_gradient_in_the_ops_type(T, B, n, step, dtype, wanted):
@@ -631,3 +631,32 @@ def test_bwd_weight_gradient_in_the_ops_type(T, B, n, step, dtype, wanted):
     if wanted[0]:
         arr[0].DW_act += 4
         assert cabi.rtn_native_lstm2_bwd_multi(arr, 2, T, B, n, code, ws.data_ptr(), ws.numel(), None) == lib.RTN_ERR_ARG
+
+
+# No error on the final cell state, without an array for it: persistent kernels (one XCD, all), one launch per frame, padded copies, no frame at all
+@pytest.mark.parametrize("T,B,n,kernel", [(6, 5, 64, 0), (5, 20, 1280, 0), (4, 3, 32, 1), (4, 3, 45, 0), (0, 3, 32, 0)])
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_bwd_without_error_on_the_final_state(T, B, n, kernel, dtype, monkeypatch):
+    announce("bwd without Dd", T, B, n, kernel, dtype)
+    monkeypatch.setenv("RTN_LSTM2_BWD_KERNEL", str(kernel))
+    cabi = lib.load()
+    act, code = (torch.bfloat16, lib.DTYPE_BF16) if dtype == "bf16" else (torch.float32, lib.DTYPE_F32)
+    X, W, y0, c0, i = random_problem(810, T, B, n)
+    args = [to_dev(X, dtype), to_dev(W, dtype), to_dev(y0, dtype), to_dev(c0, "f32"), to_dev(i, "f32")]
+    Y, C, H, _ = get_op()(*args, 0, 1)
+    DY = to_dev(numpy.random.default_rng(61).normal(0, 1, (T, B, n)), dtype)
+    zeros = torch.zeros((B, n), device="cuda")
+    ws = torch.empty(int(cabi.rtn_native_lstm2_bwd_multi_workspace_bytes(1, T, B, n, code)), dtype=torch.uint8, device="cuda")
+    results = []
+    for absent in (False, True):
+        outs = [torch.full(s, float("nan"), device="cuda", dtype=d) for s, d in (((T, B, 4 * n), act), ((n, 4 * n), torch.float32), ((B, n), act), ((B, n), torch.float32))]
+        call = (lib.Lstm2BwdCall * 1)(lib.Lstm2BwdCall(*[a.data_ptr() for a in args[1:]], 0, 1, Y.data_ptr(), C.data_ptr(), H.data_ptr(), DY.data_ptr(),
+                                                       None if absent else zeros.data_ptr(), *[o.data_ptr() for o in outs], 0, 0, 0, None, int(absent)))  # fmt: skip
+        lib.check(cabi.rtn_native_lstm2_bwd_multi(call, 1, T, B, n, code, ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream))
+        results.append(outs)
+        call[0].Dd, call[0].Dd_is_zero = None, 0
+        assert cabi.rtn_native_lstm2_bwd_multi(call, 1, T, B, n, code, ws.data_ptr(), ws.numel(), None) == lib.RTN_ERR_ARG
+    for k, (a, b) in enumerate(zip(*results)):
+        assert torch.isfinite(a.float()).all()
+        # (the products' partial sums may be added in another order)
+        assert torch.equal(a, b) if k != 1 else float((a - b).abs().max()) <= 2.0**-20 * max(1.0, float(a.abs().max())) * (T * B) ** 0.5, k
