@@ -2713,12 +2713,12 @@ int bwd_own_weight_gradients(const BwdCtx& x, const BwdLayout& lay, const std::v
 
 // The share y0^T dx0 of the weight gradients, added to DW (where there is anything yet), and DW in the wanted type, for as many calls per launch as the
 // kernel takes; *done: whether it does.  (Few rows: the float32 product then hides behind the pass over DW.  Training steps, us, library product and
-// conversion / this: bf16 one layer n = 2048, B = 64 1288 / 1266, B = 16 670 / 642, n = 1024, T = 32, B = 128 396 / 395, B = 250 733 / 739, three bidirectional
-// layers n = 512, B = 32 870 / 829, n = 1024 2290 / 2237; float32 three of n = 500, B = 40 2195 / 2179, one n = 512, B = 128 649 / 651.)
+// conversion / this: bf16 one layer n = 2048, B = 64 1272 / 1264, n = 1024, B = 128 387 / 388, B = 250 701 / 707, three bidirectional layers n = 1024,
+// B = 32 2242 / 2190; float32 three of n = 500, B = 40 2188 / 2166, one n = 1024, B = 64 1008 / 1009, n = 512, B = 128 647 / 654.)
 int bwd_last_weight_gradients(const BwdCtx& x, const std::vector<BwdJob>& jobs, bool* done) {
   const int n = x.n;
   *done = false;
-  if (n % 4 != 0 || x.B > (x.dtype == RTN_DTYPE_BF16 ? 128 : 64)) return RTN_OK;
+  if (n % 4 != 0 || x.B > 64) return RTN_OK;
   WeightGradArgs args;
   memset(&args, 0, sizeof(args));
   args.m = n;
@@ -2743,13 +2743,13 @@ int bwd_last_weight_gradients(const BwdCtx& x, const std::vector<BwdJob>& jobs, 
       q.add = j.num_steps > 1;
       acts += c.DW_act != nullptr;
     }
-    const dim3 grid((unsigned)weight_tiles(args.m, args.n), (unsigned)now), block(kWgThreads);
+    const dim3 grid((unsigned)(((args.m + 31) / 32 * ((args.n + kWeightTile - 1) / kWeightTile) + kWaves - 1) / kWaves), (unsigned)now), block(kWgThreads);
     if (x.dtype != RTN_DTYPE_BF16)
-      hipLaunchKernelGGL((k_weight_grad<float, false, float>), grid, block, 0, x.stream, args);
+      hipLaunchKernelGGL((k_weight_last<float, float>), grid, block, 0, x.stream, args);
     else if (acts)
-      hipLaunchKernelGGL((k_weight_grad<__bf16, false, __bf16>), grid, block, 0, x.stream, args);
+      hipLaunchKernelGGL((k_weight_last<__bf16, __bf16>), grid, block, 0, x.stream, args);
     else
-      hipLaunchKernelGGL((k_weight_grad<__bf16, false, float>), grid, block, 0, x.stream, args);
+      hipLaunchKernelGGL((k_weight_last<__bf16, float>), grid, block, 0, x.stream, args);
     RTN_HIP(hipGetLastError());
   }
   *done = true;

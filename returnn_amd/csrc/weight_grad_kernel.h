@@ -30,7 +30,7 @@ struct WeightGradCall {
   long long rows[2], lda[2], ldb[2];  // elements from one row to the next
   float* part;                        // [parts][m][n]
   void* out;                          // [m][n]
-  int add;                            // OT: out = part + A^T B
+  int add;                            // k_weight_last: out = part + A^T B
 };
 struct WeightGradArgs {
   int m, n;                           // m: a multiple of 4
@@ -41,10 +41,7 @@ struct WeightGradArgs {
 };
 
 // ANY: n, and the distance between the rows of B, need not be multiples of 4: B comes in and the result goes out by element.
-// OT (one short product, slices = parts = 1): out = A^T B in that type, plus what is in part if the call says so: the last frame's share y0^T dx0
-// of a wide layer's gradient, whose long product is the library's, and the conversion to the parameter's type in one pass over DW for all
-// directions.  Bound by that pass.
-template <typename AT, bool ANY, typename OT = void>
+template <typename AT, bool ANY>
 __global__ __launch_bounds__(kWgThreads) void k_weight_grad(const WeightGradArgs args) {
   constexpr int ES = (int)sizeof(AT);
   typedef std::conditional_t<ES == 4, u32x4, u32x2> Quad4;  // four neighbouring elements
@@ -127,29 +124,15 @@ __global__ __launch_bounds__(kWgThreads) void k_weight_grad(const WeightGradArgs
         }
   };
   constexpr int kRows = 4 * kWaves * kWeightAhead;
-  constexpr bool LAST = !std::is_void_v<OT>;
   // entry 4 a + r of a lane: row 4 (4 kg + r) + a of the tile, columns 4 i ... 4 i + 3
   auto row_of = [&](int entry) { return m0 + 4 * (4 * kg + (entry & 3)) + (entry >> 2); };
   const int col = n0 + 4 * i;
-  f32x4 before[4];
   fetch(IntTag<0>{});
-  if constexpr (LAST) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {  // (on their way during the product)
-      const int row = row_of(4 * wave + e);
-      before[e] = q.add && row < args.m && col < args.n ? *(const f32x4*)(q.part + (size_t)row * args.n + col) : f32x4{0.f, 0.f, 0.f, 0.f};
-    }
-    for (int r = 0; r < rows; r += kRows) {
-      multiply(IntTag<0>{});
-      if (r + kRows < rows) fetch(IntTag<0>{});
-    }
-  } else {
-    for (int r = 0; r < rows; r += 2 * kRows) {
-      fetch(IntTag<1>{});
-      multiply(IntTag<0>{});
-      fetch(IntTag<0>{});
-      multiply(IntTag<1>{});
-    }
+  for (int r = 0; r < rows; r += 2 * kRows) {
+    fetch(IntTag<1>{});
+    multiply(IntTag<0>{});
+    fetch(IntTag<0>{});
+    multiply(IntTag<1>{});
   }
 #pragma unroll
   for (int a = 0; a < 4; ++a)
@@ -161,19 +144,7 @@ __global__ __launch_bounds__(kWgThreads) void k_weight_grad(const WeightGradArgs
   for (int e = 0; e < 4; ++e) {
     const int entry = 4 * wave + e, row = row_of(entry);
     const f32x4 sum = ((red[0][entry][lane] + red[1][entry][lane]) + red[2][entry][lane]) + red[3][entry][lane];
-    if constexpr (LAST) {
-      static_assert(!ANY);
-      if (row < args.m && col < args.n) {
-        const f32x4 all = before[e] + sum;
-        const size_t at = (size_t)row * args.n + col;
-        if constexpr (std::is_same_v<OT, float>) {
-          *(f32x4*)((float*)q.out + at) = all;
-        } else {
-          typedef OT Out4v __attribute__((ext_vector_type(4)));
-          *(Out4v*)((OT*)q.out + at) = __builtin_convertvector(all, Out4v);
-        }
-      }
-    } else if constexpr (ANY) {
+    if constexpr (ANY) {
 #pragma unroll
       for (int k = 0; k < 4; ++k)
         if (row < args.m && col + k < args.n) out[(size_t)row * args.n + col + k] = sum[k];
@@ -181,6 +152,100 @@ __global__ __launch_bounds__(kWgThreads) void k_weight_grad(const WeightGradArgs
       if (row < args.m && col < args.n) *(f32x4*)(out + (size_t)row * args.n + col) = sum;
     }
   }
+}
+
+// out = A^T B of few rows (a[0], b[0]), plus what is in part if the call says so: the last frame's share y0^T dx0 of a wide layer's gradient, whose
+// long product is the library's, and the conversion to the parameter's type, in one pass over DW for all directions.  Every wavefront has a tile of
+// 32 x 64 of its own, asks for what is there first, multiplies meanwhile (operands as above, two neighbouring columns of A per lane) and writes 16 bytes
+// (8 in bf16) per lane, 256 (128) of a row together.  Bound by that pass (96 MB at bf16 n = 2048: 20 us) and the float32 matrix rate (14 us at 64
+// rows); 33.5 us, with tiles of 64 x 64 and half the wavefronts 40, with a tile per workgroup, its rows dealt to the wavefronts and added
+// through LDS, 47; library product and conversion 45.  Both directions of float32 n = 500, 40 rows: 8.4 us, 11.1, 8.1 and 14.6.
+template <typename AT, typename OT>
+__global__ __launch_bounds__(kWgThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_weight_last(const WeightGradArgs args) {
+  constexpr int ES = (int)sizeof(AT);
+  typedef std::conditional_t<ES == 4, u32x4, u32x2> Quad4;
+  typedef std::conditional_t<ES == 4, u32x2, unsigned> Pair;
+  const WeightGradCall& q = args.call[blockIdx.y];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), kg = lane >> 4, i = lane & 15;
+  const int tiles_n = (args.n + kWeightTile - 1) / kWeightTile, tile = (int)blockIdx.x * kWaves + wave;
+  const int m0 = 32 * (tile / tiles_n), n0 = kWeightTile * (tile % tiles_n);
+  if (m0 >= args.m) return;
+  const int rows = (int)q.rows[0], col = n0 + 4 * i;
+  auto row_of = [&](int a, int r) { return m0 + 2 * (4 * kg + r) + a; };
+  f32x4 before[2][4];
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      before[a][r] = q.add && row_of(a, r) < args.m && col < args.n ? *(const f32x4*)(q.part + (size_t)row_of(a, r) * args.n + col) : f32x4{0.f, 0.f, 0.f, 0.f};
+  const unsigned pitch_a = (unsigned)(q.lda[0] * ES), pitch_b = (unsigned)(q.ldb[0] * ES);
+  __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)q.a[0], 0, rows > 0 ? (rows - 1) * pitch_a + args.m * ES : 0u, kBufFlags);
+  __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void*)q.b[0], 0, rows > 0 ? (rows - 1) * pitch_b + args.n * ES : 0u, kBufFlags);
+  unsigned at_a = m0 + 2 * i < args.m ? kg * pitch_a + (m0 + 2 * i) * ES : kOobOffset, at_b = col < args.n ? kg * pitch_b + col * ES : kOobOffset;
+  auto load = [](__amdgpu_buffer_rsrc_t rs, unsigned at) {
+    if constexpr (ES == 4)
+      return __builtin_bit_cast(Quad4, __builtin_amdgcn_raw_buffer_load_b128(rs, at, 0, 0));
+    else
+      return __builtin_bit_cast(Quad4, __builtin_amdgcn_raw_buffer_load_b64(rs, at, 0, 0));
+  };
+  auto element = [](Quad4 v, int k) {
+    if constexpr (ES == 4)
+      return __builtin_bit_cast(float, (unsigned)v[k]);
+    else
+      return __builtin_bit_cast(float, k & 1 ? v[k >> 1] & 0xFFFF0000u : v[k >> 1] << 16);
+  };
+  auto left = [](Pair v, int k) {
+    if constexpr (ES == 4)
+      return __builtin_bit_cast(float, (unsigned)v[k]);
+    else
+      return __builtin_bit_cast(float, k ? v & 0xFFFF0000u : v << 16);
+  };
+  f32x4 acc[2][4];
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 4; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+  Pair va[2][kWeightAhead];
+  Quad4 vb[2][kWeightAhead];
+  auto fetch = [&](auto set_tag) {
+    constexpr int S = decltype(set_tag)::value;
+#pragma unroll
+    for (int u = 0; u < kWeightAhead; ++u) {
+      if constexpr (ES == 4)
+        va[S][u] = __builtin_bit_cast(Pair, __builtin_amdgcn_raw_buffer_load_b64(ra, at_a, 0, 0));
+      else
+        va[S][u] = __builtin_amdgcn_raw_buffer_load_b32(ra, at_a, 0, 0);
+      vb[S][u] = load(rb, at_b);
+      at_a += 4 * pitch_a;
+      at_b += 4 * pitch_b;
+    }
+  };
+  auto multiply = [&](auto set_tag) {
+    constexpr int S = decltype(set_tag)::value;
+#pragma unroll
+    for (int u = 0; u < kWeightAhead; ++u)
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < 4; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(left(va[S][u], a), element(vb[S][u], b), acc[a][b], 0, 0, 0);
+  };
+  constexpr int kRows = 4 * kWeightAhead;
+  fetch(IntTag<0>{});
+  for (int r = 0; r < rows; r += 2 * kRows) {
+    fetch(IntTag<1>{});
+    multiply(IntTag<0>{});
+    fetch(IntTag<0>{});
+    if (r + kRows < rows) multiply(IntTag<1>{});
+  }
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      if (row_of(a, r) >= args.m || col >= args.n) continue;
+      const f32x4 all = before[a][r] + f32x4{acc[a][0][r], acc[a][1][r], acc[a][2][r], acc[a][3][r]};
+      typedef OT Four __attribute__((ext_vector_type(4)));
+      *(Four*)((OT*)q.out + (size_t)row_of(a, r) * args.n + col) = __builtin_convertvector(all, Four);
+    }
 }
 
 // out := the sum of the parts, four elements per lane; the wavefronts take every fourth part.
