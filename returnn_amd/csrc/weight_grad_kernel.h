@@ -25,6 +25,7 @@ namespace rtn {
 constexpr int kWeightTile = 64;       // columns of A and of B per workgroup
 constexpr int kWeightAhead = 4;       // steps of 16 rows whose loads are in flight together
 constexpr int kMaxWeightCalls = 2;
+constexpr unsigned kNoColumn = 0x80000000u;  // an offset that stays out of range while rows are stepped over (those of a slice end below 2^30)
 struct WeightGradCall {
   const void *a[2], *b[2];            // [rows][m], [rows][n]: the long product's and the other's
   long long rows[2], lda[2], ldb[2];  // elements from one row to the next
@@ -61,9 +62,9 @@ __global__ __launch_bounds__(kWgThreads) void k_weight_grad(const WeightGradArgs
   unsigned at_each[ANY ? 4 : 1];
   if constexpr (ANY) {
 #pragma unroll
-    for (int k = 0; k < 4; ++k) at_each[k] = n0 + 4 * i + k < args.n ? (4 * wave + kg) * pitch_b + (n0 + 4 * i + k) * ES : kOobOffset;
+    for (int k = 0; k < 4; ++k) at_each[k] = n0 + 4 * i + k < args.n ? (4 * wave + kg) * pitch_b + (n0 + 4 * i + k) * ES : kNoColumn;
   }
-  unsigned at_a = m0 + 4 * i < args.m ? (4 * wave + kg) * pitch_a + (m0 + 4 * i) * ES : kOobOffset, at_b = n0 + 4 * i < args.n ? (4 * wave + kg) * pitch_b + (n0 + 4 * i) * ES : kOobOffset;
+  unsigned at_a = m0 + 4 * i < args.m ? (4 * wave + kg) * pitch_a + (m0 + 4 * i) * ES : kNoColumn, at_b = n0 + 4 * i < args.n ? (4 * wave + kg) * pitch_b + (n0 + 4 * i) * ES : kNoColumn;
   const unsigned step_a = 4 * kWaves * pitch_a, step_b = 4 * kWaves * pitch_b;
   auto load = [](__amdgpu_buffer_rsrc_t rs, unsigned at) {
     if constexpr (ES == 4)
@@ -181,7 +182,7 @@ __global__ __launch_bounds__(kWgThreads) __attribute__((amdgpu_waves_per_eu(4)))
   const unsigned pitch_a = (unsigned)(q.lda[0] * ES), pitch_b = (unsigned)(q.ldb[0] * ES);
   __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)q.a[0], 0, rows > 0 ? (rows - 1) * pitch_a + args.m * ES : 0u, kBufFlags);
   __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void*)q.b[0], 0, rows > 0 ? (rows - 1) * pitch_b + args.n * ES : 0u, kBufFlags);
-  unsigned at_a = m0 + 2 * i < args.m ? kg * pitch_a + (m0 + 2 * i) * ES : kOobOffset, at_b = col < args.n ? kg * pitch_b + col * ES : kOobOffset;
+  unsigned at_a = m0 + 2 * i < args.m ? kg * pitch_a + (m0 + 2 * i) * ES : kNoColumn, at_b = col < args.n ? kg * pitch_b + col * ES : kNoColumn;
   auto load = [](__amdgpu_buffer_rsrc_t rs, unsigned at) {
     if constexpr (ES == 4)
       return __builtin_bit_cast(Quad4, __builtin_amdgcn_raw_buffer_load_b128(rs, at, 0, 0));
