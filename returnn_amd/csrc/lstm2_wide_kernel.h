@@ -227,13 +227,21 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_wide(const Lstm2Params p) 
   fetch(0);
   take();
   RTN_TRACE_DECL
+  // float32, two tiles of cells and one of rows: a delay that adapts, from 4 units on.  us per step in 1200 steps of n = 1722, 2 rows: none 6.16, fixed at 4
+  // 6.12, adapting 6.05 (from 20 on, which costs 120 steps 6.67 instead of 6.52 with none); the other float32 builds lose by it: n = 2048, 32 rows 10.95 / 11.19,
+  // n = 2816, 16 rows 10.93 / 11.16.
+  constexpr bool kAdapts = sizeof(AT) == 4 && MT == 2 && NT == 1;
+  int delay = 4;
   for (int s = 0; s < nsteps; ++s) {
     const unsigned slot = (unsigned)(s & (kHxRing - 1)) * slot_bytes, old = (unsigned)((s + 2) & (kHxRing - 1)) * slot_bytes;
     // ---- bring this workgroup's part of h_s over
     {
       // (No delay in front of the first read, as the kernels whose CUs read all of h across the XCDs have it: a repeat is 4 KB per CU and
       // costs the others nothing.  us per step without / with one that adapts: n = 4096, 16 rows 4.85 / 5.05, one row 5.18 / 5.63; n = 2560, 16 rows 4.01 / 4.45,
-      // 32 rows 6.05 / 6.43.)
+      // 32 rows 6.05 / 6.43.  In float32 one of the builds gains by one: see kAdapts.)
+      if constexpr (kAdapts)
+        if (s > 0)
+          for (int k = 0; k < delay; ++k) __builtin_amdgcn_s_sleep(1);
       i32x4 fv[kWideForward];
       unsigned spins = 0;
       bool again;
@@ -247,6 +255,12 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_wide(const Lstm2Params p) 
         for (int i = 0; i < kWideForward; ++i) fold(m, fv[i]);
         again = seen_mark(m) && keep_waiting(spins);
       } while (again);
+      if constexpr (kAdapts) {
+        if (spins)
+          delay = min(delay + p.delay_inc, 64);
+        else if (p.delay_inc && (s & p.delay_dec_mask) == p.delay_dec_mask && delay > 0)
+          --delay;
+      }
       RTN_TRACE_MARK(0)  // h_s arrives across the XCDs
       RTN_TRACE_ADD(6, spins)
       const u32x4 ones = u32x4{~0u, ~0u, ~0u, ~0u};
