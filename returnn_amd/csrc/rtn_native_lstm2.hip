@@ -1631,7 +1631,8 @@ int weight_grad_slices(int n, int dtype) {
 struct BwdLayout {
   size_t off_sync = 0, off_dyw = 0, off_dx0 = 0, off_wpk = 0, off_ex = 0, off_part = 0, total = 0;  // [0, off_wpk) is cleared at the start of a call
 };
-BwdLayout bwd_layout(int B, int n, int dtype) {
+// n: the width the kernels work at; cells: the caller's, the same or (where the persistent kernel pads on the fly) one that is padded to n.
+BwdLayout bwd_layout(int B, int n, int dtype, int cells) {
   BwdLayout l;
   size_t off = 256;  // status block, as in the forward workspace
   l.off_sync = off;  // two words per batch group (at most B groups): the XCD check of the persistent kernel
@@ -1646,8 +1647,9 @@ BwdLayout bwd_layout(int B, int n, int dtype) {
   // rows in frames of 8, or of more than 8 rows in frames of 16: never more than 2B + 16 rows in all
   l.off_ex = off;
   if (n % 16 == 0) off = align_up(off + (size_t)kExRing * 4 * n * esize(dtype) * (2 * (size_t)B + 16), 256);
-  l.off_part = off;  // the weight gradient's slices and y0^T dx0
-  if (const int slices = weight_grad_slices(n, dtype)) off = align_up(off + (size_t)(slices + 1) * 4 * n * n * 4, 256);
+  // the weight gradient's slices and y0^T dx0, of the caller's width (float32 324 has 4 slices, more bytes than the 3 of 352)
+  l.off_part = off;
+  if (const int slices = weight_grad_slices(cells, dtype)) off = align_up(off + (size_t)(slices + 1) * 4 * cells * cells * 4, 256);
   l.total = off;
   return l;
 }
@@ -2106,9 +2108,9 @@ int rtn_lstm_low_mem_fwd(const void* X, const void* W, const void* b, const void
 size_t rtn_native_lstm2_bwd_workspace_bytes(int64_t T, int32_t B, int32_t n, int32_t dtype) {
   if (check_dims(T, B, n, dtype) != RTN_OK) return 0;
   const int np = padded_width(n);
-  if (np == n || T == 0 || B == 0) return bwd_layout(B, n, dtype).total;
-  // a padded width: the workspace of the padded problem, then the padded copies
-  return bwd_layout(B, np, dtype).total + bwd_pad_layout(T, B, np, dtype).total;
+  if (np == n || T == 0 || B == 0) return bwd_layout(B, n, dtype, n).total;
+  // a padded width: the workspace of the padded problem, then the padded copies; or padded on the fly
+  return std::max(bwd_layout(B, np, dtype, np).total + bwd_pad_layout(T, B, np, dtype).total, bwd_layout(B, np, dtype, n).total);
 }
 
 namespace {
@@ -2218,7 +2220,7 @@ int bwd_convert_weights(const BwdCtx& x, const rtn_lstm2_bwd_call& c) {
 // k = the workspace of the padded call k, then its copies.
 int bwd_padded(const BwdCtx& x, int np, void* workspace, size_t workspace_bytes) {
   const int n = x.n, B = x.B;
-  const BwdLayout lay_p = bwd_layout(B, np, x.dtype);
+  const BwdLayout lay_p = bwd_layout(B, np, x.dtype, np);
   const BwdPadLayout L = bwd_pad_layout(x.T, B, np, x.dtype);
   const size_t each = lay_p.total + L.total;
   const size_t need = (size_t)x.count * each;
@@ -2823,7 +2825,6 @@ int bwd_calls(const rtn_lstm2_bwd_call* calls, int count, int64_t T, int32_t B, 
   // handle must exist already: run the op once outside the capture first, as for any library that sets itself up on
   // first use).
   x.capturing = cap_status != hipStreamCaptureStatusNone;
-  if (!x.capturing && T > 0 && x.bn > 0 && (rc = probe_xcds(x.stream)) != RTN_OK) return rc;
   if ((rc = bwd_check(x)) != RTN_OK) return rc;
   if (T == 0 || x.bn == 0 || count == 0) return RTN_OK;
   // A width that the kernels take padded: the persistent kernel pads on the fly as long as rows stay 16-byte aligned
@@ -2831,7 +2832,7 @@ int bwd_calls(const rtn_lstm2_bwd_call* calls, int count, int64_t T, int32_t B, 
   const int np = x.np;
   if (np != n && n % (int)(16 / x.es) != 0) return bwd_padded(x, np, workspace, workspace_bytes);
 
-  const BwdLayout lay = bwd_layout(B, np, dtype);
+  const BwdLayout lay = bwd_layout(B, np, dtype, n);
   // distance between the calls' workspaces
   const size_t stride = ws_stride ? ws_stride : rtn_native_lstm2_bwd_workspace_bytes(T, B, n, dtype);
   if (stride < lay.total) return fail(RTN_ERR_WORKSPACE, "NativeLstm2 backward: internal: workspace slice %zu < layout %zu", stride, lay.total);
@@ -2839,6 +2840,7 @@ int bwd_calls(const rtn_lstm2_bwd_call* calls, int count, int64_t T, int32_t B, 
     return fail(RTN_ERR_WORKSPACE, "NativeLstm2 backward: workspace of %zu bytes needed, got %zu", stride * (size_t)(count - 1) + lay.total,
                 workspace ? workspace_bytes : (size_t)0);
   if (!aligned16(workspace)) return fail(RTN_ERR_ARG, "NativeLstm2 backward: workspace must be 16-byte aligned");
+  if (!x.capturing && (rc = probe_xcds(x.stream)) != RTN_OK) return rc;
   rocblas_handle blas = nullptr;
   rc = blas_handle(&blas);
   if (rc != RTN_OK) return rc;

@@ -140,6 +140,29 @@ def test_plan_of_large_batches_padded_widths_and_wide_layers(cabi):
     assert "mode=graph" in text and "kernel=mfma_lds" in text and "lds=4096 " in text, text
 
 
+def _gradient_needs(cabi, T, B, n, dtype):
+    """The workspace the gradient entry asks for when it is given none (it then has not looked for a device yet)."""
+    p = ctypes.c_void_p(4096)
+    assert cabi.rtn_native_lstm2_bwd(p, p, p, p, 0, 1, p, p, p, p, p, p, p, p, p, T, B, n, dtype, None, 0, None) == lib.RTN_ERR_WORKSPACE, lib.last_error()
+    return int(re.search(r"workspace of (\d+) bytes needed", lib.last_error()).group(1))
+
+
+# widths that run padded on the fly (rows stay 16-byte aligned), with slices of the weight gradient of more bytes than the padded
+# width's (float32 268, 272, 324 ... 336), and others
+@pytest.mark.parametrize("dtype,n", [(lib.DTYPE_F32, k) for k in (36, 100, 260, 268, 272, 324, 328, 332, 336, 380)] + [(lib.DTYPE_BF16, k) for k in (40, 104, 200, 248)])
+def test_gradient_workspace_of_widths_padded_on_the_fly(cabi, dtype, n):
+    """What the gradient entry accepts as its workspace holds what the kernels write into it: the exchange ring and W at the padded width,
+    the slices of the weight gradient (64 x 64 tiles, two workgroups per CU, and y0^T dx0 beside them) at the caller's."""
+    T, B = 400, 32
+    padded, size = (n + 31) // 32 * 32, 2 if dtype == lib.DTYPE_BF16 else 4
+    slices = 512 // ((n + 63) // 64 * ((4 * n + 63) // 64))
+    slices = slices // 8 * 8 if slices >= 8 else slices
+    parts = (slices + 1) * n * 4 * n * 4
+    ring, w = 4 * 4 * padded * size * (2 * B + 16), 4 * padded * padded * size
+    assert _gradient_needs(cabi, T, B, n, dtype) >= parts + ring + w
+    assert cabi.rtn_native_lstm2_bwd_workspace_bytes(T, B, n, dtype) >= _gradient_needs(cabi, T, B, n, dtype)
+
+
 def test_xcd_local_plans(cabi):
     """Which shapes put every batch group on one XCD (planned for MI355X's 8 XCDs of 32 CUs when no device is visible)."""
     pair = lib.describe_multi_plan(2, 1000, 32, 1024, lib.DTYPE_BF16, lib.MODE_AUTO)  # the benchmark pair

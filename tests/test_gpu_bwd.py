@@ -561,6 +561,36 @@ def test_bwd_weight_gradient_of_small_layers(T, B, n, count, dtype):
         assert (numpy.abs(f(DW) - before.T @ DX) <= bound).all()
 
 
+@pytest.mark.parametrize("T,B,n", [(260, 32, 324), (260, 33, 268), (3, 2, 324)])
+def test_bwd_smallest_accepted_workspace(T, B, n):
+    """Widths padded on the fly whose slices of the weight gradient take more bytes than the padded width's: on the least workspace that the
+    entry accepts nothing is written behind it, and the weight gradient is that of float64 products (bound as above)."""
+    announce("bwd least workspace", T, B, n)
+    X, W, y0, c0, i = random_problem(n, T, B, n)
+    i[:] = 1.0
+    args = [to_dev(a, "f32") for a in (X, W, y0, c0, i)]
+    Y, C, H, _ = get_op()(*args, 0, 1)
+    rng = numpy.random.default_rng(9)
+    DY, Dd = to_dev(rng.normal(0, 1, (T, B, n)), "f32"), to_dev(rng.normal(0, 1, (B, n)), "f32")
+    DX, DW, Dy0, Dc0 = (torch.empty(shape, device="cuda") for shape in ((T, B, 4 * n), (n, 4 * n), (B, n), (B, n)))
+    cabi = lib.load()
+
+    def call(ws, size):
+        return cabi.rtn_native_lstm2_bwd(*[a.data_ptr() for a in args[1:]], 0, 1, Y.data_ptr(), C.data_ptr(), H.data_ptr(), DY.data_ptr(), Dd.data_ptr(), DX.data_ptr(),
+                                         DW.data_ptr(), Dy0.data_ptr(), Dc0.data_ptr(), T, B, n, lib.DTYPE_F32, ws, size, torch.cuda.current_stream().cuda_stream)  # fmt: skip
+
+    assert call(None, 0) == lib.RTN_ERR_WORKSPACE
+    need = int(lib.last_error().split("workspace of ")[1].split()[0])
+    ws = torch.full((need + 2**21,), 0x5A, dtype=torch.uint8, device="cuda")
+    lib.check(call(ws.data_ptr(), need))
+    torch.cuda.synchronize()
+    assert bool((ws[need:] == 0x5A).all())
+    f = lambda t: t.cpu().numpy().astype(numpy.float64)  # noqa: E731
+    before, dx = numpy.concatenate([f(args[2])[None], f(Y)[:-1]]).reshape(T * B, n), f(DX).reshape(T * B, 4 * n)
+    bound = 64 * 2.0**-24 * (numpy.abs(before).T @ numpy.abs(dx)) + 1e-30
+    assert (numpy.abs(f(DW) - before.T @ dx) <= bound).all()
+
+
 # a^T b in slices of the rows: widths that cut a tile, odd ones and rows that are farther apart (by element), one row, a slice's edge, and
 # more rows than a round of every slice takes
 @pytest.mark.parametrize("rows,m,n", [(1, 4, 1), (127, 64, 64), (129, 68, 77), (700, 180, 45), (9001, 256, 40), (20000, 128, 3)])
