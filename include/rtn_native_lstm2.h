@@ -238,7 +238,8 @@ int rtn_mfma_issue_probe(int32_t count, int64_t T, int32_t B, int32_t n, int32_t
  * capture the kernels (the persistent one as a node of its own, see rtn_native_lstm2_capture_report) and the rocBLAS calls
  * are recorded into the caller's graph (the counterpart of the
  * reference's whole-step graph capture, returnn/torch/util/graph_capture.py); the library's rocBLAS handle (one per host
- * thread and device) has to exist by then: run the entry once outside the capture first, on the capturing thread.  `workspace`: rtn_native_lstm2_bwd_workspace_bytes();
+ * thread and device) has to exist by then: run the entry once outside the capture first, on the capturing thread.  `workspace`: rtn_native_lstm2_bwd_workspace_bytes()
+ * of this T, B and n or of more frames (never less for more: a buffer for the longest call serves all of them);
  * rtn_native_lstm2_fwd_status(workspace, stream) reports an expired bounded wait of the persistent kernel.
  */
 int rtn_native_lstm2_bwd(const void* W, const void* y0, const float* c0, const float* i, int32_t start, int32_t step,

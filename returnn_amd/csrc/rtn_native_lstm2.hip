@@ -1619,20 +1619,23 @@ int product_slices(long long rows, int m, int n, int dtype) {
   return (int)slices;
 }
 
-// Slices of the rows that the weight gradient of a layer of width n is summed in at most (see weight_grad_kernel.h): two workgroups per CU
+// Slices of the rows that the weight gradient of a layer of width n is summed in (see weight_grad_kernel.h): at most two workgroups per CU
 // in all; 0: the product goes to the library, which with more tiles of output fills the chip itself (gradient op, us, library / this, for T B = 80, 2000, 30 000:
 // float32 n = 256 55 / 53, 189 / 187, 937 / 662, n = 384 72 / 73, 275 / 266, 1398 / 1292, n = 512 73 / 79, 289 / 291, 1415 / 1474; bf16, whose products the library takes at 8
 // times the rate, n = 192 60 / 43, 162 / 152, 538 / 514, n = 256 62 / 44, 165 / 162, 555 / 535, n = 320 63 / 50, 175 / 180, 675 / 758).
-int weight_grad_slices(int n, int dtype) {
+// Never fewer with more rows.  0 also for few rows of a wide layer (float32 n = 320, 2000 rows: 251 us in the library, 257
+// here; 30 000 rows 1384 and 1154).
+int weight_grad_slices(long long rows, int n, int dtype) {
   if (n % 4 != 0 || n < 4 || n > (dtype == RTN_DTYPE_BF16 ? 256 : 384)) return 0;
-  return slices_of_tiles(weight_tiles(n, 4 * n));
+  if (n > 256 && rows < 8192) return 0;
+  return (int)std::max<long long>(1, std::min<long long>(slices_of_tiles(weight_tiles(n, 4 * n)), (rows + kWeightRound - 1) / kWeightRound));
 }
 
 struct BwdLayout {
   size_t off_sync = 0, off_dyw = 0, off_dx0 = 0, off_wpk = 0, off_ex = 0, off_part = 0, total = 0;  // [0, off_wpk) is cleared at the start of a call
 };
 // n: the width the kernels work at; cells: the caller's, the same or (where the persistent kernel pads on the fly) one that is padded to n.
-BwdLayout bwd_layout(int B, int n, int dtype, int cells) {
+BwdLayout bwd_layout(int64_t T, int B, int n, int dtype, int cells) {
   BwdLayout l;
   size_t off = 256;  // status block, as in the forward workspace
   l.off_sync = off;  // two words per batch group (at most B groups): the XCD check of the persistent kernel
@@ -1647,9 +1650,10 @@ BwdLayout bwd_layout(int B, int n, int dtype, int cells) {
   // rows in frames of 8, or of more than 8 rows in frames of 16: never more than 2B + 16 rows in all
   l.off_ex = off;
   if (n % 16 == 0) off = align_up(off + (size_t)kExRing * 4 * n * esize(dtype) * (2 * (size_t)B + 16), 256);
-  // the weight gradient's slices and y0^T dx0, of the caller's width (float32 324 has 4 slices, more bytes than the 3 of 352)
+  // the weight gradient's slices and y0^T dx0, of the caller's width (float32 324 has 4 slices, more bytes than the 3 of 352) and as many as
+  // all frames' rows need (129 of n = 64 are 8 MB, a single frame has 2)
   l.off_part = off;
-  if (const int slices = weight_grad_slices(cells, dtype)) off = align_up(off + (size_t)(slices + 1) * 4 * cells * cells * 4, 256);
+  if (const int slices = weight_grad_slices(T * B, cells, dtype)) off = align_up(off + (size_t)(slices + 1) * 4 * cells * cells * 4, 256);
   l.total = off;
   return l;
 }
@@ -2108,9 +2112,9 @@ int rtn_lstm_low_mem_fwd(const void* X, const void* W, const void* b, const void
 size_t rtn_native_lstm2_bwd_workspace_bytes(int64_t T, int32_t B, int32_t n, int32_t dtype) {
   if (check_dims(T, B, n, dtype) != RTN_OK) return 0;
   const int np = padded_width(n);
-  if (np == n || T == 0 || B == 0) return bwd_layout(B, n, dtype, n).total;
+  if (np == n || T == 0 || B == 0) return bwd_layout(T, B, n, dtype, n).total;
   // a padded width: the workspace of the padded problem, then the padded copies; or padded on the fly
-  return std::max(bwd_layout(B, np, dtype, np).total + bwd_pad_layout(T, B, np, dtype).total, bwd_layout(B, np, dtype, n).total);
+  return std::max(bwd_layout(T, B, np, dtype, np).total + bwd_pad_layout(T, B, np, dtype).total, bwd_layout(T, B, np, dtype, n).total);
 }
 
 namespace {
@@ -2220,7 +2224,7 @@ int bwd_convert_weights(const BwdCtx& x, const rtn_lstm2_bwd_call& c) {
 // k = the workspace of the padded call k, then its copies.
 int bwd_padded(const BwdCtx& x, int np, void* workspace, size_t workspace_bytes) {
   const int n = x.n, B = x.B;
-  const BwdLayout lay_p = bwd_layout(B, np, x.dtype, np);
+  const BwdLayout lay_p = bwd_layout(x.T, B, np, x.dtype, np);
   const BwdPadLayout L = bwd_pad_layout(x.T, B, np, x.dtype);
   const size_t each = lay_p.total + L.total;
   const size_t need = (size_t)x.count * each;
@@ -2650,9 +2654,8 @@ bool same_weight_type(const BwdCtx& x) {
 // The weight gradients of x's calls by k_weight_grad, as many calls per launch as it takes; *done: whether it does (layers for which the
 // library's products leave most of the chip idle; consecutive frames; rows a multiple of four elements apart).
 int bwd_own_weight_gradients(const BwdCtx& x, const BwdLayout& lay, const std::vector<BwdJob>& jobs, bool* done) {
-  const int n = x.n, max_slices = weight_grad_slices(n, x.dtype);
+  const int n = x.n;
   *done = false;
-  if (!max_slices) return RTN_OK;
   long long longest = 0, widest = 4LL * n;
   for (int k = 0; k < x.count; ++k) {
     const BwdJob& j = jobs[(size_t)k];
@@ -2665,11 +2668,10 @@ int bwd_own_weight_gradients(const BwdCtx& x, const BwdLayout& lay, const std::v
   memset(&args, 0, sizeof(args));
   args.m = n;
   args.n = 4 * n;
-  args.slices = (int)std::max<long long>(1, std::min<long long>(max_slices, (longest + kWeightRound - 1) / kWeightRound));
+  args.slices = weight_grad_slices(longest, n, x.dtype);
+  if (!args.slices) return RTN_OK;
   args.slice_rows = (std::max<long long>(longest, 1) + args.slices - 1) / args.slices;
   args.parts = args.slices + 1;
-  // (float32 n = 320, 2000 rows: 251 us in the library, 257 here; 30 000 rows 1384 and 1154)
-  if (n > 256 && longest < 8192) return RTN_OK;
   // (offsets inside a slice, with the rows asked for behind it, are 32 bits wide)
   if ((std::max<long long>(args.slice_rows, x.B) + 2 * kWeightRound) * widest * (long long)x.es >= (1LL << 30)) return RTN_OK;
   const int tiles = weight_tiles(args.m, args.n);
@@ -2832,7 +2834,7 @@ int bwd_calls(const rtn_lstm2_bwd_call* calls, int count, int64_t T, int32_t B, 
   const int np = x.np;
   if (np != n && n % (int)(16 / x.es) != 0) return bwd_padded(x, np, workspace, workspace_bytes);
 
-  const BwdLayout lay = bwd_layout(B, np, dtype, n);
+  const BwdLayout lay = bwd_layout(T, B, np, dtype, n);
   // distance between the calls' workspaces
   const size_t stride = ws_stride ? ws_stride : rtn_native_lstm2_bwd_workspace_bytes(T, B, n, dtype);
   if (stride < lay.total) return fail(RTN_ERR_WORKSPACE, "NativeLstm2 backward: internal: workspace slice %zu < layout %zu", stride, lay.total);

@@ -153,7 +153,7 @@ def _gradient_needs(cabi, T, B, n, dtype):
 def test_gradient_workspace_of_widths_padded_on_the_fly(cabi, dtype, n):
     """What the gradient entry accepts as its workspace holds what the kernels write into it: the exchange ring and W at the padded width,
     the slices of the weight gradient (64 x 64 tiles, two workgroups per CU, and y0^T dx0 beside them) at the caller's."""
-    T, B = 400, 32
+    T, B = 4000, 32  # (rows enough for all slices of every width)
     padded, size = (n + 31) // 32 * 32, 2 if dtype == lib.DTYPE_BF16 else 4
     slices = 512 // ((n + 63) // 64 * ((4 * n + 63) // 64))
     slices = slices // 8 * 8 if slices >= 8 else slices
@@ -161,6 +161,20 @@ def test_gradient_workspace_of_widths_padded_on_the_fly(cabi, dtype, n):
     ring, w = 4 * 4 * padded * size * (2 * B + 16), 4 * padded * padded * size
     assert _gradient_needs(cabi, T, B, n, dtype) >= parts + ring + w
     assert cabi.rtn_native_lstm2_bwd_workspace_bytes(T, B, n, dtype) >= _gradient_needs(cabi, T, B, n, dtype)
+
+
+def test_gradient_workspace_grows_with_the_rows(cabi):
+    """The slices of the weight gradient's rows take room where there are rows for them: from one (and y0^T dx0) for a frame to all of a width's,
+    never less for more frames; none for few rows of the widths that leave them to the library."""
+    f32, bf16 = lib.DTYPE_F32, lib.DTYPE_BF16
+    size = cabi.rtn_native_lstm2_bwd_workspace_bytes
+    for dtype, n, most in [(f32, 64, 128), (f32, 256, 8), (bf16, 64, 128), (bf16, 128, 32)]:
+        part = n * 4 * n * 4
+        assert size(10**6, 1, n, dtype) - size(1, 1, n, dtype) == (most - 1) * part
+        sizes = [size(T, 3, n, dtype) for T in (1, 42, 43, 100, 1000, 10**4, 10**6)]
+        assert sizes == sorted(sizes) and sizes[2] == sizes[0] + part  # (126 rows, 129: a second slice)
+    assert size(8191, 1, 320, f32) == size(1, 1, 320, f32) < size(8192, 1, 320, f32)
+    assert size(10**4, 1, 512, f32) == size(1, 1, 512, f32)
 
 
 def test_xcd_local_plans(cabi):
