@@ -85,6 +85,16 @@ def test_bwd_forced_decompositions(rows, tiles, waves, dtype):
         assert _rel_to_max(a, b) <= bar, (name, _rel_to_max(a, b), plan)
 
 
+def test_bwd_ring_that_does_not_fit_its_section_is_refused():
+    """Groups of one row, which only the environment asks for, have frames of eight: the ring would reach into the section behind its own."""
+    from _gpu_util import env
+
+    announce("bwd ring beyond its section")
+    with env(RTN_LSTM2_BWD_KERNEL=2, RTN_LSTM2_BWD_ROWS=1):
+        with pytest.raises(RuntimeError, match="exchange ring"):
+            _run(200, 21, 64, "f32", 0, 1)
+
+
 # float32 groups of up to 8 rows on one XCD each: one and two quads of rows with 1, 2 and 4 tiles, cut quads and groups, every
 # number of macro steps per wavefront, odd widths
 @pytest.mark.parametrize("B,n,tiles,quads", [(1, 512, 1, 1), (30, 500, 1, 1), (61, 512, 2, 1), (37, 512, 1, 2), (128, 512, 2, 2), (97, 301, 2, 2), (60, 256, 1, 1), (205, 224, 2, 2),
