@@ -1148,6 +1148,17 @@ class PadList {
   long long blocks_ = 0;
 };
 
+// `bytes` bytes := 0, an even number of them (an odd number of bfloat16 elements: the last one by itself, not with the two bytes behind it)
+int launch_zeros(void* dst, long long bytes, hipStream_t stream) {
+  hipLaunchKernelGGL(k_fill_u32, dim3(256), dim3(256), 0, stream, (unsigned*)dst, 0u, bytes / 4);
+  RTN_HIP(hipGetLastError());
+  if (bytes % 4 == 0) return RTN_OK;
+  PadList last(stream);
+  unsigned char* at = (unsigned char*)dst + bytes / 4 * 4;
+  const int rc = last.add(at, 0, 1, 0, at, 0, 1, 1, 1, 2);  // (a row of no source)
+  return rc != RTN_OK ? rc : last.launch();
+}
+
 // rows x row_elems elements := 0, rows pitch elements apart (row_elems * es a multiple of 4)
 int launch_clear_rows(void* dst, long long rows, long long row_elems, long long pitch, size_t es, hipStream_t stream) {
   if (rows <= 0 || row_elems <= 0) return RTN_OK;
@@ -2184,8 +2195,7 @@ int bwd_check(const BwdCtx& x) {
       }
       if (x.bn > 0) {
         start_cell_error(x, c);
-        hipLaunchKernelGGL(k_fill_u32, fill_grid, fill_block, 0, x.stream, (unsigned*)c.Dy0, 0u, (long long)(((size_t)x.bn * x.es + 3) / 4));
-        RTN_HIP(hipGetLastError());
+        if (const int rc = launch_zeros(c.Dy0, x.bn * (long long)x.es, x.stream); rc != RTN_OK) return rc;
       }
     }
     return RTN_OK;
@@ -2984,8 +2994,7 @@ int rtn_lstm_low_mem_bwd(const void* X, const void* W, const void* b, const void
   if (bn == 0) {
     if (n_in > 0 && rows > 0) {
       if (!DX) return fail(RTN_ERR_ARG, "LstmLowMem gradient: DX must not be null");
-      hipLaunchKernelGGL(k_fill_u32, dim3(256), dim3(256), 0, stream, (unsigned*)DX, 0u, (long long)(((size_t)rows * n_in * es + 3) / 4));
-      RTN_HIP(hipGetLastError());
+      return launch_zeros(DX, rows * n_in * (long long)es, stream);
     }
     return RTN_OK;
   }

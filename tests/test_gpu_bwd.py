@@ -571,6 +571,28 @@ def test_bwd_weight_gradient_of_small_layers(T, B, n, count, dtype):
         assert (numpy.abs(f(DW) - before.T @ DX) <= bound).all()
 
 
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_bwd_without_frames_or_cells_writes_its_outputs_only(dtype):
+    """Gradients of no frames (Dy0 of three rows of five cells: an odd number of elements) and of no cells (LstmLowMem's DX): zeros, up to the last element."""
+    announce("bwd zeros", dtype)
+    get_op()
+    cabi = lib.load()
+    act, code = (torch.bfloat16, lib.DTYPE_BF16) if dtype == "bf16" else (torch.float32, lib.DTYPE_F32)
+    stream = torch.cuda.current_stream().cuda_stream
+    B, n = 3, 5
+    z = lambda *s: torch.zeros(s, device="cuda")  # noqa: E731
+    out = torch.full((32,), 7.0, dtype=act, device="cuda")
+    any_, Dd, DW, Dc0 = z(64), torch.ones((B, n), device="cuda"), z(n, 4 * n), z(B, n)
+    lib.check(cabi.rtn_native_lstm2_bwd(*[any_.data_ptr()] * 4, 0, 1, *[any_.data_ptr()] * 4, Dd.data_ptr(), any_.data_ptr(), DW.data_ptr(), out.data_ptr(), Dc0.data_ptr(),
+                                        0, B, n, code, None, 0, stream))  # fmt: skip
+    assert bool((out[: B * n] == 0).all()) and bool((out[B * n :] == 7.0).all()) and torch.equal(Dc0, Dd)
+    out.fill_(7.0)
+    args = [any_.data_ptr()] * 15
+    args[10] = out.data_ptr()
+    lib.check(cabi.rtn_lstm_low_mem_bwd(*args[:6], 0, 1, *args[6:], 3, 1, 5, 0, code, None, 0, stream))
+    assert bool((out[:15] == 0).all()) and bool((out[15:] == 7.0).all())
+
+
 @pytest.mark.parametrize("T,B,n", [(260, 32, 324), (260, 33, 268), (3, 2, 324)])
 def test_bwd_smallest_accepted_workspace(T, B, n):
     """Widths padded on the fly whose slices of the weight gradient take more bytes than the padded width's: on the least workspace that the
