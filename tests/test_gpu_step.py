@@ -104,3 +104,24 @@ def test_module_step_takes_the_same_way_as_the_function(source, params):
             module(x, state=state, direction=2)
         with pytest.raises(RuntimeError, match="HIP"):
             module(x.cpu(), state=state)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_step_of_a_module_with_weights_of_its_own(dtype):
+    """What a subclass's ``weights`` returns is what a step computes with: the bits of the same step of a plain layer with those parameters."""
+    class Halved(lstm_mod.LSTM):
+        def weights(self, act):
+            w = super().weights(act)
+            return w._replace(rec=0.5 * w.rec)
+
+    announce("lstm_step, own weights", dtype)
+    B, k, n = 5, 24, 40
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    halved, plain = (cls(k, n, device="cuda", dtype=dtype).requires_grad_(False) for cls in (Halved, lstm_mod.LSTM))
+    halved.reset_parameters(gen)
+    plain.load_state_dict(halved.state_dict())
+    plain.rec.mul_(0.5)
+    x, h = (torch.randn((B, j), device="cuda", generator=gen).to(dtype) for j in (k, n))
+    state = lstm_mod.LstmState(h=h, c=torch.randn((B, n), device="cuda", generator=gen))
+    (y, new), (want, want_new) = halved(x, state=state), plain(x, state=state)
+    assert torch.equal(y, want) and torch.equal(new.h, want_new.h) and torch.equal(new.c, want_new.c)

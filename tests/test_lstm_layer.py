@@ -174,3 +174,32 @@ def test_encoder_config_shapes():
     del sd["layers.0.fwd.bias"]
     with pytest.raises(RuntimeError, match="layers.0.fwd.bias"):
         other.load_state_dict(sd)
+
+
+def test_an_own_weights_method_has_the_last_word_on_a_step(monkeypatch):
+    """The module's short way of one step takes the parameters as they are; a subclass or an instance with a ``weights`` of its own gets what
+    that returns, in a step as in a sequence."""
+    def way(module):
+        taken = []
+        monkeypatch.setattr(rlstm, "_one_launch_step", lambda x, h, c, ff, rec, bias: taken.append(("parameters", rec)) or (h, h, c))
+        monkeypatch.setattr(rlstm, "lstm", lambda source, *, state_h, state_c, weights, **_: taken.append(("weights", weights.rec)) or (state_h, (state_h, state_c)))
+        for x in (torch.zeros(2, 3), torch.zeros(1, 2, 3)):
+            module(x, state=rlstm.LstmState(h=torch.zeros(2, 4), c=torch.zeros(2, 4)))
+        return taken
+
+    class Halved(rlstm.LSTM):
+        def weights(self, act):
+            w = super().weights(act)
+            return w._replace(rec=0.5 * w.rec)
+
+    class Plain(rlstm.LSTM):
+        pass
+
+    plain = Plain(3, 4)
+    (step, rec), (sequence, _) = way(plain)
+    assert step == "parameters" and rec is plain.rec and sequence == "weights"
+    halved = Halved(3, 4)
+    masked = rlstm.LSTM(3, 4)
+    masked.weights = lambda act: rlstm.LSTM.weights(masked, act)._replace(rec=torch.zeros(4, 16))
+    for module, want in ((halved, 0.5 * halved.rec), (masked, torch.zeros(4, 16))):
+        assert [(name, torch.equal(rec, want)) for name, rec in way(module)] == [("weights", True)] * 2
