@@ -66,10 +66,17 @@ def measured_traffic(workload: str, launches: int, plan: str):
 def forward_kernel(plan: str):
     """-> (the kernel a forward plan runs on, whether that is the register kernel whose steps the library's probes repeat)"""
     name = plan.split("kernel=")[1].split()[0]
-    kernel = {"mfma_regw_solo": "k_lstm2_solo", "mfma_regw_wide": "k_lstm2_wide", "mfma_lds": "k_lstm2_mfma"}.get(name, "k_step_generic")
+    solo = "k_lstm2_solo_row" if "rows_per_group=1 " in plan else "k_lstm2_solo"
+    kernel = {"mfma_regw_solo": solo, "mfma_regw_wide": "k_lstm2_wide", "mfma_lds": "k_lstm2_mfma"}.get(name, "k_step_generic")
     if name in ("mfma_regw", "mfma_regw_xcd", "mfma_regw_xcd_half"):
         kernel = "k_lstm2_dual" if "interleaved=2" in plan else "k_lstm2_regw"
     return kernel, kernel == "k_lstm2_regw"
+
+
+def gradient_kernels(plan: str):
+    """-> (the kernel the recurrence of a gradient call ran on, what its weight gradients came from), of lib.bwd_plan_text()"""
+    fields = dict(word.split("=", 1) for word in plan.split())
+    return fields["name"], fields["weight_gradient"]
 
 
 def algorithmic_bytes_per_unit(n: int, dtype: str) -> int:
@@ -565,9 +572,10 @@ def bench_gradient(args, dev, cabi):
     units = T * B * len(steps_of)
     flops = 16.0 * n * n * units
     peak = PEAK_MFMA[dtype]
+    kernel, weight_gradient = gradient_kernels(lib.bwd_plan_text())
     bwd_traffic, bwd_traffic_source = measured_traffic(
         args.workload + " gradient", 1 if (fused or len(steps_of) == 1) else len(steps_of),
-        "persistent kernel, %i problem(s) per launch" % (len(steps_of) if fused else 1))
+        "%s, %i problem(s) per launch" % (kernel, len(steps_of) if fused else 1))
     result = {
         "metric": "LSTM gradient op timesteps*seqs/sec (T*B/s) at n=%i" % n,
         "value": units * args.steps / elapsed,
@@ -600,8 +608,8 @@ def bench_gradient(args, dev, cabi):
             "traffic_unit": "bytes per launch of the persistent kernel (transcribed from the profile summary named in traffic_source, "
             "not measured by this run); algorithmic (read H, DY, C, mask; write DX): %i"
             % (((9 * (2 if dtype == "bf16" else 4) + 4) * n + 4) * units),
-            "kernel": "whole gradient call: the persistent k_lstm2_bwd_regw (or one k_bwd_step launch per frame) with the "
-            "recurrent GEMM, 8*n^2 flops per unit, then the weight-gradient GEMM in rocBLAS, 8*n^2 flops per unit",
+            "kernel": "whole gradient call: %s with the recurrent GEMM, 8*n^2 flops per unit, then the weight gradient (%s), 8*n^2 flops per unit"
+            % (kernel, weight_gradient),
             "launch_ms": call_ms,
         },
     }

@@ -2808,6 +2808,7 @@ int bwd_weight_gradients(const BwdCtx& x, rocblas_handle blas, const BwdLayout& 
   }
   bool last = own;
   if (!own && (rc = bwd_last_weight_gradients(x, jobs, &last)) != RTN_OK) return rc;
+  g_bwd_plan_text += own ? " weight_gradient=k_weight_grad" : last ? " weight_gradient=rocblas,k_weight_last" : " weight_gradient=rocblas";
   for (int k = 0; k < x.count && !last; ++k) {
     const rtn_lstm2_bwd_call& c = x.calls[k];
     const BwdJob& j = jobs[(size_t)k];
@@ -2879,11 +2880,12 @@ int bwd_calls(const rtn_lstm2_bwd_call* calls, int count, int64_t T, int32_t B, 
     const int bgroups = (B + ch.rows_per_group - 1) / ch.rows_per_group;
     char buf[256];
     if (ch.kernel)
-      snprintf(buf, sizeof(buf), "kernel=%s problems=%d rows_per_group=%d groups=%d tiles=%d waves=%d wgs_per_group=%d launches=%d row_quads=%d",
+      snprintf(buf, sizeof(buf), "kernel=%s problems=%d rows_per_group=%d groups=%d tiles=%d waves=%d wgs_per_group=%d launches=%d row_quads=%d name=%s",
                ch.local ? "bwd_regw_xcd" : "bwd_regw", count, ch.rows_per_group, bgroups, ch.tiles, ch.waves, np / (16 * ch.tiles),
-               (bgroups + ch.groups_per_launch - 1) / std::max(ch.groups_per_launch, 1), ch.rq);
+               (bgroups + ch.groups_per_launch - 1) / std::max(ch.groups_per_launch, 1), ch.rq, ch.one_xcd_kernel ? "k_lstm2_bwd_local" : "k_lstm2_bwd_regw");
     else
-      snprintf(buf, sizeof(buf), "kernel=%s problems=%d launches_per_frame=%d", mfma ? "bwd_step" : "bwd_generic", count, mfma ? 1 : 2);
+      snprintf(buf, sizeof(buf), "kernel=%s problems=%d launches_per_frame=%d name=%s", mfma ? "bwd_step" : "bwd_generic", count, mfma ? 1 : 2,
+               mfma ? "k_bwd_step" : "k_bwd_pointwise");
     g_bwd_plan_text = buf;
   }
 

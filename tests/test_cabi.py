@@ -329,4 +329,7 @@ def test_bench_names_the_kernel_of_the_plan():
                        ("mfma_regw_wide", "k_lstm2_wide"), ("mfma_lds", "k_lstm2_mfma"), ("generic", "k_step_generic")):  # fmt: skip
         assert bench.forward_kernel(plan % name) == (want, want == "k_lstm2_regw")
     assert bench.forward_kernel(plan % "mfma_regw_xcd" + " interleaved=2") == ("k_lstm2_dual", False)
+    assert bench.forward_kernel((plan % "mfma_regw_solo").replace("rows_per_group=8 ", "rows_per_group=1 ")) == ("k_lstm2_solo_row", False)
+    gradient = "kernel=bwd_regw_xcd problems=2 rows_per_group=8 groups=4 tiles=2 waves=4 wgs_per_group=32 launches=1 row_quads=0 name=k_lstm2_bwd_local"
+    assert bench.gradient_kernels(gradient + " weight_gradient=rocblas,k_weight_last") == ("k_lstm2_bwd_local", "rocblas,k_weight_last")
     assert bench.forward_kernel(lib.describe_plan(1000, 32, 1024, lib.DTYPE_BF16, lib.MODE_AUTO)) == ("k_lstm2_regw", True)

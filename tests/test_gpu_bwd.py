@@ -104,7 +104,7 @@ def test_bwd_quads_of_rows(B, n, tiles, quads):
     for start, step in [(0, 1), (1, -2)]:
         got, want, _ = _run(6, B, n, "f32", start, step, seed=B + n)
         plan = lib.bwd_plan_text()
-        assert "bwd_regw_xcd" in plan and "tiles=%i " % tiles in plan and "row_quads=%i" % quads in plan, plan
+        assert "bwd_regw_xcd" in plan and "tiles=%i " % tiles in plan and "row_quads=%i" % quads in plan and "name=k_lstm2_bwd_local " in plan, plan
         for name, a, b in zip(("DX", "DW", "Dy0", "Dc0"), got, want):
             assert numpy.isfinite(a).all(), name
             assert _rel_to_max(a, b) <= 2e-5, (name, _rel_to_max(a, b), plan)
@@ -125,10 +125,10 @@ def test_bwd_groups_of_one_xcd(dtype, B, n):
     for T, start, step in [(1, 0, 1), (2, 0, -1), (7, 1, 2)]:
         got, want, _ = _run(T, B, n, dtype, start, step, seed=T + B + n)
         plan = lib.bwd_plan_text()
-        assert "bwd_regw_xcd" in plan, plan
+        assert "bwd_regw_xcd" in plan and "name=k_lstm2_bwd_local " in plan, plan
         with env(RTN_LSTM2_BWD_LOCAL=0):
             spread, _, _ = _run(T, B, n, dtype, start, step, seed=T + B + n)
-            assert "bwd_regw_xcd" not in lib.bwd_plan_text(), lib.bwd_plan_text()
+            assert "bwd_regw_xcd" not in lib.bwd_plan_text() and "name=k_lstm2_bwd_regw " in lib.bwd_plan_text(), lib.bwd_plan_text()
         for name, a, b, c in zip(("DX", "DW", "Dy0", "Dc0"), got, want, spread):
             assert _rel_to_max(a, b) <= bar, (T, name, _rel_to_max(a, b), plan)
             assert _rel_to_max(a, c) <= step_bar, (T, name, _rel_to_max(a, c), plan)
@@ -147,6 +147,24 @@ def test_bwd_groups_of_one_xcd(dtype, B, n):
         assert torch.equal(hit[0][:, others], clean[0][:, others]) and torch.equal(hit[2][others], clean[2][others]) and torch.equal(hit[3][others], clean[3][others])
         assert not torch.isfinite(hit[0][:4, row].float()).all(-1).any()
         assert torch.equal(hit[0][4, row], clean[0][4, row])
+
+
+# Groups of up to 8 rows on one XCD each: their own kernel, the general one where fewer of the launch's groups fit the device with that, groups
+# over all XCDs, launches per frame; and what the weight gradient came from.
+@pytest.mark.parametrize("dtype,B,n,kernel,plan,weights", [
+    ("bf16", 30, 512, 0, "bwd_regw_xcd k_lstm2_bwd_local", "rocblas,k_weight_last"), ("bf16", 200, 512, 0, "bwd_regw_xcd k_lstm2_bwd_regw", "rocblas"),
+    ("bf16", 5, 2048, 0, "bwd_regw k_lstm2_bwd_regw", "rocblas,k_weight_last"), ("f32", 9, 64, 0, "bwd_regw_xcd k_lstm2_bwd_local", "k_weight_grad"),
+    ("f32", 9, 64, 1, "bwd_step k_bwd_step", "k_weight_grad"), ("bf16", 4, 24, 0, "bwd_generic k_bwd_pointwise", "k_weight_grad"), ("f32", 70, 30, 0, "bwd_generic k_bwd_pointwise", "rocblas")])  # fmt: skip
+def test_bwd_plan_names_its_kernels(dtype, B, n, kernel, plan, weights):
+    from _gpu_util import env
+
+    announce("bwd plan names", dtype, B, n, kernel)
+    with env(RTN_LSTM2_BWD_KERNEL=kernel):
+        got, want, _ = _run(3, B, n, dtype, 0, 1, seed=n)
+        fields = dict(word.split("=", 1) for word in lib.bwd_plan_text().split())
+    assert (fields["kernel"] + " " + fields["name"], fields["weight_gradient"]) == (plan, weights), lib.bwd_plan_text()
+    for name, a, b in zip(("DX", "DW", "Dy0", "Dc0"), got, want):
+        assert _rel_to_max(a, b) <= (2e-2 if dtype == "bf16" else 2e-5), name
 
 
 def test_bwd_read_delay_only_moves_time():
@@ -544,7 +562,7 @@ def test_bwd_padded_copies(dtype, B, n):
 # the weight gradient of small layers in slices of the rows: one slice and many, rows that leave a slice cut or empty, widths that cut a tile,
 # rows further apart than they are wide (two calls side by side), no frame but the first
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
-@pytest.mark.parametrize("T,B,n,count", [(1, 3, 32, 1), (2, 1, 64, 2), (9, 15, 4, 1), (40, 33, 100, 2), (130, 9, 68, 1), (65, 64, 256, 1), (30, 7, 192, 2), (300, 40, 36, 1), (64, 130, 384, 1)])
+@pytest.mark.parametrize("T,B,n,count", [(1, 3, 32, 1), (2, 1, 64, 2), (9, 15, 4, 1), (40, 33, 100, 2), (130, 9, 68, 1), (65, 64, 256, 1), (30, 7, 192, 2), (300, 40, 36, 1), (64, 131, 384, 1)])
 def test_bwd_weight_gradient_of_small_layers(T, B, n, count, dtype):
     """Against float64 products of what the op itself returned (dx0 is DX of the first visited frame where no frame is masked): the order of
     additions is all that differs, so within a few float32 roundings of the sum of magnitudes (64 of them, for up to 12 000 terms in slices)."""
@@ -561,7 +579,9 @@ def test_bwd_weight_gradient_of_small_layers(T, B, n, count, dtype):
         Y, C, H, _ = op(Xd, Wd, y0d, c0d, id_, 0, 1 - 2 * k)
         calls.append((Wd, y0d, c0d, id_, 0, 1 - 2 * k, Y, C, H, wide[..., k * n : (k + 1) * n], to_dev(rng.normal(0, 1, (B, n)), "f32")))
     f = lambda t: t.float().cpu().numpy().astype(numpy.float64)  # noqa: E731
-    for call, (DX, DW, _, _) in zip(calls, torch_native_op.native_lstm2_grad_multi(calls)):
+    results = torch_native_op.native_lstm2_grad_multi(calls)
+    assert ("weight_gradient=k_weight_grad" in lib.bwd_plan_text()) == (n <= 256 or dtype == "f32"), lib.bwd_plan_text()
+    for call, (DX, DW, _, _) in zip(calls, results):
         Y, DX = f(call[6]), f(DX)
         if call[5] < 0:
             Y, DX = Y[::-1], DX[::-1]
@@ -683,6 +703,8 @@ def test_bwd_weight_gradient_in_the_ops_type(T, B, n, step, dtype, wanted):
         keep.append((args, Y, C, H, DY, Dd, DX, DW, DW_act, Dy0, Dc0, want))
     ws = torch.empty(int(cabi.rtn_native_lstm2_bwd_multi_workspace_bytes(2, T, B, n, code)), dtype=torch.uint8, device="cuda")
     lib.check(cabi.rtn_native_lstm2_bwd_multi(arr, 2, T, B, n, code, ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream))
+    way = "k_weight_grad" if n <= 64 else "rocblas,k_weight_last" if B <= 64 else "rocblas"
+    assert lib.bwd_plan_text().endswith(" weight_gradient=" + way), lib.bwd_plan_text()
     for k in range(2):
         got, want = keep[k][8] if wanted[k] else keep[k][7], keep[k][11]
         scale = float(numpy.abs(want).max())
