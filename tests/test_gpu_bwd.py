@@ -720,9 +720,10 @@ def test_bwd_weight_gradient_in_the_ops_type(T, B, n, step, dtype, wanted):
 # No error on the final cell state, without an array for it: persistent kernels (one XCD, all), one launch per frame, padded copies, no frame at all
 @pytest.mark.parametrize("T,B,n,kernel", [(6, 5, 64, 0), (5, 20, 1280, 0), (4, 3, 32, 1), (4, 3, 45, 0), (0, 3, 32, 0)])
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
-def test_bwd_without_error_on_the_final_state(T, B, n, kernel, dtype, monkeypatch):
+def test_bwd_without_error_on_the_final_state(T, B, n, kernel, dtype):
+    from _gpu_util import env
+
     announce("bwd without Dd", T, B, n, kernel, dtype)
-    monkeypatch.setenv("RTN_LSTM2_BWD_KERNEL", str(kernel))
     cabi = lib.load()
     act, code = (torch.bfloat16, lib.DTYPE_BF16) if dtype == "bf16" else (torch.float32, lib.DTYPE_F32)
     X, W, y0, c0, i = random_problem(810, T, B, n)
@@ -736,7 +737,10 @@ def test_bwd_without_error_on_the_final_state(T, B, n, kernel, dtype, monkeypatc
         outs = [torch.full(s, float("nan"), device="cuda", dtype=d) for s, d in (((T, B, 4 * n), act), ((n, 4 * n), torch.float32), ((B, n), act), ((B, n), torch.float32))]
         call = (lib.Lstm2BwdCall * 1)(lib.Lstm2BwdCall(*[a.data_ptr() for a in args[1:]], 0, 1, Y.data_ptr(), C.data_ptr(), H.data_ptr(), DY.data_ptr(),
                                                        None if absent else zeros.data_ptr(), *[o.data_ptr() for o in outs], 0, 0, 0, None, int(absent)))  # fmt: skip
-        lib.check(cabi.rtn_native_lstm2_bwd_multi(call, 1, T, B, n, code, ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream))
+        with env(RTN_LSTM2_BWD_KERNEL=kernel):
+            lib.check(cabi.rtn_native_lstm2_bwd_multi(call, 1, T, B, n, code, ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream))
+            name = "k_bwd_step" if kernel == 1 or (n, dtype) == (1280, "f32") else "k_lstm2_bwd_regw" if n == 1280 else "k_lstm2_bwd_local"
+            assert T == 0 or "name=%s " % name in lib.bwd_plan_text(), lib.bwd_plan_text()
         results.append(outs)
         call[0].Dd, call[0].Dd_is_zero = None, 0
         assert cabi.rtn_native_lstm2_bwd_multi(call, 1, T, B, n, code, ws.data_ptr(), ws.numel(), None) == lib.RTN_ERR_ARG
