@@ -51,13 +51,14 @@ extern "C" {
 /* Execution mode.
  * AUTO:       PERSISTENT when the shape and device allow it, else GRAPH.
  * PERSISTENT: one kernel runs all time steps, all its workgroups on the device together
- *             (a cooperative launch; under stream capture a kernel node that the library
- *             adds to the capturing graph itself, see rtn_native_lstm2_capture_report).  Where the device's registers hold
+ *             (an ordinary launch behind an occupancy check, ordered with the library's others of the
+ *             device; under stream capture a kernel node that the library adds to the capturing graph
+ *             itself, see rtn_native_lstm2_capture_report).  Where the device's registers hold
  *             the recurrent weights (the usual case) every workgroup keeps its slice of W
  *             in registers and the workgroups hand the hidden state over through a ring
  *             of buffers in the workspace that validates itself (a word that still holds
  *             the "not yet written" pattern is read again): no barrier and no flags.
- *             Small layers need no other workgroup: each takes four rows through all steps
+ *             Small layers need no other workgroup: each takes one row, or four, through all steps
  *             by itself.  Wider layers keep W in the registers and the LDS of the whole device
  *             (calls with frames enough to pay for loading it) or, where it fits, in LDS alone
  *             with a flag wait between the steps.  Every wait is bounded: when one expires the
@@ -136,7 +137,7 @@ int rtn_native_lstm2_fwd_status(const void* workspace, void* hip_stream);
  * directions of a bidirectional layer (one op call with step=+1 and one with step=-1 on the same
  * frames, returnn/tf/layers/rec.py:1229-1270), or the same layer of several streams.  Each element
  * holds the arguments of one rtn_native_lstm2_fwd call and gets exactly that call's results.  When
- * the device can hold the persistent kernel of all of them at once, they run in ONE cooperative
+ * the device can hold the persistent kernel of all of them at once, they run in ONE
  * launch and hide each other's exchange latency; otherwise they are enqueued back to back.
  * `workspace` holds `count` equal slices, slice k for call k;
  * rtn_native_lstm2_fwd_multi_workspace_bytes(count, ...) gives the total (a slice can be larger than a single
@@ -230,11 +231,12 @@ int rtn_mfma_issue_probe(int32_t count, int64_t T, int32_t B, int32_t n, int32_t
  *
  * Element type `dtype` for W y0 Y H DY DX Dy0; c0 C i Dd Dc0 DW are float32.  Where the shape allows (n a multiple of
  * 16, a wavefront's share of 16 rows of W fits its registers, all workgroups fit on the device) ONE persistent
- * cooperative kernel runs all frames: W stays in registers, and the gate derivatives of a frame travel between the
+ * kernel runs all frames: W stays in registers, and the gate derivatives of a frame travel between the
  * workgroups through a ring of 4 frames in the workspace (MFMA operand order, self-validating: a slot is all-ones until
  * written); DX itself is a plain output stream, written once.  Otherwise one launch per visited frame (the MFMA GEMM Dy0 += DX[t'] W^T of the frame processed before,
- * fused with the frame's pointwise part), replayed through a library-owned hipGraph.  The large weight-gradient GEMM
- * (Y^T DX over all frames) is left to rocBLAS, which may allocate its own device workspace on first use.  Under stream
+ * fused with the frame's pointwise part), replayed through a library-owned hipGraph.  The weight gradient
+ * (Y^T DX over all frames) of small layers (up to n = 256 in bf16, 384 in float32) is a kernel of the library's, with room in the workspace for its
+ * slices of the rows; wider layers' is left to rocBLAS, which may allocate its own device workspace on first use.  Under stream
  * capture the kernels (the persistent one as a node of its own, see rtn_native_lstm2_capture_report) and the rocBLAS calls
  * are recorded into the caller's graph (the counterpart of the
  * reference's whole-step graph capture, returnn/torch/util/graph_capture.py); the library's rocBLAS handle (one per host
@@ -254,7 +256,7 @@ size_t rtn_native_lstm2_bwd_workspace_bytes(int64_t T, int32_t B, int32_t n, int
  * bidirectional layer, which the reference runs as two op calls (the gradient of tf/layers/rec.py:1229-1270).  Element k
  * gives what rtn_native_lstm2_bwd gives for the same arguments, up to float32 rounding (the joint launch may split the
  * work differently, which changes the order of the partial sums).  When the persistent kernel can hold all `count`
- * problems on the device at once (count <= 2) they share one cooperative launch, each workgroup taking more values of k
+ * problems on the device at once (count <= 2) they share one launch, each workgroup taking more values of k
  * so that every workgroup still has a CU; otherwise the calls are enqueued one after the other.
  * `workspace`: rtn_native_lstm2_bwd_multi_workspace_bytes(); call k uses the k-th equal slice of it, and
  * rtn_native_lstm2_fwd_status(slice k, stream) reports an expired bounded wait of that problem.
@@ -461,7 +463,8 @@ const char* rtn_native_lstm2_bwd_plan_text(void);
  */
 void rtn_native_lstm2_reload_env(void);
 
-/* ABI version of this header: 15. */
+/* ABI version of this header: 18.  (The structs of calls grow at their end: a caller built against an older header passes shorter ones and has to
+ * be built again, which a look at this number tells it.) */
 int rtn_native_lstm2_abi_version(void);
 
 #ifdef __cplusplus

@@ -282,7 +282,7 @@ __global__ void k_convert_from_f32(const float* src, void* dst, long long count)
 
 
 // ---------------------------------------------------------------------------------------------------------------
-// Persistent gradient kernel: all frames in one cooperative launch, W on chip for the whole call.
+// Persistent gradient kernel: all frames in one launch, W on chip for the whole call.  (Groups of up to 8 rows on one XCD each: k_lstm2_bwd_local.)
 //
 //  * decomposition: `groups` batch groups of up to 16 rows; inside a group, workgroup r owns 16*MT values of k: the
 //    rows k of W (A operand of  d_h[b,k] = sum_j DX[b,j] W[k,j],  16*MT x 4n values, in registers for the whole call:

@@ -43,7 +43,8 @@ __host__ __device__ constexpr DualLds dual_lds(int es, int MT) {
 // of one group woven into the other's MFMAs left the hand-over exposed: 842 us against 690.)
 // SPREAD: groups over all XCDs, for layers of 1024 < n <= 2048, which no XCD holds.  There a step alone is mostly hand-over (of 7400 clocks
 // of 32 rows of n = 2048 the matrix cores had 1400): n = 2048, B = 64, T = 64 4.3 us per step of both, 5.7 in turns; n = 1280, B = 90 3.8, 9.5 in the
-// three turns that two tiles of rows per workgroup made.
+// three turns that two tiles of rows per workgroup made.  What is left of it, 8800 clocks per step of both: MFMAs 2050, vector instructions 2100, 3200 with an
+// instruction waiting for its turn, 2000 with none to issue (all 256 registers are taken, and 12 more in scratch).
 // The order of additions is that of k_lstm2_regw: the same bits.
 template <typename AT, int MT, int KS, bool SPREAD>
 __global__ __launch_bounds__(kWgThreads) void k_lstm2_dual(const Lstm2Multi multi) {

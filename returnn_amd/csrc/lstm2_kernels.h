@@ -431,7 +431,7 @@ __global__ void k_step_generic(Lstm2Params p, int s) {
 // and publishes its new hidden value in B-operand order for everybody's next step.
 //
 // s_begin/s_end: steps run by this launch.  With s_end - s_begin > 1 the launch must be
-// co-resident (cooperative launch): steps are separated by a flag wait, bounded by
+// co-resident (the host asks the occupancy first): steps are separated by a flag wait, bounded by
 // timeout_ticks; an expired wait sets status[0] and every later wait returns at once,
 // so the grid always drains.
 // ---------------------------------------------------------------------------------------------

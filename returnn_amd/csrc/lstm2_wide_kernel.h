@@ -10,9 +10,9 @@ namespace rtn {
 
 // ---------------------------------------------------------------------------------------------
 // W of n = 4096 in bf16 is 128 MB: 512 KB for each of the 256 CUs, which have 512 KB of registers and 160 KB of LDS.
-// Launches per step read W from memory every step (22.6 us at 6 TB/s); here a turn reads it once, and a step takes 4.6 us: T = 200,
-// B = 16 4.58 ms as launches per step, 0.97 now, 0.05 of it for the packing.  What bounds a step: the matrix cores are busy for
-// 2048 of its 10 800 clocks, vector instructions issue in 1700, and half of the clocks a wavefront waits for memory -- the
+// Launches per step read W from memory every step (22.6 us at 6 TB/s); here a turn reads it once, and a step takes 4.5 us: T = 200,
+// B = 16 4.58 ms as launches per step, 0.95 now, 0.05 of it for the packing.  What bounds a step: the matrix cores are busy for
+// 2048 of its 10 600 clocks, vector instructions issue in 1700, and half of the clocks a wavefront waits for memory -- the
 // two hops of h.  (More of h in flight, 14 loads per wavefront instead of 8, in smaller chunks: 5 % slower.  What a chunk
 // waits for is the last workgroup that brings its part over.)  (Fewer frames than pay for a turn's load of W run as launches per step: wide_turns_us in the host code.)
 //
@@ -227,9 +227,11 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_wide(const Lstm2Params p) 
   fetch(0);
   take();
   RTN_TRACE_DECL
-  // float32, two tiles of cells and one of rows: a delay that adapts, from 4 units on.  us per step in 1200 steps of n = 1722, 2 rows: none 6.16, fixed at 4
-  // 6.12, adapting 6.05 (from 20 on, which costs 120 steps 6.67 instead of 6.52 with none); the other float32 builds lose by it: n = 2048, 32 rows 10.95 / 11.19,
-  // n = 2816, 16 rows 10.93 / 11.16.
+  // float32, two tiles of cells and one of rows (1024 < n <= 2048, up to 16 rows): a delay that adapts, from 4 units on.  us per step without / with
+  // it: 1, 2, 4 and 8 rows of n = 1088, 1280, 1536, 1722 and 2048, 120 and 1200 steps, all 1.4 ... 2.9 % less with it (n = 1722, 2 rows 6.20 / 6.05; n = 2048,
+  // 8 rows 6.61 / 6.51 in 120 steps); 16 rows 0 ... 2.9 % less (n = 1088 6.69 / 6.52), n = 1280 in 1200 steps 6.66 / 6.82.  (Fixed at 4 units 6.12 where it takes
+  // 6.05; from 20 units on, 120 steps of n = 1722 take 6.67.)  The other float32 builds lose by it or are level: 32 rows of n = 1280, 1722, 2048 10.99 / 11.17,
+  // 11.03 / 11.19, 11.03 / 11.19; n = 2304, 2 and 16 rows 10.14 / 10.11, 10.84 / 10.98; n = 2816 10.25 / 10.22, 11.04 / 11.18.
   constexpr bool kAdapts = sizeof(AT) == 4 && MT == 2 && NT == 1;
   int delay = 4;
   for (int s = 0; s < nsteps; ++s) {
@@ -237,8 +239,8 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_wide(const Lstm2Params p) 
     // ---- bring this workgroup's part of h_s over
     {
       // (No delay in front of the first read, as the kernels whose CUs read all of h across the XCDs have it: a repeat is 4 KB per CU and
-      // costs the others nothing.  us per step without / with one that adapts: n = 4096, 16 rows 4.85 / 5.05, one row 5.18 / 5.63; n = 2560, 16 rows 4.01 / 4.45,
-      // 32 rows 6.05 / 6.43.  In float32 one of the builds gains by one: see kAdapts.)
+      // costs the others nothing.  us per step of 600 without / with one that adapts: n = 4096, 16 rows 4.41 / 4.51, one row 3.71 / 3.78; n = 2560, 16 rows 3.73 / 3.83,
+      // 32 rows 5.74 / 5.87.  In float32 one of the builds gains by one: see kAdapts.)
       if constexpr (kAdapts)
         if (s > 0)
           for (int k = 0; k < delay; ++k) __builtin_amdgcn_s_sleep(1);

@@ -17,10 +17,11 @@ namespace rtn {
 // four neighbouring columns per lane one load of 16 bytes (8 in bf16, widened: the products are exact) is the operand of four tiles, whose columns are then
 // 4 apart: tile t has columns 4 i + t.  Four rows are 2 loads for 16 MFMAs of 32 clocks, no LDS, no transposition.  The four wavefronts take
 // every fourth four rows and add their tiles through LDS.  A slice's workgroups are on one XCD (slice = id % slices), whose L2 they share.
-// Bound by the float32 matrix rate from n = 256 on (26 GFLOP at n = 256, T B = 49 750: 172 us at 152 TFLOP/s), below by the two launches.
+// Bound by the float32 matrix rate from n = 256 on (26 GFLOP at n = 256, T B = 49 750: 202 ... 255 us, the matrix cores busy for 95 % of it; the library's
+// best rate, 152 TFLOP/s, would be 172), below by the two launches.
 // Measured (gradient op with the recurrence, us, library / this): float32 n = 128, T = 300, B = 100 804 / 437, n = 256 937 / 662; bf16 n = 64 422 / 333,
-// n = 128 474 / 399, T = 20, B = 4 61 / 40.  Largest error against float64, of the largest element: float32 1.9e-7 ... 4.9e-7 / 0.9e-7 ... 1.5e-7,
-// bf16 inputs 0.9e-7 ... 6.9e-7 / 0.7e-7 ... 1.3e-7.
+// n = 128 474 / 399, T = 20, B = 4 61 / 40.  Largest error against float64, of the largest element, for n = 64 ... 384 and 80 ... 50 000 rows: float32 7e-7 ...
+// 31e-7 / 1.3e-7 ... 8.3e-7, bf16 inputs 0.9e-7 ... 16e-7 / 0.9e-7 ... 4.1e-7.
 // ---------------------------------------------------------------------------------------------------------------
 constexpr int kWeightTile = 64;       // columns of A and of B per workgroup
 constexpr int kWeightAhead = 4;       // steps of 16 rows whose loads are in flight together
@@ -158,7 +159,7 @@ __global__ __launch_bounds__(kWgThreads) void k_weight_grad(const WeightGradArgs
 // out = A^T B of few rows (a[0], b[0]), plus what is in part if the call says so: the last frame's share y0^T dx0 of a wide layer's gradient, whose
 // long product is the library's, and the conversion to the parameter's type, in one pass over DW for all directions.  Every wavefront has a tile of
 // 32 x 64 of its own, asks for what is there first, multiplies meanwhile (operands as above, two neighbouring columns of A per lane) and writes 16 bytes
-// (8 in bf16) per lane, 256 (128) of a row together.  Bound by that pass (96 MB at bf16 n = 2048: 20 us) and the float32 matrix rate (14 us at 64
+// (8 in bf16) per lane, 256 (128) of a row together.  Bound by that pass (101 MB at bf16 n = 2048: 20 us) and the float32 matrix rate (14 us at 64
 // rows); 33.5 us, with tiles of 64 x 64 and half the wavefronts 40, with a tile per workgroup, its rows dealt to the wavefronts and added
 // through LDS, 47; library product and conversion 45.  Both directions of float32 n = 500, 40 rows: 8.4 us, 11.1, 8.1 and 14.6.
 template <typename AT, typename OT>

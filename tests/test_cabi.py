@@ -33,6 +33,8 @@ def test_header_symbols_are_exported(cabi):
 
 def test_abi_version(cabi):
     assert cabi.rtn_native_lstm2_abi_version() == lib.EXPECTED_ABI
+    header = open(os.path.join(_root, "include", "rtn_native_lstm2.h")).read()
+    assert re.findall(r"ABI version of this header: (\d+)\.", header) == [str(lib.EXPECTED_ABI)]
 
 
 def test_loader_refuses_another_abi_version(monkeypatch):

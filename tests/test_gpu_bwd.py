@@ -369,8 +369,8 @@ def test_bwd_bounded_wait_expires_cleanly(T, B, n, dtype):
 
 @pytest.mark.parametrize("T,B,n,dtype", [(10, 8, 128, "bf16"), (8, 5, 100, "f32"), (6, 3, 20, "f32")])
 def test_forward_and_gradient_recorded_into_a_callers_graph(T, B, n, dtype):
-    """A training step under stream capture: forward op and gradient op (one launch per frame plus the rocBLAS weight
-    gradient) are recorded into the caller's graph after one eager run (which creates the library's rocBLAS handle).
+    """A training step under stream capture: forward op and gradient op (persistent kernel and weight gradient, or one
+    launch per frame) are recorded into the caller's graph after one eager run (which creates the library's rocBLAS handle).
     The graph is replayed three times with new inputs and eager work in between; every replay must agree with the
     eager gradient op (another decomposition: equal up to rounding) and with the oracle."""
     announce("captured training step", T, B, n, dtype)
