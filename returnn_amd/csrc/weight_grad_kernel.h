@@ -42,11 +42,29 @@ struct WeightGradArgs {
   WeightGradCall call[kMaxWeightCalls];
 };
 
+// Four neighbouring elements, as one load brings them.
+template <typename AT>
+struct FourOf {
+  typedef std::conditional_t<sizeof(AT) == 4, u32x4, u32x2> T;
+  static __device__ __forceinline__ T load(__amdgpu_buffer_rsrc_t rs, unsigned at) {
+    if constexpr (sizeof(AT) == 4)
+      return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b128(rs, at, 0, 0));
+    else
+      return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(rs, at, 0, 0));
+  }
+  static __device__ __forceinline__ float get(T v, int k) {
+    if constexpr (sizeof(AT) == 4)
+      return __builtin_bit_cast(float, (unsigned)v[k]);
+    else
+      return __builtin_bit_cast(float, k & 1 ? v[k >> 1] & 0xFFFF0000u : v[k >> 1] << 16);
+  }
+};
+
 // ANY: n, and the distance between the rows of B, need not be multiples of 4: B comes in and the result goes out by element.
 template <typename AT, bool ANY>
 __global__ __launch_bounds__(kWgThreads) void k_weight_grad(const WeightGradArgs args) {
   constexpr int ES = (int)sizeof(AT);
-  typedef std::conditional_t<ES == 4, u32x4, u32x2> Quad4;  // four neighbouring elements
+  typedef typename FourOf<AT>::T Quad4;
   __shared__ f32x4 red[kWaves][16][64];
   const WeightGradCall& q = args.call[blockIdx.y];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), kg = lane >> 4, i = lane & 15;
@@ -67,18 +85,6 @@ __global__ __launch_bounds__(kWgThreads) void k_weight_grad(const WeightGradArgs
   }
   unsigned at_a = m0 + 4 * i < args.m ? (4 * wave + kg) * pitch_a + (m0 + 4 * i) * ES : kNoColumn, at_b = n0 + 4 * i < args.n ? (4 * wave + kg) * pitch_b + (n0 + 4 * i) * ES : kNoColumn;
   const unsigned step_a = 4 * kWaves * pitch_a, step_b = 4 * kWaves * pitch_b;
-  auto load = [](__amdgpu_buffer_rsrc_t rs, unsigned at) {
-    if constexpr (ES == 4)
-      return __builtin_bit_cast(Quad4, __builtin_amdgcn_raw_buffer_load_b128(rs, at, 0, 0));
-    else
-      return __builtin_bit_cast(Quad4, __builtin_amdgcn_raw_buffer_load_b64(rs, at, 0, 0));
-  };
-  auto element = [](Quad4 v, int k) {
-    if constexpr (ES == 4)
-      return __builtin_bit_cast(float, (unsigned)v[k]);
-    else
-      return __builtin_bit_cast(float, k & 1 ? v[k >> 1] & 0xFFFF0000u : v[k >> 1] << 16);
-  };
   f32x4 acc[4][4];
 #pragma unroll
   for (int a = 0; a < 4; ++a)
@@ -90,7 +96,7 @@ __global__ __launch_bounds__(kWgThreads) void k_weight_grad(const WeightGradArgs
     constexpr int S = decltype(set_tag)::value;
 #pragma unroll
     for (int u = 0; u < kWeightAhead; ++u) {
-      va[S][u] = load(ra, at_a);
+      va[S][u] = FourOf<AT>::load(ra, at_a);
       if constexpr (ANY) {
         unsigned v[4];
 #pragma unroll
@@ -103,7 +109,7 @@ __global__ __launch_bounds__(kWgThreads) void k_weight_grad(const WeightGradArgs
         }
         each[S][u] = u32x4{v[0], v[1], v[2], v[3]};
       } else {
-        vb[S][u] = load(rb, at_b);
+        vb[S][u] = FourOf<AT>::load(rb, at_b);
         at_b += step_b;
       }
       at_a += step_a;
@@ -121,8 +127,8 @@ __global__ __launch_bounds__(kWgThreads) void k_weight_grad(const WeightGradArgs
           if constexpr (ANY)
             right = __builtin_bit_cast(float, ES == 4 ? (unsigned)each[S][u][b] : (unsigned)each[S][u][b] << 16);
           else
-            right = element(vb[S][u], b);
-          acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(element(va[S][u], a), right, acc[a][b], 0, 0, 0);
+            right = FourOf<AT>::get(vb[S][u], b);
+          acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(FourOf<AT>::get(va[S][u], a), right, acc[a][b], 0, 0, 0);
         }
   };
   constexpr int kRows = 4 * kWaves * kWeightAhead;
@@ -165,7 +171,7 @@ __global__ __launch_bounds__(kWgThreads) void k_weight_grad(const WeightGradArgs
 template <typename AT, typename OT>
 __global__ __launch_bounds__(kWgThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_weight_last(const WeightGradArgs args) {
   constexpr int ES = (int)sizeof(AT);
-  typedef std::conditional_t<ES == 4, u32x4, u32x2> Quad4;
+  typedef typename FourOf<AT>::T Quad4;
   typedef std::conditional_t<ES == 4, u32x2, unsigned> Pair;
   const WeightGradCall& q = args.call[blockIdx.y];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), kg = lane >> 4, i = lane & 15;
@@ -184,18 +190,6 @@ __global__ __launch_bounds__(kWgThreads) __attribute__((amdgpu_waves_per_eu(4)))
   __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)q.a[0], 0, rows > 0 ? (rows - 1) * pitch_a + args.m * ES : 0u, kBufFlags);
   __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void*)q.b[0], 0, rows > 0 ? (rows - 1) * pitch_b + args.n * ES : 0u, kBufFlags);
   unsigned at_a = m0 + 2 * i < args.m ? kg * pitch_a + (m0 + 2 * i) * ES : kNoColumn, at_b = col < args.n ? kg * pitch_b + col * ES : kNoColumn;
-  auto load = [](__amdgpu_buffer_rsrc_t rs, unsigned at) {
-    if constexpr (ES == 4)
-      return __builtin_bit_cast(Quad4, __builtin_amdgcn_raw_buffer_load_b128(rs, at, 0, 0));
-    else
-      return __builtin_bit_cast(Quad4, __builtin_amdgcn_raw_buffer_load_b64(rs, at, 0, 0));
-  };
-  auto element = [](Quad4 v, int k) {
-    if constexpr (ES == 4)
-      return __builtin_bit_cast(float, (unsigned)v[k]);
-    else
-      return __builtin_bit_cast(float, k & 1 ? v[k >> 1] & 0xFFFF0000u : v[k >> 1] << 16);
-  };
   auto left = [](Pair v, int k) {
     if constexpr (ES == 4)
       return __builtin_bit_cast(float, (unsigned)v[k]);
@@ -217,7 +211,7 @@ __global__ __launch_bounds__(kWgThreads) __attribute__((amdgpu_waves_per_eu(4)))
         va[S][u] = __builtin_bit_cast(Pair, __builtin_amdgcn_raw_buffer_load_b64(ra, at_a, 0, 0));
       else
         va[S][u] = __builtin_amdgcn_raw_buffer_load_b32(ra, at_a, 0, 0);
-      vb[S][u] = load(rb, at_b);
+      vb[S][u] = FourOf<AT>::load(rb, at_b);
       at_a += 4 * pitch_a;
       at_b += 4 * pitch_b;
     }
@@ -229,7 +223,7 @@ __global__ __launch_bounds__(kWgThreads) __attribute__((amdgpu_waves_per_eu(4)))
 #pragma unroll
       for (int a = 0; a < 2; ++a)
 #pragma unroll
-        for (int b = 0; b < 4; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(left(va[S][u], a), element(vb[S][u], b), acc[a][b], 0, 0, 0);
+        for (int b = 0; b < 4; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(left(va[S][u], a), FourOf<AT>::get(vb[S][u], b), acc[a][b], 0, 0, 0);
   };
   constexpr int kRows = 4 * kWeightAhead;
   fetch(IntTag<0>{});
