@@ -351,7 +351,8 @@ class LSTM(torch.nn.Module):
                 self.bias.zero_()
 
     def weights(self, act: torch.dtype) -> LstmWeights:
-        """The parameters as :func:`lstm` takes them (views; a cast only when the run's type is not the parameters')."""
+        """The parameters as :func:`lstm` takes them (views; a cast only when the run's type is not the parameters').  An override is what the
+        layer computes with, in sequences and in single steps."""
         return LstmWeights(ff=self.ff.to(act).t(), rec=self.rec.to(act), bias=None if self.bias is None else self.bias.to(act))
 
     def frontend_params(self) -> dict:
