@@ -69,7 +69,7 @@ def forward_kernel(plan: str):
     solo = "k_lstm2_solo_row" if "rows_per_group=1 " in plan else "k_lstm2_solo"
     kernel = {"mfma_regw_solo": solo, "mfma_regw_wide": "k_lstm2_wide", "mfma_lds": "k_lstm2_mfma"}.get(name, "k_step_generic")
     if name in ("mfma_regw", "mfma_regw_xcd", "mfma_regw_xcd_half"):
-        kernel = "k_lstm2_dual" if "interleaved=2" in plan else "k_lstm2_regw"
+        kernel = "k_lstm2_dual" if "interleaved=2" in plan else "k_lstm2_sparse" if "product=sparse" in plan else "k_lstm2_regw"
     return kernel, kernel == "k_lstm2_regw"
 
 
@@ -931,7 +931,8 @@ def main():
         return min(a.elapsed_time(b) for a, b in se[1:])
 
     seq_ms = time_probe(cabi.rtn_mfma_sequence_probe) if has_probes else None
-    issue_ms = time_probe(cabi.rtn_mfma_issue_probe) if has_probes else None
+    # (k_lstm2_sparse multiplies in other instructions than the probes do: the matrix cores' rate on the dense ones is a ceiling it can exceed)
+    issue_ms = time_probe(cabi.rtn_mfma_issue_probe) if has_probes or kernel == "k_lstm2_sparse" else None
     issue_clock_mhz = None
     if issue_ms is not None:
         # threads 1 and 2 of every workgroup of the issue probe leave the loop's duration in shader clocks and in ticks

@@ -418,7 +418,8 @@ const char* rtn_last_error(void);
 /* The plan the library would use for this problem, as text
  * ("mode=persistent kernel=mfma_regw mt=2 nt=1 groups=2 wgs_per_group=128 wgs=256 rows_per_group=16
  * launches=1 lds=22176 workspace=...": groups, workgroups and rows per group of one persistent launch, and how many
- * launches in turn take the whole batch; "interleaved=2": two of these turns share a launch; "row_quads=q": the float32
+ * launches in turn take the whole batch; "interleaved=2": two of these turns share a launch; "product=sparse": the product
+ * goes in sparse matrix instructions; "row_quads=q": the float32
  * product goes in q quads of rows; "padded_width=n": of a width that is no multiple of 32); for logs and tests.
  * kernel: mfma_regw (W in registers), _xcd (every batch group on one XCD), _xcd_half (of at most 8 rows), mfma_regw_solo (small
  * layers), mfma_regw_wide (W in registers and LDS of the whole device), mfma_lds, generic.

@@ -53,7 +53,8 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_dual(const Lstm2Multi mult
   using LM = LaneMax<AT>;
   constexpr int KE = E::KE, KM = E::KM, ES = (int)sizeof(AT);
   constexpr int EPT = MT / kWaves, CELLS = 4 * MT, ROWS = 16;
-  static_assert(MT % kWaves == 0, "whole tiles per wavefront in the pointwise part");
+  static_assert(MT == kWaves || MT == 2 * kWaves, "one or two pairs per thread in the pointwise part");
+  typedef AT Cells __attribute__((ext_vector_type(EPT)));  // the thread's cells of a row
   constexpr DualLds L = dual_lds(ES, MT);
   const Lstm2Params p = multi.p[0];
   const int X = multi.xcds, G = p.wgs_per_group;
@@ -79,11 +80,14 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_dual(const Lstm2Multi mult
 
   // Streams, as in k_lstm2_regw; offsets are relative to a group's first row, rows beyond the batch end lie behind the frame.
   constexpr int SEG = CELLS * ES, CPS = SEG / 16, XCH = (ROWS * 4 * CPS + kWgThreads - 1) / kWgThreads;
-  constexpr int YCH = (ROWS * CPS + kWgThreads - 1) / kWgThreads;
-  constexpr int SEGC = CELLS * 4, CCH = (ROWS * (SEGC / 16) + kWgThreads - 1) / kWgThreads;
+  constexpr int SEGC = CELLS * 4;
+  static_assert(ROWS * CPS <= 64 && ROWS * (SEGC / 16) <= 128, "wavefront 0 moves Y, wavefronts 1 and 2 move C");
   typedef Chunk<16> CK;
   const int cell0 = CELLS * r;
-  unsigned xoff[XCH], hoff[XCH], yoff[YCH], coff[CCH], xlds[XCH], ylds[YCH], clds[CCH];
+  unsigned xoff[XCH], hoff[XCH], xlds[XCH];
+  // (a chunk of Y or of C per thread, by wavefront: one load from LDS and one store where one of each left most lanes without any)
+  const bool moves_y = wave == 0;
+  unsigned ycoff = kOobOffset, yclds = 0;
 #pragma unroll
   for (int i = 0; i < XCH; ++i) {
     const int c = tid + kWgThreads * i;
@@ -93,17 +97,14 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_dual(const Lstm2Multi mult
     hoff[i] = there ? (unsigned)(((long long)row * 4 * nc + gate * nc + cell0) * ES + part * 16) : kOobOffset;
     xlds[i] = row < ROWS ? (unsigned)(row * L.x_row + gate * SEG + part * 16) : (unsigned)(ROWS * L.x_row);
   }
-#pragma unroll
-  for (int i = 0; i < YCH; ++i) {
-    const int c = tid + kWgThreads * i, row = c / CPS, part = c % CPS;
-    yoff[i] = row < p.Bg && cell0 + (part + 1) * KE <= nc ? (unsigned)(((long long)row * p.ldY + cell0) * ES + part * 16) : kOobOffset;
-    ylds[i] = (unsigned)(min(row, ROWS - 1) * L.y_row + part * 16);
-  }
-#pragma unroll
-  for (int i = 0; i < CCH; ++i) {
-    const int c = tid + kWgThreads * i, row = c / (SEGC / 16), part = c % (SEGC / 16);
-    coff[i] = row < p.Bg && cell0 + (part + 1) * 4 <= nc ? (unsigned)((row * nc + cell0) * 4 + part * 16) : kOobOffset;
-    clds[i] = (unsigned)(min(row, ROWS - 1) * L.c_row + part * 16);
+  if (moves_y) {
+    const int row = tid / CPS, part = tid % CPS;
+    if (row < p.Bg && cell0 + (part + 1) * KE <= nc) ycoff = (unsigned)(((long long)row * p.ldY + cell0) * ES + part * 16);
+    yclds = L.ys + (unsigned)(min(row, ROWS - 1) * L.y_row + part * 16);
+  } else {
+    const int c = tid - 64, row = c / (SEGC / 16), part = c % (SEGC / 16);
+    if (row < p.Bg && cell0 + (part + 1) * 4 <= nc) ycoff = (unsigned)((row * nc + cell0) * 4 + part * 16);
+    yclds = L.cs + (unsigned)(min(row, ROWS - 1) * L.c_row + part * 16);
   }
   const unsigned moff = tid < p.Bg ? (unsigned)(tid * 4) : kOobOffset;
   const long long frame_x = (long long)p.B * p.ldX * ES, frame_h = (long long)p.B * 4 * nc * ES, frame_y = (long long)p.B * p.ldY * ES,
@@ -113,8 +114,8 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_dual(const Lstm2Multi mult
   const unsigned hx_buf_bytes = (unsigned)((size_t)n * p.Bp * ES);
   __amdgpu_buffer_rsrc_t ring[2];
   const unsigned char *x_at[2], *m_at[2];  // the frame that is fetched next, at the group's first row
-  unsigned char *h_at[2], *y_at[2], *c_at[2];  // the frame whose staged outputs leave next
-  unsigned left_x[2], left_h[2], left_y[2], left_c[2], left_m[2];  // bytes of a frame from the group's first row on (0: no such row)
+  unsigned char *h_at[2], *yc_at[2];  // the frame whose staged outputs leave next
+  unsigned left_x[2], left_h[2], left_yc[2], left_m[2];  // bytes of a frame from the group's first row on (0: no such row)
   unsigned frag[2];  // this lane's fragment of macro step `wave` in a ring buffer; out of range: a row the group does not have
   int rows[2];
 #pragma unroll
@@ -126,17 +127,15 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_dual(const Lstm2Multi mult
     x_at[d] = (const unsigned char*)p.X + t0 * frame_x + bs * p.ldX * ES;
     m_at[d] = (const unsigned char*)p.mask + t0 * frame_m + bs * 4;
     h_at[d] = (unsigned char*)p.H + t0 * frame_h + bs * 4 * nc * ES;
-    y_at[d] = (unsigned char*)p.Y + t0 * frame_y + bs * p.ldY * ES;
-    c_at[d] = (unsigned char*)p.C + t0 * frame_c + bs * nc * 4;
+    yc_at[d] = moves_y ? (unsigned char*)p.Y + t0 * frame_y + bs * p.ldY * ES : (unsigned char*)p.C + t0 * frame_c + bs * nc * 4;
     left_x[d] = (unsigned)(frame_x - bs * p.ldX * ES);
     left_h[d] = (unsigned)(frame_h - bs * 4 * nc * ES);
-    left_y[d] = (unsigned)(frame_y - bs * p.ldY * ES);
-    left_c[d] = (unsigned)(frame_c - bs * nc * 4);
+    left_yc[d] = moves_y ? (unsigned)(frame_y - bs * p.ldY * ES) : (unsigned)(frame_c - bs * nc * 4);
     left_m[d] = (unsigned)(frame_m - bs * 4);
     frag[d] = jl < rows[d] ? (unsigned)(((4 * wave + kg) * p.Bp + jl) * kFragBytes) : kOobOffset;
   }
-  const long long step_x = (long long)p.step * frame_x, step_h = (long long)p.step * frame_h, step_y = (long long)p.step * frame_y,
-                  step_c = (long long)p.step * frame_c, step_m = (long long)p.step * frame_m;
+  const long long step_x = (long long)p.step * frame_x, step_h = (long long)p.step * frame_h, step_yc = (long long)p.step * (moves_y ? frame_y : frame_c),
+                  step_m = (long long)p.step * frame_m;
   CK::T xv[2][XCH];
   float mv[2] = {0.f, 0.f};
   auto fetch = [&](auto set_tag, bool enabled) {  // the next frame of X and the mask into registers
@@ -156,31 +155,23 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_dual(const Lstm2Multi mult
     for (int i = 0; i < XCH; ++i) *(CK::T*)(base + L.xl + xlds[i]) = xv[D][i];
     ((float*)(base + L.ml))[tid < ROWS ? tid : ROWS] = mv[D];
   };
-  CK::T fh[XCH], fy[YCH], fc[CCH];
+  CK::T fh[XCH], fyc;
   auto flush_read = [&](auto set_tag) {  // staged outputs -> registers
     constexpr int D = decltype(set_tag)::value;
     const unsigned char* base = smem + L.red + D * L.set;
 #pragma unroll
     for (int i = 0; i < XCH; ++i) fh[i] = *(const CK::T*)(base + L.hs + xlds[i]);
-#pragma unroll
-    for (int i = 0; i < YCH; ++i) fy[i] = *(const CK::T*)(base + L.ys + ylds[i]);
-#pragma unroll
-    for (int i = 0; i < CCH; ++i) fc[i] = *(const CK::T*)(base + L.cs + clds[i]);
+    fyc = *(const CK::T*)(base + yclds);
   };
   auto flush_write = [&](auto set_tag, bool enabled) {  // ... -> H, Y, C (a frame that does not exist: a buffer of no bytes)
     constexpr int D = decltype(set_tag)::value;
     __amdgpu_buffer_rsrc_t hr = __builtin_amdgcn_make_buffer_rsrc((void*)h_at[D], 0, enabled ? left_h[D] : 0u, kBufFlags);
-    __amdgpu_buffer_rsrc_t yr = __builtin_amdgcn_make_buffer_rsrc((void*)y_at[D], 0, enabled ? left_y[D] : 0u, kBufFlags);
-    __amdgpu_buffer_rsrc_t cr = __builtin_amdgcn_make_buffer_rsrc((void*)c_at[D], 0, enabled ? left_c[D] : 0u, kBufFlags);
+    __amdgpu_buffer_rsrc_t ycr = __builtin_amdgcn_make_buffer_rsrc((void*)yc_at[D], 0, enabled ? left_yc[D] : 0u, kBufFlags);
 #pragma unroll
     for (int i = 0; i < XCH; ++i) CK::store(fh[i], hr, hoff[i]);
-#pragma unroll
-    for (int i = 0; i < YCH; ++i) CK::store(fy[i], yr, yoff[i]);
-#pragma unroll
-    for (int i = 0; i < CCH; ++i) CK::store(fc[i], cr, coff[i]);
+    CK::store(fyc, ycr, ycoff);
     h_at[D] += enabled ? step_h : 0;
-    y_at[D] += enabled ? step_y : 0;
-    c_at[D] += enabled ? step_c : 0;
+    yc_at[D] += enabled ? step_yc : 0;
   };
 
   // W: this wavefront's macro steps of the workgroup's tiles; slots past its share hold zeros and meet the fragment of slot 0.
@@ -195,12 +186,13 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_dual(const Lstm2Multi mult
     }
 
   // The (sequence, cell) pairs of this thread, the same in both groups.
+  // (Two pairs per thread are neighbouring cells: half the accesses to LDS and to the ring, two conversions in one.)
   float c_state[2][EPT], h_prev[2][EPT];
   unsigned e_hoff[EPT], e_cl[EPT];
   const unsigned e_row = (unsigned)jl;
 #pragma unroll
   for (int j = 0; j < EPT; ++j) {
-    const int cl = 4 * (wave + kWaves * j) + kg, cell = cell0 + cl;
+    const int cl = EPT * (kWaves * wave + kg) + j, cell = cell0 + cl;
     e_cl[j] = (unsigned)cl;
     e_hoff[j] = (unsigned)((((cell / KE) * p.Bp + jl) * KE + (cell % KE)) * ES);
 #pragma unroll
@@ -267,34 +259,38 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_dual(const Lstm2Multi mult
       RTN_TRACE_MARK(0)  // wait for h_{s-1}
       // (Vector memory operations of a wavefront end in the order they were issued: with h_{s-1}, asked for behind the stores
       // of this group's step s-1, the re-arming stores of that step have ended too, before anything of step s goes out.)
-      f32x4 acc[MT];
+      Cells x_in[4];
+      const unsigned char* xin = base + L.xl + e_row * L.x_row + e_cl[0] * ES;
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt) acc[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
-      AT x_in[EPT][4];
-      const unsigned char* xin = base + L.xl + e_row * L.x_row;
-#pragma unroll
-      for (int j = 0; j < EPT; ++j)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) x_in[j][q] = *(const AT*)(xin + e_cl[j] * ES + q * SEG);
+      for (int q = 0; q < 4; ++q) x_in[q] = *(const Cells*)(xin + q * SEG);
       const float m = ((const float*)(base + L.ml))[e_row];
       flush_read(set_tag);
       put(IntTag<O>{});
-      flush_write(set_tag, s > 0);
+      if (SPREAD) flush_write(set_tag, s > 0);
       // The other group's hidden state is asked for between the MFMAs of the second half, a load every MT / 2 of them (a CU
       // takes 16 clocks for each of the four wavefronts' loads): it was handed over a quarter of a step before, about the time
       // it takes to be visible on the other CUs.  (n = 1024, B = 256: 669 us for 200 steps; all loads behind the last MFMA 690,
       // behind the barrier 735, behind the gates 797, at the end 852; all in the middle 710, in front of the MFMAs 807.)
       asm volatile("" ::: "memory");
+      // (Two chains of additions per wavefront: four tiles at a time, and a four's partial tiles are added and leave for LDS behind the
+      // next one's MFMAs.)
+      constexpr int CHAINS = two_chains<AT>(KS) ? 2 : 1, GRP = CHAINS == 2 ? 4 : MT;
+      f32x4 acc[GRP][CHAINS];
 #pragma unroll
       for (int i = 0; i < KS * MT; ++i) {
-        const int ks = i / MT, mt = i % MT;
+        const int ks = i / GRP % KS, mt = i / (GRP * KS) * GRP + i % GRP;
         if (!SPREAD && i >= KS * MT / 2 && i % (MT / 2) == 0) {
           __builtin_amdgcn_sched_barrier(0);
           load(IntTag<O>{}, D ? s + 1 : s, i / (MT / 2) - KS);
         }
-        acc[mt] = E::mma(wreg[mt][ks], bf[D % SETS][ks], acc[mt]);
+        if (ks < CHAINS) acc[mt % GRP][ks] = f32x4{0.f, 0.f, 0.f, 0.f};
+        acc[mt % GRP][ks % CHAINS] = E::mma(wreg[mt][ks], bf[D % SETS][ks], acc[mt % GRP][ks % CHAINS]);
         __builtin_amdgcn_sched_group_barrier(0x008, sizeof(AT) == 2 ? 1 : 4, 0);
         __builtin_amdgcn_sched_group_barrier(0x096, 3, 0);
+        if (CHAINS == 2 && ks == KS - 1) {
+          asm("" : "+v"(acc[mt % GRP][0]), "+v"(acc[mt % GRP][CHAINS - 1]));  // (accumulation registers would be copied for the additions)
+          red[D][wave][mt][lane] = acc[mt % GRP][0] + acc[mt % GRP][CHAINS - 1];
+        }
       }
       asm volatile("" ::: "memory");
       __builtin_amdgcn_sched_barrier(0);
@@ -304,8 +300,10 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_dual(const Lstm2Multi mult
       if (SPREAD) issue(IntTag<O>{}, D ? s + 1 : s);
       // The other group's X for the half step after next: behind the loads of h, which would wait for it otherwise.
       fetch(IntTag<O>{}, D ? s + 2 < nsteps : s + 1 < nsteps);
+      if constexpr (CHAINS == 1) {
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt) red[D][wave][mt][lane] = acc[mt];
+        for (int mt = 0; mt < MT; ++mt) red[D][wave][mt][lane] = acc[mt][0];
+      }
       RTN_TRACE_MARK(1)  // MFMAs, streams, partial tiles to LDS
       __syncthreads();
       RTN_TRACE_MARK(2)  // barrier
@@ -315,15 +313,15 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_dual(const Lstm2Multi mult
       for (int j = 0; j < EPT; ++j) {
         f32x4 part[kWaves];
 #pragma unroll
-        for (int w = 0; w < kWaves; ++w) part[w] = red[D][w][wave + kWaves * j][lane];
+        for (int w = 0; w < kWaves; ++w) part[w] = red[D][w][e_cl[j] >> 2][16 * (e_cl[j] & 3) + jl];
         __builtin_amdgcn_sched_barrier(0);
         f32x4 gsum = part[0];
 #pragma unroll
         for (int w = 1; w < kWaves; ++w) gsum += part[w];
-        const float a0 = Act<AT>::tanh(gsum[0] + (float)x_in[j][0]);
-        const float a1 = Act<AT>::sigmoid(gsum[1] + (float)x_in[j][1]);
-        const float a2 = Act<AT>::sigmoid(gsum[2] + (float)x_in[j][2]);
-        const float a3 = Act<AT>::sigmoid(gsum[3] + (float)x_in[j][3]);
+        const float a0 = Act<AT>::tanh(gsum[0] + (float)x_in[0][j]);
+        const float a1 = Act<AT>::sigmoid(gsum[1] + (float)x_in[1][j]);
+        const float a2 = Act<AT>::sigmoid(gsum[2] + (float)x_in[2][j]);
+        const float a3 = Act<AT>::sigmoid(gsum[3] + (float)x_in[3][j]);
         const float om = 1.f - m, pc = c_state[D][j];
         const float c = (pc * a2 + a0 * a1) * m + pc * om;
         const float y = E::round(Act<AT>::tanh(c) * a3 * m);
@@ -336,19 +334,32 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_dual(const Lstm2Multi mult
         y_out[j] = y;
       }
       const unsigned nxt = (unsigned)((s + 1) & (kHxRing - 1)) * hx_buf_bytes, arm = (unsigned)((s + 3) & (kHxRing - 1)) * hx_buf_bytes;
-#pragma unroll
-      for (int j = 0; j < EPT; ++j) SN::template store<AUXS>(ring[D], e_hoff[j] + nxt, h_bits[j]);
-#pragma unroll
-      for (int j = 0; j < EPT; ++j) SN::template store<AUXS>(ring[D], e_hoff[j] + arm, SN::kSentinel);
+      if constexpr (EPT == 2) {
+        __builtin_amdgcn_raw_buffer_store_b32(h_bits[0] | h_bits[EPT - 1] << 16, ring[D], e_hoff[0] + nxt, 0, AUXS);
+        __builtin_amdgcn_raw_buffer_store_b32(0xFFFFFFFFu, ring[D], e_hoff[0] + arm, 0, AUXS);
+      } else {
+        SN::template store<AUXS>(ring[D], e_hoff[0] + nxt, h_bits[0]);
+        SN::template store<AUXS>(ring[D], e_hoff[0] + arm, SN::kSentinel);
+      }
       RTN_TRACE_MARK(3)  // gates, exchange stores
+      // (Staged outputs of the step before leave here, behind everything that the other group's hidden state could wait for.)
+      if (!SPREAD) flush_write(set_tag, s > 0);
+      unsigned char* hq = base + L.hs + e_row * L.x_row + e_cl[0] * ES;
+      Cells v;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+#pragma unroll
+        for (int j = 0; j < EPT; ++j) v[j] = (AT)g_act[j][q];
+        *(Cells*)(hq + q * SEG) = v;
+      }
+      struct __attribute__((aligned(4 * EPT))) { float c[EPT]; } cs;
 #pragma unroll
       for (int j = 0; j < EPT; ++j) {
-        unsigned char* hq = base + L.hs + e_row * L.x_row + e_cl[j] * ES;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) *(AT*)(hq + q * SEG) = (AT)g_act[j][q];
-        *(AT*)(base + L.ys + e_row * L.y_row + e_cl[j] * ES) = (AT)y_out[j];
-        *(float*)(base + L.cs + e_row * L.c_row + e_cl[j] * 4) = c_state[D][j];
+        v[j] = (AT)y_out[j];
+        cs.c[j] = c_state[D][j];
       }
+      *(Cells*)(base + L.ys + e_row * L.y_row + e_cl[0] * ES) = v;
+      *(decltype(cs)*)(base + L.cs + e_row * L.c_row + e_cl[0] * 4) = cs;
       RTN_TRACE_MARK(4)  // staging
     };
     fetch(IntTag<0>{}, true);
@@ -378,10 +389,7 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_dual(const Lstm2Multi mult
   auto finish = [&](auto set_tag) {
     constexpr int D = decltype(set_tag)::value;
     flush_read(set_tag);
-    if (expired) {
-#pragma unroll
-      for (int i = 0; i < YCH; ++i) fy[i] = CK::fill(kNanWords<AT>);
-    }
+    if (expired && moves_y) fyc = CK::fill(kNanWords<AT>);
     flush_write(set_tag, true);
 #pragma unroll
     for (int j = 0; j < EPT; ++j)

@@ -9,6 +9,7 @@
 #include "lstm2_kernels.h"
 #include "lstm2_dual_kernel.h"
 #include "lstm2_solo_kernel.h"
+#include "lstm2_sparse_kernel.h"
 #include "lstm2_wide_kernel.h"
 
 namespace rtn {
@@ -22,6 +23,9 @@ RegwKernel regw_table_bf16_lo(int MT, int NT, int KSMAX, bool half, bool tail);
 RegwKernel regw_table_bf16_hi(int MT, int NT, int KSMAX, bool half, bool tail);
 RegwKernel regw_table_f32_lo(int MT, int NT, int KSMAX, bool half, bool tail);
 RegwKernel regw_table_f32_hi(int MT, int NT, int KSMAX, bool half, bool tail);
+
+// k_lstm2_sparse<MT, KSMAX, TAIL>: bfloat16 groups of up to 8 rows.
+RegwKernel sparse_kernel(int MT, int KSMAX, bool tail);
 
 // Forward kernel for small layers k_lstm2_solo<AT, S, R>: the build for width n (one_row: the one with a row per workgroup, if
 // the width has it); kernel null: none.
@@ -63,6 +67,7 @@ RegwKernel regw_table_f32_quad(int MT, int KSMAX, bool tail, int RQ);
 // rq > 0: the product in quads of rows (float32)
 inline RegwKernel regw_kernel(int dtype, int MT, int NT, int KSMAX, bool half, bool tail, int rq) {
   if (rq > 0) return dtype == 0 && NT == 1 ? regw_table_f32_quad(MT, KSMAX, tail, rq) : nullptr;
+  if (half && dtype == 1 && two_chains<__bf16>(KSMAX)) return sparse_kernel(MT, KSMAX, tail);
   const bool lo = KSMAX <= 4;
   if (dtype == 1 /* RTN_DTYPE_BF16 */) return lo ? regw_table_bf16_lo(MT, NT, KSMAX, half, tail) : regw_table_bf16_hi(MT, NT, KSMAX, half, tail);
   return lo ? regw_table_f32_lo(MT, NT, KSMAX, half, tail) : regw_table_f32_hi(MT, NT, KSMAX, half, tail);

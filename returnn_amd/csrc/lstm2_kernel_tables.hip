@@ -5,7 +5,7 @@
 #include "lstm2_kernel_tables.h"
 
 #ifndef RTN_TABLE_PART
-#error "compile with -DRTN_TABLE_PART=<1..15>"
+#error "compile with -DRTN_TABLE_PART=<1..16>"
 #endif
 
 namespace rtn {
@@ -17,13 +17,14 @@ RegwKernel regw_table(int MT, int NT, int KSMAX, bool half) {
   if (half) {
 #define RTN_CASE(mt, ks) \
   if (MT == mt && NT == 1 && KSMAX == ks) return &k_lstm2_regw<AT, mt, 1, ks, true, TAIL>;
-    if constexpr (HI) {
-      RTN_CASE(2, 8) RTN_CASE(2, 16)
-      RTN_CASE(4, 8)
-      RTN_CASE(8, 8)
-    } else {
-      RTN_CASE(2, 2) RTN_CASE(2, 4)
-      RTN_CASE(4, 2) RTN_CASE(4, 4)
+    if constexpr (HI) { RTN_CASE(2, 16) }
+    if constexpr (sizeof(AT) == 4) {  // (bfloat16: k_lstm2_sparse)
+      if constexpr (HI) {
+        RTN_CASE(2, 8) RTN_CASE(4, 8) RTN_CASE(8, 8)
+      } else {
+        RTN_CASE(2, 2) RTN_CASE(2, 4)
+        RTN_CASE(4, 2) RTN_CASE(4, 4)
+      }
     }
 #undef RTN_CASE
     return nullptr;
@@ -180,8 +181,18 @@ RegwKernel dual_kernel(int MT, int KSMAX, bool local) {
 }
 #elif RTN_TABLE_PART == 15
 BwdRegwKernel bwd_local_table_bf16(int KSB, int MT) { return bwd_local_table<__bf16, 0>(KSB, MT); }
+#elif RTN_TABLE_PART == 16
+RegwKernel sparse_kernel(int MT, int KSMAX, bool tail) {
+#define RTN_CASE(mt, ks) \
+  if (MT == mt && KSMAX == ks) return tail ? &k_lstm2_sparse<mt, ks, true> : &k_lstm2_sparse<mt, ks, false>;
+  RTN_CASE(2, 2) RTN_CASE(2, 4) RTN_CASE(2, 8)
+  RTN_CASE(4, 2) RTN_CASE(4, 4) RTN_CASE(4, 8)
+  RTN_CASE(8, 8)
+#undef RTN_CASE
+  return nullptr;
+}
 #else
-#error "RTN_TABLE_PART must be 1..15"
+#error "RTN_TABLE_PART must be 1..16"
 #endif
 
 }  // namespace rtn

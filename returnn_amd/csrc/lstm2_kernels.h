@@ -21,10 +21,13 @@
 namespace rtn {
 
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
+typedef __attribute__((__vector_size__(2 * sizeof(float)))) float f32x2;
 typedef __attribute__((__vector_size__(4 * sizeof(int)))) int i32x4;
 typedef __attribute__((__vector_size__(4 * sizeof(unsigned)))) unsigned u32x4;
 typedef __attribute__((__vector_size__(2 * sizeof(unsigned)))) unsigned u32x2;
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
+typedef __attribute__((__vector_size__(16 * sizeof(__bf16)))) __bf16 bf16x16;
+typedef __attribute__((__vector_size__(8 * sizeof(int)))) int i32x8;
 typedef u32x4 __attribute__((aligned(2))) u32x4_any;  // 16 bytes at any element's address (rows of odd widths)
 
 constexpr int kWgThreads = 256;  // 4 wavefronts of 64
@@ -168,6 +171,20 @@ __global__ void k_fill_unvisited(Lstm2Params p) {
   }
 }
 
+// Where products in sparse matrix instructions (k_lstm2_sparse) take macro step sm: the macro steps of a wavefront go in pairs, pair
+// P = 4 (sm / 8) + sm % 4 (wavefront sm % 4), of which sm is the first or the second half.
+__host__ __device__ constexpr int sparse_pair(int sm) { return 4 * (sm >> 3) + (sm & 3); }
+__host__ __device__ constexpr int sparse_half(int sm) { return (sm >> 2) & 1; }
+__host__ __device__ constexpr int sparse_pairs(int S) { return 4 * ((S - 1) >> 3) + (S - 8 * ((S - 1) >> 3) < 4 ? S - 8 * ((S - 1) >> 3) : 4); }
+// Row and half in row m of the instruction's result: the two halves of a row in one lane.
+__device__ __forceinline__ int sparse_row(int m) { return 2 * (m >> 2) + (m & 1); }
+__device__ __forceinline__ int sparse_row_half(int m) { return (m >> 1) & 1; }
+// Element (row, cell) of the hidden state in a ring buffer of that kernel: a wavefront's fragment of a pair is 1 KB in the order of its lanes.
+__device__ __forceinline__ unsigned sparse_hx(int row, int cell) {
+  const int sm = cell >> 5;
+  return (unsigned)(((sparse_pair(sm) * 4 + ((cell >> 3) & 3)) * 16 + 4 * (row >> 1) + 2 * sparse_half(sm) + (row & 1)) * 8 + (cell & 7));
+}
+
 // Before the MFMA kernels: clears status and flags, writes y0 into buffer 0 of every group's
 // hidden-state exchange area (in B-operand order) and packs W into A-operand order.
 //
@@ -191,7 +208,8 @@ __device__ __forceinline__ void prepare_mfma(const Lstm2Params& p, int n_flags) 
   for (long long idx = gtid; idx < bn; idx += gsz) {
     const int b = (int)(idx / p.n), c = (int)(idx % p.n);
     const int g = b / p.Bg, bl = b % p.Bg;
-    const long long dst = ((long long)g * p.hx_bufs) * hx_buf + ((long long)(c / KE) * p.Bp + bl) * KE + (c % KE);
+    const long long dst = ((long long)g * p.hx_bufs) * hx_buf +
+                          (p.sparse ? (long long)sparse_hx(bl, c) : ((long long)(c / KE) * p.Bp + bl) * KE + (c % KE));
     ((AT*)p.hx)[dst] = c < p.nc ? ((const AT*)p.y0)[(long long)b * p.nc + c] : (AT)0.f;
   }
   if (p.hx_sentinel) {
@@ -216,6 +234,49 @@ __device__ __forceinline__ void prepare_mfma(const Lstm2Params& p, int n_flags) 
   constexpr int CPS = SEG / 16;
   __shared__ unsigned tile[KM * ROWP / 4];
   const int m_tiles = p.n / 4, m_blocks = (m_tiles + MB - 1) / MB;
+  if constexpr (ES == 2) {
+    if (p.sparse) {
+      // The same with a pair of macro steps interleaved word by word (see k_lstm2_sparse): a block's turn takes the 32 rows
+      // of W that one half of the lane groups of a pair reads, and leaves 2 x 16 bytes for every lane and tile of 16 gate columns.
+      const int NP = sparse_pairs(S);
+      for (int t = (int)blockIdx.x; t < 2 * NP * m_blocks; t += (int)gridDim.x) {
+        const int P = (t % (2 * NP)) >> 1, f0 = t & 1, m0 = t / (2 * NP) * MB;
+        for (int c = (int)threadIdx.x; c < KM * 4 * CPS; c += (int)blockDim.x) {
+          const int part = c % CPS, gate = (c / CPS) % 4, k = c / (4 * CPS);
+          const int cell = 4 * m0 + part * 8, row = KM * (8 * (P >> 2) + (P & 3) + 4 * (k >> 4)) + 8 * (f0 + 2 * ((k >> 3) & 1)) + (k & 7);
+          if (cell < p.n) {
+            u32x4 v = u32x4{0, 0, 0, 0};
+            const AT* src = (const AT*)p.W + (long long)row * 4 * p.nc + gate * p.nc + cell;
+            if (row < p.nc && cell + 8 <= p.nc) {
+              v = *(const u32x4_any*)src;
+            } else if (row < p.nc && cell < p.nc) {
+              struct { AT v[8]; } piece;
+#pragma unroll
+              for (int e = 0; e < 8; ++e) piece.v[e] = cell + e < p.nc ? src[e] : (AT)0.f;
+              v = __builtin_bit_cast(u32x4, piece);
+            }
+            unsigned* dst = tile + (k * ROWP + gate * SEGP + part * 16) / 4;
+            dst[0] = v[0]; dst[1] = v[1]; dst[2] = v[2]; dst[3] = v[3];
+          }
+        }
+        __syncthreads();
+        for (int fi = (int)threadIdx.x; fi < MB * 64; fi += (int)blockDim.x) {
+          const int col = fi & 15, hi = (fi >> 4) & 1, xy = (fi >> 5) & 1, tl = fi >> 6;
+          const int cell = p.sparse >= 16 ? 16 * (tl >> 2) + col : 8 * (tl >> 1) + (col & 7);
+          const int gate = p.sparse >= 16 ? tl & 3 : 2 * (col >> 3) + (tl & 1);
+          if (m0 + tl < m_tiles) {
+            const unsigned char* src = (const unsigned char*)tile + (8 * xy + 4 * hi) * ROWP + gate * SEGP + cell * ES;
+            struct { AT v[8]; } frag;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) frag.v[e] = *(const AT*)(src + (16 * ((e >> 1) & 1) + 2 * (e >> 2) + (e & 1)) * ROWP);
+            *(u32x4*)((AT*)p.Wp + ((((long long)(m0 + tl) * NP + P) * 2 + xy) * 64 + 16 * (2 * f0 + hi) + col) * 8) = __builtin_bit_cast(u32x4, frag);
+          }
+        }
+        __syncthreads();
+      }
+      return;
+    }
+  }
   for (int t = (int)blockIdx.x; t < S * m_blocks; t += (int)gridDim.x) {
     const int sm = t % S, m0 = (t / S) * MB;
     for (int c = (int)threadIdx.x; c < KM * 4 * CPS; c += (int)blockDim.x) {
@@ -478,7 +539,9 @@ __device__ __forceinline__ void wait_flags(const Lstm2Params& p, const unsigned*
   if (p.sync_policy & kAcquireFence) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
 }
 
-template <typename AT, int MT, int NT>
+// TWO: two chains of additions per wavefront, the first over its even macro steps and the second over its odd ones, added at the
+// end: the order of k_lstm2_sparse's products, which every kernel of these widths follows.
+template <typename AT, int MT, int NT, bool TWO>
 __global__ __launch_bounds__(kWgThreads) void k_lstm2_mfma(const Lstm2Params p, const int s_begin, const int s_end) {
   using E = Elem<AT>;
   constexpr int KE = E::KE;
@@ -566,11 +629,14 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_mfma(const Lstm2Params p, 
     if (persist && s > s_begin) wait_flags(p, flags_g, p.wgs_per_group, (unsigned)s, lane);
 
     // Recurrent GEMM: this wave's share of k.
-    f32x4 acc[MT][NT];
+    constexpr int CHAINS = TWO ? 2 : 1;
+    f32x4 acc[MT][NT][CHAINS];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-      for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int q = 0; q < CHAINS; ++q) acc[mt][nt][q] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     const unsigned char* hx_cur = hx_g + (size_t)(s & 1) * hx_buf_bytes;
     __amdgpu_buffer_rsrc_t hx_rs = __builtin_amdgcn_make_buffer_rsrc((void*)hx_cur, 0, 0x7fffffff, kBufFlags);
@@ -603,7 +669,7 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_mfma(const Lstm2Params p, 
           for (int mt = 0; mt < MT; ++mt) {
             const i32x4 af = direct ? afd[u][mt] : Wl[(mt * S + sm) * 64 + lane];
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = E::mma(af, bf[u][nt], acc[mt][nt]);
+            for (int nt = 0; nt < NT; ++nt) acc[mt][nt][u % CHAINS] = E::mma(af, bf[u][nt], acc[mt][nt][u % CHAINS]);
           }
         }
       }
@@ -613,7 +679,7 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_mfma(const Lstm2Params p, 
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-      for (int nt = 0; nt < NT; ++nt) red[(wave * TILES + mt * NT + nt) * 64 + lane] = acc[mt][nt];
+      for (int nt = 0; nt < NT; ++nt) red[(wave * TILES + mt * NT + nt) * 64 + lane] = TWO ? acc[mt][nt][0] + acc[mt][nt][CHAINS - 1] : acc[mt][nt][0];
     __syncthreads();
 
     // Epilogue: gates, cell update, mask; publish the new hidden value first (critical path).
@@ -963,10 +1029,16 @@ __device__ __forceinline__ void quad_macro_step(const i32x4 (&wbits)[MT], const 
 // results are the same bits.  What comes out is gate by gate in the lanes of a quad, and is transposed there.
 // (n = 512, groups of 8 rows on one XCD: 2048 clocks of MFMAs per step instead of 4096, which is what makes the XCD-local
 // plan the better one in float32.)
+// TWO (bf16, up to 8 macro steps per wavefront): two chains of additions per wavefront, over its even and its odd macro steps, as
+// k_lstm2_sparse makes them.
+template <typename AT>
+__host__ __device__ constexpr bool two_chains(int KSMAX) { return sizeof(AT) == 2 && KSMAX <= 8; }
 template <typename AT, int MT, int NT, int KSMAX, bool HALF = false, bool TAIL = false, int RQ = 0>
 __global__ __launch_bounds__(kWgThreads) void k_lstm2_regw(const Lstm2Multi multi) {
   constexpr bool QUAD = RQ > 0;
   static_assert(!QUAD || (sizeof(AT) == 4 && NT == 1 && MT % 4 == 0 && RQ <= 4), "quads of rows: float32, one batch tile, whole blocks of 64 columns");
+  constexpr bool TWO = !QUAD && two_chains<AT>(KSMAX);
+  static_assert(!(TWO && HALF), "groups of up to 8 rows at these widths: k_lstm2_sparse");
   static_assert(!HALF || (NT == 1 && MT % 2 == 0), "half-tile mapping: one batch tile, an even number of cell tiles");
   // Which of the launch's problems and which (group, rank) this workgroup works on (uniform over the workgroup).
   int which, g, r;
@@ -1386,7 +1458,7 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_regw(const Lstm2Multi mult
       // accumulator: columns 0-7 collect tile 2u, columns 8-15 tile 2u+1 (the other tile contributes exact zeros, so
       // every sum is bit for bit what a tile of its own would hold).  Half the accumulators, half the partial tiles
       // through LDS -- written by all 64 lanes, in the very lane order the pointwise part reads them in.
-      constexpr int NACC = QUAD ? TILES : PAIRED ? MT / 2 : MT;
+      constexpr int NACC = TWO ? 1 : QUAD ? TILES : PAIRED ? MT / 2 : MT;
       f32x4 acc[NACC][NT];
 #pragma unroll
       for (int mt = 0; mt < NACC; ++mt)
@@ -1473,6 +1545,34 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_regw(const Lstm2Multi mult
           __builtin_amdgcn_sched_barrier(0);
           opnd = opnd_next;
         }
+      } else if constexpr (TWO) {
+        // Tiles in groups of up to four, both chains of each; a group's partial tiles are added and leave for LDS behind the next group's MFMAs.
+        flush_read_at(rd_h, rd_y, rd_c);
+        load_gate_inputs(IntTag<1 - PAR>{});
+        put(par_tag);
+        flush_write_at(h_out, y_out_p, c_out, s >= 2);
+        fetch_at(x_next, m_next, s + 4 < nsteps, par_tag);
+        widen_gate_inputs(par_tag);
+        constexpr int GRP = TILES < 4 ? TILES : 4;
+#pragma unroll
+        for (int t0 = 0; t0 < TILES; t0 += GRP) {
+          f32x4 two[GRP][2];
+#pragma unroll
+          for (int i = 0; i < GRP; ++i) two[i][0] = two[i][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int ks = 0; ks < KSMAX; ++ks)
+#pragma unroll
+            for (int i = 0; i < GRP; ++i) {
+              two[i][ks & 1] = E::mma(wreg[(t0 + i) / NT][ks], bf[ks][(t0 + i) % NT], two[i][ks & 1]);
+              __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+              __builtin_amdgcn_sched_group_barrier(0x096, 3, 0);
+            }
+#pragma unroll
+          for (int i = 0; i < GRP; ++i) {
+            asm("" : "+v"(two[i][0]), "+v"(two[i][1]));  // (accumulation registers would be copied for the additions)
+            redbuf[wave][t0 + i][lane] = two[i][0] + two[i][1];
+          }
+        }
       } else {
         flush_read_at(rd_h, rd_y, rd_c);
         load_gate_inputs(IntTag<1 - PAR>{});
@@ -1492,7 +1592,9 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_regw(const Lstm2Multi mult
             }
       }
       h_out += step_h; y_out_p += step_y; c_out += step_c; x_next += step_x; m_next += step_m;
-      if constexpr (PAIRED || QUAD) {
+      if constexpr (TWO) {
+        // (there already)
+      } else if constexpr (PAIRED || QUAD) {
 #pragma unroll
         for (int u = 0; u < NACC; ++u) redbuf[wave][u][lane] = acc[u][0];
       } else if (!HALF || (lane & 8) == 0) {  // (with at most 8 rows only the lanes of rows 0..7 hold columns anybody reads)

@@ -72,6 +72,7 @@ struct Lstm2Params {
   int Bg;             // batch rows per group
   int Bp;             // rows of one hx buffer (= 16*NT)
   int hx_bufs;        // buffers in the hx ring: 2 with the flag barrier, 4 with self-validating data
+  int sparse;         // cells per workgroup where W and h lie as k_lstm2_sparse reads them, else 0
   int hx_sentinel;    // 1: buffers 1.. start filled with the "not yet written" bit pattern (all ones)
   int xcds;           // XCDs assumed for the blockIdx -> (group, rank) mapping
   int exchange;       // register kernel: 0 = normal operation; 3, 4 = measurement aids (see kExNoWait, kExProbe)

@@ -205,6 +205,9 @@ size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 size_t esize(int dtype) { return dtype == RTN_DTYPE_BF16 ? 2 : 4; }
 int round_nt(int nt) { return nt <= 1 ? 1 : (nt <= 2 ? 2 : 4); }
 
+// Lstm2Params::sparse: groups of up to 8 rows whose product goes in sparse matrix instructions (k_lstm2_sparse)
+int sparse_cells(const Plan& pl, int dtype) { return dtype == RTN_DTYPE_BF16 && pl.regw && pl.half && two_chains<__bf16>(pl.KSMAX) ? 4 * pl.MT : 0; }
+
 size_t mfma_lds_bytes(int n, int dtype, int MT, int NT) {
   const int KM = dtype == RTN_DTYPE_BF16 ? 32 : 16;
   return (size_t)MT * (n / KM) * kTileBytes + (size_t)kWaves * MT * NT * kTileBytes;
@@ -500,6 +503,8 @@ bool make_plan_uncached(int64_t T, int B, int n, int dtype, int want_mode, bool 
         // two launches, 669 as one; n = 2048, B = 64, T = 64 362 and 276, n = 1536, B = 40 314 and 246.)
         pl.dual = di.valid && pl.passes > 1 && dtype == RTN_DTYPE_BF16 && chosen.regw && chosen.NT == 1 && dual_kernel(chosen.MT, chosen.KSMAX, chosen.local) &&
                   dual_lds((int)es, chosen.MT).total + 64 <= di.lds_per_wg && !env_long("RTN_LSTM2_NO_DUAL", 0);
+        if (pl.dual) pl.half = false;  // (a last turn of its own reads W as the interleaved ones do)
+        if (sparse_cells(pl, dtype)) pl.lds_bytes = sparse_lds(pl.MT).total;
         persistent_ok = true;
       }
       // Layers beyond the register kernel's widths (n > 2048 in bf16, > 1024 in float32): the wide kernel, which takes the
@@ -596,7 +601,8 @@ bool make_plan_uncached(int64_t T, int B, int n, int dtype, int want_mode, bool 
       off = align_up(off + (size_t)di.xcds * kHxRing * n * pl.Bp * es, 256);
     }
     pl.off_wp = off;
-    off = align_up(off + (size_t)4 * n * n * es, 256);
+    // (pairs of macro steps take the room of two where the second does not exist)
+    off = align_up(off + (sparse_cells(pl, dtype) ? (size_t)n * 2 * kTileBytes / 4 * sparse_pairs(n / 32) : (size_t)4 * n * n * es), 256);
   } else if (pl.kind != kPlanSolo) {
     pl.off_ycarry = off;
     off = align_up(off + (size_t)2 * B * n * es, 256);
@@ -667,10 +673,10 @@ const char* mode_name(int mode) {
 
 typedef void (*MfmaKernel)(const Lstm2Params, const int, const int);
 
-template <typename AT>
+template <typename AT, bool TWO>
 MfmaKernel mfma_kernel_for(int MT, int NT) {
 #define RTN_CASE(mt, nt) \
-  if (MT == mt && NT == nt) return &k_lstm2_mfma<AT, mt, nt>;
+  if (MT == mt && NT == nt) return &k_lstm2_mfma<AT, mt, nt, TWO>;
   RTN_CASE(1, 1) RTN_CASE(1, 2) RTN_CASE(1, 4)
   RTN_CASE(2, 1) RTN_CASE(2, 2) RTN_CASE(2, 4)
   RTN_CASE(4, 1) RTN_CASE(4, 2) RTN_CASE(4, 4)
@@ -678,8 +684,10 @@ MfmaKernel mfma_kernel_for(int MT, int NT) {
   return nullptr;
 }
 
-MfmaKernel mfma_kernel(int dtype, int MT, int NT) {
-  return dtype == RTN_DTYPE_BF16 ? mfma_kernel_for<__bf16>(MT, NT) : mfma_kernel_for<float>(MT, NT);
+// (up to 8 macro steps per wavefront in bf16: the order of additions of the register kernel's builds for these widths)
+MfmaKernel mfma_kernel(int dtype, int n, int MT, int NT) {
+  if (dtype != RTN_DTYPE_BF16) return mfma_kernel_for<float, false>(MT, NT);
+  return two_chains<__bf16>((n / Elem<__bf16>::KM + kWaves - 1) / kWaves) ? mfma_kernel_for<__bf16, true>(MT, NT) : mfma_kernel_for<__bf16, false>(MT, NT);
 }
 
 // Kernels that use more than the default LDS limit need the limit raised once per device.
@@ -894,7 +902,7 @@ int replay_graph(const std::string& shape_key, const void* block, size_t bytes, 
 
 int launch_steps(const Lstm2Params& p, const Plan& pl, int dtype, LaunchSink& sink) {
   if (pl.kind == kPlanMfma) {
-    MfmaKernel k = mfma_kernel(dtype, pl.MT, pl.NT);
+    MfmaKernel k = mfma_kernel(dtype, p.n, pl.MT, pl.NT);
     const dim3 grid(pl.groups * pl.wgs_per_group), block(kWgThreads);
     for (int s = 0; s < p.nsteps; ++s) {
       const int rc = enqueue(sink, k, grid, block, pl.lds_bytes, p, s, s + 1);
@@ -1262,7 +1270,7 @@ int settle_fwd_plan(int count, int64_t T, int B, int nc, int n, int dtype, int m
   if (!make_plan(T, B, n, dtype, mode, capturing, &pl, &why, 2, plan_count))
     return fail(RTN_ERR_UNSUPPORTED, "NativeLstm2: persistent mode unavailable for T=%lld B=%d n=%d: %s", (long long)T, B, n, why.c_str());
   for (int attempt = 0; pl.kind == kPlanMfma && pl.mode == RTN_MODE_PERSISTENT; ++attempt) {
-    *pk = pl.wide ? (const void*)pl.wide_build.kernel : pl.regw ? (const void*)regw_kernel(dtype, pl.MT, pl.NT, pl.KSMAX, pl.half, nc % (int)(std::min<size_t>(16, 4 * pl.MT * esize(dtype)) / esize(dtype)) != 0, pl.rq) : (const void*)mfma_kernel(dtype, pl.MT, pl.NT);
+    *pk = pl.wide ? (const void*)pl.wide_build.kernel : pl.regw ? (const void*)regw_kernel(dtype, pl.MT, pl.NT, pl.KSMAX, pl.half, nc % (int)(std::min<size_t>(16, 4 * pl.MT * esize(dtype)) / esize(dtype)) != 0, pl.rq) : (const void*)mfma_kernel(dtype, n, pl.MT, pl.NT);
     if (!*pk) return fail(RTN_ERR_UNSUPPORTED, "NativeLstm2: no kernel for mt=%d nt=%d ks=%d", pl.MT, pl.NT, pl.KSMAX);
     if ((rc = ensure_lds_limit(*pk, pl.lds_bytes)) != RTN_OK) return rc;
     const int wgs = pl.regw || pl.wide ? pl.grid : pl.groups * pl.wgs_per_group;
@@ -1333,6 +1341,7 @@ int fill_fwd_params(const rtn_lstm2_call& c, const Plan& pl, bool persistent, un
   p.op_flags = op_flags;
   p.w_direct = (!persistent && pl.kind == kPlanMfma && pl.w_direct) ? 1 : 0;
   p.hx_bufs = kHxRing;
+  p.sparse = sparse_cells(pl, dtype);
   p.hx_sentinel = pl.regw || pl.wide ? 1 : 0;
   p.exchange = (int)env_long("RTN_LSTM2_EXCHANGE", 0);
   if (p.exchange != kExNoWait) p.exchange = kExDevice;  // no-wait: a timing aid, results invalid (status 2)
@@ -1340,7 +1349,7 @@ int fill_fwd_params(const rtn_lstm2_call& c, const Plan& pl, bool persistent, un
   // come back incomplete and cost a second round trip, so it is held back, and the kernel adapts the delay.  Within an
   // XCD the delay is a fixed one (tuned on MI355X over n = 64 ... 1024 and 1 ... 16 rows per group: the best fixed
   // delay is within 2 % of these four everywhere, and 4 % to 13 % ahead of the adaptive one).
-  p.poll_delay = (int)std::max<long>(0, std::min<long>(64, env_long("RTN_LSTM2_POLL_DELAY", pl.local ? (pl.Bg > 8 ? 10 : (dtype != RTN_DTYPE_BF16 ? 5 : (pl.MT >= 8 ? 6 : 3))) : 20)));
+  p.poll_delay = (int)std::max<long>(0, std::min<long>(64, env_long("RTN_LSTM2_POLL_DELAY", pl.local ? (pl.Bg > 8 ? 10 : (dtype != RTN_DTYPE_BF16 || pl.MT >= 8 ? 5 : 3)) : 20)));
   {
     long dec = env_long("RTN_LSTM2_DELAY_DEC", 8);  // steps per unit of downward adaptation: a power of two
     int mask = 0;
@@ -1451,7 +1460,7 @@ int fwd_calls(const rtn_lstm2_call* calls, int count, int64_t T, int32_t B, int3
     }
     if (pl.kind == kPlanMfma) {
       if (!pk) {
-        MfmaKernel mk = mfma_kernel(dtype, pl.MT, pl.NT);
+        MfmaKernel mk = mfma_kernel(dtype, np, pl.MT, pl.NT);
         if (!mk) return fail(RTN_ERR_UNSUPPORTED, "NativeLstm2: no kernel for mt=%d nt=%d", pl.MT, pl.NT);
         rc = ensure_lds_limit((const void*)mk, pl.lds_bytes);
         if (rc != RTN_OK) return rc;
@@ -1877,6 +1886,7 @@ const char* rtn_native_lstm2_describe_multi_plan(int32_t count, int64_t T, int32
              (count > 1 || n != n_asked) ? workspace_each(count, T, B, n_asked, dtype, mode) : pl.total);
     if (pl.dual) snprintf(buf + strlen(buf), sizeof(buf) - strlen(buf), " interleaved=2");
     if (pl.rq) snprintf(buf + strlen(buf), sizeof(buf) - strlen(buf), " row_quads=%d", pl.rq);
+    if (sparse_cells(pl, dtype)) snprintf(buf + strlen(buf), sizeof(buf) - strlen(buf), " product=sparse");
     if (n != n_asked) snprintf(buf + strlen(buf), sizeof(buf) - strlen(buf), " padded_width=%d", n);
     if (pl.off_trace) snprintf(buf + strlen(buf), sizeof(buf) - strlen(buf), " trace_offset=%zu", pl.off_trace);
     g_plan_text = buf;
