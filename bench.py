@@ -69,7 +69,7 @@ def forward_kernel(plan: str):
     solo = "k_lstm2_solo_row" if "rows_per_group=1 " in plan else "k_lstm2_solo"
     kernel = {"mfma_regw_solo": solo, "mfma_regw_wide": "k_lstm2_wide", "mfma_lds": "k_lstm2_mfma"}.get(name, "k_step_generic")
     if name in ("mfma_regw", "mfma_regw_xcd", "mfma_regw_xcd_half"):
-        kernel = "k_lstm2_dual" if "interleaved=2" in plan else "k_lstm2_sparse" if "product=sparse" in plan else "k_lstm2_regw"
+        kernel = "k_lstm2_dual" if "interleaved=2" in plan else "k_lstm2_regw"
     return kernel, kernel == "k_lstm2_regw"
 
 
@@ -893,6 +893,8 @@ def main():
     call_ms = sum(a.elapsed_time(b) for a, b in events) / len(events)
     plan = lib.describe_multi_plan(2 if fused else 1, T, B, n, dt_code, mode)
     kernel, has_probes = forward_kernel(plan)
+    if "product=sparse" in plan:  # (the form of the register kernel for groups of up to 8 rows in bf16)
+        kernel, has_probes = "k_lstm2_sparse", False
 
     # The latency of one hand-over of values between CUs (device-scope store -> load), measured live with the library's
     # probe: a lower bound of a time step of any kernel that keeps W spread over CUs.
