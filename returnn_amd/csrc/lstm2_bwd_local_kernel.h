@@ -2,6 +2,7 @@
 #pragma once
 
 #include "lstm2_bwd_kernels.h"
+#include "lstm2_sparse_kernel.h"
 
 namespace rtn {
 
@@ -9,29 +10,28 @@ namespace rtn {
 // The frame of k_lstm2_bwd_regw (decomposition, exchange ring, bounded waits and who re-arms what are described there), for
 // groups whose ring of 8 rows per frame stays in one XCD's L2.  A workgroup is 4 wavefronts with W in their registers; one
 // load takes two macro steps of the contraction at once (lanes of rows 0-7 step 2a, lanes of rows 8-15 step 2a + 1, 1 KB of
-// consecutive memory), which is right in columns 0-7 as the B operand of W's fragment 2a and in columns 8-15 as that of
-// fragment 2a + 1.
+// consecutive memory).  In bfloat16 that is the stored operand of a sparse matrix instruction as it is (see k_lstm2_sparse): rows 8-15 name
+// the places of step 2a + 1 among W's interleaved words, and one instruction per tile takes both steps.  The two halves of a row's sum are added across the lanes.
 //
 // What bounds a frame is the ring: the stores are visible to the XCD after some 500 clocks, then every CU takes in all of the
 // group's derivatives (64 KB at n = 1024: 550 clocks to issue the loads and 950 until the last is back, measured with nothing
-// else on the way), then 1024 clocks of MFMAs per wavefront, the sum over the wavefronts and the gates.  So
+// else on the way), then 512 clocks of MFMAs per wavefront, the sum over the wavefronts and the gates.  So
 //  * the product begins on the first half of the registers and checks the second behind the first one's MFMAs;
 //  * the MFMAs of a register go to accumulators of their own with a fence behind (left alone, the scheduler lines up those of
-//    two accumulators, each waiting for the one before the last: 1790 clocks for 64 MFMAs of 16);
+//    one accumulator, each waiting for the one before);
 //  * nothing that does not need the errors is left to the time between the product and the stores: the gates' factors are
 //    worked out while the stores travel;
 //  * derivatives go from the lanes that have them to the ring, 8 or 16 bytes each (see Quad), without LDS and a barrier;
-//  * a frame's inputs are asked for behind most of the MFMAs, when the other wavefronts' ring loads are through: 4 loads
-//    per pair instead of 8 and behind the MFMAs instead of in front of them is 0.2 of 2.5 us per frame.
+//  * inputs are asked for behind most of the MFMAs, when the other wavefronts' ring loads are through, and for four frames at once (kBwdBatch).
 // Nothing in the loop may be reached with loads in flight that the frame's own path does not have there: the compiler then waits
 // for all of them, and a fetch from memory that was just asked for stood between the sum and the stores (0.15 us of a frame).
-//
-// Of 4600 clocks per wavefront and frame (n = 1024, both directions of 32 rows; k_lstm2_bwd_regw 4980) the MFMAs are 1024, vector instructions 1110, 770
-// go by with an instruction waiting for its turn and 2080 with none to issue: the ring.
 //
 // Measured (gradient op, us per frame with the weight gradient, k_lstm2_bwd_regw / this): bf16 n = 1024, both directions of 32 rows
 // 2.74 / 2.50, one direction 2.60 / 2.31; n = 768 2.51 / 2.23; n = 512, 32 rows 1.90 / 1.64; n = 128, both of 8 rows 1.74 / 1.38; n = 64,
 // 4 rows 1.42 / 1.03; float32 n = 500, both of 40 rows 5.26 / 4.89; n = 256, 100 rows 3.69 / 3.09; n = 64, both of 32 rows 1.56 / 1.25.
+// With the sparse product and inputs in turns (whole backward pass of a layer over 500 frames, us before / now): bf16 n = 1024, both directions of 32 rows
+// 1580 / 1525, n = 768, 32 rows 1272 / 1168, n = 512, both of 32 rows 1124 / 1025, n = 256, both of 16 rows 767 / 690, n = 128, 8 rows 608 / 554; float32
+// n = 256, 30 rows 869 / 859, n = 64, 8 rows 546 / 525.
 // ---------------------------------------------------------------------------------------------------------------
 
 // Four elements (8 or 16 bytes) per lane, and the transposition of 4 x 4 of them over the lanes of a quad: with it lane i, which
@@ -72,6 +72,12 @@ struct Quad<__bf16> {
   static __device__ __forceinline__ void store(T v, __amdgpu_buffer_rsrc_t rs, unsigned off, unsigned soff = 0) { __builtin_amdgcn_raw_buffer_store_b64(v, rs, off, soff, AUX); }
   static __device__ __forceinline__ T ones() { return T{~0u, ~0u}; }
 };
+
+// Frames whose inputs are asked for at once, but where a wavefront's share of W is 64 fragments (or 32 in float32), whose ring loads and products take
+// so long that the burst is felt more than a frame's loads are: us per frame one at a time / four: bf16 n = 512, both directions of 32 rows 1.75 / 1.45,
+// n = 1024 2.52 / 2.63, float32 n = 500, both of 40 rows 5.21 / 5.25, n = 256, 30 rows 1.36 / 1.33.  (A load from memory holds up the ring loads
+// behind it in the CU's first-level cache: see k_lstm2_sparse.)
+constexpr int kBwdBatch = 4;
 
 // RQ > 0 (float32, groups of at most 4 RQ rows): the product in v_mfma_f32_4x4x1, whose 16 blocks of 4 rows x 4 values of k are
 // 4 rows x 64 products in 8 clocks, the rate of the 16x16x4 without its padding of 8 rows to 16.  With MT tiles of 16 values
@@ -114,7 +120,7 @@ __device__ __forceinline__ f32x4 lane_pair_sum(f32x4 a, f32x4 b) {
 template <typename AT, int KSB, int MT, int RQ = 0>
 __global__ __launch_bounds__(kWgThreads) void k_lstm2_bwd_local(const Lstm2BwdMulti multi) {
   constexpr bool QUAD = RQ > 0;
-  static_assert(KSB % 2 == 0 && (!QUAD || (sizeof(AT) == 4 && RQ <= 2)), "paired loads; quads of rows: float32");
+  static_assert(KSB % 2 == 0 && QUAD == (sizeof(AT) == 4) && RQ <= 2, "paired loads; float32 in quads of rows, bfloat16 in sparse matrix instructions");
   // tiles whose pairs a thread keeps: with at most 8 rows the threads of the upper 8 row slots take every other tile (SPLIT)
   constexpr bool SPLIT = MT % 2 == 0;
   constexpr int PT = SPLIT ? MT / 2 : MT;
@@ -130,14 +136,11 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_bwd_local(const Lstm2BwdMu
   using LM = LaneMax<AT>;
   constexpr int KE = E::KE, KM = E::KM, ES = (int)sizeof(AT);
   const Lstm2BwdParams& p = q.p;
-  // partial tiles of the wavefronts; a lane group's 16 entries are followed by 4 unused ones, so that the four groups of
-  // k that a wavefront's threads read together start 16 banks apart (without the gap they met in the same banks)
-  constexpr int kRedGroup = 20;
-  // (two copies: no barrier between the sums of one frame and the partial tiles of the next)
+  // partial tiles of the wavefronts, in two copies: no barrier between the sums of one frame and the partial tiles of the next
   // (QUAD: [quad][k] of 4 rows each, two quads of up to 32 values of k in one 64 lanes wide slot)
-  // (else: two tiles in one slot, see gemm)
-  constexpr int kRedSlots = QUAD ? (MT == 4 ? RQ : 1) : (MT + 1) / 2, kRedLanes = QUAD ? 64 : 4 * kRedGroup;
-  __shared__ f32x4 red2[2][kWaves][kRedSlots][kRedLanes];
+  // (else: [tile][quad of rows][k] of 4 rows each, two tiles in one slot, see gemm)
+  constexpr int kRedSlots = QUAD ? (MT == 4 ? RQ : 1) : (MT + 1) / 2;
+  __shared__ f32x4 red2[2][kWaves][kRedSlots][64];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = p.n, n4 = 4 * n;
@@ -164,7 +167,25 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_bwd_local(const Lstm2BwdMu
   // KSB runs on this kernel.
   const int ksb = q.ksb;
   const int ks_here = max(0, min(ksb, n4 / KM - ksb * wave));  // uniform over the wavefront
-  i32x4 wreg[MT][KSB];
+  // (bfloat16: a register pair of macro steps 2a and 2a + 1 is interleaved word by word, see k_lstm2_sparse; lane group g holds elements
+  // 8 (g / 2) + 4 (g % 2) ... + 3 and those 16 further of either.)
+  i32x4 wreg[QUAD ? MT : 1][KSB];
+  i32x8 wsp[QUAD ? 1 : MT][KSB / 2];
+  if constexpr (!QUAD) {
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      const AT* Wr = (const AT*)p.W + (size_t)(k0 + 16 * mt + (lane & 15)) * n4 + (size_t)KM * ksb * wave + 4 * (lane >> 4);
+#pragma unroll
+      for (int a = 0; a < KSB / 2; ++a) {
+        i32x2 v[2][2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int h = 0; h < 2; ++h) v[u][h] = 2 * a + u < ks_here ? *(const i32x2*)(Wr + KM * (2 * a + u) + 16 * h) : i32x2{0, 0};
+        wsp[mt][a] = i32x8{v[0][0][0], v[1][0][0], v[0][0][1], v[1][0][1], v[0][1][0], v[1][1][0], v[0][1][1], v[1][1][1]};
+      }
+    }
+  } else {
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
     // (QUAD: register i of a lane is k = lane % (16 MT), elements 4 (i + MT * (lane / (16 MT))) ... + 3 of the macro step)
@@ -173,9 +194,11 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_bwd_local(const Lstm2BwdMu
 #pragma unroll
     for (int ks = 0; ks < KSB; ++ks) wreg[mt][ks] = (ks < ks_here) ? *(const i32x4*)(Wr + (size_t)KM * ks) : i32x4{0, 0, 0, 0};
   }
+  }
   // Byte offsets of this lane's B fragments inside a ring frame.  The lanes of rows the group lacks and slots without a share
   // carry an out-of-range one: 0 comes back and no memory is touched.  (The offsets stay in registers over the frames, which measured faster than
   // instruction immediates.)
+  const int places = (lane & 8) ? (int)0xEEEEEEEE : 0x44444444;  // rows 8-15 hold the odd macro step's values: places 2 and 3 of every four
   constexpr int NB = KSB / 2;                   // registers of B fragments
   constexpr int PARTS = NB >= 8 ? 2 : 1, N1 = NB / PARTS;  // ... checked and multiplied in parts (four of them: no faster)
   i32x4 bf[NB];
@@ -214,9 +237,9 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_bwd_local(const Lstm2BwdMu
 #pragma unroll
     for (int gq = 0; gq < 4; ++gq) dx0[j][gq] = 0.f;
   }
-  // where a pair's element of the summed tile is: tile element D[kl][bl] sits in lane (kl/4)*16 + bl, component kl%4
-  const int red_lane = QUAD ? (RQ == 2 ? (bl >> 2) & 1 : 0) * (MT == 4 ? 64 : 32) + kl : (kl >> 2) * kRedGroup + (bl & 7);  // (+ 8 for an odd tile)
-  const int red_comp = QUAD ? bl & 3 : kl & 3;
+  // where a pair's element of the summed tile is
+  const int red_lane = QUAD ? (RQ == 2 ? (bl >> 2) & 1 : 0) * (MT == 4 ? 64 : 32) + kl : 16 * ((bl >> 2) & 1) + kl;  // (+ 32 for an odd tile)
+  const int red_comp = bl & 3;
 
   // Inputs of a frame: asked for behind the MFMAs of the product two frames before it, turned into the factors of the pointwise
   // part a frame before it.  (A wavefront's loads count as returned in the order they were issued: asked for in front of the
@@ -227,9 +250,10 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_bwd_local(const Lstm2BwdMu
   typedef Quad<AT> QD;
   const unsigned quad_sel = QD::selector(lane);
   typedef std::conditional_t<ES == 2, unsigned short, unsigned> Raw;
-  typename QD::T nx_gates[PT];
-  Raw nx_dy[PT];
-  unsigned nx_pc[PT], nx_m;
+  constexpr int FB = MT * KSB >= 64 || (QUAD && KSB >= 32) ? 1 : kBwdBatch;
+  typename QD::T nx_gates[FB][PT];
+  Raw nx_dy[FB][PT];
+  unsigned nx_pc[FB][PT], nx_m[FB];
   BwdCell<AT> cell[PT];
   float in_dy[PT], in_m;
   auto widen = [](Raw raw) {
@@ -248,56 +272,56 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_bwd_local(const Lstm2BwdMu
   const bool h0_cell = (p.op_flags & kOpH0IsCell) != 0;
   // The frame that is fetched next: its ordinal, and where it lies in H, DY, C (the frame before it) and the mask.
   int nf = 0;
-  bool cell_from_h = false;  // what nx_pc holds
+  bool cell_from_h[FB];  // what nx_pc holds
   const long long stride_h = -(long long)q.step * frame_bytes, stride_dy = -(long long)q.step * dy_frame_bytes, stride_c = -(long long)q.step * bn * 4,
                   stride_m = -(long long)q.step * p.B * 4;
   const unsigned char *at_h = (const unsigned char*)p.H + q.t_end * (long long)frame_bytes, *at_dy = (const unsigned char*)p.DY + q.t_end * (long long)dy_frame_bytes,
                       *at_c = (const unsigned char*)p.C + (q.t_end - q.step) * bn * 4, *at_m = (const unsigned char*)(p.mask + q.t_end * p.B);
-  auto fetch_gates = [&]() {
+  auto fetch_gates = [&](int slot) {
     __amdgpu_buffer_rsrc_t rs_h = __builtin_amdgcn_make_buffer_rsrc((void*)at_h, 0, nf < q.nframes ? frame_bytes : 0u, kBufFlags);
 #pragma unroll
-    for (int j = 0; j < PT; ++j) nx_gates[j] = QD::load(rs_h, off_gates[j]);
+    for (int j = 0; j < PT; ++j) nx_gates[slot][j] = QD::load(rs_h, off_gates[j]);
     at_h += stride_h;
   };
-  auto fetch_errors = [&]() {
+  auto fetch_errors = [&](int slot) {
     const bool there = nf < q.nframes;
     __amdgpu_buffer_rsrc_t rs_dy = __builtin_amdgcn_make_buffer_rsrc((void*)at_dy, 0, there ? dy_frame_bytes : 0u, kBufFlags);
     __amdgpu_buffer_rsrc_t rs_m = __builtin_amdgcn_make_buffer_rsrc((void*)at_m, 0, there ? (unsigned)(p.B * 4) : 0u, kBufFlags);
 #pragma unroll
-    for (int j = 0; j < PT; ++j) nx_dy[j] = load(rs_dy, off_dy[j], 0);
-    nx_m = __builtin_amdgcn_raw_buffer_load_b32(rs_m, m_off, 0, 0);
+    for (int j = 0; j < PT; ++j) nx_dy[slot][j] = load(rs_dy, off_dy[j], 0);
+    nx_m[slot] = __builtin_amdgcn_raw_buffer_load_b32(rs_m, m_off, 0, 0);
     at_dy += stride_dy;
     at_m += stride_m;
   };
   // The cell state of the frame before: C, c0 in front of the first frame, or (kOpH0IsCell) the word of H that holds the pair's
   // element of its first block.  (Behind fetch_gates: at_h is the frame before the one fetched.)
-  auto fetch_cell = [&]() {
+  auto fetch_cell = [&](int slot) {
     const bool first = q.nframes - nf == 1;
-    cell_from_h = h0_cell && !first;
-    const unsigned char* src = first ? (const unsigned char*)p.c0 : cell_from_h ? at_h : at_c;
-    __amdgpu_buffer_rsrc_t rs_c = __builtin_amdgcn_make_buffer_rsrc((void*)src, 0, nf >= q.nframes ? 0u : cell_from_h ? frame_bytes : (unsigned)(bn * 4), kBufFlags);
+    const bool from_h = cell_from_h[slot] = h0_cell && !first;
+    const unsigned char* src = first ? (const unsigned char*)p.c0 : from_h ? at_h : at_c;
+    __amdgpu_buffer_rsrc_t rs_c = __builtin_amdgcn_make_buffer_rsrc((void*)src, 0, nf >= q.nframes ? 0u : from_h ? frame_bytes : (unsigned)(bn * 4), kBufFlags);
 #pragma unroll
-    for (int j = 0; j < PT; ++j) nx_pc[j] = __builtin_amdgcn_raw_buffer_load_b32(rs_c, cell_from_h ? off_h0[j] & ~3u : off_c[j], 0, 0);
+    for (int j = 0; j < PT; ++j) nx_pc[slot][j] = __builtin_amdgcn_raw_buffer_load_b32(rs_c, from_h ? off_h0[j] & ~3u : off_c[j], 0, 0);
     at_c += stride_c;
     ++nf;
   };
-  auto fetch = [&]() {
-    fetch_gates();
-    fetch_errors();
-    fetch_cell();
+  auto fetch = [&](int slot) {
+    fetch_gates(slot);
+    fetch_errors(slot);
+    fetch_cell(slot);
   };
-  auto take_next = [&]() {  // what was asked for becomes the current frame's inputs
+  auto take_next = [&](int slot) {  // what was asked for becomes the current frame's inputs
 #pragma unroll
     for (int j = 0; j < PT; ++j) {
-      const typename QD::T g = QD::transpose(nx_gates[j], lane, quad_sel);
-      float before = __builtin_bit_cast(float, nx_pc[j]);
+      const typename QD::T g = QD::transpose(nx_gates[slot][j], lane, quad_sel);
+      float before = __builtin_bit_cast(float, nx_pc[slot][j]);
       if constexpr (ES == 2)
-        if (cell_from_h) before = __builtin_bit_cast(float, off_h0[j] & 2 ? nx_pc[j] & 0xFFFF0000u : nx_pc[j] << 16);
+        if (cell_from_h[slot]) before = __builtin_bit_cast(float, off_h0[j] & 2 ? nx_pc[slot][j] & 0xFFFF0000u : nx_pc[slot][j] << 16);
       cell[j] = BwdCell<AT>::of(p.op_flags, QD::get(g, 0), QD::get(g, 1), QD::get(g, 2), QD::get(g, 3), before);
-      in_dy[j] = widen(nx_dy[j]);
+      in_dy[j] = widen(nx_dy[slot][j]);
       asm volatile("" : "+v"(in_dy[j]));
     }
-    in_m = __builtin_bit_cast(float, nx_m);
+    in_m = __builtin_bit_cast(float, nx_m[slot]);
     // (of registers of their own from here on: used as the loads left them, they would be waited for behind the next fetch)
     asm volatile("" : "+v"(in_m));
   };
@@ -355,12 +379,22 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_bwd_local(const Lstm2BwdMu
     } while (marked(from));
     return spins;
   };
-  auto gemm = [&](int t) {  // t: ordinal of the frame whose derivatives go through the product
+  auto gemm = [&](int t, auto ph_tag) {  // t: ordinal of the frame whose derivatives go through the product
+    constexpr int PH = decltype(ph_tag)::value;  // (t + 1) % FB
     RTN_BTRACE_MARK(4)  // pointwise tail, delay, first read, factors of the next frame
     auto& red = red2[t & 1];
     // (at least four accumulators keep the MFMA pipeline full)
-    constexpr int NACC = MT == 1 ? 4 : 2;
+    constexpr int NACC = MT >= 4 ? 1 : 4 / MT;
     f32x4 part[MT][NACC];
+    if constexpr (!QUAD) {  // (cleared here, where nothing else is to do)
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int a = 0; a < NACC; ++a) {
+          part[mt][a] = f32x4{0.f, 0.f, 0.f, 0.f};
+          asm volatile("" : "+v"(part[mt][a]));
+        }
+    }
     f32x4 quad[QUAD ? RQ : 1][2];
     unsigned spins = 0;
     if (marked(0)) spins = read_again(t, 0);
@@ -373,16 +407,12 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_bwd_local(const Lstm2BwdMu
     // W lives in accumulation registers where it is at most half of that file: the B fragments fill up to half of
     // the ordinary registers, and a matrix instruction reads an A operand from either file (without this the compiler
     // parks part of W there anyway and copies four registers back in front of every MFMA, which halves the MFMA rate).
-    if constexpr (MT * KSB <= 32) {
+    if constexpr (QUAD && MT * KSB <= 32) {
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
         for (int ks = 0; ks < KSB; ++ks) asm volatile("" : "+a"(wreg[mt][ks]));
     }
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-      for (int a = 0; a < NACC; ++a) part[mt][a] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int q = 0; q < (QUAD ? RQ : 1); ++q) quad[q][0] = quad[q][1] = f32x4{0.f, 0.f, 0.f, 0.f};
     // Register by register, with a fence behind and a piece of the other work -- the check of the next part, the fetch of the
@@ -395,9 +425,21 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_bwd_local(const Lstm2BwdMu
 #pragma unroll
         for (int w = 0; w < 4; ++w) m2[w] = 0;
       }
-      if (a == (NB >= 3 ? NB - 3 : 0)) fetch_gates();
-      if (a == (NB >= 3 ? NB - 2 : NB - 1)) fetch_errors();
-      if (a == NB - 1) fetch_cell();
+      if (PH == 1 % FB) {
+        if (a == (NB >= 3 ? NB - 3 : 0)) {
+#pragma unroll
+          for (int i = 1; i <= FB / 2; ++i) fetch((PH + i) % FB);
+        }
+        if (FB > 1 && a == NB - 1) {
+#pragma unroll
+          for (int i = FB / 2 + 1; i <= FB; ++i) fetch((PH + i) % FB);
+        }
+        if (FB == 1) {
+          if (a == (NB >= 3 ? NB - 3 : 0)) fetch_gates(0);
+          if (a == (NB >= 3 ? NB - 2 : NB - 1)) fetch_errors(0);
+          if (a == NB - 1) fetch_cell(0);
+        }
+      }
       if (a + N1 < NB) fold(m2, bf[a + N1]);
       if constexpr (QUAD) {
         i32x4 w0[MT], w1[MT];
@@ -414,14 +456,11 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_bwd_local(const Lstm2BwdMu
         }
       } else {
 #pragma unroll
-        for (int u = 0; u < 2; ++u)  // u = 0: valid in columns 0-7, 1: in columns 8-15
-#pragma unroll
-          for (int mt = 0; mt < MT; ++mt) {
-            const int acc = NACC == 4 ? 2 * (a & 1) + u : u;
-            part[mt][acc] = E::mma(wreg[mt][2 * a + u], bf[a], part[mt][acc]);
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x096, 2, 0);
-          }
+        for (int mt = 0; mt < MT; ++mt) {
+          part[mt][a % NACC] = smfmac(bf[a], wsp[mt][a], part[mt][a % NACC], places);
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x096, 3, 0);
+        }
       }
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -438,32 +477,19 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_bwd_local(const Lstm2BwdMu
         red[wave][0][lane] = acc;
       }
     } else {
-      // Columns 0-7 of the first accumulator and 8-15 of the second are the two halves of a tile's sum.  An even tile's end up
-      // in the lanes of columns 0-7, the odd tile's beside it in those of columns 8-15: one slot for both, half the reads.
+      // Rows 0-7 of a result are the sums over the even macro steps, 8-15 those over the odd ones, 32 lanes away: added, an even tile's sums
+      // end up in the lower lanes and the odd tile's beside it in the upper ones, one slot for both.
 #pragma unroll
       for (int slot = 0; slot < kRedSlots; ++slot) {
-        const int m0 = 2 * slot, m1 = 2 * slot + 1 < MT ? 2 * slot + 1 : m0;
-        f32x4 lo[2], hi[2];
+        f32x4 tile[2];
 #pragma unroll
         for (int k = 0; k < 2; ++k) {
-          const int mt = k ? m1 : m0;
-          lo[k] = part[mt][0];
-          hi[k] = part[mt][1];
-          if constexpr (NACC == 4) {
-            lo[k] += part[mt][NACC - 2];
-            hi[k] += part[mt][NACC - 1];
-          }
-        }
-        f32x4 acc;
-        const bool upper = (lane & 8) != 0;
+          const int mt = 2 * slot + k < MT ? 2 * slot + k : 2 * slot;
+          tile[k] = part[mt][0];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          // row_shl:8 / row_shr:8: from the lane 8 above / below inside a group of 16 (lanes without a source take 0)
-          const float even = lo[0][r] + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, (float)hi[0][r]), 0x108, 0xF, 0xF, true));
-          const float odd = hi[1][r] + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, (float)lo[1][r]), 0x118, 0xF, 0xF, true));
-          acc[r] = MT > 1 && upper ? odd : even;
+          for (int a = 1; a < NACC; ++a) tile[k] += part[mt][a];
         }
-        red[wave][slot][(lane >> 4) * kRedGroup + (lane & 15)] = acc;
+        red[wave][slot][lane] = lane_pair_sum<32>(tile[0], tile[1]);
       }
     }
     RTN_BTRACE_MARK(1)  // MFMA, partial tiles to LDS
@@ -478,7 +504,7 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_bwd_local(const Lstm2BwdMu
         if constexpr (QUAD)
           sum += ((const float*)(&red[w][0][0] + red_lane + 16 * mt))[red_comp];
         else
-          sum += ((const float*)&red[w][mt >> 1][red_lane + 8 * (mt & 1)])[red_comp];
+          sum += ((const float*)&red[w][mt >> 1][red_lane + 32 * (mt & 1)])[red_comp];
       }
       dyw[j] += sum;
     }
@@ -497,7 +523,7 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_bwd_local(const Lstm2BwdMu
     at_dx += stride_dx;
     asm volatile("" : "+s"(to), "+s"(arm), "+s"(dx_to));  // scalar arithmetic ahead of the wait, not behind it
   };
-  auto pointwise = [&](int f) {
+  auto pointwise = [&](int f, int next) {
     __amdgpu_buffer_rsrc_t rs_dx = __builtin_amdgcn_make_buffer_rsrc(dx_to, 0, dx_frame_bytes, kBufFlags);
     // pointwise part of frame t (returnn/native_op.py:1123-1180); the derivatives out as soon as they are there, then all-ones
     // into the slot that was read two frames ago, DX, and what the errors carry on
@@ -533,22 +559,35 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_bwd_local(const Lstm2BwdMu
     RTN_BTRACE_MARK(5)  // pointwise part, stores
     // while the derivatives travel: what the next frame's pointwise part can do without the errors, and after the delay the
     // first read of this frame's ring slot
-    take_next();
+    take_next(next);
     if (!aborted)
       for (int d = 0; d < delay; ++d) __builtin_amdgcn_s_sleep(1);
     issue(f);
   };
-  fetch();
-  take_next();
-  fetch();
+  fetch(0);
+  take_next(0);
+  fetch(1 % FB);
   aim(0);
   // (The first frame in front of the loop: a way into its pointwise part without a product in front, on which loads are still
   // in flight, made every frame wait for the inputs it had just asked for.)
-  if (F > 0) pointwise(0);
-  for (int f = 1; f <= F; ++f) {
-    aim(f);
-    gemm(f - 1);
-    if (f < F) pointwise(f);
+  if (F > 0) pointwise(0, 1 % FB);
+  for (int f = 1; f <= F; f += FB) {
+    auto frame = [&](int f, auto ph_tag) {
+      aim(f);
+      gemm(f - 1, ph_tag);
+      if (f < F) pointwise(f, (decltype(ph_tag)::value + 1) % FB);
+    };
+    frame(f, IntTag<1 % FB>{});
+    if constexpr (FB > 1) {
+      if (f + 1 > F) break;
+      frame(f + 1, IntTag<2 % FB>{});
+    }
+    if constexpr (FB > 2) {
+      if (f + 2 > F) break;
+      frame(f + 2, IntTag<3>{});
+      if (f + 3 > F) break;
+      frame(f + 3, IntTag<0>{});
+    }
   }
   RTN_BTRACE_ADD(7, (unsigned long long)delay)
   RTN_BTRACE_FLUSH()

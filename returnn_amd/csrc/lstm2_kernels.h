@@ -28,6 +28,7 @@ typedef __attribute__((__vector_size__(2 * sizeof(unsigned)))) unsigned u32x2;
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef __attribute__((__vector_size__(16 * sizeof(__bf16)))) __bf16 bf16x16;
 typedef __attribute__((__vector_size__(8 * sizeof(int)))) int i32x8;
+typedef __attribute__((__vector_size__(2 * sizeof(int)))) int i32x2;
 typedef u32x4 __attribute__((aligned(2))) u32x4_any;  // 16 bytes at any element's address (rows of odd widths)
 
 constexpr int kWgThreads = 256;  // 4 wavefronts of 64

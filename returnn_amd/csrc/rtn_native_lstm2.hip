@@ -2523,12 +2523,12 @@ int bwd_launch_persistent(const BwdCtx& x, const BwdChoice& ch, const BwdLayout&
     q.ksb = ch.ksb;
     // A fixed delay between a frame's stores and the read of its ring slot for groups of up to 8 rows inside an XCD, as in the forward
     // kernel; the others adapt.  In the kernel for such groups what passes of it with the next frame's factors is not counted.  (us per frame
-    // of the gradient op at 0 / 2 / 4 / 8 / 12 units: bf16 n = 1024, two of 32 rows, 2.52 / 2.52 / 2.50 / 2.58 / 2.67; n = 512, two of 16 rows,
-    // 1.76 / 1.76 / 1.74 / 1.71 / 1.74; float32 n = 500, two of 40 rows, 4.90 / 4.90 / 4.94 / 5.03 / 5.14.  The general kernel: 2.77 ms for a
+    // of a layer's gradient at 3 / 5 / 7 / 8 units: bf16 n = 1024, two of 32 rows, 3.07 / 3.05 / 3.07 / 3.08; n = 512 the same, 2.15 / 2.11 / 2.05 / 2.06; n = 256, 100 rows,
+    // 1.89 / 1.85 / 1.83 / 1.82, n = 128, 8 rows, 1.14 / 1.12 / 1.10 / 1.12; at 0 / 2 / 4 / 8 / 12 float32 n = 500, two of 40 rows, 4.90 / 4.90 / 4.94 / 5.03 / 5.14.  The general kernel: 2.77 ms for a
     // layer at 10 units, 2.82 adaptive, 2.87 / 2.86 at 4 / 16.)
     const bool one_pair = ch.rows_per_group <= 8 && ((ch.tiles + ch.waves / 4 - 1) / (ch.waves / 4)) % 2 == 0;
     const bool fixed_delay = ch.one_xcd_kernel || (ch.local && one_pair);
-    const long first_delay = !fixed_delay ? 20 : !ch.one_xcd_kernel ? 10 : x.dtype == RTN_DTYPE_BF16 && n > 256 ? (ch.tiles == 1 ? 8 : 4) : 2;
+    const long first_delay = !fixed_delay ? 20 : !ch.one_xcd_kernel ? 10 : x.dtype != RTN_DTYPE_BF16 ? 2 : n > 256 && ch.tiles > 1 ? 4 : 7;
     q.poll_delay = (int)std::max<long>(0, std::min<long>(64, env_long("RTN_LSTM2_BWD_POLL_DELAY", first_delay)));
     q.delay_inc = (int)std::max<long>(0, std::min<long>(16, env_long("RTN_LSTM2_BWD_DELAY_INC", fixed_delay ? 0 : 2)));
     {
