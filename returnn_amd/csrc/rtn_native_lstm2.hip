@@ -1964,7 +1964,9 @@ int rtn_lstm_step(const void* x, const void* h, const float* c, const void* ff, 
   if (in_dim < 0 || (long long)in_dim * n > 0x7fffffffLL / 16) return fail(RTN_ERR_SHAPE, "LSTM step: bad input dimension %d (n=%d)", in_dim, n);
   if ((long long)B * n == 0) return RTN_OK;
   if (!h || !c || !rec || !y || !h_out || !c_out || (in_dim > 0 && (!x || !ff))) return fail(RTN_ERR_ARG, "LSTM step: null pointer");
-  LstmStepParams p = {x, h, c, ff, rec, bias, y, h_out, c_out, B, in_dim, n};
+  LstmStepParams p = {x, h, c, ff, rec, bias, y, h_out, c_out, B, in_dim, n, 0};
+  const long long ke = 16 / (long long)esize(dtype), largest = std::max<long long>(std::max<long long>(4LL * n * std::max(in_dim, n), (long long)B * std::max(in_dim, n)), 1) * (long long)esize(dtype);
+  p.by_fragments = n % kStepCells == 0 && in_dim % ke == 0 && largest < 0x80000000LL && aligned16(x) && aligned16(h) && aligned16(ff) && aligned16(rec);
   // 16, 32 or 64 rows per workgroup, several shares of the batch beyond that (the weights then come from the L2 again)
   const int NT = B <= 16 ? 1 : (B <= 32 ? 2 : 4);
   const int blocks = (n + kStepCells - 1) / kStepCells;

@@ -10,6 +10,7 @@ import pytest
 
 from returnn_amd import lib
 from _gpu_util import announce, random_problem, run_multi_raw, run_raw
+from test_gpu_bwd import _rel_to_max, _run
 
 pytestmark = pytest.mark.gpu
 
@@ -51,3 +52,15 @@ def test_large_infinite_and_nan_states_stay_in_their_row():
         for name, a, b in zip("YCHd", outs, want):
             assert numpy.array_equal(a, b, equal_nan=True), name
         assert numpy.isfinite(outs[0][:, [0, 2, 4, 5, 7]]).all()
+
+
+# (the frames' inputs come four at a time where a wavefront's share of W is small; the first frame stands in front of the loop)
+@pytest.mark.parametrize("dtype,B,n", [("bf16", 9, 256), ("bf16", 17, 512), ("bf16", 6, 96), ("f32", 7, 128)])
+@pytest.mark.parametrize("T", [1, 2, 3, 4, 5, 6, 7, 9, 10])
+def test_gradients_of_any_number_of_frames(T, dtype, B, n):
+    announce("gradient, inputs in turns", T, B, n, dtype)
+    for start, step in [(0, 1), (0, -2)]:
+        got, want, _ = _run(T, B, n, dtype, start, step, seed=T + n)
+        assert "name=k_lstm2_bwd_local " in lib.bwd_plan_text()
+        for name, a, b in zip(("DX", "DW", "Dy0", "Dc0"), got, want):
+            assert _rel_to_max(a, b) <= (2e-2 if dtype == "bf16" else 2e-5), (name, _rel_to_max(a, b))
