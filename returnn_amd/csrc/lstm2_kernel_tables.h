@@ -38,10 +38,10 @@ SoloBuild solo_kernel(int dtype, int n, bool one_row);
 // k_lstm2_dual<__bf16, MT, KSMAX, !local>: two turns of a large batch in one launch; null if the decomposition has no build.
 RegwKernel dual_kernel(int MT, int KSMAX, bool local);
 
-// Forward kernel for wide layers k_lstm2_wide<AT, MT, NT, KS, LF>.
+// Forward kernel for wide layers k_lstm2_wide<AT, MT, NT, KS, LF, STAGED>.
 typedef void (*WideKernel)(const Lstm2Params);
 struct WideBuild {
-  WideKernel kernel;
+  WideKernel kernel, staged;  // staged: for rows that begin on 16 bytes; null: none
   int dtype, MT, NT, KS, LF;
 };
 // The build for a layer of width n on `cus` CUs and `rows` rows per launch; the last one in the list if rows are more than

@@ -125,13 +125,13 @@ BwdRegwKernel bwd_regw_lds_table_f32(int WV) { return bwd_regw_lds_table<float>(
 // Ascending by the width that MT tiles on 256 CUs and KS macro steps per wavefront take, then by rows.  What bounds NT: W,
 // 4 MT NT accumulator registers and two chunks of h per wavefront in 512 registers.
 WideBuild wide_kernel(int dtype, int n, int cus, int rows) {
-#define RTN_WIDE(at, dt, mt, nt, ks, lf) {&k_lstm2_wide<at, mt, nt, ks, lf>, dt, mt, nt, ks, lf}
+#define RTN_WIDE(at, dt, mt, nt, ks, lf) {&k_lstm2_wide<at, mt, nt, ks, lf, false>, wide_stage_bytes(mt, nt, lf, (int)sizeof(at)) ? &k_lstm2_wide<at, mt, nt, ks, lf, !(lf && sizeof(at) == 4)> : nullptr, dt, mt, nt, ks, lf}
   static const WideBuild builds[] = {
       RTN_WIDE(float, 0, 2, 1, 32, 0), RTN_WIDE(float, 0, 2, 2, 32, 0), RTN_WIDE(float, 0, 3, 1, 44, 36),
       RTN_WIDE(__bf16, 1, 3, 1, 24, 0), RTN_WIDE(__bf16, 1, 3, 2, 24, 0), RTN_WIDE(__bf16, 1, 4, 1, 32, 35),
   };
 #undef RTN_WIDE
-  WideBuild best = {nullptr, 0, 0, 0, 0, 0};
+  WideBuild best = {nullptr, nullptr, 0, 0, 0, 0, 0};
   for (const WideBuild& b : builds) {
     if (b.dtype != dtype) continue;
     const int KM = dtype == 1 ? 32 : 16;

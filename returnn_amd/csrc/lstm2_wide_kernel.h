@@ -10,9 +10,9 @@ namespace rtn {
 
 // ---------------------------------------------------------------------------------------------
 // W of n = 4096 in bf16 is 128 MB: 512 KB for each of the 256 CUs, which have 512 KB of registers and 160 KB of LDS.
-// Launches per step read W from memory every step (22.6 us at 6 TB/s); here a turn reads it once, and a step takes 4.5 us: T = 200,
-// B = 16 4.58 ms as launches per step, 0.95 now, 0.05 of it for the packing.  What bounds a step: the matrix cores are busy for
-// 2048 of its 10 600 clocks, vector instructions issue in 1700, and half of the clocks a wavefront waits for memory -- the
+// Launches per step read W from memory every step (22.6 us at 6 TB/s); here a turn reads it once, and a step takes 4.1 us: T = 200,
+// B = 16 4.58 ms as launches per step, 0.88 now, 0.05 of it for the packing.  What bounds a step: the matrix cores are busy for
+// 2048 of its 9700 clocks, vector instructions issue in 1700, and half of the clocks a wavefront waits for memory -- the
 // two hops of h.  (More of h in flight, 14 loads per wavefront instead of 8, in smaller chunks: 5 % slower.  What a chunk
 // waits for is the last workgroup that brings its part over.)  (Fewer frames than pay for a turn's load of W run as launches per step: wide_turns_us in the host code.)
 //
@@ -45,14 +45,37 @@ constexpr int wide_lds_slot(int MT, int KS, int RF, int ks, int mt) {
   return count;
 }
 
-constexpr unsigned wide_lds_bytes(int MT, int NT, int LF) {
-  return (unsigned)(kWaves * LF * kTileBytes + kWaves * MT * NT * kTileBytes);
+// What a staged step's streams take in LDS: X in, H out of the same places; Y; C.  (0: no such build, see WideStage.)
+constexpr unsigned wide_stage_bytes(int MT, int NT, int LF, int ES) {
+  return LF && ES == 4 ? 0u : (unsigned)(16 * NT * 4 * MT * (4 * ES + ES + 4));
 }
+
+constexpr unsigned wide_lds_bytes(int MT, int NT, int LF, int ES) {
+  return (unsigned)(kWaves * LF * kTileBytes + kWaves * MT * NT * kTileBytes) + wide_stage_bytes(MT, NT, LF, ES);
+}
+
+// The op's streams of a workgroup in pieces of CB bytes of a row: PR pieces of each of X's and H's four blocks and of Y, PC of
+// C.  64 pieces of one stream are a unit, a wavefront's access; the units are dealt to the wavefronts, SL to each at most.
+template <typename AT, int MT, int NT>
+struct WideStage {
+  static constexpr int ES = (int)sizeof(AT), RC = 4 * MT, CB = (RC * ES) % 16 == 0 ? 16 : 8;
+  static constexpr int PR = RC * ES / CB, PC = RC * 4 / CB;
+  static constexpr int UH = NT * PR, UC = (16 * NT * PC + 63) / 64, UY = (16 * NT * PR + 63) / 64;
+  static constexpr int SL = (UH + UC + UY + kWaves - 1) / kWaves;
+  static constexpr int kC = 16 * NT * RC * 4 * ES, kY = kC + 16 * NT * RC * 4;  // where C and Y begin
+};
 
 // Fragments of h (16 bytes) that a workgroup brings over per thread at most: n / KE * 16 NT fragments over G / xcds workgroups.
 constexpr int kWideForward = 2;
 
-template <typename AT, int MT, int NT, int KS, int LF>
+// STAGED: the op's streams go through LDS.  X comes in as up to 16 bytes of a row per thread, H, Y and C leave so; a thread by
+// itself has 2 or 4 bytes of 4 cells next to each other, and every one of the 11 accesses per step touches 16 lines for a few bytes
+// of each.  us per 200 steps without / with it: bf16 n = 4096 with 1, 4 and 16 rows 793 / 778, 805 / 785, 949 / 877, n = 2560 with 16 and 32
+// rows 767 / 696, 1182 / 960; float32 n = 1280 with 16 rows 1356 / 1240, n = 2048 with 3 and 32 rows 1261 / 1258, 2231 / 2103.  (n = 4096, 16 rows
+// without any streams: 823.)  h as one store of 8 or 16 bytes per row of a tile instead of one per cell, the lanes' values brought
+// together first: 871, 697 and 971, 1262, 1282 and 2087; not kept.
+// Where rows may begin anywhere (p.nc < p.n), and in float32 beyond n = 2048, where W leaves no room, pair by pair.
+template <typename AT, int MT, int NT, int KS, int LF, bool STAGED>
 __global__ __launch_bounds__(kWgThreads) void k_lstm2_wide(const Lstm2Params p) {
   using E = Elem<AT>;
   using SN = Sentinel<AT>;
@@ -65,6 +88,9 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_wide(const Lstm2Params p) 
   extern __shared__ __align__(16) unsigned char smem[];
   i32x4* Wl = (i32x4*)smem;                                            // [kWaves][LF][64]
   f32x4* red = (f32x4*)(smem + (size_t)kWaves * LF * kTileBytes);      // [kWaves][TILES][64]
+  using Stage = WideStage<AT, MT, NT>;
+  constexpr int RC = Stage::RC, CB = Stage::CB, SL = Stage::SL;
+  unsigned char* stage = (unsigned char*)(red + kWaves * TILES * 64);  // X and H [4][16 NT][RC], C [16 NT][RC], Y [16 NT][RC]
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = p.n, S = n / KM, nc = p.nc, G = p.wgs_per_group, X = p.xcds;
@@ -135,7 +161,7 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_wide(const Lstm2Params p) 
   __syncthreads();
   const bool one_xcd = s_one_xcd != 0;
 
-  // The op's streams, a pair per thread: gate inputs and mask come in one step ahead, behind the loads of the product; a step's
+  // The op's streams, a pair per thread or (STAGED) a piece of a row: gate inputs and mask come in one step ahead, behind the loads of the product; a step's
   // outputs leave behind the next step's.  Without a branch: pairs and frames that do not exist have offsets beyond any
   // frame.  (With branches the compiler has to wait for these loads and stores, and the
   // trip to memory they take, wherever it waits for a chunk of h.)
@@ -151,6 +177,26 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_wide(const Lstm2Params p) 
   }
   const unsigned frame_x = (unsigned)((size_t)p.B * p.ldX * ES), frame_h = (unsigned)((size_t)p.B * 4 * nc * ES), frame_y = (unsigned)((size_t)p.B * p.ldY * ES),
                  frame_c = (unsigned)(bn * 4), frame_m = (unsigned)(p.B * 4), gate = (unsigned)(nc * ES);  // (gate: from one of a row's four blocks to the next)
+  // A staged unit's stream, and this thread's piece of it: its offset in X's frame (H's units) and in the output's, and where it
+  // is in LDS.
+  using Piece = std::conditional_t<CB == 16, i32x4, i32x2>;
+  unsigned xp_at[SL], op_at[SL], lp_at[SL];
+  Piece xp[SL];
+  if constexpr (STAGED) {
+#pragma unroll
+    for (int i = 0; i < SL; ++i) {
+      const int u = wave + kWaves * i;
+      const bool is_h = u < Stage::UH, is_c = !is_h && u < Stage::UH + Stage::UC;
+      const int k = 64 * (is_h ? u : is_c ? u - Stage::UH : u - Stage::UH - Stage::UC) + lane;  // the piece of the stream
+      const int per_row = is_c ? Stage::PC : Stage::PR, block = k / (16 * NT * per_row), row = k / per_row % (16 * NT);
+      const int in_block = block * nc, cell = 4 * r * MT + k % per_row * (CB / (is_c ? 4 : ES));
+      const bool there = u < Stage::UH + Stage::UC + Stage::UY && block < (is_h ? 4 : 1) && row < rows && cell < nc;
+      const long long at = b_base + row;
+      xp_at[i] = is_h && there ? (unsigned)((at * p.ldX + in_block + cell) * ES) : kOobOffset;
+      op_at[i] = !there ? kOobOffset : is_h ? (unsigned)((at * 4 * nc + in_block + cell) * ES) : is_c ? (unsigned)((at * nc + cell) * 4) : (unsigned)((at * p.ldY + cell) * ES);
+      lp_at[i] = block < (is_h ? 4 : 1) ? (unsigned)((is_h ? 0 : is_c ? Stage::kC : Stage::kY) + k * CB) : 0u;
+    }
+  }
   AT xin[EPT][4], xnext[EPT][4];
   float msk[EPT], mnext[EPT];
   // (frames that do not exist: all offsets beyond; not a buffer of no bytes, whose range check a scalar offset would wrap)
@@ -160,12 +206,25 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_wide(const Lstm2Params p) 
   auto fetch = [&](int s) {
     const bool there = s < nsteps;
     __amdgpu_buffer_rsrc_t xr = frame(p.X, s, frame_x, there), mr = frame(p.mask, s, frame_m, there);
+    if constexpr (STAGED) {
+#pragma unroll
+      for (int i = 0; i < SL; ++i) {
+        if (kWaves * i >= Stage::UH) continue;
+        const unsigned at = there ? xp_at[i] : kOobOffset;
+        if constexpr (CB == 16)
+          xp[i] = __builtin_bit_cast(Piece, __builtin_amdgcn_raw_buffer_load_b128(xr, at, 0, 0));
+        else
+          xp[i] = __builtin_bit_cast(Piece, __builtin_amdgcn_raw_buffer_load_b64(xr, at, 0, 0));
+      }
+    }
 #pragma unroll
     for (int j = 0; j < EPT; ++j) {
       const unsigned at = there ? x_at[j] : kOobOffset;
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        if constexpr (ES == 2)
+        if constexpr (STAGED)
+          continue;
+        else if constexpr (ES == 2)
           xnext[j][q] = __builtin_bit_cast(AT, __builtin_amdgcn_raw_buffer_load_b16(xr, at, q * gate, 0));
         else
           xnext[j][q] = __builtin_bit_cast(AT, __builtin_amdgcn_raw_buffer_load_b32(xr, at, q * gate, 0));
@@ -177,7 +236,7 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_wide(const Lstm2Params p) 
 #pragma unroll
     for (int j = 0; j < EPT; ++j) {
 #pragma unroll
-      for (int q = 0; q < 4; ++q) xin[j][q] = xnext[j][q];
+      for (int q = 0; q < 4 && !STAGED; ++q) xin[j][q] = xnext[j][q];
       msk[j] = mnext[j];
     }
   };
@@ -187,6 +246,20 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_wide(const Lstm2Params p) 
   auto put = [&](int s) {
     const bool there = s >= 0;
     __amdgpu_buffer_rsrc_t hr = frame(p.H, s, frame_h, there), yr = frame(p.Y, s, frame_y, there), cr = frame(p.C, s, frame_c, there);
+    if constexpr (STAGED) {
+#pragma unroll
+      for (int i = 0; i < SL; ++i) {
+        const int u = wave + kWaves * i;
+        const Piece v = *(const Piece*)(stage + lp_at[i]);
+        __amdgpu_buffer_rsrc_t rs = u < Stage::UH ? hr : u < Stage::UH + Stage::UC ? cr : yr;
+        const unsigned at = there ? op_at[i] : kOobOffset;
+        if constexpr (CB == 16)
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), rs, at, 0, 0);
+        else
+          __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), rs, at, 0, 0);
+      }
+      return;
+    }
     auto store = [&](AT v, __amdgpu_buffer_rsrc_t rs, unsigned off, unsigned block) {
       if constexpr (ES == 2)
         __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(unsigned short, v), rs, off, block, 0);
@@ -201,6 +274,15 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_wide(const Lstm2Params p) 
       store(y_out[j], yr, there ? y_at[j] : kOobOffset, 0);
     }
   };
+  // X of the step, in the places that H of the step before has been read from.
+  auto stage_x = [&]() {
+    if constexpr (STAGED) {
+#pragma unroll
+      for (int i = 0; i < SL; ++i)
+        if (wave + kWaves * i < Stage::UH) *(Piece*)(stage + lp_at[i]) = xp[i];
+    }
+  };
+  auto staged_pair = [&](int j) { return (e_b[j] * RC + (e_cell[j] - 4 * r * MT)); };  // a pair's place in a staged block
   // Bookkeeping of one repeated read: false when the wait is over for good.
   unsigned long long t0 = 0;
   auto keep_waiting = [&](unsigned& spins) {
@@ -330,6 +412,7 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_wide(const Lstm2Params p) 
       if (c + NB - 1 < NC) load_chunk(c + NB - 1);
       if (c + NB - 1 == NC - 1 || (NC < NB && c == 0)) {
         put(s - 1);
+        stage_x();
         fetch(s + 1);
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -374,6 +457,12 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_wide(const Lstm2Params p) 
 #pragma unroll
         for (int w = 1; w < kWaves; ++w) gsum += part[w];
         const float m = msk[j];
+        AT* const hs = (AT*)stage + staged_pair(j);  // X's and H's place in the first block
+        constexpr int block = 16 * NT * RC;
+        if constexpr (STAGED) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) xin[j][q] = hs[q * block];
+        }
         const float a0 = Act<AT>::tanh(gsum[0] + (float)xin[j][0]);
         const float a1 = Act<AT>::sigmoid(gsum[1] + (float)xin[j][1]);
         const float a2 = Act<AT>::sigmoid(gsum[2] + (float)xin[j][2]);
@@ -387,6 +476,12 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_wide(const Lstm2Params p) 
         y_out[j] = (AT)y;
         a_out[j][0] = (AT)((p.op_flags & kOpH0IsCell) ? c : a0);
         a_out[j][1] = (AT)a1; a_out[j][2] = (AT)a2; a_out[j][3] = (AT)a3;
+        if constexpr (STAGED) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) hs[q * block] = a_out[j][q];
+          ((float*)(stage + Stage::kC))[staged_pair(j)] = c;
+          ((AT*)(stage + Stage::kY))[staged_pair(j)] = (AT)y;
+        }
         if (e_own[j]) {
           const unsigned ho = (unsigned)((((e_cell[j] / KE) * p.Bp + e_b[j]) * KE + (e_cell[j] % KE)) * ES);
           SN::template store<kAuxDevice>(ring, ho + nxt, SN::bits(hn));
@@ -402,6 +497,7 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_wide(const Lstm2Params p) 
   RTN_TRACE_FLUSH(p, blockIdx.x)
 
   put(nsteps - 1);
+  if constexpr (STAGED) __syncthreads();  // (the mark below goes over what another thread has stored)
 
   // after a wait that ran into its bound: NaN as the final cell state and in the last visited frame of Y
   const bool expired = wait_expired(p.status);

@@ -174,7 +174,7 @@ struct Plan {
   int rq = 0;                    // regw, float32: quads of rows per group where the product goes in them, else 0
   bool dual = false;             // regw in turns: two turns' groups in one launch, taken in turn step by step
   bool wide = false;             // persistent kernel for layers whose W takes registers and LDS of the whole device
-  WideBuild wide_build = {nullptr, 0, 0, 0, 0, 0};
+  WideBuild wide_build = {nullptr, nullptr, 0, 0, 0, 0, 0};
   bool solo = false;             // small layer: every workgroup takes 4 rows through all steps by itself
   SoloBuild solo_build = {nullptr, 0, 0};
   bool half = false;             // regw: groups of at most 8 rows, two tiles folded into one pass of the pointwise part
@@ -515,7 +515,7 @@ bool make_plan_uncached(int64_t T, int B, int n, int dtype, int want_mode, bool 
         const int rows = 16 * wb.NT, turns = wb.kernel ? (B + rows - 1) / rows : 0;
         const int G = wb.kernel ? (n / 4 + wb.MT - 1) / wb.MT : 0;
         const long env_passes = env_long("RTN_LSTM2_MAX_PASSES", -1);
-        const size_t lds = wb.kernel ? wide_lds_bytes(wb.MT, wb.NT, wb.LF) + 64 : 0;
+        const size_t lds = wb.kernel ? wide_lds_bytes(wb.MT, wb.NT, wb.LF, (int)esize(dtype)) + 64 : 0;
         // Few frames in many turns: launches per step, which read W once per step for up to 64 rows, are ahead of turns that
         // load all of it for 16 or 32.  The two estimates are fitted to MI355X (us per call, wide / per step: bf16 n = 4096 with
         // B = 256, T = 1, 8, 16: 806 / 206, 1359 / 1176, 1958 / 2287; n = 2080, B = 768, T = 1, 8: 625 / 184, 1720 / 1263; float32
@@ -1270,7 +1270,7 @@ int settle_fwd_plan(int count, int64_t T, int B, int nc, int n, int dtype, int m
   if (!make_plan(T, B, n, dtype, mode, capturing, &pl, &why, 2, plan_count))
     return fail(RTN_ERR_UNSUPPORTED, "NativeLstm2: persistent mode unavailable for T=%lld B=%d n=%d: %s", (long long)T, B, n, why.c_str());
   for (int attempt = 0; pl.kind == kPlanMfma && pl.mode == RTN_MODE_PERSISTENT; ++attempt) {
-    *pk = pl.wide ? (const void*)pl.wide_build.kernel : pl.regw ? (const void*)regw_kernel(dtype, pl.MT, pl.NT, pl.KSMAX, pl.half, nc % (int)(std::min<size_t>(16, 4 * pl.MT * esize(dtype)) / esize(dtype)) != 0, pl.rq) : (const void*)mfma_kernel(dtype, n, pl.MT, pl.NT);
+    *pk = pl.wide ? (const void*)(nc == n && pl.wide_build.staged ? pl.wide_build.staged : pl.wide_build.kernel) : pl.regw ? (const void*)regw_kernel(dtype, pl.MT, pl.NT, pl.KSMAX, pl.half, nc % (int)(std::min<size_t>(16, 4 * pl.MT * esize(dtype)) / esize(dtype)) != 0, pl.rq) : (const void*)mfma_kernel(dtype, n, pl.MT, pl.NT);
     if (!*pk) return fail(RTN_ERR_UNSUPPORTED, "NativeLstm2: no kernel for mt=%d nt=%d ks=%d", pl.MT, pl.NT, pl.KSMAX);
     if ((rc = ensure_lds_limit(*pk, pl.lds_bytes)) != RTN_OK) return rc;
     const int wgs = pl.regw || pl.wide ? pl.grid : pl.groups * pl.wgs_per_group;

@@ -10,6 +10,7 @@ import torch
 from returnn_amd import lib
 
 from _gpu_util import announce, env, get_op, random_problem, run_raw, to_dev
+from test_gpu_pitch import POISON, _fwd_multi, _pair_problem
 
 pytestmark = pytest.mark.gpu
 
@@ -97,3 +98,19 @@ def test_few_frames_of_many_rows_run_as_one_launch_per_step(T, B, n, dtype):
         torch.cuda.synchronize()
         for name, a, b in zip("YCHd", recorded, want):
             assert numpy.array_equal(a.float().cpu().numpy(), b), name
+
+
+# every build whose streams go in pieces of rows: a last workgroup of fewer tiles, a last turn of fewer rows, pieces of 8 and 16 bytes
+@pytest.mark.parametrize("T,B,n,dtype,gap_x,gap_y", [(4, 17, 4096, "bf16", 0, 0), (5, 9, 2080, "bf16", 8, 8), (4, 33, 2576, "bf16", 0, 16), (4, 1, 1040, "f32", 4, 0), (5, 35, 2032, "f32", 0, 4)])
+def test_rows_with_a_pitch(T, B, n, dtype, gap_x, gap_y):
+    announce("wide kernel, pitched", T, B, n, dtype, gap_x, gap_y)
+    problems = _pair_problem(7200 + n, T, B, n)
+    with env(RTN_LSTM2_KERNEL=3):
+        assert "kernel=mfma_regw_wide" in lib.describe_plan(T, B, n, lib.DTYPE_BF16 if dtype == "bf16" else lib.DTYPE_F32, lib.MODE_AUTO)
+        got, _, Yj = _fwd_multi(problems, (1, -1), dtype, "auto", gap_x=gap_x, gap_y=gap_y, pitched=True)
+    want, _, _ = _fwd_multi(problems, (1, -1), dtype, "stepwise", gap_x=0, gap_y=0, pitched=False)
+    for k in range(2):
+        for name, a, b in zip("YCHd", got[k], want[k]):
+            assert bool(torch.isfinite(a).all()) and torch.equal(a, b), (k, name)
+    if gap_y:
+        assert bool((torch.cat([Yj[:, :, n : n + gap_y], Yj[:, :, 2 * n + gap_y :]], dim=-1) == POISON).all())
