@@ -1,0 +1,40 @@
+"""The gates' non-linearities in float32 against 64 bits: with recurrent weights of zero, H of a frame is the non-linearity of X."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from _gpu_util import announce, get_op
+
+pytestmark = pytest.mark.gpu
+
+INF, NAN = float("inf"), float("nan")
+# around where one formula takes over from another, and what must not come out of a range reduction as something else
+EDGES = [0.0, -0.0, 0.75, -0.75, 0.7499999, -0.7500001, 1e-30, -1e-40, 16.6, -16.7, -86.9, -87.1, 88.8, 99.9, 101.0, -104.0, 3.4e38, -3.4e38, INF, -INF, NAN]
+
+
+# one row per workgroup, groups on one XCD, a width that leaves no room for staging
+@pytest.mark.parametrize("n", [64, 512, 2304])
+@pytest.mark.parametrize("limit", [0.0, 0.2, 1.0, 4.0, 30.0, 80.0])
+def test_float32_gates(n, limit):
+    announce("float32 gates", n, limit)
+    T, B = 3, 4
+    if limit:
+        X = (torch.rand(T, B, 4 * n, generator=torch.Generator().manual_seed(n), dtype=torch.float32) * 2 - 1) * limit
+    else:
+        X = torch.tensor(EDGES, dtype=torch.float32).repeat(T * B * 4 * n // len(EDGES) + 1)[: T * B * 4 * n].view(T, B, 4 * n)
+    zero = torch.zeros(B, n, device="cuda")
+    H = get_op()(X.cuda(), torch.zeros(n, 4 * n, device="cuda"), zero, zero.clone(), torch.ones(T, B, device="cuda"), 0, 1)[2].double().cpu()
+    x = X.double()
+    want = torch.cat([torch.tanh(x[..., :n]), torch.sigmoid(x[..., n:])], dim=-1)
+    # (what left the first frame's y as NaN or infinity goes through the weights of zero into every gate of the row)
+    frames = slice(0, 1) if not limit else slice(None)
+    got, want = H[frames], want[frames]
+    assert torch.equal(got.isnan(), want.isnan())
+    # 4 ulp: e^x from the hardware and its correction 1.5 ulp, which are up to 3 of a result in the upper half of a binade, and 0.5 for each of
+    # the two roundings behind it; below the normal numbers zero
+    ulp = torch.exp2(torch.floor(torch.log2(want.abs().clamp(min=2.0**-126))) - 23)
+    error = (got - want).abs().nan_to_num(0.0)
+    allowed = torch.where(want.abs() < 2.0**-125, torch.full_like(ulp, 2.0**-125), 4 * ulp).nan_to_num(1.0)
+    assert bool((error <= allowed).all()), float((error / allowed).max())
