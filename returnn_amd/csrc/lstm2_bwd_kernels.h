@@ -346,7 +346,7 @@ struct Lstm2BwdMulti {
   int wgs_each;  // workgroups per problem = groups * n / (16 * MT)
   int local;     // 1: every batch group sits on one XCD (workgroup id = slot * xcds + xcd; the groups of the launch, all
                  // problems counted through, are dealt round-robin to the XCDs)
-  int xcds;      // XCDs the workgroup ids are dealt to (local plans)
+  int xcds;      // XCDs the workgroup ids are dealt to
   Lstm2BwdPersistent q[kMaxBwdMulti];
 };
 
@@ -384,8 +384,11 @@ __global__ __launch_bounds__(64 * WV) void k_lstm2_bwd_regw(const Lstm2BwdMulti 
     which = gg / groups_now;
     bid = (gg - which * groups_now) * kb + slot % kb;
   } else {
-    which = (int)blockIdx.x / multi.wgs_each;
-    bid = (int)blockIdx.x - which * multi.wgs_each;
+    // Ids go round-robin over the XCDs; a group gets as few XCDs as it fits, whose caches then hold its derivatives alone.  (us per gradient call of
+    // 64 frames of 64 rows, n = 2048, two groups per launch: 960 with each group on all XCDs, 919 on four.)
+    const int X = multi.xcds, all = (int)gridDim.x, id = all % X == 0 ? (int)blockIdx.x % X * (all / X) + (int)blockIdx.x / X : (int)blockIdx.x;
+    which = id / multi.wgs_each;
+    bid = id - which * multi.wgs_each;
   }
   if (which >= multi.count) return;
   const Lstm2BwdPersistent q = multi.q[which];

@@ -58,8 +58,8 @@ BwdRegwKernel bwd_regw_table_f32_full(int KSB, int MT, int WV);
 BwdRegwKernel bwd_local_table_bf16(int KSB, int MT);
 BwdRegwKernel bwd_local_table_f32(int KSB, int MT, int RQ);
 // The variants with half of a wavefront's share of W in registers and half in LDS (one tile per workgroup).
-BwdRegwKernel bwd_regw_lds_table_bf16(int WV);
-BwdRegwKernel bwd_regw_lds_table_f32(int WV);
+BwdRegwKernel bwd_regw_lds_table_bf16();
+BwdRegwKernel bwd_regw_lds_table_f32();
 
 // k_lstm2_regw<float, MT, 1, KSMAX, false, TAIL, RQ>: the product in quads of rows.
 RegwKernel regw_table_f32_quad(int MT, int KSMAX, bool tail, int RQ);

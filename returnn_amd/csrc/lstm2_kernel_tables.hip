@@ -96,10 +96,7 @@ BwdRegwKernel bwd_local_table(int KSB, int MT) {
 }
 
 template <typename AT>
-BwdRegwKernel bwd_regw_lds_table(int WV) {
-  if (WV == 8) return &k_lstm2_bwd_regw<AT, 16, 1, 8, 16>;
-  return &k_lstm2_bwd_regw<AT, 32, 1, 4, 32>;
-}
+BwdRegwKernel bwd_regw_lds_table() { return &k_lstm2_bwd_regw<AT, 16, 1, 8, 16>; }
 
 }  // namespace
 
@@ -115,12 +112,12 @@ RegwKernel regw_table_f32_hi(int MT, int NT, int KSMAX, bool half, bool tail) { 
 BwdRegwKernel bwd_regw_table_bf16_half(int KSB, int MT, int WV) { return bwd_regw_table<__bf16, true>(KSB, MT, WV); }
 #elif RTN_TABLE_PART == 6
 BwdRegwKernel bwd_regw_table_bf16_full(int KSB, int MT, int WV) { return bwd_regw_table<__bf16, false>(KSB, MT, WV); }
-BwdRegwKernel bwd_regw_lds_table_bf16(int WV) { return bwd_regw_lds_table<__bf16>(WV); }
+BwdRegwKernel bwd_regw_lds_table_bf16() { return bwd_regw_lds_table<__bf16>(); }
 #elif RTN_TABLE_PART == 7
 BwdRegwKernel bwd_regw_table_f32_half(int KSB, int MT, int WV) { return bwd_regw_table<float, true>(KSB, MT, WV); }
 #elif RTN_TABLE_PART == 8
 BwdRegwKernel bwd_regw_table_f32_full(int KSB, int MT, int WV) { return bwd_regw_table<float, false>(KSB, MT, WV); }
-BwdRegwKernel bwd_regw_lds_table_f32(int WV) { return bwd_regw_lds_table<float>(WV); }
+BwdRegwKernel bwd_regw_lds_table_f32() { return bwd_regw_lds_table<float>(); }
 #elif RTN_TABLE_PART == 9
 // Ascending by the width that MT tiles on 256 CUs and KS macro steps per wavefront take, then by rows.  What bounds NT: W,
 // 4 MT NT accumulator registers and two chunks of h per wavefront in 512 registers.

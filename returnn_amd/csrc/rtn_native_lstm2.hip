@@ -2373,10 +2373,13 @@ int choose_bwd_kernel(const BwdCtx& x, BwdChoice* out) {
     // A share of 64 fragments does not fit the registers next to a frame's DX (with all of it in registers the compiler
     // spills part of W, in float32 most of it): half of it lives in LDS.
     const bool lds_share = ksb_room * wv == 256;
-    if (lds_share && (mt != 1 || (wv != 4 && wv != 8))) continue;
+    // 8 wavefronts there: as many loads in flight, with a chunk's products over sooner.  (us per gradient call of 64 frames with 4 / 8: bf16 n = 1280, 2, 16 and 40 rows
+    // 332 / 308, 358 / 336, 456 / 418; n = 1536, 64 rows 840 / 805; n = 1792, 100 rows 1533 / 1481; n = 2048, 8, 64 and 256 rows 398 / 373, 919 / 900, 3060 / 2940;
+    // float32 n = 640, 40 rows 572 / 567, n = 768, 16 rows 526 / 519, n = 1024, 2 and 64 rows 495 / 489, 787 / 764.)
+    if (lds_share && (mt != 1 || wv != 8)) continue;
     BwdRegwKernel kfn = nullptr;
     if (lds_share)
-      kfn = dtype == RTN_DTYPE_BF16 ? bwd_regw_lds_table_bf16(wv) : bwd_regw_lds_table_f32(wv);
+      kfn = dtype == RTN_DTYPE_BF16 ? bwd_regw_lds_table_bf16() : bwd_regw_lds_table_f32();
     else
       // ring frames of 8 rows: the variant whose loads take two macro steps at once
       kfn = use_rows <= 8 ? (dtype == RTN_DTYPE_BF16 ? bwd_regw_table_bf16_half(ksb_room, mt, wv) : bwd_regw_table_f32_half(ksb_room, mt, wv))
