@@ -26,7 +26,7 @@ TABLE_PARTS = 16
 VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]
 VGPR_FORM_PARTS = (1, 2, 14)
 SOURCES = [HOST_SOURCE, TABLES_SOURCE]
-HEADERS = ["lstm2_kernels.h", "lstm2_step_kernel.h", "lstm2_wide_kernel.h", "lstm2_solo_kernel.h", "lstm2_dual_kernel.h", "lstm2_sparse_kernel.h", "lstm2_bwd_kernels.h", "lstm2_bwd_local_kernel.h", "weight_grad_kernel.h", "lstm2_params.h", "lstm2_kernel_tables.h",
+HEADERS = ["lstm2_kernels.h", "lstm2_step_kernel.h", "lstm2_wide_kernel.h", "lstm2_solo_kernel.h", "lstm2_dual_kernel.h", "lstm2_sparse_kernel.h", "lstm2_bwd_kernels.h", "lstm2_bwd_local_kernel.h", "lstm2_bwd_wide_kernel.h", "weight_grad_kernel.h", "lstm2_params.h", "lstm2_kernel_tables.h",
            os.path.join("..", "..", "include", "rtn_native_lstm2.h")]  # fmt: skip
 # the torch side of the calls (host code only)
 BINDING_SOURCE = "rtn_torch_binding.cpp"

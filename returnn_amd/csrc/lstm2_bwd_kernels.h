@@ -318,6 +318,7 @@ struct Lstm2BwdPersistent {
   int poll_delay, delay_inc, delay_dec_mask;
   unsigned long long timeout_ticks;
   unsigned* sync;     // [2 * groups of the whole problem] words of the XCD check (cleared before the launch)
+  void* exl;          // k_lstm2_bwd_wide: [xcds][kExRing][4n * 16] AT, the XCDs' rings (all-ones before every launch)
   void* ex;           // [groups of the whole problem][kExRing][4n * Bp] AT: the exchange ring (all-ones before the launch)
   int Bp, bp_shift;   // rows of a ring frame: 8 or 16 (= 1 << bp_shift), >= Bg
 };
@@ -347,6 +348,7 @@ struct Lstm2BwdMulti {
   int local;     // 1: every batch group sits on one XCD (workgroup id = slot * xcds + xcd; the groups of the launch, all
                  // problems counted through, are dealt round-robin to the XCDs)
   int xcds;      // XCDs the workgroup ids are dealt to
+  int slots;     // k_lstm2_bwd_wide: groups that the grid has room for
   Lstm2BwdPersistent q[kMaxBwdMulti];
 };
 

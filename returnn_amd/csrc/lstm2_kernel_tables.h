@@ -6,6 +6,7 @@
 
 #include "lstm2_bwd_kernels.h"
 #include "lstm2_bwd_local_kernel.h"
+#include "lstm2_bwd_wide_kernel.h"
 #include "lstm2_kernels.h"
 #include "lstm2_dual_kernel.h"
 #include "lstm2_solo_kernel.h"
@@ -60,6 +61,12 @@ BwdRegwKernel bwd_local_table_f32(int KSB, int MT, int RQ);
 // The variants with half of a wavefront's share of W in registers and half in LDS (one tile per workgroup).
 BwdRegwKernel bwd_regw_lds_table_bf16();
 BwdRegwKernel bwd_regw_lds_table_f32();
+// k_lstm2_bwd_wide<__bf16, MT, KST, LF>: the build for `steps` macro steps per wavefront; kernel null: none.
+struct BwdWideBuild {
+  BwdRegwKernel kernel;
+  int tiles, lds_fragments;
+};
+BwdWideBuild bwd_wide_build(int steps);
 
 // k_lstm2_regw<float, MT, 1, KSMAX, false, TAIL, RQ>: the product in quads of rows.
 RegwKernel regw_table_f32_quad(int MT, int KSMAX, bool tail, int RQ);

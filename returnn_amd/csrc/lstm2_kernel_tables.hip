@@ -113,6 +113,11 @@ BwdRegwKernel bwd_regw_table_bf16_half(int KSB, int MT, int WV) { return bwd_reg
 #elif RTN_TABLE_PART == 6
 BwdRegwKernel bwd_regw_table_bf16_full(int KSB, int MT, int WV) { return bwd_regw_table<__bf16, false>(KSB, MT, WV); }
 BwdRegwKernel bwd_regw_lds_table_bf16() { return bwd_regw_lds_table<__bf16>(); }
+BwdWideBuild bwd_wide_build(int steps) {
+  if (steps > 32 && steps <= 48) return {&k_lstm2_bwd_wide<__bf16, 2, 48, 4>, 2, 4};
+  if (steps > 48 && steps <= 64) return {&k_lstm2_bwd_wide<__bf16, 2, 64, 36>, 2, 36};
+  return {nullptr, 0, 0};
+}
 #elif RTN_TABLE_PART == 7
 BwdRegwKernel bwd_regw_table_f32_half(int KSB, int MT, int WV) { return bwd_regw_table<float, true>(KSB, MT, WV); }
 #elif RTN_TABLE_PART == 8

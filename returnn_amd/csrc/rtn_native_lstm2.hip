@@ -1564,6 +1564,9 @@ int fwd_calls(const rtn_lstm2_call* calls, int count, int64_t T, int32_t B, int3
 
 // Bytes of dynamic shared memory of the gradient kernel's variants that keep half of a wavefront's share of W in LDS (4
 // wavefronts with 32 + 32 fragments, or 8 wavefronts with 16 + 16).
+// k_lstm2_bwd_wide: groups that a launch's grid has room for, rings that a call's workspace has room for (one per XCD), LDS besides the weights'.
+constexpr int kBwdWideSlots = 4, kBwdWideRings = 8;
+constexpr size_t kBwdWideStaticLds = 14 * 1024 + 64;
 constexpr size_t kBwdLdsShareBytes = (size_t)kWaves * 32 * 64 * 16;
 
 // One rocBLAS handle per host thread and device, created on first use and kept for the life of the thread (never
@@ -1652,7 +1655,7 @@ int weight_grad_slices(long long rows, int n, int dtype) {
 }
 
 struct BwdLayout {
-  size_t off_sync = 0, off_dyw = 0, off_dx0 = 0, off_wpk = 0, off_ex = 0, off_part = 0, total = 0;  // [0, off_wpk) is cleared at the start of a call
+  size_t off_sync = 0, off_dyw = 0, off_dx0 = 0, off_wpk = 0, off_ex = 0, off_exl = 0, off_part = 0, total = 0;  // [0, off_wpk) is cleared at the start of a call
 };
 // n: the width the kernels work at; cells: the caller's, the same or (where the persistent kernel pads on the fly) one that is padded to n.
 BwdLayout bwd_layout(int64_t T, int B, int n, int dtype, int cells) {
@@ -1670,6 +1673,9 @@ BwdLayout bwd_layout(int64_t T, int B, int n, int dtype, int cells) {
   // rows in frames of 8, or of more than 8 rows in frames of 16: never more than 2B + 16 rows in all
   l.off_ex = off;
   if (n % 16 == 0) off = align_up(off + (size_t)kExRing * 4 * n * esize(dtype) * (2 * (size_t)B + 16), 256);
+  // the XCDs' rings of k_lstm2_bwd_wide
+  l.off_exl = off;
+  if (dtype == RTN_DTYPE_BF16 && bwd_wide_build((4 * n / 32 + kWaves - 1) / kWaves).kernel) off = align_up(off + (size_t)kBwdWideRings * kExRing * 4 * n * esize(dtype) * 16, 256);
   // the weight gradient's slices and y0^T dx0, of the caller's width (float32 324 has 4 slices, more bytes than the 3 of 352) and as many as
   // all frames' rows need (129 of n = 64 are 8 MB, a single frame has 2)
   l.off_part = off;
@@ -2174,6 +2180,7 @@ struct BwdChoice {
   size_t lds = 0;              // dynamic shared memory of the kernel
   bool one_xcd_kernel = false; // k_lstm2_bwd_local: local, rows_per_group <= 8
   int rq = 0;                  // float32: quads of rows per group where the product goes in them, else 0
+  int slots = 0;               // k_lstm2_bwd_wide: groups of all problems that the grid has room for, else 0
 };
 
 int bwd_calls(const rtn_lstm2_bwd_call* calls, int count, int64_t T, int32_t B, int32_t n, int32_t dtype, void* workspace,
@@ -2354,6 +2361,38 @@ int choose_bwd_kernel(const BwdCtx& x, BwdChoice* out) {
     if (best.kernel) {
       *out = best;
       return RTN_OK;
+    }
+  }
+  // Layers whose W takes a CU's registers and LDS: two tiles per workgroup and four groups at once.
+  // Its launch takes longer than one of k_lstm2_bwd_regw, which reads as much per workgroup and multiplies half: it has to
+  // spare more than a fifth of the launches.  (us per gradient call of 64 frames, one tile / two: as many launches n = 1088, 80 rows 705 / 751, n = 1280, 40 rows
+  // 419 / 469, n = 2048, 32 rows 429 / 536; 3 launches for 4, n = 1280, 192 rows 1692 / 1367; 2 for 3, n = 1408, 96 rows 998 / 827.)
+  // RTN_LSTM2_BWD_WIDE: 0 never, 2 wherever it fits.
+  if (dtype == RTN_DTYPE_BF16 && !env_mt && !env_rows && !env_waves && count <= kBwdWideSlots && env_long("RTN_LSTM2_BWD_WIDE", 1)) {
+    const int steps = (S + kWaves - 1) / kWaves, groups = (B + 15) / 16, per = kBwdWideSlots / count, xpg = di.xcds / kBwdWideSlots;
+    const int one_tile = std::max(1, di.cus / (n / 16) / count), turns_of_one_tile = (groups + one_tile - 1) / one_tile;
+    const BwdWideBuild wb = bwd_wide_build(steps);
+    const int kb = wb.kernel ? n / (16 * wb.tiles) : 0;
+    if (wb.kernel && n % (16 * wb.tiles) == 0 && di.xcds <= kBwdWideRings && di.xcds % kBwdWideSlots == 0 && kb % xpg == 0 && (env_long("RTN_LSTM2_BWD_WIDE", 1) == 2 || 5 * ((groups + per - 1) / per) < 4 * turns_of_one_tile)) {
+      const int members = kb / xpg, pieces = S * 4 * 16;  // workgroups of a group on one XCD; fragments of a frame
+      const size_t lds = (size_t)kWaves * wb.lds_fragments * 64 * 16;
+      int per_cu = 0;
+      if (di.xcds * members <= di.cus && (pieces + members - 1) / members <= kBwdWideForward * kWgThreads && lds + kBwdWideStaticLds <= di.lds_per_wg &&
+          (groups + per - 1) / per <= env_long("RTN_LSTM2_MAX_PASSES", kMaxPassesOverSteps)) {
+        if ((rc = ensure_lds_limit((const void*)wb.kernel, lds)) != RTN_OK) return rc;
+        if ((rc = occupancy_per_cu((const void*)wb.kernel, kWgThreads, lds, &per_cu)) != RTN_OK) return rc;
+        if (per_cu >= 1) {
+          BwdChoice c;
+          c.kernel = (const void*)wb.kernel;
+          c.ksb = steps;
+          c.tiles = wb.tiles;
+          c.groups_per_launch = std::min(per, groups);
+          c.lds = lds;
+          c.slots = kBwdWideSlots;
+          *out = c;
+          return RTN_OK;
+        }
+      }
     }
   }
   for (const auto& cand : candidates) {
@@ -2545,6 +2584,7 @@ int bwd_launch_persistent(const BwdCtx& x, const BwdChoice& ch, const BwdLayout&
     q.timeout_ticks = (unsigned long long)env_long("RTN_LSTM2_TIMEOUT_TICKS", 200000000L);
     q.sync = (unsigned*)(j.ws + lay.off_sync);
     q.ex = j.ws + lay.off_ex;
+    q.exl = j.ws + lay.off_exl;
     q.Bp = ch.rows_per_group > 8 ? 16 : 8;
     q.bp_shift = ch.rows_per_group > 8 ? 4 : 3;
     prep.words[k] = (unsigned*)j.ws;
@@ -2566,6 +2606,7 @@ int bwd_launch_persistent(const BwdCtx& x, const BwdChoice& ch, const BwdLayout&
   }
   multi.local = ch.local ? 1 : 0;
   multi.xcds = device_info().xcds;
+  multi.slots = ch.slots;
   const int wgs_per_group = n / (16 * ch.tiles);
   for (int g0 = 0; g0 < bgroups; g0 += ch.groups_per_launch) {
     const int groups_now = std::min(ch.groups_per_launch, bgroups - g0);
@@ -2580,6 +2621,12 @@ int bwd_launch_persistent(const BwdCtx& x, const BwdChoice& ch, const BwdLayout&
       // workgroup id = slot * xcds + xcd: the groups of the launch are dealt round-robin to the XCDs
       const int total_groups = count * groups_now;
       grid = (unsigned)(multi.xcds * wgs_per_group * ((total_groups + multi.xcds - 1) / multi.xcds));
+    }
+    if (ch.slots) {
+      grid = (unsigned)(ch.slots * wgs_per_group);
+      const long long words = (long long)((size_t)multi.xcds * kExRing * 4 * n * x.es * 16 / 4);
+      for (int k = 0; k < count; ++k) hipLaunchKernelGGL(k_fill_u32, dim3(512), fill_block, 0, x.stream, (unsigned*)multi.q[k].exl, ~0u, words);
+      RTN_HIP(hipGetLastError());
     }
     const int rc = launch_coresident(ch.kernel, dim3(grid), dim3((unsigned)(64 * ch.waves)), args, (unsigned)ch.lds, x.stream, x.capturing);
     if (rc != RTN_OK) return rc;
@@ -2897,7 +2944,7 @@ int bwd_calls(const rtn_lstm2_bwd_call* calls, int count, int64_t T, int32_t B, 
     if (ch.kernel)
       snprintf(buf, sizeof(buf), "kernel=%s problems=%d rows_per_group=%d groups=%d tiles=%d waves=%d wgs_per_group=%d launches=%d row_quads=%d name=%s",
                ch.local ? "bwd_regw_xcd" : "bwd_regw", count, ch.rows_per_group, bgroups, ch.tiles, ch.waves, np / (16 * ch.tiles),
-               (bgroups + ch.groups_per_launch - 1) / std::max(ch.groups_per_launch, 1), ch.rq, ch.one_xcd_kernel ? "k_lstm2_bwd_local" : "k_lstm2_bwd_regw");
+               (bgroups + ch.groups_per_launch - 1) / std::max(ch.groups_per_launch, 1), ch.rq, ch.one_xcd_kernel ? "k_lstm2_bwd_local" : ch.slots ? "k_lstm2_bwd_wide" : "k_lstm2_bwd_regw");
     else
       snprintf(buf, sizeof(buf), "kernel=%s problems=%d launches_per_frame=%d name=%s", mfma ? "bwd_step" : "bwd_generic", count, mfma ? 1 : 2,
                mfma ? "k_bwd_step" : "k_bwd_pointwise");
