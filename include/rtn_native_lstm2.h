@@ -450,7 +450,7 @@ const char* rtn_native_lstm2_capture_report(void);
 /* The decomposition the last gradient call of the calling thread ran on (kernel, rows per batch group, tiles and
  * wavefronts per workgroup, launches): the gradient entries' counterpart of rtn_native_lstm2_describe_plan, for logs,
  * the benchmark line and tests.  "kernel=bwd_regw_xcd": every batch group on one XCD; "name=": the device kernel
- * (k_lstm2_bwd_local there for groups of up to 8 rows, k_lstm2_bwd_regw, or k_bwd_step / k_bwd_pointwise per frame);
+ * (k_lstm2_bwd_local there for groups of up to 8 rows, k_lstm2_bwd_regw, k_lstm2_bwd_wide, or k_bwd_step / k_bwd_pointwise per frame);
  * "weight_gradient=": k_weight_grad, rocblas, or rocblas with k_weight_last behind it. */
 const char* rtn_native_lstm2_bwd_plan_text(void);
 

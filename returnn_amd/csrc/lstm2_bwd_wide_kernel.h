@@ -13,8 +13,9 @@ namespace rtn {
 // W of n = 2048 in bf16 is 32 MB, and what bounds k_lstm2_bwd_regw there is not W but how many rows a launch takes: a workgroup
 // with one tile of 16 values of k reads all of its group's derivatives every frame (16 rows x 4n values, 256 KB), 128 of them are a group of
 // 16 rows, and the device holds two such groups.  Here a workgroup has MT = 2 tiles for the same 256 KB: four groups at once.
-// What bounds a frame (5.4 us at n = 2048) is those 256 KB on their way from the XCD's L2, 47 KB per microsecond and CU of the 150 that its
-// path takes: 12 loads per wavefront in flight are what the registers have room for.  The MFMAs are 0.85 us of it.
+// What bounds a frame (6.3 us at n = 2048) is those 256 KB on their way from the XCD's L2, 40 KB per microsecond and CU of the 150 that its
+// path takes: 12 loads per wavefront in flight are what the registers have room for.  Of a frame's 14 000 clocks the MFMAs are 2048, vector
+// instructions 2800, and half of them a wavefront waits for memory.
 // us per gradient call of 64 frames, k_lstm2_bwd_regw / here: n = 2048, 48, 64, 100 and 256 rows 737 / 588, 877 / 743, 1446 / 1149, 2939 / 2380, two
 // problems of 32 rows 842 / 699; n = 1792, 100 rows 1479 / 1121; n = 1536, 48, 64 and 160 rows 685 / 455, 784 / 551, 1754 / 1326; n = 1280, 64 rows 700 / 437.
 // (Chunks of 2 macro steps, six of them in flight: 783 at n = 2048 and 64 rows; the next frame's inputs behind the last chunk: 773.)

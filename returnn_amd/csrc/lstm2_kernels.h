@@ -1052,7 +1052,7 @@ __device__ __forceinline__ void quad_macro_step(const i32x4 (&wbits)[MT], const 
    ...);
 }
 
-// HALF: the groups have at most 8 rows (NT == 1, MT even).  A tile then holds valid results in the lanes of rows 0..7
+// HALF: the groups have at most 8 rows (NT == 1, MT even; float32, and bf16 with 16 macro steps per wavefront: k_lstm2_sparse takes fewer).  A tile then holds valid results in the lanes of rows 0..7
 // only, and the pointwise part folds two tiles into one pass: lanes of rows 0..7 take tile 2u, lanes of rows 8..15 take
 // rows 0..7 of tile 2u + 1, so that a thread owns one (sequence, cell) pair where the plain mapping gives it two, one
 // of them of a row that does not exist.
