@@ -86,26 +86,38 @@ struct Elem<__bf16> {
 //  * 1 / d by a Newton step from the hardware's reciprocal; `lo` is what d = 1 + e lost by rounding.
 // Error against 64 bits, 2-norm, of 2^20 arguments evenly spread over +-0.1, +-1, +-3, +-8 and +-20, with expf and a division / here: 4.4e-8 / 3.0e-8,
 // 4.0e-8 / 2.9e-8, 3.8e-8 / 2.4e-8, 3.8e-8 / 1.9e-8, 3.5e-8 / 1.8e-8.
-__device__ __forceinline__ float sigmoid_f32(float x) {
-  const float z = __builtin_elementwise_minimum(x, 100.f);  // (keeps a NaN; at infinity r would be one)
-  const float t = z * -1.44269504088896f;
-  float e = __builtin_amdgcn_exp2f(t);
-  const float r = __builtin_fmaf(t, 1.904654299957767e-09f, __builtin_fmaf(t, -0.693147182464599609375f, -z));  // ln 2 in two parts
-  e = __builtin_fmaf(e, r, e);
-  const float d = 1.f + e, lo = e - (d - 1.f);
-  const float q = __builtin_amdgcn_rcpf(d);
+__device__ __forceinline__ float exp_f32(float w) {
+  const float t = w * 1.44269504088896f;
+  const float e = __builtin_amdgcn_exp2f(t);
+  const float r = __builtin_fmaf(t, 1.904654299957767e-09f, __builtin_fmaf(t, -0.693147182464599609375f, w));  // ln 2 in two parts
+  return __builtin_fmaf(e, r, e);
+}
+// what goes through exp_f32 (minimum keeps a NaN; at infinity r would be one)
+__device__ __forceinline__ float sigmoid_exponent(float x) { return -__builtin_elementwise_minimum(x, 100.f); }
+// sigmoid of x from e = exp_f32 of that, d = 1 + e and q, the hardware's 1 / d
+__device__ __forceinline__ float sigmoid_of(float x, float e, float d, float q) {
+  const float lo = e - (d - 1.f);
   const float s = __builtin_fmaf(__builtin_fmaf(-lo, q, __builtin_fmaf(-d, q, 1.f)), q, q);
   return x < -87.f ? 0.f : s;  // (beyond the normal numbers, down to minus infinity)
 }
+__device__ __forceinline__ float sigmoid_f32(float x) {
+  const float e = exp_f32(sigmoid_exponent(x)), d = 1.f + e;
+  return sigmoid_of(x, e, d, __builtin_amdgcn_rcpf(d));
+}
 
-// tanh in float32 without a branch: both sides of |x| = 0.75, 22 instructions that the compiler puts between those of other gates.  (tanhf branches
+// tanh in float32 without a branch: both sides of |x| = 0.75, 23 instructions that the compiler puts between those of other gates.  (tanhf branches
 // at 0.625: 16 and 28 instructions, both of them as soon as one lane is on the other side.)
 //  * near: x + x u P(u), u = x^2, P of degree 5 by least squares of the relative error, reweighted to its maximum: 0.03 ulp.
-//  * far: 1 - 2 / (1 + e^2|x|), e^2|x| as in sigmoid_f32; what is subtracted is below 0.37, and so are its errors.
+//  * far: 1 - 2 / (1 + e^2|x|), what is subtracted is below 0.37, and so are its errors.
 // Error against 64 bits, 2-norm and largest in ulp, of arguments evenly spread over +-0.1, +-1, +-3 and +-20, tanhf / here: 2.56e-8 / 2.54e-8, 3.43e-8 /
 // 3.18e-8, 2.13e-8 / 2.10e-8, 1.24e-8 / 1.23e-8; 0.55 / 0.52, 1.38 / 1.31, 1.38 / 1.28, 1.30 / 1.23.  us per call, with tanhf / this, of arguments that
 // nearly all were near: T = 32, 4 rows of n = 64 19.0 / 18.2; T = 300, 32 rows of n = 1024 1077 / 1071; T = 200, 3 rows of n = 2048 1235 / 1222.
-__device__ __forceinline__ float tanh_f32(float x) {
+__device__ __forceinline__ float tanh_exponent(float x) {
+  const float a = __builtin_elementwise_minimum(__builtin_fabsf(x), 20.f);
+  return a + a;
+}
+// tanh of x from q = 1 / (1 + exp_f32 of that)
+__device__ __forceinline__ float tanh_of(float x, float q) {
   const float u = x * x;
   float p = __builtin_fmaf(u, 0.001736935111694038f, -0.007657254114747047f);
   p = __builtin_fmaf(u, p, 0.021452033892273903f);
@@ -113,13 +125,10 @@ __device__ __forceinline__ float tanh_f32(float x) {
   p = __builtin_fmaf(u, p, 0.1333269476890564f);
   p = __builtin_fmaf(u, p, -0.33333316445350647f);
   const float near = __builtin_fmaf(u, x * p, x);
-  const float a = __builtin_elementwise_minimum(__builtin_fabsf(x), 20.f), z = a + a;  // (keeps a NaN)
-  const float t = z * 1.44269504088896f;
-  float e = __builtin_amdgcn_exp2f(t);
-  e = __builtin_fmaf(e, __builtin_fmaf(t, -0.693147182464599609375f, z), e);
-  const float far = __builtin_fmaf(__builtin_amdgcn_rcpf(1.f + e), -2.f, 1.f);
+  const float far = __builtin_fmaf(q, -2.f, 1.f);
   return __builtin_fabsf(x) < 0.75f ? near : __builtin_copysignf(far, x);
 }
+__device__ __forceinline__ float tanh_f32(float x) { return tanh_of(x, __builtin_amdgcn_rcpf(1.f + exp_f32(tanh_exponent(x)))); }
 
 // Gate non-linearities.  float32 runs keep to 32 bits (1e-5 relative is the bar there).  bfloat16 runs round every result to 8 bits of
 // mantissa anyway, so they use the hardware exp2 and reciprocal (about 1 ulp of float32 each):

@@ -31,6 +31,8 @@ namespace rtn {
 // Measured, us per step (T = 300, 4 rows; four rows per workgroup / one): float32 n = 32 0.64 / 0.44, n = 64 0.74 / 0.51; bf16 n = 32 0.41 / 0.29,
 // n = 64 0.62 / 0.38, n = 96 0.71 / 0.60, n = 128 0.87 / 0.73.  float32 against k_lstm2_regw: n = 96 1.07 / 0.88, n = 128 1.06 / 1.01, with 256 rows
 // 1.37 / 0.91 and 1.39 / 1.07.  One call with T = 32, B = 4, n = 64: 45 us with packing (5.3) and k_lstm2_regw (36.5), 27 with four rows per workgroup, 20 with one.
+// All of these with library functions in the float32 gates; one row without: n = 32 0.36, 64 0.45, 96 0.84, 128 0.99, the call 18.2 us; with one exponential and one
+// reciprocal for whichever gate a lane has: 0.34, 0.43, 0.81, 0.96 and 17.5.  (h as one read of all macro steps' elements per lane: 0.35, 0.44, 0.81, 0.95 and 17.8.)
 // ---------------------------------------------------------------------------------------------
 constexpr int kSoloRows = 4;
 constexpr int kSoloCells = 16;  // cells per wavefront
@@ -152,7 +154,8 @@ __device__ __forceinline__ float quad_lane(float v) { return __builtin_bit_cast(
 template <typename AT>
 __device__ __forceinline__ float solo_gate(float x, bool first) {
   if constexpr (sizeof(AT) == 4) {
-    const float t = Act<AT>::tanh(x), s = Act<AT>::sigmoid(x);
+    const float e = exp_f32(first ? tanh_exponent(x) : sigmoid_exponent(x)), d = 1.f + e, q = __builtin_amdgcn_rcpf(d);  // (one of each for both)
+    const float t = tanh_of(x, q), s = sigmoid_of(x, e, d, q);
     return first ? t : s;
   } else {  // Act<__bf16>'s two with one exponential and one reciprocal
     const float r = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f((first ? -2.8853900817779268f : -1.4426950408889634f) * x));
