@@ -154,7 +154,7 @@ __device__ __forceinline__ float quad_lane(float v) { return __builtin_bit_cast(
 template <typename AT>
 __device__ __forceinline__ float solo_gate(float x, bool first) {
   if constexpr (sizeof(AT) == 4) {
-    const float e = exp_f32(first ? tanh_exponent(x) : sigmoid_exponent(x)), d = 1.f + e, q = __builtin_amdgcn_rcpf(d);  // (one of each for both)
+    const float e = exp_f32(first ? tanh_exponent(x) : sigmoid_exponent(x)), d = 1.f + e, q = reciprocal_f32(d);  // (one of each for both)
     const float t = tanh_of(x, q), s = sigmoid_of(x, e, d, q);
     return first ? t : s;
   } else {  // Act<__bf16>'s two with one exponential and one reciprocal

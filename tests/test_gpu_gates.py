@@ -38,3 +38,18 @@ def test_float32_gates(n, limit):
     error = (got - want).abs().nan_to_num(0.0)
     allowed = torch.where(want.abs() < 2.0**-125, torch.full_like(ulp, 2.0**-125), 4 * ulp).nan_to_num(1.0)
     assert bool((error <= allowed).all()), float((error / allowed).max())
+
+
+@pytest.mark.parametrize("n", [64, 512, 2304])
+def test_small_results_of_sigmoid(n):
+    """Down to where e^-x is no float32 any more a sigmoid is not cut off."""
+    announce("float32 gates, small results", n)
+    T, B = 2, 4
+    X = -80.0 - 8.7228 * torch.rand(T, B, 4 * n, generator=torch.Generator().manual_seed(n), dtype=torch.float32)
+    X[0, 0, n : n + 4] = torch.tensor([-87.0, -87.33655, -87.4, -88.722])
+    zero = torch.zeros(B, n, device="cuda")
+    H = get_op()(X.cuda(), torch.zeros(n, 4 * n, device="cuda"), zero, zero.clone(), torch.ones(T, B, device="cuda"), 0, 1)[2].cpu()
+    got, want = H[..., n:].double(), torch.sigmoid(X[..., n:].double())
+    # 4 ulp as above; below the normal numbers an ulp is the smallest number, and a result is rounded to it twice
+    ulp = torch.exp2(torch.floor(torch.log2(want.clamp(min=2.0**-126))) - 23)
+    assert bool(((got - want).abs() <= 4 * ulp).all()), float(((got - want).abs() / ulp).max())
