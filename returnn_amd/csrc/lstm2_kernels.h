@@ -130,7 +130,7 @@ __device__ __forceinline__ float tanh_of(float x, float q) {
   p = __builtin_fmaf(u, p, -0.33333316445350647f);
   const float near = __builtin_fmaf(u, x * p, x);
   const float far = __builtin_fmaf(q, -2.f, 1.f);
-  return __builtin_fabsf(x) < 0.75f ? near : __builtin_copysignf(far, x);
+  return __builtin_copysignf(__builtin_fabsf(x) < 0.75f ? near : far, x);  // (of -0 as well, where the sum of `near` is +0)
 }
 __device__ __forceinline__ float tanh_f32(float x) { return tanh_of(x, __builtin_amdgcn_rcpf(1.f + exp_f32(tanh_exponent(x)))); }
 

@@ -53,3 +53,20 @@ def test_small_results_of_sigmoid(n):
     # 4 ulp as above; below the normal numbers an ulp is the smallest number, and a result is rounded to it twice
     ulp = torch.exp2(torch.floor(torch.log2(want.clamp(min=2.0**-126))) - 23)
     assert bool(((got - want).abs() <= 4 * ulp).all()), float(((got - want).abs() / ulp).max())
+
+
+@pytest.mark.parametrize("n", [64, 512, 2304])
+def test_tanh_keeps_the_sign_of_zero(n):
+    """A cell state of -0, to which a gate adds what rounds to -0, comes out as -0."""
+    announce("float32 gates, signed zero", n)
+    T, B = 3, 2
+    X = torch.zeros(T, B, 4 * n, dtype=torch.float32)
+    X[..., :n] = -1e-45  # times a sigmoid below a half: rounds to -0
+    X[..., n : 2 * n] = -5.0
+    X[:, 1, :n] = 1e-45
+    W, y0, c0 = torch.zeros(n, 4 * n, device="cuda"), torch.zeros(B, n), torch.zeros(B, n)
+    y0[0] = c0[0] = -0.0
+    Y, C, _, d = get_op()(X.cuda(), W, y0.cuda(), c0.cuda(), torch.ones(T, B, device="cuda"), 0, 1)
+    assert not Y.any() and not C.any()
+    assert bool(torch.signbit(C[:, 0]).all()) and bool(torch.signbit(Y[:, 0]).all()) and bool(torch.signbit(d[0]).all())
+    assert not torch.signbit(C[:, 1]).any() and not torch.signbit(Y[:, 1]).any()
