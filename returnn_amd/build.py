@@ -20,9 +20,11 @@ LIB_NAME = "librtn_native_lstm2.so"
 LIB_PATH = os.path.join(CSRC_DIR, LIB_NAME)
 HOST_SOURCE = "rtn_native_lstm2.hip"
 TABLES_SOURCE = "lstm2_kernel_tables.hip"  # compiled once per part: the instantiations of the persistent kernels
-TABLE_PARTS = 16
+TABLE_PARTS = 17
 # Matrix instructions that leave their results where vector instructions read them: the bf16 forward kernels add two accumulators per
 # tile, and out of accumulation registers every one of them is copied first (B=256 T=200 n=1024: 717 us, 690 without the copies).
+# (Not part 17, layers beyond n = 1024, whose tiles have one accumulator: with it T=100 n=2048, 16 and 32 rows, 250 and 273 us, 247 and 271
+# without; n=1536, 17 rows 249 / 245; n=1280, 48 rows 255 / 251.)
 VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]
 VGPR_FORM_PARTS = (1, 2, 14)
 SOURCES = [HOST_SOURCE, TABLES_SOURCE]

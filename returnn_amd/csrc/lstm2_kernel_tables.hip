@@ -5,22 +5,21 @@
 #include "lstm2_kernel_tables.h"
 
 #ifndef RTN_TABLE_PART
-#error "compile with -DRTN_TABLE_PART=<1..16>"
+#error "compile with -DRTN_TABLE_PART=<1..17>"
 #endif
 
 namespace rtn {
 namespace {
 
-// Forward.  HI: the builds with 8 or 16 macro steps of the contraction per wavefront, else those with 2 or 4.
+// Forward.  HI: the builds with 8 or 16 macro steps of the contraction per wavefront, else those with 2 or 4.  (bfloat16 with 16: regw_table_16.)
 template <typename AT, bool HI, bool TAIL>
 RegwKernel regw_table(int MT, int NT, int KSMAX, bool half) {
   if (half) {
 #define RTN_CASE(mt, ks) \
   if (MT == mt && NT == 1 && KSMAX == ks) return &k_lstm2_regw<AT, mt, 1, ks, true, TAIL>;
-    if constexpr (HI) { RTN_CASE(2, 16) }
     if constexpr (sizeof(AT) == 4) {  // (bfloat16: k_lstm2_sparse)
       if constexpr (HI) {
-        RTN_CASE(2, 8) RTN_CASE(4, 8) RTN_CASE(8, 8)
+        RTN_CASE(2, 16) RTN_CASE(2, 8) RTN_CASE(4, 8) RTN_CASE(8, 8)
       } else {
         RTN_CASE(2, 2) RTN_CASE(2, 4)
         RTN_CASE(4, 2) RTN_CASE(4, 4)
@@ -36,9 +35,10 @@ RegwKernel regw_table(int MT, int NT, int KSMAX, bool half) {
     RTN_CASE(2, 1, 8) RTN_CASE(2, 2, 8) RTN_CASE(2, 4, 8)
     RTN_CASE(4, 1, 8) RTN_CASE(4, 2, 8)
     RTN_CASE(8, 1, 8)
-    RTN_CASE(1, 1, 16) RTN_CASE(1, 2, 16)
-    RTN_CASE(2, 1, 16) RTN_CASE(2, 2, 16)
-    if constexpr (sizeof(AT) == 2) { RTN_CASE(4, 1, 16) }
+    if constexpr (sizeof(AT) == 4) {
+      RTN_CASE(1, 1, 16) RTN_CASE(1, 2, 16)
+      RTN_CASE(2, 1, 16) RTN_CASE(2, 2, 16)
+    }
   } else {
     RTN_CASE(1, 1, 2) RTN_CASE(1, 2, 2) RTN_CASE(1, 4, 2)
     RTN_CASE(2, 1, 2) RTN_CASE(2, 2, 2) RTN_CASE(2, 4, 2)
@@ -47,6 +47,19 @@ RegwKernel regw_table(int MT, int NT, int KSMAX, bool half) {
     RTN_CASE(2, 1, 4) RTN_CASE(2, 2, 4) RTN_CASE(2, 4, 4)
     RTN_CASE(4, 1, 4) RTN_CASE(4, 2, 4)
   }
+#undef RTN_CASE
+  return nullptr;
+}
+
+// Forward, bfloat16 with 16 macro steps per wavefront.
+template <bool TAIL>
+RegwKernel regw_table_16(int MT, int NT, bool half) {
+  if (half) return MT == 2 && NT == 1 ? &k_lstm2_regw<__bf16, 2, 1, 16, true, TAIL> : nullptr;
+#define RTN_CASE(mt, nt) \
+  if (MT == mt && NT == nt) return &k_lstm2_regw<__bf16, mt, nt, 16, false, TAIL>;
+  RTN_CASE(1, 1) RTN_CASE(1, 2)
+  RTN_CASE(2, 1) RTN_CASE(2, 2)
+  RTN_CASE(4, 1)
 #undef RTN_CASE
   return nullptr;
 }
@@ -193,8 +206,10 @@ RegwKernel sparse_kernel(int MT, int KSMAX, bool tail) {
 #undef RTN_CASE
   return nullptr;
 }
+#elif RTN_TABLE_PART == 17
+RegwKernel regw_table_bf16_16(int MT, int NT, bool half, bool tail) { return tail ? regw_table_16<true>(MT, NT, half) : regw_table_16<false>(MT, NT, half); }
 #else
-#error "RTN_TABLE_PART must be 1..16"
+#error "RTN_TABLE_PART must be 1..17"
 #endif
 
 }  // namespace rtn

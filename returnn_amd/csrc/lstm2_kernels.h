@@ -1597,7 +1597,7 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_regw(const Lstm2Multi mult
           opnd = opnd_next;
         }
       } else if constexpr (TWO) {
-        // Tiles in groups of up to four, both chains of each; a group's partial tiles are added and leave for LDS behind the next group's MFMAs.
+        // Tiles in groups of up to four, both chains of each.
         flush_read_at(rd_h, rd_y, rd_c);
         load_gate_inputs(IntTag<1 - PAR>{});
         put(par_tag);
@@ -1610,19 +1610,35 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_regw(const Lstm2Multi mult
           f32x4 two[GRP][2];
 #pragma unroll
           for (int i = 0; i < GRP; ++i) two[i][0] = two[i][1] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int ks = 0; ks < KSMAX; ++ks)
-#pragma unroll
-            for (int i = 0; i < GRP; ++i) {
-              two[i][ks & 1] = E::mma(wreg[(t0 + i) / NT][ks], bf[ks][(t0 + i) % NT], two[i][ks & 1]);
-              __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-              __builtin_amdgcn_sched_group_barrier(0x096, 3, 0);
-            }
-#pragma unroll
-          for (int i = 0; i < GRP; ++i) {
+          auto product = [&](int ks, int i) {
+            two[i][ks & 1] = E::mma(wreg[(t0 + i) / NT][ks], bf[ks][(t0 + i) % NT], two[i][ks & 1]);
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x096, 3, 0);
+          };
+          auto sum = [&](int i) {
             asm("" : "+v"(two[i][0]), "+v"(two[i][1]));  // (accumulation registers would be copied for the additions)
             redbuf[wave][t0 + i][lane] = two[i][0] + two[i][1];
+          };
+          // A tile's two sums are added behind the MFMAs of other tiles where there is a choice.  With 2 macro steps, tile by tile; with 8, the
+          // last two so, a fence behind every tile and a tile's sum two tiles later; with 4, all sums behind the last MFMA: the order
+          // of the others was 0-2 % slower.  (us per 200 steps, one chain / two and all sums at the end / this: n = 256, 300 and 512 rows 366 / 362 / 345,
+          // 394 / 393 / 369; n = 1024, 100 and 128 rows 458 / 457 / 451, 488 / 489 / 476; n = 1001, 100 rows 448 / 465 / 456; n = 768, 72 rows 397 / 400 / 392; n = 512, 96 and 256
+          // rows 243 / 250 / the same, 448 / 447 / the same.)
+          constexpr int LAST = KSMAX == 4 ? 0 : 2, LAG = !LAST ? GRP : KSMAX == 8 ? 2 : 1;
+#pragma unroll
+          for (int ks = 0; ks < KSMAX - LAST; ++ks)
+#pragma unroll
+            for (int i = 0; i < GRP; ++i) product(ks, i);
+          if (KSMAX == 8) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int i = 0; i < GRP; ++i) {
+#pragma unroll
+            for (int ks = KSMAX - LAST; ks < KSMAX; ++ks) product(ks, i);
+            if (i >= LAG) sum(i - LAG);
+            if (KSMAX == 8) __builtin_amdgcn_sched_barrier(0);
           }
+#pragma unroll
+          for (int i = GRP > LAG ? GRP - LAG : 0; i < GRP; ++i) sum(i);
         }
       } else {
         flush_read_at(rd_h, rd_y, rd_c);
