@@ -2551,7 +2551,7 @@ int bwd_launch_persistent(const BwdCtx& x, const BwdChoice& ch, const BwdLayout&
   prep.n_words = (long long)(lay.off_dyw / 4);  // status and the words of the XCD check
   prep.abort_word = (unsigned long long)(uintptr_t)t_abort_word;
   prep.abort_id = t_abort_id;
-  if ((size_t)prep.ring_words * 4 > lay.off_part - lay.off_ex)
+  if ((size_t)prep.ring_words * 4 > lay.off_exl - lay.off_ex)
     return fail(RTN_ERR_WORKSPACE, "NativeLstm2 backward: internal: exchange ring of %lld bytes does not fit its section", prep.ring_words * 4);
   for (int k = 0; k < count; ++k) {
     Lstm2BwdPersistent& q = multi.q[k];

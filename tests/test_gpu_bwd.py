@@ -95,6 +95,16 @@ def test_bwd_ring_that_does_not_fit_its_section_is_refused():
             _run(200, 21, 64, "f32", 0, 1)
 
 
+def test_bwd_ring_is_held_against_its_own_section_alone():
+    """The same at a width whose workspace has the rings of another kernel behind the exchange ring."""
+    from _gpu_util import env
+
+    announce("bwd ring beyond its section, wide layer")
+    with env(RTN_LSTM2_BWD_KERNEL=2, RTN_LSTM2_BWD_ROWS=1):
+        with pytest.raises(RuntimeError, match="exchange ring"):
+            _run(4, 24, 1280, "bf16", 0, 1)
+
+
 # float32 groups of up to 8 rows on one XCD each: one and two quads of rows with 1, 2 and 4 tiles, cut quads and groups, every
 # number of macro steps per wavefront, odd widths
 @pytest.mark.parametrize("B,n,tiles,quads", [(1, 512, 1, 1), (30, 500, 1, 1), (61, 512, 2, 1), (37, 512, 1, 2), (128, 512, 2, 2), (97, 301, 2, 2), (60, 256, 1, 1), (205, 224, 2, 2),
