@@ -1566,7 +1566,20 @@ int fwd_calls(const rtn_lstm2_call* calls, int count, int64_t T, int32_t B, int3
 // wavefronts with 32 + 32 fragments, or 8 wavefronts with 16 + 16).
 // k_lstm2_bwd_wide: groups that a launch's grid has room for, rings that a call's workspace has room for (one per XCD), LDS besides the weights'.
 constexpr int kBwdWideSlots = 4, kBwdWideRings = 8;
+static_assert(kMaxBwdMulti <= kBwdWideSlots, "a group of every problem of a launch");
 constexpr size_t kBwdWideStaticLds = 14 * 1024 + 64;
+// Whether it is the kernel for `count` problems of B rows each, as far as rows and launches go: four groups at once instead of two or fewer.
+// Its launch takes longer than one of k_lstm2_bwd_regw, which reads as much per workgroup and multiplies half: it has to
+// spare more than a fifth of the launches.  (us per gradient call of 64 frames, one tile / two: as many launches n = 1088, 80 rows 705 / 751, n = 1280, 40 rows
+// 419 / 469, n = 2048, 32 rows 429 / 536; 3 launches for 4, n = 1280, 192 rows 1692 / 1367; 2 for 3, n = 1408, 96 rows 998 / 827.)
+// RTN_LSTM2_BWD_WIDE: 0 never, 2 wherever it fits.
+bool bwd_wide_spares_launches(int count, int B, int n, int cus) {
+  const long want = env_long("RTN_LSTM2_BWD_WIDE", 1);
+  if (want == 0 || want == 2) return want == 2;
+  const int groups = (B + 15) / 16, per = kBwdWideSlots / count;
+  const int one_tile = std::max(1, cus / (n / 16) / count), turns_of_one_tile = (groups + one_tile - 1) / one_tile;
+  return 5 * ((groups + per - 1) / per) < 4 * turns_of_one_tile;
+}
 constexpr size_t kBwdLdsShareBytes = (size_t)kWaves * 32 * 64 * 16;
 
 // One rocBLAS handle per host thread and device, created on first use and kept for the life of the thread (never
@@ -1673,9 +1686,13 @@ BwdLayout bwd_layout(int64_t T, int B, int n, int dtype, int cells) {
   // rows in frames of 8, or of more than 8 rows in frames of 16: never more than 2B + 16 rows in all
   l.off_ex = off;
   if (n % 16 == 0) off = align_up(off + (size_t)kExRing * 4 * n * esize(dtype) * (2 * (size_t)B + 16), 256);
-  // the XCDs' rings of k_lstm2_bwd_wide
+  // the XCDs' rings of k_lstm2_bwd_wide, where one call or those that share a launch can come to it (n = 2048: 8 MB)
   l.off_exl = off;
-  if (dtype == RTN_DTYPE_BF16 && bwd_wide_build((4 * n / 32 + kWaves - 1) / kWaves).kernel) off = align_up(off + (size_t)kBwdWideRings * kExRing * 4 * n * esize(dtype) * 16, 256);
+  if (dtype == RTN_DTYPE_BF16 && bwd_wide_build((4 * n / 32 + kWaves - 1) / kWaves).kernel) {
+    bool wide = false;
+    for (int count = 1; count <= kMaxBwdMulti; ++count) wide = wide || bwd_wide_spares_launches(count, B, n, device_info().cus);
+    if (wide) off = align_up(off + (size_t)kBwdWideRings * kExRing * 4 * n * esize(dtype) * 16, 256);
+  }
   // the weight gradient's slices and y0^T dx0, of the caller's width (float32 324 has 4 slices, more bytes than the 3 of 352) and as many as
   // all frames' rows need (129 of n = 64 are 8 MB, a single frame has 2)
   l.off_part = off;
@@ -2364,16 +2381,11 @@ int choose_bwd_kernel(const BwdCtx& x, BwdChoice* out) {
     }
   }
   // Layers whose W takes a CU's registers and LDS: two tiles per workgroup and four groups at once.
-  // Its launch takes longer than one of k_lstm2_bwd_regw, which reads as much per workgroup and multiplies half: it has to
-  // spare more than a fifth of the launches.  (us per gradient call of 64 frames, one tile / two: as many launches n = 1088, 80 rows 705 / 751, n = 1280, 40 rows
-  // 419 / 469, n = 2048, 32 rows 429 / 536; 3 launches for 4, n = 1280, 192 rows 1692 / 1367; 2 for 3, n = 1408, 96 rows 998 / 827.)
-  // RTN_LSTM2_BWD_WIDE: 0 never, 2 wherever it fits.
-  if (dtype == RTN_DTYPE_BF16 && !env_mt && !env_rows && !env_waves && count <= kBwdWideSlots && env_long("RTN_LSTM2_BWD_WIDE", 1)) {
+  if (dtype == RTN_DTYPE_BF16 && !env_mt && !env_rows && !env_waves) {
     const int steps = (S + kWaves - 1) / kWaves, groups = (B + 15) / 16, per = kBwdWideSlots / count, xpg = di.xcds / kBwdWideSlots;
-    const int one_tile = std::max(1, di.cus / (n / 16) / count), turns_of_one_tile = (groups + one_tile - 1) / one_tile;
     const BwdWideBuild wb = bwd_wide_build(steps);
     const int kb = wb.kernel ? n / (16 * wb.tiles) : 0;
-    if (wb.kernel && n % (16 * wb.tiles) == 0 && di.xcds <= kBwdWideRings && di.xcds % kBwdWideSlots == 0 && kb % xpg == 0 && (env_long("RTN_LSTM2_BWD_WIDE", 1) == 2 || 5 * ((groups + per - 1) / per) < 4 * turns_of_one_tile)) {
+    if (wb.kernel && n % (16 * wb.tiles) == 0 && di.xcds <= kBwdWideRings && di.xcds % kBwdWideSlots == 0 && kb % xpg == 0 && bwd_wide_spares_launches(count, B, n, di.cus)) {
       const int members = kb / xpg, pieces = S * 4 * 16;  // workgroups of a group on one XCD; fragments of a frame
       const size_t lds = (size_t)kWaves * wb.lds_fragments * 64 * 16;
       int per_cu = 0;
@@ -2607,6 +2619,9 @@ int bwd_launch_persistent(const BwdCtx& x, const BwdChoice& ch, const BwdLayout&
   multi.local = ch.local ? 1 : 0;
   multi.xcds = device_info().xcds;
   multi.slots = ch.slots;
+  const long long xcd_ring_words = ch.slots ? (long long)((size_t)multi.xcds * kExRing * 4 * n * x.es * 16 / 4) : 0;
+  if ((size_t)xcd_ring_words * 4 > lay.off_part - lay.off_exl)
+    return fail(RTN_ERR_WORKSPACE, "NativeLstm2 backward: internal: XCDs' rings of %lld bytes do not fit their section", xcd_ring_words * 4);
   const int wgs_per_group = n / (16 * ch.tiles);
   for (int g0 = 0; g0 < bgroups; g0 += ch.groups_per_launch) {
     const int groups_now = std::min(ch.groups_per_launch, bgroups - g0);
@@ -2624,8 +2639,7 @@ int bwd_launch_persistent(const BwdCtx& x, const BwdChoice& ch, const BwdLayout&
     }
     if (ch.slots) {
       grid = (unsigned)(ch.slots * wgs_per_group);
-      const long long words = (long long)((size_t)multi.xcds * kExRing * 4 * n * x.es * 16 / 4);
-      for (int k = 0; k < count; ++k) hipLaunchKernelGGL(k_fill_u32, dim3(512), fill_block, 0, x.stream, (unsigned*)multi.q[k].exl, ~0u, words);
+      for (int k = 0; k < count; ++k) hipLaunchKernelGGL(k_fill_u32, dim3(512), fill_block, 0, x.stream, (unsigned*)multi.q[k].exl, ~0u, xcd_ring_words);
       RTN_HIP(hipGetLastError());
     }
     const int rc = launch_coresident(ch.kernel, dim3(grid), dim3((unsigned)(64 * ch.waves)), args, (unsigned)ch.lds, x.stream, x.capturing);

@@ -105,6 +105,26 @@ def test_range_and_argument_errors(cabi):
     assert _call(cabi, 3, 2, 3, mode=lib.MODE_PERSISTENT) == lib.RTN_ERR_UNSUPPORTED
 
 
+def test_gradient_workspace_has_the_xcd_rings_of_calls_that_use_them(cabi):
+    """The gradient of wide layers has a ring per XCD (8 rings of 4 frames of 16 rows) behind its other sections, up from 17 rows: with fewer no number of
+    problems in one launch makes four groups of 16 rows at once the better choice.  RTN_LSTM2_BWD_WIDE=2 asks for it with any number of rows."""
+    from _gpu_util import env
+
+    size = lambda B, n: int(cabi.rtn_native_lstm2_bwd_workspace_bytes(20, B, n, lib.DTYPE_BF16))  # noqa: E731
+    for n in (1280, 2048):
+        rings = 8 * 4 * 4 * n * 2 * 16
+        row = size(16, n) - size(15, n)
+        assert size(2, n) - size(1, n) <= row + 1024
+        # (the smallest width: three groups of 16 rows per launch, four of them are the first that it spares a launch)
+        first = 17 if n == 2048 else next(B for B in range(17, 200, 16) if size(B, n) - size(B - 1, n) > rings)
+        assert rings - 1024 <= size(first, n) - size(first - 1, n) - row <= rings + 1024, (n, row)
+        small = size(4, n)
+        with env(RTN_LSTM2_BWD_WIDE=2):
+            assert rings - 1024 <= size(4, n) - small <= rings + 1024
+        with env(RTN_LSTM2_BWD_WIDE=0):
+            assert size(64, n) - size(63, n) <= row + 1024
+
+
 def test_workspace_and_plan(cabi):
     # benchmark configuration cfg3 (returnn_amd/synthetic.py): bf16, T=1000, B=32, n=1024: persistent, all weights on chip
     text = lib.describe_plan(1000, 32, 1024, lib.DTYPE_BF16, lib.MODE_AUTO)
