@@ -467,6 +467,8 @@ __global__ __launch_bounds__(64 * WV) void k_lstm2_bwd_regw(const Lstm2BwdMulti 
   long long idx[PT], io[PT];
   unsigned off_h[PT], off_dy[PT], off_c[PT];  // byte offsets inside a frame of H, DY and C; out of range (0 comes back) for cells beyond nc
   float dyw[PT], dc[PT], dx0[PT][4];
+  // (no branch around the load: behind one that some lanes skip, a full register file has cost those lanes values)
+  __amdgpu_buffer_rsrc_t rs_dd = __builtin_amdgcn_make_buffer_rsrc((void*)q.Dd, 0, q.Dd ? (unsigned)(bn * 4) : 0u, kBufFlags);
 #pragma unroll
   for (int j = 0; j < PT; ++j) {
     const int mt = tile_of(j);
@@ -478,7 +480,7 @@ __global__ __launch_bounds__(64 * WV) void k_lstm2_bwd_regw(const Lstm2BwdMulti 
     off_dy[j] = k < nc ? (unsigned)(((long long)b * p.ldDY + k) * ES) : kOobOffset;
     off_c[j] = k < nc ? (unsigned)(idx[j] * 4) : kOobOffset;
     dyw[j] = 0.f;
-    dc[j] = act[j] && q.Dd ? q.Dd[idx[j]] : 0.f;
+    dc[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs_dd, act[j] ? off_c[j] : kOobOffset, 0, 0));
 #pragma unroll
     for (int gq = 0; gq < 4; ++gq) dx0[j][gq] = 0.f;
   }

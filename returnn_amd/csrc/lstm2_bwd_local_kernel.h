@@ -218,6 +218,8 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_bwd_local(const Lstm2BwdMu
   unsigned off_gates[PT], off_h0[PT], off_dy[PT], off_c[PT];  // byte offsets inside a frame of H (gate lane % 4 of the quad's cells; the pair's own first block), DY and C; out of range (0 comes back) for cells beyond nc
   unsigned ring_at[PT], dx_at[PT];  // where the four cells of gate lane % 4 go, inside a frame of the ring and of DX (out of range: nowhere)
   float dyw[PT], dc[PT], dx0[PT][4];
+  // (no branch around the load: behind one that some lanes skip, a full register file has cost those lanes values)
+  __amdgpu_buffer_rsrc_t rs_dd = __builtin_amdgcn_make_buffer_rsrc((void*)q.Dd, 0, q.Dd ? (unsigned)(bn * 4) : 0u, kBufFlags);
 #pragma unroll
   for (int j = 0; j < PT; ++j) {
     const int mt = tile_of(j);
@@ -233,7 +235,7 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_bwd_local(const Lstm2BwdMu
     ring_at[j] = bl < rows ? (unsigned)((((gate * n + first) / KE * 8 + bl) * KE + first % KE) * ES) : kOobOffset;
     dx_at[j] = bl < rows && first < nc ? (unsigned)(((long long)b * p.ldDX + (long long)gate * nc + first) * ES) : kOobOffset;
     dyw[j] = 0.f;
-    dc[j] = act[j] && q.Dd ? q.Dd[idx[j]] : 0.f;
+    dc[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs_dd, act[j] ? off_c[j] : kOobOffset, 0, 0));
 #pragma unroll
     for (int gq = 0; gq < 4; ++gq) dx0[j][gq] = 0.f;
   }

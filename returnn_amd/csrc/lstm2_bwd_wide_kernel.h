@@ -106,6 +106,8 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_bwd_wide(const Lstm2BwdMul
   bool act[MT];
   unsigned off_h[MT], off_dy[MT], off_c[MT];  // byte offsets inside a frame; out of range (0 comes back) for cells beyond nc
   float dyw[MT], dc[MT], dx0[MT][4];
+  // (no branch around the load: behind one that some lanes skip, a full register file has cost those lanes values)
+  __amdgpu_buffer_rsrc_t rs_dd = __builtin_amdgcn_make_buffer_rsrc((void*)q.Dd, 0, q.Dd ? (unsigned)(bn * 4) : 0u, kBufFlags);
 #pragma unroll
   for (int j = 0; j < MT; ++j) {
     const int k = k0 + 16 * j + kl;
@@ -114,7 +116,7 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_bwd_wide(const Lstm2BwdMul
     off_dy[j] = k < nc ? (unsigned)(((long long)b * p.ldDY + k) * ES) : kOobOffset;
     off_c[j] = k < nc ? (unsigned)(((long long)b * nc + k) * 4) : kOobOffset;
     dyw[j] = 0.f;
-    dc[j] = act[j] && q.Dd ? q.Dd[(long long)b * nc + k] : 0.f;
+    dc[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs_dd, act[j] ? off_c[j] : kOobOffset, 0, 0));
 #pragma unroll
     for (int gq = 0; gq < 4; ++gq) dx0[j][gq] = 0.f;
   }

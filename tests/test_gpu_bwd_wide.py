@@ -71,3 +71,34 @@ def test_recorded_gradients_agree_with_eager_ones():
                         assert float((a - b).abs().max()) <= 1e-5 * float(b.abs().max()), (k, name)
                     else:
                         assert torch.equal(a, b) and torch.equal(c, b), (k, name)
+
+
+def _gradients(problems, dtype="bf16"):
+    """:param problems: of (T, B, n); -> the gradients of all of them, as one call"""
+    calls = []
+    for k, (T, B, n) in enumerate(problems):
+        X, W, y0, c0, i = random_problem(41 + k, T, B, n)
+        rng = numpy.random.default_rng(42 + k)
+        Xd, Wd, y0d, c0d, id_ = to_dev(X, dtype), to_dev(W, dtype), to_dev(y0, dtype), to_dev(c0, "f32"), to_dev(i, "f32")
+        Y, C, H, _ = get_op()(Xd, Wd, y0d, c0d, id_, 0, (1, -1)[k % 2])
+        DY, Dd = to_dev(rng.normal(0, 1, (T, B, n)), dtype), to_dev(rng.normal(0, 1, (B, n)), "f32")
+        calls.append((Wd, y0d, c0d, id_, 0, (1, -1)[k % 2], Y, C, H, DY, Dd))
+    got = torch_native_op.native_lstm2_grad_multi(calls)
+    return got, lib.bwd_plan_text(), calls
+
+
+def test_no_error_on_the_final_state_is_an_error_of_zero():
+    announce("wide gradient without Dd")
+    T, B, n = 4, 40, 1152
+    with env(RTN_LSTM2_BWD_WIDE=2):
+        _, _, calls = _gradients([(T, B, n)])
+        W, y0, c0, i, _, _, Y, C, H, DY, Dd = calls[0]
+        want = torch_native_op.native_lstm2_grad(*calls[0][:-1], torch.zeros_like(Dd))
+        got = [torch.full_like(t, float("nan")) for t in want]
+        c = lib.Lstm2BwdCall(*(t.data_ptr() for t in (W, y0, c0, i)), 0, 1, *(t.data_ptr() for t in (Y, C, H, DY)), None, *(t.data_ptr() for t in got), 0, 0, 0, None, 1)
+        ws = torch.empty(int(lib.load().rtn_native_lstm2_bwd_multi_workspace_bytes(1, T, B, n, lib.DTYPE_BF16)), dtype=torch.uint8, device="cuda")
+        lib.check(lib.load().rtn_native_lstm2_bwd_multi((lib.Lstm2BwdCall * 1)(c), 1, T, B, n, lib.DTYPE_BF16, ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream))
+        torch.cuda.synchronize()
+        assert "name=k_lstm2_bwd_wide" in lib.bwd_plan_text()
+    for name, x, y in zip(("DX", "Dy0", "Dc0"), (got[0], got[2], got[3]), (want[0], want[2], want[3])):
+        assert torch.equal(x, y), name
