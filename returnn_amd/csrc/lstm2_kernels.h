@@ -1818,6 +1818,9 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_regw(const Lstm2Multi mult
 #pragma unroll
   for (int j = 0; j < EPT; ++j)
     if (e_valid[j]) {
+      // (the tail's cells of the last frame, which went out by themselves)
+      if (expired && has_tail && (int)e_cl[j] >= tail_x)
+        E::store(p.Y, ((long long)frame_of(p, nsteps - 1) * p.B + b_base + e_row[j]) * p.ldY + cell0 + (int)e_cl[j], __builtin_nanf(""));
       const long long bc = (long long)(b_base + e_row[j]) * nc + 4 * MT * r + e_cl[j];
       p.d[bc] = expired ? __builtin_nanf("") : c_state[j];
       if (p.hN) E::store(p.hN, bc, expired ? __builtin_nanf("") : h_prev[j]);

@@ -459,6 +459,8 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_sparse(const Lstm2Multi mu
     if (expired && s0 + wave == nsteps - 1) fy = CK::fill(kNanWords<AT>);
     flush_yc(s0);
   }
+  if (expired && has_tail && in_tail && nsteps > 0)  // (the tail's cells of the last frame, which went out by themselves)
+    E::store(p.Y, ((long long)frame_of(p, nsteps - 1) * p.B + b_base + row) * p.ldY + cell, __builtin_nanf(""));
   if (valid) {
     const long long bc = (long long)(b_base + row) * nc + cell;
     p.d[bc] = expired ? __builtin_nanf("") : c_state;

@@ -541,6 +541,37 @@ def test_bounded_wait_expires_cleanly():
         check_f32(got, oracle.native_lstm2_fwd(*p, 0, 1)[:4], "after bounded wait")
 
 
+# widths that cut a workgroup's cells, of both register kernels and in both types: the columns behind the cut leave by themselves
+@pytest.mark.parametrize("T,B,n,dtype", [(40, 32, 1001, "bf16"), (40, 100, 1001, "bf16"), (40, 32, 509, "f32"), (40, 40, 301, "f32"), (40, 32, 1333, "bf16"), (9, 4, 2100, "bf16")])
+def test_expired_wait_marks_every_column(T, B, n, dtype):
+    """
+    Where a wait that expired leaves NaN in the final cell state, the last frame of Y is NaN as well, in every column.  Products on another stream
+    hold some workgroups back, so that those that run wait for them, with a bound of zero ticks (not in every call: the widths with groups over all XCDs
+    mostly do).
+    """
+    from returnn_amd import lib
+
+    announce("bounded wait, cut widths", T, B, n, dtype)
+    p = random_problem(62, T, B, n, ragged=False)
+    side, a = torch.cuda.Stream(), torch.zeros((4096, 4096), device="cuda")
+    for _ in range(3):
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side):
+            for _ in range(100):
+                a @ a
+        with env(RTN_LSTM2_TIMEOUT_TICKS=0):
+            rc, status, (Y, _, _, d) = run_raw(*p, 0, 1, dtype=dtype, mode="persistent")
+        assert rc == 0 and status in (lib.RTN_OK, lib.RTN_ERR_ABORTED)
+        print("status", status, "NaN in d", int(numpy.isnan(d).sum()), "of", d.size)
+        assert numpy.isnan(d).any() == (status == lib.RTN_ERR_ABORTED)
+        assert numpy.isnan(Y[-1])[numpy.isnan(d)].all(), numpy.unique(numpy.nonzero(numpy.isnan(d) & ~numpy.isnan(Y[-1]))[1])
+        if status == lib.RTN_ERR_ABORTED:
+            break
+    torch.cuda.synchronize()
+    rc, status, got = run_raw(*p, 0, 1, dtype=dtype, mode="persistent")
+    assert rc == 0 and status == 0 and all(numpy.isfinite(x).all() for x in got)
+
+
 def test_expired_wait_reaches_the_torch_caller():
     """The same forced expiry through the torch op: the status watch raises at the next look (lazily, without
     waiting for the device, or at once in its synchronous setting) exactly when the outputs carry the NaN marks."""
