@@ -8,6 +8,8 @@ import torch
 
 from returnn_amd import lib, torch_native_op
 
+import test_gpu_bwd
+import test_gpu_siblings as siblings
 from _gpu_util import announce, env, get_op, random_problem, to_dev
 from test_gpu_bwd import _rel_to_max, _run
 
@@ -87,6 +89,41 @@ def _gradients(problems, dtype="bf16"):
     return got, lib.bwd_plan_text(), calls
 
 
+# both sides of the rule: as many launches as with one tile per workgroup, 2 for 3, 1 for 2; problems that share a launch
+@pytest.mark.parametrize(
+    "count,B,n,wide",
+    [(1, 64, 2048, True), (1, 32, 2048, False), (2, 32, 2048, True), (2, 16, 2048, False), (1, 64, 1280, True), (1, 40, 1280, False), (1, 80, 1088, False), (1, 96, 1408, True)],
+)
+def test_rule_takes_it_where_it_spares_launches(count, B, n, wide):
+    """Without an override; the general kernel splits the contraction in another way: equal to one bfloat16 step of the largest magnitude."""
+    announce("wide gradient, rule", count, B, n)
+    problems = [(3, B, n)] * count
+    got, plan, _ = _gradients(problems)
+    assert ("name=k_lstm2_bwd_wide" in plan) == wide and ("name=k_lstm2_bwd_regw" in plan) != wide, plan
+    if wide:
+        with env(RTN_LSTM2_BWD_WIDE=0):
+            want, plan, _ = _gradients(problems)
+        assert "name=k_lstm2_bwd_regw" in plan, plan
+        for a, b in zip(got, want):
+            for name, x, y in zip(("DX", "DW", "Dy0", "Dc0"), a, b):
+                assert bool(torch.isfinite(x).all()) and float((x.float() - y.float()).abs().max()) <= 2.0**-7 * float(y.float().abs().max()), name
+
+
+# (a launch takes two problems; calls with more run one by one)
+@pytest.mark.parametrize("count,last", [(2, 2), (3, 1)])
+def test_problems_with_groups_of_their_own(count, last):
+    announce("wide gradient, problems", count)
+    problems = [(5, 16, 1152)] * count
+    with env(RTN_LSTM2_BWD_WIDE=2):
+        got, plan, calls = _gradients(problems)
+        assert "problems=%i" % last in plan and "name=k_lstm2_bwd_wide" in plan, plan
+        alone = [torch_native_op.native_lstm2_grad(*c) for c in calls]
+        assert "name=k_lstm2_bwd_wide" in lib.bwd_plan_text()
+    for a, b in zip(got, alone):
+        for name, x, y in zip(("DX", "Dy0", "Dc0"), (a[0], a[2], a[3]), (b[0], b[2], b[3])):
+            assert torch.equal(x, y), name
+
+
 def test_no_error_on_the_final_state_is_an_error_of_zero():
     announce("wide gradient without Dd")
     T, B, n = 4, 40, 1152
@@ -102,3 +139,21 @@ def test_no_error_on_the_final_state_is_an_error_of_zero():
         assert "name=k_lstm2_bwd_wide" in lib.bwd_plan_text()
     for name, x, y in zip(("DX", "Dy0", "Dc0"), (got[0], got[2], got[3]), (want[0], want[2], want[3])):
         assert torch.equal(x, y), name
+
+
+def test_other_ops_on_the_same_kernel():
+    """LstmGenericBase (cell states in H, nothing carried over a masked frame) and LstmLowMem (errors of the output before the mask)."""
+    with env(RTN_LSTM2_BWD_WIDE=2):
+        siblings.test_generic_base_gradient(5, 40, 1152, "bf16")
+        assert "name=k_lstm2_bwd_wide" in lib.bwd_plan_text(), lib.bwd_plan_text()
+        announce("wide gradient, low_mem")
+        got, want = siblings._low_mem_grad_case(60, 5, 40, 64, 1152, 0, 1, "bf16")
+        assert "name=k_lstm2_bwd_wide" in lib.bwd_plan_text(), lib.bwd_plan_text()
+    for a, b in zip(got, want):
+        assert numpy.isfinite(a).all() and _rel_to_max(a, b) <= 3e-2, _rel_to_max(a, b)  # (the bound of that op's other tests)
+
+
+def test_bounded_wait_expires_cleanly():
+    with env(RTN_LSTM2_BWD_WIDE=2):
+        test_gpu_bwd.test_bwd_bounded_wait_expires_cleanly(6, 40, 1152, "bf16")
+        assert "name=k_lstm2_bwd_wide" in lib.bwd_plan_text(), lib.bwd_plan_text()
