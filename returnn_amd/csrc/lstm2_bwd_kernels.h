@@ -426,7 +426,7 @@ __global__ __launch_bounds__(64 * WV) void k_lstm2_bwd_regw(const Lstm2BwdMulti 
 
   // An XCD-local plan rests on all workgroups of a group being on one XCD: checked here.
   __shared__ int s_local;
-  if (tid == 0) s_local = multi.local ? (int)group_on_one_xcd(q.sync + 2 * (size_t)g, (unsigned)kblocks, q.status, q.timeout_ticks) : 0;
+  if (wave == 0) s_local = multi.local ? (int)group_on_one_xcd(q.sync + 2 * (size_t)g, (unsigned)kblocks, q.status, q.timeout_ticks) : 0;
   __syncthreads();
   const bool local = s_local != 0;
 

@@ -158,7 +158,7 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_bwd_local(const Lstm2BwdMu
 
   // An XCD-local plan rests on all workgroups of a group being on one XCD: checked here.
   __shared__ int s_local;
-  if (tid == 0) s_local = (int)group_on_one_xcd(q.sync + 2 * (size_t)g, (unsigned)kblocks, q.status, q.timeout_ticks);
+  if (wave == 0) s_local = (int)group_on_one_xcd(q.sync + 2 * (size_t)g, (unsigned)kblocks, q.status, q.timeout_ticks);
   __syncthreads();
   const bool local = s_local != 0;
 

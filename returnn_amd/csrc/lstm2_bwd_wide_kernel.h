@@ -63,7 +63,7 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_bwd_wide(const Lstm2BwdMul
   __shared__ f32x4 red[kWaves][MT][4 * kRedGroup];
   __shared__ i32x4 stage[4 * KGW * Bp];  // [gate][piece][row]: the workgroup's derivatives of a frame in ring order
   __shared__ int s_one_xcd;
-  if (tid == 0) s_one_xcd = (int)group_on_one_xcd(q.sync + 2 * (size_t)(g * xpg + xcd % xpg), (unsigned)members, q.status, q.timeout_ticks);
+  if (wave == 0) s_one_xcd = (int)group_on_one_xcd(q.sync + 2 * (size_t)(g * xpg + xcd % xpg), (unsigned)members, q.status, q.timeout_ticks);
 
   const unsigned frame_bytes = (unsigned)((size_t)p.B * 4 * nc * ES);
   const unsigned dx_frame_bytes = (unsigned)((size_t)p.B * p.ldDX * ES), dy_frame_bytes = (unsigned)((size_t)p.B * p.ldDY * ES);

@@ -208,7 +208,7 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_dual(const Lstm2Multi mult
 
   // That all workgroups of a group share an XCD is checked (both groups of a workgroup have the same workgroups).
   __shared__ int s_local;
-  if (!SPREAD && tid == 0) s_local = group_on_one_xcd(p.flags + (size_t)group[0] * G, (unsigned)G, p.status, p.timeout_ticks) ? 1 : 0;
+  if (!SPREAD && wave == 0) s_local = group_on_one_xcd(p.flags + (size_t)group[0] * G, (unsigned)G, p.status, p.timeout_ticks) ? 1 : 0;
 
   auto run = [&](auto ex_tag) {
     constexpr int AUXS = decltype(ex_tag)::value == kExDevice ? kAuxDevice : 0, AUXL = kAuxDevice;

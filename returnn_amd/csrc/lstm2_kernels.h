@@ -1000,35 +1000,60 @@ static __global__ void k_probe_xcds(unsigned* mask) {
   if (threadIdx.x == 0) (void)__hip_atomic_fetch_or(mask, 1u << xcc_id(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// One thread per workgroup: are all `members` workgroups that share `words` on one XCD?  Every caller adds its XCD to the
-// mask words[1] and then itself to the count words[0] (both cleared before the launch; device-scope atomics whose result
-// is waited for, so the mask is complete when the count is).  The wait is bounded like every other (status[0] = 1 when it
-// expires; the answer is then "no").  A group found on several XCDs leaves its mask in status[1] for the record.
+// One wavefront per workgroup, all its lanes: are all `members` workgroups that share `words` on one XCD?  Every caller adds itself to the byte of its
+// XCD (8 of them in two words, cleared before the launch; a CU has at most two workgroups of a group, an XCD fewer than 256); the answer is there when the bytes' sum is
+// `members`.  The wait is bounded like every other (status[0] = 1 when it expires; the answer is then "no").  A group found on
+// several XCDs leaves their mask in status[1] for the record.
+// No lane is switched off: all but one have an address out of range for the addition, what else they do is the same.  (A block of one lane stood here,
+// around which the compiler parks values in accumulation registers where a kernel fills the register file, and it has done so behind the block while the
+// other lanes were still off: see tests/test_generated_code.py.)
 __device__ __forceinline__ bool group_on_one_xcd(unsigned* words, unsigned members, unsigned* status, unsigned long long timeout_ticks) {
   if (members <= 1) return true;
-  (void)__hip_atomic_fetch_or(words + 1, 1u << xcc_id(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  (void)__hip_atomic_fetch_add(words, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const unsigned lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0)), xcd = xcc_id() & 7u;
+  __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)words, 0, 8u, kBufFlags);
+  (void)__builtin_amdgcn_raw_ptr_buffer_atomic_add_i32((int)(1u << (8 * (xcd & 3))), rs, lane == 0 ? 4 * (xcd >> 2) : 0x80000000u, 0, 0);
   unsigned long long t0 = 0;
-  unsigned spins = 0;
+  unsigned spins = 0, lo, hi;
   bool complete = true;
-  while (__hip_atomic_load(words, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < members) {
+  for (;;) {
+    asm volatile("" ::: "memory");  // (really load again)
+    const auto both = __builtin_amdgcn_raw_buffer_load_b64(rs, 0, 0, kAuxDevice);
+    lo = (unsigned)__builtin_amdgcn_readfirstlane((int)both[0]);
+    hi = (unsigned)__builtin_amdgcn_readfirstlane((int)both[1]);
+    const unsigned pairs = (lo & 0x00FF00FFu) + ((lo >> 8) & 0x00FF00FFu) + (hi & 0x00FF00FFu) + ((hi >> 8) & 0x00FF00FFu);
+    if ((pairs & 0xFFFFu) + (pairs >> 16) >= members) break;
     if ((spins++ & 15u) == 0) {
-      if (__hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) { complete = false; break; }
+      const unsigned ended = (unsigned)__builtin_amdgcn_readfirstlane((int)__hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
       const unsigned long long now = wall_clock64();
-      if (spins == 1) {
-        t0 = now;
-      } else if (now - t0 > timeout_ticks) {
-        __hip_atomic_store(status, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (ended == 0 && spins > 1 && now - t0 > timeout_ticks) __hip_atomic_store(status, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (ended != 0 || (spins > 1 && now - t0 > timeout_ticks)) {
         complete = false;
         break;
       }
+      if (spins == 1) t0 = now;
     }
     __builtin_amdgcn_s_sleep(2);
   }
-  const unsigned mask = __hip_atomic_load(words + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  unsigned mask = 0;
+#pragma unroll
+  for (int x = 0; x < 4; ++x) mask |= ((lo >> (8 * x) & 0xFFu) ? 1u << x : 0u) | ((hi >> (8 * x) & 0xFFu) ? 16u << x : 0u);
   const bool ok = complete && (mask & (mask - 1)) == 0;
   if (!ok) __hip_atomic_store(status + 1, mask, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   return ok;
+}
+
+// c0 and y0 of element `at` of [B, nc]; zeros where the pair does not exist.  Without a branch (see group_on_one_xcd).
+template <typename AT>
+__device__ __forceinline__ void start_state(const Lstm2Params& p, bool valid, int at, float* c, float* h) {
+  constexpr unsigned ES = sizeof(AT);
+  const unsigned count = (unsigned)(p.B * p.nc);  // (below 2^27)
+  __amdgpu_buffer_rsrc_t rs_c = __builtin_amdgcn_make_buffer_rsrc((void*)p.c0, 0, count * 4, kBufFlags);
+  __amdgpu_buffer_rsrc_t rs_y = __builtin_amdgcn_make_buffer_rsrc((void*)p.y0, 0, count * ES, kBufFlags);
+  *c = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs_c, valid ? (unsigned)at * 4 : kOobOffset, 0, 0));
+  if constexpr (ES == 2)
+    *h = __builtin_bit_cast(float, (unsigned)(unsigned short)__builtin_amdgcn_raw_buffer_load_b16(rs_y, valid ? (unsigned)at * ES : kOobOffset, 0, 0) << 16);
+  else
+    *h = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs_y, valid ? (unsigned)at * ES : kOobOffset, 0, 0));
 }
 
 // Float32 products in quads of rows (see k_lstm2_regw).
@@ -1310,7 +1335,12 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_regw(const Lstm2Multi mult
     }
   }
 
-  // The (sequence, cell) pairs whose state this thread keeps.
+  // The (sequence, cell) pairs whose state this thread keeps: tile, row and cell inside the workgroup's of pass u.
+  auto pair_of = [](int u, int lane, int* e, int* bl, int* cl) {
+    *e = HALF && !QUAD ? 2 * u + ((lane >> 3) & 1) : u;
+    *bl = QUAD ? 4 * (u % (QUAD ? RQ : 1)) + (lane & 3) : HALF ? lane & 7 : 16 * (*e % NT) + (lane & 15);
+    *cl = QUAD ? 16 * (u / (QUAD ? RQ : 1)) + (lane >> 2) : 4 * (*e / NT) + (lane >> 4);
+  };
   float c_state[EPT], h_prev[EPT];
   bool e_valid[EPT];
   unsigned e_hoff[EPT];            // byte offset of the pair's element in an exchange buffer
@@ -1319,21 +1349,9 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_regw(const Lstm2Multi mult
 #pragma unroll
   for (int j = 0; j < EPT; ++j) {
     const int u = min(wave + kWaves * j, UNITS - 1);
-    int e, bl, src;
-    if (QUAD) {
-      e = u;
-      bl = 4 * (u % RQ) + (lane & 3);
-      src = lane;
-    } else if (HALF) {
-      e = 2 * u + ((lane >> 3) & 1);
-      bl = lane & 7;
-      src = (lane & 0x30) | bl;
-    } else {
-      e = u;
-      bl = 16 * (e % NT) + (lane & 15);
-      src = lane;
-    }
-    const int cl = QUAD ? 16 * (u / RQ) + (lane >> 2) : 4 * (e / NT) + (lane >> 4);  // cell inside the workgroup's
+    int e, bl, cl, src = lane;
+    pair_of(u, lane, &e, &bl, &cl);
+    if (HALF && !QUAD) src = (lane & 0x30) | bl;
     const int cell = 4 * r * MT + cl;
     e_tile[j] = (unsigned)e;
     e_src[j] = (unsigned)src;
@@ -1341,13 +1359,7 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_regw(const Lstm2Multi mult
     e_cl[j] = (unsigned)cl;
     e_valid[j] = (wave + kWaves * j < UNITS) && (bl < rows) && cell < nc;
     e_hoff[j] = (unsigned)((((cell / KE) * p.Bp + bl) * KE + (cell % KE)) * ES);
-    c_state[j] = 0.f;
-    h_prev[j] = 0.f;
-    if (e_valid[j]) {
-      const long long bc = (long long)(b_base + bl) * nc + cell;
-      c_state[j] = p.c0[bc];
-      h_prev[j] = E::load(p.y0, bc);
-    }
+    start_state<AT>(p, e_valid[j], (b_base + bl) * nc + cell, &c_state[j], &h_prev[j]);
   }
   // The tail: first cell (inside this workgroup's tile) of the chunk of X, H and Y, and of C, that the width cuts.
   const int tail_x = nc - nc % (CH / ES) - cell0, tail_c = nc - nc % 4 - cell0;
@@ -1372,7 +1384,7 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_regw(const Lstm2Multi mult
   // atomics whose result is waited for, so the mask is complete when the count is); with one XCD in the mask the hidden
   // state travels through that XCD's L2 (plain stores, loads that bypass the first-level cache), else with device scope.
   __shared__ int s_local;
-  if (multi.local && tid == 0)
+  if (multi.local && wave == 0)
     s_local = group_on_one_xcd(p.flags + (size_t)g * p.wgs_per_group, (unsigned)p.wgs_per_group, p.status, p.timeout_ticks) ? 1 : 0;
 
   auto run = [&](auto ex_tag) {
@@ -1818,13 +1830,23 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_regw(const Lstm2Multi mult
 #pragma unroll
   for (int j = 0; j < EPT; ++j)
     if (e_valid[j]) {
-      // (the tail's cells of the last frame, which went out by themselves)
-      if (expired && has_tail && (int)e_cl[j] >= tail_x)
-        E::store(p.Y, ((long long)frame_of(p, nsteps - 1) * p.B + b_base + e_row[j]) * p.ldY + cell0 + (int)e_cl[j], __builtin_nanf(""));
       const long long bc = (long long)(b_base + e_row[j]) * nc + 4 * MT * r + e_cl[j];
       p.d[bc] = expired ? __builtin_nanf("") : c_state[j];
       if (p.hN) E::store(p.hN, bc, expired ? __builtin_nanf("") : h_prev[j]);
     }
+  if (expired && has_tail) {
+    // The tail's cells of the last frame, which went out by themselves.  (Their places are worked out again, from scalars and the lane's number: kept over the whole
+    // sequence, they were among the values that the compiler parks behind a block of one lane only, see tests/test_generated_code.py.)
+    const int l = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0));
+#pragma unroll
+    for (int j = 0; j < EPT; ++j) {
+      const int u = wave + kWaves * j;
+      int e, bl, cl;
+      pair_of(min(u, UNITS - 1), l, &e, &bl, &cl);
+      if (u < UNITS && bl < rows && cl >= tail_x && cell0 + cl < nc)
+        E::store(p.Y, ((long long)frame_of(p, nsteps - 1) * p.B + b_base + bl) * p.ldY + cell0 + cl, __builtin_nanf(""));
+    }
+  }
 }
 
 

@@ -216,12 +216,8 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_sparse(const Lstm2Multi mu
   for (int q = 0; q < 4; ++q) goff[q] = (unsigned)(row * (16 * XROW) + ((q * CPS + unit) ^ sw_x(row)) * 16 + (lane & 7) * ES);
   const unsigned y_in = (unsigned)(row * 16 * CPS + (unit ^ sw_y(row)) * 16 + (lane & 7) * ES);
   const unsigned c_in = (unsigned)(row * 16 * MT + (unit ^ sw_c(row)) * 32 + (lane & 7) * 4);
-  float c_state = 0.f, h_prev = 0.f;
-  if (valid) {
-    const long long bc = (long long)(b_base + row) * nc + cell;
-    c_state = p.c0[bc];
-    h_prev = E::load(p.y0, bc);
-  }
+  float c_state, h_prev;
+  start_state<AT>(p, valid, (b_base + row) * nc + cell, &c_state, &h_prev);
   // The tail (see k_lstm2_regw): first cell of the chunk of X, H and Y, and of C, that the width cuts.
   const int tail_x = nc - nc % 8 - cell0, tail_c = nc - nc % 4 - cell0;
   const bool has_tail = TAIL && nc % 8 != 0 && tail_x >= 0 && tail_x < CELLS;  // uniform over the workgroup
@@ -236,7 +232,7 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_sparse(const Lstm2Multi mu
   };
 
   __shared__ int s_local;  // (that all workgroups of a group share an XCD is checked, as in k_lstm2_regw)
-  if (tid == 0)
+  if (wave == 0)
     s_local = group_on_one_xcd(p.flags + (size_t)g * p.wgs_per_group, (unsigned)p.wgs_per_group, p.status, p.timeout_ticks) ? 1 : 0;
 
   auto run = [&](auto ex_tag) {
@@ -459,12 +455,15 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_sparse(const Lstm2Multi mu
     if (expired && s0 + wave == nsteps - 1) fy = CK::fill(kNanWords<AT>);
     flush_yc(s0);
   }
-  if (expired && has_tail && in_tail && nsteps > 0)  // (the tail's cells of the last frame, which went out by themselves)
-    E::store(p.Y, ((long long)frame_of(p, nsteps - 1) * p.B + b_base + row) * p.ldY + cell, __builtin_nanf(""));
   if (valid) {
     const long long bc = (long long)(b_base + row) * nc + cell;
     p.d[bc] = expired ? __builtin_nanf("") : c_state;
     if (p.hN) E::store(p.hN, bc, expired ? __builtin_nanf("") : h_prev);
+  }
+  if (expired && has_tail) {  // the tail's cells of the last frame, which went out by themselves (see k_lstm2_regw)
+    const int l = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0)), bl = l >> 3, in = 8 * unit + (l & 7);
+    if (active && bl < rows && in >= tail_x && cell0 + in < nc)
+      E::store(p.Y, ((long long)frame_of(p, nsteps - 1) * p.B + b_base + bl) * p.ldY + cell0 + in, __builtin_nanf(""));
   }
 }
 

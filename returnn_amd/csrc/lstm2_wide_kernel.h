@@ -133,12 +133,7 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_wide(const Lstm2Params p) 
     e_b[j] = 16 * (e % NT) + jl;
     e_own[j] = e < TILES && e_cell[j] < n;
     e_valid[j] = e_own[j] && e_b[j] < rows && e_cell[j] < nc;
-    c_state[j] = h_prev[j] = 0.f;
-    if (e_valid[j]) {
-      const long long bc = (long long)(b_base + e_b[j]) * nc + e_cell[j];
-      c_state[j] = p.c0[bc];
-      h_prev[j] = E::load(p.y0, bc);
-    }
+    start_state<AT>(p, e_valid[j], (b_base + e_b[j]) * nc + e_cell[j], &c_state[j], &h_prev[j]);
   }
 
   // This thread's fragments of the XCD's copy: offsets inside a slot (fragments of rows that do not exist are nobody's).
@@ -157,7 +152,7 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_wide(const Lstm2Params p) 
   const unsigned ks_stride = (unsigned)(4 * kWaves * p.Bp * kFragBytes);  // from one macro step of the share to the next
 
   __shared__ int s_one_xcd;
-  if (tid == 0) s_one_xcd = group_on_one_xcd(p.flags + (size_t)g * G + 2 * xcd, (unsigned)members, p.status, p.timeout_ticks) ? 1 : 0;
+  if (wave == 0) s_one_xcd = group_on_one_xcd(p.flags + (size_t)g * G + 2 * xcd, (unsigned)members, p.status, p.timeout_ticks) ? 1 : 0;
   __syncthreads();
   const bool one_xcd = s_one_xcd != 0;
 
