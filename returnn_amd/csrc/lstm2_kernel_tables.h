@@ -22,7 +22,7 @@ typedef void (*BwdRegwKernel)(const Lstm2BwdMulti);
 // "lo": KSMAX of 2 or 4 macro steps per wavefront, "hi": 8 or 16.
 RegwKernel regw_table_bf16_lo(int MT, int NT, int KSMAX, bool half, bool tail);
 RegwKernel regw_table_bf16_hi(int MT, int NT, int KSMAX, bool half, bool tail);
-RegwKernel regw_table_bf16_16(int MT, int NT, bool half, bool tail);
+RegwKernel regw_table_bf16_16(int MT, int NT, bool tail);
 RegwKernel regw_table_f32_lo(int MT, int NT, int KSMAX, bool half, bool tail);
 RegwKernel regw_table_f32_hi(int MT, int NT, int KSMAX, bool half, bool tail);
 
@@ -76,7 +76,7 @@ RegwKernel regw_table_f32_quad(int MT, int KSMAX, bool tail, int RQ);
 inline RegwKernel regw_kernel(int dtype, int MT, int NT, int KSMAX, bool half, bool tail, int rq) {
   if (rq > 0) return dtype == 0 && NT == 1 ? regw_table_f32_quad(MT, KSMAX, tail, rq) : nullptr;
   if (half && dtype == 1 && two_chains<__bf16>(KSMAX)) return sparse_kernel(MT, KSMAX, tail);
-  if (dtype == 1 && KSMAX == 16) return regw_table_bf16_16(MT, NT, half, tail);
+  if (dtype == 1 && KSMAX == 16) return half ? nullptr : regw_table_bf16_16(MT, NT, tail);
   const bool lo = KSMAX <= 4;
   if (dtype == 1 /* RTN_DTYPE_BF16 */) return lo ? regw_table_bf16_lo(MT, NT, KSMAX, half, tail) : regw_table_bf16_hi(MT, NT, KSMAX, half, tail);
   return lo ? regw_table_f32_lo(MT, NT, KSMAX, half, tail) : regw_table_f32_hi(MT, NT, KSMAX, half, tail);

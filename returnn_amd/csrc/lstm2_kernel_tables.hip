@@ -19,7 +19,7 @@ RegwKernel regw_table(int MT, int NT, int KSMAX, bool half) {
   if (MT == mt && NT == 1 && KSMAX == ks) return &k_lstm2_regw<AT, mt, 1, ks, true, TAIL>;
     if constexpr (sizeof(AT) == 4) {  // (bfloat16: k_lstm2_sparse)
       if constexpr (HI) {
-        RTN_CASE(2, 16) RTN_CASE(2, 8) RTN_CASE(4, 8) RTN_CASE(8, 8)
+        RTN_CASE(2, 8) RTN_CASE(4, 8) RTN_CASE(8, 8)
       } else {
         RTN_CASE(2, 2) RTN_CASE(2, 4)
         RTN_CASE(4, 2) RTN_CASE(4, 4)
@@ -53,8 +53,7 @@ RegwKernel regw_table(int MT, int NT, int KSMAX, bool half) {
 
 // Forward, bfloat16 with 16 macro steps per wavefront.
 template <bool TAIL>
-RegwKernel regw_table_16(int MT, int NT, bool half) {
-  if (half) return MT == 2 && NT == 1 ? &k_lstm2_regw<__bf16, 2, 1, 16, true, TAIL> : nullptr;
+RegwKernel regw_table_16(int MT, int NT) {
 #define RTN_CASE(mt, nt) \
   if (MT == mt && NT == nt) return &k_lstm2_regw<__bf16, mt, nt, 16, false, TAIL>;
   RTN_CASE(1, 1) RTN_CASE(1, 2)
@@ -207,7 +206,7 @@ RegwKernel sparse_kernel(int MT, int KSMAX, bool tail) {
   return nullptr;
 }
 #elif RTN_TABLE_PART == 17
-RegwKernel regw_table_bf16_16(int MT, int NT, bool half, bool tail) { return tail ? regw_table_16<true>(MT, NT, half) : regw_table_16<false>(MT, NT, half); }
+RegwKernel regw_table_bf16_16(int MT, int NT, bool tail) { return tail ? regw_table_16<true>(MT, NT) : regw_table_16<false>(MT, NT); }
 #else
 #error "RTN_TABLE_PART must be 1..17"
 #endif

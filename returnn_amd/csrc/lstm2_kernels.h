@@ -1090,7 +1090,7 @@ __device__ __forceinline__ void quad_macro_step(const i32x4 (&wbits)[MT], const 
    ...);
 }
 
-// HALF: the groups have at most 8 rows (NT == 1, MT even; float32, and bf16 with 16 macro steps per wavefront: k_lstm2_sparse takes fewer).  A tile then holds valid results in the lanes of rows 0..7
+// HALF: the groups have at most 8 rows (NT == 1, MT even; float32: bf16 has k_lstm2_sparse).  A tile then holds valid results in the lanes of rows 0..7
 // only, and the pointwise part folds two tiles into one pass: lanes of rows 0..7 take tile 2u, lanes of rows 8..15 take
 // rows 0..7 of tile 2u + 1, so that a thread owns one (sequence, cell) pair where the plain mapping gives it two, one
 // of them of a row that does not exist.
@@ -1114,7 +1114,7 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_regw(const Lstm2Multi mult
   constexpr bool QUAD = RQ > 0;
   static_assert(!QUAD || (sizeof(AT) == 4 && NT == 1 && MT % 4 == 0 && RQ <= 4), "quads of rows: float32, one batch tile, whole blocks of 64 columns");
   constexpr bool TWO = !QUAD && two_chains<AT>(KSMAX);
-  static_assert(!(TWO && HALF), "groups of up to 8 rows at these widths: k_lstm2_sparse");
+  static_assert(!HALF || sizeof(AT) == 4, "groups of up to 8 rows in bf16: k_lstm2_sparse");
   static_assert(!HALF || (NT == 1 && MT % 2 == 0), "half-tile mapping: one batch tile, an even number of cell tiles");
   // Which of the launch's problems and which (group, rank) this workgroup works on (uniform over the workgroup).
   int which, g, r;
@@ -1602,8 +1602,8 @@ __global__ __launch_bounds__(kWgThreads) void k_lstm2_regw(const Lstm2Multi mult
 #pragma unroll
           for (int u = 0; u < NACC; ++u) {
             acc[u][0] = E::mma(wreg[2 * u + odd][ks], opnd, acc[u][0]);
-            __builtin_amdgcn_sched_group_barrier(0x008, sizeof(AT) == 2 ? 1 : 4, 0);  // the MFMA(s) of one fragment ...
-            __builtin_amdgcn_sched_group_barrier(0x096, 2, 0);                        // ... then up to two of the rest (three: 0-1 % slower; four or five: 2-3 %)
+            __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);  // the MFMAs of one fragment ...
+            __builtin_amdgcn_sched_group_barrier(0x096, 2, 0);  // ... then up to two of the rest
           }
           __builtin_amdgcn_sched_barrier(0);
           opnd = opnd_next;

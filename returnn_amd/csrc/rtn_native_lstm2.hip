@@ -346,7 +346,8 @@ bool make_plan_uncached(int64_t T, int B, int n, int dtype, int want_mode, bool 
           if ((Bg + 15) / 16 > 4) continue;
           const int NT = round_nt((Bg + 15) / 16);
           if (NT * KSMAX > 32 || MT * NT > 8) continue;
-          const bool half = Bg <= 8 && NT == 1 && MT % 2 == 0 && !env_long("RTN_LSTM2_NO_HALF", 0);
+          // (beyond 8 macro steps per wavefront no XCD's CUs hold W; only another number of XCDs than the device's has such plans)
+          const bool half = Bg <= 8 && NT == 1 && MT % 2 == 0 && KSMAX <= 8 && !env_long("RTN_LSTM2_NO_HALF", 0);
           const size_t lds = (size_t)regw_lds((int)es, MT, NT).total;
           if (lds > di.lds_per_wg) continue;
           const int rq = quads(MT, NT, Bg);
