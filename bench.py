@@ -69,7 +69,7 @@ def forward_kernel(plan: str):
     solo = "k_lstm2_solo_row" if "rows_per_group=1 " in plan else "k_lstm2_solo"
     kernel = {"mfma_regw_solo": solo, "mfma_regw_wide": "k_lstm2_wide", "mfma_lds": "k_lstm2_mfma"}.get(name, "k_step_generic")
     if name in ("mfma_regw", "mfma_regw_xcd", "mfma_regw_xcd_half"):
-        kernel = "k_lstm2_dual" if "interleaved=2" in plan else "k_lstm2_regw"
+        kernel = "k_lstm2_dual" if "interleaved=2" in plan else "k_lstm2_sparse" if "product=sparse" in plan else "k_lstm2_regw"
     return kernel, kernel == "k_lstm2_regw"
 
 
@@ -86,7 +86,7 @@ def algorithmic_bytes_per_unit(n: int, dtype: str) -> int:
     return e * 4 * n + e * 4 * n + e * n + 4 * n + 4
 
 
-def ceiling_fields(probe_us, seq_ms, issue_ms, rows, n, dtype, T, call_ms):
+def ceiling_fields(probe_us, between_xcds, seq_ms, issue_ms, rows, n, dtype, T, call_ms):
     """
     Three ceilings of the recurrent GEMM next to the nominal matrix peak.
 
@@ -105,7 +105,8 @@ def ceiling_fields(probe_us, seq_ms, issue_ms, rows, n, dtype, T, call_ms):
     between the CUs that hold W (``probe_us``: the library's latency probe -- device-scope store, visible on every CU,
     device-scope load, at a tiny volume) plus the time the whole chip's matrix cores need for the step's GEMM at their
     peak.  A latency bound, not a roofline: the rate at that bound and ``frac_of_latency_ceiling`` say how far the
-    kernel is from a perfect hand-over.
+    kernel is from a perfect hand-over.  Only where a group's CUs are on several XCDs (``between_xcds``): inside an XCD's L2 a hand-over
+    takes less than the probe's.
     """
     out = {}
     step_flops = 8.0 * n * n * rows
@@ -122,10 +123,11 @@ def ceiling_fields(probe_us, seq_ms, issue_ms, rows, n, dtype, T, call_ms):
             "frac_of_decomposition_ceiling": seq_ms / call_ms,
         })
     if probe_us is not None:
+        out["handover_latency_us"] = probe_us
+    if probe_us is not None and between_xcds:
         mfma_us = step_flops / PEAK_MFMA[dtype] * 1e6
         ceiling_ms = (probe_us + mfma_us) * T * 1e-3
         out.update({
-            "handover_latency_us": probe_us,
             "mfma_peak_us_per_step": mfma_us,
             "latency_ceiling": step_flops * T / (ceiling_ms * 1e-3) / 1e12,
             "frac_of_latency_ceiling": ceiling_ms / call_ms,
@@ -893,8 +895,6 @@ def main():
     call_ms = sum(a.elapsed_time(b) for a, b in events) / len(events)
     plan = lib.describe_multi_plan(2 if fused else 1, T, B, n, dt_code, mode)
     kernel, has_probes = forward_kernel(plan)
-    if "product=sparse" in plan:  # (the form of the register kernel for groups of up to 8 rows in bf16)
-        kernel, has_probes = "k_lstm2_sparse", False
 
     # The latency of one hand-over of values between CUs (device-scope store -> load), measured live with the library's
     # probe: a lower bound of a time step of any kernel that keeps W spread over CUs.
@@ -1041,7 +1041,7 @@ def main():
             "kernel": "%s (one launch = %i op call(s) = %i units of T*B, 8*n^2 flops each)"
             % (kernel, len(directions) // launches, units_per_launch),
             "launch_ms": call_ms,
-            **ceiling_fields(probe_us, seq_ms, issue_ms, units_per_launch // T, n, dtype, T, call_ms),
+            **ceiling_fields(probe_us, "kernel=mfma_regw_xcd" not in plan, seq_ms, issue_ms, units_per_launch // T, n, dtype, T, call_ms),
             "mfma_issue_clock_mhz": issue_clock_mhz,
             "mfma_issue_clocks_per_mfma_by_instructions_behind": issue_clocks,
             "step_budget_us": step_budget(call_ms, nowait_ms, seq_ms, issue_ms, T),

@@ -354,4 +354,16 @@ def test_bench_names_the_kernel_of_the_plan():
     assert bench.forward_kernel((plan % "mfma_regw_solo").replace("rows_per_group=8 ", "rows_per_group=1 ")) == ("k_lstm2_solo_row", False)
     gradient = "kernel=bwd_regw_xcd problems=2 rows_per_group=8 groups=4 tiles=2 waves=4 wgs_per_group=32 launches=1 row_quads=0 name=k_lstm2_bwd_local"
     assert bench.gradient_kernels(gradient + " weight_gradient=rocblas,k_weight_last") == ("k_lstm2_bwd_local", "rocblas,k_weight_last")
-    assert bench.forward_kernel(lib.describe_plan(1000, 32, 1024, lib.DTYPE_BF16, lib.MODE_AUTO)) == ("k_lstm2_regw", True)
+    # the benchmark's own plan: groups of up to 8 rows in bf16, in the form of the register kernel that the probes do not repeat
+    assert bench.forward_kernel(plan % "mfma_regw_xcd_half" + " product=sparse") == ("k_lstm2_sparse", False)
+    assert bench.forward_kernel(lib.describe_plan(1000, 32, 1024, lib.DTYPE_BF16, lib.MODE_AUTO)) == ("k_lstm2_sparse", False)
+    assert bench.forward_kernel(lib.describe_plan(1000, 128, 1024, lib.DTYPE_BF16, lib.MODE_AUTO)) == ("k_lstm2_regw", True)
+
+
+def test_bench_has_a_latency_ceiling_only_between_xcds():
+    """The hand-over that bench.py measures is one at device scope: no bound for a plan whose groups are on one XCD each."""
+    import bench
+
+    inside, between = (bench.ceiling_fields(1.0, b, None, None, 64, 1024, "bf16", 1000, 1.26) for b in (False, True))
+    assert inside == {"handover_latency_us": 1.0}
+    assert between["handover_latency_us"] == 1.0 and 0.8 < between["frac_of_latency_ceiling"] < 1.0
