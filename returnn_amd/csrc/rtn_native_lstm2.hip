@@ -1675,8 +1675,8 @@ struct BwdLayout {
 BwdLayout bwd_layout(int64_t T, int B, int n, int dtype, int cells) {
   BwdLayout l;
   size_t off = 256;  // status block, as in the forward workspace
-  l.off_sync = off;  // two words per batch group (at most B groups): the XCD check of the persistent kernel
-  off = align_up(off + (size_t)B * 8, 256);
+  l.off_sync = off;  // the XCD check of the persistent kernels: two words per batch group (at most B groups), in k_lstm2_bwd_wide per group of 16 rows and XCD
+  off = align_up(off + std::max((size_t)B, (size_t)((B + 15) / 16) * kBwdWideRings) * 8, 256);
   l.off_dyw = off;
   off = align_up(off + (size_t)B * n * 4, 256);
   l.off_dx0 = off;
