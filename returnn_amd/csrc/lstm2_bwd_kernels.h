@@ -317,7 +317,7 @@ struct Lstm2BwdPersistent {
   int ksb;            // macro steps of the contraction per wavefront (<= the kernel's KSB; the rest of its slots stay empty)
   int poll_delay, delay_inc, delay_dec_mask;
   unsigned long long timeout_ticks;
-  unsigned* sync;     // [2 * groups of the whole problem] words of the XCD check (cleared before the launch)
+  unsigned* sync;     // words of the XCD check (cleared before the launch): two per group of the whole problem, k_lstm2_bwd_wide two per group and XCD
   void* exl;          // k_lstm2_bwd_wide: [xcds][kExRing][4n * 16] AT, the XCDs' rings (all-ones before every launch)
   void* ex;           // [groups of the whole problem][kExRing][4n * Bp] AT: the exchange ring (all-ones before the launch)
   int Bp, bp_shift;   // rows of a ring frame: 8 or 16 (= 1 << bp_shift), >= Bg

@@ -1349,7 +1349,7 @@ int fill_fwd_params(const rtn_lstm2_call& c, const Plan& pl, bool persistent, un
   // Device-scope stores take about a microsecond to become visible: a first read issued at once would
   // come back incomplete and cost a second round trip, so it is held back, and the kernel adapts the delay.  Within an
   // XCD the delay is a fixed one (tuned on MI355X over n = 64 ... 1024 and 1 ... 16 rows per group: the best fixed
-  // delay is within 2 % of these four everywhere, and 4 % to 13 % ahead of the adaptive one).
+  // delay is within 2 % of these three everywhere, and 4 % to 13 % ahead of the adaptive one).
   p.poll_delay = (int)std::max<long>(0, std::min<long>(64, env_long("RTN_LSTM2_POLL_DELAY", pl.local ? (pl.Bg > 8 ? 10 : (dtype != RTN_DTYPE_BF16 || pl.MT >= 8 ? 5 : 3)) : 20)));
   {
     long dec = env_long("RTN_LSTM2_DELAY_DEC", 8);  // steps per unit of downward adaptation: a power of two
@@ -1563,8 +1563,6 @@ int fwd_calls(const rtn_lstm2_call* calls, int count, int64_t T, int32_t B, int3
 }
 
 
-// Bytes of dynamic shared memory of the gradient kernel's variants that keep half of a wavefront's share of W in LDS (4
-// wavefronts with 32 + 32 fragments, or 8 wavefronts with 16 + 16).
 // k_lstm2_bwd_wide: groups that a launch's grid has room for, rings that a call's workspace has room for (one per XCD), LDS besides the weights'.
 constexpr int kBwdWideSlots = 4, kBwdWideRings = 8;
 static_assert(kMaxBwdMulti <= kBwdWideSlots, "a group of every problem of a launch");
@@ -1581,6 +1579,7 @@ bool bwd_wide_spares_launches(int count, int B, int n, int cus) {
   const int one_tile = std::max(1, cus / (n / 16) / count), turns_of_one_tile = (groups + one_tile - 1) / one_tile;
   return 5 * ((groups + per - 1) / per) < 4 * turns_of_one_tile;
 }
+// Bytes of dynamic shared memory of the gradient kernel's variants that keep half of a wavefront's share of W in LDS (8 wavefronts with 16 + 16 fragments).
 constexpr size_t kBwdLdsShareBytes = (size_t)kWaves * 32 * 64 * 16;
 
 // One rocBLAS handle per host thread and device, created on first use and kept for the life of the thread (never
